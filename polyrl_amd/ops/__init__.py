@@ -216,13 +216,15 @@ def varlen_prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if q.is_cuda:
         ext = _require_ext()
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        tile_seq, tile_q0 = _build_prefill_tiles(cu_seqlens_q)
+        none = torch.Tensor()
         lse = (torch.empty(q.shape[0], q.shape[1], dtype=torch.float32,
-                           device=q.device) if return_lse else torch.Tensor())
+                           device=q.device) if return_lse else none)
+        # no tile table: the kernel finds its row tiles from cu_seqlens_q,
+        # so the lengths need not come back to the host (the table cost a
+        # device-to-host wait and two uploads on every layer's call)
         ext.varlen_prefill_attention(
             out, q, k, v, cu_seqlens_q.int(),
-            cu_seqlens_k.int(), tile_seq.to(q.device), tile_q0.to(q.device),
-            scale, causal, lse)
+            cu_seqlens_k.int(), none, none, scale, causal, lse)
         return (out, lse) if return_lse else out
     out = ref.varlen_prefill_attention(q, k, v, cu_seqlens_q, cu_seqlens_k,
                                        scale, causal)

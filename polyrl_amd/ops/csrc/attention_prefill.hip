@@ -1,44 +1,41 @@
 // Varlen causal prefill attention, bf16, head_dim 64/128, GQA — MFMA forward.
 //
 // Reference capability: chunked-prefill flash attention (SURVEY.md §2.4.3
-// row 2).  MI355X-first structure (flash-style online softmax, no S matrix
-// materialized):
-//   * grid = (q_tiles, Hq); a workgroup = 4 waves = 64 query rows of one
-//     (sequence, q-head); wave w owns 16 rows.
-//   * per KV tile (KVBLK=32 keys): K and V staged to LDS — K XOR-swizzled
-//     (guide G4: row-major [32][128] bf16 would be a 16-way bank conflict on
-//     ds_read_b128), V row-major.
-//   * QK^T and P·V on v_mfma_f32_16x16x32_bf16.  Q fragments are
-//     register-resident for the whole kernel.
-//   * online softmax per row: running (m, l), O rescale by exp(m_old-m_new);
-//     row stats via 16-lane shfl_xor reduce (C-fragment rows live in 16-lane
-//     groups).
-//   * P changes fragment layout (C-layout -> A-layout) through a wave-private
-//     LDS tile (correctness-first; a permlane path can replace it later).
+// row 2).  Flash-style online softmax, no score matrix in memory.
+//
+// Split.  A wave owns 32 query rows of one head; a block is four such units
+// of one 64-row tile and one key/value head, heads of the group first (four
+// heads x 32 rows with a group of four), so the four waves read the same
+// keys and end at the same causal border.  K and V tiles of 64 keys come
+// through registers (the tile after next is in flight during a tile's
+// products) into one of two LDS buffers: one barrier per tile, 64 KiB at
+// D = 128, two blocks per CU.
+//
+// Products.  Scores are computed as S^T = K Q^T with the queries held in
+// registers: a lane's accumulators are 16 keys of ONE row, so the softmax
+// takes one lane exchange per tile, the row's maximum and sum are scalars of
+// the lane, and the weights, rounded to bf16, are at once the operand of
+// O^T += V^T P^T, whose V^T comes from the row-major tile by transposed LDS
+// reads (layouts: attention_tile.h).  The output is rescaled only in tiles
+// that move some row's maximum; only tiles that touch the causal border or
+// the sequence's end are masked.
+//
+// What bounds it: exponentials and matrix instructions of the two waves of a
+// SIMD, about as many cycles of each at D = 128 (the 16-row score tiles with
+// scalar LDS gathers for V that this replaces ran at 160 TFLOP/s).  Measured,
+// eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads of 64: 671 us a call
+// before (50 us of it the tile table's trip through the host), 174 us now
+// (610 TFLOP/s of live pairs).
+//
 // Chunked-prefill semantics: query block aligned to the END of the keys
 // (q row i at absolute kv position (Lk - Lq) + i), matching ops/ref.py.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include "attention_tile.h"
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
-#define KVBLK 64
-#define QROWS_PER_WAVE 16
-#define NWAVE 4
-#define QTILE (QROWS_PER_WAVE * NWAVE)  // 64
-
-// K-tile swizzle: byte_col ^= (row & 7) << 4  (16-B granularity, preserves
-// ds_read_b128 alignment; spreads a 16-lane group over 8 slots)
 template <int D>
-DEV_INLINE int kswz(int row, int byte_col) {
-  return row * (D * 2) + (byte_col ^ ((row & 7) << 4));
-}
-
-template <int HEAD_DIM>
-__global__ __launch_bounds__(256) void prefill_attn_kernel(
+__global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     bf16_t* __restrict__ out,        // (total_q, Hq, D)
     float* __restrict__ lse,         // (total_q, Hq) log-sum-exp, or null
     const bf16_t* __restrict__ q,    // (total_q, Hq, D)
@@ -46,209 +43,179 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
     const bf16_t* __restrict__ v,    // (total_k, Hk, D)
     const int* __restrict__ cu_q,    // (B+1,)
     const int* __restrict__ cu_k,
-    const int* __restrict__ tile_seq,  // (ntiles,)
+    const int* __restrict__ tile_seq,  // (ntiles,) or null
     const int* __restrict__ tile_q0,   // (ntiles,) local first q row
-    int Hq, int Hk, float scale, int causal, long ldq, long ldk, long ldv) {
-  __shared__ bf16_t Ks[KVBLK * HEAD_DIM];          // swizzled
-  __shared__ bf16_t Vs[KVBLK * HEAD_DIM];          // row-major
-  __shared__ bf16_t Ps[NWAVE][QROWS_PER_WAVE * KVBLK];
+    int nseq, int ntiles, int nparts, int Hq, int Hk, float scale, int causal,
+    long ldq, long ldk, long ldv) {
+  typedef AttnTile<D> T;
+  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
 
-  const int tile = blockIdx.x;
-  const int hq = blockIdx.y;
-  const int hk = hq / (Hq / Hk);
-  const int seq = tile_seq[tile];
-  const int q0 = tile_q0[tile];                    // local
-  const int qbeg = cu_q[seq], qend = cu_q[seq + 1];
-  const int kbeg = cu_k[seq], kend = cu_k[seq + 1];
-  const int Lq = qend - qbeg, Lk = kend - kbeg;
+  const int G = Hq / Hk;
+  const int item = die_item(ntiles * Hk * nparts);
+  if (item >= ntiles * Hk * nparts) return;
+  const int hk = item / (ntiles * nparts);
+  // later tiles of a sequence see more keys: they start first
+  const int tile = ntiles - 1 - item / nparts % ntiles;
+  int seq, q0;
+  if (!find_tile(tile, tile_seq, tile_q0, cu_q, nseq, seq, q0)) return;
+  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
+  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;                      // chunked-prefill alignment
 
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
-  const int l15 = lane & 15;
-  const int lhi = lane >> 4;                       // 0..3
-  constexpr int KS = HEAD_DIM / 32;                // A/B k-steps over d
-  constexpr int NDT = HEAD_DIM / 16;               // 16-wide d-tiles of O
+  constexpr int KS = D / 16, DT = D / 32;
+  const int unit = item % nparts * 4 + wid;        // (row half, head)
+  const int hq = hk * G + unit % G;
+  const int wq0 = q0 + unit / G * 32;              // this wave's first row
+  const bool busy = unit < 2 * G && wq0 < Lq;
+  const int row = wq0 + (lane & 31);               // this lane's row
+  const int qpos = causal ? qk_off + row : Lk;     // last key it sees
 
-  // this wave's q rows: local q0 + wid*16 + (row index 0..15)
-  const int wq0 = q0 + wid * QROWS_PER_WAVE;
+  // keys that this wave and this block walk
+  const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
+  const int wend = busy ? seen : 0;
+  const int last_half = min(item % nparts * 4 + 3, 2 * G - 1) / G;
+  const int bend = causal
+      ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
-  // ---- Q fragments (A-layout): row i = l15, k-elem = lhi*8 + j ----
-  // 4 k-steps cover d = 0..127.  Rows past Lq load row 0 (masked later).
-  bf16x8_t qfrag[KS];
-  {
-    const int qrow_l = wq0 + l15;
-    const long grow = (long)qbeg + ((qrow_l < Lq) ? qrow_l : 0);
-    const bf16_t* qp = q + grow * ldq + (long)hq * HEAD_DIM + lhi * 8;
+  bf16x8_t qf[KS];
+  frag_global<D>(qf, q + (long)(qbeg + min(busy ? row : 0, Lq - 1)) * ldq +
+                         (long)hq * D * (busy ? 1 : 0));
+
+  const FragAt<D> at;
+  const float s2 = scale * 1.4426950408889634f;    // scores in powers of two
+  float m_run = -1e30f, l_run = 0.f;               // l: this lane's keys only
+  f32x16_t o[DT];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qfrag[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+
+  const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
+  const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
+  i32x4_t rk[T::LOADS], rv[T::LOADS];
+  if (bend > 0) {
+    T::fetch(rk, kb, ldk, 0, Lk);
+    T::fetch(rv, vb, ldv, 0, Lk);
+    T::store(lds[0][0], rk);
+    T::store(lds[0][1], rv);
+    if (ATILE < bend) {
+      T::fetch(rk, kb, ldk, ATILE, Lk);
+      T::fetch(rv, vb, ldv, ATILE, Lk);
+    }
   }
+  __syncthreads();
 
-  // online-softmax state: rows (lhi*4 + r) for r=0..3 (C-layout rows)
-  float m_run[4], l_run[4];
-  f32x4_t o_acc[NDT];  // d-tiles of 16; reg r = row lhi*4+r
+  int buf = 0;
+  for (int t0 = 0; t0 < bend; t0 += ATILE, buf ^= 1) {
+    // the next tile into the other buffer (its readers passed the barrier)
+    if (t0 + ATILE < bend) {
+      T::store(lds[buf ^ 1][0], rk);
+      T::store(lds[buf ^ 1][1], rv);
+      if (t0 + 2 * ATILE < bend) {
+        T::fetch(rk, kb, ldk, t0 + 2 * ATILE, Lk);
+        T::fetch(rv, vb, ldv, t0 + 2 * ATILE, Lk);
+      }
+    }
+    if (t0 < wend) {
+      const char* ks_ = lds[buf][0];
+      const char* vs_ = lds[buf][1];
+      // ---- S^T: 64 keys x 32 rows ------------------------------------------
+      f32x16_t s[2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m_run[r] = -1e30f;
-    l_run[r] = 0.f;
-  }
+      for (int n = 0; n < 2; ++n) {
 #pragma unroll
-  for (int nt = 0; nt < NDT; ++nt) o_acc[nt] = {0.f, 0.f, 0.f, 0.f};
-
-  // causal kv extent for this block
-  const int max_qpos = qk_off + min(q0 + QTILE - 1, Lq - 1);
-  const int kv_end = causal ? min(Lk, max_qpos + 1) : Lk;
-
-  for (int t0 = 0; t0 < kv_end; t0 += KVBLK) {
-    // ---------------- stage K (swizzled) and V (row-major) ----------------
-    // 256 threads x 2 iters x 8 elems = 4096 elems = 32x128
-    {
-      const int tid = threadIdx.x;
+        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
 #pragma unroll
-      for (int it = 0; it < KVBLK * HEAD_DIM / (256 * 8); ++it) {
-        const int flat = (tid + it * 256) * 8;
-        const int row = flat / HEAD_DIM;
-        const int col = flat % HEAD_DIM;
-        const int krow = t0 + row;
-        bf16x8 kv8, vv8;
-        if (krow < Lk) {
-          kv8 = *reinterpret_cast<const bf16x8*>(
-              k + (long)(kbeg + krow) * ldk + (long)hk * HEAD_DIM + col);
-          vv8 = *reinterpret_cast<const bf16x8*>(
-              v + (long)(kbeg + krow) * ldv + (long)hk * HEAD_DIM + col);
-        } else {
-          for (int j = 0; j < 8; ++j) kv8.v[j] = f2bf(0.f), vv8.v[j] = f2bf(0.f);
+        for (int ks = 0; ks < KS; ++ks)
+          s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_rows<D>(ks_, at, n, ks), qf[ks], s[n], 0, 0, 0);
+      }
+      // ---- mask (wave-uniform: some key of the tile is hidden) --------------
+      if (t0 + ATILE > Lk || (causal && t0 + ATILE - 1 > qk_off + wq0)) {
+        const int last = min(qpos, Lk - 1) - t0;
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (n * 32 + acc_row(r) > last) s[n][r] = -INFINITY;
+      }
+      // ---- online softmax -----------------------------------------------------
+      float mx = s[0][0];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
+      const float mn = fmaxf(m_run, half_max(mx) * s2);
+      if (__any(mn > m_run)) {
+        const float alpha = exp2_hw(m_run - mn);
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+        m_run = mn;
+      }
+      float sum = 0.f;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          s[n][r] = exp2_hw(__builtin_fmaf(s[n][r], s2, -m_run));
+          sum += s[n][r];
         }
-        *reinterpret_cast<bf16x8*>(
-            reinterpret_cast<char*>(Ks) + kswz<HEAD_DIM>(row, col * 2)) = kv8;
-        *reinterpret_cast<bf16x8*>(Vs + row * HEAD_DIM + col) = vv8;
+      l_run += sum;
+      // ---- O^T += V^T P^T ------------------------------------------------------
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const bf16x8_t p = acc_operand(s[st >> 1], st & 1);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(vs_, at, dt, st), p, o[dt], 0, 0, 0);
       }
     }
     __syncthreads();
-
-    // ---------------- QK^T: S[16 q][KVBLK keys] = Q @ K^T -----------------
-    // B-frag (d x key): lane reads K[key = nt*16 + l15][d = ks*32 + lhi*8 ..]
-    constexpr int NKT = KVBLK / 16;
-    f32x4_t c[NKT];
-#pragma unroll
-    for (int nt = 0; nt < NKT; ++nt) c[nt] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int nt = 0; nt < NKT; ++nt) {
-      const int krow = nt * 16 + l15;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8_t bf = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<char*>(Ks) +
-            kswz<HEAD_DIM>(krow, (ks * 32 + lhi * 8) * 2));
-        c[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qfrag[ks], bf, c[nt],
-                                                        0, 0, 0);
-      }
-    }
-
-    // ---------------- scale + causal mask ---------------------------------
-    // C layout: row = lhi*4 + r, col = l15.  Interior tiles (every (q, k)
-    // pair live: tile fully below the causal diagonal of the wave's
-    // earliest row, all rows/keys in range) skip the per-element mask —
-    // the kernels are VALU-bound (PMC: 16:1 VALU:MFMA), not memory-bound.
-    float s[NKT][4];
-    const bool interior = (t0 + KVBLK <= Lk) && (wq0 + 16 <= Lq) &&
-                          (!causal || t0 + KVBLK - 1 <= qk_off + wq0);
-    if (interior) {
-#pragma unroll
-      for (int nt = 0; nt < NKT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[nt][r] = c[nt][r] * scale;
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < NKT; ++nt) {
-        const int kpos = t0 + nt * 16 + l15;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int qrow_l = wq0 + lhi * 4 + r;
-          const int qpos = qk_off + qrow_l;
-          const bool dead = (kpos >= Lk) || (qrow_l >= Lq) ||
-                            (causal && kpos > qpos);
-          s[nt][r] = dead ? -1e30f : c[nt][r] * scale;
-        }
-      }
-    }
-
-    // ---------------- online softmax (per C-row) ---------------------------
-    float p[NKT][4];
-    float alpha[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float rm = s[0][r];
-#pragma unroll
-      for (int nt = 1; nt < NKT; ++nt) rm = fmaxf(rm, s[nt][r]);
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) rm = fmaxf(rm, __shfl_xor(rm, off, 64));
-      const float mn = fmaxf(m_run[r], rm);
-      alpha[r] = __expf(m_run[r] - mn);
-      m_run[r] = mn;
-      float rs = 0.f;
-#pragma unroll
-      for (int nt = 0; nt < NKT; ++nt) {
-        p[nt][r] = __expf(s[nt][r] - mn);
-        rs += p[nt][r];
-      }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) rs += __shfl_xor(rs, off, 64);
-      l_run[r] = l_run[r] * alpha[r] + rs;
-    }
-    // rescale O
-#pragma unroll
-    for (int nt = 0; nt < NDT; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o_acc[nt][r] *= alpha[r];
-
-    // ---------------- P: C-layout -> A-layout through wave-private LDS ----
-    bf16_t* ps = Ps[wid];
-#pragma unroll
-    for (int nt = 0; nt < NKT; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ps[(lhi * 4 + r) * KVBLK + nt * 16 + l15] = f2bf(p[nt][r]);
-    // wave-private tile: the compiler orders ds_write -> ds_read by lgkmcnt
-
-    // ---------------- P @ V ------------------------------------------------
-    // k runs over the KVBLK keys in 32-deep steps (A-frag k = kq*32+lhi*8)
-#pragma unroll
-    for (int kq = 0; kq < KVBLK / 32; ++kq) {
-      const bf16x8_t pa = *reinterpret_cast<const bf16x8_t*>(
-          ps + l15 * KVBLK + kq * 32 + lhi * 8);
-#pragma unroll
-      for (int nt = 0; nt < NDT; ++nt) {
-        bf16x8_t bv;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          bv[j] = *reinterpret_cast<const __bf16*>(
-              Vs + (kq * 32 + lhi * 8 + j) * HEAD_DIM + nt * 16 + l15);
-        o_acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, bv,
-                                                            o_acc[nt],
-                                                            0, 0, 0);
-      }
-    }
-    __syncthreads();  // all waves done with Ks/Vs before restage
   }
 
-  // ---------------- epilogue: out = O / l; lse = m + log l ----------------
+  // ---- out = O / l, turned through LDS to whole rows; lse = m + log l --------
+  const float l = half_sum(l_run);
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
+  if (busy) {
+    if (lse != nullptr && lane < 32 && row < Lq)
+      lse[((long)qbeg + row) * Hq + hq] =
+          l > 0.f ? m_run * 0.6931471805599453f + __logf(l) : -1e30f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int qrow_l = wq0 + lhi * 4 + r;
-    if (qrow_l >= Lq) continue;
-    const float inv = (l_run[r] > 0.f) ? 1.0f / l_run[r] : 0.f;
-    bf16_t* op = out + (((long)qbeg + qrow_l) * Hq + hq) * HEAD_DIM;
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int nt = 0; nt < NDT; ++nt)
-      op[nt * 16 + l15] = f2bf(o_acc[nt][r] * inv);
-    if (lse != nullptr && l15 == 0)
-      lse[((long)qbeg + qrow_l) * Hq + hq] =
-          (l_run[r] > 0.f) ? (m_run[r] + __logf(l_run[r])) : -1e30f;
+      for (int i = 0; i < 4; ++i) {
+        bf16x4 w;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) w.v[t] = f2bf(o[dt][4 * i + t] * inv);
+        const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
+        *reinterpret_cast<bf16x4*>(
+            mine + (lane & 31) * (2 * D) +
+            (((d >> 3) ^ T::swz(lane & 31)) << 4) + (d & 4) * 2) = w;
+      }
+  }
+  __syncthreads();
+  if (!busy) return;
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    const int at16 = lane + i * 64;
+    const int r = at16 / T::GR, g = at16 % T::GR;
+    if (wq0 + r < Lq)
+      *reinterpret_cast<bf16x8*>(
+          out + (((long)qbeg + wq0 + r) * Hq + hq) * D + g * 8) =
+          *reinterpret_cast<const bf16x8*>(mine + r * (2 * D) +
+                                           ((g ^ T::swz(r)) << 4));
   }
 }
 
+// tile_seq / tile_q0: the 64-row tiles of the packed rows, or empty: the
+// kernel then finds them from cu_seqlens_q itself.
 void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
                               torch::Tensor k, torch::Tensor v,
                               torch::Tensor cu_seqlens_q,
@@ -269,20 +236,32 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
               "q/k/v heads and dims must be packed (token stride free)");
   TORCH_CHECK(out.is_contiguous());
   TORCH_CHECK(cu_seqlens_q.dtype() == torch::kInt32);
-  TORCH_CHECK(tile_seq.dtype() == torch::kInt32 && tile_q0.dtype() == torch::kInt32);
+  const bool table = tile_seq.defined() && tile_seq.numel() > 0;
+  if (table)
+    TORCH_CHECK(tile_seq.dtype() == torch::kInt32 &&
+                tile_q0.dtype() == torch::kInt32);
   const int Hq = q.size(1), D = q.size(2), Hk = k.size(1);
   TORCH_CHECK(D == 128 || D == 64, "prefill kernel supports head_dim 64/128");
   TORCH_CHECK(Hq % Hk == 0);
-  const int ntiles = tile_seq.size(0);
+  const int nseq = cu_seqlens_q.size(0) - 1;
+  const long ntiles = table ? tile_seq.size(0)
+                            : q.size(0) / ATILE + nseq;
+  if (ntiles == 0 || q.size(0) == 0) return;
+  const int nparts = (2 * (Hq / Hk) + 3) / 4;      // blocks of a tile's units
+  const long items = ntiles * Hk * nparts;
+  const long blocks = (items + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
+  TORCH_CHECK(blocks < (1L << 31), "grid too large");
   auto stream = at::hip::getCurrentHIPStream();
   auto kern = (D == 128) ? prefill_attn_kernel<128> : prefill_attn_kernel<64>;
-  kern<<<dim3(ntiles, Hq), dim3(256), 0, stream>>>(
+  kern<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
       (bf16_t*)out.data_ptr(),
       want_lse ? lse.data_ptr<float>() : nullptr,
       (const bf16_t*)q.data_ptr(),
       (const bf16_t*)k.data_ptr(), (const bf16_t*)v.data_ptr(),
       cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
-      tile_seq.data_ptr<int>(), tile_q0.data_ptr<int>(), Hq, Hk, (float)scale,
-      causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
+      table ? tile_seq.data_ptr<int>() : nullptr,
+      table ? tile_q0.data_ptr<int>() : nullptr, nseq, (int)ntiles, nparts,
+      Hq, Hk, (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0),
+      v.stride(0));
   HIP_CHECK_KERNEL();
 }

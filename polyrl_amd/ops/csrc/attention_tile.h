@@ -1,0 +1,185 @@
+// Tiles of the matrix-core attention kernels (attention_prefill.hip,
+// attention_backward_v3.hip): 64 rows x D bf16 numbers in LDS, their
+// fragments for v_mfma_f32_32x32x16_bf16, and the table of row tiles.
+//
+// Layout.  A tile row is D numbers in 16-byte granules; granule g of row r
+// lies at place g ^ swz(r).  Two kinds of reads are free of bank conflicts
+// (64 banks of 4 bytes):
+//   * rows as they are (frag_rows, ds_read_b128): 16 neighbouring rows read
+//     the same granule, so the places of 16 rows must differ;
+//   * columns (frag_cols, ds_read_b64_tr_b16): four neighbouring rows read
+//     the same 64 bytes, so their 64-byte windows must differ: the window
+//     bits of swz come from the row's lowest bits.
+//
+// Operands.  32x32x16: lane l holds row (A) or column (B) l % 32 and eight
+// numbers of the inner dimension from 8 * (l / 32); accumulator register r
+// is row 8 * (r / 4) + 4 * (l / 32) + r % 4 of column l % 32.  A product's
+// inner order is free as long as both operands use the same one, so an
+// accumulator, rounded to bf16, is at once the B operand of the next product:
+// registers 8s .. 8s+7 are inner step s, in the order that frag_cols reads.
+#pragma once
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+typedef __attribute__((ext_vector_type(4))) short i16x4_t;
+typedef __attribute__((ext_vector_type(8))) short i16x8_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_p;
+
+#define ATILE 64                      // rows of a tile
+#define ATTN_XCDS 8                   // dies, each with an L2 of its own
+
+template <int D>
+struct AttnTile {
+  static constexpr int BYTES = ATILE * D * 2;
+  static constexpr int GR = D / 8;    // granules of a row
+  static constexpr int LOADS = ATILE * GR / 256;  // granules per thread
+
+  DEV_INLINE static int swz(int r) {
+    return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3)
+                    : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  }
+
+  // this thread's granules of rows [r0, r0 + 64) of one head; rows from
+  // ``rows`` on repeat the last one (what they give is masked or dropped)
+  DEV_INLINE static void fetch(i32x4_t (&reg)[LOADS], const bf16_t* base,
+                               long ld, int r0, int rows) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int at = threadIdx.x + i * 256;
+      const int r = min(r0 + at / GR, rows - 1);
+      reg[i] = *reinterpret_cast<const i32x4_t*>(base + r * ld + at % GR * 8);
+    }
+  }
+
+  DEV_INLINE static void store(char* tile, const i32x4_t (&reg)[LOADS]) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int at = threadIdx.x + i * 256;
+      const int r = at / GR;
+      *reinterpret_cast<i32x4_t*>(tile + r * (2 * D) +
+                                 ((at % GR ^ swz(r)) << 4)) = reg[i];
+    }
+  }
+};
+
+// Per-lane offsets of the two kinds of fragments.
+template <int D>
+struct FragAt {
+  int rows, cols0, cols1;
+  DEV_INLINE FragAt() {
+    const int lane = threadIdx.x & 63;
+    const int h = lane >> 5, r = lane & 31, c = lane & 15;
+    rows = r * (2 * D) + ((h ^ AttnTile<D>::swz(r)) << 4);
+    const int ra = 4 * h + (c >> 2), rb = ra + 8;
+    const int g = ((lane >> 4) & 1) * 2 + ((c & 3) >> 1);
+    cols0 = ra * (2 * D) + ((g ^ AttnTile<D>::swz(ra)) << 4) + (c & 1) * 8;
+    cols1 = rb * (2 * D) + ((g ^ AttnTile<D>::swz(rb)) << 4) + (c & 1) * 8;
+  }
+};
+
+// A operand with the tile's rows [32 * sub, +32) as its rows, inner step ks
+// over D
+template <int D>
+DEV_INLINE bf16x8_t frag_rows(const char* tile, const FragAt<D>& at, int sub,
+                              int ks) {
+  return *reinterpret_cast<const bf16x8_t*>(
+      tile + sub * 32 * (2 * D) + (at.rows ^ (ks << 5)));
+}
+
+// A operand with the tile's columns [32 * dt, +32) as its rows, inner step s
+// over the tile's rows [16 * s, +16) in the accumulators' order
+template <int D>
+DEV_INLINE bf16x8_t frag_cols(const char* tile, const FragAt<D>& at, int dt,
+                              int s) {
+  const char* p = tile + s * 16 * (2 * D);
+  const i16x4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_i16x4_p)(p + (at.cols0 ^ (dt << 6))));
+  const i16x4_t b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_i16x4_p)(p + (at.cols1 ^ (dt << 6))));
+  const i16x8_t v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// row (or column) fragments of one head straight from memory: lane l holds
+// row l % 32 of 32 rows, numbers 16 * ks + 8 * (l / 32) ..
+template <int D>
+DEV_INLINE void frag_global(bf16x8_t (&f)[D / 16], const bf16_t* row) {
+  const int h = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks)
+    f[ks] = *reinterpret_cast<const bf16x8_t*>(row + ks * 16 + h * 8);
+}
+
+// B operand from accumulator registers 8s .. 8s+7
+DEV_INLINE bf16x8_t acc_operand(const f32x16_t& c, int s) {
+  bf16x8_t v;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = (__bf16)c[8 * s + j];
+  return v;
+}
+
+// row of a 32-row accumulator that register r holds in this lane
+DEV_INLINE int acc_row(int r) {
+  return 8 * (r >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (r & 3);
+}
+
+// the larger / the sum of a lane's value and that of the lane 32 away
+DEV_INLINE float half_max(float x) {
+  const auto p = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+DEV_INLINE float half_sum(float x) {
+  const auto p = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+// 2^x in one instruction; results below 2^-126 become 0
+DEV_INLINE float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Sequence and first row of row tile ``tile``.  With a table it is looked
+// up; without one the tiles are the sequences' 64-row pieces in order, found
+// from cu_q by one scan (64 sequences a step), so that a caller that does
+// not know the lengths on the host launches rows / 64 + sequences tiles and
+// the ones past the last return false.
+DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
+                          const int* cu, int nseq, int& seq, int& r0) {
+  if (tile_seq != nullptr) {
+    seq = tile_seq[tile];
+    r0 = tile_r0[tile];
+    return true;
+  }
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int s0 = 0; s0 < nseq; s0 += 64) {
+    const int s = s0 + lane;
+    const int n = s < nseq ? (cu[s + 1] - cu[s] + ATILE - 1) / ATILE : 0;
+    int upto = n;                      // tiles of sequences s0 .. s
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += o;
+    }
+    const unsigned long long past = __ballot(before + upto > tile);
+    if (past) {
+      const int l = __ffsll((long long)past) - 1;
+      seq = s0 + l;
+      r0 = (tile - before - __shfl(upto - n, l, 64)) * ATILE;
+      return true;
+    }
+    before += __shfl(upto, 63, 64);
+  }
+  return false;
+}
+
+// Work item of a block.  Blocks go to the dies in turn (id % 8); each die
+// takes one stretch of the items, whose order is key/value head, row tile,
+// part, so the tiles that read the same keys share an L2.
+DEV_INLINE int die_item(int items) {
+  const int per = (items + ATTN_XCDS - 1) / ATTN_XCDS;
+  return (int)(blockIdx.x % ATTN_XCDS) * per + (int)(blockIdx.x / ATTN_XCDS);
+}
