@@ -264,15 +264,13 @@ class _FlashAttnVarlen(torch.autograd.Function):
         ver = _os.environ.get("POLYRL_ATTN_BWD", "v3")
         if ver == "v3":
             # atomic-free dkv+dq split: every output row written exactly
-            # once, so the grad buffers need no zero-fill
-            dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-            dk = torch.empty(k.shape, dtype=torch.float32, device=q.device)
-            dv = torch.empty(v.shape, dtype=torch.float32, device=q.device)
+            # once and in the inputs' type, so the grad buffers need no
+            # zero-fill and no cast
+            dq, dk, dv = (torch.empty_like(t) for t in (q, k, v))
             ext.varlen_attention_backward_v3(
                 dq, dk, dv, q, k, v, out, dout.contiguous(), lse,
                 cu, cu, t64_seq, t64_q0, ctx.scale, ctx.causal)
-            return (dq.to(q.dtype), dk.to(q.dtype), dv.to(q.dtype),
-                    None, None, None, None, None, None, None)
+            return (dq, dk, dv, None, None, None, None, None, None, None)
         dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
         dk = torch.zeros(k.shape, dtype=torch.float32, device=q.device)
         dv = torch.zeros(v.shape, dtype=torch.float32, device=q.device)

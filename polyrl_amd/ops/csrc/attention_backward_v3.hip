@@ -3,477 +3,497 @@
 // Reference capability: the training-side flash-attn backward the reference
 // reaches through the flash-attn package (SURVEY.md §2.2.2 'flash-attn').
 //
-// v1/v2 (attention_backward.hip) are KV-stationary single-kernel designs
-// whose dQ (every q-block) and dK/dV (every block) updates go through
-// global fp32 atomics, at 104 KiB LDS = 1 block/CU.  Measured ~10% MFU,
-// and a fully-vectorized-LDS v2 ran at exactly v1's speed — the kernel is
-// atomics/occupancy-bound, not LDS-issue-bound (profiles/PROFILES.md).
+// Two kernels that each OWN the rows they write: no atomics, no zero-fill,
+// the same bits on every run; gradients are rounded to bf16 once, as they are
+// written.  The recompute of S and dP in both is 7 products instead of 5.
+// Layouts and operands: attention_tile.h.
 //
-// v3 removes every atomic by splitting the backward into two kernels that
-// each OWN their output rows exclusively (the extra recompute of S/dP is
-// ~1.4x FLOPs for >5x less memory traffic):
+//  * dq kernel — units, blocks and tiles of the forward kernel
+//    (attention_prefill.hip): a wave holds Q and dO of 32 rows of one head in
+//    registers and walks the keys; S^T = K Q^T and dP^T = V dO^T, whose
+//    difference dS^T, rounded to bf16, is at once the operand of
+//    dQ^T += K^T dS^T (K^T by transposed LDS reads of the K tile).  It
+//    starts with delta = rowsum(dO * O) of its rows, from the fragments it
+//    loads anyway, and leaves it for the other kernel: it runs first.
+//  * dkv kernel — a block owns 64 keys of one key/value head and walks the
+//    64-row query tiles of the group's heads; wave = (32 keys, 32 rows).
+//    S = Q K^T and dP = dO V^T have keys as columns, so P and dS are the
+//    operands of dV^T += dO^T P and dK^T += Q^T dS.  256 registers a wave
+//    (two waves per SIMD, so that one's exponentials run beside the other's
+//    products) hold both gradients and K at D = 128 but not V, which is read
+//    from LDS; the next Q tile is in flight during the first two products,
+//    the next dO tile during the last two, in the same 16 registers.  Q has
+//    two LDS buffers, dO one (stored between two barriers).  The two waves of
+//    a key half meet at the end: each adds the other's share of one gradient.
+//    With few blocks the group's heads are divided among several (their
+//    shares then pass through fp32 and one summing kernel).
 //
-//  * dkv kernel — grid (kv-tile of 64 keys, kv-head).  The GQA group's G
-//    q-heads are a register-accumulated loop INSIDE the block, so dK/dV
-//    for the tile are complete when the block ends: one plain store pass.
-//    4 waves split the 64-q-row block by q (16 rows each) for S/dP and by
-//    d-slice (D/4 columns each) for the dV/dK MFMAs.  LDS 80 KiB (D=128)
-//    -> 2 blocks/CU.
-//  * dq kernel — grid (q-tile of 64 rows, q-head).  Waves own 16 q rows
-//    for the whole kv loop and accumulate dQ in registers; one store pass
-//    at the end.  LDS 56 KiB (D=128).
-//
-// Both kernels reuse the 64-granularity tile table the forward already
-// builds (build_varlen_tiles t64), so no extra host work per batch.
+// What bounds it: matrix instructions and LDS reads of their operands (one
+// fragment of 1 KiB per 32-cycle product).  Measured, forward and backward of
+// packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with kernels
+// that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
+// gradients for a cast to read, 349 us now; 2 of up to 4096, 28/4 heads,
+// 4000 -> 1580 us.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include "attention_tile.h"
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
-#define KB3 64             // keys per kv tile
-#define QB3 64             // q rows per block / iteration
-#define NWAVE3 4
-
-// swizzled row-major [rows][D] image (byte addressing), 16-B granules
+// ------------------------------------------------------------------- dQ
 template <int D>
-DEV_INLINE int kswz3(int row, int byte_col) {
-  return row * (D * 2) + (byte_col ^ ((row & 7) << 4));
-}
+__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
+    bf16_t* __restrict__ dq,         // (total_q, Hq, D)
+    float* __restrict__ delta,       // (total_q, Hq)
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
+    const bf16_t* __restrict__ v, const bf16_t* __restrict__ out,
+    const bf16_t* __restrict__ dout, // (total_q, Hq, D) contiguous, like out
+    const float* __restrict__ lse, const int* __restrict__ cu_q,
+    const int* __restrict__ cu_k, const int* __restrict__ tile_seq,
+    const int* __restrict__ tile_q0, int ntiles, int nparts, int Hq, int Hk,
+    float scale, int causal, long ldq, long ldk, long ldv) {
+  typedef AttnTile<D> T;
+  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
 
-// transposed [d][X] image (element addressing), 8-element granules
-DEV_INLINE int trid3(int d, int x, int X) {
-  return d * X + (x ^ ((d & 3) << 3));
-}
-DEV_INLINE int trid3_vec(int d, int xblock, int X) {
-  return d * X + ((xblock * 8) ^ ((d & 3) << 3));
-}
-
-// ------------------------------------------------------- delta preprocess
-// delta[t, h] = sum_d dO[t,h,d] * O[t,h,d]   (fp32)
-template <int D>
-__global__ void attn_bwd_delta_kernel3(float* __restrict__ delta,
-                                       const bf16_t* __restrict__ dout,
-                                       const bf16_t* __restrict__ out,
-                                       long rows /* total_q * Hq */) {
-  const long row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int lane = threadIdx.x & 63;
-  const bf16x8* dp = reinterpret_cast<const bf16x8*>(dout + row * D);
-  const bf16x8* op = reinterpret_cast<const bf16x8*>(out + row * D);
-  float acc = 0.f;
-  if (lane < D / 8) {
-    bf16x8 d8 = dp[lane], o8 = op[lane];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc += bf2f(d8.v[j]) * bf2f(o8.v[j]);
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if (lane == 0) delta[row] = acc;
-}
-
-// ---------------------------------------------------------------- dK/dV
-template <int D>
-__global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(
-    float* __restrict__ dk,          // (total_k, Hk, D) fp32 (fully written)
-    float* __restrict__ dv,
-    const bf16_t* __restrict__ q,    // packed (strided) inputs
-    const bf16_t* __restrict__ k,
-    const bf16_t* __restrict__ v,
-    const bf16_t* __restrict__ dout, // (total_q, Hq, D) contiguous
-    const float* __restrict__ lse,   // (total_q, Hq)
-    const float* __restrict__ delta, // (total_q, Hq)
-    const int* __restrict__ cu_q, const int* __restrict__ cu_k,
-    const int* __restrict__ tile_seq, const int* __restrict__ tile_k0,
-    int Hq, int Hk, float scale, int causal,
-    long ldq, long ldk, long ldv) {
-  __shared__ bf16_t KsSwz[KB3 * D];          // B-frags of S = Q K^T
-  __shared__ bf16_t VsSwz[KB3 * D];          // B-frags of dP = dO V^T
-  __shared__ bf16_t QsT[D * QB3];            // [d][q] for dK += dS^T Q
-  __shared__ bf16_t DOsT[D * QB3];           // [d][q] for dV += P^T dO
-  __shared__ bf16_t Pt[KB3 * QB3];           // [key][q]
-  __shared__ bf16_t DSt[KB3 * QB3];
-
-  const int tile = blockIdx.x;
-  const int hk = blockIdx.y;
   const int G = Hq / Hk;
-  const int seq = tile_seq[tile];
-  const int t0 = tile_k0[tile];              // local first key of this tile
-  const int qbeg = cu_q[seq], qend = cu_q[seq + 1];
-  const int kbeg = cu_k[seq], kend = cu_k[seq + 1];
-  const int Lq = qend - qbeg, Lk = kend - kbeg;
+  const int item = die_item(ntiles * Hk * nparts);
+  if (item >= ntiles * Hk * nparts) return;
+  const int hk = item / (ntiles * nparts);
+  const int tile = ntiles - 1 - item / nparts % ntiles;   // long rows first
+  const int seq = tile_seq[tile], q0 = tile_q0[tile];
+  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
+  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;
 
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
-  const int l15 = lane & 15;
-  const int lhi = lane >> 4;                 // 0..3
-  constexpr int KS = D / 32;                 // k-steps over head_dim
-  constexpr int NDT = D / 64;                // 16-wide d-tiles per wave slice
+  constexpr int KS = D / 16, DT = D / 32;
+  const int unit = item % nparts * 4 + wid;        // (row half, head)
+  const int wq0 = q0 + unit / G * 32;
+  const bool busy = unit < 2 * G && wq0 < Lq;
+  const int hq = busy ? hk * G + unit % G : hk * G;
+  const int row = wq0 + (lane & 31);
+  const int qpos = causal ? qk_off + row : Lk;
 
-  // ---- stage K/V swizzled (once per block) ------------------------------
+  const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
+  const int wend = busy ? seen : 0;
+  const int last_half = min(item % nparts * 4 + 3, 2 * G - 1) / G;
+  const int bend = causal
+      ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
+
+  const long tok = qbeg + min(busy ? row : 0, Lq - 1);
+  bf16x8_t qf[KS], df[KS];
+  frag_global<D>(df, dout + (tok * Hq + hq) * D);
+  float del = 0.f;
   {
-    const int tid = threadIdx.x;
+    bf16x8_t of[KS];
+    frag_global<D>(of, out + (tok * Hq + hq) * D);
 #pragma unroll
-    for (int it = 0; it < KB3 * D / (256 * 8); ++it) {
-      const int flat = (tid + it * 256) * 8;
-      const int row = flat / D;
-      const int col = flat % D;
-      const int krow = t0 + row;
-      bf16x8 k8, v8;
-      if (krow < Lk) {
-        k8 = *reinterpret_cast<const bf16x8*>(
-            k + (long)(kbeg + krow) * ldk + (long)hk * D + col);
-        v8 = *reinterpret_cast<const bf16x8*>(
-            v + (long)(kbeg + krow) * ldv + (long)hk * D + col);
-      } else {
-        for (int j = 0; j < 8; ++j) k8.v[j] = f2bf(0.f), v8.v[j] = f2bf(0.f);
-      }
-      *reinterpret_cast<bf16x8*>(
-          reinterpret_cast<char*>(KsSwz) + kswz3<D>(row, col * 2)) = k8;
-      *reinterpret_cast<bf16x8*>(
-          reinterpret_cast<char*>(VsSwz) + kswz3<D>(row, col * 2)) = v8;
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) del += (float)df[ks][j] * (float)of[ks][j];
+    del = half_sum(del);
+  }
+  if (busy && lane < 32 && row < Lq) delta[tok * Hq + hq] = del;
+  frag_global<D>(qf, q + tok * ldq + (long)hq * D);
+  const float s2 = scale * 1.4426950408889634f;
+  const float lse2 = lse[tok * Hq + hq] * 1.4426950408889634f;
+
+  const FragAt<D> at;
+  f32x16_t acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+
+  const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
+  const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
+  i32x4_t rk[T::LOADS], rv[T::LOADS];
+  if (bend > 0) {
+    T::fetch(rk, kb, ldk, 0, Lk);
+    T::fetch(rv, vb, ldv, 0, Lk);
+    T::store(lds[0][0], rk);
+    T::store(lds[0][1], rv);
+    if (ATILE < bend) {
+      T::fetch(rk, kb, ldk, ATILE, Lk);
+      T::fetch(rv, vb, ldv, ATILE, Lk);
     }
   }
   __syncthreads();
 
-  // dK/dV accumulators: wave owns d-slice [wid*D/4, wid*D/4 + D/4);
-  // rows = 4 key sub-tiles of 16; survive the g-loop (GQA row sum).
-  f32x4_t dv_acc[4][NDT], dk_acc[4][NDT];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int nt = 0; nt < NDT; ++nt) {
-      dv_acc[a][nt] = {0.f, 0.f, 0.f, 0.f};
-      dk_acc[a][nt] = {0.f, 0.f, 0.f, 0.f};
+  int buf = 0;
+  for (int t0 = 0; t0 < bend; t0 += ATILE, buf ^= 1) {
+    if (t0 + ATILE < bend) {
+      T::store(lds[buf ^ 1][0], rk);
+      T::store(lds[buf ^ 1][1], rv);
+      if (t0 + 2 * ATILE < bend) {
+        T::fetch(rk, kb, ldk, t0 + 2 * ATILE, Lk);
+        T::fetch(rv, vb, ldv, t0 + 2 * ATILE, Lk);
+      }
     }
-
-  // causal: first q row that can see key t0
-  int q_start = causal ? ((t0 - qk_off) > 0 ? (t0 - qk_off) : 0) : 0;
-  q_start -= q_start % QB3;
-
-  for (int g = 0; g < G; ++g) {
-    const int hq = hk * G + g;
-    for (int qb = q_start; qb < Lq; qb += QB3) {
-      __syncthreads();   // prior iteration's Pt/DSt/QsT/DOsT reads done
-      // ---- wave w loads its 16 q rows' A-frags; stages transposed ------
-      const int qrow_l = qb + wid * 16 + l15;
-      const bool live = qrow_l < Lq;
-      const long gq = (long)(qbeg + (live ? qrow_l : 0));
-      bf16x8_t qa[KS], da[KS];
+    const char* ks_ = lds[buf][0];
+    const char* vs_ = lds[buf][1];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {                  // 32 keys at a time
+      const int k0 = t0 + n * 32;
+      if (k0 >= wend) continue;
+      f32x16_t s, dp;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f, dp[r] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        if (live) {
-          qa[ks] = *reinterpret_cast<const bf16x8_t*>(
-              q + gq * ldq + (long)hq * D + ks * 32 + lhi * 8);
-          da[ks] = *reinterpret_cast<const bf16x8_t*>(
-              dout + (gq * Hq + hq) * D + ks * 32 + lhi * 8);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            qa[ks][j] = (__bf16)0.f;
-            da[ks][j] = (__bf16)0.f;
-          }
-        }
-        const int qcol = wid * 16 + l15;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int d = ks * 32 + lhi * 8 + j;
-          QsT[trid3(d, qcol, QB3)] = (bf16_t)qa[ks][j];
-          DOsT[trid3(d, qcol, QB3)] = (bf16_t)da[ks][j];
-        }
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            frag_rows<D>(ks_, at, n, ks), qf[ks], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            frag_rows<D>(vs_, at, n, ks), df[ks], dp, 0, 0, 0);
       }
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[r] = exp2_hw(__builtin_fmaf(s[r], s2, -lse2));
+      if (k0 + 32 > Lk || (causal && k0 + 31 > qk_off + wq0)) {
+        const int last = min(qpos, Lk - 1) - k0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (acc_row(r) > last) s[r] = 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] *= dp[r] - del;
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const bf16x8_t ds = acc_operand(s, st);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(ks_, at, dt, n * 2 + st), ds, acc[dt], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
 
-      // ---- S = Q K^T, dP = dO V^T  (wave's 16 q rows x 64 keys) --------
-      f32x4_t sc[4], dpc[4];
+  // ---- dQ = scale * acc, turned through LDS to whole rows -------------------
+  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        sc[nt] = {0.f, 0.f, 0.f, 0.f};
-        dpc[nt] = {0.f, 0.f, 0.f, 0.f};
-      }
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int krow = nt * 16 + l15;
+    for (int i = 0; i < 4; ++i) {
+      bf16x4 w;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t kb = *reinterpret_cast<const bf16x8_t*>(
-              reinterpret_cast<char*>(KsSwz) +
-              kswz3<D>(krow, (ks * 32 + lhi * 8) * 2));
-          const bf16x8_t vb = *reinterpret_cast<const bf16x8_t*>(
-              reinterpret_cast<char*>(VsSwz) +
-              kswz3<D>(krow, (ks * 32 + lhi * 8) * 2));
-          sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              qa[ks], kb, sc[nt], 0, 0, 0);
-          dpc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              da[ks], vb, dpc[nt], 0, 0, 0);
-        }
-      }
+      for (int t = 0; t < 4; ++t) w.v[t] = f2bf(acc[dt][4 * i + t] * scale);
+      const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
+      *reinterpret_cast<bf16x4*>(
+          mine + (lane & 31) * (2 * D) +
+          (((d >> 3) ^ T::swz(lane & 31)) << 4) + (d & 4) * 2) = w;
+    }
+  __syncthreads();
+  if (!busy) return;
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    const int at16 = lane + i * 64;
+    const int r = at16 / T::GR, g = at16 % T::GR;
+    if (wq0 + r < Lq)
+      *reinterpret_cast<bf16x8*>(
+          dq + (((long)qbeg + wq0 + r) * Hq + hq) * D + g * 8) =
+          *reinterpret_cast<const bf16x8*>(mine + r * (2 * D) +
+                                           ((g ^ T::swz(r)) << 4));
+  }
+}
 
-      // ---- P, dS -> transposed LDS (interior tiles skip the mask:
-      // VALU-bound kernels, PMC 6:1 VALU:MFMA) -----------------------
-      const bool interior =
-          (t0 + KB3 <= Lk) && (qb + wid * 16 + 16 <= Lq) &&
-          (!causal || t0 + KB3 - 1 <= qk_off + qb + wid * 16);
+// ---------------------------------------------------------------- dK/dV
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
+    bf16_t* __restrict__ dk,         // (total_k, Hk, D); nsplit == 1
+    bf16_t* __restrict__ dv,
+    float* __restrict__ part,        // (nsplit, 2, total_k, Hk, D), else
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
+    const bf16_t* __restrict__ v, const bf16_t* __restrict__ dout,
+    const float* __restrict__ lse, const float* __restrict__ delta,
+    const int* __restrict__ cu_q, const int* __restrict__ cu_k,
+    const int* __restrict__ tile_seq, const int* __restrict__ tile_k0,
+    int ntiles, int nsplit, long total_k, int Hq, int Hk, float scale,
+    int causal, long ldq, long ldk, long ldv) {
+  typedef AttnTile<D> T;
+  constexpr bool V_LDS = D == 128;   // V does not fit beside the gradients
+  // Q (two buffers), dO, V; at the end the exchange of 4 x 32 x D floats
+  __shared__ __attribute__((aligned(16))) char lds[4][T::BYTES];
+  __shared__ __attribute__((aligned(16))) float row_s[2][ATILE];  // lse, delta
+
+  const int G = Hq / Hk;
+  const int item = die_item(ntiles * Hk * nsplit);
+  if (item >= ntiles * Hk * nsplit) return;
+  const int hk = item / (ntiles * nsplit);
+  const int tile = item / nsplit % ntiles;         // early keys: most rows
+  const int split = item % nsplit;
+  const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
+  const int seq = tile_seq[tile], t0 = tile_k0[tile];
+  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
+  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
+  const int qk_off = Lk - Lq;
+  if (t0 >= Lk) return;
+
+  const int lane = threadIdx.x & 63;
+  const int wid = threadIdx.x >> 6;
+  const int kh = wid & 1, qh = wid >> 1;           // key half, row half
+  constexpr int KS = D / 16, DT = D / 32;
+  const int wk0 = t0 + kh * 32;                    // this wave's first key
+  const int key = wk0 + (lane & 31);               // this lane's key
+  const int krow = kbeg + min(key, Lk - 1);
+
+  bf16x8_t kf[KS], vf[V_LDS ? 1 : KS];
+  frag_global<D>(kf, k + (long)krow * ldk + (long)hk * D);
+  if constexpr (!V_LDS)
+    frag_global<D>(vf, v + (long)krow * ldv + (long)hk * D);
+  const float s2 = scale * 1.4426950408889634f;
+
+  const FragAt<D> at;
+  f32x16_t ak[DT], av[DT];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qrow_c = qb + wid * 16 + lhi * 4 + r;   // C-layout row
-        const bool qdead = qrow_c >= Lq;
-        const long gqc = (long)(qbeg + (qdead ? 0 : qrow_c)) * Hq + hq;
-        const float lse_r = qdead ? 0.f : lse[gqc];
-        const float del_r = qdead ? 0.f : delta[gqc];
-        const int qpos = qk_off + qrow_c;
-        const int qcol = wid * 16 + lhi * 4 + r;
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-          const int key = nt * 16 + l15;
-          float p;
-          if (interior) {
-            p = __expf(sc[nt][r] * scale - lse_r);
-          } else {
-            const int kpos = t0 + key;
-            const bool dead = qdead || (kpos >= Lk) ||
-                              (causal && kpos > qpos);
-            p = dead ? 0.f : __expf(sc[nt][r] * scale - lse_r);
-          }
-          const float ds = p * (dpc[nt][r] - del_r) * scale;
-          Pt[trid3(key, qcol, QB3)] = f2bf(p);
-          DSt[trid3(key, qcol, QB3)] = f2bf(ds);
+    for (int r = 0; r < 16; ++r) ak[dt][r] = 0.f, av[dt][r] = 0.f;
+
+  // query tiles that see key t0, one head after the other
+  const int qs = causal ? max(t0 - qk_off, 0) / ATILE * ATILE : 0;
+  const int nq = qs < Lq ? (Lq - qs + ATILE - 1) / ATILE : 0;
+  const int steps = (g1 - g0) * nq;
+  const bf16_t* qb0 = q + (long)qbeg * ldq + (long)hk * G * D;
+  const bf16_t* db0 = dout + ((long)qbeg * Hq + (long)hk * G) * D;
+
+  i32x4_t reg[T::LOADS];
+  float rowv = 0.f;                                // lse or delta of a row
+  auto fetch_rows = [&](int st) {                  // threads 0 .. 127
+    if (threadIdx.x < 2 * ATILE) {
+      const int r = qs + st % nq * ATILE + (threadIdx.x & (ATILE - 1));
+      const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + g0 + st / nq;
+      // rows past the end weigh nothing: 2^(s - inf) = 0
+      rowv = threadIdx.x < ATILE
+          ? (r < Lq ? lse[i] * 1.4426950408889634f : INFINITY)
+          : (r < Lq ? delta[i] : 0.f);
+    }
+  };
+  auto store_rows = [&]() {
+    if (threadIdx.x < 2 * ATILE) (&row_s[0][0])[threadIdx.x] = rowv;
+  };
+  auto fetch_q = [&](int st) {
+    T::fetch(reg, qb0 + (long)(g0 + st / nq) * D, ldq, qs + st % nq * ATILE,
+             Lq);
+  };
+  auto fetch_do = [&](int st) {
+    T::fetch(reg, db0 + (long)(g0 + st / nq) * D, (long)Hq * D,
+             qs + st % nq * ATILE, Lq);
+  };
+  if (steps > 0) {
+    if constexpr (V_LDS) {
+      T::fetch(reg, v + (long)kbeg * ldv + (long)hk * D, ldv, t0, Lk);
+      T::store(lds[3], reg);
+    }
+    fetch_rows(0);
+    fetch_q(0);
+    T::store(lds[0], reg);
+    fetch_do(0);
+    T::store(lds[2], reg);
+    store_rows();
+  }
+  __syncthreads();
+
+  for (int st = 0; st < steps; ++st) {
+    const int buf = st & 1;
+    const bool more = st + 1 < steps;
+    const int wq0 = qs + st % nq * ATILE + qh * 32;   // this wave's rows
+    const bool work = wq0 < Lq && wk0 < Lk &&
+                      (!causal || qk_off + wq0 + 31 >= wk0);
+    const char* qs_ = lds[buf];
+    const char* ds_ = lds[2];
+    if (more) {
+      fetch_rows(st + 1);
+      fetch_q(st + 1);
+    }
+    f32x16_t s, dp;
+    if (work) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f, dp[r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            frag_rows<D>(qs_, at, qh, ks), kf[ks], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            frag_rows<D>(ds_, at, qh, ks),
+            V_LDS ? frag_rows<D>(lds[3], at, kh, ks) : vf[V_LDS ? 0 : ks], dp,
+            0, 0, 0);
+      }
+      const bool edge = causal && qk_off + wq0 < wk0 + 31;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r0 = qh * 32 + 8 * i + 4 * (lane >> 5);
+        const float4 le = *reinterpret_cast<const float4*>(&row_s[0][r0]);
+        const float4 de = *reinterpret_cast<const float4*>(&row_s[1][r0]);
+        const float l4[4] = {le.x, le.y, le.z, le.w};
+        const float d4[4] = {de.x, de.y, de.z, de.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int r = 4 * i + t;
+          float p = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
+          if (edge && qk_off + wq0 + acc_row(r) < key) p = 0.f;
+          s[r] = p;
+          dp[r] = p * (dp[r] - d4[t]);
         }
       }
+    }
+    if (more) {
+      T::store(lds[buf ^ 1], reg);
+      fetch_do(st + 1);
+    }
+    if (work) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8_t p = acc_operand(s, h), ds = acc_operand(dp, h);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          av[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(ds_, at, dt, qh * 2 + h), p, av[dt], 0, 0, 0);
+          ak[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(qs_, at, dt, qh * 2 + h), ds, ak[dt], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();                   // every wave is done with the dO tile
+    if (more) {
+      T::store(lds[2], reg);
+      store_rows();
       __syncthreads();
-
-      // ---- dV += P^T dO ; dK += dS^T Q  (wave owns d-slice wid*D/4) ----
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {          // key sub-tile (rows)
-        const int keyrow = a * 16 + l15;
-#pragma unroll
-        for (int kq = 0; kq < 2; ++kq) {     // k = q rows, 2 x 32
-          const bf16x8_t pa = *reinterpret_cast<const bf16x8_t*>(
-              Pt + trid3_vec(keyrow, kq * 4 + lhi, QB3));
-          const bf16x8_t dsa = *reinterpret_cast<const bf16x8_t*>(
-              DSt + trid3_vec(keyrow, kq * 4 + lhi, QB3));
-#pragma unroll
-          for (int nt = 0; nt < NDT; ++nt) {
-            const int d = wid * (D / 4) + nt * 16 + l15;
-            const bf16x8_t dob = *reinterpret_cast<const bf16x8_t*>(
-                DOsT + trid3_vec(d, kq * 4 + lhi, QB3));
-            const bf16x8_t qb_ = *reinterpret_cast<const bf16x8_t*>(
-                QsT + trid3_vec(d, kq * 4 + lhi, QB3));
-            dv_acc[a][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                pa, dob, dv_acc[a][nt], 0, 0, 0);
-            dk_acc[a][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                dsa, qb_, dk_acc[a][nt], 0, 0, 0);
-          }
-        }
-      }
     }
   }
 
-  // ---- store dK/dV (exclusive ownership: plain stores, no zero-init) ----
+  // ---- the two waves of a key half: one completes dV, the other dK ----------
+  float* mine = reinterpret_cast<float*>(&lds[0][0]) + wid * (D * 32);
+  const float* other =
+      reinterpret_cast<const float*>(&lds[0][0]) + (wid ^ 2) * (D * 32);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int krow_l = t0 + a * 16 + lhi * 4 + r;
-      if (krow_l >= Lk) continue;
-      float* dkp = dk + ((long)(kbeg + krow_l) * Hk + hk) * D;
-      float* dvp = dv + ((long)(kbeg + krow_l) * Hk + hk) * D;
+    for (int r = 0; r < 16; ++r)
+      mine[(dt * 16 + r) * 64 + lane] = qh == 0 ? ak[dt][r] : av[dt][r];
+  __syncthreads();
+  const bool ok = key < Lk;
+  const long o = ((long)krow * Hk + hk) * D;
+  const float f = qh == 0 ? 1.f : scale;           // dK carries the scale
 #pragma unroll
-      for (int nt = 0; nt < NDT; ++nt) {
-        dkp[wid * (D / 4) + nt * 16 + l15] = dk_acc[a][nt][r];
-        dvp[wid * (D / 4) + nt * 16 + l15] = dv_acc[a][nt][r];
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f32x4v w;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 4 * i + t;
+        w.v[t] = f * ((qh == 0 ? av[dt][r] : ak[dt][r]) +
+                      other[(dt * 16 + r) * 64 + lane]);
+      }
+      const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
+      if (!ok) continue;
+      if (part != nullptr) {
+        *reinterpret_cast<f32x4v*>(
+            part + (split * 2 + (qh == 0 ? 1 : 0)) * (total_k * Hk * D) + o +
+            d) = w;
+      } else {
+        bf16x4 b;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) b.v[t] = f2bf(w.v[t]);
+        *reinterpret_cast<bf16x4*>((qh == 0 ? dv : dk) + o + d) = b;
       }
     }
 }
 
-// ------------------------------------------------------------------- dQ
-template <int D>
-__global__ __launch_bounds__(256) void attn_bwd_dq_kernel(
-    float* __restrict__ dq,          // (total_q, Hq, D) fp32 (fully written)
-    const bf16_t* __restrict__ q,
-    const bf16_t* __restrict__ k,
-    const bf16_t* __restrict__ v,
-    const bf16_t* __restrict__ dout,
-    const float* __restrict__ lse,
-    const float* __restrict__ delta,
-    const int* __restrict__ cu_q, const int* __restrict__ cu_k,
-    const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
-    int Hq, int Hk, float scale, int causal,
-    long ldq, long ldk, long ldv) {
-  __shared__ bf16_t KsSwz[KB3 * D];          // B-frags of S
-  __shared__ bf16_t VsSwz[KB3 * D];          // B-frags of dP
-  __shared__ bf16_t KsRowT[D * KB3];         // [d][key] for dQ += dS K
-  __shared__ bf16_t DSq[QB3 * KB3];          // [q][key] (wave-private rows)
-
-  const int tile = blockIdx.x;
-  const int hq = blockIdx.y;
-  const int G = Hq / Hk;
-  const int hk = hq / G;
-  const int seq = tile_seq[tile];
-  const int qt0 = tile_q0[tile];             // local first q row of tile
-  const int qbeg = cu_q[seq], qend = cu_q[seq + 1];
-  const int kbeg = cu_k[seq], kend = cu_k[seq + 1];
-  const int Lq = qend - qbeg, Lk = kend - kbeg;
-  const int qk_off = Lk - Lq;
-
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int l15 = lane & 15;
-  const int lhi = lane >> 4;
-  constexpr int KS = D / 32;
-  constexpr int NDQ = D / 16;                // 16-wide d-tiles of dQ
-
-  // ---- wave's 16 q rows: A-frags of Q / dO, lse/delta ------------------
-  const int qrow_l = qt0 + wid * 16 + l15;
-  const bool live = qrow_l < Lq;
-  const long gq = (long)(qbeg + (live ? qrow_l : 0));
-  bf16x8_t qa[KS], da[KS];
+// dK, dV = sums over the head shares
+__global__ void attn_bwd_sum_kernel(bf16_t* __restrict__ dk,
+                                    bf16_t* __restrict__ dv,
+                                    const float* __restrict__ part,
+                                    int nsplit, long n /* of one gradient */) {
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= n) return;
+  bf16_t* const to[2] = {dk, dv};
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    if (live) {
-      qa[ks] = *reinterpret_cast<const bf16x8_t*>(
-          q + gq * ldq + (long)hq * D + ks * 32 + lhi * 8);
-      da[ks] = *reinterpret_cast<const bf16x8_t*>(
-          dout + (gq * Hq + hq) * D + ks * 32 + lhi * 8);
-    } else {
+  for (int w = 0; w < 2; ++w) {
+    f32x4v a = *reinterpret_cast<const f32x4v*>(part + w * n + i);
+    for (int s = 1; s < nsplit; ++s) {
+      const f32x4v b =
+          *reinterpret_cast<const f32x4v*>(part + (2 * s + w) * n + i);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        qa[ks][j] = (__bf16)0.f;
-        da[ks][j] = (__bf16)0.f;
-      }
+      for (int t = 0; t < 4; ++t) a.v[t] += b.v[t];
     }
-  }
-
-  f32x4_t dq_acc[NDQ];
+    bf16x4 o;
 #pragma unroll
-  for (int nt = 0; nt < NDQ; ++nt) dq_acc[nt] = {0.f, 0.f, 0.f, 0.f};
-
-  // kv range: causal stops after the last key row qt0+63 can see
-  int kv_last = Lk;
-  if (causal) {
-    const int vis = qk_off + qt0 + QB3;      // exclusive
-    kv_last = vis < Lk ? vis : Lk;
-  }
-  if (kv_last < 0) kv_last = 0;
-
-  for (int t0 = 0; t0 < kv_last; t0 += KB3) {
-    __syncthreads();   // prior iteration's K/V reads done
-    // ---- cooperative stage of K/V (swizzled) + K^T --------------------
-    {
-      const int tid = threadIdx.x;
-#pragma unroll
-      for (int it = 0; it < KB3 * D / (256 * 8); ++it) {
-        const int flat = (tid + it * 256) * 8;
-        const int row = flat / D;
-        const int col = flat % D;
-        const int krow = t0 + row;
-        bf16x8 k8, v8;
-        if (krow < Lk) {
-          k8 = *reinterpret_cast<const bf16x8*>(
-              k + (long)(kbeg + krow) * ldk + (long)hk * D + col);
-          v8 = *reinterpret_cast<const bf16x8*>(
-              v + (long)(kbeg + krow) * ldv + (long)hk * D + col);
-        } else {
-          for (int j = 0; j < 8; ++j)
-            k8.v[j] = f2bf(0.f), v8.v[j] = f2bf(0.f);
-        }
-        *reinterpret_cast<bf16x8*>(
-            reinterpret_cast<char*>(KsSwz) + kswz3<D>(row, col * 2)) = k8;
-        *reinterpret_cast<bf16x8*>(
-            reinterpret_cast<char*>(VsSwz) + kswz3<D>(row, col * 2)) = v8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          KsRowT[trid3(col + j, row, KB3)] = k8.v[j];
-      }
-    }
-    __syncthreads();
-
-    // ---- S, dP over wave's 16 q rows x 64 keys -------------------------
-    f32x4_t sc[4], dpc[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      sc[nt] = {0.f, 0.f, 0.f, 0.f};
-      dpc[nt] = {0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int krow = nt * 16 + l15;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8_t kb = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<char*>(KsSwz) +
-            kswz3<D>(krow, (ks * 32 + lhi * 8) * 2));
-        const bf16x8_t vb = *reinterpret_cast<const bf16x8_t*>(
-            reinterpret_cast<char*>(VsSwz) +
-            kswz3<D>(krow, (ks * 32 + lhi * 8) * 2));
-        sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            qa[ks], kb, sc[nt], 0, 0, 0);
-        dpc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            da[ks], vb, dpc[nt], 0, 0, 0);
-      }
-    }
-
-    // ---- dS -> wave-private LDS rows (no barrier needed; interior
-    // tiles skip the mask — PMC 8.9:1 VALU:MFMA) ----------------------
-    const bool interior =
-        (t0 + KB3 <= Lk) && (qt0 + wid * 16 + 16 <= Lq) &&
-        (!causal || t0 + KB3 - 1 <= qk_off + qt0 + wid * 16);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qrow_c = qt0 + wid * 16 + lhi * 4 + r;
-      const bool qdead = qrow_c >= Lq;
-      const long gqc = (long)(qbeg + (qdead ? 0 : qrow_c)) * Hq + hq;
-      const float lse_r = qdead ? 0.f : lse[gqc];
-      const float del_r = qdead ? 0.f : delta[gqc];
-      const int qpos = qk_off + qrow_c;
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        float p;
-        if (interior) {
-          p = __expf(sc[nt][r] * scale - lse_r);
-        } else {
-          const int kpos = t0 + nt * 16 + l15;
-          const bool dead = qdead || (kpos >= Lk) ||
-                            (causal && kpos > qpos);
-          p = dead ? 0.f : __expf(sc[nt][r] * scale - lse_r);
-        }
-        const float ds = p * (dpc[nt][r] - del_r) * scale;
-        DSq[trid3(wid * 16 + lhi * 4 + r, nt * 16 + l15, KB3)] = f2bf(ds);
-      }
-    }
-
-    // ---- dQ += dS K  (A: DSq rows, B: KsRowT) --------------------------
-#pragma unroll
-    for (int kq = 0; kq < 2; ++kq) {         // k = keys, 2 x 32
-      const bf16x8_t dsa = *reinterpret_cast<const bf16x8_t*>(
-          DSq + trid3_vec(wid * 16 + l15, kq * 4 + lhi, KB3));
-#pragma unroll
-      for (int nt = 0; nt < NDQ; ++nt) {
-        const int d = nt * 16 + l15;
-        const bf16x8_t kb = *reinterpret_cast<const bf16x8_t*>(
-            KsRowT + trid3_vec(d, kq * 4 + lhi, KB3));
-        dq_acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            dsa, kb, dq_acc[nt], 0, 0, 0);
-      }
-    }
-  }
-
-  // ---- store dQ (exclusive ownership) -----------------------------------
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int qrow_c = qt0 + wid * 16 + lhi * 4 + r;
-    if (qrow_c >= Lq) continue;
-    float* dqp = dq + ((long)(qbeg + qrow_c) * Hq + hq) * D;
-#pragma unroll
-    for (int nt = 0; nt < NDQ; ++nt) dqp[nt * 16 + l15] = dq_acc[nt][r];
+    for (int t = 0; t < 4; ++t) o.v[t] = f2bf(a.v[t]);
+    *reinterpret_cast<bf16x4*>(to[w] + i) = o;
   }
 }
 
 // ---------------------------------------------------------------- launcher
+template <int D>
+static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
+                       torch::Tensor& dv, const torch::Tensor& q,
+                       const torch::Tensor& k, const torch::Tensor& v,
+                       const torch::Tensor& out, const torch::Tensor& dout,
+                       const torch::Tensor& lse, const torch::Tensor& cu_q,
+                       const torch::Tensor& cu_k, const torch::Tensor& t_seq,
+                       const torch::Tensor& t_q0, float scale, bool causal) {
+  const int Hq = q.size(1), Hk = k.size(1), G = Hq / Hk;
+  const long ntiles = t_seq.size(0), total_k = k.size(0);
+  auto stream = at::hip::getCurrentHIPStream();
+  auto blocks = [&](long items) {
+    const long b = (items + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
+    TORCH_CHECK(b < (1L << 31), "grid too large");
+    return dim3((unsigned)b);
+  };
+  auto delta = torch::empty_like(lse);
+  const int nparts = (2 * G + 3) / 4;
+  attn_bwd_dq_kernel<D>
+      <<<blocks(ntiles * Hk * nparts), dim3(256), 0, stream>>>(
+          (bf16_t*)dq.data_ptr(), delta.data_ptr<float>(),
+          (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
+          (const bf16_t*)v.data_ptr(), (const bf16_t*)out.data_ptr(),
+          (const bf16_t*)dout.data_ptr(), lse.data_ptr<float>(),
+          cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), t_seq.data_ptr<int>(),
+          t_q0.data_ptr<int>(), (int)ntiles, nparts, Hq, Hk, scale,
+          causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
+  // Blocks of the dkv kernel are as long as their key is early, so the chip
+  // needs several per slot (512: two per CU) to end together; with fewer than
+  // 768 a block takes fewer heads of the group.  The shares' trip through
+  // fp32 costs as much whatever the length, so long sequences are cut finer.
+  // Measured, forward and backward: 2 sequences of 4096, 28/4 heads (476
+  // blocks) 2166 us whole, 1644 with two heads a block, 1578 with one; 16 of
+  // up to 512, 32/8 heads (896 blocks) 349 us whole, 376 with two heads.
+  const long base = ntiles * Hk, nseq = cu_q.size(0) - 1;
+  int nsplit = 1;
+  if (base < 768) {
+    const long target = ntiles >= 16 * nseq ? 4096 : 1536;
+    const int per = (int)std::max<long>(1, G * base / target);
+    nsplit = (G + per - 1) / per;
+  }
+  torch::Tensor part;
+  if (nsplit > 1)
+    part = torch::empty({nsplit, 2, total_k, (long)Hk, (long)D},
+                        lse.options());
+  attn_bwd_dkv_kernel<D><<<blocks(base * nsplit), dim3(256), 0, stream>>>(
+      (bf16_t*)dk.data_ptr(), (bf16_t*)dv.data_ptr(),
+      nsplit > 1 ? part.data_ptr<float>() : nullptr,
+      (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
+      (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
+      lse.data_ptr<float>(), delta.data_ptr<float>(), cu_q.data_ptr<int>(),
+      cu_k.data_ptr<int>(), t_seq.data_ptr<int>(), t_q0.data_ptr<int>(),
+      (int)ntiles, nsplit, total_k, Hq, Hk, scale, causal ? 1 : 0,
+      q.stride(0), k.stride(0), v.stride(0));
+  if (nsplit > 1) {
+    const long n = total_k * Hk * D;
+    attn_bwd_sum_kernel<<<dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0,
+                          stream>>>((bf16_t*)dk.data_ptr(),
+                                    (bf16_t*)dv.data_ptr(),
+                                    part.data_ptr<float>(), nsplit, n);
+  }
+  HIP_CHECK_KERNEL();
+}
+
+// t64_seq / t64_q0: the 64-row tiles of the packed rows (build_varlen_tiles);
+// query and key rows share them, so both sides are cut alike.
 void varlen_attention_backward_v3(
-    torch::Tensor dq, torch::Tensor dk, torch::Tensor dv,  // fp32 (empty ok)
+    torch::Tensor dq, torch::Tensor dk, torch::Tensor dv,  // bf16 (empty ok)
     torch::Tensor q, torch::Tensor k, torch::Tensor v,
     torch::Tensor out, torch::Tensor dout, torch::Tensor lse,
     torch::Tensor cu_seqlens_q, torch::Tensor cu_seqlens_k,
@@ -485,58 +505,16 @@ void varlen_attention_backward_v3(
   };
   TORCH_CHECK(packed(q) && packed(k) && packed(v));
   TORCH_CHECK(out.is_contiguous() && dout.is_contiguous());
+  TORCH_CHECK(out.dtype() == torch::kBFloat16 &&
+              dout.dtype() == torch::kBFloat16);
   TORCH_CHECK(lse.is_contiguous() && lse.dtype() == torch::kFloat32);
-  TORCH_CHECK(dq.dtype() == torch::kFloat32 && dq.is_contiguous());
+  for (const auto* g : {&dq, &dk, &dv})
+    TORCH_CHECK(g->dtype() == torch::kBFloat16 && g->is_contiguous());
   const int Hq = q.size(1), D = q.size(2), Hk = k.size(1);
   TORCH_CHECK(D == 128 || D == 64, "backward v3 supports head_dim 64/128");
   TORCH_CHECK(Hq % Hk == 0);
-  const long tq = q.size(0);
-  auto stream = at::hip::getCurrentHIPStream();
-
-  auto delta = torch::empty({tq, (long)Hq}, lse.options());
-  const long rows = tq * Hq;
-  const int ntiles = t64_seq.size(0);
-  const dim3 blk(256);
-  if (D == 128) {
-    attn_bwd_delta_kernel3<128><<<dim3((rows + 3) / 4), blk, 0, stream>>>(
-        delta.data_ptr<float>(), (const bf16_t*)dout.data_ptr(),
-        (const bf16_t*)out.data_ptr(), rows);
-    attn_bwd_dkv_kernel<128><<<dim3(ntiles, Hk), blk, 0, stream>>>(
-        dk.data_ptr<float>(), dv.data_ptr<float>(),
-        (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
-        (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
-        lse.data_ptr<float>(), delta.data_ptr<float>(),
-        cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
-        t64_seq.data_ptr<int>(), t64_q0.data_ptr<int>(), Hq, Hk,
-        (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
-    attn_bwd_dq_kernel<128><<<dim3(ntiles, Hq), blk, 0, stream>>>(
-        dq.data_ptr<float>(),
-        (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
-        (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
-        lse.data_ptr<float>(), delta.data_ptr<float>(),
-        cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
-        t64_seq.data_ptr<int>(), t64_q0.data_ptr<int>(), Hq, Hk,
-        (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
-  } else {
-    attn_bwd_delta_kernel3<64><<<dim3((rows + 3) / 4), blk, 0, stream>>>(
-        delta.data_ptr<float>(), (const bf16_t*)dout.data_ptr(),
-        (const bf16_t*)out.data_ptr(), rows);
-    attn_bwd_dkv_kernel<64><<<dim3(ntiles, Hk), blk, 0, stream>>>(
-        dk.data_ptr<float>(), dv.data_ptr<float>(),
-        (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
-        (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
-        lse.data_ptr<float>(), delta.data_ptr<float>(),
-        cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
-        t64_seq.data_ptr<int>(), t64_q0.data_ptr<int>(), Hq, Hk,
-        (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
-    attn_bwd_dq_kernel<64><<<dim3(ntiles, Hq), blk, 0, stream>>>(
-        dq.data_ptr<float>(),
-        (const bf16_t*)q.data_ptr(), (const bf16_t*)k.data_ptr(),
-        (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
-        lse.data_ptr<float>(), delta.data_ptr<float>(),
-        cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
-        t64_seq.data_ptr<int>(), t64_q0.data_ptr<int>(), Hq, Hk,
-        (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
-  }
-  HIP_CHECK_KERNEL();
+  if (t64_seq.size(0) == 0) return;
+  (D == 128 ? launch_bwd<128> : launch_bwd<64>)(
+      dq, dk, dv, q, k, v, out, dout, lse, cu_seqlens_q, cu_seqlens_k,
+      t64_seq, t64_q0, (float)scale, causal);
 }

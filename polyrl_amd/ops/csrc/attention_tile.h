@@ -46,11 +46,13 @@ struct AttnTile {
   // ``rows`` on repeat the last one (what they give is masked or dropped)
   DEV_INLINE static void fetch(i32x4_t (&reg)[LOADS], const bf16_t* base,
                                long ld, int r0, int rows) {
+    const bf16_t* from = base + r0 * ld;           // the same for the block
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int at = threadIdx.x + i * 256;
-      const int r = min(r0 + at / GR, rows - 1);
-      reg[i] = *reinterpret_cast<const i32x4_t*>(base + r * ld + at % GR * 8);
+      const int r = min(at / GR, rows - 1 - r0);
+      reg[i] = *reinterpret_cast<const i32x4_t*>(
+          from + (unsigned)(r * (int)ld + at % GR * 8));
     }
   }
 

@@ -77,3 +77,55 @@ def test_forward(name, hq, hk, d, hist, causal, table):
         assert ((out[a].double() - want).abs() <= bound).all(), (name, n)
         # 32-bit scores (|s| < 64) and sums
         assert (lse[a].double() - wl).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("name,hq,hk,d", [
+    ("edges", 8, 2, 128), ("edges", 7, 1, 64), ("one", 3, 3, 128),
+    ("ragged", 12, 2, 128), ("ragged", 4, 4, 64), ("many", 8, 1, 64),
+    ("ragged", 10, 2, 64)])
+def test_backward(name, hq, hk, d, causal):
+    """Gradients of every sequence against float64 autograd.  With P and dS
+    rounded once to bf16, sums in 32 bits and the result rounded once, an
+    entry is off by at most 2^-8 of the sum of its terms' magnitudes, plus
+    what the bf16 output in delta = rowsum(dO * O) adds."""
+    torch.manual_seed(6)
+    lens, scale = LENS[name], d ** -0.5
+    cu = cu_of(lens)
+    n = sum(lens)
+    q, k, v = (torch.randn(n, h, d, device=DEV).bfloat16().requires_grad_()
+               for h in (hq, hk, hk))
+    dout = torch.randn(n, hq, d, device=DEV).bfloat16()
+    out = ops.flash_attn_varlen(q, k, v, cu.to(DEV), scale, causal)
+    got = torch.autograd.grad(out, (q, k, v), dout)
+    again = torch.autograd.grad(
+        ops.flash_attn_varlen(q, k, v, cu.to(DEV), scale, causal), (q, k, v),
+        dout)
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)            # no atomics: the same bits
+    for i in range(len(lens)):
+        a = slice(cu[i], cu[i + 1])
+        x = [t.detach()[a].double() for t in (q, k, v)]
+        kk, vv, do = heads(x[1], hq), heads(x[2], hq), dout[a].double()
+        s = torch.einsum("qhd,khd->hqk", x[0], kk) * scale
+        if causal:
+            r = torch.arange(lens[i], device=DEV)
+            s = s.masked_fill(r[None] > r[:, None], -float("inf"))
+        p = torch.softmax(s, -1)
+        dp = torch.einsum("qhd,khd->hqk", do, vv)
+        o = torch.einsum("hqk,khd->qhd", p, vv)
+        delta = (do * o).sum(-1).t()[..., None]
+        ds = p * (dp - delta)
+        # the magnitudes: |dS| plus the share of delta that rounding O moves
+        big = p * ((dp - delta).abs()
+                   + (do * o).abs().sum(-1).t()[..., None])
+        group = lambda t: t.unflatten(1, (hk, hq // hk)).sum(2)
+        pair = lambda w, t: torch.einsum("hqk,qhd->khd", w, t)
+        want = (torch.einsum("hqk,khd->qhd", ds, kk) * scale,
+                group(pair(ds, x[0])) * scale, group(pair(p, do)))
+        size = (torch.einsum("hqk,khd->qhd", big, kk.abs()) * scale,
+                group(pair(big, x[0].abs())) * scale,
+                group(pair(p, do.abs())))
+        for name_, g, w, m in zip(("dq", "dk", "dv"), got, want, size):
+            off = (g[a].double() - w).abs() - 2 ** -8 * (m + w.abs())
+            assert off.max() <= 0, (name_, lens[i], off.max())
