@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int qk_off = Lk - Lq;
 
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
+  const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
   const int unit = item % nparts * 4 + wid;        // (row half, head)
   const int wq0 = q0 + unit / G * 32;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const float s2 = scale * 1.4426950408889634f;
   const float lse2 = lse[tok * Hq + hq] * 1.4426950408889634f;
 
-  const FragAt<D> at;
+  FragAt<D> at;
   f32x16_t acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -107,34 +107,33 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 
   const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
   const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
-  i32x4_t rk[T::LOADS], rv[T::LOADS];
+  // one set of registers: the next K tile is in flight during a tile's first
+  // 32 keys, the next V tile during the others
+  i32x4_t reg[T::LOADS];
   if (bend > 0) {
-    T::fetch(rk, kb, ldk, 0, Lk);
-    T::fetch(rv, vb, ldv, 0, Lk);
-    T::store(lds[0][0], rk);
-    T::store(lds[0][1], rv);
-    if (ATILE < bend) {
-      T::fetch(rk, kb, ldk, ATILE, Lk);
-      T::fetch(rv, vb, ldv, ATILE, Lk);
-    }
+    T::fetch(reg, kb, ldk, 0, Lk);
+    T::store(lds[0][0], reg);
+    T::fetch(reg, vb, ldv, 0, Lk);
+    T::store(lds[0][1], reg);
   }
+  wait_loads();
   __syncthreads();
 
   int buf = 0;
   for (int t0 = 0; t0 < bend; t0 += ATILE, buf ^= 1) {
-    if (t0 + ATILE < bend) {
-      T::store(lds[buf ^ 1][0], rk);
-      T::store(lds[buf ^ 1][1], rv);
-      if (t0 + 2 * ATILE < bend) {
-        T::fetch(rk, kb, ldk, t0 + 2 * ATILE, Lk);
-        T::fetch(rv, vb, ldv, t0 + 2 * ATILE, Lk);
-      }
-    }
+    const bool more = t0 + ATILE < bend;
+    if (more) T::fetch(reg, kb, ldk, t0 + ATILE, Lk);
     const char* ks_ = lds[buf][0];
     const char* vs_ = lds[buf][1];
+    at.renew();
 #pragma unroll
     for (int n = 0; n < 2; ++n) {                  // 32 keys at a time
       const int k0 = t0 + n * 32;
+      // the other buffer's readers passed the last barrier
+      if (n == 1 && more) {
+        T::store(lds[buf ^ 1][0], reg);
+        T::fetch(reg, vb, ldv, t0 + ATILE, Lk);
+      }
       if (k0 >= wend) continue;
       f32x16_t s, dp;
 #pragma unroll
@@ -146,6 +145,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             frag_rows<D>(vs_, at, n, ks), df[ks], dp, 0, 0, 0);
       }
+      SCHED_LDS(6);
+#pragma unroll
+      for (int i = 0; i < 2 * KS - 6; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(1);
+      }
+      SCHED_MFMA(6);
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         s[r] = exp2_hw(__builtin_fmaf(s[r], s2, -lse2));
@@ -165,7 +171,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
           acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_cols<D>(ks_, at, dt, n * 2 + st), ds, acc[dt], 0, 0, 0);
       }
+      SCHED_LDS(8);
+#pragma unroll
+      for (int i = 0; i < 2 * DT - 4; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(2);
+      }
+      SCHED_MFMA(4);
     }
+    if (more) T::store(lds[buf ^ 1][1], reg);
     __syncthreads();
   }
 
@@ -230,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   if (t0 >= Lk) return;
 
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
+  const int wid = wave_id();
   const int kh = wid & 1, qh = wid >> 1;           // key half, row half
   constexpr int KS = D / 16, DT = D / 32;
   const int wk0 = t0 + kh * 32;                    // this wave's first key
@@ -243,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     frag_global<D>(vf, v + (long)krow * ldv + (long)hk * D);
   const float s2 = scale * 1.4426950408889634f;
 
-  const FragAt<D> at;
+  FragAt<D> at;
   f32x16_t ak[DT], av[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -259,18 +273,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 
   i32x4_t reg[T::LOADS];
   float rowv = 0.f;                                // lse or delta of a row
-  auto fetch_rows = [&](int st) {                  // threads 0 .. 127
-    if (threadIdx.x < 2 * ATILE) {
-      const int r = qs + st % nq * ATILE + (threadIdx.x & (ATILE - 1));
-      const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + g0 + st / nq;
-      // rows past the end weigh nothing: 2^(s - inf) = 0
-      rowv = threadIdx.x < ATILE
-          ? (r < Lq ? lse[i] * 1.4426950408889634f : INFINITY)
-          : (r < Lq ? delta[i] : 0.f);
-    }
+  bool rlive = false;
+  auto fetch_rows = [&](int st) {   // the first two waves' are stored
+    const int r = qs + st % nq * ATILE + lane;
+    const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + g0 + st / nq;
+    rlive = r < Lq;
+    rowv = (wid == 0 ? lse : delta)[i];
   };
   auto store_rows = [&]() {
-    if (threadIdx.x < 2 * ATILE) (&row_s[0][0])[threadIdx.x] = rowv;
+    // rows past the end weigh nothing: 2^(s - inf) = 0
+    if (wid == 0) row_s[0][lane] = rlive ? rowv * 1.4426950408889634f : INFINITY;
+    if (wid == 1) row_s[1][lane] = rlive ? rowv : 0.f;
   };
   auto fetch_q = [&](int st) {
     T::fetch(reg, qb0 + (long)(g0 + st / nq) * D, ldq, qs + st % nq * ATILE,
@@ -292,6 +305,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     T::store(lds[2], reg);
     store_rows();
   }
+  wait_loads();
   __syncthreads();
 
   for (int st = 0; st < steps; ++st) {
@@ -302,12 +316,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
                       (!causal || qk_off + wq0 + 31 >= wk0);
     const char* qs_ = lds[buf];
     const char* ds_ = lds[2];
+    at.renew();
     if (more) {
       fetch_rows(st + 1);
       fetch_q(st + 1);
     }
-    f32x16_t s, dp;
+    bf16x8_t p[2], ds[2];
     if (work) {
+      f32x16_t s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = 0.f, dp[r] = 0.f;
 #pragma unroll
@@ -319,6 +335,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
             V_LDS ? frag_rows<D>(lds[3], at, kh, ks) : vf[V_LDS ? 0 : ks], dp,
             0, 0, 0);
       }
+      constexpr int PER = V_LDS ? 3 : 2;           // fragments of a pair
+      SCHED_LDS(2 * PER);
+#pragma unroll
+      for (int i = 0; i < KS - 2; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(1);
+        SCHED_MFMA(1);
+        SCHED_LDS(PER - 1);
+      }
+      SCHED_MFMA(4);
       const bool edge = causal && qk_off + wq0 < wk0 + 31;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -330,11 +356,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * i + t;
-          float p = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
-          if (edge && qk_off + wq0 + acc_row(r) < key) p = 0.f;
-          s[r] = p;
-          dp[r] = p * (dp[r] - d4[t]);
+          float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
+          if (edge && qk_off + wq0 + acc_row(r) < key) w = 0.f;
+          s[r] = w;
+          dp[r] = w * (dp[r] - d4[t]);
         }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        p[h] = acc_operand(s, h);
+        ds[h] = acc_operand(dp, h);
       }
     }
     if (more) {
@@ -344,15 +375,21 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     if (work) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const bf16x8_t p = acc_operand(s, h), ds = acc_operand(dp, h);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           av[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              frag_cols<D>(ds_, at, dt, qh * 2 + h), p, av[dt], 0, 0, 0);
+              frag_cols<D>(ds_, at, dt, qh * 2 + h), p[h], av[dt], 0, 0, 0);
           ak[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              frag_cols<D>(qs_, at, dt, qh * 2 + h), ds, ak[dt], 0, 0, 0);
+              frag_cols<D>(qs_, at, dt, qh * 2 + h), ds[h], ak[dt], 0, 0, 0);
         }
       }
+      SCHED_LDS(6);
+#pragma unroll
+      for (int i = 0; i < 4 * DT - 3; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(2);
+      }
+      SCHED_MFMA(3);
     }
     __syncthreads();                   // every wave is done with the dO tile
     if (more) {

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
   const int qk_off = Lk - Lq;                      // chunked-prefill alignment
 
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
+  const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
   const int unit = item % nparts * 4 + wid;        // (row half, head)
   const int hq = hk * G + unit % G;
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
   frag_global<D>(qf, q + (long)(qbeg + min(busy ? row : 0, Lq - 1)) * ldq +
                          (long)hq * D * (busy ? 1 : 0));
 
-  const FragAt<D> at;
+  FragAt<D> at;
   const float s2 = scale * 1.4426950408889634f;    // scores in powers of two
   float m_run = -1e30f, l_run = 0.f;               // l: this lane's keys only
   f32x16_t o[DT];
@@ -100,10 +100,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     T::fetch(rv, vb, ldv, 0, Lk);
     T::store(lds[0][0], rk);
     T::store(lds[0][1], rv);
-    if (ATILE < bend) {
-      T::fetch(rk, kb, ldk, ATILE, Lk);
-      T::fetch(rv, vb, ldv, ATILE, Lk);
-    }
+  }
+  wait_loads();
+  if (ATILE < bend) {
+    T::fetch(rk, kb, ldk, ATILE, Lk);
+    T::fetch(rv, vb, ldv, ATILE, Lk);
   }
   __syncthreads();
 
@@ -121,17 +122,24 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     if (t0 < wend) {
       const char* ks_ = lds[buf][0];
       const char* vs_ = lds[buf][1];
+      at.renew();
       // ---- S^T: 64 keys x 32 rows ------------------------------------------
       f32x16_t s[2];
 #pragma unroll
-      for (int n = 0; n < 2; ++n) {
+      for (int r = 0; r < 16; ++r) s[0][r] = 0.f, s[1][r] = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+      for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+        for (int n = 0; n < 2; ++n)
           s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_rows<D>(ks_, at, n, ks), qf[ks], s[n], 0, 0, 0);
+      SCHED_LDS(6);
+#pragma unroll
+      for (int i = 0; i < 2 * KS - 6; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(1);
       }
+      SCHED_MFMA(6);
       // ---- mask (wave-uniform: some key of the tile is hidden) --------------
       if (t0 + ATILE > Lk || (causal && t0 + ATILE - 1 > qk_off + wq0)) {
         const int last = min(qpos, Lk - 1) - t0;
@@ -175,6 +183,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_cols<D>(vs_, at, dt, st), p, o[dt], 0, 0, 0);
       }
+      SCHED_LDS(8);
+#pragma unroll
+      for (int i = 0; i < 4 * DT - 4; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(2);
+      }
+      SCHED_MFMA(4);
     }
     __syncthreads();
   }

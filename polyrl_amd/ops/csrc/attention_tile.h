@@ -46,13 +46,15 @@ struct AttnTile {
   // ``rows`` on repeat the last one (what they give is masked or dropped)
   DEV_INLINE static void fetch(i32x4_t (&reg)[LOADS], const bf16_t* base,
                                long ld, int r0, int rows) {
-    const bf16_t* from = base + r0 * ld;           // the same for the block
+    // a block-uniform base and 32-bit offsets inside the tile
+    const char* from = reinterpret_cast<const char*>(base + r0 * ld);
+    const unsigned ldb = (unsigned)ld * 2;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int at = threadIdx.x + i * 256;
-      const int r = min(at / GR, rows - 1 - r0);
-      reg[i] = *reinterpret_cast<const i32x4_t*>(
-          from + (unsigned)(r * (int)ld + at % GR * 8));
+      const unsigned r = min(at / GR, rows - 1 - r0);
+      reg[i] = *reinterpret_cast<const i32x4_t*>(from + (r * ldb +
+                                                         at % GR * 16));
     }
   }
 
@@ -67,7 +69,9 @@ struct AttnTile {
   }
 };
 
-// Per-lane offsets of the two kinds of fragments.
+// Per-lane offsets of the two kinds of fragments.  renew() makes them new to
+// the compiler: called once per tile it keeps the sixteen and more derived
+// addresses from living in registers through the whole loop.
 template <int D>
 struct FragAt {
   int rows, cols0, cols1;
@@ -79,6 +83,9 @@ struct FragAt {
     const int g = ((lane >> 4) & 1) * 2 + ((c & 3) >> 1);
     cols0 = ra * (2 * D) + ((g ^ AttnTile<D>::swz(ra)) << 4) + (c & 1) * 8;
     cols1 = rb * (2 * D) + ((g ^ AttnTile<D>::swz(rb)) << 4) + (c & 1) * 8;
+  }
+  DEV_INLINE void renew() {
+    asm volatile("" : "+v"(rows), "+v"(cols0), "+v"(cols1));
   }
 };
 
@@ -143,6 +150,17 @@ DEV_INLINE float half_sum(float x) {
 // 2^x in one instruction; results below 2^-126 become 0
 DEV_INLINE float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Order of a stretch of straight-line code: ``n`` of the named kind next.  Left
+// to itself the compiler reads one fragment, waits for it and multiplies, so
+// that every product pays the LDS latency.
+#define SCHED_MFMA(n) __builtin_amdgcn_sched_group_barrier(0x008, n, 0)
+#define SCHED_LDS(n) __builtin_amdgcn_sched_group_barrier(0x100, n, 0)
+
+// all loads so far are there.  Before a loop with loads in flight: the wait
+// for a register that was loaded before the loop would otherwise stand inside
+// it and catch the loop's own loads.
+DEV_INLINE void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 // Sequence and first row of row tile ``tile``.  With a table it is looked
 // up; without one the tiles are the sequences' 64-row pieces in order, found
 // from cu_q by one scan (64 sequences a step), so that a caller that does
@@ -170,12 +188,17 @@ DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
     if (past) {
       const int l = __ffsll((long long)past) - 1;
       seq = s0 + l;
-      r0 = (tile - before - __shfl(upto - n, l, 64)) * ATILE;
+      r0 = (tile - __builtin_amdgcn_readlane(before + upto - n, l)) * ATILE;
       return true;
     }
-    before += __shfl(upto, 63, 64);
+    before += __builtin_amdgcn_readlane(upto, 63);
   }
   return false;
+}
+
+// wave of the block, known to the compiler to be the same for all its lanes
+DEV_INLINE int wave_id() {
+  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
 // Work item of a block.  Blocks go to the dies in turn (id % 8); each die
