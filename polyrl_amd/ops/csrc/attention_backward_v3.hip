@@ -32,8 +32,8 @@
 // fragment of 1 KiB per 32-cycle product).  Measured, forward and backward of
 // packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with kernels
 // that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
-// gradients for a cast to read, 349 us now; 2 of up to 4096, 28/4 heads,
-// 4000 -> 1580 us.
+// gradients for a cast to read, 267 us now (349 with every fragment read just
+// before its product); 2 of up to 4096, 28/4 heads, 4000 -> 1305 us.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   if (item >= ntiles * Hk * nparts) return;
   const int hk = item / (ntiles * nparts);
   const int tile = ntiles - 1 - item / nparts % ntiles;   // long rows first
-  const int seq = tile_seq[tile], q0 = tile_q0[tile];
+  const int seq = uniform(tile_seq[tile]), q0 = uniform(tile_q0[tile]);
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const int tile = item / nsplit % ntiles;         // early keys: most rows
   const int split = item % nsplit;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
-  const int seq = tile_seq[tile], t0 = tile_k0[tile];
+  const int seq = uniform(tile_seq[tile]), t0 = uniform(tile_k0[tile]);
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;
@@ -274,9 +274,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   i32x4_t reg[T::LOADS];
   float rowv = 0.f;                                // lse or delta of a row
   bool rlive = false;
-  auto fetch_rows = [&](int st) {   // the first two waves' are stored
-    const int r = qs + st % nq * ATILE + lane;
-    const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + g0 + st / nq;
+  int fg = g0, fq = qs;               // head and first row of the next fetch
+  auto fetch_rows = [&]() {           // the first two waves' are stored
+    const int r = fq + lane;
+    const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + fg;
     rlive = r < Lq;
     rowv = (wid == 0 ? lse : delta)[i];
   };
@@ -285,41 +286,41 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     if (wid == 0) row_s[0][lane] = rlive ? rowv * 1.4426950408889634f : INFINITY;
     if (wid == 1) row_s[1][lane] = rlive ? rowv : 0.f;
   };
-  auto fetch_q = [&](int st) {
-    T::fetch(reg, qb0 + (long)(g0 + st / nq) * D, ldq, qs + st % nq * ATILE,
-             Lq);
-  };
-  auto fetch_do = [&](int st) {
-    T::fetch(reg, db0 + (long)(g0 + st / nq) * D, (long)Hq * D,
-             qs + st % nq * ATILE, Lq);
+  auto fetch_q = [&]() { T::fetch(reg, qb0 + (long)fg * D, ldq, fq, Lq); };
+  auto fetch_do = [&]() {             // and on to the next tile
+    T::fetch(reg, db0 + (long)fg * D, (long)Hq * D, fq, Lq);
+    fq += ATILE;
+    if (fq >= Lq) fq = qs, ++fg;
   };
   if (steps > 0) {
     if constexpr (V_LDS) {
       T::fetch(reg, v + (long)kbeg * ldv + (long)hk * D, ldv, t0, Lk);
       T::store(lds[3], reg);
     }
-    fetch_rows(0);
-    fetch_q(0);
+    fetch_rows();
+    fetch_q();
     T::store(lds[0], reg);
-    fetch_do(0);
+    fetch_do();
     T::store(lds[2], reg);
     store_rows();
   }
   wait_loads();
   __syncthreads();
 
+  int q0 = qs;
   for (int st = 0; st < steps; ++st) {
     const int buf = st & 1;
     const bool more = st + 1 < steps;
-    const int wq0 = qs + st % nq * ATILE + qh * 32;   // this wave's rows
+    const int wq0 = q0 + qh * 32;                     // this wave's rows
+    q0 = q0 + ATILE < Lq ? q0 + ATILE : qs;
     const bool work = wq0 < Lq && wk0 < Lk &&
                       (!causal || qk_off + wq0 + 31 >= wk0);
     const char* qs_ = lds[buf];
     const char* ds_ = lds[2];
     at.renew();
     if (more) {
-      fetch_rows(st + 1);
-      fetch_q(st + 1);
+      fetch_rows();
+      fetch_q();
     }
     bf16x8_t p[2], ds[2];
     if (work) {
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     }
     if (more) {
       T::store(lds[buf ^ 1], reg);
-      fetch_do(st + 1);
+      fetch_do();
     }
     if (work) {
 #pragma unroll
@@ -495,7 +496,8 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
   // 768 a block takes fewer heads of the group.  The shares' trip through
   // fp32 costs as much whatever the length, so long sequences are cut finer.
   // Measured, forward and backward: 2 sequences of 4096, 28/4 heads (476
-  // blocks) 2166 us whole, 1644 with two heads a block, 1578 with one; 16 of
+  // blocks) 2166 us whole, 1644 with two heads a block, 1578 with one (before
+  // the fragments were read ahead); 16 of
   // up to 512, 32/8 heads (896 blocks) 349 us whole, 376 with two heads.
   const long base = ntiles * Hk, nseq = cu_q.size(0) - 1;
   int nsplit = 1;

@@ -161,6 +161,8 @@ DEV_INLINE float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 // it and catch the loop's own loads.
 DEV_INLINE void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+DEV_INLINE int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
 // Sequence and first row of row tile ``tile``.  With a table it is looked
 // up; without one the tiles are the sequences' 64-row pieces in order, found
 // from cu_q by one scan (64 sequences a step), so that a caller that does
@@ -169,8 +171,8 @@ DEV_INLINE void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
                           const int* cu, int nseq, int& seq, int& r0) {
   if (tile_seq != nullptr) {
-    seq = tile_seq[tile];
-    r0 = tile_r0[tile];
+    seq = uniform(tile_seq[tile]);
+    r0 = uniform(tile_r0[tile]);
     return true;
   }
   const int lane = threadIdx.x & 63;
@@ -187,7 +189,7 @@ DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
     const unsigned long long past = __ballot(before + upto > tile);
     if (past) {
       const int l = __ffsll((long long)past) - 1;
-      seq = s0 + l;
+      seq = uniform(s0 + l);
       r0 = (tile - __builtin_amdgcn_readlane(before + upto - n, l)) * ATILE;
       return true;
     }
@@ -198,7 +200,7 @@ DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
 
 // wave of the block, known to the compiler to be the same for all its lanes
 DEV_INLINE int wave_id() {
-  return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  return uniform(threadIdx.x >> 6);
 }
 
 // Work item of a block.  Blocks go to the dies in turn (id % 8); each die
