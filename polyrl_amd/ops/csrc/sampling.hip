@@ -1,23 +1,35 @@
 // Fused sampling: temperature + top-k + top-p filter + categorical draw +
-// sampled-token logprob capture, one workgroup per row.
+// sampled-token logprob capture.
 //
 // Reference capability: the engine-side sampling + per-token logprob kernels
-// (SURVEY.md §2.4.3).  Design (MI355X-first, no sort):
-//  * top-k threshold = k-th largest logit, found by LDS-histogram radix
-//    select over the monotone uint32 encoding of the logit (temperature
-//    doesn't change order, so select on raw logits).
-//  * top-p threshold found by the same radix walk, accumulating per-bin
+// (SURVEY.md §2.4.3).  Semantics:
+//  * top-k threshold = k-th largest logit, found by radix select over the
+//    monotone uint32 encoding of the logit (temperature doesn't change order,
+//    so select on raw logits).
+//  * top-p threshold found by the same walk, accumulating per-bin
 //    sum(exp(x/T - m/T)) mass instead of counts.
 //  * the draw is Gumbel-argmax over the kept set: argmax(x/T + G_i), exact
 //    categorical sampling in one streaming pass, counter-based RNG
 //    (splitmix64 keyed by (seed, row, i)) so replay is deterministic.
 //  * reported logprob is under the raw (unfiltered, T=1) softmax, matching
 //    what rollout clients consume as output_token_logprobs.
-// bf16 logits have 16 payload bits -> 2 radix rounds are exact; fp32 runs 4.
+//
+// Split.  A row is cut into ``split`` pieces, one block each, so that a few
+// rows fill the chip too (a block per row left half of it idle at 128 rows);
+// the pieces meet in small per-row arrays and a merging launch.  Without a
+// filter that is one pass: sums of the raw softmax and the draw together.
+// With one: sums, one pass per radix digit (11 bits, then the rest of a bf16
+// number's 16 or an fp32 number's 32), the draw over the kept set.
+//
+// What bounds it: integer multiplies of the generator (two 64-bit products a
+// number).  The two logarithms of a number's noise are only taken where its
+// 24 random bits can beat the wave's best so far: z > best means
+// u > exp(-exp(x/T - best)), one threshold per 16-byte word of logits from
+// the word's largest, with a margin far above the rounding of either side.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include "vocab_row.h"
 
 DEV_INLINE uint32_t enc_f32(float x) {
   uint32_t b = __float_as_uint(x);
@@ -31,281 +43,458 @@ DEV_INLINE uint64_t splitmix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// uniform in (0,1]
-DEV_INLINE float rng_uniform(uint64_t seed, uint64_t idx) {
-  uint64_t r = splitmix64(seed ^ (idx * 0xd1342543de82ef95ull + 0x2545f4914f6cdd1dull));
-  return ((r >> 40) + 1.0f) * (1.0f / 16777216.0f);  // 24-bit mantissa
+// 24 random bits of entry i0 + j (one product for the entries of a word)
+DEV_INLINE uint32_t rng_bits(uint64_t rowkey, int i0, int j) {
+  constexpr uint64_t mul = 0xd1342543de82ef95ull;
+  const uint64_t at =
+      (uint64_t)(int64_t)i0 * mul + (mul * (unsigned)j + 0x2545f4914f6cdd1dull);
+  return (uint32_t)(splitmix64(rowkey ^ at) >> 40);
 }
 
-struct ArgMax {
-  float v;
-  int i;
+// Gumbel noise of these bits: u uniform in (0, 1]
+DEV_INLINE float gumbel(uint32_t bits) {
+  const float u = ((float)bits + 1.0f) * (1.0f / 16777216.0f);
+  return -__logf(-__logf(u));
+}
+
+constexpr int SNT = 256;              // threads of a block
+constexpr int SNW = SNT / 64;
+constexpr int DIGIT = 2048;           // bins of a radix pass
+
+// A piece's share of a row: raw softmax sums relative to m, the same at the
+// temperature, and the best entry of the draw (or the largest logit).
+struct alignas(8) Share {
+  float m, s, st;
+  float best;
+  int best_i;
+  int pad;
 };
 
-template <int NW>
-DEV_INLINE ArgMax block_argmax(float v, int idx, float* lds_v, int* lds_i) {
-  int lane = threadIdx.x & 63;
-  int wid = threadIdx.x >> 6;
+DEV_INLINE bool better(float v, int i, float w, int j) {
+  return v > w || (v == w && i < j);
+}
+
+DEV_INLINE void wave_best(float& v, int& i) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(v, off, 64);
-    int oi = __shfl_xor(idx, off, 64);
-    if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
+    const float ov = __shfl_xor(v, off, 64);
+    const int oi = __shfl_xor(i, off, 64);
+    if (better(ov, oi, v, i)) v = ov, i = oi;
   }
-  if (lane == 0) { lds_v[wid] = v; lds_i[wid] = idx; }
-  __syncthreads();
-  // re-broadcast through LDS: a shfl would only reach wave 0
-  if (threadIdx.x == 0) {
-    float rv = lds_v[0];
-    int ri = lds_i[0];
+}
+
+// running maximum and softmax sums of a thread
+template <bool TEMP>
+struct Sums {
+  float m = -INFINITY, s = 0.f, st = 0.f;
+  // c: the largest of v
+  template <int N>
+  DEV_INLINE void add(const float (&v)[N], float c, float inv_temp) {
+    if (c > m) {
+      s *= __expf(m - c);              // 0 at the first numbers
+      if (TEMP) st *= __expf((m - c) * inv_temp);
+      m = c;
+    }
+    if (m == -INFINITY) return;
 #pragma unroll
-    for (int w = 1; w < NW; ++w) {
-      if (lds_v[w] > rv || (lds_v[w] == rv && lds_i[w] < ri)) {
-        rv = lds_v[w];
-        ri = lds_i[w];
-      }
+    for (int j = 0; j < N; ++j) {
+      s += __expf(v[j] - m);
+      if (TEMP) st += __expf((v[j] - m) * inv_temp);
     }
-    lds_v[0] = rv;
-    lds_i[0] = ri;
   }
-  __syncthreads();
-  ArgMax out;
-  out.v = lds_v[0];
-  out.i = lds_i[0];
-  return out;
-}
-
-// radix walk: find enc-threshold tau such that the kept set {enc >= tau}
-// satisfies the constraint (count >= k for top-k, mass >= target for top-p).
-// COUNT mode: WANT_MASS=false.  hist built over elements matching prefix.
-template <typename T, bool WANT_MASS>
-DEV_INLINE uint32_t radix_select(const T* __restrict__ x, int V, int rounds,
-                                 float inv_temp, float m_scaled,
-                                 float need_count, float target_mass,
-                                 uint32_t* h_cnt, float* h_mass) {
-  uint32_t prefix = 0;  // high bits decided so far (left-aligned)
-  float committed_cnt = 0.f, committed_mass = 0.f;
-  for (int r = 0; r < rounds; ++r) {
-    const int shift = 24 - 8 * r;
-    // zero histogram
-    for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-      h_cnt[b] = 0;
-      if (WANT_MASS) h_mass[b] = 0.f;
+  // relative to the larger maximum of the two
+  DEV_INLINE void merge(float om, float os, float ot, float inv_temp) {
+    const float c = fmaxf(m, om);
+    if (c == -INFINITY) return;
+    const float a = m == c ? 1.f : __expf(m - c);
+    const float b = om == c ? 1.f : __expf(om - c);
+    s = s * a + os * b;
+    if (TEMP) {
+      const float at = m == c ? 1.f : __expf((m - c) * inv_temp);
+      const float bt = om == c ? 1.f : __expf((om - c) * inv_temp);
+      st = st * at + ot * bt;
     }
-    __syncthreads();
-    const uint32_t pmask = (r == 0) ? 0u : (0xFFFFFFFFu << (shift + 8));
-    for (int i = threadIdx.x; i < V; i += blockDim.x) {
-      float xi = (float)x[i];
-      uint32_t e = enc_f32(xi);
-      if ((e & pmask) != prefix) continue;
-      uint32_t bin = (e >> shift) & 0xFFu;
-      atomicAdd(&h_cnt[bin], 1u);
-      if (WANT_MASS) atomicAdd(&h_mass[bin], __expf(xi * inv_temp - m_scaled));
-    }
-    __syncthreads();
-    // single-thread walk (256 bins) then broadcast via LDS
-    __shared__ uint32_t sel_bin;
-    __shared__ float sel_cnt, sel_mass;
-    if (threadIdx.x == 0) {
-      float cum_c = committed_cnt, cum_m = committed_mass;
-      int b = 255;
-      for (; b >= 0; --b) {
-        cum_c += (float)h_cnt[b];
-        if (WANT_MASS) cum_m += h_mass[b];
-        bool ok = WANT_MASS ? (cum_m >= target_mass) : (cum_c >= need_count);
-        if (ok) break;
-      }
-      if (b < 0) b = 0;  // numerical slack: keep everything in lowest bin
-      sel_bin = (uint32_t)b;
-      sel_cnt = cum_c - (float)h_cnt[b];
-      sel_mass = WANT_MASS ? (cum_m - h_mass[b]) : 0.f;
-    }
-    __syncthreads();
-    prefix |= (sel_bin << shift);
-    committed_cnt = sel_cnt;
-    committed_mass = sel_mass;
-    __syncthreads();
+    m = c;
   }
-  // tau = lower edge of the final selected bin
-  return prefix;
-}
+  DEV_INLINE void wave(float inv_temp) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      merge(__shfl_xor(m, off, 64), __shfl_xor(s, off, 64),
+            TEMP ? __shfl_xor(st, off, 64) : 0.f, inv_temp);
+  }
+};
 
-// Fast path: no top-k / top-p filter (the common RL rollout setting).
-// ONE streaming pass computes simultaneously, 8 elements per lane per step
-// (vectorized bf16x8/float4 loads, G13):
-//   * online max m + sumexp s (for the reported raw logprob),
-//   * raw argmax (greedy),
-//   * Gumbel-argmax z = x/T + G_i with the winner's logit tracked inline.
-// 1024 threads/block, one block per row: at decode batch >= 256 the whole
-// chip is busy; a second grid dim is unnecessary because decode sampling
-// runs alongside nothing.
-template <typename T, int VEC>
-__global__ __launch_bounds__(1024) void sample_fast_kernel(
-    int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
-    const T* __restrict__ logits, const float* __restrict__ temperature,
-    uint64_t seed, const long long* __restrict__ seed_ptr, int V) {
-  if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
-  __shared__ float red_f[16];
-  __shared__ int red_i[16];
-  const long row = blockIdx.x;
-  const T* x = logits + row * V;
-  const float temp = temperature[row];
-  const bool greedy = (temp == 0.f);
-  const float inv_temp = greedy ? 1.f : (1.0f / temp);
-  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-
-  float m = -INFINITY, s = 0.f;       // online raw softmax state
-  float rmax = -INFINITY;             // raw argmax (greedy pick)
-  int rarg = 0;
-  float best = -INFINITY;             // gumbel winner
+// the draw of a thread, pruned by the wave's best
+struct Draw {
+  float best = -INFINITY, wbest = -INFINITY;
   int best_i = 0;
-  float best_logit = 0.f;
 
-  const int nvec = V / VEC;
-  using vec_t = typename std::conditional<sizeof(T) == 2, bf16x8, float4>::type;
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-    vec_t pack = reinterpret_cast<const vec_t*>(x)[i];
+  // v: entries i0 .. of the row, c the largest; tau: encoding that an entry
+  // must reach (0: all)
+  template <int N>
+  DEV_INLINE void add(const float (&v)[N], float c, int i0, int V,
+                      uint64_t rowkey, float inv_temp, uint32_t tau) {
+    if (tau != 0 && !__any(enc_f32(c) >= tau)) return;
+    // 24-bit numbers below this lose whatever the logit (all may win at a
+    // negative temperature, where c is no bound)
+    int least = 0;
+    if (inv_temp > 0.f) {
+      const float u = __expf(-__expf(c * inv_temp - wbest));
+      least = (int)(u * (16777216.f * (1.f - 1e-5f))) - 2;
+    }
+    uint32_t bits[N];
+    bool hit = false;
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      float xi;
-      if constexpr (sizeof(T) == 2) xi = bf2f(((const bf16x8&)pack).v[j]);
-      else xi = ((const float*)&pack)[j];
-      const int idx = i * VEC + j;
-      if (xi > rmax) { rmax = xi; rarg = idx; }
-      if (xi > m) { s *= __expf(m - xi); m = xi; }
-      s += __expf(xi - m);
-      if (!greedy) {
-        float u = rng_uniform(rowkey, (uint64_t)idx);
-        float z = __fmaf_rn(xi, inv_temp, -__logf(-__logf(u)));
-        if (z > best) { best = z; best_i = idx; best_logit = xi; }
+    for (int j = 0; j < N; ++j) {
+      bits[j] = rng_bits(rowkey, i0, j);
+      hit |= (int)bits[j] >= least;
+    }
+    if (!__any(hit)) return;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if ((int)bits[j] < least || (unsigned)(i0 + j) >= (unsigned)V ||
+          (tau != 0 && enc_f32(v[j]) < tau))
+        continue;
+      const float z = __fmaf_rn(v[j], inv_temp, gumbel(bits[j]));
+      if (better(z, i0 + j, best, best_i)) best = z, best_i = i0 + j;
+    }
+    float w = best;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      w = fmaxf(w, __shfl_xor(w, off, 64));
+    wbest = w;
+  }
+};
+
+// ------------------------------------------------------------- one pass
+// MODE 0: sums and draw in one (no filter); 1: sums (and the largest logit)
+// of a filtered row; 2: its draw.
+template <typename T, int MODE>
+__global__ __launch_bounds__(SNT) void sample_pass_kernel(
+    Share* __restrict__ share, uint32_t* __restrict__ hist, int hist_words,
+    const uint32_t* __restrict__ tau_of, const T* __restrict__ logits,
+    const float* __restrict__ temperature, uint64_t seed,
+    const long long* __restrict__ seed_ptr, int V, int split) {
+  __shared__ Share part[SNW];
+  const long row = blockIdx.x / split;
+  const int piece = blockIdx.x % split;
+  if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
+  const VocabRow<T> r(logits + row * V, V);
+  const float temp = temperature[row];
+  const bool greedy = temp == 0.f;
+  if (MODE == 2 && greedy) return;    // the first pass found it
+  const float inv_temp = greedy ? 1.f : 1.0f / temp;
+  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
+  const uint32_t tau = MODE == 2 ? tau_of[row] : 0;
+  if (MODE == 1) {                    // the digit passes' bins start at 0
+    uint32_t* h = hist + row * hist_words;
+    for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
+      h[i] = 0;
+  }
+
+  constexpr int VEC = VocabRow<T>::VEC;
+  const int groups = r.groups();
+  Sums<MODE == 1> sums;
+  Draw d;
+  // every lane of a wave takes part in every round (the draw votes)
+  for (int g0 = piece * SNT; g0 < groups; g0 += split * SNT) {
+    const int g = g0 + threadIdx.x;
+    float v[VEC];
+    if (g < groups) {
+      r.load(g, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) v[j] = -INFINITY;
+    }
+    float c = v[0];
+#pragma unroll
+    for (int j = 1; j < VEC; ++j) c = fmaxf(c, v[j]);
+    if (MODE != 2) sums.add(v, c, inv_temp);
+    const int i0 = r.first(g);
+    if (MODE == 1 || greedy) {
+      if (c > d.best) {
+        d.best = c;
+#pragma unroll
+        for (int j = VEC - 1; j >= 0; --j)
+          if (v[j] == c) d.best_i = i0 + j;
       }
+    } else {
+      d.add(v, c, i0, V, rowkey, inv_temp, tau);
     }
   }
-  for (int idx = nvec * VEC + threadIdx.x; idx < V; idx += blockDim.x) {
-    float xi = (float)x[idx];
-    if (xi > rmax) { rmax = xi; rarg = idx; }
-    if (xi > m) { s *= __expf(m - xi); m = xi; }
-    s += __expf(xi - m);
-    if (!greedy) {
-      float u = rng_uniform(rowkey, (uint64_t)idx);
-      float z = __fmaf_rn(xi, inv_temp, -__logf(-__logf(u)));
-      if (z > best) { best = z; best_i = idx; best_logit = xi; }
-    }
-  }
-
-  // block reductions (16 waves)
-  ArgMax am = block_argmax<16>(rmax, rarg, red_f, red_i);
+  if (MODE != 2) sums.wave(inv_temp);
+  wave_best(d.best, d.best_i);
+  if ((threadIdx.x & 63) == 0)
+    part[threadIdx.x >> 6] = {sums.m, sums.s, sums.st, d.best, d.best_i, 0};
   __syncthreads();
-  const float gm = am.v;
-  s *= (m == -INFINITY) ? 0.f : __expf(m - gm);
-  float gs = block_reduce_sum<16>(s, red_f);
-  __syncthreads();
-  const float lz_raw = gm + __logf(gs);
-
-  if (greedy) {
-    if (threadIdx.x == 0) {
-      out_tokens[row] = am.i;
-      out_logprobs[row] = (float)x[am.i] - lz_raw;
-    }
-    return;
-  }
-  // winner's raw logit rides along through a second argmax reduce keyed on z
-  ArgMax pick = block_argmax<16>(best, best_i, red_f, red_i);
   if (threadIdx.x == 0) {
-    out_tokens[row] = pick.i;
-    out_logprobs[row] = (float)x[pick.i] - lz_raw;
+    for (int w = 1; w < SNW; ++w) {
+      if (MODE != 2)
+        sums.merge(part[w].m, part[w].s, part[w].st, inv_temp);
+      if (better(part[w].best, part[w].best_i, d.best, d.best_i))
+        d.best = part[w].best, d.best_i = part[w].best_i;
+    }
+    Share* out = share + row * split + piece;
+    if (MODE != 2) out->m = sums.m, out->s = sums.s, out->st = sums.st;
+    out->best = d.best;
+    out->best_i = d.best_i;
   }
-  (void)best_logit;
+}
+
+// sums of a whole row (every lane of the wave gets them); split <= 64
+template <bool TEMP>
+DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
+  const int lane = threadIdx.x & 63;
+  Sums<TEMP> a;
+  if (lane < split)
+    a.m = share[lane].m, a.s = share[lane].s, a.st = share[lane].st;
+  a.wave(inv_temp);
+  return a;
 }
 
 template <typename T>
-__global__ void sample_kernel(int64_t* __restrict__ out_tokens,
-                              float* __restrict__ out_logprobs,
-                              const T* __restrict__ logits,
-                              const float* __restrict__ temperature,
-                              const int* __restrict__ top_k,
-                              const float* __restrict__ top_p,
-                              uint64_t seed, int V, int rounds) {
-  __shared__ float red_f[8];
-  __shared__ int red_i[8];
-  __shared__ uint32_t h_cnt[256];
-  __shared__ float h_mass[256];
-
+__global__ __launch_bounds__(64) void sample_merge_kernel(
+    int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
+    const Share* __restrict__ share, const T* __restrict__ logits, int V,
+    int split) {
   const long row = blockIdx.x;
-  const T* x = logits + row * V;
+  const int lane = threadIdx.x;
+  share += row * split;
+  const Sums<false> a = row_sums<false>(share, split, 1.f);
+  float best = lane < split ? share[lane].best : -INFINITY;
+  int best_i = lane < split ? share[lane].best_i : 0x7fffffff;
+  wave_best(best, best_i);
+  if (lane == 0) {
+    out_tokens[row] = best_i;
+    out_logprobs[row] =
+        (float)logits[row * V + best_i] - (a.m + __logf(a.s));
+  }
+}
+
+// ------------------------------------------------------- radix selection
+// Bins of a digit of the encoding: [shift, shift + bits).  Per row and digit
+// four arrays of DIGIT words: counts and mass for top-k's prefix, the same
+// for top-p's (they part after the first digit).
+struct Pick {                         // where a selection stands
+  uint32_t prefix;                    // digits decided so far, left-aligned
+  float cnt, mass;                    // count / mass above them
+};
+
+// Walks the bins from the top until the running count reaches ``need`` (or
+// the running mass ``target``); bin 0 if none does.  All threads of the block
+// get the bin and the sum above it.
+template <bool MASS>
+DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
+                         float* lds, int& bin, float& before) {
+  // thread t sums bins [t*per, +per) counted from the top
+  const int per = (n + SNT - 1) / SNT;
+  auto at = [&](int i) -> float {     // i-th bin from the top
+    if (i >= n) return 0.f;
+    return MASS ? __uint_as_float(bins[n - 1 - i]) : (float)bins[n - 1 - i];
+  };
+  float own = 0.f;
+  for (int i = 0; i < per; ++i) own += at(threadIdx.x * per + i);
+  float upto = own;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const float o = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += o;
+  }
+  __syncthreads();
+  if (lane == 63) lds[wid] = upto;
+  int* found = reinterpret_cast<int*>(lds + SNW);
+  if (threadIdx.x == 0) *found = SNT;
+  __syncthreads();
+  float base = above;
+  for (int w = 0; w < wid; ++w) base += lds[w];
+  if (base + upto >= goal) atomicMin(found, (int)threadIdx.x);
+  __syncthreads();
+  const int who = *found;
+  if (who == SNT) {                   // numerical slack: keep everything
+    bin = 0;
+    before = 0.f;
+    return;
+  }
+  if ((int)threadIdx.x == who) {
+    float run = base + upto - own;
+    int i = 0;
+    for (; i < per - 1; ++i) {
+      const float next = run + at(who * per + i);
+      if (next >= goal) break;
+      run = next;
+    }
+    lds[SNW + 1] = run;
+    *found = max(n - 1 - (who * per + i), 0);
+  }
+  __syncthreads();
+  bin = *found;
+  before = lds[SNW + 1];
+}
+
+DEV_INLINE int digit_shift(int d) { return d == 0 ? 21 : d == 1 ? 10 : 0; }
+// digits of a type: bf16 numbers have 16 bits, 11 + 5; fp32 11 + 11 + 10
+template <typename T>
+DEV_INLINE int digit_low(int d) {     // lowest bit of digit d
+  return sizeof(T) == 2 && d == 1 ? 16 : digit_shift(d);
+}
+template <typename T>
+DEV_INLINE int digit_bins(int d) {
+  return d == 0 ? DIGIT : sizeof(T) == 2 ? 32 : d == 1 ? DIGIT : 1024;
+}
+
+// The two selections after the first ``digits`` digits of a row.
+template <typename T>
+DEV_INLINE void select_digits(const uint32_t* h, int digits, bool by_k,
+                              bool by_p, float k, float target, float* lds,
+                              Pick& pk, Pick& pp) {
+  pk = {0, 0.f, 0.f};
+  pp = {0, 0.f, 0.f};
+  for (int d = 0; d < digits; ++d, h += 4 * DIGIT) {
+    int bin;
+    if (by_k) {
+      find_bin<false>(h, digit_bins<T>(d), pk.cnt, k, lds, bin, pk.cnt);
+      pk.prefix |= (uint32_t)bin << digit_low<T>(d);
+    }
+    if (by_p) {
+      // the first digit's mass serves both; later ones have their own
+      find_bin<true>(h + (d == 0 ? DIGIT : 3 * DIGIT), digit_bins<T>(d),
+                     pp.mass, target, lds, bin, pp.mass);
+      pp.prefix |= (uint32_t)bin << digit_low<T>(d);
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(SNT) void sample_digit_kernel(
+    uint32_t* __restrict__ hist, int hist_words, const Share* __restrict__ share,
+    const T* __restrict__ logits, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, int digit,
+    int V, int split) {
+  __shared__ uint32_t cnt[DIGIT];
+  __shared__ float mass[DIGIT];
+  __shared__ float lds[SNW + 2];
+  const long row = blockIdx.x / split;
+  const int piece = blockIdx.x % split;
   const float temp = temperature[row];
   const int k = top_k[row];
   const float p = top_p[row];
-
-  // pass 1: raw max + argmax + raw sumexp (for logprob report / greedy)
-  float m = -INFINITY, s = 0.f;
-  float local_max = -INFINITY;
-  int local_arg = 0;
-  for (int i = threadIdx.x; i < V; i += blockDim.x) {
-    float xi = (float)x[i];
-    if (xi > local_max) { local_max = xi; local_arg = i; }
-    if (xi > m) {
-      s *= __expf(m - xi);
-      m = xi;
-    }
-    s += __expf(xi - m);
-  }
-  ArgMax am = block_argmax<4>(local_max, local_arg, red_f, red_i);
-  __syncthreads();
-  float gm = am.v;
-  s *= (m == -INFINITY) ? 0.f : __expf(m - gm);
-  float gs = block_reduce_sum<4>(s, red_f);
-  __syncthreads();
-  const float lz_raw = gm + __logf(gs);
-
-  if (temp == 0.f) {  // greedy
-    if (threadIdx.x == 0) {
-      out_tokens[row] = am.i;
-      out_logprobs[row] = (float)x[am.i] - lz_raw;
-    }
-    return;
-  }
-
+  const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
+  if (temp == 0.f || (!by_k && !by_p)) return;
   const float inv_temp = 1.0f / temp;
-  // thresholds (enc-space); default: keep everything
-  uint32_t tau = 0;
-  if (k > 0 && k < V) {
-    uint32_t tk = radix_select<T, false>(x, V, rounds, inv_temp, 0.f,
-                                         (float)k, 0.f, h_cnt, h_mass);
-    tau = max(tau, tk);
-    __syncthreads();
-  }
-  if (p < 1.0f) {
-    // total scaled mass
-    float st = 0.f;
-    const float m_scaled = gm * inv_temp;
-    for (int i = threadIdx.x; i < V; i += blockDim.x)
-      st += __expf((float)x[i] * inv_temp - m_scaled);
-    float gst = block_reduce_sum<4>(st, red_f);
-    __syncthreads();
-    uint32_t tp = radix_select<T, true>(x, V, rounds, inv_temp, m_scaled,
-                                        0.f, p * gst, h_cnt, h_mass);
-    tau = max(tau, tp);
-    __syncthreads();
-  }
+  const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
+  const float m_scaled = all.m * inv_temp;
+  uint32_t* h = hist + row * hist_words;
+  Pick pk, pp;
+  select_digits<T>(h, digit, by_k, by_p, (float)k, p * all.st, lds, pk, pp);
+  h += digit * 4 * DIGIT;
 
-  // Gumbel-argmax over kept set
-  float best = -INFINITY;
-  int best_i = 0;
-  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  for (int i = threadIdx.x; i < V; i += blockDim.x) {
-    float xi = (float)x[i];
-    if (enc_f32(xi) < tau) continue;
-    float u = rng_uniform(rowkey, (uint64_t)i);
-    float g = -__logf(-__logf(u));
-    float z = xi * inv_temp + g;
-    if (z > best) { best = z; best_i = i; }
+  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+  const uint32_t above = digit == 0 ? 0u
+      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
+  __syncthreads();
+  for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
+  __syncthreads();
+  const VocabRow<T> r(logits + row * V, V);
+  constexpr int VEC = VocabRow<T>::VEC;
+  const int groups = r.groups();
+  for (int g = piece * SNT + threadIdx.x; g < groups; g += split * SNT) {
+    float v[VEC];
+    r.load(g, v);
+    const int i0 = r.first(g);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if ((unsigned)(i0 + j) >= (unsigned)V) continue;
+      const uint32_t e = enc_f32(v[j]);
+      const uint32_t bin = (e >> low) & (bins - 1);
+      if (by_k && (e & above) == pk.prefix) atomicAdd(&cnt[bin], 1u);
+      if (by_p && (e & above) == pp.prefix)
+        atomicAdd(&mass[bin], __expf(v[j] * inv_temp - m_scaled));
+    }
   }
-  ArgMax pick = block_argmax<4>(best, best_i, red_f, red_i);
-  if (threadIdx.x == 0) {
-    out_tokens[row] = pick.i;
-    out_logprobs[row] = (float)x[pick.i] - lz_raw;
+  __syncthreads();
+  uint32_t* hc = h;
+  float* hm = reinterpret_cast<float*>(h + (digit == 0 ? 1 : 3) * DIGIT);
+  for (int i = threadIdx.x; i < bins; i += SNT) {
+    if (cnt[i]) atomicAdd(&hc[i], cnt[i]);
+    if (mass[i] != 0.f) atomicAdd(&hm[i], mass[i]);
   }
+}
+
+// the encoding that a row's kept entries reach
+template <typename T>
+__global__ __launch_bounds__(SNT) void sample_tau_kernel(
+    uint32_t* __restrict__ tau, const uint32_t* __restrict__ hist,
+    int hist_words, const Share* __restrict__ share,
+    const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, int digits, int V, int split) {
+  __shared__ float lds[SNW + 2];
+  const long row = blockIdx.x;
+  const float temp = temperature[row];
+  const int k = top_k[row];
+  const float p = top_p[row];
+  const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
+  if (temp == 0.f) return;
+  const float inv_temp = 1.0f / temp;
+  const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
+  Pick pk, pp;
+  select_digits<T>(hist + row * hist_words, digits, by_k, by_p, (float)k,
+                   p * all.st, lds, pk, pp);
+  if (threadIdx.x == 0) tau[row] = max(pk.prefix, pp.prefix);
+}
+
+template <typename T>
+static void launch_sample(torch::Tensor& out_tokens,
+                          torch::Tensor& out_logprobs,
+                          const torch::Tensor& logits,
+                          const torch::Tensor& temperature,
+                          const torch::Tensor& top_k,
+                          const torch::Tensor& top_p, uint64_t seed,
+                          const long long* seed_ptr, bool no_filter) {
+  const long N = logits.size(0);
+  const int V = logits.size(1);
+  if (N == 0) return;
+  auto stream = at::hip::getCurrentHIPStream();
+  // pieces of a row: 2048 blocks in all (eight per CU), none under two
+  // rounds of 256 words
+  const long words = (V + VocabRow<T>::VEC - 1) / VocabRow<T>::VEC;
+  const int split = (int)std::max<long>(
+      1, std::min<long>({64, (2048 + N - 1) / N, words / (2 * SNT)}));
+  const int digits = sizeof(T) == 2 ? 2 : 3;
+  const int hist_words = no_filter ? 0 : digits * 4 * DIGIT;
+  // per row: the pieces' shares, the bins, the threshold.  From the caching
+  // allocator: a block per call and stream, also while a graph is captured
+  const long share_words = (long)split * (sizeof(Share) / 4);
+  auto ws = torch::empty({N * (share_words + hist_words + 1)},
+                         logits.options().dtype(torch::kInt32));
+  Share* share = reinterpret_cast<Share*>(ws.data_ptr<int>());
+  uint32_t* hist =
+      reinterpret_cast<uint32_t*>(ws.data_ptr<int>()) + N * share_words;
+  uint32_t* tau = hist + N * hist_words;
+  const T* x = (const T*)logits.data_ptr();
+  const float* temp = temperature.data_ptr<float>();
+  TORCH_CHECK(N * split < (1L << 31), "too many rows");
+  const dim3 grid((unsigned)(N * split)), block(SNT);
+  if (no_filter) {
+    sample_pass_kernel<T, 0><<<grid, block, 0, stream>>>(
+        share, hist, 0, tau, x, temp, seed, seed_ptr, V, split);
+  } else {
+    const int* k = top_k.data_ptr<int>();
+    const float* p = top_p.data_ptr<float>();
+    sample_pass_kernel<T, 1><<<grid, block, 0, stream>>>(
+        share, hist, hist_words, tau, x, temp, seed, seed_ptr, V, split);
+    for (int d = 0; d < digits; ++d)
+      sample_digit_kernel<T><<<grid, block, 0, stream>>>(
+          hist, hist_words, share, x, temp, k, p, d, V, split);
+    sample_tau_kernel<T><<<dim3(N), block, 0, stream>>>(
+        tau, hist, hist_words, share, temp, k, p, digits, V, split);
+    sample_pass_kernel<T, 2><<<grid, block, 0, stream>>>(
+        share, hist, hist_words, tau, x, temp, seed, seed_ptr, V, split);
+  }
+  sample_merge_kernel<T><<<dim3(N), dim3(64), 0, stream>>>(
+      out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(), share, x,
+      V, split);
+  HIP_CHECK_KERNEL();
 }
 
 void sample(torch::Tensor out_tokens, torch::Tensor out_logprobs,
@@ -318,41 +507,16 @@ void sample(torch::Tensor out_tokens, torch::Tensor out_logprobs,
   TORCH_CHECK(temperature.dtype() == torch::kFloat32);
   TORCH_CHECK(top_k.dtype() == torch::kInt32);
   TORCH_CHECK(top_p.dtype() == torch::kFloat32);
-  const long N = logits.size(0);
-  const int V = logits.size(1);
-  auto stream = at::hip::getCurrentHIPStream();
-  if (no_filter) {  // fused single-pass path (no top-k/top-p), G13-vectorized
-    const long long* sp = seed_dev.defined() && seed_dev.numel() > 0
-                              ? (const long long*)seed_dev.data_ptr<int64_t>()
-                              : nullptr;
-    if (logits.dtype() == torch::kBFloat16) {
-      sample_fast_kernel<bf16_t, 8><<<dim3(N), dim3(1024), 0, stream>>>(
-          out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
-          (const bf16_t*)logits.data_ptr(), temperature.data_ptr<float>(),
-          (uint64_t)seed, sp, V);
-    } else {
-      sample_fast_kernel<float, 4><<<dim3(N), dim3(1024), 0, stream>>>(
-          out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
-          (const float*)logits.data_ptr(), temperature.data_ptr<float>(),
-          (uint64_t)seed, sp, V);
-    }
-    HIP_CHECK_KERNEL();
-    return;
-  }
-  if (logits.dtype() == torch::kBFloat16) {
-    sample_kernel<bf16_t><<<dim3(N), dim3(256), 0, stream>>>(
-        out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
-        (const bf16_t*)logits.data_ptr(), temperature.data_ptr<float>(),
-        top_k.data_ptr<int>(), top_p.data_ptr<float>(), (uint64_t)seed, V,
-        /*rounds=*/2);
-  } else if (logits.dtype() == torch::kFloat32) {
-    sample_kernel<float><<<dim3(N), dim3(256), 0, stream>>>(
-        out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
-        (const float*)logits.data_ptr(), temperature.data_ptr<float>(),
-        top_k.data_ptr<int>(), top_p.data_ptr<float>(), (uint64_t)seed, V,
-        /*rounds=*/4);
-  } else {
+  // the device seed counts for unfiltered rows only
+  const long long* sp = no_filter && seed_dev.defined() && seed_dev.numel() > 0
+                            ? (const long long*)seed_dev.data_ptr<int64_t>()
+                            : nullptr;
+  if (logits.dtype() == torch::kBFloat16)
+    launch_sample<bf16_t>(out_tokens, out_logprobs, logits, temperature, top_k,
+                          top_p, (uint64_t)seed, sp, no_filter);
+  else if (logits.dtype() == torch::kFloat32)
+    launch_sample<float>(out_tokens, out_logprobs, logits, temperature, top_k,
+                         top_p, (uint64_t)seed, sp, no_filter);
+  else
     TORCH_CHECK(false, "sample: dtype must be bf16 or fp32");
-  }
-  HIP_CHECK_KERNEL();
 }

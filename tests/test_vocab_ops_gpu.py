@@ -54,3 +54,78 @@ def test_logprobs_minus_infinity(v):
     lab = torch.tensor([v - 1, v // 2], device=DEV)
     want = torch.log_softmax(x.double(), -1).gather(1, lab[:, None])[:, 0]
     assert (ops.gather_logprobs(x, lab).double() - want).abs().max() < 1e-5
+
+
+# ------------------------------------------------------------------ sampling
+
+
+def noise(seed, row, v):
+    """Gumbel noise of a row's entries, from the documented generator:
+    splitmix64 keyed by (seed, row, entry), 24 bits, -log(-log u)."""
+    import numpy as np
+    with np.errstate(over="ignore"):
+        u64 = np.uint64
+        key = u64(seed) + u64(row) * u64(0x9e3779b97f4a7c15)
+        z = key ^ (np.arange(v, dtype=u64) * u64(0xd1342543de82ef95)
+                   + u64(0x2545f4914f6cdd1d))
+        z = z + u64(0x9e3779b97f4a7c15)
+        z = (z ^ (z >> u64(30))) * u64(0xbf58476d1ce4e5b9)
+        z = (z ^ (z >> u64(27))) * u64(0x94d049bb133111eb)
+        u = ((z >> u64(40)).astype("f8") + 1) / 16777216.0
+        return torch.from_numpy(-np.log(-np.log(u)))
+
+
+def kept(x, temp, k, p):
+    """Mask of the kept entries, and of those within 1e-4 of the top-p
+    boundary (32-bit mass)."""
+    v = x.numel()
+    s, order = x.sort(descending=True)
+    low = s[k - 1] if 0 < k < v else torch.tensor(-float("inf"))
+    sure, maybe = x >= low, x >= low
+    if p < 1.0:
+        mass = torch.softmax(s / temp, -1).cumsum(-1)
+        for slack, which in ((1e-4, "maybe"), (-1e-4, "sure")):
+            j = int((mass < p + slack).sum().clamp(max=v - 1))
+            cut = x >= s[j]
+            if which == "maybe":
+                maybe = maybe & cut
+            else:
+                sure = sure & cut
+    return sure, maybe
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v", [(1, 9), (3, 1000), (2, 50257), (70, 4099),
+                                 (2100, 300), (4, 151936)])
+@pytest.mark.parametrize("temp,k,p", [(1.0, -1, 1.0), (0.7, 5, 1.0),
+                                      (1.3, -1, 0.9), (0.7, 50, 0.6),
+                                      (0.0, 3, 0.5), (1.0, 10 ** 6, 0.999)])
+def test_sample_against_its_definition(n, v, dtype, temp, k, p):
+    torch.manual_seed(3)
+    x = (torch.randn(n, v, device=DEV) * 2.5).to(dtype)
+    if v > 20:
+        x[:, 7] = -float("inf")
+    seed = 12345
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    args = (x, full(temp, torch.float32), full(k, torch.int32),
+            full(p, torch.float32), seed)
+    plain = (k <= 0 or k >= v) and p >= 1.0
+    tok, lp = ops.sample(*args, no_filter=plain)
+    again = ops.sample(*args, no_filter=plain)
+    assert torch.equal(tok, again[0])
+    if plain:      # the filtered path keeps everything: the same draw
+        assert torch.equal(tok, ops.sample(*args, no_filter=False)[0])
+    want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+    assert (lp.double() - want).abs().max() <= 1e-5 * (1 + want.abs().max())
+    for r in list(range(min(n, 3))) + [n - 1]:
+        row = x[r].double().cpu()
+        t = int(tok[r])
+        assert 0 <= t < v
+        if temp == 0.0:
+            assert t == int(row.argmax())
+            continue
+        sure, maybe = kept(row, temp, k, p)
+        assert maybe[t]
+        z = row / temp + noise(seed, r, v)
+        # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
+        assert z[t] >= z[sure].max() - 1e-3
