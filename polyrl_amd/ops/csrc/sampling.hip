@@ -21,6 +21,13 @@
 // With one: sums, one pass per radix digit (11 bits, then the rest of a bf16
 // number's 16 or an fp32 number's 32), the draw over the kept set.
 //
+// Only entries that can stand at a threshold go into a digit's bins (cut_of):
+// with k at most the number of lane groups, the k-th largest of the groups'
+// maxima is no more than the k-th largest entry; and entries that each have
+// less than (1 - p) / V of the mass have less than 1 - p together, so the
+// nucleus ends above them.  All entries of 64 x 151936 (0.7, 50, 0.9) in LDS
+// atomics took 73 us a digit.
+//
 // What bounds it: integer multiplies of the generator (two 64-bit products a
 // number).  The two logarithms of a number's noise are only taken where its
 // 24 random bits can beat the wave's best so far: z > best means
@@ -60,6 +67,7 @@ DEV_INLINE float gumbel(uint32_t bits) {
 constexpr int SNT = 256;              // threads of a block
 constexpr int SNW = SNT / 64;
 constexpr int DIGIT = 2048;           // bins of a radix pass
+constexpr int TOPS = SNT / 16;        // maxima that a piece leaves
 
 // A piece's share of a row: raw softmax sums relative to m, the same at the
 // temperature, and the best entry of the draw (or the largest logit).
@@ -166,13 +174,188 @@ struct Draw {
   }
 };
 
+// sums of a whole row (every lane of the wave gets them); split <= 64
+template <bool TEMP>
+DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
+  const int lane = threadIdx.x & 63;
+  Sums<TEMP> a;
+  if (lane < split)
+    a.m = share[lane].m, a.s = share[lane].s, a.st = share[lane].st;
+  a.wave(inv_temp);
+  return a;
+}
+
+// ------------------------------------------------------- radix selection
+// Bins of a digit of the encoding: [shift, shift + bits).  Per row and digit
+// four arrays of DIGIT words: counts and mass for top-k's prefix, the same
+// for top-p's (they part after the first digit).
+struct alignas(8) Plan {              // where a row's two selections stand
+  float cut;                          // entries below it stand at neither
+  float m_scaled, target;             // top-p: largest x/T, mass to reach
+  uint32_t prefix_k, prefix_p;        // digits decided so far, left-aligned
+  float cnt, mass;                    // count / mass above them
+  int by;                             // 1: top-k, 2: top-p
+};
+
+// Walks the bins from the top until the running count reaches ``need`` (or
+// the running mass ``target``); bin 0 if none does.  All threads of the block
+// get the bin and the sum above it.
+template <bool MASS>
+DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
+                         float* lds, int& bin, float& before) {
+  // thread t has bins [t*per, +per) counted from the top
+  const int per = (n + SNT - 1) / SNT;   // at most DIGIT / SNT
+  constexpr int MOST = DIGIT / SNT;
+  float val[MOST], own = 0.f;
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int at = threadIdx.x * per + i;
+    val[i] = 0.f;
+    if (i < per && at < n)
+      val[i] = MASS ? __uint_as_float(bins[n - 1 - at]) : (float)bins[n - 1 - at];
+  }
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) own += val[i];
+  float upto = own;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const float o = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += o;
+  }
+  __syncthreads();
+  if (lane == 63) lds[wid] = upto;
+  int* found = reinterpret_cast<int*>(lds + SNW);
+  if (threadIdx.x == 0) *found = SNT;
+  __syncthreads();
+  float base = above;
+  for (int w = 0; w < wid; ++w) base += lds[w];
+  if (base + upto >= goal) atomicMin(found, (int)threadIdx.x);
+  __syncthreads();
+  const int who = *found;
+  if (who == SNT) {                   // numerical slack: keep everything
+    bin = 0;
+    before = 0.f;
+    return;
+  }
+  if ((int)threadIdx.x == who) {
+    float run = base + upto - own, at_run = run;
+    int at = per - 1;                  // the last one, if rounding hides it
+    bool done = false;
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) {
+      if (done || i >= per) continue;
+      at_run = run;
+      run += val[i];
+      if (run >= goal) at = i, done = true;
+    }
+    run = at_run;
+    lds[SNW + 1] = run;
+    *found = max(n - 1 - (who * per + at), 0);
+  }
+  __syncthreads();
+  bin = *found;
+  before = lds[SNW + 1];
+}
+
+DEV_INLINE int digit_shift(int d) { return d == 0 ? 21 : d == 1 ? 10 : 0; }
+// digits of a type: bf16 numbers have 16 bits, 11 + 5; fp32 11 + 11 + 10
+template <typename T>
+DEV_INLINE int digit_low(int d) {     // lowest bit of digit d
+  return sizeof(T) == 2 && d == 1 ? 16 : digit_shift(d);
+}
+template <typename T>
+DEV_INLINE int digit_bins(int d) {
+  return d == 0 ? DIGIT : sizeof(T) == 2 ? 32 : d == 1 ? DIGIT : 1024;
+}
+
+// Entries below this stand at neither threshold of their row (the top of this
+// file); lds: TOPS * split floats.
+DEV_INLINE float cut_of(const float* tops, bool by_k, bool by_p, int k, float p,
+                        float inv_temp, const Sums<true>& all, int V, int split,
+                        float* lds) {
+  float cut = -INFINITY;
+  if (by_p && inv_temp > 0.f && p > 0.f)
+    cut = all.m + __logf(0.99f * (1.f - p) * all.st / V) / inv_temp;
+  const int n = TOPS * split;
+  if (!by_k || k > n) return cut;
+  // waves' maxima where they are enough, else those of 16 lanes
+  const int width = k <= n / 4 ? 4 : 1, m = n / width;
+  __syncthreads();
+  for (int i = threadIdx.x; i < m; i += SNT) {
+    float t = tops[i * width];
+    for (int j = 1; j < width; ++j) t = fmaxf(t, tops[i * width + j]);
+    lds[i] = t;
+  }
+  __syncthreads();
+  __shared__ float kth;
+  for (int i = threadIdx.x; i < m; i += SNT) {
+    const float t = lds[i];
+    int rank = 0;
+    for (int j = 0; j < m; ++j) {
+      const float o = lds[j];
+      rank += o > t || (o == t && j < i);
+    }
+    if (rank == k - 1) kth = t;
+  }
+  __syncthreads();
+  return fmaxf(cut, kth);
+}
+
+// One block per row between the passes (in every block of the passes the same
+// work took longer than the passes): after the sums (``digit`` -1) the cut and
+// the goals, after a digit pass its bins.
+template <typename T>
+__global__ __launch_bounds__(SNT) void sample_plan_kernel(
+    Plan* __restrict__ plans, const uint32_t* __restrict__ hist,
+    int hist_words, const Share* __restrict__ share,
+    const float* __restrict__ tops, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, int digit,
+    int V, int split) {
+  __shared__ float lds[TOPS * 64];
+  const long row = blockIdx.x;
+  Plan& plan = plans[row];
+  const int k = top_k[row];
+  if (digit < 0) {
+    const float temp = temperature[row], p = top_p[row];
+    const bool by_k = temp != 0.f && k > 0 && k < V;
+    const bool by_p = temp != 0.f && p < 1.0f;
+    const float inv_temp = temp == 0.f ? 1.f : 1.0f / temp;
+    const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
+    const float cut = cut_of(tops + row * split * TOPS, by_k, by_p, k, p,
+                             inv_temp, all, V, split, lds);
+    if (threadIdx.x == 0)
+      plan = {cut, all.m * inv_temp, p * all.st, 0u, 0u, 0.f, 0.f,
+              (by_k ? 1 : 0) + (by_p ? 2 : 0)};
+    return;
+  }
+  const Plan now = plan;
+  const uint32_t* h = hist + row * hist_words + digit * 4 * DIGIT;
+  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+  int bin;
+  float before;
+  if (now.by & 1) {
+    find_bin<false>(h, bins, now.cnt, (float)k, lds, bin, before);
+    if (threadIdx.x == 0)
+      plan.prefix_k = now.prefix_k | (uint32_t)bin << low, plan.cnt = before;
+  }
+  if (now.by & 2) {
+    // the first digit's mass serves both; later ones have their own
+    find_bin<true>(h + (digit == 0 ? DIGIT : 3 * DIGIT), bins, now.mass,
+                   now.target, lds, bin, before);
+    if (threadIdx.x == 0)
+      plan.prefix_p = now.prefix_p | (uint32_t)bin << low, plan.mass = before;
+  }
+}
+
 // ------------------------------------------------------------- one pass
 // MODE 0: sums and draw in one (no filter); 1: sums (and the largest logit)
 // of a filtered row; 2: its draw.
 template <typename T, int MODE>
 __global__ __launch_bounds__(SNT) void sample_pass_kernel(
-    Share* __restrict__ share, uint32_t* __restrict__ hist, int hist_words,
-    const uint32_t* __restrict__ tau_of, const T* __restrict__ logits,
+    Share* __restrict__ share, float* __restrict__ tops,
+    uint32_t* __restrict__ hist, int hist_words,
+    const Plan* __restrict__ plans, const T* __restrict__ logits,
     const float* __restrict__ temperature, uint64_t seed,
     const long long* __restrict__ seed_ptr, int V, int split) {
   __shared__ Share part[SNW];
@@ -185,7 +368,9 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   if (MODE == 2 && greedy) return;    // the first pass found it
   const float inv_temp = greedy ? 1.f : 1.0f / temp;
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  const uint32_t tau = MODE == 2 ? tau_of[row] : 0;
+  // encoding that a kept entry reaches
+  const uint32_t tau =
+      MODE == 2 ? max(plans[row].prefix_k, plans[row].prefix_p) : 0;
   if (MODE == 1) {                    // the digit passes' bins start at 0
     uint32_t* h = hist + row * hist_words;
     for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
@@ -222,6 +407,13 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
       d.add(v, c, i0, V, rowkey, inv_temp, tau);
     }
   }
+  if (MODE == 1) {                    // largest of each 16 lanes
+    float t = d.best;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) t = fmaxf(t, __shfl_xor(t, off, 64));
+    if (threadIdx.x % 16 == 0)
+      tops[(row * split + piece) * TOPS + threadIdx.x / 16] = t;
+  }
   if (MODE != 2) sums.wave(inv_temp);
   wave_best(d.best, d.best_i);
   if ((threadIdx.x & 63) == 0)
@@ -239,17 +431,6 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
     out->best = d.best;
     out->best_i = d.best_i;
   }
-}
-
-// sums of a whole row (every lane of the wave gets them); split <= 64
-template <bool TEMP>
-DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
-  const int lane = threadIdx.x & 63;
-  Sums<TEMP> a;
-  if (lane < split)
-    a.m = share[lane].m, a.s = share[lane].s, a.st = share[lane].st;
-  a.wave(inv_temp);
-  return a;
 }
 
 template <typename T>
@@ -271,128 +452,24 @@ __global__ __launch_bounds__(64) void sample_merge_kernel(
   }
 }
 
-// ------------------------------------------------------- radix selection
-// Bins of a digit of the encoding: [shift, shift + bits).  Per row and digit
-// four arrays of DIGIT words: counts and mass for top-k's prefix, the same
-// for top-p's (they part after the first digit).
-struct Pick {                         // where a selection stands
-  uint32_t prefix;                    // digits decided so far, left-aligned
-  float cnt, mass;                    // count / mass above them
-};
-
-// Walks the bins from the top until the running count reaches ``need`` (or
-// the running mass ``target``); bin 0 if none does.  All threads of the block
-// get the bin and the sum above it.
-template <bool MASS>
-DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
-                         float* lds, int& bin, float& before) {
-  // thread t sums bins [t*per, +per) counted from the top
-  const int per = (n + SNT - 1) / SNT;
-  auto at = [&](int i) -> float {     // i-th bin from the top
-    if (i >= n) return 0.f;
-    return MASS ? __uint_as_float(bins[n - 1 - i]) : (float)bins[n - 1 - i];
-  };
-  float own = 0.f;
-  for (int i = 0; i < per; ++i) own += at(threadIdx.x * per + i);
-  float upto = own;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const float o = __shfl_up(upto, off, 64);
-    if (lane >= off) upto += o;
-  }
-  __syncthreads();
-  if (lane == 63) lds[wid] = upto;
-  int* found = reinterpret_cast<int*>(lds + SNW);
-  if (threadIdx.x == 0) *found = SNT;
-  __syncthreads();
-  float base = above;
-  for (int w = 0; w < wid; ++w) base += lds[w];
-  if (base + upto >= goal) atomicMin(found, (int)threadIdx.x);
-  __syncthreads();
-  const int who = *found;
-  if (who == SNT) {                   // numerical slack: keep everything
-    bin = 0;
-    before = 0.f;
-    return;
-  }
-  if ((int)threadIdx.x == who) {
-    float run = base + upto - own;
-    int i = 0;
-    for (; i < per - 1; ++i) {
-      const float next = run + at(who * per + i);
-      if (next >= goal) break;
-      run = next;
-    }
-    lds[SNW + 1] = run;
-    *found = max(n - 1 - (who * per + i), 0);
-  }
-  __syncthreads();
-  bin = *found;
-  before = lds[SNW + 1];
-}
-
-DEV_INLINE int digit_shift(int d) { return d == 0 ? 21 : d == 1 ? 10 : 0; }
-// digits of a type: bf16 numbers have 16 bits, 11 + 5; fp32 11 + 11 + 10
-template <typename T>
-DEV_INLINE int digit_low(int d) {     // lowest bit of digit d
-  return sizeof(T) == 2 && d == 1 ? 16 : digit_shift(d);
-}
-template <typename T>
-DEV_INLINE int digit_bins(int d) {
-  return d == 0 ? DIGIT : sizeof(T) == 2 ? 32 : d == 1 ? DIGIT : 1024;
-}
-
-// The two selections after the first ``digits`` digits of a row.
-template <typename T>
-DEV_INLINE void select_digits(const uint32_t* h, int digits, bool by_k,
-                              bool by_p, float k, float target, float* lds,
-                              Pick& pk, Pick& pp) {
-  pk = {0, 0.f, 0.f};
-  pp = {0, 0.f, 0.f};
-  for (int d = 0; d < digits; ++d, h += 4 * DIGIT) {
-    int bin;
-    if (by_k) {
-      find_bin<false>(h, digit_bins<T>(d), pk.cnt, k, lds, bin, pk.cnt);
-      pk.prefix |= (uint32_t)bin << digit_low<T>(d);
-    }
-    if (by_p) {
-      // the first digit's mass serves both; later ones have their own
-      find_bin<true>(h + (d == 0 ? DIGIT : 3 * DIGIT), digit_bins<T>(d),
-                     pp.mass, target, lds, bin, pp.mass);
-      pp.prefix |= (uint32_t)bin << digit_low<T>(d);
-    }
-  }
-}
-
 template <typename T>
 __global__ __launch_bounds__(SNT) void sample_digit_kernel(
-    uint32_t* __restrict__ hist, int hist_words, const Share* __restrict__ share,
-    const T* __restrict__ logits, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ top_p, int digit,
-    int V, int split) {
+    uint32_t* __restrict__ hist, int hist_words,
+    const Plan* __restrict__ plans, const T* __restrict__ logits,
+    const float* __restrict__ temperature, int digit, int V, int split) {
   __shared__ uint32_t cnt[DIGIT];
   __shared__ float mass[DIGIT];
-  __shared__ float lds[SNW + 2];
   const long row = blockIdx.x / split;
   const int piece = blockIdx.x % split;
-  const float temp = temperature[row];
-  const int k = top_k[row];
-  const float p = top_p[row];
-  const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
-  if (temp == 0.f || (!by_k && !by_p)) return;
-  const float inv_temp = 1.0f / temp;
-  const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
-  const float m_scaled = all.m * inv_temp;
-  uint32_t* h = hist + row * hist_words;
-  Pick pk, pp;
-  select_digits<T>(h, digit, by_k, by_p, (float)k, p * all.st, lds, pk, pp);
-  h += digit * 4 * DIGIT;
+  const Plan plan = plans[row];
+  if (plan.by == 0) return;
+  const bool by_k = plan.by & 1, by_p = plan.by & 2;
+  const float inv_temp = 1.0f / temperature[row];
+  uint32_t* h = hist + row * hist_words + digit * 4 * DIGIT;
 
   const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
   const uint32_t above = digit == 0 ? 0u
       : 0xFFFFFFFFu << digit_low<T>(digit - 1);
-  __syncthreads();
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
   __syncthreads();
   const VocabRow<T> r(logits + row * V, V);
@@ -404,12 +481,12 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
     const int i0 = r.first(g);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
-      if ((unsigned)(i0 + j) >= (unsigned)V) continue;
+      if (v[j] < plan.cut || (unsigned)(i0 + j) >= (unsigned)V) continue;
       const uint32_t e = enc_f32(v[j]);
       const uint32_t bin = (e >> low) & (bins - 1);
-      if (by_k && (e & above) == pk.prefix) atomicAdd(&cnt[bin], 1u);
-      if (by_p && (e & above) == pp.prefix)
-        atomicAdd(&mass[bin], __expf(v[j] * inv_temp - m_scaled));
+      if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
+      if (by_p && (e & above) == plan.prefix_p)
+        atomicAdd(&mass[bin], __expf(v[j] * inv_temp - plan.m_scaled));
     }
   }
   __syncthreads();
@@ -419,28 +496,6 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
     if (cnt[i]) atomicAdd(&hc[i], cnt[i]);
     if (mass[i] != 0.f) atomicAdd(&hm[i], mass[i]);
   }
-}
-
-// the encoding that a row's kept entries reach
-template <typename T>
-__global__ __launch_bounds__(SNT) void sample_tau_kernel(
-    uint32_t* __restrict__ tau, const uint32_t* __restrict__ hist,
-    int hist_words, const Share* __restrict__ share,
-    const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, int digits, int V, int split) {
-  __shared__ float lds[SNW + 2];
-  const long row = blockIdx.x;
-  const float temp = temperature[row];
-  const int k = top_k[row];
-  const float p = top_p[row];
-  const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
-  if (temp == 0.f) return;
-  const float inv_temp = 1.0f / temp;
-  const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
-  Pick pk, pp;
-  select_digits<T>(hist + row * hist_words, digits, by_k, by_p, (float)k,
-                   p * all.st, lds, pk, pp);
-  if (threadIdx.x == 0) tau[row] = max(pk.prefix, pp.prefix);
 }
 
 template <typename T>
@@ -462,34 +517,43 @@ static void launch_sample(torch::Tensor& out_tokens,
       1, std::min<long>({64, (2048 + N - 1) / N, words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
   const int hist_words = no_filter ? 0 : digits * 4 * DIGIT;
-  // per row: the pieces' shares, the bins, the threshold.  From the caching
-  // allocator: a block per call and stream, also while a graph is captured
+  // per row: the pieces' shares and maxima, the plan, the bins.  From the
+  // caching allocator: a block per call and stream, also while a graph is captured
   const long share_words = (long)split * (sizeof(Share) / 4);
-  auto ws = torch::empty({N * (share_words + hist_words + 1)},
-                         logits.options().dtype(torch::kInt32));
-  Share* share = reinterpret_cast<Share*>(ws.data_ptr<int>());
-  uint32_t* hist =
-      reinterpret_cast<uint32_t*>(ws.data_ptr<int>()) + N * share_words;
-  uint32_t* tau = hist + N * hist_words;
+  const long row_words =
+      no_filter ? share_words
+                : share_words + split * TOPS + sizeof(Plan) / 4 + hist_words;
+  auto ws = torch::empty({N * row_words}, logits.options().dtype(torch::kInt32));
+  int* w = ws.data_ptr<int>();
+  Share* share = reinterpret_cast<Share*>(w);
+  Plan* plans = reinterpret_cast<Plan*>(w + N * share_words);
+  float* tops = reinterpret_cast<float*>(plans + N);
+  uint32_t* hist = reinterpret_cast<uint32_t*>(tops + N * split * TOPS);
   const T* x = (const T*)logits.data_ptr();
   const float* temp = temperature.data_ptr<float>();
   TORCH_CHECK(N * split < (1L << 31), "too many rows");
   const dim3 grid((unsigned)(N * split)), block(SNT);
+  const int* k = top_k.data_ptr<int>();
+  const float* p = top_p.data_ptr<float>();
+  auto pass = [&](auto kern) {
+    kern<<<grid, block, 0, stream>>>(share, tops, hist, hist_words, plans, x,
+                                     temp, seed, seed_ptr, V, split);
+  };
+  auto plan = [&](int digit) {
+    sample_plan_kernel<T><<<dim3((unsigned)N), block, 0, stream>>>(
+        plans, hist, hist_words, share, tops, temp, k, p, digit, V, split);
+  };
   if (no_filter) {
-    sample_pass_kernel<T, 0><<<grid, block, 0, stream>>>(
-        share, hist, 0, tau, x, temp, seed, seed_ptr, V, split);
+    pass(sample_pass_kernel<T, 0>);
   } else {
-    const int* k = top_k.data_ptr<int>();
-    const float* p = top_p.data_ptr<float>();
-    sample_pass_kernel<T, 1><<<grid, block, 0, stream>>>(
-        share, hist, hist_words, tau, x, temp, seed, seed_ptr, V, split);
-    for (int d = 0; d < digits; ++d)
+    pass(sample_pass_kernel<T, 1>);
+    plan(-1);
+    for (int d = 0; d < digits; ++d) {
       sample_digit_kernel<T><<<grid, block, 0, stream>>>(
-          hist, hist_words, share, x, temp, k, p, d, V, split);
-    sample_tau_kernel<T><<<dim3(N), block, 0, stream>>>(
-        tau, hist, hist_words, share, temp, k, p, digits, V, split);
-    sample_pass_kernel<T, 2><<<grid, block, 0, stream>>>(
-        share, hist, hist_words, tau, x, temp, seed, seed_ptr, V, split);
+          hist, hist_words, plans, x, temp, d, V, split);
+      plan(d);
+    }
+    pass(sample_pass_kernel<T, 2>);
   }
   sample_merge_kernel<T><<<dim3(N), dim3(64), 0, stream>>>(
       out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(), share, x,
