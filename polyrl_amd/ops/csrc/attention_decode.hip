@@ -3,24 +3,45 @@
 // Reference capability: the paged/continuous-batching decode attention the
 // reference reaches through its inference engine.
 //
-// MI355X-first design: the op is HBM-bound (each step reads the whole KV
-// history once), so the kernel is built around streaming K/V at 16 B/lane:
-//   * grid = (B * Hk) workgroups (batch x kv-head); 4 waves each.
-//   * a wave's 64 lanes split into GROUPS = 64/(D/8) lane-groups; each group
-//     owns one key per iteration, lane j of a group loads K[t, hk, 8j:8j+8]
-//     (one bf16x8 = 16 B -> coalesced 1 KiB per wave instruction).
-//   * q(x G heads) is register-resident; scores via an in-group shfl_xor
-//     reduce; online softmax state (m, l, o[8]) per (group, head) in VGPRs.
-//   * partial states merge wave-internally by shfl (groups are lane slices),
-//     then across the 4 waves through LDS.
-// GQA group size G (= Hq/Hk) and head_dim D are compile-time (guide rule 20:
-// runtime-indexed register arrays spill to scratch), dispatched below.
+// A block serves one key/value head of one sequence (or a stretch of its
+// context) for all G query heads of the group; each of its four waves takes
+// 32 keys at a time, on its own: no barrier until the waves' results meet.
+//   * S^T = K Q^T on v_mfma_f32_16x16x32_bf16, 16 keys x 16 head columns (G of
+//     them in use): a lane's K fragment is 16 bytes of one cached row, loaded
+//     straight from the page, and its accumulators are keys of ONE head, so
+//     maximum and sum take two lane exchanges per 32 keys.
+//   * O^T += V^T P^T: V rows go through 8 KiB of LDS of the wave's own and come
+//     back turned (ds_read_b64_tr_b16); the weights are the operand as they
+//     stand in the accumulators.  They stay as exact as 32-bit ones: each is
+//     the sum of two bf16 numbers, and both are multiplied.
+// What bounds it: reading K and V once.  (With per-key dot products, shuffles
+// and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
+// at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
+// tokens, 32/8 heads of 128, 59.5 -> 44.6 us; 33 rows of 1900 .. 8192, 28/4
+// heads, 264 -> 86 us (4.1 TB/s).
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-#include "common.h"
+#include "attention_tile.h"
 
-template <int D, int G>
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+constexpr int DEC_KEYS = 32;          // keys of a wave's round
+constexpr int DEC_HEADS = 8;          // most query heads of a group
+
+// the larger / the sum of the four lanes l, l+16, l+32, l+48
+DEV_INLINE float quad_max(float x) {
+  const auto p = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return half_max(fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1])));
+}
+DEV_INLINE float quad_sum(float x) {
+  const auto p = __builtin_amdgcn_permlane16_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return half_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
+}
+
+template <int D>
 __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
     bf16_t* __restrict__ out,              // (B, Hq, D)
     float* __restrict__ partial,           // (B, Hq, S, D+2) when nsplit>1
@@ -31,152 +52,184 @@ __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
     const int* __restrict__ context_lens,  // (B,)
     int Hq, int Hk, int page_size, int max_pages, float scale, long ldq,
     int nsplit) {
-  constexpr int GL = D / 8;        // lanes per key group
-  constexpr int KPW = 64 / GL;     // keys per wave per iteration
-  constexpr int NW = 4;            // waves per block
-  // flash-decoding context split (PMC-measured: at B*Hk < ~1024 blocks
-  // the kernel is occupancy/latency-bound — 1 wave/SIMD cannot hide the
-  // online-update chain; splitting the context across nsplit blocks per
-  // (b, hk) restores the wave supply, a tiny merge kernel combines)
+  typedef AttnTile<D> T;
+  constexpr int KS = D / 32, DT = D / 16;
+  constexpr int RPI = 64 / T::GR;          // V rows of one load instruction
+  constexpr int NV = DEC_KEYS / RPI;
+  __shared__ __attribute__((aligned(16))) char lds[4][DEC_KEYS * D * 2];
+  __shared__ float ml[4][DEC_HEADS][2];
+
   const int b = blockIdx.x / (Hk * nsplit);
   const int rem = blockIdx.x % (Hk * nsplit);
   const int hk = rem / nsplit;
   const int sp = rem % nsplit;
+  const int G = Hq / Hk;
   const int L = context_lens[b];
-  const int Lc = (L + nsplit - 1) / nsplit;
+  // a stretch per block, in whole rounds of a wave
+  const int Lc = ((L + nsplit - 1) / nsplit + DEC_KEYS - 1) / DEC_KEYS *
+                 DEC_KEYS;
   const int cbeg = sp * Lc;
-  const int cend = (cbeg + Lc < L) ? (cbeg + Lc) : L;
+  const int cend = min(cbeg + Lc, L);
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int grp = lane / GL;       // key-group within wave
-  const int gl = lane % GL;        // lane within group
-  const int d0 = gl * 8;           // this lane's d-slice
+  const int wid = wave_id();
+  const int l15 = lane & 15, lhi = lane >> 4;
 
-  // q registers: G heads x 8 elems (this lane's slice), pre-scaled
-  float qr[G][8];
+  // Q of head l15 (columns past the group repeat its last head)
+  bf16x8_t qf[KS];
+  {
+    const bf16_t* qp = q + (long)b * ldq +
+                       (long)(hk * G + min(l15, G - 1)) * D + lhi * 8;
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    const bf16x8 qv = *reinterpret_cast<const bf16x8*>(
-        q + ((long)b * ldq + (long)(hk * G + h) * D + d0));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qr[h][j] = bf2f(qv.v[j]) * scale;
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
   }
-
-  // online-softmax state per head.  m starts at a large negative FINITE
-  // value: merging two empty partials with -inf init would compute
-  // exp(-inf - -inf) = NaN; with -1e30 the empty state contributes
-  // exp(0)*0 = 0 and any real score immediately dominates the max.
-  float m[G], l[G], o[G][8];
+  const float s2 = scale * 1.4426950408889634f;
+  // m starts at a large negative FINITE value: an empty stretch then weighs
+  // 2^(m - largest) = 0 in the merges instead of inf - inf
+  float m_run = -1e30f, l_run = 0.f;
+  f32x4_t o[DT];
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m[h] = -1e30f;
-    l[h] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[h][j] = 0.f;
-  }
+  for (int dt = 0; dt < DT; ++dt) o[dt] = {0.f, 0.f, 0.f, 0.f};
 
-  const int kv_stride = Hk * D;  // row stride inside a page slot
+  const long kv_stride = (long)Hk * D;
   const int* ptab = page_table + (long)b * max_pages;
+  char* vs = lds[wid];
+  // turned reads of V: rows 4 * lhi + l15 / 4 (+16), columns 16 dt + ..
+  const int ra = 4 * lhi + (l15 >> 2), rb = ra + 16;
+  const int vg = (l15 & 3) >> 1;
+  const int va = ra * (2 * D) + ((vg ^ T::swz(ra)) << 4) + (l15 & 1) * 8;
+  const int vb = rb * (2 * D) + ((vg ^ T::swz(rb)) << 4) + (l15 & 1) * 8;
+  const int vrow = lane / T::GR, vcol = lane % T::GR;
 
-  // stream keys: token t = cbeg + iter*NW*KPW + wid*KPW + grp
-  for (int t0 = cbeg + wid * KPW + grp; t0 < cend; t0 += NW * KPW) {
-    const int page = ptab[t0 / page_size];
-    const long slot = (long)page * page_size + (t0 % page_size);
-    const bf16_t* kp = k_cache + slot * kv_stride + hk * D + d0;
-    const bf16_t* vp = v_cache + slot * kv_stride + hk * D + d0;
-    const bf16x8 kv = *reinterpret_cast<const bf16x8*>(kp);
-    const bf16x8 vv = *reinterpret_cast<const bf16x8*>(vp);
-    float kf[8], vf[8];
+  // cache row of key t0 + lane % 32 (keys past the stretch: its last)
+  auto slot_of = [&](int t0) {
+    const int t = min(t0 + (lane & 31), cend - 1);
+    const int pg = t / page_size;
+    return ptab[pg] * page_size + (t - pg * page_size);
+  };
+  int t0 = cbeg + wid * DEC_KEYS;
+  int slot = t0 < cend ? slot_of(t0) : 0;
+  for (; t0 < cend; t0 += 4 * DEC_KEYS) {
+    bf16x8_t kf[2][KS];
+    i32x4_t vv[NV];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      kf[j] = bf2f(kv.v[j]);
-      vf[j] = bf2f(vv.v[j]);
+    for (int n = 0; n < 2; ++n) {
+      const bf16_t* kp = k_cache + __shfl(slot, n * 16 + l15, 64) * kv_stride +
+                         hk * D + lhi * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        kf[n][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
     }
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float s = 0.f;
+    for (int i = 0; i < NV; ++i)
+      vv[i] = *reinterpret_cast<const i32x4_t*>(
+          v_cache + __shfl(slot, i * RPI + vrow, 64) * kv_stride + hk * D +
+          vcol * 8);
+    if (t0 + 4 * DEC_KEYS < cend) slot = slot_of(t0 + 4 * DEC_KEYS);
+
+    // ---- S^T: 32 keys x 16 heads; this lane: head l15, keys 4 lhi + r -------
+    f32x4_t s[2];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += qr[h][j] * kf[j];
-      // reduce over the GL lanes of this group
+    for (int n = 0; n < 2; ++n) {
+      s[n] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int off = GL / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-      // online update (score s is group-uniform)
-      const float mn = fmaxf(m[h], s);
-      const float alpha = __expf(m[h] - mn);
-      const float pt = __expf(s - mn);
-      l[h] = l[h] * alpha + pt;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[h][j] = o[h][j] * alpha + pt * vf[j];
-      m[h] = mn;
+      for (int ks = 0; ks < KS; ++ks)
+        s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[n][ks], qf[ks], s[n],
+                                                       0, 0, 0);
     }
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[n][r] *= s2;
+    if (t0 + DEC_KEYS > cend) {
+      const int last = cend - 1 - t0;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n * 16 + 4 * lhi + r > last) s[n][r] = -INFINITY;
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[n][r]);
+    const float mn = fmaxf(m_run, quad_max(mx));
+    const float alpha = exp2_hw(m_run - mn);
+    m_run = mn;
+    l_run *= alpha;
+    // weights as hi + lo, both bf16: the remainder is below 2^-17 of a weight
+    bf16x8_t hi, lo;
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = exp2_hw(s[n][r] - mn);
+        l_run += p;
+        hi[4 * n + r] = (__bf16)p;
+        lo[4 * n + r] = (__bf16)(p - (float)hi[4 * n + r]);
+      }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
+
+    // ---- V rows into the wave's LDS, turned fragments back --------------------
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int r = i * RPI + vrow;
+      *reinterpret_cast<i32x4_t*>(vs + r * (2 * D) +
+                                  ((vcol ^ T::swz(r)) << 4)) = vv[i];
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const i16x4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_i16x4_p)(vs + (va ^ (dt << 5))));
+      const i16x4_t c = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_i16x4_p)(vs + (vb ^ (dt << 5))));
+      const bf16x8_t vt = __builtin_bit_cast(
+          bf16x8_t, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, hi, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, lo, o[dt], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
+  l_run = quad_sum(l_run);
 
-  // ---- merge the KPW groups within each wave (shfl across lane slices) ----
+  // ---- the four waves' shares meet in LDS ------------------------------------
+  if (l15 < G) {
+    float* mine = reinterpret_cast<float*>(vs) + l15 * D + lhi * 4;
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-#pragma unroll
-    for (int step = 1; step < KPW; step <<= 1) {
-      const int src = lane ^ (step * GL);
-      const float om = __shfl(m[h], src, 64);
-      const float ol = __shfl(l[h], src, 64);
-      float ov[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ov[j] = __shfl(o[h][j], src, 64);
-      const float mn = fmaxf(m[h], om);
-      const float a = __expf(m[h] - mn), bta = __expf(om - mn);
-      l[h] = l[h] * a + ol * bta;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[h][j] = o[h][j] * a + ov[j] * bta;
-      m[h] = mn;
-    }
-  }
-
-  // ---- merge the 4 waves through LDS (group 0 of each wave holds state) ---
-  // LDS layout: [NW][G][GL][10] floats: 8 o + m + l  (D=128,G<=8: 20.5 KiB)
-  __shared__ float mrg[NW][G][GL][10];
-  if (grp == 0) {
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) mrg[wid][h][gl][j] = o[h][j];
-      mrg[wid][h][gl][8] = m[h];
-      mrg[wid][h][gl][9] = l[h];
+    for (int dt = 0; dt < DT; ++dt)
+      *reinterpret_cast<f32x4_t*>(mine + dt * 16) = o[dt];
+    if (lhi == 0) {
+      ml[wid][l15][0] = m_run;
+      ml[wid][l15][1] = l_run;
     }
   }
   __syncthreads();
-  // wave 0, group 0 merges and writes
-  if (wid == 0 && grp == 0) {
+  for (int i = threadIdx.x; i < G * D; i += 256) {
+    const int h = i / D, d = i % D;
+    float gm = ml[0][h][0];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float gm = -INFINITY;
+    for (int w = 1; w < 4; ++w) gm = fmaxf(gm, ml[w][h][0]);
+    float l = 0.f, acc = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) gm = fmaxf(gm, mrg[w][h][gl][8]);
-      float gl_sum = 0.f, go[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) go[j] = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const float a = __expf(mrg[w][h][gl][8] - gm);
-        gl_sum += mrg[w][h][gl][9] * a;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) go[j] += mrg[w][h][gl][j] * a;
-      }
-      if (nsplit == 1) {
-        const float inv = (gl_sum > 0.f) ? 1.0f / gl_sum : 0.f;
-        bf16x8 ov;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ov.v[j] = f2bf(go[j] * inv);
-        *reinterpret_cast<bf16x8*>(
-            out + (((long)b * Hq + hk * G + h) * D + d0)) = ov;
-      } else {
-        float* pp = partial +
-            ((((long)b * Hq + hk * G + h) * nsplit) + sp) * (D + 2);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pp[d0 + j] = go[j];
-        if (gl == 0) {
-          pp[D] = gm;
-          pp[D + 1] = gl_sum;
-        }
+    for (int w = 0; w < 4; ++w) {
+      const float a = exp2_hw(ml[w][h][0] - gm);
+      l += ml[w][h][1] * a;
+      acc += reinterpret_cast<const float*>(lds[w])[i] * a;
+    }
+    const long row = (long)b * Hq + hk * G + h;
+    if (nsplit == 1) {
+      out[row * D + d] = f2bf(l > 0.f ? acc / l : 0.f);
+    } else {
+      float* pp = partial + (row * nsplit + sp) * (D + 2);
+      pp[d] = acc;
+      if (d == 0) {
+        pp[D] = gm * 0.6931471805599453f;
+        pp[D + 1] = l;
       }
     }
   }
@@ -192,17 +245,17 @@ __global__ void paged_decode_merge_kernel(
   const long row = blockIdx.x;             // b*Hq + hq
   const int lane = threadIdx.x;
   const float* base = partial + row * (long)nsplit * (D + 2);
-  float gm = -1e30f;
-  for (int sp = 0; sp < nsplit; ++sp)
-    gm = fmaxf(gm, base[sp * (D + 2) + D]);
-  float gl_sum = 0.f;
+  // stretch lane: its maximum and sum (nsplit <= 64)
+  const float m = lane < nsplit ? base[lane * (D + 2) + D] : -1e30f;
+  const float w = __expf(m - wave_reduce_max(m));
+  const float gl_sum = wave_reduce_sum(
+      lane < nsplit ? base[lane * (D + 2) + D + 1] * w : 0.f);
   float acc[EPL];
 #pragma unroll
   for (int j = 0; j < EPL; ++j) acc[j] = 0.f;
   for (int sp = 0; sp < nsplit; ++sp) {
     const float* pp = base + sp * (D + 2);
-    const float a = __expf(pp[D] - gm);
-    gl_sum += pp[D + 1] * a;
+    const float a = __shfl(w, sp, 64);
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
       acc[j] += pp[lane + j * 64] * a;
@@ -215,10 +268,9 @@ __global__ void paged_decode_merge_kernel(
 
 // EXPERIMENTAL round-3 candidate (default OFF, opt-in POLYRL_DECODE_MFMA=1
 // for on-box A/B): MFMA S/PV decode — moves the per-key dot products and
-// P·V off the VALU (PMC: decode is exactly VALU-throughput-bound at
-// B*Hk>=1024, profiles/PROFILES.md).  Textual include: -fno-gpu-rdc builds
+// P·V off the VALU.  Textual include: -fno-gpu-rdc builds
 // cannot launch kernels defined in another TU.  Falls back to the
-// production VALU kernel for (D, G) combos the prototype doesn't cover.
+// production kernel for (D, G) combos the prototype doesn't cover.
 #include "experimental/attention_decode_mfma.hip"
 
 static bool use_mfma_decode() {
@@ -238,31 +290,25 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
                        hipStream_t stream) {
   const int G = Hq / Hk;
   const long B = q.size(0);
-  // flash-decoding context split: pick nsplit from the grid size alone
-  // (L-independent => hipGraph-replay-safe).  Target >= 1024 blocks so
-  // the latency-bound online-update chain has wave supply; PMC measured
-  // B=32 x Hk=8 (256 blocks) at 7x the KV-read bound from occupancy.
-  int nsplit = 1;
+  // Context split: from the sizes alone, not from the lengths on the device,
+  // so that a captured graph may replay it with longer contexts.  At least
+  // 1024 blocks (four per CU: the loads in flight cover the memory's latency),
+  // but no stretch under 128 keys (a round of the four waves) of the longest
+  // context that the page table holds: there the merging launch costs more
+  // than the split gains (37 cached tokens: 16.8 us in 16 stretches, 6.8 in
+  // one).
   const long base_blocks = B * Hk;
-  if (base_blocks < 1024) {
-    nsplit = (int)((1024 + base_blocks - 1) / base_blocks);
-    if (nsplit > 16) nsplit = 16;
-  }
+  const long most = (long)max_pages * page_size;
+  int nsplit = 1;
+  if (base_blocks < 1024)
+    nsplit = (int)std::max<long>(
+        1, std::min<long>({(1024 + base_blocks - 1) / base_blocks, 16,
+                           (most + 127) / 128}));
+  torch::Tensor ws;                     // per call: any stream, any capture
   float* ppart = nullptr;
   if (nsplit > 1) {
-    // Thread-local grow-only workspace: a fresh torch::empty every call
-    // would allocate DURING hipGraph capture (the engine's graphed decode
-    // wraps this op) and can deadlock/fail the capture.  The warmup pass
-    // that precedes every capture (rollout/engine.py::_decode_graphed)
-    // sizes this buffer on the same thread, so the captured call reuses a
-    // stable pointer and replays are correct (partials are written then
-    // merged within one launch sequence).
-    static thread_local torch::Tensor ws;
-    const long need = B * Hq * (long)nsplit * (D + 2);
-    if (!ws.defined() || ws.numel() < need ||
-        ws.device() != q.device()) {
-      ws = torch::empty({need}, q.options().dtype(torch::kFloat32));
-    }
+    ws = torch::empty({B * Hq * (long)nsplit * (D + 2)},
+                      q.options().dtype(torch::kFloat32));
     ppart = ws.data_ptr<float>();
   }
   const dim3 grid(B * Hk * nsplit), block(256);
@@ -285,20 +331,11 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
     } else if constexpr (D == 64) {
       if (G == 4) { args(paged_decode_attn_mfma_kernel<64, 4>); return; }
     }
-    // uncovered combo: fall through to the production VALU kernel
+    // uncovered combo: fall through to the production kernel
   }
-  switch (G) {
-    case 1: args(paged_decode_attn_kernel<D, 1>); break;
-    case 2: args(paged_decode_attn_kernel<D, 2>); break;
-    case 3: args(paged_decode_attn_kernel<D, 3>); break;
-    case 4: args(paged_decode_attn_kernel<D, 4>); break;
-    case 5: args(paged_decode_attn_kernel<D, 5>); break;
-    case 6: args(paged_decode_attn_kernel<D, 6>); break;
-    case 7: args(paged_decode_attn_kernel<D, 7>); break;
-    case 8: args(paged_decode_attn_kernel<D, 8>); break;
-    default:
-      TORCH_CHECK(false, "GQA group size ", G, " unsupported (1..8)");
-  }
+  TORCH_CHECK(G >= 1 && G <= DEC_HEADS, "GQA group size ", G,
+              " unsupported (1..8)");
+  args(paged_decode_attn_kernel<D>);
 }
 
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,

@@ -129,3 +129,40 @@ def test_backward(name, hq, hk, d, causal):
         for name_, g, w, m in zip(("dq", "dk", "dv"), got, want, size):
             off = (g[a].double() - w).abs() - 2 ** -8 * (m + w.abs())
             assert off.max() <= 0, (name_, lens[i], off.max())
+
+
+@pytest.mark.parametrize("page_size,wide", [(16, False), (16, True), (1, False),
+                                            (7, True)])
+@pytest.mark.parametrize("hq,hk,d", [(8, 8, 128), (7, 1, 128), (12, 4, 64),
+                                     (16, 2, 64), (28, 4, 128), (5, 1, 64)])
+def test_decode(hq, hk, d, page_size, wide):
+    """Paged decode at the edges of its 32-key rounds and 128-key stretches;
+    ``wide``: a page table far wider than the contexts (a captured graph's),
+    which divides them further.  The weights are as exact as 32-bit ones, so
+    an entry is off by its rounding to bf16 and 2^-14 of its terms."""
+    torch.manual_seed(9)
+    lens = [1, 31, 32, 33, 127, 128, 129, 300, 1025, 2]
+    need = [-(-n // page_size) for n in lens]
+    pages = torch.randperm(sum(need), device=DEV).int()
+    table = torch.zeros(len(lens), max(need) * (4 if wide else 1),
+                        dtype=torch.int32, device=DEV)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    k, v = (torch.randn(sum(need), page_size, hk, d, device=DEV).bfloat16()
+            for _ in range(2))
+    q = torch.randn(len(lens), (hq + 2) * d, device=DEV).bfloat16()[
+        :, :hq * d].unflatten(1, (hq, d))
+    out = ops.paged_attention_decode(
+        q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+        d ** -0.5)
+    for i, n in enumerate(lens):
+        p = table[i, :need[i]].long()
+        kk = heads(k[p].view(-1, hk, d)[:n].double(), hq)
+        vv = heads(v[p].view(-1, hk, d)[:n].double(), hq)
+        want, _ = attend(q[i:i + 1].double(), kk, vv, n - 1, True, d ** -0.5)
+        mass, _ = attend(q[i:i + 1].double(), kk, vv.abs(), n - 1, True,
+                         d ** -0.5)
+        bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
+        assert ((out[i:i + 1].double() - want).abs() <= bound).all(), n
