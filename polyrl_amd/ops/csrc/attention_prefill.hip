@@ -87,6 +87,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
 
   FragAt<D> at;
   const float s2 = scale * 1.4426950408889634f;    // scores in powers of two
+  const float hidden = s2 >= 0.f ? -INFINITY : INFINITY;
   float m_run = -1e30f, l_run = 0.f;               // l: this lane's keys only
   f32x16_t o[DT];
 #pragma unroll
@@ -151,15 +152,23 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
         for (int n = 0; n < 2; ++n)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            if (n * 32 + acc_row(r) > last) s[n][r] = -INFINITY;
+            if (n * 32 + acc_row(r) > last) s[n][r] = hidden;
       }
       // ---- online softmax -----------------------------------------------------
+      // (largest score: the smallest product where the scale is negative)
       float mx = s[0][0];
+      if (s2 >= 0.f) {
 #pragma unroll
-      for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < 2; ++n)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
-      const float mn = fmaxf(m_run, half_max(mx) * s2);
+          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mx = fminf(mx, s[n][r]);
+      }
+      const float mn = fmaxf(m_run, half_max(mx * s2));
       // m_run may lag behind the maximum by 2^SLACK: weights up to 2^SLACK
       // lose nothing in 32-bit sums and bf16 operands, and with random rows
       // most tiles move some row's maximum a little
