@@ -44,6 +44,7 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include "attention_tile.h"
 #include "seq_common.h"
 
 // tanh through the hardware exponential and reciprocal: 1 - 2 / (1 + e^2x),
@@ -53,9 +54,7 @@ DEV_INLINE float tanhf_fast(float x) {
                          1.f + __builtin_amdgcn_exp2f(2.8853900817779268f * x));
 }
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) int i32x4_t;
 
 constexpr int GQA_MAX_REL = 256; // bias-table rows held in LDS
 constexpr int GQA_XCDS = 8;      // accelerator dies, each with its own L2
@@ -370,6 +369,248 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
   }
 }
 
+// ------------------------------------------------- softmax, equal heads of 64, 128
+// Keys and values of the same size, 64 or 128, and plain softmax weights (the
+// grouped-query layers of every preset but the distance-bias and the sigmoid
+// ones): the same walk on 32-row units and 64-key tiles.  A wave owns 32 rows
+// of one head; a block is four such units of one row tile and one key/value
+// head, heads of the group first, so four heads share each K and V tile where
+// the general kernel fetches it for every head.  Values stay row-major in LDS
+// and are read turned (layouts and operands: attention_tile.h); tiles are
+// fetched 16 bytes a lane, whole rows together, where the general kernel
+// collects values 8 bytes at a time, one row per lane.  The next K tile is in
+// flight during a tile's score products, the next V tile during its value
+// products, in the same registers.  Measured, eight prompts of 1200 .. 2048
+// tokens, window 1024, 32/8 heads of 64: 547 us in the general kernel, 151 here.
+template <int D>
+__global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
+    bf16_t* __restrict__ out,            // (N, H*D), row stride ldo
+    const bf16_t* __restrict__ q,        // (N, H*D)
+    const bf16_t* __restrict__ cache,    // (slots, 2*G*D)
+    const int* __restrict__ page_table, int max_pages,
+    const int* __restrict__ seq_of_tok, const int* __restrict__ positions,
+    const int* __restrict__ tile_n0, const int* __restrict__ tile_cnt,
+    int ntiles_rows, int nparts, const bf16_t* __restrict__ gate, long ldg,
+    int H, int G, int page_size, int window, int keep, float scale,
+    const float* __restrict__ sink, float qt_coef, int qt_every, int chunk,
+    long ldo, float out_scale) {
+  typedef AttnTile<D> T;
+  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
+  __shared__ int slot_s[2][ATILE];       // cache rows of a tile's keys
+  constexpr int KS = D / 16, DT = D / 32;
+  constexpr float L2E = 1.4426950408889634f, SLACK = 6.f;
+
+  const int per = H / G;                 // query heads per key/value head
+  const int item = die_item(ntiles_rows * G * nparts);
+  if (item >= ntiles_rows * G * nparts) return;
+  const int g = item / (ntiles_rows * nparts);
+  // later row tiles see more keys: they start first
+  const int tile = ntiles_rows - 1 - item / nparts % ntiles_rows;
+  const int n0 = uniform(tile_n0[tile]);
+  const int cnt = uniform(tile_cnt[tile]);
+  const int* ptab = page_table + (long)uniform(seq_of_tok[n0]) * max_pages;
+  const int pos0 = uniform(positions[n0]);
+  const int pmax = pos0 + cnt - 1;
+
+  const int lane = threadIdx.x & 63;
+  const int wid = wave_id();
+  const int unit = item % nparts * 4 + wid;        // (row half, head)
+  const int w0 = unit / per * 32;                  // this wave's first row
+  const bool busy = unit < 2 * per && w0 < cnt;
+  const int h = busy ? g * per + unit % per : g * per;
+
+  // first windowed key of the row at position p
+  auto row_lo = [&](int p) {
+    int lo = p - window + 1 > 0 ? p - window + 1 : 0;
+    if (chunk > 0) lo = max(lo, p / chunk * chunk);
+    return lo;
+  };
+  // the block's walk: kept keys before its first row's window, then from
+  // there to the last row's position
+  const int kmin = row_lo(pos0);
+  const int nk = keep < kmin ? keep : kmin;
+  const int nkt = (nk + ATILE - 1) / ATILE;
+  const int ntiles = nkt + (pmax - kmin) / ATILE + 1;
+  auto tile_t0 = [&](int ti) {
+    return ti < nkt ? ti * ATILE : kmin + (ti - nkt) * ATILE;
+  };
+  auto tile_jmax = [&](int ti) { return ti < nkt ? nk - 1 : pmax; };
+  // cache row of a tile's key i (keys past the tile's last: that one)
+  auto slot_of = [&](int ti, int i) {
+    const int j = min(tile_t0(ti) + i, tile_jmax(ti));
+    const int pg = j / page_size;
+    return ptab[pg] * page_size + (j - pg * page_size);
+  };
+  if (wid < 2 && wid < ntiles) slot_s[wid][lane] = slot_of(wid, lane);
+
+  const int ri = min(w0 + (lane & 31), cnt - 1);   // this lane's row
+  const int rpos = pos0 + ri, rlo = row_lo(rpos);
+  const int wp0 = pos0 + w0, wp1 = min(wp0 + 31, pmax);   // the wave's rows
+  const int wlo0 = row_lo(wp0), wlo = row_lo(wp1);
+  bf16x8_t qf[KS];
+  frag_global<D>(qf, q + ((long)(n0 + ri) * H + h) * D);
+  float s2 = scale * L2E;                // scores in powers of two
+  if (qt_coef != 0.f)
+    s2 *= 1.f + qt_coef * logf((float)((rpos + 1) / qt_every + 1));
+  // running maximum of the row, in powers of two; each of its two lanes sums
+  // its own keys
+  float m_run = sink ? fmaxf(sink[h] * L2E, -1e30f) : -1e30f;
+  float l_run = sink && lane < 32 ? exp2_hw(sink[h] * L2E - m_run) : 0.f;
+  f32x16_t o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+
+  FragAt<D> at;
+  const long row = 2L * G * D;
+  const bf16_t* kb = cache + (long)g * D;
+  const bf16_t* vb = kb + (long)G * D;
+  i32x4_t reg[T::LOADS];                 // the tile in flight, K and V in turn
+  auto fetch = [&](const bf16_t* from, int ti) {
+#pragma unroll
+    for (int i = 0; i < T::LOADS; ++i) {
+      const int a = threadIdx.x + i * 256;
+      reg[i] = *reinterpret_cast<const i32x4_t*>(
+          from + slot_s[ti & 1][a / T::GR] * row + a % T::GR * 8);
+    }
+  };
+  __syncthreads();
+  fetch(kb, 0);
+  T::store(lds[0][0], reg);
+  fetch(vb, 0);
+  T::store(lds[0][1], reg);
+  wait_loads();
+  __syncthreads();
+
+  for (int ti = 0; ti < ntiles; ++ti) {
+    const int buf = ti & 1;
+    const int t0 = tile_t0(ti), jmax = tile_jmax(ti);
+    const char* ks_ = lds[buf][0];
+    const char* vs_ = lds[buf][1];
+    at.renew();
+    // a key of the tile that some row of the wave sees
+    const bool work = busy && t0 <= wp1 &&
+                      (ti < nkt || min(t0 + ATILE - 1, jmax) >= wlo0 ||
+                       t0 < keep);
+    const bool more = ti + 1 < ntiles;
+    if (more) fetch(kb, ti + 1);
+    f32x16_t s[2];
+    if (work) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[0][r] = 0.f, s[1][r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+          s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_rows<D>(ks_, at, n, ks), qf[ks], s[n], 0, 0, 0);
+      SCHED_LDS(6);
+#pragma unroll
+      for (int i = 0; i < 2 * KS - 6; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(1);
+      }
+      SCHED_MFMA(6);
+    }
+    // into the other buffer (its readers passed the last barrier)
+    if (more) {
+      T::store(lds[buf ^ 1][0], reg);
+      fetch(vb, ti + 1);
+    }
+    if (work) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] *= s2;
+      if (!(t0 + ATILE - 1 <= min(wp0, jmax) && t0 >= wlo)) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int j = t0 + n * 32 + acc_row(r);
+            const bool live = j <= jmax && j <= rpos && (j >= rlo || j < keep);
+            if (!live) s[n][r] = -INFINITY;
+          }
+      }
+      float mx = s[0][0];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
+      const float mn = fmaxf(m_run, half_max(mx));
+      if (__any(mn > m_run + SLACK)) {     // weights up to 2^SLACK lose nothing
+        const float alpha = exp2_hw(m_run - mn);
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+        m_run = mn;
+      }
+      float sum = 0.f;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          s[n][r] = exp2_hw(s[n][r] - m_run);
+          sum += s[n][r];
+        }
+      l_run += sum;
+      // ---- O^T += V^T P^T ------------------------------------------------------
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const bf16x8_t p = acc_operand(s[st >> 1], st & 1);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(vs_, at, dt, st), p, o[dt], 0, 0, 0);
+      }
+      SCHED_LDS(8);
+#pragma unroll
+      for (int i = 0; i < 4 * DT - 4; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(2);
+      }
+      SCHED_MFMA(4);
+    }
+    if (more) T::store(lds[buf ^ 1][1], reg);
+    // (the rows of this tile were last looked up before the last barrier)
+    if (wid == 0 && ti + 2 < ntiles) slot_s[buf][lane] = slot_of(ti + 2, lane);
+    __syncthreads();
+  }
+
+  // ---- out: 32 rows turned through LDS to whole rows -------------------------
+  const float l = half_sum(l_run);
+  float inv = 1.f / l * out_scale;
+  if (gate) inv *= sigmoidf_acc(bf2f(gate[(long)(n0 + ri) * ldg + h]));
+  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      bf16x4 w;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w.v[t] = f2bf(o[dt][4 * i + t] * inv);
+      const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
+      *reinterpret_cast<bf16x4*>(
+          mine + (lane & 31) * (2 * D) +
+          (((d >> 3) ^ T::swz(lane & 31)) << 4) + (d & 4) * 2) = w;
+    }
+  __syncthreads();
+  if (!busy) return;
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    const int a = lane + i * 64;
+    const int r = a / T::GR, gr = a % T::GR;
+    if (w0 + r < cnt)
+      *reinterpret_cast<i32x4_t*>(out + (n0 + w0 + r) * ldo + (long)h * D +
+                                  gr * 8) =
+          *reinterpret_cast<const i32x4_t*>(mine + r * (2 * D) +
+                                            ((gr ^ T::swz(r)) << 4));
+  }
+}
+
 void gqa_attention_check(torch::Tensor out, torch::Tensor q,
                          torch::Tensor cache, torch::Tensor page_table,
                          torch::Tensor seq_of_tok, torch::Tensor positions,
@@ -459,6 +700,39 @@ void seq_gqa_window_attention_mfma(
   if (v_rot) {
     sums = torch::empty({q.size(0), H * Dv}, q.options().dtype(torch::kFloat32));
     o32 = sums.data_ptr<float>();
+  }
+  // Shared tiles of a head group where the kernel for them serves the call
+  // (above; it stores 16 bytes at a time); the general kernel keeps the rest:
+  // other sizes, biases, caps, sigmoid weights, values to turn back.
+  auto by16 = [](const torch::Tensor& t) {
+    return ((uintptr_t)t.data_ptr() & 15) == 0;
+  };
+  if (D == Dv && (D == 64 || D == 128) && !has_rel && softcap <= 0.0 &&
+      !has_hb && !sigmoid_weights && !v_rot && by16(out) && by16(q) &&
+      by16(cache) && out.stride(0) % 8 == 0) {
+    const int nparts = (int)(2 * (H / G) + 3) / 4;
+    const long items = (long)ntiles * G * nparts;
+    const long blocks = (items + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
+    TORCH_CHECK(blocks < (1L << 31), "grid too large");
+    auto launch = [&](auto kern) {
+      kern<<<dim3((unsigned)blocks), dim3(256), 0,
+             at::hip::getCurrentHIPStream()>>>(
+          (bf16_t*)out.data_ptr(), (const bf16_t*)q.data_ptr(),
+          (const bf16_t*)cache.data_ptr(), page_table.data_ptr<int>(),
+          (int)page_table.size(1), seq_of_tok.data_ptr<int>(),
+          positions.data_ptr<int>(), tile_n0.data_ptr<int>(),
+          tile_cnt.data_ptr<int>(), ntiles, nparts,
+          has_gate ? (const bf16_t*)gate.data_ptr() : nullptr,
+          has_gate ? gate.stride(0) : 0, (int)H, (int)G, (int)cache.size(1),
+          (int)window, (int)keep_first, (float)scale,
+          has_sink ? sink.data_ptr<float>() : nullptr, (float)q_temp_coef,
+          (int)q_temp_every, (int)chunk, (long)out.stride(0),
+          (float)out_scale);
+    };
+    D == 128 ? launch(gqa_attn_tile_kernel<128>)
+             : launch(gqa_attn_tile_kernel<64>);
+    HIP_CHECK_KERNEL();
+    return;
   }
   // (tile, kv head) units in rounds of one per XCD, H/G heads per unit
   const long units = (long)ntiles * G;

@@ -166,3 +166,74 @@ def test_decode(hq, hk, d, page_size, wide):
                          d ** -0.5)
         bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
         assert ((out[i:i + 1].double() - want).abs() <= bound).all(), n
+
+
+@pytest.mark.parametrize("hq,hk,d", [(8, 2, 64), (7, 1, 64), (4, 4, 128),
+                                     (12, 2, 128)])
+@pytest.mark.parametrize("window,keep,chunk", [(1 << 20, 0, 0), (100, 0, 0),
+                                               (64, 4, 0), (70, 130, 0),
+                                               (1 << 20, 0, 96), (1, 0, 0)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_window_prompts(hq, hk, d, window, keep, chunk, extras):
+    """Paged window attention of prompt portions (some behind cached rows):
+    tile edges, windows shorter and longer than a tile, kept first tokens
+    before the window, chunks; sink, gate, row temperature and an output
+    column slice together."""
+    torch.manual_seed(8)
+    lens, hist = [1, 31, 33, 64, 65, 200, 7], [0, 5, 0, 300, 63, 0, 129]
+    page = 16
+    need = [-(-(n + m) // page) for n, m in zip(lens, hist)]
+    pages = torch.randperm(sum(need), device=DEV).int()
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32, device=DEV)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    rows = torch.randn(sum(need), page, 2 * hk * d, device=DEV).bfloat16()
+    n = sum(lens)
+    q = torch.randn(n, hq * d, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(len(lens), **i32),
+                                  torch.tensor(lens, device=DEV))
+    pos = torch.cat([torch.arange(m, m + x, **i32)
+                     for x, m in zip(lens, hist)])
+    sink = torch.randn(hq, device=DEV) * 3 if extras else None
+    gate = torch.randn(n, hq, device=DEV).bfloat16() if extras else None
+    wide = torch.zeros(n, hq * d + 24, device=DEV).bfloat16()
+    out = wide[:, 8:8 + hq * d] if extras else None
+    coef, scale, mult = (0.1, d ** -0.5, 0.5) if extras else \
+        (0.0, d ** -0.5, 1.0)
+    got = ops.seq.gqa_window_attention(
+        q, rows, table, seq, pos, hq, hk, d, d, window, keep, None, None,
+        gate, scale, torch.bfloat16, tiles=ops.seq.attention_tiles(lens, DEV),
+        sink=sink, q_temp_coef=coef, q_temp_every=16, chunk=chunk, out=out,
+        out_scale=mult)
+    a = 0
+    for i, (x, m) in enumerate(zip(lens, hist)):
+        kv = rows[table[i, :need[i]].long()].view(-1, 2, hk, d)[:x + m].double()
+        k, v = heads(kv[:, 0], hq), heads(kv[:, 1], hq)
+        r = pos[a:a + x].long()[:, None]
+        j = torch.arange(x + m, device=DEV)[None]
+        live = (r - j < window)
+        if chunk:
+            live = live & (j // chunk == r // chunk)
+        live = (live | (j < keep)) & (j <= r)
+        temp = 1 + coef * torch.log((r[:, 0].double() + 1).div(
+            16, rounding_mode="floor") + 1)
+        s = torch.einsum("qhd,khd->hqk", q[a:a + x].double().view(x, hq, d),
+                         k) * scale * temp[None, :, None]
+        s = s.masked_fill(~live, -float("inf"))
+        if sink is not None:
+            s = torch.cat([s, sink.double()[:, None, None].expand(
+                -1, x, 1)], -1)
+        p = torch.softmax(s, -1)[..., :x + m]
+        want = torch.einsum("hqk,khd->qhd", p, v)
+        mass = torch.einsum("hqk,khd->qhd", p, v.abs())
+        f = mult * (torch.sigmoid(gate[a:a + x].double())[..., None]
+                    if gate is not None else 1.0)
+        bound = 2 ** -8 * (mass + want.abs()) * f
+        off = (got[a:a + x].double().view(x, hq, d) - want * f).abs() - bound
+        assert off.max() <= 0, (i, off.max())
+        a += x
+    if extras:                         # nothing written beside the slice
+        assert (wide[:, :8] == 0).all() and (wide[:, 8 + hq * d:] == 0).all()
