@@ -286,7 +286,8 @@ class _FlashAttnVarlen(torch.autograd.Function):
 class _RMSNormTrain(torch.autograd.Function):
     """Trainer RMSNorm with optional fused residual add — hand-written
     CDNA4 fwd+bwd (rmsnorm_train.hip).  Returns (y, h) where h = x + res
-    (the next residual); grads flow through both outputs."""
+    (the next residual); grads flow through both outputs, and the one that
+    reaches h past the norm is added inside the backward kernel."""
 
     @staticmethod
     def forward(ctx, x, res, w, eps):

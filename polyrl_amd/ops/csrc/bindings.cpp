@@ -40,6 +40,7 @@ std::vector<torch::Tensor> rmsnorm_train_fwd(torch::Tensor x,
                                              torch::Tensor res,
                                              torch::Tensor w, double eps);
 std::vector<torch::Tensor> rmsnorm_train_bwd(torch::Tensor dy,
+                                             torch::Tensor dh,
                                              torch::Tensor h,
                                              torch::Tensor w,
                                              torch::Tensor rstd);

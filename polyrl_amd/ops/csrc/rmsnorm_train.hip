@@ -71,7 +71,105 @@ __global__ __launch_bounds__(256) void rmsnorm_train_fwd_kernel(
   }
 }
 
-// ------------------------------------------------------------ backward dh
+// ------------------------------------------------------- backward, one pass
+// dx (+ the gradient that reaches h past the norm) and the rows' share of dw.
+// A block walks its rows with its columns' dw in registers, so dy and h are
+// read once, and leaves them to one summing kernel: no atomics.  The next
+// row's words are requested before this row's sum meets.  What bounds it:
+// memory (dy, h in, dx out; 201 MB at 8192 x 4096).  Measured there: 36 us for
+// dx and 140 us for dw in a second pass (row by row, two bytes a lane, sums by
+// atomics), 36 us for both now and 7 us for the sum.
+template <int NV>                    // 16-byte words of a row per thread
+__global__ __launch_bounds__(256) void rmsnorm_train_bwd_kernel(
+    bf16_t* __restrict__ dx,         // (T, H)
+    float* __restrict__ part,        // (blocks, H)
+    const bf16_t* __restrict__ dy, const bf16_t* __restrict__ dh,  // dh: or null
+    const bf16_t* __restrict__ h, const bf16_t* __restrict__ w,
+    const float* __restrict__ rstd, long T, int H) {
+  __shared__ float red[2][4];
+  const int n8 = H / 8, tid = threadIdx.x;
+  const bf16x8* wp = reinterpret_cast<const bf16x8*>(w);
+  float dw[NV][8];
+  bf16x8 w8[NV], d8[NV], h8[NV], dn[NV], hn[NV];
+  auto load = [&](bf16x8 (&d)[NV], bf16x8 (&x)[NV], long row) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      if (tid + v * 256 < n8) {
+        d[v] = reinterpret_cast<const bf16x8*>(dy + row * H)[tid + v * 256];
+        x[v] = reinterpret_cast<const bf16x8*>(h + row * H)[tid + v * 256];
+      }
+  };
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (tid + v * 256 < n8) w8[v] = wp[tid + v * 256];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dw[v][j] = 0.f;
+  }
+  long row = blockIdx.x;
+  if (row < T) load(d8, h8, row);
+  for (int it = 0; row < T; row += gridDim.x, it ^= 1) {
+    const float r = rstd[row];
+    if (row + gridDim.x < T) load(dn, hn, row + gridDim.x);
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      if (tid + v * 256 < n8)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          s += bf2f(d8[v].v[j]) * bf2f(w8[v].v[j]) * bf2f(h8[v].v[j]);
+    s = wave_reduce_sum(s);
+    if ((tid & 63) == 0) red[it][tid >> 6] = s;
+    __syncthreads();                 // (the other buffer holds the last row's)
+    s = red[it][0] + red[it][1] + red[it][2] + red[it][3];
+    const float k = r * r * r / H * s;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (tid + v * 256 >= n8) continue;
+      bf16x8 o, a;
+      if (dh) a = reinterpret_cast<const bf16x8*>(dh + row * H)[tid + v * 256];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float d = bf2f(d8[v].v[j]), x = bf2f(h8[v].v[j]);
+        float g = r * d * bf2f(w8[v].v[j]) - x * k;
+        if (dh) g += bf2f(a.v[j]);
+        o.v[j] = f2bf(g);
+        dw[v][j] += d * x * r;
+      }
+      reinterpret_cast<bf16x8*>(dx + row * H)[tid + v * 256] = o;
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) d8[v] = dn[v], h8[v] = hn[v];
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+    if (tid + v * 256 < n8) {
+      float* p = part + (long)blockIdx.x * H + (tid + v * 256) * 8;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = dw[v][j];
+    }
+}
+
+// dw = sum of the blocks' shares; 16 columns a block, 16 rows at a time
+__global__ __launch_bounds__(256) void rmsnorm_train_dw_sum_kernel(
+    float* __restrict__ dw, const float* __restrict__ part, int blocks, int H) {
+  __shared__ float s[16][17];
+  const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int col = blockIdx.x * 16 + c;
+  float a = 0.f;
+  if (col < H) {
+#pragma unroll 8                     // loads in flight: the loop is latency
+    for (int b = g; b < blocks; b += 16) a += part[(long)b * H + col];
+  }
+  s[g][c] = a;
+  __syncthreads();
+  if (g == 0 && col < H) {
+#pragma unroll
+    for (int i = 1; i < 16; ++i) a += s[i][c];
+    dw[col] = a;
+  }
+}
+
+// ------------------------------- backward of rows too wide for the one above
 __global__ __launch_bounds__(256) void rmsnorm_train_bwd_dx_kernel(
     bf16_t* __restrict__ dx,         // (T, H)
     const bf16_t* __restrict__ dy,
@@ -152,18 +250,49 @@ std::vector<torch::Tensor> rmsnorm_train_fwd(torch::Tensor x,
   return {y, h, rstd};
 }
 
+// dx, dw (fp32); dh: gradient that reaches h past the norm, or undefined
 std::vector<torch::Tensor> rmsnorm_train_bwd(torch::Tensor dy,
+                                             torch::Tensor dh,
                                              torch::Tensor h,
                                              torch::Tensor w,
                                              torch::Tensor rstd) {
   TORCH_CHECK(dy.is_cuda() && dy.dtype() == torch::kBFloat16);
   auto dyc = dy.contiguous();
+  const bool has_dh = dh.defined() && dh.numel() > 0;
+  if (has_dh) {
+    TORCH_CHECK(dh.dtype() == torch::kBFloat16 && dh.sizes() == h.sizes());
+    dh = dh.contiguous();
+  }
   const long T = h.numel() / h.size(-1);
   const int H = h.size(-1);
   auto dx = torch::empty_like(h);
-  // dw zero-filled: gridDim.y partial sums accumulate with atomics
-  auto dw = torch::zeros({(long)H}, h.options().dtype(torch::kFloat32));
+  auto f32 = h.options().dtype(torch::kFloat32);
   auto stream = at::hip::getCurrentHIPStream();
+  const int words = (H / 8 + 255) / 256;
+  if (T > 0 && words <= 8) {
+    // four blocks per CU: two rows in flight each, and 1024 shares of dw
+    const int blocks = (int)std::min<long>(T, 1024);
+    auto part = torch::empty({blocks, (long)H}, f32);
+    auto dw = torch::empty({(long)H}, f32);
+    auto run = [&](auto kern) {
+      kern<<<dim3(blocks), dim3(256), 0, stream>>>(
+          (bf16_t*)dx.data_ptr(), part.data_ptr<float>(),
+          (const bf16_t*)dyc.data_ptr(),
+          has_dh ? (const bf16_t*)dh.data_ptr() : nullptr,
+          (const bf16_t*)h.data_ptr(), (const bf16_t*)w.data_ptr(),
+          rstd.data_ptr<float>(), T, H);
+    };
+    if (words == 1) run(rmsnorm_train_bwd_kernel<1>);
+    else if (words == 2) run(rmsnorm_train_bwd_kernel<2>);
+    else if (words <= 4) run(rmsnorm_train_bwd_kernel<4>);
+    else run(rmsnorm_train_bwd_kernel<8>);
+    rmsnorm_train_dw_sum_kernel<<<dim3((H + 15) / 16), dim3(256), 0, stream>>>(
+        dw.data_ptr<float>(), part.data_ptr<float>(), blocks, H);
+    HIP_CHECK_KERNEL();
+    return {dx, dw};
+  }
+  // dw zero-filled: gridDim.y partial sums accumulate with atomics
+  auto dw = torch::zeros({(long)H}, f32);
   rmsnorm_train_bwd_dx_kernel<<<dim3(T), dim3(256), 0, stream>>>(
       (bf16_t*)dx.data_ptr(), (const bf16_t*)dyc.data_ptr(),
       (const bf16_t*)h.data_ptr(), (const bf16_t*)w.data_ptr(),
@@ -179,5 +308,6 @@ std::vector<torch::Tensor> rmsnorm_train_bwd(torch::Tensor dy,
       (const bf16_t*)h.data_ptr(), rstd.data_ptr<float>(), T, H,
       rows_per_block);
   HIP_CHECK_KERNEL();
+  if (has_dh) dx = dx + dh;
   return {dx, dw};
 }
