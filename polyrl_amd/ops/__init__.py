@@ -179,6 +179,23 @@ def kv_cache_append(k_cache: torch.Tensor, v_cache: torch.Tensor,
     flat_v[slot_mapping[valid].long()] = v[valid]
 
 
+def rope_kv_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                   positions: torch.Tensor, table: RopeTable,
+                   k_cache: torch.Tensor, v_cache: torch.Tensor,
+                   slot_mapping: torch.Tensor
+                   ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """:func:`apply_rope_inplace` on q and k, then :func:`kv_cache_append` of
+    the rotated k and of v; one launch on the GPU.  Returns (q, k)."""
+    if q.is_cuda:
+        ext = _require_ext()
+        ext.rope_kv_append(q, k, v, positions.int(), table.cos, table.sin,
+                           k_cache, v_cache, slot_mapping.int())
+        return q, k
+    q, k = apply_rope_inplace(q, k, positions, table)
+    kv_cache_append(k_cache, v_cache, k, v, slot_mapping)
+    return q, k
+
+
 # ----------------------------------------------------------------- attention
 
 
@@ -296,15 +313,17 @@ class _RMSNormTrain(torch.autograd.Function):
         y, h, rstd = ext.rmsnorm_train_fwd(x.contiguous(), res_t, w, eps)
         ctx.save_for_backward(h, w, rstd)
         ctx.has_res = res is not None
+        ctx.set_materialize_grads(False)    # an unused output: no zeros
         return y, h
 
     @staticmethod
     def backward(ctx, dy, dh_out):
+        if dy is None:
+            return dh_out, dh_out if ctx.has_res else None, None, None
         h, w, rstd = ctx.saved_tensors
         ext = _require_ext()
-        dx, dw = ext.rmsnorm_train_bwd(dy, h, w, rstd)
-        if dh_out is not None:
-            dx = dx + dh_out
+        dx, dw = ext.rmsnorm_train_bwd(
+            dy, dh_out if dh_out is not None else torch.Tensor(), h, w, rstd)
         return (dx, dx if ctx.has_res else None, dw.to(w.dtype), None)
 
 

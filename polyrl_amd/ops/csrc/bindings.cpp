@@ -9,6 +9,10 @@ void fused_add_rmsnorm(torch::Tensor out, torch::Tensor residual,
 void silu_mul(torch::Tensor out, torch::Tensor gate, torch::Tensor up);
 void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
                   torch::Tensor cos_tab, torch::Tensor sin_tab);
+void rope_kv_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                    torch::Tensor positions, torch::Tensor cos_tab,
+                    torch::Tensor sin_tab, torch::Tensor k_cache,
+                    torch::Tensor v_cache, torch::Tensor slot_mapping);
 void gather_logprobs(torch::Tensor out_lp, torch::Tensor out_ent,
                      torch::Tensor logits, torch::Tensor labels,
                      bool want_entropy);
@@ -71,6 +75,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual-add + RMSNorm, residual updated in place");
   m.def("silu_mul", &silu_mul, "SiLU(gate) * up");
   m.def("rope_inplace", &rope_inplace, "NEOX RoPE in place (table-driven)");
+  m.def("rope_kv_append", &rope_kv_append,
+        "NEOX RoPE in place on q, k + paged KV cache rows, one launch");
   m.def("gather_logprobs", &gather_logprobs,
         "log-softmax gather at labels (+optional entropy)");
   m.def("sample", &sample,

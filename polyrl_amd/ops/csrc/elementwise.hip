@@ -239,3 +239,91 @@ void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
       sin_tab.data_ptr<float>(), Hq, Hk, D, q.stride(0), k.stride(0));
   HIP_CHECK_KERNEL();
 }
+
+// ------------------------------------------------------ RoPE + KV cache rows
+// rope_kernel on q and k, and the token's rotated k and its v into their page
+// slot, in one launch: a prompt or decode step's k row is read and turned once
+// and goes to both places from registers (two launches read it twice).
+// Measured, 5700 tokens, 16/4 heads of 64: 7.1 + 5.0 us, 8.4 us.
+__global__ void rope_kv_append_kernel(
+    bf16_t* __restrict__ q, bf16_t* __restrict__ k,
+    const bf16_t* __restrict__ v, const int* __restrict__ positions,
+    const float* __restrict__ cos_tab, const float* __restrict__ sin_tab,
+    bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
+    const int* __restrict__ slot_mapping, int Hq, int Hk, int D, long ldq,
+    long ldk, long ldv /* token strides */) {
+  const long tok = blockIdx.x;
+  const int half = D / 2, quads = half / 4;
+  const float* c = cos_tab + (long)positions[tok] * half;
+  const float* s = sin_tab + (long)positions[tok] * half;
+  const long slot = slot_mapping[tok];   // < 0: a padding token
+  bf16_t* kc = k_cache + slot * Hk * D;
+  bf16_t* vc = v_cache + slot * Hk * D;
+  const int nrope = (Hq + Hk) * quads;
+  for (int t = threadIdx.x; t < nrope + Hk * D / 8; t += blockDim.x) {
+    if (t >= nrope) {
+      const int at = (t - nrope) * 8;
+      if (slot >= 0)
+        *reinterpret_cast<bf16x8*>(vc + at) =
+            *reinterpret_cast<const bf16x8*>(v + tok * ldv + at);
+      continue;
+    }
+    const int h = t / quads;
+    const int d = (t % quads) * 4;
+    bf16_t* base = h < Hq ? q + tok * ldq + (long)h * D
+                          : k + tok * ldk + (long)(h - Hq) * D;
+    const bf16x4 x1 = *reinterpret_cast<bf16x4*>(base + d);
+    const bf16x4 x2 = *reinterpret_cast<bf16x4*>(base + half + d);
+    const f32x4v cv = *reinterpret_cast<const f32x4v*>(c + d);
+    const f32x4v sv = *reinterpret_cast<const f32x4v*>(s + d);
+    bf16x4 o1, o2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = bf2f(x1.v[j]), b = bf2f(x2.v[j]);
+      // (fused as the compiler fuses rope_kernel's: the same bits)
+      o1.v[j] = f2bf(__fmaf_rn(a, cv.v[j], -(b * sv.v[j])));
+      o2.v[j] = f2bf(__fmaf_rn(a, sv.v[j], b * cv.v[j]));
+    }
+    *reinterpret_cast<bf16x4*>(base + d) = o1;
+    *reinterpret_cast<bf16x4*>(base + half + d) = o2;
+    if (h >= Hq && slot >= 0) {
+      bf16_t* to = kc + (h - Hq) * D + d;
+      *reinterpret_cast<bf16x4*>(to) = o1;
+      *reinterpret_cast<bf16x4*>(to + half) = o2;
+    }
+  }
+}
+
+void rope_kv_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                    torch::Tensor positions, torch::Tensor cos_tab,
+                    torch::Tensor sin_tab, torch::Tensor k_cache,
+                    torch::Tensor v_cache, torch::Tensor slot_mapping) {
+  TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16 &&
+              k.dtype() == torch::kBFloat16 && v.dtype() == torch::kBFloat16);
+  TORCH_CHECK(k_cache.is_cuda() && k_cache.dtype() == torch::kBFloat16 &&
+              v_cache.dtype() == torch::kBFloat16 &&
+              k_cache.is_contiguous() && v_cache.is_contiguous());
+  TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
+  for (const auto* t : {&q, &k, &v})
+    TORCH_CHECK(t->stride(2) == 1 && t->stride(1) == t->size(2),
+                "heads and head dim must be packed");
+  TORCH_CHECK(positions.dtype() == torch::kInt32 &&
+              slot_mapping.dtype() == torch::kInt32);
+  const int N = q.size(0), Hq = q.size(1), D = q.size(2), Hk = k.size(1);
+  TORCH_CHECK(D % 8 == 0, "head_dim must be a multiple of 8");
+  TORCH_CHECK(k_cache.size(2) == Hk && k_cache.size(3) == D &&
+              v.size(1) == Hk && v.size(2) == D);
+  if (N == 0) return;
+  // a thread per rotary quad and value word, in whole waves
+  const int work = (Hq + Hk) * (D / 8) + Hk * D / 8;
+  const int threads = std::min(256, (work + 63) / 64 * 64);
+  auto stream = at::hip::getCurrentHIPStream();
+  rope_kv_append_kernel<<<dim3(N), dim3(threads), 0, stream>>>(
+      (bf16_t*)q.data_ptr(), (bf16_t*)k.data_ptr(),
+      (const bf16_t*)v.data_ptr(), positions.data_ptr<int>(),
+      cos_tab.data_ptr<float>(), sin_tab.data_ptr<float>(),
+      (bf16_t*)k_cache.data_ptr(), (bf16_t*)v_cache.data_ptr(),
+      slot_mapping.data_ptr<int>(), Hq, Hk, D, q.stride(0), k.stride(0),
+      v.stride(0));
+  HIP_CHECK_KERNEL();
+}

@@ -303,13 +303,12 @@ class InferenceModel:
             if lw.bqkv is not None:
                 qkv = qkv + lw.bqkv
             # strided head views into the fused qkv row (no copies: the
-            # rope/kv-append/attention kernels take a free token stride)
+            # rope + kv-append and attention kernels take a free token stride)
             q = qkv.narrow(1, 0, Hq * D).unflatten(1, (Hq, D))
             k = qkv.narrow(1, Hq * D, Hk * D).unflatten(1, (Hk, D))
             v = qkv.narrow(1, (Hq + Hk) * D, Hk * D).unflatten(1, (Hk, D))
-            ops.apply_rope_inplace(q, k, positions, self.rope)
-            ops.kv_cache_append(kv.k_cache[li], kv.v_cache[li], k, v,
-                                slot_mapping)
+            ops.rope_kv_append(q, k, v, positions, self.rope,
+                               kv.k_cache[li], kv.v_cache[li], slot_mapping)
             attn_out = attn_fn(li, q, k, v)           # (N, Hq, D)
             hidden = _mm_nt(attn_out.reshape(-1, Hq * D), lw.wo)
             self.tp.all_reduce_(hidden)               # col-parallel o_proj
