@@ -18,6 +18,7 @@ import time
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional
 
+import numpy as np
 import torch
 
 import polyrl_amd.ops as ops
@@ -802,7 +803,6 @@ class Engine:
     def _hybrid_batch(self, items):
         """Pack [(request, start, tokens)] into one HybridBatch: pages for
         the new tokens are already allocated by the caller."""
-        import numpy as np
         from .hybrid_model import HybridBatch
         dev = self.device
         tok, pos, sot, cu, slots, sids, maps = [], [], [], [0], [], [], []
@@ -999,7 +999,7 @@ class Engine:
                     [it[0] for it in items], [it[1] for it in items],
                     [len(it[2]) for it in items])[0]
             if rows:
-                idx = torch.tensor(rows, dtype=torch.long, device=self.device)
+                idx, = self._upload([np.asarray(rows, np.int32)])
                 logits = self.model.logits(hidden.index_select(0, idx)).float()
         for rid in end:
             r = self._forced.pop(rid, None)
@@ -1012,41 +1012,53 @@ class Engine:
                           lens: List[int]):
         """Hidden rows of each request's tokens [start, start+len) against
         its cached history (dense decoders); returns (hidden, cu_q)."""
-        dev = self.device
-        tok_list, pos_list, slot_list = [], [], []
-        cu_q = [0]
-        cu_k = [0]
-        for r, start, take in zip(reqs, starts, lens):
-            sid = self._seq_ids[r.rid]
-            tok_list.extend(r.input_ids[start:start + take])
-            pos_list.extend(range(start, start + take))
-            slot_list.append(self.kv.slots_for(sid, start, take))
+        cu_q, cu_k = [0], [0]
+        for start, take in zip(starts, lens):
             cu_q.append(cu_q[-1] + take)
             cu_k.append(cu_k[-1] + start + take)
-        tokens = torch.tensor(tok_list, dtype=torch.long, device=dev)
-        positions = torch.tensor(pos_list, dtype=torch.int32, device=dev)
-        slots = torch.cat(slot_list).to(dev)
-        cu_q_t = torch.tensor(cu_q, dtype=torch.int32, device=dev)
-        cu_k_t = torch.tensor(cu_k, dtype=torch.int32, device=dev)
-        seq_ids = [self._seq_ids[r.rid] for r in reqs]
-        ctx_lens = torch.tensor([s + t for s, t in zip(starts, lens)],
-                                dtype=torch.int32, device=dev)
+        n = cu_q[-1]
+        sids = [self._seq_ids[r.rid] for r in reqs]
         fresh = all(s == 0 for s in starts)
+        # all descriptors in one upload that nothing waits for: the host
+        # prepares a step while the GPU still works on the one before (16
+        # prompts of the 400M model: 3.78 -> 3.02 ms a step of 3.0 ms of
+        # kernels; five blocking copies, one tensor per request before)
+        tok = np.fromiter((t for r, s, m in zip(reqs, starts, lens)
+                           for t in r.input_ids[s:s + m]), np.int32, n)
+        pos = np.concatenate([np.arange(s, s + m, dtype=np.int32)
+                              for s, m in zip(starts, lens)])
+        slots = [self.kv.slots_for_host(sid, s, m)
+                 for sid, s, m in zip(sids, starts, lens)]
+        parts = [tok, pos, np.concatenate(slots),
+                 np.asarray(cu_q, np.int32), np.asarray(cu_k, np.int32)]
+        if not fresh:
+            # portions behind cached tokens attend to the FULL history: the
+            # cache rows of every key, gathered once per layer
+            parts.append(np.concatenate(
+                [self.kv.slots_for_host(sid, 0, s + m)
+                 for sid, s, m in zip(sids, starts, lens)]))
+        tokens, positions, slots, cu_q_t, cu_k_t, *hist = self._upload(parts)
 
         def attn_fn(li, q, k, v):
-            # portions after the first attend to the FULL cached history
-            # (cu_k spans include earlier portions): gather K/V from the
-            # cache pages of this layer
-            if fresh:
-                return ops.varlen_prefill_attention(q, k, v, cu_q_t, cu_k_t,
-                                                    self._scale, causal=True)
-            kf, vf = self._gather_kv(li, seq_ids, ctx_lens)
-            return ops.varlen_prefill_attention(q, kf, vf, cu_q_t, cu_k_t,
+            if not fresh:
+                k, v = (c[li].view(-1, *c[li].shape[2:])
+                        .index_select(0, hist[0])
+                        for c in (self.kv.k_cache, self.kv.v_cache))
+            return ops.varlen_prefill_attention(q, k, v, cu_q_t, cu_k_t,
                                                 self._scale, causal=True)
 
-        hidden = self.model.forward_tokens(tokens, positions, self.kv, slots,
-                                           attn_fn)
+        hidden = self.model.forward_tokens(tokens.long(), positions, self.kv,
+                                           slots, attn_fn)
         return hidden, cu_q
+
+    def _upload(self, parts) -> List[torch.Tensor]:
+        """int32 arrays as device tensors, through one pinned buffer and one
+        copy that the host does not wait for (its memory stays reserved until
+        the copy is done)."""
+        flat = torch.from_numpy(np.concatenate(parts))
+        if str(self.device) != "cpu":
+            flat = flat.pin_memory().to(self.device, non_blocking=True)
+        return list(flat.split([len(p) for p in parts]))
 
     def _run_prefill(self, reqs: List[Request], lens: List[int]):
         dev = self.device
@@ -1112,20 +1124,6 @@ class Engine:
         rows = last_hidden.unsqueeze(0).expand(n, -1).contiguous()
         self.running.extend(children)
         self._sample_last([parent] + children, rows)
-
-    def _gather_kv(self, li: int, seq_ids: List[int], ctx_lens: torch.Tensor):
-        """Materialize contiguous K/V for chunked-prefill history (per layer)."""
-        ks, vs = [], []
-        flat_k = self.kv.k_cache[li].view(-1, self.cfg.num_key_value_heads,
-                                          self.cfg.head_dim)
-        flat_v = self.kv.v_cache[li].view(-1, self.cfg.num_key_value_heads,
-                                          self.cfg.head_dim)
-        for i, sid in enumerate(seq_ids):
-            L = int(ctx_lens[i])
-            slots = self.kv.slots_for(sid, 0, L).to(flat_k.device)
-            ks.append(flat_k[slots.long()])
-            vs.append(flat_v[slots.long()])
-        return torch.cat(ks), torch.cat(vs)
 
     def _decode_chunk_len(self, reqs: List[Request]) -> int:
         """How many decode iterations can run device-side without a host

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 
@@ -164,6 +165,14 @@ class PageAllocator:
         pos = torch.arange(start, start + count, dtype=torch.int64)
         return (pages[pos // self.page_size] * self.page_size
                 + pos % self.page_size).to(torch.int32)
+
+    def slots_for_host(self, seq_id: int, start: int,
+                       count: int) -> np.ndarray:
+        """:meth:`slots_for` as an int32 array."""
+        pages = np.asarray(self._seq_pages[seq_id], dtype=np.int32)
+        pos = np.arange(start, start + count, dtype=np.int32)
+        return pages[pos // self.page_size] * self.page_size \
+            + pos % self.page_size
 
     def page_table(self, seq_ids: List[int], max_pages: Optional[int] = None
                    ) -> torch.Tensor:

@@ -531,3 +531,33 @@ def test_decode_scratch_survives_release_resume(setup):
     assert 0 <= page < eng.kv.num_pages
     assert eng.kv.k_cache[0][page].abs().sum().item() == 0.0
     eng.kv.free_seq(eng._SCRATCH_SEQ)               # leave the engine clean
+
+
+def test_portions_behind_cached_tokens_match_whole_prompts():
+    """Prompts fed in unequal portions (fresh ones beside ones with cached
+    history, pages out of order) give the logits of whole prompts."""
+    from polyrl_amd.models import get_model_config
+    cfg = get_model_config("llama-debug-cpu")
+    eng = Engine(cfg, device="cpu", dtype=torch.float32, page_size=4,
+                 kv_token_capacity=400, max_running_requests=8)
+    g = torch.Generator().manual_seed(3)
+    for t in eng.model._name_map.values():
+        t.normal_(0, 0.05, generator=g)
+    prompts = [torch.randint(0, cfg.vocab_size, (n,), generator=g).tolist()
+               for n in (1, 9, 23, 30)]
+    whole = eng.step_forced([(f"w{i}", p, [len(p) - 1])
+                             for i, p in enumerate(prompts)],
+                            end=[f"w{i}" for i in range(4)])
+    cuts = [(0, 1, 1, 1), (0, 4, 4, 9), (0, 7, 8, 23), (0, 0, 29, 30)]
+    last = {}
+    for step in range(3):
+        entries = []
+        for i, (p, c) in enumerate(zip(prompts, cuts)):
+            toks = p[c[step]:c[step + 1]]
+            if toks:
+                entries.append((f"p{i}", toks, [len(toks) - 1]))
+        out = eng.step_forced(entries)
+        for (rid, _, _), row in zip(entries, out):
+            last[rid] = row
+    got = torch.stack([last[f"p{i}"] for i in range(4)])
+    assert torch.allclose(got, whole, atol=1e-4, rtol=1e-4)
