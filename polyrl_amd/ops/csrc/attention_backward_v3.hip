@@ -32,7 +32,7 @@
 // fragment of 1 KiB per 32-cycle product).  Measured, forward and backward of
 // packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with kernels
 // that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
-// gradients for a cast to read, 267 us now (349 with every fragment read just
+// gradients for a cast to read, 258 us now (349 with every fragment read just
 // before its product); 2 of up to 4096, 28/4 heads, 4000 -> 1305 us.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -277,7 +277,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   int fg = g0, fq = qs;               // head and first row of the next fetch
   auto fetch_rows = [&]() {           // the first two waves' are stored
     const int r = fq + lane;
-    const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G + fg;
+    const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G +
+                   min(fg, g1 - 1);
     rlive = r < Lq;
     rowv = (wid == 0 ? lse : delta)[i];
   };
@@ -318,10 +319,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     const char* qs_ = lds[buf];
     const char* ds_ = lds[2];
     at.renew();
-    if (more) {
-      fetch_rows();
-      fetch_q();
-    }
+    // (in every step: under a condition the register would be copied at the
+    // join, and the copy would wait for the load)
+    fetch_rows();
+    if (more) fetch_q();
     bf16x8_t p[2], ds[2];
     if (work) {
       f32x16_t s, dp;
