@@ -347,7 +347,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         SCHED_LDS(PER - 1);
       }
       SCHED_MFMA(4);
-      const bool edge = causal && qk_off + wq0 < wk0 + 31;
+      // accumulator rows before this lane's key, at the causal border only
+      const int border = causal && qk_off + wq0 < wk0 + 31
+          ? key - (qk_off + wq0) - 4 * (lane >> 5) : 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r0 = qh * 32 + 8 * i + 4 * (lane >> 5);
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * i + t;
           float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
-          if (edge && qk_off + wq0 + acc_row(r) < key) w = 0.f;
+          if (8 * i + t < border) w = 0.f;
           s[r] = w;
           dp[r] = w * (dp[r] - d4[t]);
         }
