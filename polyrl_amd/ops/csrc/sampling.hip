@@ -510,11 +510,14 @@ static void launch_sample(torch::Tensor& out_tokens,
   const int V = logits.size(1);
   if (N == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  // pieces of a row: 2048 blocks in all (eight per CU), none under two
-  // rounds of 256 words
+  // pieces of a row: 2048 blocks in all (eight per CU; 128 x 128256 takes 37
+  // us with 512 blocks, 33 with 1024, 32 with 2048, 36 with 4096), half of
+  // that for the short passes of filtered rows (64 x 151936: 63, 55, 60, 62
+  // us), none under two rounds of 256 words
   const long words = (V + VocabRow<T>::VEC - 1) / VocabRow<T>::VEC;
   const int split = (int)std::max<long>(
-      1, std::min<long>({64, (2048 + N - 1) / N, words / (2 * SNT)}));
+      1, std::min<long>({64, ((no_filter ? 2048 : 1024) + N - 1) / N,
+                         words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
   const int hist_words = no_filter ? 0 : digits * 4 * DIGIT;
   // per row: the pieces' shares and maxima, the plan, the bins.  From the
