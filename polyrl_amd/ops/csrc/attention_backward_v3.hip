@@ -1,7 +1,7 @@
 // Varlen causal flash-attention backward v3 (bf16, head_dim 64/128, MFMA).
 //
 // Reference capability: the training-side flash-attn backward the reference
-// reaches through the flash-attn package (SURVEY.md §2.2.2 'flash-attn').
+// reaches through the flash-attn package.
 //
 // Two kernels that each OWN the rows they write: no atomics, no zero-fill,
 // the same bits on every run; gradients are rounded to bf16 once, as they are
@@ -32,8 +32,8 @@
 // fragment of 1 KiB per 32-cycle product).  Measured, forward and backward of
 // packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with kernels
 // that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
-// gradients for a cast to read, 260 us now (349 with every fragment read just
-// before its product); 2 of up to 4096, 28/4 heads, 4000 -> 1339 us.
+// gradients for a cast to read, 257 us now (349 with every fragment read just
+// before its product); 2 of up to 4096, 28/4 heads, 4000 -> 1295 us.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

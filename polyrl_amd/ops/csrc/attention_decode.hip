@@ -1,7 +1,7 @@
 // Paged decode attention (continuous-batching, one new token per sequence).
 //
 // Reference capability: the paged/continuous-batching decode attention the
-// reference reaches through its inference engine (SURVEY.md §2.4.3 row 1).
+// reference reaches through its inference engine.
 //
 // A block serves one key/value head of one sequence (or a stretch of its
 // context) for all G query heads of the group; each of its four waves takes

@@ -1,7 +1,7 @@
 // Varlen causal prefill attention, bf16, head_dim 64/128, GQA — MFMA forward.
 //
-// Reference capability: chunked-prefill flash attention (SURVEY.md §2.4.3
-// row 2).  Flash-style online softmax, no score matrix in memory.
+// Reference capability: chunked-prefill flash attention.  Flash-style online
+// softmax, no score matrix in memory.
 //
 // Split.  A wave owns 32 query rows of one head; a block is four such units
 // of one 64-row tile and one key/value head, heads of the group first (four
@@ -24,8 +24,8 @@
 // SIMD, about as many cycles of each at D = 128 (the 16-row score tiles with
 // scalar LDS gathers for V that this replaces ran at 160 TFLOP/s).  Measured,
 // eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads of 64: 671 us a call
-// before (50 us of it the tile table's trip through the host), 171 us now
-// (620 TFLOP/s of live pairs).  A maximum that may lag by 2^6 saves the
+// before (50 us of it the tile table's trip through the host), 164 us now
+// (645 TFLOP/s of live pairs).  A maximum that may lag by 2^6 saves the
 // rescaling in most tiles (158 us), but then a row's largest weight is no
 // longer exactly 1 and takes part in the rounding to bf16: the error against
 // 64 bits grows by 2 to 3% (2.03e-3 for 1.98e-3, rms, 1024 keys).

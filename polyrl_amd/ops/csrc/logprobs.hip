@@ -1,7 +1,6 @@
 // Fused per-token log-prob gather (+ entropy) over the vocab dim.
 //
-// Replaces the logprobs_from_logits / entropy_from_logits pair (reference
-// capability: SURVEY.md §2.4.3 'logprobs_from_logits + entropy', consumed by
+// Replaces the logprobs_from_logits / entropy_from_logits pair (consumed by
 // compute_log_prob and the rollout logprob capture).  One streaming pass:
 // online max + sum-exp + weighted-sum for entropy, then lp = x[label] - LZ.
 //

@@ -3,9 +3,8 @@
 //
 // Why: the autograd path's eager norm (x.float() -> F.rms_norm -> .to(bf16)
 // -> *w) materializes an fp32 copy of every (T, 4096) activation and runs
-// ~6 elementwise passes per call; rocprof r01 attributed ~1.9 s of a
-// 2-step window to eager elementwise (profiles/PROFILES.md item 4).  This
-// fuses each norm to one read/write pass (fwd) + two passes (bwd).
+// ~6 elementwise passes per call.  This fuses each norm to one read/write
+// pass forward and one backward (two for rows wider than 16384).
 //
 // Math (fp32 accumulation):
 //   h = x + res                  (res optional)
@@ -17,7 +16,7 @@
 //   dw_j = sum_t dy[t,j] * h[t,j] * r[t]  (column-reduction kernel)
 //
 // Reference capability: the fused RMSNorm the reference stack reaches via
-// flash-attn/apex inside verl models (SURVEY.md §2.4.3 RMSNorm row) —
+// flash-attn/apex inside verl models —
 // here with a hand-written backward as well.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>

@@ -1,8 +1,8 @@
 // Fused sampling: temperature + top-k + top-p filter + categorical draw +
 // sampled-token logprob capture.
 //
-// Reference capability: the engine-side sampling + per-token logprob kernels
-// (SURVEY.md §2.4.3).  Semantics:
+// Reference capability: the engine-side sampling + per-token logprob kernels.
+// Semantics:
 //  * top-k threshold = k-th largest logit, found by radix select over the
 //    monotone uint32 encoding of the logit (temperature doesn't change order,
 //    so select on raw logits).

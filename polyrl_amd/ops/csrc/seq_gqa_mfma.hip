@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
 // collects values 8 bytes at a time, one row per lane.  The next K tile is in
 // flight during a tile's score products, the next V tile during its value
 // products, in the same registers.  Measured, eight prompts of 1200 .. 2048
-// tokens, window 1024, 32/8 heads of 64: 547 us in the general kernel, 166 here.
+// tokens, window 1024, 32/8 heads of 64: 547 us in the general kernel, 159 here.
 template <int D>
 __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
     bf16_t* __restrict__ out,            // (N, H*D), row stride ldo
