@@ -199,7 +199,9 @@ struct alignas(8) Plan {              // where a row's two selections stand
 
 // Walks the bins from the top until the running count reaches ``need`` (or
 // the running mass ``target``); bin 0 if none does.  All threads of the block
-// get the bin and the sum above it.
+// get the bin and the sum above it.  lds: the waves' sums, the first thread
+// that reaches the goal, its bin and the sum above that, each in words of its
+// own: a wave may still read the thread while that thread writes its bin.
 template <bool MASS>
 DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
                          float* lds, int& bin, float& before) {
@@ -251,10 +253,10 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
     }
     run = at_run;
     lds[SNW + 1] = run;
-    *found = max(n - 1 - (who * per + at), 0);
+    found[2] = max(n - 1 - (who * per + at), 0);
   }
   __syncthreads();
-  bin = *found;
+  bin = found[2];
   before = lds[SNW + 1];
 }
 

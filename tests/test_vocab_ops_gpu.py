@@ -129,3 +129,46 @@ def test_sample_against_its_definition(n, v, dtype, temp, k, p):
         z = row / temp + noise(seed, r, v)
         # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
         assert z[t] >= z[sure].max() - 1e-3
+
+
+@pytest.mark.parametrize("b1,b2", [(0, 0), (1, 63), (5, 64), (64, 255),
+                                   (255, 200), (256, 256), (2047, 1023)])
+def test_sample_low_bins_of_later_digits(b1, b2):
+    """fp32 rows whose k-th largest entry has small second and third digits
+    (bin numbers like thread numbers and like the block size among them):
+    what is kept is exactly the k largest."""
+    n, v, k = 128, 3000, 40
+    g = torch.Generator().manual_seed(b1 * 4096 + b2)
+
+    def number(d0, d1, d2):           # its bits but the sign, as digits
+        return ((d0 << 21) | (d1 << 10) | d2).to(torch.int32).view(
+            torch.float32)
+
+    rand = lambda lo, hi, m: torch.randint(lo, hi, (m,), generator=g)
+    top = 0x7f << 2                   # exponent of numbers from 1 on
+    rows = []
+    for _ in range(n):
+        m = v - 1
+        x = number(torch.full((m,), top), rand(0, 2048, m), rand(0, 1024, m))
+        # the larger ones share as many digits with the k-th as there are
+        at = torch.tensor([top, b1, b2])
+        kth = number(*at.view(3, 1))
+        x = torch.where(x > kth, kth - x, x)     # not above: below zero
+        up = number(torch.full((k - 1,), top),
+                    torch.full((k - 1,), b1).minimum(torch.tensor(2047)),
+                    rand(b2, 1024, k - 1))
+        x = torch.cat([up, kth, x])
+        rows.append(x[torch.randperm(v, generator=g)])
+    x = torch.stack(rows)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    temp, seed = 0.7, 77
+    tok, _ = ops.sample(x.to(DEV), full(temp, torch.float32),
+                        full(k, torch.int32), full(1.0, torch.float32), seed,
+                        no_filter=False)
+    for r in range(n):
+        row = x[r].double()
+        sure, _ = kept(row, temp, k, 1.0)
+        t = int(tok[r])
+        assert sure[t]
+        z = row / temp + noise(seed, r, v)
+        assert z[t] >= z[sure].max() - 1e-3
