@@ -58,10 +58,13 @@ DEV_INLINE uint32_t rng_bits(uint64_t rowkey, int i0, int j) {
   return (uint32_t)(splitmix64(rowkey ^ at) >> 40);
 }
 
-// Gumbel noise of these bits: u uniform in (0, 1]
+// Gumbel noise of these bits: u = (bits + 1) / 2^24.  The largest bits stand
+// for the numbers between 1 - 2^-24 and 1: -log u is 2^-25 in their middle (at
+// u = 1 the noise would be infinite and the entry drawn whatever its logit,
+// in one row of 130 at 128256 entries).
 DEV_INLINE float gumbel(uint32_t bits) {
   const float u = ((float)bits + 1.0f) * (1.0f / 16777216.0f);
-  return -__logf(-__logf(u));
+  return -__logf(bits == 0xFFFFFFu ? 0x1p-25f : -__logf(u));
 }
 
 constexpr int SNT = 256;              // threads of a block
@@ -147,7 +150,7 @@ struct Draw {
     // negative temperature, where c is no bound)
     int least = 0;
     if (inv_temp > 0.f) {
-      const float u = __expf(-__expf(c * inv_temp - wbest));
+      const float u = __expf(-__expf(__fmaf_rn(c, inv_temp, -wbest)));
       least = (int)(u * (16777216.f * (1.f - 1e-5f))) - 2;
     }
     uint32_t bits[N];

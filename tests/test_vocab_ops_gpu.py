@@ -61,7 +61,8 @@ def test_logprobs_minus_infinity(v):
 
 def noise(seed, row, v):
     """Gumbel noise of a row's entries, from the documented generator:
-    splitmix64 keyed by (seed, row, entry), 24 bits, -log(-log u)."""
+    splitmix64 keyed by (seed, row, entry), 24 bits, -log(-log u); -log u of
+    the largest number is 2^-25."""
     import numpy as np
     with np.errstate(over="ignore"):
         u64 = np.uint64
@@ -72,7 +73,8 @@ def noise(seed, row, v):
         z = (z ^ (z >> u64(30))) * u64(0xbf58476d1ce4e5b9)
         z = (z ^ (z >> u64(27))) * u64(0x94d049bb133111eb)
         u = ((z >> u64(40)).astype("f8") + 1) / 16777216.0
-        return torch.from_numpy(-np.log(-np.log(u)))
+        return torch.from_numpy(-np.log(np.where(u == 1.0, 2.0 ** -25,
+                                                 -np.log(u))))
 
 
 def kept(x, temp, k, p):
@@ -172,3 +174,19 @@ def test_sample_low_bins_of_later_digits(b1, b2):
         assert sure[t]
         z = row / temp + noise(seed, r, v)
         assert z[t] >= z[sure].max() - 1e-3
+
+
+@pytest.mark.parametrize("seed,at", [(4116, 1462), (5128, 2925)])
+@pytest.mark.parametrize("filtered", [False, True])
+def test_sample_largest_random_number(seed, at, filtered):
+    """An entry whose 24 random bits are all ones has the largest noise there
+    is, but finite noise: it does not win against any logit."""
+    v = 4096
+    assert noise(seed, 0, v).argmax() == at
+    x = torch.zeros(1, v, device=DEV)
+    x[0, at] = -40.0
+    full = lambda t, ty: torch.full((1,), t, dtype=ty, device=DEV)
+    tok, _ = ops.sample(x, full(1.0, torch.float32), full(-1, torch.int32),
+                        full(1.0, torch.float32), seed,
+                        no_filter=not filtered)
+    assert int(tok) == int((x[0].double().cpu() + noise(seed, 0, v)).argmax())
