@@ -98,19 +98,27 @@ DEV_INLINE void wave_best(float& v, int& i) {
 template <bool TEMP>
 struct Sums {
   float m = -INFINITY, s = 0.f, st = 0.f;
+  // what a sum relative to m counts relative to c; without numbers so far
+  // (m = -inf) nothing, whatever the temperature's sign
+  DEV_INLINE static float shift(float m, float c, float inv_temp) {
+    return m == c ? 1.f : m == -INFINITY ? 0.f : __expf((m - c) * inv_temp);
+  }
   // c: the largest of v
   template <int N>
   DEV_INLINE void add(const float (&v)[N], float c, float inv_temp) {
     if (c > m) {
       s *= __expf(m - c);              // 0 at the first numbers
-      if (TEMP) st *= __expf((m - c) * inv_temp);
+      if (TEMP) st *= shift(m, c, inv_temp);
       m = c;
     }
     if (m == -INFINITY) return;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       s += __expf(v[j] - m);
-      if (TEMP) st += __expf((v[j] - m) * inv_temp);
+      // (-inf, also what stands in for entries outside the row, has no mass
+      // at a negative or infinite temperature either)
+      if (TEMP)
+        st += v[j] == -INFINITY ? 0.f : __expf((v[j] - m) * inv_temp);
     }
   }
   // relative to the larger maximum of the two
@@ -121,9 +129,7 @@ struct Sums {
     const float b = om == c ? 1.f : __expf(om - c);
     s = s * a + os * b;
     if (TEMP) {
-      const float at = m == c ? 1.f : __expf((m - c) * inv_temp);
-      const float bt = om == c ? 1.f : __expf((om - c) * inv_temp);
-      st = st * at + ot * bt;
+      st = st * shift(m, c, inv_temp) + ot * shift(om, c, inv_temp);
     }
     m = c;
   }

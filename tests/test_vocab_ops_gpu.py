@@ -190,3 +190,26 @@ def test_sample_largest_random_number(seed, at, filtered):
                         full(1.0, torch.float32), seed,
                         no_filter=not filtered)
     assert int(tok) == int((x[0].double().cpu() + noise(seed, 0, v)).argmax())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sample_negative_temperature(dtype):
+    """The draw at a negative temperature, with and without top-p: the
+    filter's mass is exp(x / T) also there, from the largest logit down."""
+    torch.manual_seed(7)
+    n, v, temp, seed = 64, 3000, -0.8, 21
+    x = torch.randn(n, v, device=DEV).to(dtype)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    for p in (1.0, 0.3):
+        tok, lp = ops.sample(x, full(temp, torch.float32),
+                             full(-1, torch.int32), full(p, torch.float32),
+                             seed, no_filter=p >= 1.0)
+        want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+        assert (lp.double() - want).abs().max() <= 1e-4
+        for r in range(n):
+            row = x[r].double().cpu()
+            sure, maybe = kept(row, temp, -1, p)
+            t = int(tok[r])
+            assert maybe[t]
+            z = row / temp + noise(seed, r, v)
+            assert z[t] >= z[sure].max() - 1e-3
