@@ -111,7 +111,12 @@ struct Sums {
       if (TEMP) st *= shift(m, c, inv_temp);
       m = c;
     }
-    if (m == -INFINITY) return;
+    if (m == -INFINITY) {              // nothing but -inf and NaN so far
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (v[j] != v[j]) s = st = v[j];
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       s += __expf(v[j] - m);
@@ -124,7 +129,11 @@ struct Sums {
   // relative to the larger maximum of the two
   DEV_INLINE void merge(float om, float os, float ot, float inv_temp) {
     const float c = fmaxf(m, om);
-    if (c == -INFINITY) return;
+    if (c == -INFINITY) {              // zeros, or NaN
+      s += os;
+      if (TEMP) st += ot;
+      return;
+    }
     const float a = m == c ? 1.f : __expf(m - c);
     const float b = om == c ? 1.f : __expf(om - c);
     s = s * a + os * b;

@@ -213,3 +213,21 @@ def test_sample_negative_temperature(dtype):
             assert maybe[t]
             z = row / temp + noise(seed, r, v)
             assert z[t] >= z[sure].max() - 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("v", [300, 9000])
+@pytest.mark.parametrize("filtered", [False, True])
+@pytest.mark.parametrize("temp", [0.0, 1.0])
+def test_sample_nan_logits(v, dtype, filtered, temp):
+    """A NaN anywhere in a row shows in its log-probability, also where a
+    whole word of the row is NaN and no number was seen before it."""
+    x = torch.randn(3, v, device=DEV).to(dtype)
+    x[0, :8] = float("nan")
+    x[1, v - 1] = float("nan")
+    full = lambda t, ty: torch.full((3,), t, dtype=ty, device=DEV)
+    tok, lp = ops.sample(x, full(temp, torch.float32), full(-1, torch.int32),
+                         full(0.9 if filtered else 1.0, torch.float32), 3,
+                         no_filter=not filtered)
+    assert lp.isnan().tolist() == [True, True, False]
+    assert ((tok >= 0) & (tok < v)).all()
