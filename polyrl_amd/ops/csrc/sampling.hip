@@ -212,6 +212,7 @@ struct alignas(8) Plan {              // where a row's two selections stand
   float m_scaled, target;             // top-p: largest x/T, mass to reach
   uint32_t prefix_k, prefix_p;        // digits decided so far, left-aligned
   float cnt, mass;                    // count / mass above them
+  uint32_t most;                      // encoding of the largest entry
   int by;                             // 1: top-k, 2: top-p
 };
 
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
                              inv_temp, all, V, split, lds);
     if (threadIdx.x == 0)
       plan = {cut, all.m * inv_temp, p * all.st, 0u, 0u, 0.f, 0.f,
-              (by_k ? 1 : 0) + (by_p ? 2 : 0)};
+              enc_f32(all.m), (by_k ? 1 : 0) + (by_p ? 2 : 0)};
     return;
   }
   const Plan now = plan;
@@ -388,9 +389,12 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   if (MODE == 2 && greedy) return;    // the first pass found it
   const float inv_temp = greedy ? 1.f : 1.0f / temp;
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  // encoding that a kept entry reaches
+  // encoding that a kept entry reaches: the higher threshold, but no more than
+  // the largest entry (with p = 0 the walk stops at the topmost, empty bin)
   const uint32_t tau =
-      MODE == 2 ? max(plans[row].prefix_k, plans[row].prefix_p) : 0;
+      MODE == 2 ? min(max(plans[row].prefix_k, plans[row].prefix_p),
+                      plans[row].most)
+                : 0;
   if (MODE == 1) {                    // the digit passes' bins start at 0
     uint32_t* h = hist + row * hist_words;
     for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)

@@ -231,3 +231,17 @@ def test_sample_nan_logits(v, dtype, filtered, temp):
                          no_filter=not filtered)
     assert lp.isnan().tolist() == [True, True, False]
     assert ((tok >= 0) & (tok < v)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("p", [0.0, 1e-30, 1e-6])
+def test_sample_smallest_top_p(p, dtype):
+    """top-p always keeps the largest logit."""
+    torch.manual_seed(2)
+    x = torch.randn(5, 5000, device=DEV).to(dtype)
+    x[:, 100] = 9.0
+    x[2] -= 100.0                      # all below zero
+    full = lambda t, ty: torch.full((5,), t, dtype=ty, device=DEV)
+    tok, _ = ops.sample(x, full(1.0, torch.float32), full(-1, torch.int32),
+                        full(p, torch.float32), 5, no_filter=False)
+    assert tok.tolist() == [100] * 5
