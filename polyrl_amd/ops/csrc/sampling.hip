@@ -7,7 +7,7 @@
 //    monotone uint32 encoding of the logit (temperature doesn't change order,
 //    so select on raw logits).
 //  * top-p threshold found by the same walk, accumulating per-bin
-//    sum(exp(x/T - m/T)) mass instead of counts.
+//    sum(exp((x - m)/T)) mass instead of counts.
 //  * the draw is Gumbel-argmax over the kept set: argmax(x/T + G_i), exact
 //    categorical sampling in one streaming pass, counter-based RNG
 //    (splitmix64 keyed by (seed, row, i)) so replay is deterministic.
@@ -24,8 +24,10 @@
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
 // maxima is no more than the k-th largest entry; and entries that each have
-// less than (1 - p) / V of the mass have less than 1 - p together, so the
-// nucleus ends above them.  All entries of 64 x 151936 (0.7, 50, 0.9) in LDS
+// less than (1 - p) / 2V of the mass have less than half of 1 - p together, so
+// the nucleus ends above them, by a margin far above the rounding of the sums
+// (total and bins add the same exp((x - m)/T), which is exact near m however
+// large m/T is).  All entries of 64 x 151936 (0.7, 50, 0.9) in LDS
 // atomics took 73 us a digit.
 //
 // What bounds it: integer multiplies of the generator (two 64-bit products a
@@ -209,10 +211,10 @@ DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
 // for top-p's (they part after the first digit).
 struct alignas(8) Plan {              // where a row's two selections stand
   float cut;                          // entries below it stand at neither
-  float m_scaled, target;             // top-p: largest x/T, mass to reach
+  float m, target;                    // largest entry; top-p: mass to reach
   uint32_t prefix_k, prefix_p;        // digits decided so far, left-aligned
   float cnt, mass;                    // count / mass above them
-  uint32_t most;                      // encoding of the largest entry
+  uint32_t least, most;               // encodings of the cut (0: none) and m
   int by;                             // 1: top-k, 2: top-p
 };
 
@@ -254,7 +256,7 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
   if (base + upto >= goal) atomicMin(found, (int)threadIdx.x);
   __syncthreads();
   const int who = *found;
-  if (who == SNT) {                   // numerical slack: keep everything
+  if (who == SNT) {                   // short of the goal: keep all bins
     bin = 0;
     before = 0.f;
     return;
@@ -297,7 +299,8 @@ DEV_INLINE float cut_of(const float* tops, bool by_k, bool by_p, int k, float p,
                         float* lds) {
   float cut = -INFINITY;
   if (by_p && inv_temp > 0.f && p > 0.f)
-    cut = all.m + __logf(0.99f * (1.f - p) * all.st / V) / inv_temp;
+    cut = all.m + __logf(0.5f * (1.f - p) * all.st / V) / inv_temp;
+  if (!(cut > -INFINITY)) cut = -INFINITY;   // (NaN logits)
   const int n = TOPS * split;
   if (!by_k || k > n) return cut;
   // waves' maxima where they are enough, else those of 16 lanes
@@ -346,7 +349,9 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
     const float cut = cut_of(tops + row * split * TOPS, by_k, by_p, k, p,
                              inv_temp, all, V, split, lds);
     if (threadIdx.x == 0)
-      plan = {cut, all.m * inv_temp, p * all.st, 0u, 0u, 0.f, 0.f,
+      plan = {cut, all.m, p * all.st, 0u, 0u, 0.f, 0.f,
+              // (-0 stands below +0 in the encoding)
+              cut > -INFINITY ? enc_f32(cut == 0.f ? -0.f : cut) : 0u,
               enc_f32(all.m), (by_k ? 1 : 0) + (by_p ? 2 : 0)};
     return;
   }
@@ -389,12 +394,15 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   if (MODE == 2 && greedy) return;    // the first pass found it
   const float inv_temp = greedy ? 1.f : 1.0f / temp;
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  // encoding that a kept entry reaches: the higher threshold, but no more than
-  // the largest entry (with p = 0 the walk stops at the topmost, empty bin)
-  const uint32_t tau =
-      MODE == 2 ? min(max(plans[row].prefix_k, plans[row].prefix_p),
-                      plans[row].most)
-                : 0;
+  // encoding that a kept entry reaches: the higher threshold, but no less than
+  // the cut (where rounding leaves the mass in the bins short of its goal the
+  // walk ends at bin 0) and no more than the largest entry (with p = 0 it
+  // stops at the topmost, empty bin)
+  uint32_t tau = 0;
+  if (MODE == 2) {
+    const Plan& plan = plans[row];
+    tau = min(max(max(plan.prefix_k, plan.prefix_p), plan.least), plan.most);
+  }
   if (MODE == 1) {                    // the digit passes' bins start at 0
     uint32_t* h = hist + row * hist_words;
     for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
@@ -509,8 +517,8 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
       const uint32_t e = enc_f32(v[j]);
       const uint32_t bin = (e >> low) & (bins - 1);
       if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
-      if (by_p && (e & above) == plan.prefix_p)
-        atomicAdd(&mass[bin], __expf(v[j] * inv_temp - plan.m_scaled));
+      if (by_p && (e & above) == plan.prefix_p && v[j] != -INFINITY)
+        atomicAdd(&mass[bin], __expf((v[j] - plan.m) * inv_temp));
     }
   }
   __syncthreads();

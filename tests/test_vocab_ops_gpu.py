@@ -245,3 +245,21 @@ def test_sample_smallest_top_p(p, dtype):
     tok, _ = ops.sample(x, full(1.0, torch.float32), full(-1, torch.int32),
                         full(p, torch.float32), 5, no_filter=False)
     assert tok.tolist() == [100] * 5
+
+
+@pytest.mark.parametrize("temp,p", [(0.01, 0.99), (0.01, 0.999), (0.003, 0.9)])
+def test_sample_top_p_far_from_zero(temp, p):
+    """Large logits at a low temperature (x / T in the thousands): the filter
+    still ends where the mass reaches p."""
+    torch.manual_seed(11)
+    n, v = 4096, 1000
+    x = 30 + torch.randn(n, v, device=DEV) * temp
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    tok, _ = ops.sample(x, full(temp, torch.float32), full(-1, torch.int32),
+                        full(p, torch.float32), 9, no_filter=False)
+    s, order = (x.double() / temp).sort(-1, descending=True)
+    mass = torch.softmax(s, -1)
+    above = torch.empty_like(mass).scatter_(1, order, mass.cumsum(-1) - mass)
+    # 32-bit 1 / T moves every x / T here by less than 1e-4 of itself times
+    # the logits' spread, and so the mass above an entry by less than 1e-4
+    assert (above.gather(1, tok[:, None]) < p + 1e-4).all()
