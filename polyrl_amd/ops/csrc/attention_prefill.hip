@@ -87,7 +87,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
                          (long)hq * D * (busy ? 1 : 0));
 
   FragAt<D> at;
-  const float s2 = scale * 1.4426950408889634f;    // scores in powers of two
+  // scores in powers of two.  Hidden keys are marked before the scale is
+  // multiplied in, so a scale of 0 becomes the smallest number: every score is
+  // then 0 all the same, but a hidden one -inf and not -inf * 0
+  const float s2 = scale != 0.f ? scale * 1.4426950408889634f : 0x1p-126f;
   const float hidden = s2 >= 0.f ? -INFINITY : INFINITY;
   float m_run = -1e30f, l_run = 0.f;               // l: this lane's keys only
   f32x16_t o[DT];

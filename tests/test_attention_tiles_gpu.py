@@ -237,3 +237,31 @@ def test_window_prompts(hq, hk, d, window, keep, chunk, extras):
         a += x
     if extras:                         # nothing written beside the slice
         assert (wide[:, :8] == 0).all() and (wide[:, 8 + hq * d:] == 0).all()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("name,hq,hk,d", [("edges", 8, 2, 128),
+                                          ("ragged", 7, 1, 64)])
+def test_scale_zero(name, hq, hk, d, causal):
+    """Scores of zero: the mean of the values a row sees, and no gradient for
+    queries and keys."""
+    torch.manual_seed(3)
+    lens = LENS[name]
+    cu, n = cu_of(lens), sum(lens)
+    q, k, v = (torch.randn(n, h, d, device=DEV).bfloat16().requires_grad_()
+               for h in (hq, hk, hk))
+    out = ops.flash_attn_varlen(q, k, v, cu.to(DEV), 0.0, causal)
+    same = ops.varlen_prefill_attention(q.detach(), k.detach(), v.detach(),
+                                        cu.to(DEV), cu.to(DEV), 0.0, causal)
+    assert torch.equal(out, same)
+    dout = torch.randn(n, hq, d, device=DEV).bfloat16()
+    dq, dk, dv = torch.autograd.grad(out, (q, k, v), dout)
+    assert (dq == 0).all() and (dk == 0).all() and dv.isfinite().all()
+    for i in range(len(lens)):
+        a = slice(cu[i], cu[i + 1])
+        x = [t.detach()[a].double() for t in (q, k, v)]
+        kk, vv = heads(x[1], hq), heads(x[2], hq)
+        want, _ = attend(x[0], kk, vv, 0, causal, 0.0)
+        mass, _ = attend(x[0], kk, vv.abs(), 0, causal, 0.0)
+        bound = 2 ** -8 * (mass + want.abs())
+        assert ((out[a].double() - want).abs() <= bound).all(), lens[i]
