@@ -67,6 +67,18 @@ struct AttnTile {
                                  ((at % GR ^ swz(r)) << 4)) = reg[i];
     }
   }
+
+  // the same with zeros for the rows from ``live`` on: a value that a weight
+  // of 0 meets has to be finite, and the last row, repeated, need not be
+  DEV_INLINE static void store_live(char* tile, i32x4_t (&reg)[LOADS],
+                                    int live) {
+    if (live < ATILE) {                // the same for the whole block
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        if ((int)(threadIdx.x + i * 256) / GR >= live) reg[i] = {0, 0, 0, 0};
+    }
+    store(tile, reg);
+  }
 };
 
 // Per-lane offsets of the two kinds of fragments.  renew() makes them new to

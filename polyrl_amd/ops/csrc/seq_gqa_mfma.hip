@@ -435,6 +435,7 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
     return ti < nkt ? ti * ATILE : kmin + (ti - nkt) * ATILE;
   };
   auto tile_jmax = [&](int ti) { return ti < nkt ? nk - 1 : pmax; };
+  auto tile_live = [&](int ti) { return tile_jmax(ti) - tile_t0(ti) + 1; };
   // cache row of a tile's key i (keys past the tile's last: that one)
   auto slot_of = [&](int ti, int i) {
     const int j = min(tile_t0(ti) + i, tile_jmax(ti));
@@ -479,7 +480,7 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
   fetch(kb, 0);
   T::store(lds[0][0], reg);
   fetch(vb, 0);
-  T::store(lds[0][1], reg);
+  T::store_live(lds[0][1], reg, tile_live(0));
   wait_loads();
   __syncthreads();
 
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
       }
       SCHED_MFMA(4);
     }
-    if (more) T::store(lds[buf ^ 1][1], reg);
+    if (more) T::store_live(lds[buf ^ 1][1], reg, tile_live(ti + 1));
     // (the rows of this tile were last looked up before the last barrier)
     if (wid == 0 && ti + 2 < ntiles) slot_s[buf][lane] = slot_of(ti + 2, lane);
     __syncthreads();

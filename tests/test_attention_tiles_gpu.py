@@ -265,3 +265,44 @@ def test_scale_zero(name, hq, hk, d, causal):
         mass, _ = attend(x[0], kk, vv.abs(), 0, causal, 0.0)
         bound = 2 ** -8 * (mass + want.abs())
         assert ((out[a].double() - want).abs() <= bound).all(), lens[i]
+
+
+@pytest.mark.parametrize("hq,hk,d", [(8, 2, 128), (7, 1, 64), (4, 4, 64)])
+def test_infinite_value_of_the_last_key(hq, hk, d):
+    """An infinite entry of a sequence's last value row gives an infinite
+    entry where that row is seen: what stands in for rows past the end takes
+    no part."""
+    torch.manual_seed(4)
+    lens, page, scale = [1, 33, 200], 16, d ** -0.5
+    cu, n = cu_of(lens).to(DEV), sum(lens)
+    q = torch.randn(n, hq, d, device=DEV).bfloat16()
+    k, v = (torch.randn(n, hk, d, device=DEV).bfloat16() for _ in range(2))
+    ends = (cu[1:] - 1).long()
+    v[ends, :, 5] = float("inf")
+    need = [-(-x // page) for x in lens]
+    table = torch.zeros(3, max(need), dtype=torch.int32, device=DEV)
+    rows = torch.zeros(sum(need) * page, 2, hk, d, device=DEV).bfloat16()
+    at = 0
+    for i, x in enumerate(need):
+        table[i, :x] = torch.arange(at, at + x, device=DEV)
+        a = slice(int(cu[i]), int(cu[i + 1]))
+        rows[at * page:at * page + lens[i], 0] = k[a]
+        rows[at * page:at * page + lens[i], 1] = v[a]
+        at += x
+    i32 = dict(dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(x, **i32) for x in lens])
+    seq = torch.repeat_interleave(torch.arange(3, **i32),
+                                  torch.tensor(lens, device=DEV))
+    paged = rows.view(-1, page, 2, hk, d)
+    got = {
+        "prompt": ops.varlen_prefill_attention(q, k, v, cu, cu, scale,
+                                               True)[ends],
+        "window": ops.seq.gqa_window_attention(
+            q.flatten(1), paged.flatten(2), table, seq, pos, hq, hk, d, d,
+            1 << 20, 0, None, None, None, scale, torch.bfloat16,
+            tiles=ops.seq.attention_tiles(lens, DEV)).view(n, hq, d)[ends],
+    }
+    other = [j for j in range(d) if j != 5]
+    for name, out in got.items():
+        assert (out[:, :, 5] == float("inf")).all(), name
+        assert out[:, :, other].isfinite().all(), name
