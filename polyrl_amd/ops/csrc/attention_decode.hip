@@ -12,13 +12,13 @@
 //     maximum and sum take two lane exchanges per 32 keys.
 //   * O^T += V^T P^T: V rows go through 8 KiB of LDS of the wave's own and come
 //     back turned (ds_read_b64_tr_b16); the weights are the operand as they
-//     stand in the accumulators.  They stay as exact as 32-bit ones: each is
-//     the sum of two bf16 numbers, and both are multiplied.
+//     stand in the accumulators.  They stay the 32-bit numbers they are: each
+//     is the sum of three bf16 numbers, and all three are multiplied.
 // What bounds it: reading K and V once.  (With per-key dot products, shuffles
 // and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
 // at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
-// tokens, 32/8 heads of 128, 59.5 -> 44.6 us; 33 rows of 1900 .. 8192, 28/4
-// heads, 264 -> 86 us (4.1 TB/s).
+// tokens, 32/8 heads of 128, 59.5 -> 45.2 us; 33 rows of 1900 .. 8192, 28/4
+// heads, 264 -> 86.6 us (4.1 TB/s).  (With two parts a weight 44.6 and 86.0.)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -158,16 +158,25 @@ __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
     const float alpha = exp2_hw(m_run - mn);
     m_run = mn;
     l_run *= alpha;
-    // weights as hi + lo, both bf16: the remainder is below 2^-17 of a weight
-    bf16x8_t hi, lo;
+    // weights as the sum of three bf16 numbers, the 24 bits of a 32-bit one in
+    // groups of eight.  None is 0 unless the weight is (the smallest bf16
+    // number stands in), so that an infinite value stays infinite.
+    i16x8_t w3[3];
 #pragma unroll
     for (int n = 0; n < 2; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float p = exp2_hw(s[n][r] - mn);
         l_run += p;
-        hi[4 * n + r] = (__bf16)p;
-        lo[4 * n + r] = (__bf16)(p - (float)hi[4 * n + r]);
+        float rest = p;
+        unsigned least = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const unsigned bits = __float_as_uint(rest);
+          w3[i][4 * n + r] = (short)max(bits >> 16, least);
+          if (i == 0) least = min(bits, 1u);
+          rest -= __uint_as_float(bits & 0xFFFF0000u);
+        }
       }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -175,6 +184,13 @@ __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
       for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
 
     // ---- V rows into the wave's LDS, turned fragments back --------------------
+    // (zeros past the stretch: its last row, which stands in, need not be
+    // finite, and 0 * inf is NaN)
+    if (t0 + DEC_KEYS > cend) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (t0 + i * RPI + vrow >= cend) vv[i] = {0, 0, 0, 0};
+    }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int r = i * RPI + vrow;
@@ -190,8 +206,10 @@ __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
           (lds_i16x4_p)(vs + (vb ^ (dt << 5))));
       const bf16x8_t vt = __builtin_bit_cast(
           bf16x8_t, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, hi, o[dt], 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, lo, o[dt], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            vt, __builtin_bit_cast(bf16x8_t, w3[i]), o[dt], 0, 0, 0);
     }
     __builtin_amdgcn_wave_barrier();
   }

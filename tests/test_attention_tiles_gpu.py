@@ -138,8 +138,8 @@ def test_backward(name, hq, hk, d, causal):
 def test_decode(hq, hk, d, page_size, wide):
     """Paged decode at the edges of its 32-key rounds and 128-key stretches;
     ``wide``: a page table far wider than the contexts (a captured graph's),
-    which divides them further.  The weights are as exact as 32-bit ones, so
-    an entry is off by its rounding to bf16 and 2^-14 of its terms."""
+    which divides them further.  The weights are 32-bit ones, so an entry is
+    off by its rounding to bf16 and 2^-14 of its terms."""
     torch.manual_seed(9)
     lens = [1, 31, 32, 33, 127, 128, 129, 300, 1025, 2]
     need = [-(-n // page_size) for n in lens]
@@ -301,8 +301,38 @@ def test_infinite_value_of_the_last_key(hq, hk, d):
             q.flatten(1), paged.flatten(2), table, seq, pos, hq, hk, d, d,
             1 << 20, 0, None, None, None, scale, torch.bfloat16,
             tiles=ops.seq.attention_tiles(lens, DEV)).view(n, hq, d)[ends],
+        "decode": ops.paged_attention_decode(
+            q[ends], paged[:, :, 0].contiguous(), paged[:, :, 1].contiguous(),
+            table, torch.tensor(lens, **i32), scale),
     }
     other = [j for j in range(d) if j != 5]
     for name, out in got.items():
         assert (out[:, :, 5] == float("inf")).all(), name
         assert out[:, :, other].isfinite().all(), name
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_weights(d):
+    """Weights are held in 32 bits: the difference of two almost equal ones
+    (values +1 and -1, beside a larger weight with the value 0) is exact to a
+    bf16 rounding and a few 2^-24, where weights of 16 or 17 bits would be off
+    by 2^-20."""
+    hq, n, scale = 8, 64, 0.125
+    q = torch.zeros(n, hq, d)
+    q[:, :, 0] = 4 + 12 * torch.rand(
+        n, hq, generator=torch.Generator().manual_seed(1))
+    q[:, :, 1] = 2.0 ** -5
+    q = q.to(DEV).bfloat16()
+    k = torch.zeros(1, 16, 1, d, device=DEV).bfloat16()
+    v = torch.zeros(1, 16, 1, d, device=DEV).bfloat16()
+    k[0, 0, 0, 0], k[0, 1:3, 0, 0], k[0, 2, 0, 1] = 1.0, 0.75, 2.0 ** -5
+    v[0, 1], v[0, 2] = 1.0, -1.0
+    out = ops.paged_attention_decode(
+        q, k, v, torch.zeros(n, 1, dtype=torch.int32, device=DEV),
+        torch.full((n,), 3, dtype=torch.int32, device=DEV), scale)
+    p = torch.softmax(torch.einsum("nhd,kd->nhk", q.double(),
+                                   k[0, :3, 0].double()) * scale, -1)
+    want = (p[..., 1] - p[..., 2])[..., None]
+    # a score, its exponential and the sums are each rounded to 24 bits
+    bound = 2 ** -8 * want.abs() + 2.0 ** -22
+    assert ((out.double() - want).abs() <= bound).all()
