@@ -94,6 +94,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     del = half_sum(del);
   }
   if (busy && lane < 32 && row < Lq) delta[tok * Hq + hq] = del;
+  del *= scale;                      // dS is rounded with the scale in it
   frag_global<D>(qf, q + tok * ldq + (long)hq * D);
   const float s2 = scale * 1.4426950408889634f;
   const float lse2 = lse[tok * Hq + hq] * 1.4426950408889634f;
@@ -162,7 +163,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
           if (acc_row(r) > last) s[r] = 0.f;
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] *= dp[r] - del;
+      for (int r = 0; r < 16; ++r)
+        s[r] *= __builtin_fmaf(dp[r], scale, -del);
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const bf16x8_t ds = acc_operand(s, st);
@@ -183,7 +185,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     __syncthreads();
   }
 
-  // ---- dQ = scale * acc, turned through LDS to whole rows -------------------
+  // ---- dQ, turned through LDS to whole rows ---------------------------------
   char* mine = &lds[0][0][0] + wid * (32 * D * 2);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     for (int i = 0; i < 4; ++i) {
       bf16x4 w;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) w.v[t] = f2bf(acc[dt][4 * i + t] * scale);
+      for (int t = 0; t < 4; ++t) w.v[t] = f2bf(acc[dt][4 * i + t]);
       const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
       *reinterpret_cast<bf16x4*>(
           mine + (lane & 31) * (2 * D) +
@@ -228,7 +230,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   constexpr bool V_LDS = D == 128;   // V does not fit beside the gradients
   // Q (two buffers), dO, V; at the end the exchange of 4 x 32 x D floats
   __shared__ __attribute__((aligned(16))) char lds[4][T::BYTES];
-  __shared__ __attribute__((aligned(16))) float row_s[2][ATILE];  // lse, delta
+  // log-sum-exp (in powers of two) and scale * delta of the rows
+  __shared__ __attribute__((aligned(16))) float row_s[2][ATILE];
 
   const int G = Hq / Hk;
   const int item = die_item(ntiles * Hk * nsplit);
@@ -285,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   auto store_rows = [&]() {
     // rows past the end weigh nothing: 2^(s - inf) = 0
     if (wid == 0) row_s[0][lane] = rlive ? rowv * 1.4426950408889634f : INFINITY;
-    if (wid == 1) row_s[1][lane] = rlive ? rowv : 0.f;
+    if (wid == 1) row_s[1][lane] = rlive ? rowv * scale : 0.f;
   };
   auto fetch_q = [&]() { T::fetch(reg, qb0 + (long)fg * D, ldq, fq, Lq); };
   auto fetch_do = [&]() {             // and on to the next tile
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
           float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
           if (8 * i + t < border) w = 0.f;
           s[r] = w;
-          dp[r] = w * (dp[r] - d4[t]);
+          dp[r] = w * __builtin_fmaf(dp[r], scale, -d4[t]);
         }
       }
 #pragma unroll
@@ -415,7 +418,6 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   __syncthreads();
   const bool ok = key < Lk;
   const long o = ((long)krow * Hk + hk) * D;
-  const float f = qh == 0 ? 1.f : scale;           // dK carries the scale
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -424,8 +426,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int r = 4 * i + t;
-        w.v[t] = f * ((qh == 0 ? av[dt][r] : ak[dt][r]) +
-                      other[(dt * 16 + r) * 64 + lane]);
+        w.v[t] = (qh == 0 ? av[dt][r] : ak[dt][r]) +
+                 other[(dt * 16 + r) * 64 + lane];
       }
       const int d = dt * 32 + 8 * i + 4 * (lane >> 5);
       if (!ok) continue;
