@@ -318,9 +318,11 @@ class _RMSNormTrain(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, dh_out):
-        if dy is None:
-            return dh_out, dh_out if ctx.has_res else None, None, None
         h, w, rstd = ctx.saved_tensors
+        if dy is None:
+            dx = dh_out if dh_out is not None else torch.zeros_like(h)
+            return (dx, dx if ctx.has_res else None, torch.zeros_like(w),
+                    None)
         ext = _require_ext()
         dx, dw = ext.rmsnorm_train_bwd(
             dy, dh_out if dh_out is not None else torch.Tensor(), h, w, rstd)

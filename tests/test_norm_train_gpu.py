@@ -51,3 +51,34 @@ def test_backward(t, h, use):
         size = (gy.double() * y64 / w64).abs().sum(0)
         off = (w.grad.double() - w64.grad).abs()
         assert (off <= 2 ** -8 * w64.grad.abs() + 1e-5 * size + 1e-6).all()
+
+
+def test_backward_of_the_sum_alone():
+    """Where only the sum is used the weight's gradient is zero, not absent."""
+    x, res = (torch.randn(5, 64, device=DEV).bfloat16().requires_grad_()
+              for _ in range(2))
+    w = torch.randn(64, device=DEV).bfloat16().requires_grad_()
+    _, s = ops.fused_add_rmsnorm_train(x, res, w, 1e-5)
+    g = torch.randn(5, 64, device=DEV).bfloat16()
+    dx, dres, dw = torch.autograd.grad(s, (x, res, w), g)
+    assert torch.equal(dx, g) and torch.equal(dres, g)
+    assert dw.dtype == w.dtype and (dw == 0).all()
+
+
+def test_backward_of_nothing():
+    """No gradient reaches either output: zeros."""
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a, b):
+            return a + b
+
+        @staticmethod
+        def backward(ctx, g):
+            return None, None
+
+    x, res = (torch.randn(5, 64, device=DEV).bfloat16().requires_grad_()
+              for _ in range(2))
+    w = torch.randn(64, device=DEV).bfloat16().requires_grad_()
+    out = Drop.apply(*ops.fused_add_rmsnorm_train(x, res, w, 1e-5))
+    for g, t in zip(torch.autograd.grad(out.sum(), (x, res, w)), (x, res, w)):
+        assert g.shape == t.shape and (g == 0).all()
