@@ -67,7 +67,9 @@ def gather_logprobs_entropy(logits: torch.Tensor, labels: torch.Tensor
                             ) -> Tuple[torch.Tensor, torch.Tensor]:
     logp = torch.log_softmax(logits.float(), dim=-1)
     lp = torch.gather(logp, -1, labels.unsqueeze(-1)).squeeze(-1)
-    ent = -(logp.exp() * logp).sum(-1)
+    # a banned token (-inf) has no part in the entropy: 0, not 0 * inf
+    low = torch.finfo(logp.dtype).min
+    ent = -(logp.exp() * logp.clamp_min(low)).sum(-1)
     return lp, ent
 
 

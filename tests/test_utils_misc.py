@@ -163,3 +163,16 @@ def test_get_tokenizer_offline_branches(tmp_path):
     assert get_tokenizer("llama3-8b") is None          # registry name
     assert get_tokenizer(str(tmp_path)) is None        # dir, no tok files
     assert get_tokenizer(str(tmp_path / "nope")) is None
+
+
+def test_entropy_with_banned_tokens():
+    """-inf logits take no part in the entropy of the CPU form."""
+    import torch
+    import polyrl_amd.ops as ops
+    x = torch.randn(3, 40, generator=torch.Generator().manual_seed(0))
+    x[:, ::3] = -float("inf")
+    p = torch.softmax(x.double(), -1)
+    _, ent = ops.gather_logprobs(x, torch.ones(3, dtype=torch.long),
+                                 want_entropy=True)
+    want = -torch.special.xlogy(p, p).sum(-1)
+    assert torch.allclose(ent.double(), want, atol=1e-5)

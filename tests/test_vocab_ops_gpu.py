@@ -263,3 +263,18 @@ def test_sample_top_p_far_from_zero(temp, p):
     # 32-bit 1 / T moves every x / T here by less than 1e-4 of itself times
     # the logits' spread, and so the mass above an entry by less than 1e-4
     assert (above.gather(1, tok[:, None]) < p + 1e-4).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v", [(2, 64), (2, 50257), (1030, 500)])
+def test_entropy_with_banned_tokens(n, v, dtype):
+    """-inf logits take no part in the entropy."""
+    torch.manual_seed(6)
+    x = (torch.randn(n, v, device=DEV) * 2).to(dtype)
+    x[:, : v // 3] = -float("inf")
+    x[0, v // 2] = -float("inf")
+    lab = torch.full((n,), v - 1, device=DEV)
+    p = torch.softmax(x.double(), -1)
+    want = -torch.special.xlogy(p, p).sum(-1)
+    _, ent = ops.gather_logprobs(x, lab, want_entropy=True)
+    assert (ent.double() - want).abs().max() <= 2e-5 * (1 + want.max())
