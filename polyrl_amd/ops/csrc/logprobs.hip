@@ -149,19 +149,32 @@ __global__ void gather_logprobs_bwd_kernel(
   const float g = dlp[row];
   const float l = lse[row];
   const long lab = labels[row];
-  const bf16x8* xp = reinterpret_cast<const bf16x8*>(x);
-  bf16x8* dp = reinterpret_cast<bf16x8*>(dx);
-  const int n8 = V / 8;
+  // 16-byte words of dx from its first 16-byte address on, as in the forward;
+  // those of x too, unless the two stand differently (x may be a slice)
+  const int lead = lead_of(dx, V);
+  const int n8 = (V - lead) / 8;
+  const bool same = (((uintptr_t)(x + lead)) & 15) == 0;
   for (int i = threadIdx.x; i < n8; i += blockDim.x) {
-    bf16x8 v = xp[i], o;
+    const bf16_t* at = x + lead + (long)i * 8;
+    bf16x8 v, o;
+    if (same) {
+      v = *reinterpret_cast<const bf16x8*>(at);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v.v[j] = at[j];
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       o.v[j] = f2bf(-g * __expf(bf2f(v.v[j]) - l));
-    dp[i] = o;
+    *reinterpret_cast<bf16x8*>(dx + lead + (long)i * 8) = o;
   }
-  // tail when V % 8 != 0
-  for (int i = n8 * 8 + threadIdx.x; i < V; i += blockDim.x)
+  // the numbers before the first and behind the last whole word
+  const int rest = V - lead - n8 * 8;
+  if ((int)threadIdx.x < lead + rest) {
+    const int i = (int)threadIdx.x < lead ? threadIdx.x
+                                          : n8 * 8 + threadIdx.x;
     dx[i] = f2bf(-g * __expf(bf2f(x[i]) - l));
+  }
   // add the onehot term after every softmax write landed
   __syncthreads();
   if (threadIdx.x == 0)

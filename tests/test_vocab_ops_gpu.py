@@ -278,3 +278,23 @@ def test_entropy_with_banned_tokens(n, v, dtype):
     want = -torch.special.xlogy(p, p).sum(-1)
     _, ent = ops.gather_logprobs(x, lab, want_entropy=True)
     assert (ent.double() - want).abs().max() <= 2e-5 * (1 + want.max())
+
+
+@pytest.mark.parametrize("n,v,skip", [(3, 50257, 0), (5, 333, 3), (4, 4096, 1),
+                                      (2, 5, 0), (6, 11, 1), (3, 64, 8)])
+def test_logprob_gradients_of_unaligned_rows(n, v, skip):
+    """Rows that do not start at 16-byte addresses, and logits that do not
+    start where their gradient does."""
+    torch.manual_seed(2)
+    flat = torch.randn(skip + n * v, device=DEV).bfloat16()
+    x = flat[skip:].view(n, v)
+    lab = torch.arange(n, device=DEV) * 7 % v
+    dlp = torch.randn(n, device=DEV)
+    g = x.detach().requires_grad_()
+    ops.gather_logprobs_train(g, lab).backward(dlp)
+    dx = -dlp[:, None].double() * torch.softmax(x.double(), -1)
+    dx.scatter_add_(1, lab[:, None], dlp[:, None].double())
+    # rounded once to bf16, the label's entry twice
+    tol = 2 ** -7 * dx.abs() + 1e-6
+    tol.scatter_add_(1, lab[:, None], 2 ** -8 * dlp[:, None].abs().double())
+    assert ((g.grad.double() - dx).abs() <= tol).all()
