@@ -19,7 +19,8 @@
 // the pieces meet in small per-row arrays and a merging launch.  Without a
 // filter that is one pass: sums of the raw softmax and the draw together.
 // With one: sums, one pass per radix digit (11 bits, then the rest of a bf16
-// number's 16 or an fp32 number's 32), the draw over the kept set.
+// number's 16 or an fp32 number's 32), the draw over the kept set.  Short rows
+// take the same steps in one launch, a block each.
 //
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
@@ -216,6 +217,21 @@ struct alignas(8) Plan {              // where a row's two selections stand
   float cnt, mass;                    // count / mass above them
   uint32_t least, most;               // encodings of the cut (0: none) and m
   int by;                             // 1: top-k, 2: top-p
+
+  DEV_INLINE Plan(float cut_, const Sums<true>& all, float p, bool by_k,
+                  bool by_p)
+      : cut(cut_), m(all.m), target(p * all.st), prefix_k(0), prefix_p(0),
+        cnt(0.f), mass(0.f),
+        // (-0 stands below +0 in the encoding)
+        least(cut_ > -INFINITY ? enc_f32(cut_ == 0.f ? -0.f : cut_) : 0u),
+        most(enc_f32(all.m)), by((by_k ? 1 : 0) + (by_p ? 2 : 0)) {}
+  // encoding that a kept entry reaches: the higher threshold, but no less than
+  // the cut (where rounding leaves the mass in the bins short of its goal the
+  // walk ends at bin 0) and no more than the largest entry (with p = 0 it
+  // stops at the topmost, empty bin)
+  DEV_INLINE uint32_t threshold() const {
+    return min(max(max(prefix_k, prefix_p), least), most);
+  }
 };
 
 // Walks the bins from the top until the running count reaches ``need`` (or
@@ -293,15 +309,14 @@ DEV_INLINE int digit_bins(int d) {
 }
 
 // Entries below this stand at neither threshold of their row (the top of this
-// file); lds: TOPS * split floats.
-DEV_INLINE float cut_of(const float* tops, bool by_k, bool by_p, int k, float p,
-                        float inv_temp, const Sums<true>& all, int V, int split,
+// file).  tops: n maxima of 16 lanes each; lds: n floats.
+DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
+                        float p, float inv_temp, const Sums<true>& all, int V,
                         float* lds) {
   float cut = -INFINITY;
   if (by_p && inv_temp > 0.f && p > 0.f)
     cut = all.m + __logf(0.5f * (1.f - p) * all.st / V) / inv_temp;
   if (!(cut > -INFINITY)) cut = -INFINITY;   // (NaN logits)
-  const int n = TOPS * split;
   if (!by_k || k > n) return cut;
   // waves' maxima where they are enough, else those of 16 lanes
   const int width = k <= n / 4 ? 4 : 1, m = n / width;
@@ -346,13 +361,9 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
     const bool by_p = temp != 0.f && p < 1.0f;
     const float inv_temp = temp == 0.f ? 1.f : 1.0f / temp;
     const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
-    const float cut = cut_of(tops + row * split * TOPS, by_k, by_p, k, p,
-                             inv_temp, all, V, split, lds);
-    if (threadIdx.x == 0)
-      plan = {cut, all.m, p * all.st, 0u, 0u, 0.f, 0.f,
-              // (-0 stands below +0 in the encoding)
-              cut > -INFINITY ? enc_f32(cut == 0.f ? -0.f : cut) : 0u,
-              enc_f32(all.m), (by_k ? 1 : 0) + (by_p ? 2 : 0)};
+    const float cut = cut_of(tops + row * split * TOPS, split * TOPS, by_k, by_p,
+                             k, p, inv_temp, all, V, lds);
+    if (threadIdx.x == 0) plan = Plan(cut, all, p, by_k, by_p);
     return;
   }
   const Plan now = plan;
@@ -377,44 +388,16 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
 // ------------------------------------------------------------- one pass
 // MODE 0: sums and draw in one (no filter); 1: sums (and the largest logit)
 // of a filtered row; 2: its draw.
-template <typename T, int MODE>
-__global__ __launch_bounds__(SNT) void sample_pass_kernel(
-    Share* __restrict__ share, float* __restrict__ tops,
-    uint32_t* __restrict__ hist, int hist_words,
-    const Plan* __restrict__ plans, const T* __restrict__ logits,
-    const float* __restrict__ temperature, uint64_t seed,
-    const long long* __restrict__ seed_ptr, int V, int split) {
-  __shared__ Share part[SNW];
-  const long row = blockIdx.x / split;
-  const int piece = blockIdx.x % split;
-  if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
-  const VocabRow<T> r(logits + row * V, V);
-  const float temp = temperature[row];
-  const bool greedy = temp == 0.f;
-  if (MODE == 2 && greedy) return;    // the first pass found it
-  const float inv_temp = greedy ? 1.f : 1.0f / temp;
-  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  // encoding that a kept entry reaches: the higher threshold, but no less than
-  // the cut (where rounding leaves the mass in the bins short of its goal the
-  // walk ends at bin 0) and no more than the largest entry (with p = 0 it
-  // stops at the topmost, empty bin)
-  uint32_t tau = 0;
-  if (MODE == 2) {
-    const Plan& plan = plans[row];
-    tau = min(max(max(plan.prefix_k, plan.prefix_p), plan.least), plan.most);
-  }
-  if (MODE == 1) {                    // the digit passes' bins start at 0
-    uint32_t* h = hist + row * hist_words;
-    for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
-      h[i] = 0;
-  }
-
+//
+// One thread's part of a pass over the groups [first, first + SNT) of every
+// ``stride``.  Every lane of a wave takes part in every round (the draw votes).
+template <int MODE, typename T>
+DEV_INLINE void walk(const VocabRow<T>& r, int first, int stride, bool greedy,
+                     float inv_temp, uint64_t rowkey, uint32_t tau,
+                     Sums<MODE == 1>& sums, Draw& d) {
   constexpr int VEC = VocabRow<T>::VEC;
   const int groups = r.groups();
-  Sums<MODE == 1> sums;
-  Draw d;
-  // every lane of a wave takes part in every round (the draw votes)
-  for (int g0 = piece * SNT; g0 < groups; g0 += split * SNT) {
+  for (int g0 = first; g0 < groups; g0 += stride) {
     const int g = g0 + threadIdx.x;
     float v[VEC];
     if (g < groups) {
@@ -436,9 +419,39 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
           if (v[j] == c) d.best_i = i0 + j;
       }
     } else {
-      d.add(v, c, i0, V, rowkey, inv_temp, tau);
+      d.add(v, c, i0, r.V, rowkey, inv_temp, tau);
     }
   }
+}
+
+template <typename T, int MODE>
+__global__ __launch_bounds__(SNT) void sample_pass_kernel(
+    Share* __restrict__ share, float* __restrict__ tops,
+    uint32_t* __restrict__ hist, int hist_words,
+    const Plan* __restrict__ plans, const T* __restrict__ logits,
+    const float* __restrict__ temperature, uint64_t seed,
+    const long long* __restrict__ seed_ptr, int V, int split) {
+  __shared__ Share part[SNW];
+  const long row = blockIdx.x / split;
+  const int piece = blockIdx.x % split;
+  if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
+  const VocabRow<T> r(logits + row * V, V);
+  const float temp = temperature[row];
+  const bool greedy = temp == 0.f;
+  if (MODE == 2 && greedy) return;    // the first pass found it
+  const float inv_temp = greedy ? 1.f : 1.0f / temp;
+  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
+  const uint32_t tau = MODE == 2 ? plans[row].threshold() : 0;
+  if (MODE == 1) {                    // the digit passes' bins start at 0
+    uint32_t* h = hist + row * hist_words;
+    for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
+      h[i] = 0;
+  }
+
+  Sums<MODE == 1> sums;
+  Draw d;
+  walk<MODE>(r, piece * SNT, split * SNT, greedy, inv_temp, rowkey, tau, sums,
+             d);
   if (MODE == 1) {                    // largest of each 16 lanes
     float t = d.best;
 #pragma unroll
@@ -484,6 +497,34 @@ __global__ __launch_bounds__(64) void sample_merge_kernel(
   }
 }
 
+// a thread's entries of the groups [first, ..) of every ``stride`` into the
+// bins of a digit, if they share the digits before it with a threshold
+template <typename T>
+DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
+                          int digit, const Plan& plan, float inv_temp,
+                          uint32_t* cnt, float* mass) {
+  constexpr int VEC = VocabRow<T>::VEC;
+  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+  const uint32_t above = digit == 0 ? 0u
+      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
+  const bool by_k = plan.by & 1, by_p = plan.by & 2;
+  const int groups = r.groups();
+  for (int g = first + threadIdx.x; g < groups; g += stride) {
+    float v[VEC];
+    r.load(g, v);
+    const int i0 = r.first(g);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if (v[j] < plan.cut || (unsigned)(i0 + j) >= (unsigned)r.V) continue;
+      const uint32_t e = enc_f32(v[j]);
+      const uint32_t bin = (e >> low) & (bins - 1);
+      if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
+      if (by_p && (e & above) == plan.prefix_p && v[j] != -INFINITY)
+        atomicAdd(&mass[bin], __expf((v[j] - plan.m) * inv_temp));
+    }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(SNT) void sample_digit_kernel(
     uint32_t* __restrict__ hist, int hist_words,
@@ -495,38 +536,111 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
   const int piece = blockIdx.x % split;
   const Plan plan = plans[row];
   if (plan.by == 0) return;
-  const bool by_k = plan.by & 1, by_p = plan.by & 2;
   const float inv_temp = 1.0f / temperature[row];
   uint32_t* h = hist + row * hist_words + digit * 4 * DIGIT;
 
-  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
-  const uint32_t above = digit == 0 ? 0u
-      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
+  const int bins = digit_bins<T>(digit);
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
   __syncthreads();
   const VocabRow<T> r(logits + row * V, V);
-  constexpr int VEC = VocabRow<T>::VEC;
-  const int groups = r.groups();
-  for (int g = piece * SNT + threadIdx.x; g < groups; g += split * SNT) {
-    float v[VEC];
-    r.load(g, v);
-    const int i0 = r.first(g);
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      if (v[j] < plan.cut || (unsigned)(i0 + j) >= (unsigned)V) continue;
-      const uint32_t e = enc_f32(v[j]);
-      const uint32_t bin = (e >> low) & (bins - 1);
-      if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
-      if (by_p && (e & above) == plan.prefix_p && v[j] != -INFINITY)
-        atomicAdd(&mass[bin], __expf((v[j] - plan.m) * inv_temp));
-    }
-  }
+  fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
   __syncthreads();
   uint32_t* hc = h;
   float* hm = reinterpret_cast<float*>(h + (digit == 0 ? 1 : 3) * DIGIT);
   for (int i = threadIdx.x; i < bins; i += SNT) {
     if (cnt[i]) atomicAdd(&hc[i], cnt[i]);
     if (mass[i] != 0.f) atomicAdd(&hm[i], mass[i]);
+  }
+}
+
+// ------------------------------------------------------------- short rows
+// The same steps with one block per row, in one launch: of a short row the
+// steps are shorter than the launches of the pieces and plans.
+template <typename T, bool FILTER>
+__global__ __launch_bounds__(SNT) void sample_row_kernel(
+    int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
+    const T* __restrict__ logits, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p,
+    uint64_t seed, const long long* __restrict__ seed_ptr, int V) {
+  __shared__ Share part[SNW];
+  __shared__ float lds[TOPS], tops[FILTER ? TOPS : 1];
+  __shared__ uint32_t cnt[FILTER ? DIGIT : 1];
+  __shared__ float mass[FILTER ? DIGIT : 1];
+  const long row = blockIdx.x;
+  if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
+  const VocabRow<T> r(logits + row * V, V);
+  const float temp = temperature[row];
+  const bool greedy = temp == 0.f;
+  const float inv_temp = greedy ? 1.f : 1.0f / temp;
+  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+
+  Sums<FILTER> sums;
+  Draw d;
+  walk<FILTER ? 1 : 0>(r, 0, SNT, greedy, inv_temp, rowkey, 0u, sums, d);
+  if (FILTER) {                       // largest of each 16 lanes
+    float t = d.best;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) t = fmaxf(t, __shfl_xor(t, off, 64));
+    if (threadIdx.x % 16 == 0) tops[threadIdx.x / 16] = t;
+  }
+  sums.wave(inv_temp);
+  wave_best(d.best, d.best_i);
+  if (lane == 0) part[wid] = {sums.m, sums.s, sums.st, d.best, d.best_i, 0};
+  __syncthreads();
+  sums = Sums<FILTER>();              // of the whole row, in every thread
+  for (int w = 0; w < SNW; ++w) {
+    sums.merge(part[w].m, part[w].s, part[w].st, inv_temp);
+    if (better(part[w].best, part[w].best_i, d.best, d.best_i))
+      d.best = part[w].best, d.best_i = part[w].best_i;
+  }
+  if constexpr (FILTER) {
+    if (!greedy) {
+      const int k = top_k[row];
+      const float p = top_p[row];
+      const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
+      uint32_t tau = 0;
+      if (by_k || by_p) {
+        Plan plan(cut_of(tops, TOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
+                  sums, p, by_k, by_p);
+        for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
+          const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+          for (int i = threadIdx.x; i < bins; i += SNT)
+            cnt[i] = 0, mass[i] = 0.f;
+          __syncthreads();
+          fill_bins(r, 0, SNT, digit, plan, inv_temp, cnt, mass);
+          __syncthreads();
+          int bin;
+          float before;
+          if (by_k) {
+            find_bin<false>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
+            plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
+          }
+          if (by_p) {
+            find_bin<true>(reinterpret_cast<const uint32_t*>(mass), bins,
+                           plan.mass, plan.target, lds, bin, before);
+            plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
+          }
+          __syncthreads();            // the bins were read
+        }
+        tau = plan.threshold();
+      }
+      Draw pick;
+      Sums<false> none;
+      walk<2>(r, 0, SNT, false, inv_temp, rowkey, tau, none, pick);
+      wave_best(pick.best, pick.best_i);
+      __syncthreads();                // the shares were read
+      if (lane == 0) part[wid].best = pick.best, part[wid].best_i = pick.best_i;
+      __syncthreads();
+      d.best = part[0].best, d.best_i = part[0].best_i;
+      for (int w = 1; w < SNW; ++w)
+        if (better(part[w].best, part[w].best_i, d.best, d.best_i))
+          d.best = part[w].best, d.best_i = part[w].best_i;
+    }
+  }
+  if (threadIdx.x == 0) {
+    out_tokens[row] = d.best_i;
+    out_logprobs[row] = (float)r.x[d.best_i] - (sums.m + __logf(sums.s));
   }
 }
 
@@ -542,6 +656,21 @@ static void launch_sample(torch::Tensor& out_tokens,
   const int V = logits.size(1);
   if (N == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
+  // Short rows: one launch.  Per call, one to 128 rows of 4096 bf16 numbers: 8 to
+  // 9 us (11 in pieces), filtered 22 to 30 (36 to 51), filtered with a
+  // temperature of 0 7.6 (31).  Without a filter one block takes longer than
+  // the pieces from about 8192 numbers on (12.4 and 11.6 us, 64 rows), with
+  // one from 12000 (fp32, 58 and 55 us).
+  if (V <= (no_filter ? 4096 : 8192)) {
+    auto kern = no_filter ? sample_row_kernel<T, false>
+                          : sample_row_kernel<T, true>;
+    kern<<<dim3((unsigned)N), dim3(SNT), 0, stream>>>(
+        out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
+        (const T*)logits.data_ptr(), temperature.data_ptr<float>(),
+        top_k.data_ptr<int>(), top_p.data_ptr<float>(), seed, seed_ptr, V);
+    HIP_CHECK_KERNEL();
+    return;
+  }
   // pieces of a row: 2048 blocks in all (eight per CU; 128 x 128256 takes 37
   // us with 512 blocks, 33 with 1024, 32 with 2048, 36 with 4096), half of
   // that for the short passes of filtered rows (64 x 151936: 63, 55, 60, 62

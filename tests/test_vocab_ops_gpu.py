@@ -298,3 +298,13 @@ def test_logprob_gradients_of_unaligned_rows(n, v, skip):
     tol = 2 ** -7 * dx.abs() + 1e-6
     tol.scatter_add_(1, lab[:, None], 2 ** -8 * dlp[:, None].abs().double())
     assert ((g.grad.double() - dx).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("v", [4095, 4096, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("temp,k,p", [(1.0, -1, 1.0), (0.7, 15, 0.9),
+                                      (0.7, 17, 1.0), (0.0, 3, 0.5)])
+def test_sample_short_rows(v, dtype, temp, k, p):
+    """Rows on both sides of the lengths up to which one block takes a row;
+    k on both sides of the maxima that such a block keeps."""
+    test_sample_against_its_definition(5, v, dtype, temp, k, p)
