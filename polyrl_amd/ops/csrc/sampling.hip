@@ -25,11 +25,12 @@
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
 // maxima is no more than the k-th largest entry; and entries that each have
-// less than (1 - p) / 2V of the mass have less than half of 1 - p together, so
-// the nucleus ends above them, by a margin far above the rounding of the sums
-// (total and bins add the same exp((x - m)/T), which is exact near m however
-// large m/T is).  All entries of 64 x 151936 (0.7, 50, 0.9) in LDS
-// atomics took 73 us a digit.
+// less than 0.99 (1 - p) / V of the mass have less than 1 - p together, so the
+// nucleus ends above them.  (Total and bins add the same exp((x - m)/T), which
+// is exact near m however large m/T is; should rounding leave the bins short
+// of p all the same, the nucleus ends at the cut.)  All entries of 64 x 151936
+// (0.7, 50, 0.9) in LDS atomics took 73 us a digit; half of 1 - p in place of
+// 0.99 takes top-p 0.95 of 256 x 152064 from 229 to 254 us.
 //
 // What bounds it: integer multiplies of the generator (two 64-bit products a
 // number).  The two logarithms of a number's noise are only taken where its
@@ -67,7 +68,7 @@ DEV_INLINE uint32_t rng_bits(uint64_t rowkey, int i0, int j) {
 // in one row of 130 at 128256 entries).
 DEV_INLINE float gumbel(uint32_t bits) {
   const float u = ((float)bits + 1.0f) * (1.0f / 16777216.0f);
-  return -__logf(bits == 0xFFFFFFu ? 0x1p-25f : -__logf(u));
+  return -__logf(fmaxf(-__logf(u), 0x1p-25f));
 }
 
 constexpr int SNT = 256;              // threads of a block
@@ -101,10 +102,10 @@ DEV_INLINE void wave_best(float& v, int& i) {
 template <bool TEMP>
 struct Sums {
   float m = -INFINITY, s = 0.f, st = 0.f;
-  // what a sum relative to m counts relative to c; without numbers so far
-  // (m = -inf) nothing, whatever the temperature's sign
+  // what a sum relative to m counts relative to c, at most 2^127: finite, so
+  // that an empty sum (m = -inf) stays 0 also at a negative temperature
   DEV_INLINE static float shift(float m, float c, float inv_temp) {
-    return m == c ? 1.f : m == -INFINITY ? 0.f : __expf((m - c) * inv_temp);
+    return __expf(fminf((m - c) * inv_temp, 88.f));
   }
   // c: the largest of v
   template <int N>
@@ -117,15 +118,23 @@ struct Sums {
     if (m == -INFINITY) {              // nothing but -inf and NaN so far
 #pragma unroll
       for (int j = 0; j < N; ++j)
-        if (v[j] != v[j]) s = st = v[j];
+        if (v[j] != v[j]) {
+          s = v[j];
+          if (TEMP) st = v[j];
+        }
       return;
     }
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      s += __expf(v[j] - m);
-      // (-inf, also what stands in for entries outside the row, has no mass
-      // at a negative or infinite temperature either)
-      if (TEMP)
+    for (int j = 0; j < N; ++j) s += __expf(v[j] - m);
+    if (!TEMP) return;
+    // (-inf, also what stands in for entries outside the row, has no mass
+    // at a negative or infinite temperature either)
+    if (inv_temp > 0.f) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) st += __expf((v[j] - m) * inv_temp);
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
         st += v[j] == -INFINITY ? 0.f : __expf((v[j] - m) * inv_temp);
     }
   }
@@ -315,7 +324,7 @@ DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
                         float* lds) {
   float cut = -INFINITY;
   if (by_p && inv_temp > 0.f && p > 0.f)
-    cut = all.m + __logf(0.5f * (1.f - p) * all.st / V) / inv_temp;
+    cut = all.m + __logf(0.99f * (1.f - p) * all.st / V) / inv_temp;
   if (!(cut > -INFINITY)) cut = -INFINITY;   // (NaN logits)
   if (!by_k || k > n) return cut;
   // waves' maxima where they are enough, else those of 16 lanes
