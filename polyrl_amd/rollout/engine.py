@@ -1056,7 +1056,7 @@ class Engine:
         copy that the host does not wait for (its memory stays reserved until
         the copy is done)."""
         flat = torch.from_numpy(np.concatenate(parts))
-        if str(self.device) != "cpu":
+        if torch.device(self.device).type != "cpu":
             flat = flat.pin_memory().to(self.device, non_blocking=True)
         return list(flat.split([len(p) for p in parts]))
 

@@ -561,3 +561,12 @@ def test_portions_behind_cached_tokens_match_whole_prompts():
             last[rid] = row
     got = torch.stack([last[f"p{i}"] for i in range(4)])
     assert torch.allclose(got, whole, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("device", ["cpu", "cpu:0", torch.device("cpu")])
+def test_prompts_on_any_name_of_the_cpu(device):
+    """A prompt step takes every way to name the CPU."""
+    eng = Engine(get_model_config("llama-debug-cpu"), device=device,
+                 dtype=torch.float32, page_size=4, kv_token_capacity=64,
+                 max_running_requests=2)
+    assert eng.step_forced([("r", [1, 2, 3], [2])]).shape[0] == 1
