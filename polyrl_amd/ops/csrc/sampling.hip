@@ -217,8 +217,8 @@ DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
 
 // ------------------------------------------------------- radix selection
 // Bins of a digit of the encoding: [shift, shift + bits).  Per row and digit
-// four arrays of DIGIT words: counts and mass for top-k's prefix, the same
-// for top-p's (they part after the first digit).
+// two arrays of DIGIT words: counts of the entries with top-k's prefix, mass
+// of those with top-p's.
 struct alignas(8) Plan {              // where a row's two selections stand
   float cut;                          // entries below it stand at neither
   float m, target;                    // largest entry; top-p: mass to reach
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
     return;
   }
   const Plan now = plan;
-  const uint32_t* h = hist + row * hist_words + digit * 4 * DIGIT;
+  const uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
   const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
   int bin;
   float before;
@@ -386,9 +386,7 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
       plan.prefix_k = now.prefix_k | (uint32_t)bin << low, plan.cnt = before;
   }
   if (now.by & 2) {
-    // the first digit's mass serves both; later ones have their own
-    find_bin<true>(h + (digit == 0 ? DIGIT : 3 * DIGIT), bins, now.mass,
-                   now.target, lds, bin, before);
+    find_bin<true>(h + DIGIT, bins, now.mass, now.target, lds, bin, before);
     if (threadIdx.x == 0)
       plan.prefix_p = now.prefix_p | (uint32_t)bin << low, plan.mass = before;
   }
@@ -546,7 +544,7 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
   const Plan plan = plans[row];
   if (plan.by == 0) return;
   const float inv_temp = 1.0f / temperature[row];
-  uint32_t* h = hist + row * hist_words + digit * 4 * DIGIT;
+  uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
 
   const int bins = digit_bins<T>(digit);
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
@@ -555,7 +553,7 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
   fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
   __syncthreads();
   uint32_t* hc = h;
-  float* hm = reinterpret_cast<float*>(h + (digit == 0 ? 1 : 3) * DIGIT);
+  float* hm = reinterpret_cast<float*>(h + DIGIT);
   for (int i = threadIdx.x; i < bins; i += SNT) {
     if (cnt[i]) atomicAdd(&hc[i], cnt[i]);
     if (mass[i] != 0.f) atomicAdd(&hm[i], mass[i]);
@@ -689,7 +687,7 @@ static void launch_sample(torch::Tensor& out_tokens,
       1, std::min<long>({64, ((no_filter ? 2048 : 1024) + N - 1) / N,
                          words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
-  const int hist_words = no_filter ? 0 : digits * 4 * DIGIT;
+  const int hist_words = no_filter ? 0 : digits * 2 * DIGIT;
   // per row: the pieces' shares and maxima, the plan, the bins.  From the
   // caching allocator: a block per call and stream, also while a graph is captured
   const long share_words = (long)split * (sizeof(Share) / 4);
