@@ -89,9 +89,15 @@ DEV_INLINE bool better(float v, int i, float w, int j) {
   return v > w || (v == w && i < j);
 }
 
+DEV_INLINE float first_lane(float v) {
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+
+// over W lanes: 64, or each W neighbours
+template <int W = 64>
 DEV_INLINE void wave_best(float& v, int& i) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
+  for (int off = W / 2; off > 0; off >>= 1) {
     const float ov = __shfl_xor(v, off, 64);
     const int oi = __shfl_xor(i, off, 64);
     if (better(ov, oi, v, i)) v = ov, i = oi;
@@ -154,9 +160,10 @@ struct Sums {
     }
     m = c;
   }
+  template <int W = 64>
   DEV_INLINE void wave(float inv_temp) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
+    for (int off = W / 2; off > 0; off >>= 1)
       merge(__shfl_xor(m, off, 64), __shfl_xor(s, off, 64),
             TEMP ? __shfl_xor(st, off, 64) : 0.f, inv_temp);
   }
@@ -248,12 +255,12 @@ struct alignas(8) Plan {              // where a row's two selections stand
 // get the bin and the sum above it.  lds: the waves' sums, the first thread
 // that reaches the goal, its bin and the sum above that, each in words of its
 // own: a wave may still read the thread while that thread writes its bin.
-template <bool MASS>
+template <bool MASS, int NT = SNT>
 DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
                          float* lds, int& bin, float& before) {
   // thread t has bins [t*per, +per) counted from the top
-  const int per = (n + SNT - 1) / SNT;   // at most DIGIT / SNT
-  constexpr int MOST = DIGIT / SNT;
+  const int per = (n + NT - 1) / NT;     // at most DIGIT / NT
+  constexpr int MOST = DIGIT / NT, NW = NT / 64;
   float val[MOST], own = 0.f;
 #pragma unroll
   for (int i = 0; i < MOST; ++i) {
@@ -273,15 +280,15 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
   }
   __syncthreads();
   if (lane == 63) lds[wid] = upto;
-  int* found = reinterpret_cast<int*>(lds + SNW);
-  if (threadIdx.x == 0) *found = SNT;
+  int* found = reinterpret_cast<int*>(lds + NW);
+  if (threadIdx.x == 0) *found = NT;
   __syncthreads();
   float base = above;
   for (int w = 0; w < wid; ++w) base += lds[w];
   if (base + upto >= goal) atomicMin(found, (int)threadIdx.x);
   __syncthreads();
   const int who = *found;
-  if (who == SNT) {                   // short of the goal: keep all bins
+  if (who == NT) {                    // short of the goal: keep all bins
     bin = 0;
     before = 0.f;
     return;
@@ -298,12 +305,12 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
       if (run >= goal) at = i, done = true;
     }
     run = at_run;
-    lds[SNW + 1] = run;
+    lds[NW + 1] = run;
     found[2] = max(n - 1 - (who * per + at), 0);
   }
   __syncthreads();
   bin = found[2];
-  before = lds[SNW + 1];
+  before = lds[NW + 1];
 }
 
 DEV_INLINE int digit_shift(int d) { return d == 0 ? 21 : d == 1 ? 10 : 0; }
@@ -319,6 +326,7 @@ DEV_INLINE int digit_bins(int d) {
 
 // Entries below this stand at neither threshold of their row (the top of this
 // file).  tops: n maxima of 16 lanes each; lds: n floats.
+template <int NT = SNT>
 DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
                         float p, float inv_temp, const Sums<true>& all, int V,
                         float* lds) {
@@ -330,14 +338,14 @@ DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
   // waves' maxima where they are enough, else those of 16 lanes
   const int width = k <= n / 4 ? 4 : 1, m = n / width;
   __syncthreads();
-  for (int i = threadIdx.x; i < m; i += SNT) {
+  for (int i = threadIdx.x; i < m; i += NT) {
     float t = tops[i * width];
     for (int j = 1; j < width; ++j) t = fmaxf(t, tops[i * width + j]);
     lds[i] = t;
   }
   __syncthreads();
   __shared__ float kth;
-  for (int i = threadIdx.x; i < m; i += SNT) {
+  for (int i = threadIdx.x; i < m; i += NT) {
     const float t = lds[i];
     int rank = 0;
     for (int j = 0; j < m; ++j) {
@@ -563,14 +571,15 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
 // ------------------------------------------------------------- short rows
 // The same steps with one block per row, in one launch: of a short row the
 // steps are shorter than the launches of the pieces and plans.
-template <typename T, bool FILTER>
-__global__ __launch_bounds__(SNT) void sample_row_kernel(
+template <typename T, bool FILTER, int NT>
+__global__ __launch_bounds__(NT) void sample_row_kernel(
     int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
     const T* __restrict__ logits, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p,
     uint64_t seed, const long long* __restrict__ seed_ptr, int V) {
-  __shared__ Share part[SNW];
-  __shared__ float lds[TOPS], tops[FILTER ? TOPS : 1];
+  constexpr int NW = NT / 64, NTOPS = NT / 16;
+  __shared__ Share part[NW];
+  __shared__ float lds[NTOPS], tops[FILTER ? NTOPS : 1];
   __shared__ uint32_t cnt[FILTER ? DIGIT : 1];
   __shared__ float mass[FILTER ? DIGIT : 1];
   const long row = blockIdx.x;
@@ -584,7 +593,7 @@ __global__ __launch_bounds__(SNT) void sample_row_kernel(
 
   Sums<FILTER> sums;
   Draw d;
-  walk<FILTER ? 1 : 0>(r, 0, SNT, greedy, inv_temp, rowkey, 0u, sums, d);
+  walk<FILTER ? 1 : 0>(r, 0, NT, greedy, inv_temp, rowkey, 0u, sums, d);
   if (FILTER) {                       // largest of each 16 lanes
     float t = d.best;
 #pragma unroll
@@ -595,11 +604,14 @@ __global__ __launch_bounds__(SNT) void sample_row_kernel(
   wave_best(d.best, d.best_i);
   if (lane == 0) part[wid] = {sums.m, sums.s, sums.st, d.best, d.best_i, 0};
   __syncthreads();
-  sums = Sums<FILTER>();              // of the whole row, in every thread
-  for (int w = 0; w < SNW; ++w) {
-    sums.merge(part[w].m, part[w].s, part[w].st, inv_temp);
-    if (better(part[w].best, part[w].best_i, d.best, d.best_i))
-      d.best = part[w].best, d.best_i = part[w].best_i;
+  {                                   // of the whole row, in every thread
+    const Share& o = part[lane % NW];
+    sums.m = o.m, sums.s = o.s, sums.st = o.st;
+    sums.template wave<NW>(inv_temp);
+    // (a lane's order of the sums shows in their last bit: all take lane 0's)
+    sums.s = first_lane(sums.s), sums.st = first_lane(sums.st);
+    d.best = o.best, d.best_i = o.best_i;
+    wave_best<NW>(d.best, d.best_i);
   }
   if constexpr (FILTER) {
     if (!greedy) {
@@ -608,23 +620,23 @@ __global__ __launch_bounds__(SNT) void sample_row_kernel(
       const bool by_k = k > 0 && k < V, by_p = p < 1.0f;
       uint32_t tau = 0;
       if (by_k || by_p) {
-        Plan plan(cut_of(tops, TOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
+        Plan plan(cut_of<NT>(tops, NTOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
                   sums, p, by_k, by_p);
         for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
           const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
-          for (int i = threadIdx.x; i < bins; i += SNT)
+          for (int i = threadIdx.x; i < bins; i += NT)
             cnt[i] = 0, mass[i] = 0.f;
           __syncthreads();
-          fill_bins(r, 0, SNT, digit, plan, inv_temp, cnt, mass);
+          fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
           __syncthreads();
           int bin;
           float before;
           if (by_k) {
-            find_bin<false>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
+            find_bin<false, NT>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
             plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
           }
           if (by_p) {
-            find_bin<true>(reinterpret_cast<const uint32_t*>(mass), bins,
+            find_bin<true, NT>(reinterpret_cast<const uint32_t*>(mass), bins,
                            plan.mass, plan.target, lds, bin, before);
             plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
           }
@@ -634,15 +646,13 @@ __global__ __launch_bounds__(SNT) void sample_row_kernel(
       }
       Draw pick;
       Sums<false> none;
-      walk<2>(r, 0, SNT, false, inv_temp, rowkey, tau, none, pick);
+      walk<2>(r, 0, NT, false, inv_temp, rowkey, tau, none, pick);
       wave_best(pick.best, pick.best_i);
       __syncthreads();                // the shares were read
       if (lane == 0) part[wid].best = pick.best, part[wid].best_i = pick.best_i;
       __syncthreads();
-      d.best = part[0].best, d.best_i = part[0].best_i;
-      for (int w = 1; w < SNW; ++w)
-        if (better(part[w].best, part[w].best_i, d.best, d.best_i))
-          d.best = part[w].best, d.best_i = part[w].best_i;
+      d.best = part[lane % NW].best, d.best_i = part[lane % NW].best_i;
+      wave_best<NW>(d.best, d.best_i);
     }
   }
   if (threadIdx.x == 0) {
@@ -663,26 +673,42 @@ static void launch_sample(torch::Tensor& out_tokens,
   const int V = logits.size(1);
   if (N == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  // Short rows: one launch.  Per call, one to 128 rows of 4096 bf16 numbers: 8 to
-  // 9 us (11 in pieces), filtered 22 to 30 (36 to 51), filtered with a
-  // temperature of 0 7.6 (31).  Without a filter one block takes longer than
-  // the pieces from about 8192 numbers on (12.4 and 11.6 us, 64 rows), with
-  // one from 12000 (fp32, 58 and 55 us).
-  if (V <= (no_filter ? 4096 : 8192)) {
-    auto kern = no_filter ? sample_row_kernel<T, false>
-                          : sample_row_kernel<T, true>;
-    kern<<<dim3((unsigned)N), dim3(SNT), 0, stream>>>(
+  // Rows in one launch, a block each, while that is no longer than the pieces
+  // and their plans.  Without a filter: with few rows up to 16384 numbers (64 x
+  // 16000 bf16 12.1 us, in pieces 12.6; 64 x 32000 18.3 and 13.6), with a block
+  // for most CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768
+  // (64 x 9000 33 and 50, 64 x 32000 42 and 51; at a temperature of 0, where
+  // nothing is selected, 7.4 and 33, 9.2 and 33; one row of 50257 with top-p 55
+  // and 39).  What stays dearer than a block a row everywhere is the draw at a
+  // temperature of 0 without a filter from 16384 numbers on, 11.3 us for 8 to
+  // 10: the temperature is on the device, and at 1 the pieces take 13.5 for 21.
+  // A block of 1024 threads takes rows of more than one round of 256 words (64 x
+  // 9000 both filters 33 us, with 256 threads 37; 64 x 32000 42 and 72); where
+  // there are more rows than CUs, 256 threads take them up to ten rounds (512 x
+  // 9000 41 us, with 1024 threads 64).
+  auto rows = [&](auto kern, int threads) {
+    kern<<<dim3((unsigned)N), dim3(threads), 0, stream>>>(
         out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
         (const T*)logits.data_ptr(), temperature.data_ptr<float>(),
         top_k.data_ptr<int>(), top_p.data_ptr<float>(), seed, seed_ptr, V);
     HIP_CHECK_KERNEL();
+  };
+  const long words = (V + VocabRow<T>::VEC - 1) / VocabRow<T>::VEC;
+  const long most = !no_filter ? 32768 : N >= 192 ? 65536 : 16384;
+  if (V <= most) {
+    if (words <= (N > 256 ? 2560 : 256)) {
+      no_filter ? rows(sample_row_kernel<T, false, 256>, 256)
+                : rows(sample_row_kernel<T, true, 256>, 256);
+    } else {
+      no_filter ? rows(sample_row_kernel<T, false, 1024>, 1024)
+                : rows(sample_row_kernel<T, true, 1024>, 1024);
+    }
     return;
   }
   // pieces of a row: 2048 blocks in all (eight per CU; 128 x 128256 takes 37
   // us with 512 blocks, 33 with 1024, 32 with 2048, 36 with 4096), half of
   // that for the short passes of filtered rows (64 x 151936: 63, 55, 60, 62
   // us), none under two rounds of 256 words
-  const long words = (V + VocabRow<T>::VEC - 1) / VocabRow<T>::VEC;
   const int split = (int)std::max<long>(
       1, std::min<long>({64, ((no_filter ? 2048 : 1024) + N - 1) / N,
                          words / (2 * SNT)}));

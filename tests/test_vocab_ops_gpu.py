@@ -308,3 +308,32 @@ def test_sample_short_rows(v, dtype, temp, k, p):
     """Rows on both sides of the lengths up to which one block takes a row;
     k on both sides of the maxima that such a block keeps."""
     test_sample_against_its_definition(5, v, dtype, temp, k, p)
+
+
+@pytest.mark.parametrize("n,v", [(5, 2047), (5, 2049), (3, 16384), (3, 16385),
+                                 (2, 32768), (2, 32769), (191, 17000),
+                                 (192, 17000), (257, 2049), (257, 20481),
+                                 (192, 65537)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("temp,k,p", [(1.0, -1, 1.0), (0.7, 64, 0.9),
+                                      (0.7, 65, 1.0)])
+def test_sample_one_launch(n, v, dtype, temp, k, p):
+    """Both sides of the sizes up to which one block takes a row, and of those
+    from which it has 1024 threads; k on both sides of the maxima of such a
+    block.  Many rows: the first and the last are enough."""
+    torch.manual_seed(8)
+    x = (torch.randn(n, v, device=DEV) * 3).to(dtype)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    seed = 31
+    tok, lp = ops.sample(x, full(temp, torch.float32), full(k, torch.int32),
+                         full(p, torch.float32), seed, no_filter=k < 0)
+    want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+    assert (lp.double() - want).abs().max() <= 1e-5 * (1 + want.abs().max())
+    for r in {0, 1, n - 1}:
+        row = x[r].double().cpu()
+        sure, maybe = kept(row, temp, k, p)
+        t = int(tok[r])
+        assert maybe[t]
+        z = row / temp + noise(seed, r, v)
+        # (as above)
+        assert z[t] >= z[sure].max() - 1e-3
