@@ -41,8 +41,8 @@ DEV_INLINE float quad_sum(float x) {
   return half_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void paged_decode_attn_kernel(
+template <int D, int WAVES>                // WAVES: of a SIMD, at least
+__global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
     bf16_t* __restrict__ out,              // (B, Hq, D)
     float* __restrict__ partial,           // (B, Hq, S, D+2) when nsplit>1
     const bf16_t* __restrict__ q,          // (B, Hq, D)
@@ -253,6 +253,125 @@ __global__ __launch_bounds__(256) void paged_decode_attn_kernel(
   }
 }
 
+// One query head per key/value head, many blocks or short contexts: matrix
+// products use one column in sixteen, and with two or three of their blocks
+// resident on a CU a short context is all latency.  Here a wave streams keys
+// with D / 8 lanes each, and dot products and softmax run on the vector units
+// in 32 bits: 53 registers, eight blocks to a CU.  Bound by latency, from a few
+// hundred keys on by memory.  Measured, 300 rows of 32 heads of 128: 5 keys 14.4
+// us (51 on the matrix cores), 100 keys 90 (100), 500 keys 432 (421).
+template <int D>
+__global__ __launch_bounds__(256) void paged_decode_attn_one_kernel(
+    bf16_t* __restrict__ out,              // (B, H, D)
+    float* __restrict__ partial,           // (B, H, S, D+2) when nsplit>1
+    const bf16_t* __restrict__ q,          // (B, H, D)
+    const bf16_t* __restrict__ k_cache,    // (num_pages, page_size, H, D)
+    const bf16_t* __restrict__ v_cache,
+    const int* __restrict__ page_table,    // (B, max_pages)
+    const int* __restrict__ context_lens,  // (B,)
+    int H, int /* Hk */, int page_size, int max_pages, float scale, long ldq,
+    int nsplit) {
+  constexpr int GL = D / 8;                // lanes of a key
+  constexpr int KPW = 64 / GL;             // keys of a wave's round
+  __shared__ float mrg[4][GL][10];         // per wave: o, m, l
+
+  const int b = blockIdx.x / (H * nsplit);
+  const int rem = blockIdx.x % (H * nsplit);
+  const int h = rem / nsplit;
+  const int sp = rem % nsplit;
+  const int L = context_lens[b];
+  const int Lc = (L + nsplit - 1) / nsplit;
+  const int cbeg = sp * Lc;
+  const int cend = min(cbeg + Lc, L);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int grp = lane / GL, gl = lane % GL;
+  const int d0 = gl * 8;                   // this lane's numbers of a row
+
+  float qr[8];
+  {
+    const bf16x8 qv = *reinterpret_cast<const bf16x8*>(
+        q + (long)b * ldq + (long)h * D + d0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qr[j] = bf2f(qv.v[j]) * scale;
+  }
+  // (m starts finite, as above)
+  float m = -1e30f, l = 0.f, o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = 0.f;
+
+  const long row = (long)H * D;
+  const int* ptab = page_table + (long)b * max_pages;
+  for (int t0 = cbeg + wid * KPW + grp; t0 < cend; t0 += 4 * KPW) {
+    const long slot =
+        (long)ptab[t0 / page_size] * page_size + t0 % page_size;
+    const bf16x8 kv = *reinterpret_cast<const bf16x8*>(
+        k_cache + slot * row + h * D + d0);
+    const bf16x8 vv = *reinterpret_cast<const bf16x8*>(
+        v_cache + slot * row + h * D + d0);
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += qr[j] * bf2f(kv.v[j]);
+#pragma unroll
+    for (int off = GL / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    const float mn = fmaxf(m, s);
+    const float alpha = __expf(m - mn), p = __expf(s - mn);
+    l = l * alpha + p;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = o[j] * alpha + p * bf2f(vv.v[j]);
+    m = mn;
+  }
+
+  // the wave's key groups meet
+#pragma unroll
+  for (int off = GL; off < 64; off <<= 1) {
+    const float om = __shfl_xor(m, off, 64), ol = __shfl_xor(l, off, 64);
+    const float mn = fmaxf(m, om);
+    const float a = __expf(m - mn), c = __expf(om - mn);
+    l = l * a + ol * c;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      o[j] = o[j] * a + __shfl_xor(o[j], off, 64) * c;
+    m = mn;
+  }
+  // and the four waves
+  if (grp == 0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mrg[wid][gl][j] = o[j];
+    mrg[wid][gl][8] = m;
+    mrg[wid][gl][9] = l;
+  }
+  __syncthreads();
+  if (wid != 0 || grp != 0) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) m = fmaxf(m, mrg[w][gl][8]);
+  l = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float a = __expf(mrg[w][gl][8] - m);
+    l += mrg[w][gl][9] * a;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] += mrg[w][gl][j] * a;
+  }
+  const long at = (long)b * H + h;
+  if (nsplit == 1) {
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    bf16x8 w;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w.v[j] = f2bf(o[j] * inv);
+    *reinterpret_cast<bf16x8*>(out + at * D + d0) = w;
+  } else {
+    float* pp = partial + (at * nsplit + sp) * (D + 2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pp[d0 + j] = o[j];
+    if (gl == 0) {
+      pp[D] = m;
+      pp[D + 1] = l;
+    }
+  }
+}
+
 // combine the nsplit context partials of one (b, hq): sum-exp merge
 template <int D>
 __global__ void paged_decode_merge_kernel(
@@ -310,8 +429,8 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   const long B = q.size(0);
   // Context split: from the sizes alone, not from the lengths on the device,
   // so that a captured graph may replay it with longer contexts.  At least
-  // 1024 blocks (four per CU: the loads in flight cover the memory's latency),
-  // but no stretch under 128 keys (a round of the four waves) of the longest
+  // 1024 blocks (four per CU, two of them resident at a time at D = 128: the
+  // next start as the first end), but no stretch under 128 keys (a round of the four waves) of the longest
   // context that the page table holds: there the merging launch costs more
   // than the split gains (37 cached tokens: 16.8 us in 16 stretches, 6.8 in
   // one).
@@ -353,7 +472,22 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   }
   TORCH_CHECK(G >= 1 && G <= DEC_HEADS, "GQA group size ", G,
               " unsupported (1..8)");
-  args(paged_decode_attn_kernel<D>);
+  // One head a group: the vector kernel from four rounds of the matrix kernel's
+  // blocks on (heads of 128: 64 rows of 32 heads, 40 keys 9.7 us and 12.4, 300
+  // keys 52 and 55; 32 rows 300 keys 26.4 both, 3000 keys 306 and 278; heads
+  // of 64: 300 rows of 16, 40 keys 12.8 and 15.0, 300 keys 75.7 and 72.4, 128
+  // rows 1000 keys 97.7 and 103), and where the page table holds short contexts
+  // only (128 wide, 4 heads, 128 rows of 300 keys: 18.2 and 20.0).
+  // Groups of two and three heads of 128 keep three blocks on a CU, which short
+  // contexts need (300 rows of 16 groups of two, 5 keys: 28 us with two, 19.7
+  // with three); at larger groups the registers that this takes cost more (32
+  // rows of 8000 keys, 28/4 heads: 106 and 110 us).
+  if (G == 1 && (base_blocks >= 2048 || most <= (D == 128 ? 512 : 64)))
+    args(paged_decode_attn_one_kernel<D>);
+  else if (D == 128 && G <= 3)
+    args(paged_decode_attn_kernel<D, 3>);
+  else
+    args(paged_decode_attn_kernel<D, 1>);
 }
 
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,

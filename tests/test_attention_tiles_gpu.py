@@ -134,7 +134,8 @@ def test_backward(name, hq, hk, d, causal):
 @pytest.mark.parametrize("page_size,wide", [(16, False), (16, True), (1, False),
                                             (7, True)])
 @pytest.mark.parametrize("hq,hk,d", [(8, 8, 128), (7, 1, 128), (12, 4, 64),
-                                     (16, 2, 64), (28, 4, 128), (5, 1, 64)])
+                                     (16, 2, 64), (28, 4, 128), (5, 1, 64),
+                                     (6, 2, 128)])
 def test_decode(hq, hk, d, page_size, wide):
     """Paged decode at the edges of its 32-key rounds and 128-key stretches;
     ``wide``: a page table far wider than the contexts (a captured graph's),
@@ -336,3 +337,40 @@ def test_decode_weights(d):
     # a score, its exponential and the sums are each rounded to 24 bits
     bound = 2 ** -8 * want.abs() + 2.0 ** -22
     assert ((out.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rows,heads_,most", [(11, 3, 64), (11, 3, 65),
+                                              (11, 3, 512), (11, 3, 513),
+                                              (255, 8, 700), (256, 8, 700),
+                                              (128, 16, 3000)])
+def test_decode_one_head_a_group(rows, heads_, most, d):
+    """Groups of one head on both sides of the sizes at which the vector kernel
+    takes them: few rows divided among blocks, many rows undivided."""
+    torch.manual_seed(5)
+    page = 1 if most % 16 else 16
+    lens = ([most, 1, 2, 7, 8, 9, 16, 17, 31, 33, 64]
+            + [1 + 37 * i % 90 for i in range(rows)])[:rows]
+    need = [-(-n // page) for n in lens]
+    table = torch.zeros(rows, max(need), dtype=torch.int32, device=DEV)
+    pages = torch.randperm(sum(need), device=DEV).int()
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    k, v = (torch.randn(sum(need), page, heads_, d, device=DEV).bfloat16()
+            for _ in range(2))
+    q = torch.randn(rows, heads_, d, device=DEV).bfloat16()
+    out = ops.paged_attention_decode(
+        q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+        d ** -0.5)
+    for i in list(range(11)) + [rows - 1]:
+        n = lens[i]
+        p = table[i, :need[i]].long()
+        kk = k[p].view(-1, heads_, d)[:n].double()
+        vv = v[p].view(-1, heads_, d)[:n].double()
+        want, _ = attend(q[i:i + 1].double(), kk, vv, n - 1, True, d ** -0.5)
+        mass, _ = attend(q[i:i + 1].double(), kk, vv.abs(), n - 1, True,
+                         d ** -0.5)
+        bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
+        assert ((out[i:i + 1].double() - want).abs() <= bound).all(), (i, n)
