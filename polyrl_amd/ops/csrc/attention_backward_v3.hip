@@ -497,18 +497,22 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
           t_q0.data_ptr<int>(), (int)ntiles, nparts, Hq, Hk, scale,
           causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
   // Blocks of the dkv kernel are as long as their key is early, so the chip
-  // needs several per slot (512: two per CU) to end together; with fewer than
-  // 768 a block takes fewer heads of the group.  The shares' trip through
-  // fp32 costs as much whatever the length, so long sequences are cut finer.
-  // Measured, forward and backward: 2 sequences of 4096, 28/4 heads (476
-  // blocks) 2166 us whole, 1644 with two heads a block, 1578 with one (before
-  // the fragments were read ahead); 16 of
-  // up to 512, 32/8 heads (896 blocks) 349 us whole, 376 with two heads.
+  // needs several per slot (512: two per CU) to end together; with few blocks
+  // each takes fewer heads of the group.  Long sequences are cut finer: the
+  // shares' trip through fp32 costs as much whatever the length.  Measured,
+  // forward and backward, all heads / two / one a block: 2 sequences of 3300 and
+  // 4096, 28/4 heads (464 blocks) 1470 / 1323 / 1315 us; one of 4096, 32/8 heads
+  // (512) 848 / 773 / 770; 3 of 4096, 28/4 (768) 2250 / 2167 / 2178.  Sequences
+  // of 130 to 512, 32/8 heads: 16 (720 blocks) 184 / 192 / 228, 12 (576) 157 /
+  // 166 / 182, 8 (368) 126 / 121 / 131; 16 of 28/4 heads (372) 213 / 198 / 222.
+  // The shares take 64 KiB a block at D = 128 while the call runs: at most 48 MiB
+  // times the heads of a group.
   const long base = ntiles * Hk, nseq = cu_q.size(0) - 1;
+  const bool lengthy = ntiles >= 16 * nseq;
   int nsplit = 1;
-  if (base < 768) {
-    const long target = ntiles >= 16 * nseq ? 4096 : 1536;
-    const int per = (int)std::max<long>(1, G * base / target);
+  if (base < (lengthy ? 768 : 512)) {
+    const int per = (int)(lengthy ? std::max<long>(1, G * base / 4096)
+                                  : (G * base + 767) / 768);
     nsplit = (G + per - 1) / per;
   }
   torch::Tensor part;

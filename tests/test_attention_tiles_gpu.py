@@ -15,6 +15,7 @@ LENS = {
     "edges": [1, 31, 32, 33, 63, 64, 65, 127, 128, 129],
     "ragged": [200, 7, 321, 64],
     "many": [3] * 70 + [65],            # more sequences than a scan step
+    "shares": [65] * 20 + [33] * 130,   # dK/dV blocks of 2 to 4 heads of 7
 }
 
 
@@ -83,7 +84,7 @@ def test_forward(name, hq, hk, d, hist, causal, table):
 @pytest.mark.parametrize("name,hq,hk,d", [
     ("edges", 8, 2, 128), ("edges", 7, 1, 64), ("one", 3, 3, 128),
     ("ragged", 12, 2, 128), ("ragged", 4, 4, 64), ("many", 8, 1, 64),
-    ("ragged", 10, 2, 64)])
+    ("ragged", 10, 2, 64), ("shares", 14, 2, 128), ("shares", 4, 2, 64)])
 def test_backward(name, hq, hk, d, causal):
     """Gradients of every sequence against float64 autograd.  With P and dS
     rounded once to bf16, sums in 32 bits and the result rounded once, an
