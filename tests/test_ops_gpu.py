@@ -4,7 +4,6 @@ All tests are @pytest.mark.gpu and run on a real MI355X via gpurun / the
 driver's round-end GPU tier.
 """
 import math
-import os
 
 import pytest
 import torch
@@ -219,15 +218,10 @@ def test_paged_attention_decode(Hq, Hk, D):
     assert rel_err(out.cpu(), expect) < 3e-2
 
 
-@pytest.mark.skipif(os.environ.get("POLYRL_DECODE_MFMA") != "1",
-                    reason="experimental MFMA decode path: opt-in via "
-                           "POLYRL_DECODE_MFMA=1 (not yet validated)")
 @pytest.mark.parametrize("Hq,Hk,D", [(8, 8, 128), (32, 8, 128),
                                      (8, 2, 128), (16, 4, 64)])
 def test_paged_attention_decode_mfma(Hq, Hk, D):
-    """Numerics gate for the EXPERIMENTAL MFMA decode prototype (covered
-    (D, G): 128/{1,4,8(2 falls back)}, 64/4).  Round-3 entry point:
-    POLYRL_DECODE_MFMA=1 pytest -k decode_mfma -m gpu."""
+    """Decode attention against the CPU form: groups of one to four heads."""
     torch.manual_seed(10)
     B, page_size = 9, 16
     lens = torch.tensor([1, 5, 16, 17, 60, 64, 100, 255, 300],
