@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     T::fetch(rk, kb, ldk, 0, Lk);
     T::fetch(rv, vb, ldv, 0, Lk);
     T::store(lds[0][0], rk);
-    T::store_live(lds[0][1], rv, Lk);
+    T::store(lds[0][1], rv);
   }
   wait_loads();
   if (ATILE < bend) {
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     // the next tile into the other buffer (its readers passed the barrier)
     if (t0 + ATILE < bend) {
       T::store(lds[buf ^ 1][0], rk);
-      T::store_live(lds[buf ^ 1][1], rv, Lk - t0 - ATILE);
+      T::store(lds[buf ^ 1][1], rv);
       if (t0 + 2 * ATILE < bend) {
         T::fetch(rk, kb, ldk, t0 + 2 * ATILE, Lk);
         T::fetch(rv, vb, ldv, t0 + 2 * ATILE, Lk);

@@ -43,18 +43,22 @@ struct AttnTile {
   }
 
   // this thread's granules of rows [r0, r0 + 64) of one head; rows from
-  // ``rows`` on repeat the last one (what they give is masked or dropped)
+  // ``rows`` on are zeros (a weight of 0 meets them, and 0 * inf is NaN).  The
+  // buffer ends with the last row's granules of this head; what a lane asks
+  // for behind it is not read and returns 0.
   DEV_INLINE static void fetch(i32x4_t (&reg)[LOADS], const bf16_t* base,
                                long ld, int r0, int rows) {
-    // a block-uniform base and 32-bit offsets inside the tile
-    const char* from = reinterpret_cast<const char*>(base + r0 * ld);
-    const unsigned ldb = (unsigned)ld * 2;
+    // a block-uniform buffer and 32-bit offsets inside the tile
+    const int ldb = (int)ld * 2, live = min(rows - r0, ATILE);
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(base + r0 * ld), 0,
+        live > 0 ? (live - 1) * ldb + 2 * D : 0, 0x00020000);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int at = threadIdx.x + i * 256;
-      const unsigned r = min(at / GR, rows - 1 - r0);
-      reg[i] = *reinterpret_cast<const i32x4_t*>(from + (r * ldb +
-                                                         at % GR * 16));
+      reg[i] = __builtin_bit_cast(
+          i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                       from, at / GR * ldb + at % GR * 16, 0, 0));
     }
   }
 

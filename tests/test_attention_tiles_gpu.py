@@ -313,6 +313,24 @@ def test_infinite_value_of_the_last_key(hq, hk, d):
         assert out[:, :, other].isfinite().all(), name
 
 
+@pytest.mark.parametrize("hq,hk,d", [(8, 2, 128), (7, 1, 64), (4, 4, 64)])
+def test_infinite_gradient_of_the_last_row(hq, hk, d):
+    """An infinite entry of the gradient of a sequence's last output row gives
+    infinite entries of dV, which all of its keys share in, and no NaN: what
+    stands in for rows past the end takes no part."""
+    torch.manual_seed(4)
+    lens = [1, 33, 200]
+    cu = cu_of(lens).to(DEV)
+    q, k, v = (torch.randn(sum(lens), h, d, device=DEV).bfloat16()
+               .requires_grad_() for h in (hq, hk, hk))
+    dout = torch.randn(sum(lens), hq, d, device=DEV).bfloat16()
+    dout[(cu[1:] - 1).long(), :, 5] = float("inf")
+    out = ops.flash_attn_varlen(q, k, v, cu, d ** -0.5, True)
+    dv = torch.autograd.grad(out, (q, k, v), dout)[2]
+    assert (dv[:, :, 5] == float("inf")).all()
+    assert dv[:, :, [j for j in range(d) if j != 5]].isfinite().all()
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_decode_weights(d):
     """Weights are held in 32 bits: the difference of two almost equal ones
