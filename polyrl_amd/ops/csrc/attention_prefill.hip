@@ -37,6 +37,12 @@
 
 #include "attention_tile.h"
 
+// a * b, never fused with what it is added to
+DEV_INLINE float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
 template <int D>
 __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     bf16_t* __restrict__ out,        // (total_q, Hq, D)
@@ -183,12 +189,23 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
           for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
         m_run = mn;
       }
+      // (very large scores are rounded like their maximum: what it lost to
+      // rounding would pass the exponential's range)
+      float by = s2, less = m_run;
+      if (__any(fabsf(m_run) >= 0x1p24f)) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[n][r] = rounded_product(s[n][r], s2) - m_run;
+        by = 1.f, less = 0.f;
+      }
       float sum = 0.f;
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          s[n][r] = exp2_hw(__builtin_fmaf(s[n][r], s2, -m_run));
+          s[n][r] = exp2_hw(__builtin_fmaf(s[n][r], by, -less));
           sum += s[n][r];
         }
       l_run += sum;

@@ -331,6 +331,27 @@ def test_infinite_gradient_of_the_last_row(hq, hk, d):
     assert dv[:, :, [j for j in range(d) if j != 5]].isfinite().all()
 
 
+@pytest.mark.parametrize("hq,hk,d", [(8, 2, 128), (7, 1, 64)])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_very_large_scores(hq, hk, d, sign):
+    """Scores far beyond 2^31, where an exponent is larger than the range of
+    the exponential even in its rounding: each row gets the value of its
+    largest score."""
+    torch.manual_seed(4)
+    lens = [1, 33, 200]
+    cu = cu_of(lens)
+    q, k, v = (torch.randn(sum(lens), h, d, device=DEV).bfloat16()
+               for h in (hq, hk, hk))
+    q = q * 2.0 ** 40
+    got = ops.varlen_prefill_attention(q, k, v, cu.to(DEV), cu.to(DEV),
+                                       sign * d ** -0.5, True)
+    for i in range(len(lens)):
+        a = slice(cu[i], cu[i + 1])
+        want, _ = attend(q[a].double(), heads(k[a].double(), hq),
+                         heads(v[a].double(), hq), 0, True, sign * d ** -0.5)
+        assert torch.equal(got[a].double(), want.bfloat16().double())
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_decode_weights(d):
     """Weights are held in 32 bits: the difference of two almost equal ones
