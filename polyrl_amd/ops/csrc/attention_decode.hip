@@ -18,7 +18,7 @@
 // and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
 // at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
 // tokens, 32/8 heads of 128, 59.5 -> 45.2 us; 33 rows of 1900 .. 8192, 28/4
-// heads, 264 -> 86.6 us (4.1 TB/s).  (With two parts a weight 44.6 and 86.0.)
+// heads, 264 -> 86.5 us (4.1 TB/s).  (With two parts a weight 44.6 and 86.0.)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

@@ -20,12 +20,14 @@
 // lift some row's maximum; only tiles that touch the causal border or the
 // sequence's end are masked.
 //
-// What bounds it: exponentials and matrix instructions of the two waves of a
-// SIMD, about as many cycles of each at D = 128 (the 16-row score tiles with
-// scalar LDS gathers for V that this replaces ran at 160 TFLOP/s).  Measured,
+// What bounds it: exponentials and matrix instructions of a SIMD's waves (two
+// at D = 128, three at 64), about as many cycles of each at D = 128 (the 16-row
+// score tiles with scalar LDS gathers for V that this replaces ran at 160
+// TFLOP/s).  Blocks of a second row half that holds no row still fetch the
+// tiles (7% of the walks of 16 sequences of up to 512 rows).  Measured,
 // eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads of 64: 671 us a call
-// before (50 us of it the tile table's trip through the host), 164 us now
-// (645 TFLOP/s of live pairs).  A maximum that may lag by 2^6 saves the
+// before (50 us of it the tile table's trip through the host), 167 us now
+// (630 TFLOP/s of live pairs).  A maximum that may lag by 2^6 saves the
 // rescaling in most tiles (158 us), but then a row's largest weight is no
 // longer exactly 1 and takes part in the rounding to bf16: the error against
 // 64 bits grows by 2 to 3% (2.03e-3 for 1.98e-3, rms, 1024 keys).

@@ -1,5 +1,6 @@
 // Tiles of the matrix-core attention kernels (attention_prefill.hip,
-// attention_backward_v3.hip): 64 rows x D bf16 numbers in LDS, their
+// attention_backward_v3.hip, seq_gqa_mfma.hip; the swizzle in
+// attention_decode.hip): 64 rows x D bf16 numbers in LDS, their
 // fragments for v_mfma_f32_32x32x16_bf16, and the table of row tiles.
 //
 // Layout.  A tile row is D numbers in 16-byte granules; granule g of row r
