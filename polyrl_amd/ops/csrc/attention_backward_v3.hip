@@ -49,17 +49,19 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     const bf16_t* __restrict__ dout, // (total_q, Hq, D) contiguous, like out
     const float* __restrict__ lse, const int* __restrict__ cu_q,
     const int* __restrict__ cu_k, const int* __restrict__ tile_seq,
-    const int* __restrict__ tile_q0, int ntiles, int nparts, int Hq, int Hk,
-    float scale, int causal, long ldq, long ldk, long ldv) {
+    const int* __restrict__ tile_q0, int nseq, int ntiles, int nparts, int Hq,
+    int Hk, float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
 
   const int G = Hq / Hk;
-  const int item = die_item(ntiles * Hk * nparts);
-  if (item >= ntiles * Hk * nparts) return;
-  const int hk = item / (ntiles * nparts);
-  const int tile = ntiles - 1 - item / nparts % ntiles;   // long rows first
-  const int seq = uniform(tile_seq[tile]), q0 = uniform(tile_q0[tile]);
+  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk, part = item % nparts;
+  const int t = item / nparts;
+  int seq, q0;
+  if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
+                 : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
+                              seq, q0))
+    return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int lane = threadIdx.x & 63;
   const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
-  const int unit = item % nparts * 4 + wid;        // (row half, head)
+  const int unit = part * 4 + wid;        // (row half, head)
   const int wq0 = q0 + unit / G * 32;
   const bool busy = unit < 2 * G && wq0 < Lq;
   const int hq = busy ? hk * G + unit % G : hk * G;
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 
   const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
   const int wend = busy ? seen : 0;
-  const int last_half = min(item % nparts * 4 + 3, 2 * G - 1) / G;
+  const int last_half = min(part * 4 + 3, 2 * G - 1) / G;
   const int bend = causal
       ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
@@ -224,8 +226,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     const float* __restrict__ lse, const float* __restrict__ delta,
     const int* __restrict__ cu_q, const int* __restrict__ cu_k,
     const int* __restrict__ tile_seq, const int* __restrict__ tile_k0,
-    int ntiles, int nsplit, long total_k, int Hq, int Hk, float scale,
-    int causal, long ldq, long ldk, long ldv) {
+    int nseq, int ntiles, int nsplit, long total_k, int Hq, int Hk,
+    float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   constexpr bool V_LDS = D == 128;   // V does not fit beside the gradients
   // Q (two buffers), dO, V; at the end the exchange of 4 x 32 x D floats
@@ -234,13 +236,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   __shared__ __attribute__((aligned(16))) float row_s[2][ATILE];
 
   const int G = Hq / Hk;
-  const int item = die_item(ntiles * Hk * nsplit);
-  if (item >= ntiles * Hk * nsplit) return;
-  const int hk = item / (ntiles * nsplit);
-  const int tile = item / nsplit % ntiles;         // early keys: most rows
-  const int split = item % nsplit;
+  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
+  const int split = item % nsplit, t = item / nsplit;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
-  const int seq = uniform(tile_seq[tile]), t0 = uniform(tile_k0[tile]);
+  int seq, t0;
+  if (nseq <= 64 ? !nth_longest<true>(t, cu_q, cu_k, nseq, seq, t0)
+                 : !find_tile(t, tile_seq, tile_k0, cu_q, nseq, seq, t0))
+    return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;
@@ -480,10 +482,10 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
   const int Hq = q.size(1), Hk = k.size(1), G = Hq / Hk;
   const long ntiles = t_seq.size(0), total_k = k.size(0);
   auto stream = at::hip::getCurrentHIPStream();
+  const int nseq = cu_q.size(0) - 1;
   auto blocks = [&](long items) {
-    const long b = (items + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
-    TORCH_CHECK(b < (1L << 31), "grid too large");
-    return dim3((unsigned)b);
+    TORCH_CHECK(items < (1L << 31), "grid too large");
+    return dim3((unsigned)items);
   };
   auto delta = torch::empty_like(lse);
   const int nparts = (2 * G + 3) / 4;
@@ -494,7 +496,7 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
           (const bf16_t*)v.data_ptr(), (const bf16_t*)out.data_ptr(),
           (const bf16_t*)dout.data_ptr(), lse.data_ptr<float>(),
           cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), t_seq.data_ptr<int>(),
-          t_q0.data_ptr<int>(), (int)ntiles, nparts, Hq, Hk, scale,
+          t_q0.data_ptr<int>(), nseq, (int)ntiles, nparts, Hq, Hk, scale,
           causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
   // Blocks of the dkv kernel are as long as their key is early, so the chip
   // needs several per slot (512: two per CU) to end together; with few blocks
@@ -507,7 +509,7 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
   // 166 / 182, 8 (368) 126 / 121 / 131; 16 of 28/4 heads (372) 213 / 198 / 222.
   // The shares take 64 KiB a block at D = 128 while the call runs: at most 48 MiB
   // times the heads of a group.
-  const long base = ntiles * Hk, nseq = cu_q.size(0) - 1;
+  const long base = ntiles * Hk;
   const bool lengthy = ntiles >= 16 * nseq;
   int nsplit = 1;
   if (base < (lengthy ? 768 : 512)) {
@@ -526,7 +528,7 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
       (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
       lse.data_ptr<float>(), delta.data_ptr<float>(), cu_q.data_ptr<int>(),
       cu_k.data_ptr<int>(), t_seq.data_ptr<int>(), t_q0.data_ptr<int>(),
-      (int)ntiles, nsplit, total_k, Hq, Hk, scale, causal ? 1 : 0,
+      nseq, (int)ntiles, nsplit, total_k, Hq, Hk, scale, causal ? 1 : 0,
       q.stride(0), k.stride(0), v.stride(0));
   if (nsplit > 1) {
     const long n = total_k * Hk * D;

@@ -62,13 +62,15 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
   __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
 
   const int G = Hq / Hk;
-  const int item = die_item(ntiles * Hk * nparts);
-  if (item >= ntiles * Hk * nparts) return;
-  const int hk = item / (ntiles * nparts);
-  // later tiles of a sequence see more keys: they start first
-  const int tile = ntiles - 1 - item / nparts % ntiles;
+  // Blocks go to the dies in turn (id % 8): with the key/value head innermost a
+  // die has one head or few, and every die a share of every length
+  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk, part = item % nparts;
+  const int t = item / nparts;
   int seq, q0;
-  if (!find_tile(tile, tile_seq, tile_q0, cu_q, nseq, seq, q0)) return;
+  if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
+                 : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
+                              seq, q0))
+    return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
   const int qk_off = Lk - Lq;                      // chunked-prefill alignment
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
   const int lane = threadIdx.x & 63;
   const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
-  const int unit = item % nparts * 4 + wid;        // (row half, head)
+  const int unit = part * 4 + wid;        // (row half, head)
   const int hq = hk * G + unit % G;
   const int wq0 = q0 + unit / G * 32;              // this wave's first row
   const bool busy = unit < 2 * G && wq0 < Lq;
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
   // keys that this wave and this block walk
   const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
   const int wend = busy ? seen : 0;
-  const int last_half = min(item % nparts * 4 + 3, 2 * G - 1) / G;
+  const int last_half = min(part * 4 + 3, 2 * G - 1) / G;
   const int bend = causal
       ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
@@ -301,11 +303,10 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
   if (ntiles == 0 || q.size(0) == 0) return;
   const int nparts = (2 * (Hq / Hk) + 3) / 4;      // blocks of a tile's units
   const long items = ntiles * Hk * nparts;
-  const long blocks = (items + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
-  TORCH_CHECK(blocks < (1L << 31), "grid too large");
+  TORCH_CHECK(items < (1L << 31), "grid too large");
   auto stream = at::hip::getCurrentHIPStream();
   auto kern = (D == 128) ? prefill_attn_kernel<128> : prefill_attn_kernel<64>;
-  kern<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
+  kern<<<dim3((unsigned)items), dim3(256), 0, stream>>>(
       (bf16_t*)out.data_ptr(),
       want_lse ? lse.data_ptr<float>() : nullptr,
       (const bf16_t*)q.data_ptr(),

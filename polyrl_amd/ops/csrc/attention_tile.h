@@ -215,14 +215,64 @@ DEV_INLINE bool find_tile(int tile, const int* tile_seq, const int* tile_r0,
   return false;
 }
 
+// sum over the wave's lanes, the same in all of them
+DEV_INLINE int wave_total(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Row tile number ``t`` of a packed batch of at most 64 sequences in the order
+// of their walks, longest first; false past the last.  A causal walk is as long
+// as the row tile is late (EARLY: the walk over the query tiles that see a key
+// tile, as it is early), so the order of the table, sequence after sequence,
+// starts a longest block when most of the chip is done: two sequences of
+// 3500 .. 4096, 28/4 heads of 128, kept 1.3 of two waves a SIMD on average.
+// ``above(L)`` counts the tiles whose walk is longer than L tiles.
+template <bool EARLY>
+DEV_INLINE bool nth_longest(int t, const int* cu_q, const int* cu_k, int nseq,
+                            int& seq, int& r0) {
+  const int lane = threadIdx.x & 63;
+  int n = 0, h = 0;                    // row tiles; key tiles before the first
+  if (lane < nseq) {
+    const int lq = max(cu_q[lane + 1] - cu_q[lane], 0);
+    n = (lq + ATILE - 1) / ATILE;
+    if (!EARLY) h = max(cu_k[lane + 1] - cu_k[lane] - lq, 0) / ATILE;
+  }
+  auto above = [&](int L) { return wave_total(min(max(h + n - L, 0), n)); };
+  if (above(0) <= t) return false;
+  int lo = 0, hi = 1;
+  while (above(hi) > t) lo = hi, hi *= 2;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    if (above(mid) > t) lo = mid;
+    else hi = mid;
+  }
+  // of the sequences with a tile of this length, the one that t stands for
+  const int at = t - above(lo + 1);
+  const unsigned long long has = __ballot(h <= lo && lo < h + n);
+  const int rank = __builtin_amdgcn_mbcnt_hi(
+      (unsigned)(has >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has, 0));
+  const unsigned long long me =
+      __ballot((has >> lane & 1) && rank == at);
+  seq = __ffsll((long long)me) - 1;
+  r0 = (EARLY ? __builtin_amdgcn_readlane(n, seq) - 1 - lo
+              : lo - __builtin_amdgcn_readlane(h, seq)) * ATILE;
+  return true;
+}
+
 // wave of the block, known to the compiler to be the same for all its lanes
 DEV_INLINE int wave_id() {
   return uniform(threadIdx.x >> 6);
 }
 
-// Work item of a block.  Blocks go to the dies in turn (id % 8); each die
-// takes one stretch of the items, whose order is key/value head, row tile,
-// part, so the tiles that read the same keys share an L2.
+// Work item of a block of the window kernel.  Blocks go to the dies in turn
+// (id % 8); each die takes one stretch of the items, whose order is key/value
+// head, row tile, part, so the tiles that read the same keys share an L2.
 DEV_INLINE int die_item(int items) {
   const int per = (items + ATTN_XCDS - 1) / ATTN_XCDS;
   return (int)(blockIdx.x % ATTN_XCDS) * per + (int)(blockIdx.x / ATTN_XCDS);

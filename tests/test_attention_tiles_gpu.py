@@ -414,3 +414,35 @@ def test_decode_one_head_a_group(rows, heads_, most, d):
                          d ** -0.5)
         bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
         assert ((out[i:i + 1].double() - want).abs() <= bound).all(), (i, n)
+
+
+@pytest.mark.parametrize("nseq", [1, 63, 64, 65])
+@pytest.mark.parametrize("d", [64, 128])
+def test_every_tile_once(nseq, d):
+    """Blocks take row tiles by the length of their walk, up to 64 sequences:
+    with empty sequences, equal and different lengths and histories, and keys
+    fewer than rows, every row is written.  Values that do not depend on the
+    key make the result exact whatever the weights."""
+    r = torch.Generator().manual_seed(nseq)
+    lens = torch.randint(0, 200, (nseq,), generator=r)
+    lens[nseq // 2] = 129
+    hist = torch.randint(-3, 5, (nseq,), generator=r) * 32
+    klens = (lens + hist).clamp(min=0)
+    cu_q, cu_k = cu_of(lens.tolist()), cu_of(klens.tolist())
+    n, hq, hk = int(lens.sum()), 6, 2
+    q = torch.randn(n, hq, d, device=DEV).bfloat16()
+    k = torch.randn(int(klens.sum()) + 1, hk, d, device=DEV).bfloat16()[:-1]
+    value = torch.arange(1, nseq + 1, device=DEV)
+    v = value.repeat_interleave(klens.to(DEV)).bfloat16()[:, None, None] \
+        .expand(-1, hk, d).contiguous()
+    for causal in (True, False):
+        out = torch.full((n, hq, d), -7.0, device=DEV).bfloat16()
+        ops._require_ext().varlen_prefill_attention(
+            out, q, k, v, cu_q.to(DEV), cu_k.to(DEV), torch.empty(0),
+            torch.empty(0), d ** -0.5, causal, torch.empty(0))
+        for i in range(nseq):
+            a = out[cu_q[i]:cu_q[i + 1]].float()
+            blind = min(max(-int(hist[i]), 0), int(lens[i])) if causal else (
+                0 if klens[i] else int(lens[i]))
+            assert (a[:blind] == 0).all()    # rows that see no key
+            assert ((a[blind:] - (i + 1)).abs() <= 2 ** -8 * (i + 1)).all()
