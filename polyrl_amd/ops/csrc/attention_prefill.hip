@@ -6,10 +6,12 @@
 // Split.  A wave owns 32 query rows of one head; a block is four such units
 // of one 64-row tile and one key/value head, heads of the group first (four
 // heads x 32 rows with a group of four), so the four waves read the same
-// keys and end at the same causal border.  K and V tiles of 64 keys come
-// through registers (the tile after next is in flight during a tile's
-// products) into one of two LDS buffers: one barrier per tile, 64 KiB at
-// D = 128, two blocks per CU.
+// keys and end at the same causal border.  K and V tiles of 64 keys go straight
+// into LDS (AttnTile::copy), the next tile during this one's products.  Heads of
+// 64: two buffers of both, 32 KiB, and no more than 128 registers, so that four
+// blocks run per CU.  Heads of 128: two of K and one of V, whose next tile is
+// on its way from the last value product to the next softmax (a second barrier
+// a tile), 48 KiB and 165 registers: three blocks.
 //
 // Products.  Scores are computed as S^T = K Q^T with the queries held in
 // registers: a lane's accumulators are 16 keys of ONE row, so the softmax
@@ -20,17 +22,20 @@
 // lift some row's maximum; only tiles that touch the causal border or the
 // sequence's end are masked.
 //
-// What bounds it: exponentials and matrix instructions of a SIMD's waves (two
-// at D = 128, three at 64), about as many cycles of each at D = 128 (the 16-row
-// score tiles with scalar LDS gathers for V that this replaces ran at 160
-// TFLOP/s).  Blocks of a second row half that holds no row still fetch the
-// tiles (7% of the walks of 16 sequences of up to 512 rows).  Measured,
-// eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads of 64: 671 us a call
-// before (50 us of it the tile table's trip through the host), 167 us now
-// (630 TFLOP/s of live pairs).  A maximum that may lag by 2^6 saves the
-// rescaling in most tiles (158 us), but then a row's largest weight is no
-// longer exactly 1 and takes part in the rounding to bf16: the error against
-// 64 bits grows by 2 to 3% (2.03e-3 for 1.98e-3, rms, 1024 keys).
+// What bounds it: at 64 the vector instructions, 76% of the cycles (185 a tile of
+// a wave: exponential, scale, sum, maximum, rounding, and the rescaling of the
+// output); at 128 those and the matrix instructions, 58% and 44%, and what is
+// left of their taking turns (the 16-row score tiles with scalar LDS gathers for
+// V that this replaces ran at 160 TFLOP/s).  Blocks of a second row half that
+// holds no row still fetch the tiles (7% of the walks of 16 sequences of up to
+// 512 rows).  Measured, eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads
+// of 64: 671 us a call with those and the tile table's trip through the host (50
+// us), 154 with tiles through registers and three blocks per CU, 138 now (780
+// TFLOP/s of live pairs); of 128: 283 in the sequences' order, 280, 243 now; two sequences of 3500 ..
+// 4096, 28/4 heads of 128, 323, 265, 222.  A maximum that may lag by 2^6 saves
+// the rescaling in most tiles (5 to 7%), but then a row's largest weight is no
+// longer exactly 1 and takes part in the rounding to bf16: the error against 64
+// bits grows by 2 to 3% (2.03e-3 for 1.98e-3, rms, 1024 keys).
 //
 // Chunked-prefill semantics: query block aligned to the END of the keys
 // (q row i at absolute kv position (Lk - Lq) + i), matching ops/ref.py.
@@ -46,7 +51,7 @@ DEV_INLINE float rounded_product(float a, float b) {
 }
 
 template <int D>
-__global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
+__global__ __launch_bounds__(256, D == 64 ? 4 : 3) void prefill_attn_kernel(
     bf16_t* __restrict__ out,        // (total_q, Hq, D)
     float* __restrict__ lse,         // (total_q, Hq) log-sum-exp, or null
     const bf16_t* __restrict__ q,    // (total_q, Hq, D)
@@ -59,13 +64,19 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
     int nseq, int ntiles, int nparts, int Hq, int Hk, float scale, int causal,
     long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
-  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
+  constexpr bool ONE_V = D == 128;
+  // two buffers of K and V each; at the end the waves' rows of the output
+  __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
+      k1_s[T::BYTES], vx_s[ONE_V ? 16 : T::BYTES];
+  char* const v1_s = ONE_V ? v0_s : vx_s;
 
   const int G = Hq / Hk;
   // Blocks go to the dies in turn (id % 8): with the key/value head innermost a
-  // die has one head or few, and every die a share of every length
-  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk, part = item % nparts;
-  const int t = item / nparts;
+  // die has one head or few, and every die a share of every length.  The parts
+  // of a tile are not equal (the last may have fewer heads): they turn from tile
+  // to tile, so that no die has only the short ones
+  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
+  const int t = item / nparts, part = (item + t) % nparts;
   int seq, q0;
   if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
                  : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
@@ -111,24 +122,24 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
 
   const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
   const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
-  i32x4_t rk[T::LOADS], rv[T::LOADS];
   if (bend > 0) {
-    T::fetch(rk, kb, ldk, 0, Lk);
-    T::fetch(rv, vb, ldv, 0, Lk);
-    T::store(lds[0][0], rk);
-    T::store(lds[0][1], rv);
+    T::copy(k0_s, kb, ldk, Lk);
+    T::copy(v0_s, vb, ldv, Lk);
   }
   wait_loads();
-  if (ATILE < bend) {
-    T::fetch(rk, kb, ldk, ATILE, Lk);
-    T::fetch(rv, vb, ldv, ATILE, Lk);
-  }
   __syncthreads();
 
-  int buf = 0;
-  for (int t0 = 0; t0 < bend; t0 += ATILE, buf ^= 1) {
-    const char* ks_ = lds[buf][0];
-    const char* vs_ = lds[buf][1];
+  auto tile_step = [&](const char* ks_, const char* vs_, char* kn, char* vn,
+                       int t0) {
+    const bool more = t0 + ATILE < bend;
+    if (more) {
+      kb += ATILE * ldk;
+      T::copy(kn, kb, ldk, Lk - t0 - ATILE);
+      if (!ONE_V) {
+        vb += ATILE * ldv;
+        T::copy(vn, vb, ldv, Lk - t0 - ATILE);
+      }
+    }
     at.renew();
     f32x16_t s[2];
     if (t0 < wend) {
@@ -141,32 +152,23 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
         for (int n = 0; n < 2; ++n)
           s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_rows<D>(ks_, at, n, ks), qf[ks], s[n], 0, 0, 0);
-      SCHED_LDS(6);
+      SCHED_LDS(3);
 #pragma unroll
-      for (int i = 0; i < 2 * KS - 6; ++i) {
+      for (int i = 0; i < 2 * KS - 3; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(1);
       }
-      SCHED_MFMA(6);
-    }
-    // the next tile into the other buffer (its readers passed the barrier)
-    if (t0 + ATILE < bend) {
-      T::store(lds[buf ^ 1][0], rk);
-      T::store(lds[buf ^ 1][1], rv);
-      if (t0 + 2 * ATILE < bend) {
-        T::fetch(rk, kb, ldk, t0 + 2 * ATILE, Lk);
-        T::fetch(rv, vb, ldv, t0 + 2 * ATILE, Lk);
-      }
-    }
-    if (t0 < wend) {
+      SCHED_MFMA(3);
       // ---- mask (wave-uniform: some key of the tile is hidden) --------------
       if (t0 + ATILE > Lk || (causal && t0 + ATILE - 1 > qk_off + wq0)) {
-        const int last = min(qpos, Lk - 1) - t0;
+        // (in this lane's rows of the accumulators, so that the numbers it is
+        // compared with are literals: else they live in 32 registers)
+        const int last = min(qpos, Lk - 1) - t0 - 4 * (lane >> 5);
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            if (n * 32 + acc_row(r) > last) s[n][r] = hidden;
+            if (n * 32 + 8 * (r >> 2) + (r & 3) > last) s[n][r] = hidden;
       }
       // ---- online softmax -----------------------------------------------------
       // (largest score: the smallest product where the scale is negative)
@@ -213,6 +215,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
           sum += s[n][r];
         }
       l_run += sum;
+    }
+    if (ONE_V) {
+      // this tile's values are there, the next keys may still be on their way
+      if (more) wait_all_but<T::LOADS>();
+      else wait_loads();
+      __syncthreads();
+    }
+    if (t0 < wend) {
       // ---- O^T += V^T P^T ------------------------------------------------------
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
@@ -222,21 +232,31 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_cols<D>(vs_, at, dt, st), p, o[dt], 0, 0, 0);
       }
-      SCHED_LDS(8);
+      SCHED_LDS(4);
 #pragma unroll
-      for (int i = 0; i < 4 * DT - 4; ++i) {
+      for (int i = 0; i < 4 * DT - 2; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(2);
       }
-      SCHED_MFMA(4);
+      SCHED_MFMA(2);
     }
+    wait_loads();
     __syncthreads();
+    if (ONE_V && more) {
+      vb += ATILE * ldv;
+      T::copy(vn, vb, ldv, Lk - t0 - ATILE);
+    }
+  };
+  for (int t0 = 0; t0 < bend; t0 += 2 * ATILE) {
+    tile_step(k0_s, v0_s, k1_s, v1_s, t0);
+    if (t0 + ATILE < bend)
+      tile_step(k1_s, v1_s, k0_s, v0_s, t0 + ATILE);
   }
 
   // ---- out = O / l, turned through LDS to whole rows; lse = m + log l --------
   const float l = half_sum(l_run);
   const float inv = l > 0.f ? 1.0f / l : 0.f;
-  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
+  char* mine = (wid < 2 ? k0_s : v0_s) + wid % 2 * (32 * D * 2);
   if (busy) {
     if (lse != nullptr && lane < 32 && row < Lq)
       lse[((long)qbeg + row) * Hq + hq] =
@@ -294,6 +314,8 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
   if (table)
     TORCH_CHECK(tile_seq.dtype() == torch::kInt32 &&
                 tile_q0.dtype() == torch::kInt32);
+  k = rows_by16(k);
+  v = rows_by16(v);
   const int Hq = q.size(1), D = q.size(2), Hk = k.size(1);
   TORCH_CHECK(D == 128 || D == 64, "prefill kernel supports head_dim 64/128");
   TORCH_CHECK(Hq % Hk == 0);

@@ -28,9 +28,12 @@ typedef __attribute__((ext_vector_type(4))) short i16x4_t;
 typedef __attribute__((ext_vector_type(8))) short i16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_p;
+typedef __attribute__((address_space(3))) void* lds_p;
 
 #define ATILE 64                      // rows of a tile
 #define ATTN_XCDS 8                   // dies, each with an L2 of its own
+
+DEV_INLINE int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 template <int D>
 struct AttnTile {
@@ -60,6 +63,27 @@ struct AttnTile {
       reg[i] = __builtin_bit_cast(
           i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
                        from, at / GR * ldb + at % GR * 16, 0, 0));
+    }
+  }
+
+  // The same straight into LDS, without registers on the way: a wave's lanes
+  // write neighbouring granules, so the swizzle is in which granule of the row
+  // a lane asks for.  In flight until wait_loads().  The tiles that are read
+  // meanwhile have to be another array, else the compiler waits before it reads.
+  DEV_INLINE static void copy(char* tile, const bf16_t* rows0, long ld,
+                              int live) {
+    const int ldb = (int)ld * 2;
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(rows0), 0,
+        live > 0 ? (min(live, ATILE) - 1) * ldb + 2 * D : 0, 0x00020000);
+    const int r = threadIdx.x / GR, g = threadIdx.x % GR;
+    int at = r * ldb + ((g ^ swz(r)) << 4);
+    char* to = tile + uniform(threadIdx.x >> 6) * 1024;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          from, (lds_p)(to + i * 4096), 16, at, 0, 0, 0);
+      at += 256 / GR * ldb;              // (whole periods of the swizzle)
     }
   }
 
@@ -177,8 +201,9 @@ DEV_INLINE float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 // for a register that was loaded before the loop would otherwise stand inside
 // it and catch the loop's own loads.
 DEV_INLINE void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-DEV_INLINE int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+// all but the last N (at most 15)
+template <int N>
+DEV_INLINE void wait_all_but() { __builtin_amdgcn_s_waitcnt(0x0F70 | N); }
 
 // Sequence and first row of row tile ``tile``.  With a table it is looked
 // up; without one the tiles are the sequences' 64-row pieces in order, found
@@ -276,4 +301,12 @@ DEV_INLINE int wave_id() {
 DEV_INLINE int die_item(int items) {
   const int per = (items + ATTN_XCDS - 1) / ATTN_XCDS;
   return (int)(blockIdx.x % ATTN_XCDS) * per + (int)(blockIdx.x / ATTN_XCDS);
+}
+
+// Rows for AttnTile::copy, 16 bytes a lane: a tensor whose rows do not all start
+// at 16-byte addresses is laid out again.
+inline torch::Tensor rows_by16(const torch::Tensor& t) {
+  const bool ok = ((uintptr_t)t.data_ptr() & 15) == 0 &&
+                  (t.stride(0) % 8 == 0 || t.size(0) < 2);
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }

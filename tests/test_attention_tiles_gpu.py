@@ -446,3 +446,39 @@ def test_every_tile_once(nseq, d):
                 0 if klens[i] else int(lens[i]))
             assert (a[:blind] == 0).all()    # rows that see no key
             assert ((a[blind:] - (i + 1)).abs() <= 2 ** -8 * (i + 1)).all()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("offset,pad", [(1, 0), (0, 1), (4, 0), (0, 4)])
+def test_unaligned_rows(offset, pad, d):
+    """Keys, values, queries and gradients whose rows do not start at 16-byte
+    addresses give the bits that aligned copies give."""
+    torch.manual_seed(8)
+    lens, hq, hk, scale = [65, 130], 4, 2, d ** -0.5
+    cu, n = cu_of(lens).to(DEV), 195
+
+    def rows(h):
+        flat = torch.randn(n * (h * d + pad) + offset, device=DEV).bfloat16()
+        return flat[offset:].view(n, h * d + pad)[:, :h * d].unflatten(
+            1, (h, d))
+    q, k, v, dout = rows(hq), rows(hk), rows(hk), rows(hq)
+    got = ops.varlen_prefill_attention(q, k, v, cu, cu, scale, True)
+    want = ops.varlen_prefill_attention(*(t.clone() for t in (q, k, v)), cu,
+                                        cu, scale, True)
+    assert torch.equal(got, want)
+    ext, tiles = ops._require_ext(), ops.build_varlen_tiles(cu.cpu(), DEV)
+    out, lse = ops.varlen_prefill_attention(q, k, v, cu, cu, scale, True,
+                                            return_lse=True)
+    both = []
+    for make in (lambda t: t, lambda t: t.clone(
+            memory_format=torch.contiguous_format)):
+        grads = [torch.empty(t.shape, device=DEV).bfloat16()
+                 for t in (q, k, v)]
+        ext.varlen_attention_backward_v3(
+            *grads, make(q), make(k), make(v), out,
+            make(dout) if dout.is_contiguous() else dout.clone(
+                memory_format=torch.contiguous_format), lse, cu, cu,
+            tiles[0], tiles[1], scale, True)
+        both.append(grads)
+    for a, b in zip(*both):
+        assert torch.equal(a, b)
