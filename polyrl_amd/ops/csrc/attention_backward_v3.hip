@@ -21,19 +21,20 @@
 //    operands of dV^T += dO^T P and dK^T += Q^T dS.  256 registers a wave
 //    (two waves per SIMD, so that one's exponentials run beside the other's
 //    products) hold both gradients and K at D = 128 but not V, which is read
-//    from LDS; the next Q tile is in flight during the first two products,
-//    the next dO tile during the last two, in the same 16 registers.  Q has
-//    two LDS buffers, dO one (stored between two barriers).  The two waves of
+//    from LDS.  Tiles go straight into LDS (AttnTile::copy): Q has two buffers,
+//    dO one (two blocks with two of each are 162 KiB), whose next tile arrives
+//    beside one step's dK and the next step's S products.  The two waves of
 //    a key half meet at the end: each adds the other's share of one gradient.
 //    With few blocks the group's heads are divided among several (their
 //    shares then pass through fp32 and one summing kernel).
 //
-// What bounds it: matrix instructions and LDS reads of their operands (one
-// fragment of 1 KiB per 32-cycle product).  Measured, forward and backward of
-// packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with kernels
-// that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
-// gradients for a cast to read, 257 us now (349 with every fragment read just
-// before its product); 2 of up to 4096, 28/4 heads, 4000 -> 1295 us.
+// What bounds it: matrix instructions (about 40% of the cycles) and exponentials
+// with what surrounds them, of two waves in turn.  Measured, forward and
+// backward of packed sequences: 16 of up to 512, 32/8 heads of 128, 727 us with
+// kernels that turned Q, dO, K and dS into LDS two bytes at a time and wrote fp32
+// gradients for a cast to read, 231 with tiles through registers (whose loads and
+// stores took a fifth of the forward kernel's time), 220 now; 2 of up to 4096,
+// 28/4 heads, 4000, 1138 and 1015; 8 of up to 1024, 32/8 heads of 64, 200 and 190.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -41,7 +42,7 @@
 
 // ------------------------------------------------------------------- dQ
 template <int D>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
+__global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
     bf16_t* __restrict__ dq,         // (total_q, Hq, D)
     float* __restrict__ delta,       // (total_q, Hq)
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
@@ -52,11 +53,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
     const int* __restrict__ tile_q0, int nseq, int ntiles, int nparts, int Hq,
     int Hk, float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
-  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
+  // two buffers of K and V each; at the end the waves' rows of the gradient
+  __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
+      k1_s[T::BYTES], v1_s[T::BYTES];
 
   const int G = Hq / Hk;
-  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk, part = item % nparts;
-  const int t = item / nparts;
+  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
+  const int t = item / nparts, part = (item + t) % nparts;
   int seq, q0;
   if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
                  : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
@@ -82,6 +85,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
   const int bend = causal
       ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
+  const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
+  const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
+  if (bend > 0) {
+    T::copy(k0_s, kb, ldk, Lk);
+    T::copy(v0_s, vb, ldv, Lk);
+  }
   const long tok = qbeg + min(busy ? row : 0, Lq - 1);
   bf16x8_t qf[KS], df[KS];
   frag_global<D>(df, dout + (tok * Hq + hq) * D);
@@ -108,35 +117,23 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
 
-  const bf16_t* kb = k + (long)kbeg * ldk + (long)hk * D;
-  const bf16_t* vb = v + (long)kbeg * ldv + (long)hk * D;
-  // one set of registers: the next K tile is in flight during a tile's first
-  // 32 keys, the next V tile during the others
-  i32x4_t reg[T::LOADS];
-  if (bend > 0) {
-    T::fetch(reg, kb, ldk, 0, Lk);
-    T::store(lds[0][0], reg);
-    T::fetch(reg, vb, ldv, 0, Lk);
-    T::store(lds[0][1], reg);
-  }
   wait_loads();
   __syncthreads();
 
-  int buf = 0;
-  for (int t0 = 0; t0 < bend; t0 += ATILE, buf ^= 1) {
-    const bool more = t0 + ATILE < bend;
-    if (more) T::fetch(reg, kb, ldk, t0 + ATILE, Lk);
-    const char* ks_ = lds[buf][0];
-    const char* vs_ = lds[buf][1];
+  // one tile; the next one is on its way into the other buffers, whose readers
+  // passed the last barrier
+  auto tile_step = [&](const char* ks_, const char* vs_, char* kn, char* vn,
+                       int t0) {
+    if (t0 + ATILE < bend) {
+      kb += ATILE * ldk;
+      vb += ATILE * ldv;
+      T::copy(kn, kb, ldk, Lk - t0 - ATILE);
+      T::copy(vn, vb, ldv, Lk - t0 - ATILE);
+    }
     at.renew();
 #pragma unroll
     for (int n = 0; n < 2; ++n) {                  // 32 keys at a time
       const int k0 = t0 + n * 32;
-      // the other buffer's readers passed the last barrier
-      if (n == 1 && more) {
-        T::store(lds[buf ^ 1][0], reg);
-        T::fetch(reg, vb, ldv, t0 + ATILE, Lk);
-      }
       if (k0 >= wend) continue;
       f32x16_t s, dp;
 #pragma unroll
@@ -159,10 +156,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
       for (int r = 0; r < 16; ++r)
         s[r] = exp2_hw(__builtin_fmaf(s[r], s2, -lse2));
       if (k0 + 32 > Lk || (causal && k0 + 31 > qk_off + wq0)) {
-        const int last = min(qpos, Lk - 1) - k0;
+        // (compared with literals, in this lane's rows of the accumulators)
+        const int last = min(qpos, Lk - 1) - k0 - 4 * (lane >> 5);
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (acc_row(r) > last) s[r] = 0.f;
+          if (8 * (r >> 2) + (r & 3) > last) s[r] = 0.f;
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -183,12 +181,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(
       }
       SCHED_MFMA(4);
     }
-    if (more) T::store(lds[buf ^ 1][1], reg);
+    wait_loads();
     __syncthreads();
+  };
+  for (int t0 = 0; t0 < bend; t0 += 2 * ATILE) {
+    tile_step(k0_s, v0_s, k1_s, v1_s, t0);
+    if (t0 + ATILE < bend)
+      tile_step(k1_s, v1_s, k0_s, v0_s, t0 + ATILE);
   }
 
   // ---- dQ, turned through LDS to whole rows ---------------------------------
-  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
+  char* mine = (wid < 2 ? k0_s : v0_s) + wid % 2 * (32 * D * 2);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -230,14 +233,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   constexpr bool V_LDS = D == 128;   // V does not fit beside the gradients
-  // Q (two buffers), dO, V; at the end the exchange of 4 x 32 x D floats
-  __shared__ __attribute__((aligned(16))) char lds[4][T::BYTES];
+  __shared__ __attribute__((aligned(16))) char q0_s[T::BYTES], q1_s[T::BYTES],
+      do_s[T::BYTES], v_s[T::BYTES];
   // log-sum-exp (in powers of two) and scale * delta of the rows
-  __shared__ __attribute__((aligned(16))) float row_s[2][ATILE];
+  __shared__ __attribute__((aligned(16))) float r0_s[2][ATILE], r1_s[2][ATILE];
 
   const int G = Hq / Hk;
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
-  const int split = item % nsplit, t = item / nsplit;
+  const int t = item / nsplit, split = (item + t) % nsplit;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
   int seq, t0;
   if (nseq <= 64 ? !nth_longest<true>(t, cu_q, cu_k, nseq, seq, t0)
@@ -260,7 +263,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   frag_global<D>(kf, k + (long)krow * ldk + (long)hk * D);
   if constexpr (!V_LDS)
     frag_global<D>(vf, v + (long)krow * ldv + (long)hk * D);
-  const float s2 = scale * 1.4426950408889634f;
+  // (not 0: a hidden score is infinite, see the forward kernel)
+  const float s2 = scale != 0.f ? scale * 1.4426950408889634f : 0x1p-126f;
+  const float hidden = s2 >= 0.f ? -INFINITY : INFINITY;
 
   FragAt<D> at;
   f32x16_t ak[DT], av[DT];
@@ -276,10 +281,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const bf16_t* qb0 = q + (long)qbeg * ldq + (long)hk * G * D;
   const bf16_t* db0 = dout + ((long)qbeg * Hq + (long)hk * G) * D;
 
-  i32x4_t reg[T::LOADS];
   float rowv = 0.f;                                // lse or delta of a row
   bool rlive = false;
-  int fg = g0, fq = qs;               // head and first row of the next fetch
+  int fg = g0, fq = qs;               // head and first row of the next tile
   auto fetch_rows = [&]() {           // the first two waves' are stored
     const int r = fq + lane;
     const long i = ((long)qbeg + min(r, Lq - 1)) * Hq + hk * G +
@@ -287,74 +291,90 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     rlive = r < Lq;
     rowv = (wid == 0 ? lse : delta)[i];
   };
-  auto store_rows = [&]() {
+  auto store_rows = [&](float (*row_s)[ATILE]) {
     // rows past the end weigh nothing: 2^(s - inf) = 0
     if (wid == 0) row_s[0][lane] = rlive ? rowv * 1.4426950408889634f : INFINITY;
     if (wid == 1) row_s[1][lane] = rlive ? rowv * scale : 0.f;
   };
-  auto fetch_q = [&]() { T::fetch(reg, qb0 + (long)fg * D, ldq, fq, Lq); };
-  auto fetch_do = [&]() {             // and on to the next tile
-    T::fetch(reg, db0 + (long)fg * D, (long)Hq * D, fq, Lq);
+  auto copy_q = [&](char* to) {
+    T::copy(to, qb0 + (long)fg * D + fq * ldq, ldq, Lq - fq);
+  };
+  auto copy_do = [&]() {              // and on to the next tile
+    T::copy(do_s, db0 + (long)fg * D + (long)fq * Hq * D, (long)Hq * D,
+            Lq - fq);
     fq += ATILE;
     if (fq >= Lq) fq = qs, ++fg;
   };
   if (steps > 0) {
-    if constexpr (V_LDS) {
-      T::fetch(reg, v + (long)kbeg * ldv + (long)hk * D, ldv, t0, Lk);
-      T::store(lds[3], reg);
-    }
+    if constexpr (V_LDS)
+      T::copy(v_s, v + ((long)kbeg + t0) * ldv + (long)hk * D, ldv, Lk - t0);
     fetch_rows();
-    fetch_q();
-    T::store(lds[0], reg);
-    fetch_do();
-    T::store(lds[2], reg);
-    store_rows();
+    copy_q(q0_s);
+    copy_do();
+    store_rows(r0_s);
   }
   wait_loads();
   __syncthreads();
 
+  // One row tile.  S needs Q alone: the dO tile, whose one buffer was free only
+  // after the last step's dV product, arrives beside that step's dK and this
+  // step's S products (first barrier); the next Q tile beside the rest, up to
+  // the dV product (second).
   int q0 = qs;
-  for (int st = 0; st < steps; ++st) {
-    const int buf = st & 1;
-    const bool more = st + 1 < steps;
+  auto step = [&](const char* qs_, char* qn, float (*row_s)[ATILE],
+                  float (*row_n)[ATILE], bool more) {
     const int wq0 = q0 + qh * 32;                     // this wave's rows
     q0 = q0 + ATILE < Lq ? q0 + ATILE : qs;
     const bool work = wq0 < Lq && wk0 < Lk &&
                       (!causal || qk_off + wq0 + 31 >= wk0);
-    const char* qs_ = lds[buf];
-    const char* ds_ = lds[2];
     at.renew();
-    // (in every step: under a condition the register would be copied at the
-    // join, and the copy would wait for the load)
-    fetch_rows();
-    if (more) fetch_q();
+    f32x16_t s, dp;
     bf16x8_t p[2], ds[2];
     if (work) {
-      f32x16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = 0.f, dp[r] = 0.f;
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
+      for (int ks = 0; ks < KS; ++ks)
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             frag_rows<D>(qs_, at, qh, ks), kf[ks], s, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            frag_rows<D>(ds_, at, qh, ks),
-            V_LDS ? frag_rows<D>(lds[3], at, kh, ks) : vf[V_LDS ? 0 : ks], dp,
-            0, 0, 0);
-      }
-      constexpr int PER = V_LDS ? 3 : 2;           // fragments of a pair
-      SCHED_LDS(2 * PER);
+      SCHED_LDS(3);
 #pragma unroll
-      for (int i = 0; i < KS - 2; ++i) {
+      for (int i = 0; i < KS - 3; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(1);
-        SCHED_MFMA(1);
-        SCHED_LDS(PER - 1);
       }
-      SCHED_MFMA(4);
-      // accumulator rows before this lane's key, at the causal border only
-      const int border = causal && qk_off + wq0 < wk0 + 31
-          ? key - (qk_off + wq0) - 4 * (lane >> 5) : 0;
+      SCHED_MFMA(3);
+    }
+    wait_loads();
+    __syncthreads();
+    if (more) {
+      fetch_rows();
+      copy_q(qn);
+    }
+    if (work) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dp[r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            frag_rows<D>(do_s, at, qh, ks),
+            V_LDS ? frag_rows<D>(v_s, at, kh, ks) : vf[V_LDS ? 0 : ks], dp, 0,
+            0, 0);
+      constexpr int PER = V_LDS ? 2 : 1;           // fragments of a product
+      SCHED_LDS(3 * PER);
+#pragma unroll
+      for (int i = 0; i < KS - 3; ++i) {
+        SCHED_MFMA(1);
+        SCHED_LDS(PER);
+      }
+      SCHED_MFMA(3);
+      // rows before this lane's key (compared with literals)
+      if (causal && qk_off + wq0 < wk0 + 31) {
+        const int border = key - (qk_off + wq0) - 4 * (lane >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) < border) s[r] = hidden;
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r0 = qh * 32 + 8 * i + 4 * (lane >> 5);
@@ -365,8 +385,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * i + t;
-          float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
-          if (8 * i + t < border) w = 0.f;
+          const float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
           s[r] = w;
           dp[r] = w * __builtin_fmaf(dp[r], scale, -d4[t]);
         }
@@ -376,42 +395,46 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         p[h] = acc_operand(s, h);
         ds[h] = acc_operand(dp, h);
       }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          av[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              frag_cols<D>(do_s, at, dt, qh * 2 + h), p[h], av[dt], 0, 0, 0);
     }
-    if (more) {
-      T::store(lds[buf ^ 1], reg);
-      fetch_do();
-    }
+    if (more) store_rows(row_n);
+    wait_loads();
+    __syncthreads();
+    if (more) copy_do();
     if (work) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          av[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              frag_cols<D>(ds_, at, dt, qh * 2 + h), p[h], av[dt], 0, 0, 0);
+        for (int dt = 0; dt < DT; ++dt)
           ak[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_cols<D>(qs_, at, dt, qh * 2 + h), ds[h], ak[dt], 0, 0, 0);
-        }
-      }
       SCHED_LDS(6);
 #pragma unroll
-      for (int i = 0; i < 4 * DT - 3; ++i) {
+      for (int i = 0; i < 2 * DT - 3; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(2);
       }
       SCHED_MFMA(3);
     }
-    __syncthreads();                   // every wave is done with the dO tile
-    if (more) {
-      T::store(lds[2], reg);
-      store_rows();
-      __syncthreads();
-    }
+  };
+  for (int st = 0; st < steps; st += 2) {
+    step(q0_s, q1_s, r0_s, r1_s, st + 1 < steps);
+    if (st + 1 < steps) step(q1_s, q0_s, r1_s, r0_s, st + 2 < steps);
   }
+  __syncthreads();
 
   // ---- the two waves of a key half: one completes dV, the other dK ----------
-  float* mine = reinterpret_cast<float*>(&lds[0][0]) + wid * (D * 32);
-  const float* other =
-      reinterpret_cast<const float*>(&lds[0][0]) + (wid ^ 2) * (D * 32);
+  auto share = [&](int w) {
+    return reinterpret_cast<float*>(w == 0 ? q0_s : w == 1 ? q1_s
+                                    : w == 2 ? do_s : v_s);
+  };
+  float* mine = share(wid);
+  const float* other = share(wid ^ 2);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -498,22 +521,25 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
           cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), t_seq.data_ptr<int>(),
           t_q0.data_ptr<int>(), nseq, (int)ntiles, nparts, Hq, Hk, scale,
           causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
-  // Blocks of the dkv kernel are as long as their key is early, so the chip
-  // needs several per slot (512: two per CU) to end together; with few blocks
-  // each takes fewer heads of the group.  Long sequences are cut finer: the
-  // shares' trip through fp32 costs as much whatever the length.  Measured,
-  // forward and backward, all heads / two / one a block: 2 sequences of 3300 and
-  // 4096, 28/4 heads (464 blocks) 1470 / 1323 / 1315 us; one of 4096, 32/8 heads
-  // (512) 848 / 773 / 770; 3 of 4096, 28/4 (768) 2250 / 2167 / 2178.  Sequences
-  // of 130 to 512, 32/8 heads: 16 (720 blocks) 184 / 192 / 228, 12 (576) 157 /
-  // 166 / 182, 8 (368) 126 / 121 / 131; 16 of 28/4 heads (372) 213 / 198 / 222.
+  // Blocks of the dkv kernel are as long as their key is early and run longest
+  // first, 512 at a time (two per CU).  For all to end together the longest may
+  // not exceed a slot's share of the steps: in a sequence of m tiles the longest
+  // block takes m steps a head, a slot's share is G * base * m / 2 / 512, so a
+  // block takes 0.9 of G * base / 1024 heads of its group.  Sequences of less
+  // than 16 tiles are cut less fine: the shares' trip through fp32 costs as much
+  // whatever the length.  Measured, forward and backward: 2 sequences of 3500 ..
+  // 4096, 28/4 heads (476 key tiles), blocks of 1, 2, 3 and 4 heads 1041, 1015,
+  // 1015, 1037 us; one of 4096, 32/8 heads (512), of 1, 2 and 4 668, 669, 735; 3 of
+  // 4096, 28/4 (768), of 3, 4 and 7 1830, 1828, 1837.  Sequences of 800 .. 1024,
+  // 64/8 heads (480), of 2, 3 and 4 389, 384, 376; 16 of 130 .. 512, 28/4 heads
+  // (372), of 2, 3 and 4 170, 161, 155.
   // The shares take 64 KiB a block at D = 128 while the call runs: at most 48 MiB
   // times the heads of a group.
   const long base = ntiles * Hk;
   const bool lengthy = ntiles >= 16 * nseq;
   int nsplit = 1;
   if (base < (lengthy ? 768 : 512)) {
-    const int per = (int)(lengthy ? std::max<long>(1, G * base / 4096)
+    const int per = (int)(lengthy ? std::max<long>(1, G * base * 9 / 10240)
                                   : (G * base + 767) / 768);
     nsplit = (G + per - 1) / per;
   }
@@ -565,6 +591,7 @@ void varlen_attention_backward_v3(
   TORCH_CHECK(Hq % Hk == 0);
   if (t64_seq.size(0) == 0) return;
   (D == 128 ? launch_bwd<128> : launch_bwd<64>)(
-      dq, dk, dv, q, k, v, out, dout, lse, cu_seqlens_q, cu_seqlens_k,
+      dq, dk, dv, rows_by16(q), rows_by16(k), rows_by16(v), out,
+      rows_by16(dout), lse, cu_seqlens_q, cu_seqlens_k,
       t64_seq, t64_q0, (float)scale, causal);
 }

@@ -46,30 +46,13 @@ struct AttnTile {
                     : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
   }
 
-  // this thread's granules of rows [r0, r0 + 64) of one head; rows from
-  // ``rows`` on are zeros (a weight of 0 meets them, and 0 * inf is NaN).  The
-  // buffer ends with the last row's granules of this head; what a lane asks
-  // for behind it is not read and returns 0.
-  DEV_INLINE static void fetch(i32x4_t (&reg)[LOADS], const bf16_t* base,
-                               long ld, int r0, int rows) {
-    // a block-uniform buffer and 32-bit offsets inside the tile
-    const int ldb = (int)ld * 2, live = min(rows - r0, ATILE);
-    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16_t*>(base + r0 * ld), 0,
-        live > 0 ? (live - 1) * ldb + 2 * D : 0, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int at = threadIdx.x + i * 256;
-      reg[i] = __builtin_bit_cast(
-          i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                       from, at / GR * ldb + at % GR * 16, 0, 0));
-    }
-  }
-
-  // The same straight into LDS, without registers on the way: a wave's lanes
-  // write neighbouring granules, so the swizzle is in which granule of the row
-  // a lane asks for.  In flight until wait_loads().  The tiles that are read
-  // meanwhile have to be another array, else the compiler waits before it reads.
+  // Rows [0, min(live, 64)) of one head straight into a tile, zeros behind them
+  // (a weight of 0 meets them, and 0 * inf is NaN): the buffer ends with the last
+  // row's granules of this head, and what a lane asks for behind it is not read
+  // and is 0.  No registers on the way: a wave's lanes write neighbouring
+  // granules, so the swizzle is in which granule of its row a lane asks for.  In
+  // flight until wait_loads().  The tiles that are read meanwhile have to be
+  // another array, else the compiler waits before it reads.
   DEV_INLINE static void copy(char* tile, const bf16_t* rows0, long ld,
                               int live) {
     const int ldb = (int)ld * 2;
