@@ -44,12 +44,6 @@
 
 #include "attention_tile.h"
 
-// a * b, never fused with what it is added to
-DEV_INLINE float rounded_product(float a, float b) {
-#pragma clang fp contract(off)
-  return a * b;
-}
-
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 4 : 3) void prefill_attn_kernel(
     bf16_t* __restrict__ out,        // (total_q, Hq, D)

@@ -29,6 +29,7 @@ typedef __attribute__((ext_vector_type(8))) short i16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_p;
 typedef __attribute__((address_space(3))) void* lds_p;
+typedef __attribute__((address_space(1))) const void* global_p;
 
 #define ATILE 64                      // rows of a tile
 #define ATTN_XCDS 8                   // dies, each with an L2 of its own
@@ -70,26 +71,26 @@ struct AttnTile {
     }
   }
 
-  DEV_INLINE static void store(char* tile, const i32x4_t (&reg)[LOADS]) {
+  // The same from 64 rows that start ``start[r]`` numbers behind ``base``
+  DEV_INLINE static void gather(char* tile, const bf16_t* base,
+                                const long* start) {
+    const int r = threadIdx.x / GR, g = threadIdx.x % GR;
+    const bf16_t* from = base + (g ^ swz(r)) * 8;
+    char* to = tile + uniform(threadIdx.x >> 6) * 1024;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int at = threadIdx.x + i * 256;
-      const int r = at / GR;
-      *reinterpret_cast<i32x4_t*>(tile + r * (2 * D) +
-                                 ((at % GR ^ swz(r)) << 4)) = reg[i];
-    }
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (global_p)(from + start[r + i * (256 / GR)]), (lds_p)(to + i * 4096),
+          16, 0, 0);
   }
 
-  // the same with zeros for the rows from ``live`` on: a value that a weight
-  // of 0 meets has to be finite, and the last row, repeated, need not be
-  DEV_INLINE static void store_live(char* tile, i32x4_t (&reg)[LOADS],
-                                    int live) {
-    if (live < ATILE) {                // the same for the whole block
+  // zeros for this thread's granules of the rows from ``live`` on
+  DEV_INLINE static void clear_from(char* tile, int live) {
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i)
-        if ((int)(threadIdx.x + i * 256) / GR >= live) reg[i] = {0, 0, 0, 0};
-    }
-    store(tile, reg);
+    for (int i = 0; i < LOADS; ++i)
+      if ((int)(threadIdx.x + i * 256) / GR >= live)
+        *reinterpret_cast<i32x4_t*>(tile + (threadIdx.x + i * 256) * 16) =
+            i32x4_t{0, 0, 0, 0};
   }
 };
 
@@ -169,6 +170,12 @@ DEV_INLINE float half_sum(float x) {
   const auto p = __builtin_amdgcn_permlane32_swap(
       __float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+// a * b, never fused with what it is added to
+DEV_INLINE float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
 }
 
 // 2^x in one instruction; results below 2^-126 become 0

@@ -376,14 +376,16 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
 // of one head; a block is four such units of one row tile and one key/value
 // head, heads of the group first, so four heads share each K and V tile where
 // the general kernel fetches it for every head.  Values stay row-major in LDS
-// and are read turned (layouts and operands: attention_tile.h); tiles are
-// fetched 16 bytes a lane, whole rows together, where the general kernel
-// collects values 8 bytes at a time, one row per lane.  The next K tile is in
-// flight during a tile's score products, the next V tile during its value
-// products, in the same registers.  Measured, eight prompts of 1200 .. 2048
-// tokens, window 1024, 32/8 heads of 64: 547 us in the general kernel, 159 here.
+// and are read turned (layouts and operands: attention_tile.h); tiles go straight
+// into LDS (AttnTile::gather), buffers and blocks per CU as in
+// attention_prefill.hip.  Measured, eight prompts of 1200 .. 2048 tokens, window
+// 1024, 32/8 heads of 64: 547 us in the general kernel, 155 with tiles through
+// registers and three blocks per CU, 139 here (119 with no tile loaded after the
+// first); of 128: 270 and 243.  Row tiles run by their number: longest walk first
+// found from the tables, as attention_prefill.hip finds it from the lengths, took
+// 157 for 156 (windowed walks are alike).
 template <int D>
-__global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
+__global__ __launch_bounds__(256, D == 64 ? 4 : 3) void gqa_attn_tile_kernel(
     bf16_t* __restrict__ out,            // (N, H*D), row stride ldo
     const bf16_t* __restrict__ q,        // (N, H*D)
     const bf16_t* __restrict__ cache,    // (slots, 2*G*D)
@@ -395,8 +397,12 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
     const float* __restrict__ sink, float qt_coef, int qt_every, int chunk,
     long ldo, float out_scale) {
   typedef AttnTile<D> T;
-  __shared__ __attribute__((aligned(16))) char lds[2][2][T::BYTES];
-  __shared__ int slot_s[2][ATILE];       // cache rows of a tile's keys
+  constexpr bool ONE_V = D == 128;
+  // two buffers of K, two or one of V; at the end the waves' rows of the output
+  __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
+      k1_s[T::BYTES], vx_s[ONE_V ? 16 : T::BYTES];
+  char* const v1_s = ONE_V ? v0_s : vx_s;
+  __shared__ long slot_s[2][ATILE];      // where a tile's keys' rows start
   constexpr int KS = D / 16, DT = D / 32;
   constexpr float L2E = 1.4426950408889634f;
 
@@ -436,11 +442,12 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
   };
   auto tile_jmax = [&](int ti) { return ti < nkt ? nk - 1 : pmax; };
   auto tile_live = [&](int ti) { return tile_jmax(ti) - tile_t0(ti) + 1; };
-  // cache row of a tile's key i (keys past the tile's last: that one)
+  const long row = 2L * G * D;
+  // where the row of a tile's key i starts (keys past the tile's last: that one)
   auto slot_of = [&](int ti, int i) {
     const int j = min(tile_t0(ti) + i, tile_jmax(ti));
     const int pg = j / page_size;
-    return ptab[pg] * page_size + (j - pg * page_size);
+    return ((long)ptab[pg] * page_size + (j - pg * page_size)) * row;
   };
   if (wid < 2 && wid < ntiles) slot_s[wid][lane] = slot_of(wid, lane);
 
@@ -464,38 +471,35 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
 
   FragAt<D> at;
-  const long row = 2L * G * D;
   const bf16_t* kb = cache + (long)g * D;
   const bf16_t* vb = kb + (long)G * D;
-  i32x4_t reg[T::LOADS];                 // the tile in flight, K and V in turn
-  auto fetch = [&](const bf16_t* from, int ti) {
-#pragma unroll
-    for (int i = 0; i < T::LOADS; ++i) {
-      const int a = threadIdx.x + i * 256;
-      reg[i] = *reinterpret_cast<const i32x4_t*>(
-          from + slot_s[ti & 1][a / T::GR] * row + a % T::GR * 8);
-    }
+  auto copy = [&](char* to, const bf16_t* from, int ti) {
+    T::gather(to, from, slot_s[ti & 1]);
+  };
+  // (a weight of 0 meets what stands in for rows past the last key: zeros for
+  // the values, that row again for the keys)
+  auto end_rows = [&](char* v_s, int ti) {
+    if (tile_live(ti) < ATILE) T::clear_from(v_s, tile_live(ti));
   };
   __syncthreads();
-  fetch(kb, 0);
-  T::store(lds[0][0], reg);
-  fetch(vb, 0);
-  T::store_live(lds[0][1], reg, tile_live(0));
+  copy(k0_s, kb, 0);
+  copy(v0_s, vb, 0);
   wait_loads();
+  end_rows(v0_s, 0);
   __syncthreads();
 
-  for (int ti = 0; ti < ntiles; ++ti) {
-    const int buf = ti & 1;
+  auto tile_step = [&](const char* ks_, char* vs_, char* kn, char* vn, int ti) {
     const int t0 = tile_t0(ti), jmax = tile_jmax(ti);
-    const char* ks_ = lds[buf][0];
-    const char* vs_ = lds[buf][1];
+    const bool more = ti + 1 < ntiles;
+    if (more) {
+      copy(kn, kb, ti + 1);
+      if (!ONE_V) copy(vn, vb, ti + 1);
+    }
     at.renew();
     // a key of the tile that some row of the wave sees
     const bool work = busy && t0 <= wp1 &&
                       (ti < nkt || min(t0 + ATILE - 1, jmax) >= wlo0 ||
                        t0 < keep);
-    const bool more = ti + 1 < ntiles;
-    if (more) fetch(kb, ti + 1);
     f32x16_t s[2];
     if (work) {
 #pragma unroll
@@ -506,32 +510,34 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
         for (int n = 0; n < 2; ++n)
           s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_rows<D>(ks_, at, n, ks), qf[ks], s[n], 0, 0, 0);
-      SCHED_LDS(6);
+      SCHED_LDS(3);
 #pragma unroll
-      for (int i = 0; i < 2 * KS - 6; ++i) {
+      for (int i = 0; i < 2 * KS - 3; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(1);
       }
-      SCHED_MFMA(6);
-    }
-    // into the other buffer (its readers passed the last barrier)
-    if (more) {
-      T::store(lds[buf ^ 1][0], reg);
-      fetch(vb, ti + 1);
-    }
-    if (work) {
+      SCHED_MFMA(3);
+      // The scale goes into the exponential.  Where some row's is not positive
+      // (the largest score is then not the largest product) it is multiplied in.
+      float by = s2, less;
+      if (!__all(s2 > 0.f)) {
 #pragma unroll
-      for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < 2; ++n)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[n][r] *= s2;
+          for (int r = 0; r < 16; ++r) s[n][r] *= s2;
+        by = 1.f;
+      }
       if (!(t0 + ATILE - 1 <= min(wp0, jmax) && t0 >= wlo)) {
+        // hidden: after the row, or before its window and not kept (in this
+        // lane's rows of the accumulators, compared with literals)
+        const int base = t0 + 4 * (lane >> 5), last = min(jmax, rpos) - base,
+                  lo = rlo - base, kept = keep - base;
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int j = t0 + n * 32 + acc_row(r);
-            const bool live = j <= jmax && j <= rpos && (j >= rlo || j < keep);
-            if (!live) s[n][r] = -INFINITY;
+            const int j = n * 32 + 8 * (r >> 2) + (r & 3);
+            if (j > last || (j < lo && j >= kept)) s[n][r] = -INFINITY;
           }
       }
       float mx = s[0][0];
@@ -539,7 +545,7 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
-      const float mn = fmaxf(m_run, half_max(mx));
+      const float mn = fmaxf(m_run, half_max(mx * by));
       if (__any(mn > m_run)) {           // the largest weight is exactly 1
         const float alpha = exp2_hw(m_run - mn);
         l_run *= alpha;
@@ -549,15 +555,35 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
           for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
         m_run = mn;
       }
+      less = m_run;
+      // (very large scores are rounded like their maximum: what it lost to
+      // rounding would pass the exponential's range)
+      if (__any(fabsf(m_run) >= 0x1p24f)) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[n][r] = rounded_product(s[n][r], by) - m_run;
+        by = 1.f, less = 0.f;
+      }
       float sum = 0.f;
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          s[n][r] = exp2_hw(s[n][r] - m_run);
+          s[n][r] = exp2_hw(__builtin_fmaf(s[n][r], by, -less));
           sum += s[n][r];
         }
       l_run += sum;
+    }
+    if (ONE_V) {
+      // this tile's values are there, the next keys may still be on their way
+      if (more) wait_all_but<T::LOADS>();
+      else wait_loads();
+      end_rows(vs_, ti);
+      __syncthreads();
+    }
+    if (work) {
       // ---- O^T += V^T P^T ------------------------------------------------------
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
@@ -567,25 +593,33 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               frag_cols<D>(vs_, at, dt, st), p, o[dt], 0, 0, 0);
       }
-      SCHED_LDS(8);
+      SCHED_LDS(4);
 #pragma unroll
-      for (int i = 0; i < 4 * DT - 4; ++i) {
+      for (int i = 0; i < 4 * DT - 2; ++i) {
         SCHED_MFMA(1);
         SCHED_LDS(2);
       }
-      SCHED_MFMA(4);
+      SCHED_MFMA(2);
     }
-    if (more) T::store_live(lds[buf ^ 1][1], reg, tile_live(ti + 1));
-    // (the rows of this tile were last looked up before the last barrier)
-    if (wid == 0 && ti + 2 < ntiles) slot_s[buf][lane] = slot_of(ti + 2, lane);
+    // (this tile's rows were last looked up before the last barrier, the next
+    // one's stand in the other half)
+    if (wid == 0 && ti + 2 < ntiles)
+      slot_s[ti & 1][lane] = slot_of(ti + 2, lane);
+    wait_loads();
+    if (!ONE_V && more) end_rows(vn, ti + 1);
     __syncthreads();
+    if (ONE_V && more) copy(vn, vb, ti + 1);
+  };
+  for (int ti = 0; ti < ntiles; ti += 2) {
+    tile_step(k0_s, v0_s, k1_s, v1_s, ti);
+    if (ti + 1 < ntiles) tile_step(k1_s, v1_s, k0_s, v0_s, ti + 1);
   }
 
   // ---- out: 32 rows turned through LDS to whole rows -------------------------
   const float l = half_sum(l_run);
   float inv = 1.f / l * out_scale;
   if (gate) inv *= sigmoidf_acc(bf2f(gate[(long)(n0 + ri) * ldg + h]));
-  char* mine = &lds[0][0][0] + wid * (32 * D * 2);
+  char* mine = (wid < 2 ? k0_s : v0_s) + wid % 2 * (32 * D * 2);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll

@@ -482,3 +482,38 @@ def test_unaligned_rows(offset, pad, d):
         both.append(grads)
     for a, b in zip(*both):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("scale", [-0.1, 0.0, 2.0 ** 40, -2.0 ** 40])
+def test_window_scales(scale, d):
+    """Window attention at scales that are not positive (the largest score is
+    not the largest product) or so large that an exponent's rounding passes
+    the exponential's range: each row gets the value of its largest score."""
+    torch.manual_seed(9)
+    lens, hq, hk, page, window, keep = [3, 150], 4, 2, 16, 70, 2
+    table = torch.arange(20, dtype=torch.int32, device=DEV).view(2, 10)
+    rows = torch.randn(20, page, 2 * hk * d, device=DEV).bfloat16()
+    n = sum(lens)
+    q = torch.randn(n, hq * d, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(2, **i32),
+                                  torch.tensor(lens, device=DEV))
+    pos = torch.cat([torch.arange(x, **i32) for x in lens])
+    got = ops.seq.gqa_window_attention(
+        q, rows, table, seq, pos, hq, hk, d, d, window, keep, None, None,
+        None, scale, torch.bfloat16, tiles=ops.seq.attention_tiles(lens, DEV))
+    a = 0
+    for i, x in enumerate(lens):
+        kv = rows[table[i].long()].view(-1, 2, hk, d)[:x].double()
+        k, v = heads(kv[:, 0], hq), heads(kv[:, 1], hq)
+        r, j = torch.arange(x, device=DEV)[:, None], torch.arange(x, device=DEV)
+        live = ((r - j < window) | (j < keep)) & (j <= r)
+        s = torch.einsum("qhd,khd->hqk", q[a:a + x].double().view(x, hq, d),
+                         k) * scale
+        p = torch.softmax(s.masked_fill(~live, -float("inf")), -1)
+        want = torch.einsum("hqk,khd->qhd", p, v)
+        mass = torch.einsum("hqk,khd->qhd", p, v.abs())
+        assert ((got[a:a + x].double().view(x, hq, d) - want).abs()
+                <= 2 ** -8 * (mass + want.abs())).all(), i
+        a += x
