@@ -33,10 +33,16 @@
 // 0.99 takes top-p 0.95 of 256 x 152064 from 229 to 254 us.
 //
 // What bounds it: integer multiplies of the generator (two 64-bit products a
-// number).  The two logarithms of a number's noise are only taken where its
-// 24 random bits can beat the wave's best so far: z > best means
-// u > exp(-exp(x/T - best)), one threshold per 16-byte word of logits from
-// the word's largest, with a margin far above the rounding of either side.
+// number; a number's place in the sequence is the last one's plus a constant, kept
+// from the compiler, which would multiply).  Vector instructions are 88% of the
+// cycles, 250 a word of eight numbers and as many again a wave for the exchange
+// of its lanes, which goes by DPP (128 x 128256 at temperature 1: 33.1 us with a
+// product for the place and exchanges through LDS, 28.7 now; each lane's most
+// promising number of the first word first, as a bound, took 29.4).  The two
+// logarithms of a number's noise are only taken where its 24 random bits can beat
+// the wave's best so far: z > best means u > exp(-exp(x/T - best)), one threshold
+// per 16-byte word of logits from the word's largest, with a margin far above the
+// rounding of either side.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -54,20 +60,22 @@ DEV_INLINE uint64_t splitmix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// 24 random bits of entry i0 + j (one product for the entries of a word)
-DEV_INLINE uint32_t rng_bits(uint64_t rowkey, int i0, int j) {
-  constexpr uint64_t mul = 0xd1342543de82ef95ull;
-  const uint64_t at =
-      (uint64_t)(int64_t)i0 * mul + (mul * (unsigned)j + 0x2545f4914f6cdd1dull);
-  return (uint32_t)(splitmix64(rowkey ^ at) >> 40);
+// 32 random bits of an entry, of which the upper 24 are used.  ``at``: the entry's
+// place in the sequence, rng_at() of it or of another one plus the distance
+constexpr uint64_t RNG_STEP = 0xd1342543de82ef95ull;
+DEV_INLINE uint64_t rng_at(int i) {
+  return (uint64_t)(int64_t)i * RNG_STEP + 0x2545f4914f6cdd1dull;
+}
+DEV_INLINE uint32_t rng_bits(uint64_t rowkey, uint64_t at) {
+  return (uint32_t)(splitmix64(rowkey ^ at) >> 32);
 }
 
-// Gumbel noise of these bits: u = (bits + 1) / 2^24.  The largest bits stand
+// Gumbel noise of 24 bits: u = (bits + 1) / 2^24.  The largest bits stand
 // for the numbers between 1 - 2^-24 and 1: -log u is 2^-25 in their middle (at
 // u = 1 the noise would be infinite and the entry drawn whatever its logit,
 // in one row of 130 at 128256 entries).
 DEV_INLINE float gumbel(uint32_t bits) {
-  const float u = ((float)bits + 1.0f) * (1.0f / 16777216.0f);
+  const float u = ((float)(bits >> 8) + 1.0f) * (1.0f / 16777216.0f);
   return -__logf(fmaxf(-__logf(u), 0x1p-25f));
 }
 
@@ -89,19 +97,57 @@ DEV_INLINE bool better(float v, int i, float w, int j) {
   return v > w || (v == w && i < j);
 }
 
-DEV_INLINE float first_lane(float v) {
-  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+// x or that of the lane that CTRL names, if larger (its own where none stands)
+template <int CTRL, int ROWS>
+DEV_INLINE float larger_from(float x) {
+  const int own = __float_as_int(x);
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(
+                      own, own, CTRL, ROWS, 0xf, false)));
+}
+// the largest of the wave's numbers; all lanes take part
+DEV_INLINE float wave_largest(float x) {
+  x = larger_from<0x111, 0xf>(x);        // row_shr 1, 2, 4, 8
+  x = larger_from<0x112, 0xf>(x);
+  x = larger_from<0x114, 0xf>(x);
+  x = larger_from<0x118, 0xf>(x);
+  x = larger_from<0x142, 0xa>(x);        // row_bcast 15, 31
+  x = larger_from<0x143, 0xc>(x);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
-// over W lanes: 64, or each W neighbours
-template <int W = 64>
+template <int CTRL, int ROWS>
+DEV_INLINE float plus_from(float x) {
+  return x + __int_as_float(__builtin_amdgcn_update_dpp(
+                 0, __float_as_int(x), CTRL, ROWS, 0xf, ROWS == 0xf));
+}
+DEV_INLINE float wave_sum(float x) {
+  x = plus_from<0x111, 0xf>(x);
+  x = plus_from<0x112, 0xf>(x);
+  x = plus_from<0x114, 0xf>(x);
+  x = plus_from<0x118, 0xf>(x);
+  x = plus_from<0x142, 0xa>(x);
+  x = plus_from<0x143, 0xc>(x);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+template <int CTRL, int ROWS>
+DEV_INLINE int smaller_from(int x) {
+  return min(x, __builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false));
+}
+DEV_INLINE int wave_smallest(int x) {
+  x = smaller_from<0x111, 0xf>(x);
+  x = smaller_from<0x112, 0xf>(x);
+  x = smaller_from<0x114, 0xf>(x);
+  x = smaller_from<0x118, 0xf>(x);
+  x = smaller_from<0x142, 0xa>(x);
+  x = smaller_from<0x143, 0xc>(x);
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// the wave's best, in every lane
 DEV_INLINE void wave_best(float& v, int& i) {
-#pragma unroll
-  for (int off = W / 2; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(v, off, 64);
-    const int oi = __shfl_xor(i, off, 64);
-    if (better(ov, oi, v, i)) v = ov, i = oi;
-  }
+  const float most = wave_largest(v);
+  i = wave_smallest(v == most ? i : 0x7fffffff);
+  v = most;
 }
 
 // running maximum and softmax sums of a thread
@@ -160,12 +206,14 @@ struct Sums {
     }
     m = c;
   }
-  template <int W = 64>
+  // the wave's, in every lane
   DEV_INLINE void wave(float inv_temp) {
-#pragma unroll
-    for (int off = W / 2; off > 0; off >>= 1)
-      merge(__shfl_xor(m, off, 64), __shfl_xor(s, off, 64),
-            TEMP ? __shfl_xor(st, off, 64) : 0.f, inv_temp);
+    const float c = wave_largest(m);
+    // (equal also where both are -inf: the sum is 0 or NaN then)
+    const float own = m == c ? 1.f : __expf(m - c);
+    s = wave_sum(s * own);
+    if (TEMP) st = wave_sum(m == c ? st : st * shift(m, c, inv_temp));
+    m = c;
   }
 };
 
@@ -180,34 +228,33 @@ struct Draw {
   DEV_INLINE void add(const float (&v)[N], float c, int i0, int V,
                       uint64_t rowkey, float inv_temp, uint32_t tau) {
     if (tau != 0 && !__any(enc_f32(c) >= tau)) return;
-    // 24-bit numbers below this lose whatever the logit (all may win at a
-    // negative temperature, where c is no bound)
-    int least = 0;
+    uint32_t bits[N];
+    {
+      uint64_t at = rng_at(i0), step = RNG_STEP;
+      asm("" : "+s"(step));              // (else the sums become products)
+#pragma unroll
+      for (int j = 0; j < N; ++j) bits[j] = rng_bits(rowkey, at), at += step;
+    }
+    uint32_t most = bits[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j) most = max(most, bits[j]);
+    // bits below this lose whatever the logit (all may win at a temperature that
+    // is not positive, where c is no bound)
+    uint32_t least = 0;
     if (inv_temp > 0.f) {
       const float u = __expf(-__expf(__fmaf_rn(c, inv_temp, -wbest)));
-      least = (int)(u * (16777216.f * (1.f - 1e-5f))) - 2;
+      least = (uint32_t)max((int)(u * (16777216.f * (1.f - 1e-5f))) - 2, 0) << 8;
     }
-    uint32_t bits[N];
-    bool hit = false;
+    if (!__any(most >= least)) return;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      bits[j] = rng_bits(rowkey, i0, j);
-      hit |= (int)bits[j] >= least;
-    }
-    if (!__any(hit)) return;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      if ((int)bits[j] < least || (unsigned)(i0 + j) >= (unsigned)V ||
+      if (bits[j] < least || (unsigned)(i0 + j) >= (unsigned)V ||
           (tau != 0 && enc_f32(v[j]) < tau))
         continue;
       const float z = __fmaf_rn(v[j], inv_temp, gumbel(bits[j]));
       if (better(z, i0 + j, best, best_i)) best = z, best_i = i0 + j;
     }
-    float w = best;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      w = fmaxf(w, __shfl_xor(w, off, 64));
-    wbest = w;
+    wbest = wave_largest(best);
   }
 };
 
@@ -404,28 +451,21 @@ __global__ __launch_bounds__(SNT) void sample_plan_kernel(
 // MODE 0: sums and draw in one (no filter); 1: sums (and the largest logit)
 // of a filtered row; 2: its draw.
 //
-// One thread's part of a pass over the groups [first, first + SNT) of every
+// One thread's part of a pass over the groups [first, first + NT) of every
 // ``stride``.  Every lane of a wave takes part in every round (the draw votes).
-template <int MODE, typename T>
+// Rounds of whole words only run without a look at the row's ends, the next
+// word under way; the first, the last and the ones past them take the long form.
+template <int MODE, int NT, typename T>
 DEV_INLINE void walk(const VocabRow<T>& r, int first, int stride, bool greedy,
                      float inv_temp, uint64_t rowkey, uint32_t tau,
                      Sums<MODE == 1>& sums, Draw& d) {
   constexpr int VEC = VocabRow<T>::VEC;
   const int groups = r.groups();
-  for (int g0 = first; g0 < groups; g0 += stride) {
-    const int g = g0 + threadIdx.x;
-    float v[VEC];
-    if (g < groups) {
-      r.load(g, v);
-    } else {
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) v[j] = -INFINITY;
-    }
+  auto round = [&](const float (&v)[VEC], int i0) {
     float c = v[0];
 #pragma unroll
     for (int j = 1; j < VEC; ++j) c = fmaxf(c, v[j]);
     if (MODE != 2) sums.add(v, c, inv_temp);
-    const int i0 = r.first(g);
     if (MODE == 1 || greedy) {
       if (c > d.best) {
         d.best = c;
@@ -435,6 +475,34 @@ DEV_INLINE void walk(const VocabRow<T>& r, int first, int stride, bool greedy,
       }
     } else {
       d.add(v, c, i0, r.V, rowkey, inv_temp, tau);
+    }
+  };
+  // groups [1, whole) are whole words
+  const int whole = r.lead + (groups - 1) * VEC > r.V ? groups - 1 : groups;
+  auto inside = [&](int g0) { return g0 > 0 && g0 + NT <= whole; };
+  int g0 = first;
+  while (g0 < groups) {
+    if (inside(g0)) {
+      typename VocabRow<T>::Word next = r.word(g0 + threadIdx.x);
+      do {
+        const typename VocabRow<T>::Word w = next;
+        if (inside(g0 + stride)) next = r.word(g0 + stride + threadIdx.x);
+        float v[VEC];
+        r.numbers(w, v);
+        round(v, r.first(g0 + threadIdx.x));
+        g0 += stride;
+      } while (inside(g0));
+    } else {
+      const int g = g0 + threadIdx.x;
+      float v[VEC];
+      if (g < groups) {
+        r.load(g, v);
+      } else {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[j] = -INFINITY;
+      }
+      round(v, r.first(g));
+      g0 += stride;
     }
   }
 }
@@ -465,7 +533,7 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
 
   Sums<MODE == 1> sums;
   Draw d;
-  walk<MODE>(r, piece * SNT, split * SNT, greedy, inv_temp, rowkey, tau, sums,
+  walk<MODE, SNT>(r, piece * SNT, split * SNT, greedy, inv_temp, rowkey, tau, sums,
              d);
   if (MODE == 1) {                    // largest of each 16 lanes
     float t = d.best;
@@ -479,13 +547,15 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   if ((threadIdx.x & 63) == 0)
     part[threadIdx.x >> 6] = {sums.m, sums.s, sums.st, d.best, d.best_i, 0};
   __syncthreads();
+  if (threadIdx.x < 64) {               // the waves' shares, each once
+    const Share o = part[threadIdx.x % SNW];
+    const bool one = threadIdx.x < SNW;
+    sums.m = o.m, sums.s = one ? o.s : 0.f, sums.st = one ? o.st : 0.f;
+    if (MODE != 2) sums.wave(inv_temp);
+    d.best = o.best, d.best_i = o.best_i;
+    wave_best(d.best, d.best_i);
+  }
   if (threadIdx.x == 0) {
-    for (int w = 1; w < SNW; ++w) {
-      if (MODE != 2)
-        sums.merge(part[w].m, part[w].s, part[w].st, inv_temp);
-      if (better(part[w].best, part[w].best_i, d.best, d.best_i))
-        d.best = part[w].best, d.best_i = part[w].best_i;
-    }
     Share* out = share + row * split + piece;
     if (MODE != 2) out->m = sums.m, out->s = sums.s, out->st = sums.st;
     out->best = d.best;
@@ -593,7 +663,7 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
 
   Sums<FILTER> sums;
   Draw d;
-  walk<FILTER ? 1 : 0>(r, 0, NT, greedy, inv_temp, rowkey, 0u, sums, d);
+  walk<FILTER ? 1 : 0, NT>(r, 0, NT, greedy, inv_temp, rowkey, 0u, sums, d);
   if (FILTER) {                       // largest of each 16 lanes
     float t = d.best;
 #pragma unroll
@@ -606,12 +676,11 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
   __syncthreads();
   {                                   // of the whole row, in every thread
     const Share& o = part[lane % NW];
-    sums.m = o.m, sums.s = o.s, sums.st = o.st;
-    sums.template wave<NW>(inv_temp);
-    // (a lane's order of the sums shows in their last bit: all take lane 0's)
-    sums.s = first_lane(sums.s), sums.st = first_lane(sums.st);
+    sums.m = o.m;                       // (every wave's share once)
+    sums.s = lane < NW ? o.s : 0.f, sums.st = lane < NW ? o.st : 0.f;
+    sums.wave(inv_temp);
     d.best = o.best, d.best_i = o.best_i;
-    wave_best<NW>(d.best, d.best_i);
+    wave_best(d.best, d.best_i);
   }
   if constexpr (FILTER) {
     if (!greedy) {
@@ -646,13 +715,13 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
       }
       Draw pick;
       Sums<false> none;
-      walk<2>(r, 0, NT, false, inv_temp, rowkey, tau, none, pick);
+      walk<2, NT>(r, 0, NT, false, inv_temp, rowkey, tau, none, pick);
       wave_best(pick.best, pick.best_i);
       __syncthreads();                // the shares were read
       if (lane == 0) part[wid].best = pick.best, part[wid].best_i = pick.best_i;
       __syncthreads();
       d.best = part[lane % NW].best, d.best_i = part[lane % NW].best_i;
-      wave_best<NW>(d.best, d.best_i);
+      wave_best(d.best, d.best_i);
     }
   }
   if (threadIdx.x == 0) {
@@ -705,12 +774,12 @@ static void launch_sample(torch::Tensor& out_tokens,
     }
     return;
   }
-  // pieces of a row: 2048 blocks in all (eight per CU; 128 x 128256 takes 37
-  // us with 512 blocks, 33 with 1024, 32 with 2048, 36 with 4096), half of
-  // that for the short passes of filtered rows (64 x 151936: 63, 55, 60, 62
-  // us), none under two rounds of 256 words
+  // pieces of a row: 1024 blocks in all (four per CU; 128 x 128256 without a
+  // filter takes 29.8 us with 768 blocks, 28.7 with 1024, 29.4 with 2048; 64 x
+  // 151936 with both filters 63, 55, 60, 62 with 512, 1024, 2048, 4096), none
+  // under two rounds of 256 words
   const int split = (int)std::max<long>(
-      1, std::min<long>({64, ((no_filter ? 2048 : 1024) + N - 1) / N,
+      1, std::min<long>({64, (1024 + N - 1) / N,
                          words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
   const int hist_words = no_filter ? 0 : digits * 2 * DIGIT;

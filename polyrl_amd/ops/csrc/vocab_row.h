@@ -21,18 +21,22 @@ struct VocabRow {
   DEV_INLINE int groups() const { return 1 + (V - lead + VEC - 1) / VEC; }
   // index of a group's first entry (below 0 in a short first group)
   DEV_INLINE int first(int g) const { return lead + (g - 1) * VEC; }
+  typedef __attribute__((ext_vector_type(4))) uint32_t Word;
+  // a whole word's group, and its numbers
+  DEV_INLINE Word word(int g) const {
+    return *reinterpret_cast<const Word*>(x + first(g));
+  }
+  DEV_INLINE static void numbers(const Word& w, float (&v)[VEC]) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+      v[j] = __uint_as_float(sizeof(T) == 4 ? w[j % 4]
+                             : j % 2 ? w[j / 2] & 0xffff0000u
+                                     : w[j / 2] << 16);
+  }
   DEV_INLINE void load(int g, float (&v)[VEC]) const {
     const int i0 = first(g);
     if (i0 >= 0 && i0 + VEC <= V) {
-      if constexpr (sizeof(T) == 2) {
-        const bf16x8 w = *reinterpret_cast<const bf16x8*>(x + i0);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = bf2f(w.v[j]);
-      } else {
-        const f32x4v w = *reinterpret_cast<const f32x4v*>(x + i0);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = w.v[j];
-      }
+      numbers(word(g), v);
     } else {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
