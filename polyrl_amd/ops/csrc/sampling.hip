@@ -16,11 +16,15 @@
 //
 // Split.  A row is cut into ``split`` pieces, one block each, so that a few
 // rows fill the chip too (a block per row left half of it idle at 128 rows);
-// the pieces meet in small per-row arrays and a merging launch.  Without a
-// filter that is one pass: sums of the raw softmax and the draw together.
-// With one: sums, one pass per radix digit (11 bits, then the rest of a bf16
-// number's 16 or an fp32 number's 32), the draw over the kept set.  Short rows
-// take the same steps in one launch, a block each.
+// the pieces meet in small per-row arrays.  Without a filter that is one pass,
+// sums of the raw softmax and the draw together, and a merging launch.  With one:
+// sums; the candidates of both thresholds, from which, where they are few, the
+// row's last block has the token at once; else one pass per radix digit (11 bits,
+// then the rest of a bf16 number's 16 or an fp32 number's 32), whose last block
+// walks the bins, and the draw over the kept set, whose last block merges.  Short
+// rows take the same steps in one launch, a block each.  (64 x 151936, T 0.7, k
+// 50, p 0.9: 52.8 us with plans and a merge in launches of their own, eight in all,
+// 28 now; top-p 0.95 alone 81 and 79; at a temperature of 0 33 and 17.)
 //
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
@@ -297,12 +301,23 @@ struct alignas(8) Plan {              // where a row's two selections stand
   }
 };
 
+// Writes that blocks on other dies read in the same launch, and such reads: past
+// this die's L2
+template <typename U>
+DEV_INLINE void write_through(U* to, U v) {
+  __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+DEV_INLINE U read_through(const U* from) {
+  return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Walks the bins from the top until the running count reaches ``need`` (or
 // the running mass ``target``); bin 0 if none does.  All threads of the block
 // get the bin and the sum above it.  lds: the waves' sums, the first thread
 // that reaches the goal, its bin and the sum above that, each in words of its
 // own: a wave may still read the thread while that thread writes its bin.
-template <bool MASS, int NT = SNT>
+template <bool MASS, int NT = SNT, bool FAR = false>
 DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
                          float* lds, int& bin, float& before) {
   // thread t has bins [t*per, +per) counted from the top
@@ -313,8 +328,11 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
   for (int i = 0; i < MOST; ++i) {
     const int at = threadIdx.x * per + i;
     val[i] = 0.f;
-    if (i < per && at < n)
-      val[i] = MASS ? __uint_as_float(bins[n - 1 - at]) : (float)bins[n - 1 - at];
+    if (i < per && at < n) {
+      const uint32_t b =
+          FAR ? read_through(&bins[n - 1 - at]) : bins[n - 1 - at];
+      val[i] = MASS ? __uint_as_float(b) : (float)b;
+    }
   }
 #pragma unroll
   for (int i = 0; i < MOST; ++i) own += val[i];
@@ -405,46 +423,96 @@ DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
   return fmaxf(cut, kth);
 }
 
-// One block per row between the passes (in every block of the passes the same
-// work took longer than the passes): after the sums (``digit`` -1) the cut and
-// the goals, after a digit pass its bins.
-template <typename T>
-__global__ __launch_bounds__(SNT) void sample_plan_kernel(
-    Plan* __restrict__ plans, const uint32_t* __restrict__ hist,
-    int hist_words, const Share* __restrict__ share,
-    const float* __restrict__ tops, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ top_p, int digit,
-    int V, int split) {
-  __shared__ float lds[TOPS * 64];
-  const long row = blockIdx.x;
-  Plan& plan = plans[row];
-  const int k = top_k[row];
-  if (digit < 0) {
-    const float temp = temperature[row], p = top_p[row];
-    const bool by_k = temp != 0.f && k > 0 && k < V;
-    const bool by_p = temp != 0.f && p < 1.0f;
-    const float inv_temp = temp == 0.f ? 1.f : 1.0f / temp;
-    const Sums<true> all = row_sums<true>(share + row * split, split, inv_temp);
-    const float cut = cut_of(tops + row * split * TOPS, split * TOPS, by_k, by_p,
-                             k, p, inv_temp, all, V, lds);
-    if (threadIdx.x == 0) plan = Plan(cut, all, p, by_k, by_p);
-    return;
+// The same from a wave of a block of the passes: the k-th largest maximum is
+// found bit by bit, the lanes counting those that are no smaller.
+template <int J>
+DEV_INLINE uint32_t kth_largest(const float* tops, int m, int width, int k) {
+  const int lane = threadIdx.x & 63;
+  uint32_t e[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    e[j] = 0;
+    const int i = j * 64 + lane;
+    if (i < m) {
+      float t = tops[i * width];
+      for (int w = 1; w < width; ++w) t = fmaxf(t, tops[i * width + w]);
+      e[j] = enc_f32(t);
+    }
   }
-  const Plan now = plan;
-  const uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
+  uint32_t found = 0;
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t at = found | 1u << bit;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) n += __popcll(__ballot(e[j] >= at));
+    if (n >= k) found = at;
+  }
+  return found;
+}
+DEV_INLINE float wave_cut(const float* tops, int n, bool by_k, bool by_p, int k,
+                          float p, float inv_temp, const Sums<true>& all,
+                          int V) {
+  float cut = -INFINITY;
+  if (by_p && inv_temp > 0.f && p > 0.f)
+    cut = all.m + __logf(0.99f * (1.f - p) * all.st / V) / inv_temp;
+  if (!(cut > -INFINITY)) cut = -INFINITY;   // (NaN logits)
+  if (!by_k || k > n) return cut;
+  const int width = k <= n / 4 ? 4 : 1, m = n / width;
+  const uint32_t e = m <= 64 ? kth_largest<1>(tops, m, width, k)
+                   : m <= 256 ? kth_largest<4>(tops, m, width, k)
+                              : kth_largest<16>(tops, m, width, k);
+  return fmaxf(cut, __uint_as_float(e >> 31 ? e ^ 0x80000000u : ~e));
+}
+
+// What the passes over a filtered row tell each other, zeros at first: the
+// entries at or above the cut so far, the blocks that are through with each
+// pass, and whether the row's token is written.
+struct RowState {
+  uint32_t listed, arrived[4], done, pad[2];
+};
+constexpr int LISTED = 1024;          // entries that a row's list holds
+
+// Whether this block is the last of its row's to come here: what the others added
+// with atomics or wrote through can then be read through.  Nobody waits for
+// another block.  (Such writes have arrived when their wave's counter says so.
+// Fences would write back and drop this die's whole L2, under the blocks that
+// still read logits: 87 us for 12.)
+DEV_INLINE bool last_of_row(uint32_t* arrived, int split) {
+  __shared__ bool last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = atomicAdd(arrived, 1u) == (uint32_t)split - 1;
+  __syncthreads();
+  asm volatile("" ::: "memory");
+  return last;
+}
+
+// A digit's bins decide (all threads of a block)
+template <typename T>
+DEV_INLINE void walk_bins(Plan& plan, const uint32_t* h, int digit, int k,
+                          float* lds) {
   const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
   int bin;
   float before;
-  if (now.by & 1) {
-    find_bin<false>(h, bins, now.cnt, (float)k, lds, bin, before);
-    if (threadIdx.x == 0)
-      plan.prefix_k = now.prefix_k | (uint32_t)bin << low, plan.cnt = before;
+  if (plan.by & 1) {
+    find_bin<false, SNT, true>(h, bins, plan.cnt, (float)k, lds, bin, before);
+    plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
   }
-  if (now.by & 2) {
-    find_bin<true>(h + DIGIT, bins, now.mass, now.target, lds, bin, before);
-    if (threadIdx.x == 0)
-      plan.prefix_p = now.prefix_p | (uint32_t)bin << low, plan.mass = before;
+  if (plan.by & 2) {
+    find_bin<true, SNT, true>(h + DIGIT, bins, plan.mass, plan.target, lds, bin, before);
+    plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
   }
+}
+
+// the block's best entry, in the first wave
+DEV_INLINE void block_best(float& best, int& best_i, Share* part) {
+  wave_best(best, best_i);
+  if ((threadIdx.x & 63) == 0)
+    part[threadIdx.x >> 6].best = best, part[threadIdx.x >> 6].best_i = best_i;
+  __syncthreads();
+  best = part[threadIdx.x % SNW].best, best_i = part[threadIdx.x % SNW].best_i;
+  wave_best(best, best_i);
 }
 
 // ------------------------------------------------------------- one pass
@@ -507,8 +575,30 @@ DEV_INLINE void walk(const VocabRow<T>& r, int first, int stride, bool greedy,
   }
 }
 
+DEV_INLINE RowState* row_state(uint32_t* hist, int hist_words, long row) {
+  return reinterpret_cast<RowState*>(hist + (row + 1) * hist_words) - 1;
+}
+
+// the row's token from the pieces' shares (the first wave)
+template <typename T>
+DEV_INLINE void write_row(int64_t* out_tokens, float* out_logprobs,
+                          const Share* share, const VocabRow<T>& r, long row,
+                          int split) {
+  const int lane = threadIdx.x;
+  if (lane >= 64) return;
+  const Sums<false> a = row_sums<false>(share, split, 1.f);
+  float best = lane < split ? read_through(&share[lane].best) : -INFINITY;
+  int best_i = lane < split ? read_through(&share[lane].best_i) : 0x7fffffff;
+  wave_best(best, best_i);
+  if (lane == 0) {
+    out_tokens[row] = best_i;
+    out_logprobs[row] = (float)r.x[best_i] - (a.m + __logf(a.s));
+  }
+}
+
 template <typename T, int MODE>
 __global__ __launch_bounds__(SNT) void sample_pass_kernel(
+    int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
     Share* __restrict__ share, float* __restrict__ tops,
     uint32_t* __restrict__ hist, int hist_words,
     const Plan* __restrict__ plans, const T* __restrict__ logits,
@@ -521,11 +611,12 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   const VocabRow<T> r(logits + row * V, V);
   const float temp = temperature[row];
   const bool greedy = temp == 0.f;
-  if (MODE == 2 && greedy) return;    // the first pass found it
+  RowState* state = row_state(hist, hist_words, row);
+  if (MODE == 2 && state->done) return;
   const float inv_temp = greedy ? 1.f : 1.0f / temp;
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
   const uint32_t tau = MODE == 2 ? plans[row].threshold() : 0;
-  if (MODE == 1) {                    // the digit passes' bins start at 0
+  if (MODE == 1) {                    // the bins and the state start at 0
     uint32_t* h = hist + row * hist_words;
     for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
       h[i] = 0;
@@ -558,9 +649,11 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   if (threadIdx.x == 0) {
     Share* out = share + row * split + piece;
     if (MODE != 2) out->m = sums.m, out->s = sums.s, out->st = sums.st;
-    out->best = d.best;
-    out->best_i = d.best_i;
+    write_through(&out->best, d.best);
+    write_through(&out->best_i, d.best_i);
   }
+  if (MODE == 2 && last_of_row(&state->arrived[3], split))
+    write_row(out_tokens, out_logprobs, share + row * split, r, row, split);
 }
 
 template <typename T>
@@ -569,17 +662,8 @@ __global__ __launch_bounds__(64) void sample_merge_kernel(
     const Share* __restrict__ share, const T* __restrict__ logits, int V,
     int split) {
   const long row = blockIdx.x;
-  const int lane = threadIdx.x;
-  share += row * split;
-  const Sums<false> a = row_sums<false>(share, split, 1.f);
-  float best = lane < split ? share[lane].best : -INFINITY;
-  int best_i = lane < split ? share[lane].best_i : 0x7fffffff;
-  wave_best(best, best_i);
-  if (lane == 0) {
-    out_tokens[row] = best_i;
-    out_logprobs[row] =
-        (float)logits[row * V + best_i] - (a.m + __logf(a.s));
-  }
+  write_row(out_tokens, out_logprobs, share + row * split,
+            VocabRow<T>(logits + row * V, V), row, split);
 }
 
 // a thread's entries of the groups [first, ..) of every ``stride`` into the
@@ -610,32 +694,218 @@ DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(SNT) void sample_digit_kernel(
-    uint32_t* __restrict__ hist, int hist_words,
-    const Plan* __restrict__ plans, const T* __restrict__ logits,
-    const float* __restrict__ temperature, int digit, int V, int split) {
-  __shared__ uint32_t cnt[DIGIT];
-  __shared__ float mass[DIGIT];
-  const long row = blockIdx.x / split;
-  const int piece = blockIdx.x % split;
-  const Plan plan = plans[row];
-  if (plan.by == 0) return;
-  const float inv_temp = 1.0f / temperature[row];
-  uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
+// both selections of a row by one block
+template <int NT, typename T>
+DEV_INLINE void select_alone(const VocabRow<T>& r, Plan& plan, int k,
+                             float inv_temp, uint32_t* cnt, float* mass,
+                             float* lds) {
+  for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
+    const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+    for (int i = threadIdx.x; i < bins; i += NT) cnt[i] = 0, mass[i] = 0.f;
+    __syncthreads();
+    fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
+    __syncthreads();
+    int bin;
+    float before;
+    if (plan.by & 1) {
+      find_bin<false, NT>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
+      plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
+    }
+    if (plan.by & 2) {
+      find_bin<true, NT>(reinterpret_cast<const uint32_t*>(mass), bins,
+                         plan.mass, plan.target, lds, bin, before);
+      plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
+    }
+    __syncthreads();                    // the bins were read
+  }
+}
 
+// a piece's entries into the row's bins of a digit
+template <typename T>
+DEV_INLINE void add_bins(const VocabRow<T>& r, int piece, int split, int digit,
+                         const Plan& plan, float inv_temp, uint32_t* cnt,
+                         float* mass, uint32_t* h) {
   const int bins = digit_bins<T>(digit);
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
   __syncthreads();
-  const VocabRow<T> r(logits + row * V, V);
   fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
   __syncthreads();
-  uint32_t* hc = h;
   float* hm = reinterpret_cast<float*>(h + DIGIT);
   for (int i = threadIdx.x; i < bins; i += SNT) {
-    if (cnt[i]) atomicAdd(&hc[i], cnt[i]);
+    if (cnt[i]) atomicAdd(&h[i], cnt[i]);
     if (mass[i] != 0.f) atomicAdd(&hm[i], mass[i]);
   }
+}
+
+// The cut, and what stands at or above it: into a list if that is little, into the
+// first digit's bins else.  The row's last block then has the thresholds and the
+// token from the list (by counting, for each entry, what is no smaller), or the
+// first digit of the thresholds.  Every block finds the same cut: a launch for it
+// between the passes takes longer.
+//
+// How much it is, the maxima of the lanes' groups tell: of g groups, n entries in
+// random order leave a share of exp(-n / g) without one.  If they are not in random
+// order and the list is too short, the last block takes the steps of a short row.
+template <typename T>
+__global__ __launch_bounds__(SNT) void sample_select_kernel(
+    int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
+    Plan* __restrict__ plans, uint32_t* __restrict__ hist, int hist_words,
+    float* __restrict__ list_v, int* __restrict__ list_i,
+    const Share* __restrict__ share, const float* __restrict__ tops,
+    const T* __restrict__ logits, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p,
+    uint64_t seed, int V, int split) {
+  constexpr int VEC = VocabRow<T>::VEC;
+  __shared__ alignas(16) uint32_t cnt[DIGIT];
+  __shared__ alignas(16) float mass[DIGIT];
+  __shared__ float lds[SNW + 4];
+  __shared__ Share part[SNW];
+  __shared__ int found;
+  __shared__ uint32_t base, thr[2];
+  const long row = blockIdx.x / split;
+  const int piece = blockIdx.x % split;
+  const VocabRow<T> r(logits + row * V, V);
+  const int k = top_k[row];
+  const float temp = temperature[row], p = top_p[row];
+  const bool by_k = temp != 0.f && k > 0 && k < V;
+  const bool by_p = temp != 0.f && p < 1.0f;
+  const float inv_temp = temp == 0.f ? 1.f : 1.0f / temp;
+  uint32_t* h = hist + row * hist_words;
+  RowState* state = row_state(hist, hist_words, row);
+  share += row * split;
+  list_v += row * LISTED, list_i += row * LISTED;
+  const Sums<true> all = row_sums<true>(share, split, inv_temp);
+  if (!by_k && !by_p) {
+    if (piece != 0) return;
+    if (threadIdx.x == 0) plans[row] = Plan(-INFINITY, all, p, false, false);
+    if (temp == 0.f) {                  // the first pass found it
+      write_row(out_tokens, out_logprobs, share, r, row, split);
+      if (threadIdx.x == 0) state->done = 1;
+    }
+    return;
+  }
+  const float cut = wave_cut(tops + row * split * TOPS, split * TOPS, by_k,
+                             by_p, k, p, inv_temp, all, V);
+  Plan plan(cut, all, p, by_k, by_p);
+  // (a list needs numbers that add up)
+  bool listing = cut > -INFINITY && inv_temp > 0.f &&
+                 fabsf(all.m) < INFINITY && all.st < INFINITY;
+  if (listing) {
+    const int g = split * TOPS, lane = threadIdx.x & 63;
+    int with = 0;
+    for (int i = lane; i - lane < g; i += 64)
+      with += __popcll(__ballot(i < g && tops[row * g + i] >= cut));
+    listing = with <= g * (1.f - __expf(-0.7f * LISTED / g));
+  }
+  if (listing) {
+    int* own_i = reinterpret_cast<int*>(cnt);
+    float* own_v = mass;
+    if (threadIdx.x == 0) found = 0;
+    __syncthreads();
+    const int groups = r.groups();
+    for (int g = piece * SNT + threadIdx.x; g < groups; g += split * SNT) {
+      if (*(volatile int*)&found > LISTED) break;
+      float v[VEC];
+      r.load(g, v);
+      float c = v[0];
+#pragma unroll
+      for (int j = 1; j < VEC; ++j) c = fmaxf(c, v[j]);
+      if (c < cut) continue;
+      const int i0 = r.first(g);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        if (v[j] >= cut) {              // (-inf stands outside the row)
+          const int at = atomicAdd(&found, 1);
+          if (at < LISTED) own_v[at] = v[j], own_i[at] = i0 + j;
+        }
+    }
+    __syncthreads();
+    const int n = min(found, LISTED + 1);
+    if (threadIdx.x == 0) base = n ? atomicAdd(&state->listed, (uint32_t)n) : 0;
+    __syncthreads();
+    for (int t = threadIdx.x; t < n && base + t < LISTED; t += SNT) {
+      write_through(&list_v[base + t], own_v[t]);
+      write_through(&list_i[base + t], own_i[t]);
+    }
+  } else {
+    add_bins(r, piece, split, 0, plan, inv_temp, cnt, mass, h);
+  }
+  if (!last_of_row(&state->arrived[0], split)) return;
+
+  if (!listing) {
+    walk_bins<T>(plan, h, 0, k, lds);
+    if (threadIdx.x == 0) plans[row] = plan;
+    return;
+  }
+  const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
+  const int listed = min(read_through(&state->listed), LISTED + 1u);
+  Draw d;
+  if (listed > LISTED) {
+    select_alone<SNT>(r, plan, k, inv_temp, cnt, mass, lds);
+    Sums<false> none;
+    walk<2, SNT>(r, 0, SNT, false, inv_temp, rowkey, plan.threshold(), none, d);
+  } else {
+    // (four at a time; what fills up is no larger than any and weighs nothing)
+    for (int t = threadIdx.x; t < (listed + 3) / 4 * 4; t += SNT) {
+      const float v = t < listed ? read_through(&list_v[t]) : 0.f;
+      cnt[t] = t < listed ? enc_f32(v) : 0u;
+      mass[t] = t < listed ? __expf((v - all.m) * inv_temp) : 0.f;
+    }
+    if (threadIdx.x == 0) thr[0] = thr[1] = 0;
+    __syncthreads();
+    for (int t = threadIdx.x; t < listed; t += SNT) {
+      const uint32_t e = cnt[t];
+      int count = 0;
+      float sum = 0.f;
+      for (int j = 0; j < listed; j += 4) {
+        const uint4 ej = *reinterpret_cast<const uint4*>(&cnt[j]);
+        const float4 wj = *reinterpret_cast<const float4*>(&mass[j]);
+        count += (ej.x >= e) + (ej.y >= e) + (ej.z >= e) + (ej.w >= e);
+        sum += (ej.x >= e ? wj.x : 0.f) + (ej.y >= e ? wj.y : 0.f) +
+               (ej.z >= e ? wj.z : 0.f) + (ej.w >= e ? wj.w : 0.f);
+      }
+      if (by_k && count >= k) atomicMax(&thr[0], e);
+      if (by_p && sum >= plan.target) atomicMax(&thr[1], e);
+    }
+    __syncthreads();
+    plan.prefix_k = thr[0], plan.prefix_p = thr[1];
+    const uint32_t tau = plan.threshold();
+    for (int t = threadIdx.x; t < listed; t += SNT) {
+      if (cnt[t] < tau) continue;
+      const int i = read_through(&list_i[t]);
+      const float z = __fmaf_rn(read_through(&list_v[t]), inv_temp,
+                                gumbel(rng_bits(rowkey, rng_at(i))));
+      if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
+    }
+  }
+  block_best(d.best, d.best_i, part);
+  if (threadIdx.x == 0) {
+    out_tokens[row] = d.best_i;
+    out_logprobs[row] = (float)r.x[d.best_i] - (all.m + __logf(all.s));
+    state->done = 1;
+  }
+}
+
+// the digits after the first, of rows without a list
+template <typename T>
+__global__ __launch_bounds__(SNT) void sample_digit_kernel(
+    Plan* __restrict__ plans, uint32_t* __restrict__ hist, int hist_words,
+    const T* __restrict__ logits, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, int digit, int V, int split) {
+  __shared__ uint32_t cnt[DIGIT];
+  __shared__ float mass[DIGIT];
+  __shared__ float lds[SNW + 4];
+  const long row = blockIdx.x / split;
+  RowState* state = row_state(hist, hist_words, row);
+  if (state->done) return;
+  Plan plan = plans[row];
+  if (plan.by == 0) return;
+  uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
+  add_bins(VocabRow<T>(logits + row * V, V), blockIdx.x % split, split, digit,
+           plan, 1.0f / temperature[row], cnt, mass, h);
+  if (!last_of_row(&state->arrived[digit], split)) return;
+  walk_bins<T>(plan, h, digit, top_k[row], lds);
+  if (threadIdx.x == 0) plans[row] = plan;
 }
 
 // ------------------------------------------------------------- short rows
@@ -691,26 +961,7 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
       if (by_k || by_p) {
         Plan plan(cut_of<NT>(tops, NTOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
                   sums, p, by_k, by_p);
-        for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
-          const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
-          for (int i = threadIdx.x; i < bins; i += NT)
-            cnt[i] = 0, mass[i] = 0.f;
-          __syncthreads();
-          fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
-          __syncthreads();
-          int bin;
-          float before;
-          if (by_k) {
-            find_bin<false, NT>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
-            plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
-          }
-          if (by_p) {
-            find_bin<true, NT>(reinterpret_cast<const uint32_t*>(mass), bins,
-                           plan.mass, plan.target, lds, bin, before);
-            plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
-          }
-          __syncthreads();            // the bins were read
-        }
+        select_alone<NT>(r, plan, k, inv_temp, cnt, mass, lds);
         tau = plan.threshold();
       }
       Draw pick;
@@ -742,17 +993,17 @@ static void launch_sample(torch::Tensor& out_tokens,
   const int V = logits.size(1);
   if (N == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  // Rows in one launch, a block each, while that is no longer than the pieces
-  // and their plans.  Without a filter: with few rows up to 16384 numbers (64 x
-  // 16000 bf16 12.1 us, in pieces 12.6; 64 x 32000 18.3 and 13.6), with a block
-  // for most CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768
-  // (64 x 9000 33 and 50, 64 x 32000 42 and 51; at a temperature of 0, where
-  // nothing is selected, 7.4 and 33, 9.2 and 33; one row of 50257 with top-p 55
-  // and 39).  What stays dearer than a block a row everywhere is the draw at a
-  // temperature of 0 without a filter from 16384 numbers on, 11.3 us for 8 to
-  // 10: the temperature is on the device, and at 1 the pieces take 13.5 for 21.
+  // Rows in one launch, a block each, while that is no longer than the pieces and
+  // their passes.  Without a filter: with few rows up to 16384 numbers (64 x 16000
+  // bf16 12.1 us, in pieces 12.6; 64 x 32000 18.3 and 13.6), with a block for most
+  // CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768 (64 x 9000 31
+  // us, in pieces 70, 64 x 16000 33 and 53; 64 x 32000 37 and 26, but at a
+  // temperature of 0, where nothing is selected, 7.8 and 19).  What stays dearer
+  // than a block a row everywhere is the draw at a temperature of 0 without a
+  // filter from 16384 numbers on, 11.3 us for 8 to 10: the temperature is on the
+  // device, and at 1 the pieces take 11.5 for 21.
   // A block of 1024 threads takes rows of more than one round of 256 words (64 x
-  // 9000 both filters 33 us, with 256 threads 37; 64 x 32000 42 and 72); where
+  // 9000 both filters 31 us, with 256 threads 37; 64 x 32000 37 and 72); where
   // there are more rows than CUs, 256 threads take them up to ten rounds (512 x
   // 9000 41 us, with 1024 threads 64).
   auto rows = [&](auto kern, int threads) {
@@ -782,48 +1033,50 @@ static void launch_sample(torch::Tensor& out_tokens,
       1, std::min<long>({64, (1024 + N - 1) / N,
                          words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
-  const int hist_words = no_filter ? 0 : digits * 2 * DIGIT;
-  // per row: the pieces' shares and maxima, the plan, the bins.  From the
-  // caching allocator: a block per call and stream, also while a graph is captured
+  const int hist_words =
+      no_filter ? 0 : digits * 2 * DIGIT + (int)sizeof(RowState) / 4;
+  // per row: the pieces' shares and maxima, the plan, the bins and the state, the
+  // list.  From the caching allocator: a block per call and stream, also while a
+  // graph is captured
   const long share_words = (long)split * (sizeof(Share) / 4);
   const long row_words =
       no_filter ? share_words
-                : share_words + split * TOPS + sizeof(Plan) / 4 + hist_words;
+                : share_words + split * TOPS + sizeof(Plan) / 4 + hist_words +
+                      2 * LISTED;
   auto ws = torch::empty({N * row_words}, logits.options().dtype(torch::kInt32));
   int* w = ws.data_ptr<int>();
   Share* share = reinterpret_cast<Share*>(w);
   Plan* plans = reinterpret_cast<Plan*>(w + N * share_words);
   float* tops = reinterpret_cast<float*>(plans + N);
   uint32_t* hist = reinterpret_cast<uint32_t*>(tops + N * split * TOPS);
+  float* list_v = reinterpret_cast<float*>(hist + N * hist_words);
+  int* list_i = reinterpret_cast<int*>(list_v + N * LISTED);
+  int64_t* tokens = out_tokens.data_ptr<int64_t>();
+  float* logprobs = out_logprobs.data_ptr<float>();
   const T* x = (const T*)logits.data_ptr();
   const float* temp = temperature.data_ptr<float>();
   TORCH_CHECK(N * split < (1L << 31), "too many rows");
   const dim3 grid((unsigned)(N * split)), block(SNT);
   const int* k = top_k.data_ptr<int>();
-  const float* p = top_p.data_ptr<float>();
   auto pass = [&](auto kern) {
-    kern<<<grid, block, 0, stream>>>(share, tops, hist, hist_words, plans, x,
-                                     temp, seed, seed_ptr, V, split);
-  };
-  auto plan = [&](int digit) {
-    sample_plan_kernel<T><<<dim3((unsigned)N), block, 0, stream>>>(
-        plans, hist, hist_words, share, tops, temp, k, p, digit, V, split);
+    kern<<<grid, block, 0, stream>>>(tokens, logprobs, share, tops, hist,
+                                     hist_words, plans, x, temp, seed, seed_ptr,
+                                     V, split);
   };
   if (no_filter) {
     pass(sample_pass_kernel<T, 0>);
+    sample_merge_kernel<T><<<dim3(N), dim3(64), 0, stream>>>(
+        tokens, logprobs, share, x, V, split);
   } else {
     pass(sample_pass_kernel<T, 1>);
-    plan(-1);
-    for (int d = 0; d < digits; ++d) {
+    sample_select_kernel<T><<<grid, block, 0, stream>>>(
+        tokens, logprobs, plans, hist, hist_words, list_v, list_i, share, tops,
+        x, temp, k, top_p.data_ptr<float>(), seed, V, split);
+    for (int d = 1; d < digits; ++d)
       sample_digit_kernel<T><<<grid, block, 0, stream>>>(
-          hist, hist_words, plans, x, temp, d, V, split);
-      plan(d);
-    }
+          plans, hist, hist_words, x, temp, k, d, V, split);
     pass(sample_pass_kernel<T, 2>);
   }
-  sample_merge_kernel<T><<<dim3(N), dim3(64), 0, stream>>>(
-      out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(), share, x,
-      V, split);
   HIP_CHECK_KERNEL();
 }
 

@@ -337,3 +337,41 @@ def test_sample_one_launch(n, v, dtype, temp, k, p):
         z = row / temp + noise(seed, r, v)
         # (as above)
         assert z[t] >= z[sure].max() - 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,p", [(50, 1.0), (-1, 0.9), (50, 0.5), (900, 1.0),
+                                 (1500, 0.99)])
+@pytest.mark.parametrize("what", ["random", "cluster", "ties", "peak",
+                                  "about_full"])
+def test_sample_candidate_lists(what, k, p, dtype):
+    """Rows in pieces whose candidates are few (a list), many, more than a list
+    holds though the lanes' groups show few (neighbours), all alike, or about
+    as many as a list holds; an odd row length."""
+    torch.manual_seed(11)
+    n, v, temp, seed = 3, 70001, 0.8, 77
+    x = torch.randn(n, v, device=DEV)
+    if what == "cluster":
+        x[:, 5000:7000] = 8 + torch.rand(n, 2000, device=DEV)
+    elif what == "ties":
+        x[:] = 1.0
+    elif what == "peak":
+        x[:, 12345] = 40.0
+    elif what == "about_full":
+        for r in range(n):
+            at = torch.randperm(v, device=DEV)[:1010 + 14 * r]
+            x[r, at] = 9 + torch.rand(len(at), device=DEV)
+    x = x.to(dtype)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    tok, lp = ops.sample(x, full(temp, torch.float32), full(k, torch.int32),
+                         full(p, torch.float32), seed, no_filter=False)
+    want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+    assert (lp.double() - want).abs().max() <= 1e-5 * (1 + want.abs().max())
+    for r in range(n):
+        row = x[r].double().cpu()
+        sure, maybe = kept(row, temp, k, p)
+        t = int(tok[r])
+        assert maybe[t]
+        z = row / temp + noise(seed, r, v)
+        # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
+        assert z[t] >= z[sure].max() - 1e-3
