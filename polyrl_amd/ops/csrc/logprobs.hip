@@ -9,24 +9,32 @@
 // one exponential per number (a compare, a branch and two-byte loads per
 // number ran at 1.7 TB/s).  Rows that do not start at a 16-byte address are
 // read from the next one, their first numbers apart.  Measured, 4096 x 128256
-// bf16: 600 us before, 215 us now (4.9 TB/s); with the backward pass
-// (2.1 GB, 400 us) 995 -> 616 us.
+// bf16: log-probabilities and entropies 600 us with two-byte loads, 183 with
+// words, 162 (6.5 TB/s) past the caches; forward and backward 995, 615, 534: dx
+// through the caches drove out the rows that the backward had still to read, and
+// its blocks of 256 threads read ahead too little (1024: 546 for 551).
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
 #include "common.h"
 
-template <typename T>
+typedef __attribute__((ext_vector_type(4))) uint32_t Word16;
+
+// a 16-byte word, ONCE: of what will not be read again while a cache could hold it
+template <bool ONCE>
+DEV_INLINE Word16 load16(const void* p) {
+  const Word16* w = reinterpret_cast<const Word16*>(p);
+  return ONCE ? __builtin_nontemporal_load(w) : *w;
+}
+
+template <bool ONCE, typename T>
 DEV_INLINE void unpack16(const T* p, float (&v)[16 / sizeof(T)]) {
-  if constexpr (sizeof(T) == 2) {
-    const bf16x8 w = *reinterpret_cast<const bf16x8*>(p);
+  const Word16 w = load16<ONCE>(p);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = bf2f(w.v[j]);
-  } else {
-    const f32x4v w = *reinterpret_cast<const f32x4v*>(p);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = w.v[j];
-  }
+  for (int j = 0; j < (int)(16 / sizeof(T)); ++j)
+    v[j] = __uint_as_float(sizeof(T) == 4 ? w[j % 4]
+                           : j % 2 ? w[j / 2] & 0xffff0000u
+                                   : w[j / 2] << 16);
 }
 
 // numbers before a row's first 16-byte address
@@ -73,7 +81,7 @@ template <typename T, bool ENT, int NT>
 __global__ __launch_bounds__(NT) void gather_logprobs_kernel(
     float* __restrict__ out_lp, float* __restrict__ out_lse,
     float* __restrict__ out_ent, const T* __restrict__ logits,
-    const int64_t* __restrict__ labels, int V) {
+    const int64_t* __restrict__ labels, int V, long kept) {
   constexpr int VEC = 16 / sizeof(T), UN = 4, NW = NT / 64;
   __shared__ float red[NW];
   const long row = gridDim.x - 1 - (long)blockIdx.x;
@@ -82,20 +90,25 @@ __global__ __launch_bounds__(NT) void gather_logprobs_kernel(
   const T* xv = x + lead;
   const int nvec = (V - lead) / VEC;
   Online<ENT> a;
-  int i = threadIdx.x;
-  for (; i + (UN - 1) * NT < nvec; i += UN * NT) {
-    float v[UN][VEC];
+  auto words = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    int i = threadIdx.x;
+    for (; i + (UN - 1) * NT < nvec; i += UN * NT) {
+      float v[UN][VEC];
 #pragma unroll
-    for (int u = 0; u < UN; ++u)
-      unpack16(xv + (long)(i + u * NT) * VEC, v[u]);
+      for (int u = 0; u < UN; ++u)
+        unpack16<ONCE>(xv + (long)(i + u * NT) * VEC, v[u]);
 #pragma unroll
-    for (int u = 0; u < UN; ++u) a.add(v[u]);
-  }
-  for (; i < nvec; i += NT) {
-    float v[VEC];
-    unpack16(xv + (long)i * VEC, v);
-    a.add(v);
-  }
+      for (int u = 0; u < UN; ++u) a.add(v[u]);
+    }
+    for (; i < nvec; i += NT) {
+      float v[VEC];
+      unpack16<ONCE>(xv + (long)i * VEC, v);
+      a.add(v);
+    }
+  };
+  if (row >= kept) words(std::true_type());
+  else words(std::false_type());
   // the numbers before the first and behind the last whole word
   const int rest = V - lead - nvec * VEC;
   if ((int)threadIdx.x < lead + rest) {
@@ -135,8 +148,11 @@ __global__ __launch_bounds__(NT) void gather_logprobs_kernel(
 
 // ---------------------------------------------------- training backward
 // d lp / d logits = onehot(label) - softmax(logits); chain with dlp.
-// One streaming pass per row using the forward-saved logsumexp.
-__global__ void gather_logprobs_bwd_kernel(
+// One streaming pass per row using the forward-saved logsumexp.  dx goes past the
+// caches, which keep the rows that the forward read last for as long as they are
+// needed; the logits too, where they are more than fits (ONCE).
+template <bool ONCE>
+__global__ __launch_bounds__(1024) void gather_logprobs_bwd_kernel(
     bf16_t* __restrict__ dlogits,
     const bf16_t* __restrict__ logits,
     const int64_t* __restrict__ labels,
@@ -156,17 +172,19 @@ __global__ void gather_logprobs_bwd_kernel(
   const bool same = (((uintptr_t)(x + lead)) & 15) == 0;
   for (int i = threadIdx.x; i < n8; i += blockDim.x) {
     const bf16_t* at = x + lead + (long)i * 8;
-    bf16x8 v, o;
+    float v[8];
     if (same) {
-      v = *reinterpret_cast<const bf16x8*>(at);
+      unpack16<ONCE>(at, v);
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v.v[j] = at[j];
+      for (int j = 0; j < 8; ++j) v[j] = bf2f(at[j]);
     }
+    bf16x8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      o.v[j] = f2bf(-g * __expf(bf2f(v.v[j]) - l));
-    *reinterpret_cast<bf16x8*>(dx + lead + (long)i * 8) = o;
+    for (int j = 0; j < 8; ++j) o.v[j] = f2bf(-g * __expf(v[j] - l));
+    __builtin_nontemporal_store(
+        __builtin_bit_cast(Word16, o),
+        reinterpret_cast<Word16*>(dx + lead + (long)i * 8));
   }
   // the numbers before the first and behind the last whole word
   const int rest = V - lead - n8 * 8;
@@ -184,7 +202,7 @@ __global__ void gather_logprobs_bwd_kernel(
 template <typename T, bool ENT>
 static void launch_gather(float* lp, float* lse, float* ent,
                           const torch::Tensor& logits,
-                          const torch::Tensor& labels) {
+                          const torch::Tensor& labels, long kept) {
   const long N = logits.size(0);
   if (N == 0) return;
   const int V = logits.size(1);
@@ -195,11 +213,20 @@ static void launch_gather(float* lp, float* lse, float* ent,
   // times the threads
   if (N >= 1024)
     gather_logprobs_kernel<T, ENT, 256>
-        <<<dim3(N), dim3(256), 0, stream>>>(lp, lse, ent, x, lab, V);
+        <<<dim3(N), dim3(256), 0, stream>>>(lp, lse, ent, x, lab, V, kept);
   else
     gather_logprobs_kernel<T, ENT, 1024>
-        <<<dim3(N), dim3(1024), 0, stream>>>(lp, lse, ent, x, lab, V);
+        <<<dim3(N), dim3(1024), 0, stream>>>(lp, lse, ent, x, lab, V, kept);
   HIP_CHECK_KERNEL();
+}
+
+// Rows of logits that the 256 MB cache behind the L2s holds.  The rows that the
+// forward reads last stay there for the backward; the others, and where no
+// backward follows all, are read past the caches.  Measured, 4096 x 128256 forward
+// and backward: with 160 MB kept 542 us, 200 535, 240 534, 300 529, none 554.
+static long cached_rows(const torch::Tensor& logits) {
+  return (256L << 20) /
+         std::max<long>(1, logits.size(1) * (long)logits.element_size());
 }
 
 // training fwd: lp + logsumexp (for the hand-written backward)
@@ -211,7 +238,7 @@ void gather_logprobs_train_fwd(torch::Tensor out_lp, torch::Tensor out_lse,
   TORCH_CHECK(labels.dtype() == torch::kInt64);
   launch_gather<bf16_t, false>(out_lp.data_ptr<float>(),
                                out_lse.data_ptr<float>(), nullptr, logits,
-                               labels);
+                               labels, cached_rows(logits));
 }
 
 torch::Tensor gather_logprobs_train_bwd(torch::Tensor logits,
@@ -224,7 +251,10 @@ torch::Tensor gather_logprobs_train_bwd(torch::Tensor logits,
   const int V = logits.size(1);
   auto dlogits = torch::empty_like(logits);
   auto stream = at::hip::getCurrentHIPStream();
-  gather_logprobs_bwd_kernel<<<dim3(N), dim3(256), 0, stream>>>(
+  if (N == 0) return dlogits;
+  auto kern = N > cached_rows(logits) ? gather_logprobs_bwd_kernel<true>
+                                      : gather_logprobs_bwd_kernel<false>;
+  kern<<<dim3(N), dim3(1024), 0, stream>>>(
       (bf16_t*)dlogits.data_ptr(), (const bf16_t*)logits.data_ptr(),
       labels.data_ptr<int64_t>(), lse.data_ptr<float>(),
       dlp.contiguous().data_ptr<float>(), V);
@@ -242,10 +272,10 @@ void gather_logprobs(torch::Tensor out_lp, torch::Tensor out_ent,
   float* ent = want_entropy ? out_ent.data_ptr<float>() : nullptr;
   if (logits.dtype() == torch::kBFloat16) {
     (want_entropy ? launch_gather<bf16_t, true> : launch_gather<bf16_t, false>)(
-        lp, nullptr, ent, logits, labels);
+        lp, nullptr, ent, logits, labels, 0);
   } else if (logits.dtype() == torch::kFloat32) {
     (want_entropy ? launch_gather<float, true> : launch_gather<float, false>)(
-        lp, nullptr, ent, logits, labels);
+        lp, nullptr, ent, logits, labels, 0);
   } else {
     TORCH_CHECK(false, "gather_logprobs: dtype must be bf16 or fp32");
   }
