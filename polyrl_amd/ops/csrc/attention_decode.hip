@@ -17,8 +17,8 @@
 // What bounds it: reading K and V once.  (With per-key dot products, shuffles
 // and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
 // at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
-// tokens, 32/8 heads of 128, 59.5 -> 45.2 us; 33 rows of 1900 .. 8192, 28/4
-// heads, 264 -> 86.5 us (4.1 TB/s).  (With two parts a weight 44.6 and 86.0.)
+// tokens, 32/8 heads of 128, 59.5 -> 45.2 us, 37.6 with V read past the caches
+// (5.6 TB/s); 33 rows of 1900 .. 8192, 28/4 heads, 264 -> 86.5 -> 82 us.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -41,7 +41,8 @@ DEV_INLINE float quad_sum(float x) {
   return half_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
 }
 
-template <int D, int WAVES>                // WAVES: of a SIMD, at least
+// WAVES: of a SIMD, at least; ONCE: values are read past the caches
+template <int D, int WAVES, bool ONCE>
 __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
     bf16_t* __restrict__ out,              // (B, Hq, D)
     float* __restrict__ partial,           // (B, Hq, S, D+2) when nsplit>1
@@ -121,10 +122,12 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
         kf[n][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
     }
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      vv[i] = *reinterpret_cast<const i32x4_t*>(
+    for (int i = 0; i < NV; ++i) {
+      const i32x4_t* vp = reinterpret_cast<const i32x4_t*>(
           v_cache + __shfl(slot, i * RPI + vrow, 64) * kv_stride + hk * D +
           vcol * 8);
+      vv[i] = ONCE ? __builtin_nontemporal_load(vp) : *vp;
+    }
     if (t0 + 4 * DEC_KEYS < cend) slot = slot_of(t0 + 4 * DEC_KEYS);
 
     // ---- S^T: 32 keys x 16 heads; this lane: head l15, keys 4 lhi + r -------
@@ -452,6 +455,13 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // of 64: 300 rows of 16, 40 keys 12.8 and 15.0, 300 keys 75.7 and 72.4, 128
   // rows 1000 keys 97.7 and 103), and where the page table holds short contexts
   // only (128 wide, 4 heads, 128 rows of 300 keys: 18.2 and 20.0).
+  // Values go past the caches where the rows may hold more than the 256 MB cache
+  // behind the L2s does, as the layers of a model do in turn: V, read once in whole
+  // rows, then leaves the cache's ways to K, whose lines two instructions read
+  // (128 rows of 257 .. 512, 32/8 heads of 128, 268 MB: 44.9 us and 37.6, K past
+  // the caches too 45.9; 256 rows of 700 .. 1000, 64/8 heads, 170 and 158; but two
+  // calls in turn on 64 rows of 500 .. 1000, 32/8 heads of 64, 132 MB: 22.5 and 24.5).
+  const bool once = B * most * Hk * D * 4 > (128L << 20);
   // Groups of two and three heads of 128 keep three blocks on a CU, which short
   // contexts need (300 rows of 16 groups of two, 5 keys: 28 us with two, 19.7
   // with three); at larger groups the registers that this takes cost more (32
@@ -459,9 +469,11 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   if (G == 1 && (base_blocks >= 2048 || most <= (D == 128 ? 512 : 64)))
     args(paged_decode_attn_one_kernel<D>);
   else if (D == 128 && G <= 3)
-    args(paged_decode_attn_kernel<D, 3>);
+    once ? args(paged_decode_attn_kernel<D, 3, true>)
+         : args(paged_decode_attn_kernel<D, 3, false>);
   else
-    args(paged_decode_attn_kernel<D, 1>);
+    once ? args(paged_decode_attn_kernel<D, 1, true>)
+         : args(paged_decode_attn_kernel<D, 1, false>);
 }
 
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,

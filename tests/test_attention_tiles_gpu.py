@@ -517,3 +517,35 @@ def test_window_scales(scale, d):
         assert ((got[a:a + x].double().view(x, hq, d) - want).abs()
                 <= 2 ** -8 * (mass + want.abs())).all(), i
         a += x
+
+
+@pytest.mark.parametrize("hq,hk,d", [(12, 4, 128), (16, 4, 128), (8, 4, 64),
+                                     (28, 4, 64)])
+def test_decode_table_of_long_contexts(hq, hk, d):
+    """A page table that could hold more than the caches do: values are then
+    read past them.  Short and ragged contexts in it."""
+    torch.manual_seed(10)
+    lens, page, scale = [1, 31, 129, 700], 16, d ** -0.5
+    wide = (128 << 20) // (len(lens) * page * hk * d * 4) + 1
+    need = [-(-n // page) for n in lens]
+    table = torch.zeros(len(lens), wide, dtype=torch.int32, device=DEV)
+    pages = torch.randperm(sum(need), device=DEV).int()
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    k, v = (torch.randn(sum(need), page, hk, d, device=DEV).bfloat16()
+            for _ in range(2))
+    q = torch.randn(len(lens), hq, d, device=DEV).bfloat16()
+    got = ops.paged_attention_decode(
+        q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+        scale)
+    for i, n in enumerate(lens):
+        rows = table[i, :need[i]].long()
+        kk = heads(k[rows].view(-1, hk, d)[:n].double(), hq)
+        vv = heads(v[rows].view(-1, hk, d)[:n].double(), hq)
+        want, _ = attend(q[i:i + 1].double(), kk, vv, n - 1, True, scale)
+        mass, _ = attend(q[i:i + 1].double(), kk, vv.abs(), n - 1, True, scale)
+        # weights have all their bits, the result is rounded once
+        bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
+        assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
