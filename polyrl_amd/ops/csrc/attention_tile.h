@@ -74,7 +74,11 @@ struct AttnTile {
   // The same from 64 rows that start ``start[r]`` numbers behind ``base``
   DEV_INLINE static void gather(char* tile, const bf16_t* base,
                                 const long* start) {
-    const int r = threadIdx.x / GR, g = threadIdx.x % GR;
+    // (heads of 128 have no registers left for these through a kernel's loop:
+    // new to the compiler they are derived again for every tile)
+    int tid = threadIdx.x;
+    if constexpr (D == 128) asm volatile("" : "+v"(tid));
+    const int r = tid / GR, g = tid % GR;
     const bf16_t* from = base + (g ^ swz(r)) * 8;
     char* to = tile + uniform(threadIdx.x >> 6) * 1024;
 #pragma unroll

@@ -384,8 +384,10 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
 // first); of 128: 270 and 243.  Row tiles run by their number: longest walk first
 // found from the tables, as attention_prefill.hip finds it from the lengths, took
 // 157 for 156 (windowed walks are alike).
-template <int D>
-__global__ __launch_bounds__(256, D == 64 ? 4 : 3) void gqa_attn_tile_kernel(
+// ONE_V: one buffer of values, heads of 128 then run three blocks per CU, not two
+template <int D, bool ONE_V>
+__global__ __launch_bounds__(256, D == 64 ? 4 : ONE_V ? 3 : 2)
+void gqa_attn_tile_kernel(
     bf16_t* __restrict__ out,            // (N, H*D), row stride ldo
     const bf16_t* __restrict__ q,        // (N, H*D)
     const bf16_t* __restrict__ cache,    // (slots, 2*G*D)
@@ -397,7 +399,6 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 3) void gqa_attn_tile_kernel(
     const float* __restrict__ sink, float qt_coef, int qt_every, int chunk,
     long ldo, float out_scale) {
   typedef AttnTile<D> T;
-  constexpr bool ONE_V = D == 128;
   // two buffers of K, two or one of V; at the end the waves' rows of the output
   __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
       k1_s[T::BYTES], vx_s[ONE_V ? 16 : T::BYTES];
@@ -530,7 +531,9 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 3) void gqa_attn_tile_kernel(
       if (!(t0 + ATILE - 1 <= min(wp0, jmax) && t0 >= wlo)) {
         // hidden: after the row, or before its window and not kept (in this
         // lane's rows of the accumulators, compared with literals)
-        const int base = t0 + 4 * (lane >> 5), last = min(jmax, rpos) - base,
+        int own = lane;
+        if constexpr (D == 128) asm volatile("" : "+v"(own));
+        const int base = t0 + 4 * (own >> 5), last = min(jmax, rpos) - base,
                   lo = rlo - base, kept = keep - base;
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -764,8 +767,13 @@ void seq_gqa_window_attention_mfma(
           (int)q_temp_every, (int)chunk, (long)out.stride(0),
           (float)out_scale);
     };
-    D == 128 ? launch(gqa_attn_tile_kernel<128>)
-             : launch(gqa_attn_tile_kernel<64>);
+    // One buffer of values costs a wait in the middle of a tile, which only a
+    // third block per CU makes up for: two prompts of 200 .. 300, 32/8 heads of 128
+    // (160 blocks), 15.1 us with one and 14.3 with two; six of 300 .. 500 (670) 29.9
+    // and 30.8; eight of 1200 .. 2048 (3400) 241 and 254.
+    if (D == 64) launch(gqa_attn_tile_kernel<64, false>);
+    else if (items <= 512) launch(gqa_attn_tile_kernel<128, false>);
+    else launch(gqa_attn_tile_kernel<128, true>);
     HIP_CHECK_KERNEL();
     return;
   }

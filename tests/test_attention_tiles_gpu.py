@@ -549,3 +549,42 @@ def test_decode_table_of_long_contexts(hq, hk, d):
         # weights have all their bits, the result is rounded once
         bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
         assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
+
+
+@pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (8, 2, 128), (4, 4, 64)])
+def test_window_many_tiles(hq, hk, d):
+    """More row tiles than run at a time with two blocks per CU: heads of 128
+    then have one buffer of values."""
+    torch.manual_seed(12)
+    lens, page, window, keep, scale = [3, 70, 64, 300] * 33, 16, 90, 5, d ** -0.5
+    need = [-(-n // page) for n in lens]
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32, device=DEV)
+    pages = torch.randperm(sum(need), device=DEV).int()
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    rows = torch.randn(sum(need), page, 2 * hk * d, device=DEV).bfloat16()
+    n = sum(lens)
+    q = torch.randn(n, hq * d, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    seq = torch.repeat_interleave(torch.arange(len(lens), **i32),
+                                  torch.tensor(lens, device=DEV))
+    pos = torch.cat([torch.arange(x, **i32) for x in lens])
+    got = ops.seq.gqa_window_attention(
+        q, rows, table, seq, pos, hq, hk, d, d, window, keep, None, None,
+        None, scale, torch.bfloat16, tiles=ops.seq.attention_tiles(lens, DEV))
+    a = 0
+    for i, x in enumerate(lens):
+        kv = rows[table[i, :need[i]].long()].view(-1, 2, hk, d)[:x].double()
+        k, v = heads(kv[:, 0], hq), heads(kv[:, 1], hq)
+        r, j = torch.arange(x, device=DEV)[:, None], torch.arange(x, device=DEV)
+        live = ((r - j < window) | (j < keep)) & (j <= r)
+        s = torch.einsum("qhd,khd->hqk", q[a:a + x].double().view(x, hq, d),
+                         k) * scale
+        p = torch.softmax(s.masked_fill(~live, -float("inf")), -1)
+        want = torch.einsum("hqk,khd->qhd", p, v)
+        mass = torch.einsum("hqk,khd->qhd", p, v.abs())
+        assert ((got[a:a + x].double().view(x, hq, d) - want).abs()
+                <= 2 ** -8 * (mass + want.abs())).all(), i
+        a += x
