@@ -18,7 +18,7 @@
 // and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
 // at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
 // tokens, 32/8 heads of 128, 59.5 -> 45.2 us, 37.6 with V read past the caches
-// (5.6 TB/s); 33 rows of 1900 .. 8192, 28/4 heads, 264 -> 86.5 -> 82 us.
+// (5.6 TB/s); 33 rows of 1900 .. 8192, 28/4 heads, 264 -> 86.5 -> 82 us, 76 in ten stretches.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -416,19 +416,31 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   const int G = Hq / Hk;
   const long B = q.size(0);
   // Context split: from the sizes alone, not from the lengths on the device,
-  // so that a captured graph may replay it with longer contexts.  At least
-  // 1024 blocks (four per CU, two of them resident at a time at D = 128: the
-  // next start as the first end), but no stretch under 128 keys (a round of the four waves) of the longest
-  // context that the page table holds: there the merging launch costs more
-  // than the split gains (37 cached tokens: 16.8 us in 16 stretches, 6.8 in
-  // one).
+  // so that a captured graph may replay it with longer contexts.  No stretch
+  // under 128 keys (a round of the four waves) of the longest context that the
+  // page table holds: there the merging launch costs more than the split gains
+  // (37 cached tokens: 16.8 us in 16 stretches, 6.8 in one).  Of contexts of up to
+  // 1024 it costs as much already from 512 blocks on (two per CU; before: 1024):
+  // 64 rows of 500 .. 1000, 32/8 heads of 64, 22.6 us in two, 19.8 in one; 64 of
+  // 12/2 heads of 128 19.0 in eight, 15.6 in four; 16 of 64/8 heads 20.3 in
+  // eight, 17.0 in four.  Longer and ragged ones end together with 1600 blocks
+  // (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 11 and 15: 82, 76, 76, 76,
+  // 78; 40 of 1100 .. 2048, 32/8, in 4 and 5: 50.2, 47.7), but more than ten
+  // stretches of a row only where that is needed for 1024 (20 rows of 3000 .. 8000,
+  // 28/4 heads, in 13 and 16: 43.6, 45.0), and from 512 rows and heads on with two
+  // (110 rows of 1000 .. 2000, 32/8 heads of 64, in one and two: 75.8, 74.6).
   const long base_blocks = B * Hk;
   const long most = (long)max_pages * page_size;
   int nsplit = 1;
-  if (base_blocks < 1024)
+  if (base_blocks < 1024) {
+    const long fill = (1024 + base_blocks - 1) / base_blocks;
+    const long want =
+        most <= 1024 ? 512 / base_blocks
+        : base_blocks >= 512 ? fill
+                             : std::min(1600 / base_blocks, std::max(10L, fill));
     nsplit = (int)std::max<long>(
-        1, std::min<long>({(1024 + base_blocks - 1) / base_blocks, 16,
-                           (most + 127) / 128}));
+        1, std::min<long>({want, 16, (most + 127) / 128}));
+  }
   torch::Tensor ws;                     // per call: any stream, any capture
   float* ppart = nullptr;
   if (nsplit > 1) {
