@@ -44,8 +44,10 @@
 
 #include "attention_tile.h"
 
-template <int D>
-__global__ __launch_bounds__(256, D == 64 ? 4 : 3) void prefill_attn_kernel(
+// ONE_V: one buffer of values
+template <int D, bool ONE_V>
+__global__ __launch_bounds__(256, D == 64 ? 4 : ONE_V ? 3 : 2)
+void prefill_attn_kernel(
     bf16_t* __restrict__ out,        // (total_q, Hq, D)
     float* __restrict__ lse,         // (total_q, Hq) log-sum-exp, or null
     const bf16_t* __restrict__ q,    // (total_q, Hq, D)
@@ -58,7 +60,6 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 3) void prefill_attn_kernel(
     int nseq, int ntiles, int nparts, int Hq, int Hk, float scale, int causal,
     long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
-  constexpr bool ONE_V = D == 128;
   // two buffers of K and V each; at the end the waves' rows of the output
   __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
       k1_s[T::BYTES], vx_s[ONE_V ? 16 : T::BYTES];
@@ -321,7 +322,13 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
   const long items = ntiles * Hk * nparts;
   TORCH_CHECK(items < (1L << 31), "grid too large");
   auto stream = at::hip::getCurrentHIPStream();
-  auto kern = (D == 128) ? prefill_attn_kernel<128> : prefill_attn_kernel<64>;
+  // One buffer of values costs a wait in the middle of a tile, which only a third
+  // block per CU makes up for, so not where two per CU are all of them: one prompt
+  // of 1200, 28/4 heads of 128 (300 blocks), 31.3 us with one and 29.8 with two; one
+  // of 512, 32/8 heads 15.8 and 15.0; eight of 1200 .. 2048 (3400) 243 and 259.
+  auto kern = D == 64        ? prefill_attn_kernel<64, false>
+              : items <= 512 ? prefill_attn_kernel<128, false>
+                             : prefill_attn_kernel<128, true>;
   kern<<<dim3((unsigned)items), dim3(256), 0, stream>>>(
       (bf16_t*)out.data_ptr(),
       want_lse ? lse.data_ptr<float>() : nullptr,

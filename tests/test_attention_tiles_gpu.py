@@ -588,3 +588,23 @@ def test_window_many_tiles(hq, hk, d):
         assert ((got[a:a + x].double().view(x, hq, d) - want).abs()
                 <= 2 ** -8 * (mass + want.abs())).all(), i
         a += x
+
+
+@pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (8, 2, 128)])
+def test_forward_many_tiles(hq, hk, d):
+    """More row tiles than run at a time with two blocks per CU: heads of 128
+    then have one buffer of values."""
+    torch.manual_seed(13)
+    lens, scale = [3, 70, 64, 300] * 33 + [129], d ** -0.5
+    cu, n = cu_of(lens), sum(lens)
+    q = torch.randn(n, hq, d, device=DEV).bfloat16()
+    k, v = (torch.randn(n, hk, d, device=DEV).bfloat16() for _ in range(2))
+    out = ops.varlen_prefill_attention(q, k, v, cu.to(DEV), cu.to(DEV), scale,
+                                       True)
+    for i in range(len(lens)):
+        a = slice(cu[i], cu[i + 1])
+        kk, vv = heads(k[a].double(), hq), heads(v[a].double(), hq)
+        want, _ = attend(q[a].double(), kk, vv, 0, True, scale)
+        mass, _ = attend(q[a].double(), kk, vv.abs(), 0, True, scale)
+        bound = 2 ** -8 * (mass + want.abs())
+        assert ((out[a].double() - want).abs() <= bound).all(), i
