@@ -159,11 +159,6 @@ DEV_INLINE bf16x8_t acc_operand(const f32x16_t& c, int s) {
   return v;
 }
 
-// row of a 32-row accumulator that register r holds in this lane
-DEV_INLINE int acc_row(int r) {
-  return 8 * (r >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (r & 3);
-}
-
 // the larger / the sum of a lane's value and that of the lane 32 away
 DEV_INLINE float half_max(float x) {
   const auto p = __builtin_amdgcn_permlane32_swap(
