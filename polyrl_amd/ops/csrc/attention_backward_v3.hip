@@ -61,9 +61,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
   const int t = item / nparts, part = (item + t) % nparts;
   int seq, q0;
-  if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
-                 : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
-                              seq, q0))
+  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, seq, q0))
     return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
@@ -243,8 +241,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const int t = item / nsplit, split = (item + t) % nsplit;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
   int seq, t0;
-  if (nseq <= 64 ? !nth_longest<true>(t, cu_q, cu_k, nseq, seq, t0)
-                 : !find_tile(t, tile_seq, tile_k0, cu_q, nseq, seq, t0))
+  if (!row_tile<true>(t, ntiles, tile_seq, tile_k0, cu_q, cu_k, nseq, seq, t0))
     return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;

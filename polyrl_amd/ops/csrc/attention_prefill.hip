@@ -73,9 +73,7 @@ void prefill_attn_kernel(
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
   const int t = item / nparts, part = (item + t) % nparts;
   int seq, q0;
-  if (nseq <= 64 ? !nth_longest<false>(t, cu_q, cu_k, nseq, seq, q0)
-                 : !find_tile(ntiles - 1 - t, tile_seq, tile_q0, cu_q, nseq,
-                              seq, q0))
+  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, seq, q0))
     return;
   const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
   const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
@@ -283,8 +281,8 @@ void prefill_attn_kernel(
   }
 }
 
-// tile_seq / tile_q0: the 64-row tiles of the packed rows, or empty: the
-// kernel then finds them from cu_seqlens_q itself.
+// tile_seq / tile_q0: the 64-row tiles of the packed rows to compute (all or some
+// of them), or empty: the kernel then finds all from cu_seqlens_q itself.
 void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
                               torch::Tensor k, torch::Tensor v,
                               torch::Tensor cu_seqlens_q,

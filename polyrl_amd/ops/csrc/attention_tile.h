@@ -240,25 +240,36 @@ DEV_INLINE int wave_total(int x) {
   return __builtin_amdgcn_readlane(x, 63);
 }
 
-// Row tile number ``t`` of a packed batch of at most 64 sequences in the order
-// of their walks, longest first; false past the last.  A causal walk is as long
-// as the row tile is late (EARLY: the walk over the query tiles that see a key
-// tile, as it is early), so the order of the table, sequence after sequence,
-// starts a longest block when most of the chip is done: two sequences of
+// Row tile of block ``t`` of ``ntiles``; false past the last.
+//
+// Of at most 64 sequences: in the order of their walks, longest first.  A causal
+// walk is as long as the row tile is late (EARLY: the walk over the query tiles
+// that see a key tile, as it is early), so the order of the table, sequence after
+// sequence, starts a longest block when most of the chip is done: two sequences of
 // 3500 .. 4096, 28/4 heads of 128, kept 1.3 of two waves a SIMD on average.
-// ``above(L)`` counts the tiles whose walk is longer than L tiles.
+// ``above(L)`` counts the tiles whose walk is longer than L tiles.  A table of as
+// many tiles as the sequences have is read at the place that this tile has in
+// the sequences' order, so that every entry is taken once, whatever it names.
+//
+// Tables of another length (of some of the tiles) and more sequences than lanes:
+// in the table's order, from the end where late tiles walk longest.
 template <bool EARLY>
-DEV_INLINE bool nth_longest(int t, const int* cu_q, const int* cu_k, int nseq,
-                            int& seq, int& r0) {
+DEV_INLINE bool row_tile(int t, int ntiles, const int* tile_seq,
+                         const int* tile_r0, const int* cu_q, const int* cu_k,
+                         int nseq, int& seq, int& r0) {
   const int lane = threadIdx.x & 63;
   int n = 0, h = 0;                    // row tiles; key tiles before the first
-  if (lane < nseq) {
+  if (nseq <= 64 && lane < nseq) {
     const int lq = max(cu_q[lane + 1] - cu_q[lane], 0);
     n = (lq + ATILE - 1) / ATILE;
     if (!EARLY) h = max(cu_k[lane + 1] - cu_k[lane] - lq, 0) / ATILE;
   }
   auto above = [&](int L) { return wave_total(min(max(h + n - L, 0), n)); };
-  if (above(0) <= t) return false;
+  const int total = above(0);
+  if (nseq > 64 || (tile_seq != nullptr && ntiles != total))
+    return find_tile(EARLY ? t : ntiles - 1 - t, tile_seq, tile_r0, cu_q, nseq,
+                     seq, r0);
+  if (total <= t) return false;
   int lo = 0, hi = 1;
   while (above(hi) > t) lo = hi, hi *= 2;
   while (hi - lo > 1) {
@@ -274,8 +285,14 @@ DEV_INLINE bool nth_longest(int t, const int* cu_q, const int* cu_k, int nseq,
   const unsigned long long me =
       __ballot((has >> lane & 1) && rank == at);
   seq = __ffsll((long long)me) - 1;
-  r0 = (EARLY ? __builtin_amdgcn_readlane(n, seq) - 1 - lo
-              : lo - __builtin_amdgcn_readlane(h, seq)) * ATILE;
+  const int nth = EARLY ? __builtin_amdgcn_readlane(n, seq) - 1 - lo
+                        : lo - __builtin_amdgcn_readlane(h, seq);
+  r0 = nth * ATILE;
+  if (tile_seq != nullptr) {
+    const int i = wave_total(lane < seq ? n : 0) + nth;
+    seq = uniform(tile_seq[i]);
+    r0 = uniform(tile_r0[i]);
+  }
   return true;
 }
 

@@ -608,3 +608,44 @@ def test_forward_many_tiles(hq, hk, d):
         mass, _ = attend(q[a].double(), kk, vv.abs(), 0, True, scale)
         bound = 2 ** -8 * (mass + want.abs())
         assert ((out[a].double() - want).abs() <= bound).all(), i
+
+
+@pytest.mark.parametrize("what", ["some", "turned", "one_of_them"])
+@pytest.mark.parametrize("nseq", [3, 66])
+@pytest.mark.parametrize("d", [64, 128])
+def test_tables_of_some_tiles(nseq, d, what):
+    """A table names the tiles that are computed, in any order: rows of named
+    tiles get what a call without a table gives, others are left alone."""
+    torch.manual_seed(14)
+    lens, h, scale = ([130, 65, 200] * 22)[:nseq], 4, d ** -0.5
+    cu_cpu, n = cu_of(lens), sum(lens)
+    cu = cu_cpu.to(DEV)
+    q, k, v, dout = (torch.randn(n, h, d, device=DEV).bfloat16()
+                     for _ in range(4))
+    ext, (t_seq, t_r0) = ops._require_ext(), ops.build_varlen_tiles(
+        cu_cpu, DEV)[:2]
+    pick = {"some": torch.arange(1, len(t_seq), 3),
+            "turned": torch.arange(len(t_seq)).flip(0),
+            "one_of_them": torch.full((len(t_seq),), 2)}[what].to(DEV)
+    some = t_seq[pick].contiguous(), t_r0[pick].contiguous()
+    named = torch.zeros(n, dtype=torch.bool, device=DEV)
+    for s, r in zip(some[0].tolist(), some[1].tolist()):
+        named[cu_cpu[s] + r:min(cu_cpu[s] + r + 64, cu_cpu[s + 1])] = True
+
+    want, lse = ops.varlen_prefill_attention(q, k, v, cu, cu, scale, True,
+                                             return_lse=True)
+    got = torch.full_like(want, -7.0)
+    ext.varlen_prefill_attention(got, q, k, v, cu, cu, *some, scale, True,
+                                 torch.empty(0))
+    assert torch.equal(got[named], want[named])
+    assert (got[~named] == -7).all()
+
+    def grads(tiles):
+        g = [torch.full_like(q, -7.0) for _ in range(3)]
+        ext.varlen_attention_backward_v3(*g, q, k, v, want, dout, lse, cu, cu,
+                                         *tiles, scale, True)
+        return g
+    # (dK takes sums of the gradient from dQ's tiles)
+    for a, b in list(zip(grads(some), grads((t_seq, t_r0))))[::2]:
+        assert torch.equal(a[named], b[named])
+        assert (a[~named] == -7).all()
