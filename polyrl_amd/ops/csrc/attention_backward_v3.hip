@@ -260,9 +260,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   frag_global<D>(kf, k + (long)krow * ldk + (long)hk * D);
   if constexpr (!V_LDS)
     frag_global<D>(vf, v + (long)krow * ldv + (long)hk * D);
-  // (not 0: a hidden score is infinite, see the forward kernel)
-  const float s2 = scale != 0.f ? scale * 1.4426950408889634f : 0x1p-126f;
-  const float hidden = s2 >= 0.f ? -INFINITY : INFINITY;
+  const float s2 = scale * 1.4426950408889634f;
 
   FragAt<D> at;
   f32x16_t ak[DT], av[DT];
@@ -365,24 +363,31 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         SCHED_LDS(PER);
       }
       SCHED_MFMA(3);
-      // rows before this lane's key (compared with literals)
+      const int r0 = qh * 32 + 4 * (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 le = *reinterpret_cast<const float4*>(&row_s[0][r0 + 8 * i]);
+        const float l4[4] = {le.x, le.y, le.z, le.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          s[4 * i + t] = __builtin_fmaf(s[4 * i + t], s2, -l4[t]);
+      }
+      // rows before this lane's key (compared with literals), whatever their
+      // log-sum-exp: it may be NaN
       if (causal && qk_off + wq0 < wk0 + 31) {
         const int border = key - (qk_off + wq0) - 4 * (lane >> 5);
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (8 * (r >> 2) + (r & 3) < border) s[r] = hidden;
+          if (8 * (r >> 2) + (r & 3) < border) s[r] = -INFINITY;
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r0 = qh * 32 + 8 * i + 4 * (lane >> 5);
-        const float4 le = *reinterpret_cast<const float4*>(&row_s[0][r0]);
-        const float4 de = *reinterpret_cast<const float4*>(&row_s[1][r0]);
-        const float l4[4] = {le.x, le.y, le.z, le.w};
+        const float4 de = *reinterpret_cast<const float4*>(&row_s[1][r0 + 8 * i]);
         const float d4[4] = {de.x, de.y, de.z, de.w};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * i + t;
-          const float w = exp2_hw(__builtin_fmaf(s[r], s2, -l4[t]));
+          const float w = exp2_hw(s[r]);
           s[r] = w;
           dp[r] = w * __builtin_fmaf(dp[r], scale, -d4[t]);
         }

@@ -317,7 +317,7 @@ DEV_INLINE U read_through(const U* from) {
 // get the bin and the sum above it.  lds: the waves' sums, the first thread
 // that reaches the goal, its bin and the sum above that, each in words of its
 // own: a wave may still read the thread while that thread writes its bin.
-template <bool MASS, int NT = SNT, bool FAR = false>
+template <bool MASS, int NT>
 DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
                          float* lds, int& bin, float& before) {
   // thread t has bins [t*per, +per) counted from the top
@@ -328,11 +328,8 @@ DEV_INLINE void find_bin(const uint32_t* bins, int n, float above, float goal,
   for (int i = 0; i < MOST; ++i) {
     const int at = threadIdx.x * per + i;
     val[i] = 0.f;
-    if (i < per && at < n) {
-      const uint32_t b =
-          FAR ? read_through(&bins[n - 1 - at]) : bins[n - 1 - at];
-      val[i] = MASS ? __uint_as_float(b) : (float)b;
-    }
+    if (i < per && at < n)
+      val[i] = MASS ? __uint_as_float(bins[n - 1 - at]) : (float)bins[n - 1 - at];
   }
 #pragma unroll
   for (int i = 0; i < MOST; ++i) own += val[i];
@@ -466,11 +463,16 @@ DEV_INLINE float wave_cut(const float* tops, int n, bool by_k, bool by_p, int k,
 
 // What the passes over a filtered row tell each other, zeros at first: the
 // entries at or above the cut so far, the blocks that are through with each
-// pass, and whether the row's token is written.
+// pass, whether the row's token is written, and, if the list was too short, one
+// more than the entries in it.
 struct RowState {
-  uint32_t listed, arrived[4], done, pad[2];
+  uint32_t listed, arrived[4], done, overfull, pad;
 };
 constexpr int LISTED = 1024;          // entries that a row's list holds
+// Up to which they are counted, one a thread, and not binned: counting takes the
+// square of their number (64 x 151936, top-p 0.95 at T 0.7, 500 candidates: 65 us
+// counted, 38 binned; 58 without lists).
+constexpr int COUNTED = SNT;
 
 // Whether this block is the last of its row's to come here: what the others added
 // with atomics or wrote through can then be read through.  Nobody waits for
@@ -489,20 +491,45 @@ DEV_INLINE bool last_of_row(uint32_t* arrived, int split) {
 }
 
 // A digit's bins decide (all threads of a block)
-template <typename T>
-DEV_INLINE void walk_bins(Plan& plan, const uint32_t* h, int digit, int k,
-                          float* lds) {
+template <int NT, typename T>
+DEV_INLINE void walk_bins(Plan& plan, const uint32_t* cnt, const float* mass,
+                          int digit, int k, float* lds) {
   const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
   int bin;
   float before;
   if (plan.by & 1) {
-    find_bin<false, SNT, true>(h, bins, plan.cnt, (float)k, lds, bin, before);
+    find_bin<false, NT>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
     plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
   }
   if (plan.by & 2) {
-    find_bin<true, SNT, true>(h + DIGIT, bins, plan.mass, plan.target, lds, bin, before);
+    find_bin<true, NT>(reinterpret_cast<const uint32_t*>(mass), bins, plan.mass,
+                       plan.target, lds, bin, before);
     plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
   }
+}
+
+// The row's bins, to which the other blocks added, into LDS: whole lines, all on
+// their way at once.  No load stands under a condition: its wait would stand there
+// too, and with sixteen waits in turn for what comes past the L2 64 x 50257 fp32,
+// top-p 0.8 at T 0.7, took 62 us (the three plan launches before it 61), 58 now.
+template <typename T>
+DEV_INLINE void read_bins(int digit, const uint32_t* h, uint32_t* cnt,
+                          float* mass) {
+  constexpr int PER = DIGIT / SNT;
+  const int last = digit_bins<T>(digit) - 1;
+  uint32_t c[PER], m[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int at = min(i * SNT + (int)threadIdx.x, last);
+    c[i] = read_through(&h[at]);
+    m[i] = read_through(&h[DIGIT + at]);
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    cnt[i * SNT + threadIdx.x] = c[i];
+    mass[i * SNT + threadIdx.x] = __uint_as_float(m[i]);
+  }
+  __syncthreads();
 }
 
 // the block's best entry, in the first wave
@@ -666,17 +693,27 @@ __global__ __launch_bounds__(64) void sample_merge_kernel(
             VocabRow<T>(logits + row * V, V), row, split);
 }
 
+// an entry into the bins of a digit, if it shares the digits before it with a
+// threshold
+template <typename T>
+DEV_INLINE void add_entry(float v, int digit, const Plan& plan, float inv_temp,
+                          uint32_t* cnt, float* mass) {
+  const uint32_t above = digit == 0 ? 0u
+      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
+  const uint32_t e = enc_f32(v);
+  const uint32_t bin = (e >> digit_low<T>(digit)) & (digit_bins<T>(digit) - 1);
+  if ((plan.by & 1) && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
+  if ((plan.by & 2) && (e & above) == plan.prefix_p && v != -INFINITY)
+    atomicAdd(&mass[bin], __expf((v - plan.m) * inv_temp));
+}
+
 // a thread's entries of the groups [first, ..) of every ``stride`` into the
-// bins of a digit, if they share the digits before it with a threshold
+// bins of a digit
 template <typename T>
 DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
                           int digit, const Plan& plan, float inv_temp,
                           uint32_t* cnt, float* mass) {
   constexpr int VEC = VocabRow<T>::VEC;
-  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
-  const uint32_t above = digit == 0 ? 0u
-      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
-  const bool by_k = plan.by & 1, by_p = plan.by & 2;
   const int groups = r.groups();
   for (int g = first + threadIdx.x; g < groups; g += stride) {
     float v[VEC];
@@ -685,50 +722,34 @@ DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       if (v[j] < plan.cut || (unsigned)(i0 + j) >= (unsigned)r.V) continue;
-      const uint32_t e = enc_f32(v[j]);
-      const uint32_t bin = (e >> low) & (bins - 1);
-      if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
-      if (by_p && (e & above) == plan.prefix_p && v[j] != -INFINITY)
-        atomicAdd(&mass[bin], __expf((v[j] - plan.m) * inv_temp));
+      add_entry<T>(v[j], digit, plan, inv_temp, cnt, mass);
     }
   }
 }
 
-// both selections of a row by one block
-template <int NT, typename T>
-DEV_INLINE void select_alone(const VocabRow<T>& r, Plan& plan, int k,
-                             float inv_temp, uint32_t* cnt, float* mass,
-                             float* lds) {
+// both selections by one block; ``fill(digit)`` adds the entries to its bins
+template <int NT, typename T, typename F>
+DEV_INLINE void select_alone(Plan& plan, int k, uint32_t* cnt, float* mass,
+                             float* lds, F fill) {
   for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
-    const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+    const int bins = digit_bins<T>(digit);
     for (int i = threadIdx.x; i < bins; i += NT) cnt[i] = 0, mass[i] = 0.f;
     __syncthreads();
-    fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
+    fill(digit);
     __syncthreads();
-    int bin;
-    float before;
-    if (plan.by & 1) {
-      find_bin<false, NT>(cnt, bins, plan.cnt, (float)k, lds, bin, before);
-      plan.prefix_k |= (uint32_t)bin << low, plan.cnt = before;
-    }
-    if (plan.by & 2) {
-      find_bin<true, NT>(reinterpret_cast<const uint32_t*>(mass), bins,
-                         plan.mass, plan.target, lds, bin, before);
-      plan.prefix_p |= (uint32_t)bin << low, plan.mass = before;
-    }
+    walk_bins<NT, T>(plan, cnt, mass, digit, k, lds);
     __syncthreads();                    // the bins were read
   }
 }
 
-// a piece's entries into the row's bins of a digit
-template <typename T>
-DEV_INLINE void add_bins(const VocabRow<T>& r, int piece, int split, int digit,
-                         const Plan& plan, float inv_temp, uint32_t* cnt,
-                         float* mass, uint32_t* h) {
+// entries into the row's bins of a digit: ``fill`` adds them to the block's own
+template <typename T, typename F>
+DEV_INLINE void add_bins(int digit, uint32_t* cnt, float* mass, uint32_t* h,
+                         F fill) {
   const int bins = digit_bins<T>(digit);
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
   __syncthreads();
-  fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
+  fill();
   __syncthreads();
   float* hm = reinterpret_cast<float*>(h + DIGIT);
   for (int i = threadIdx.x; i < bins; i += SNT) {
@@ -745,7 +766,10 @@ DEV_INLINE void add_bins(const VocabRow<T>& r, int piece, int split, int digit,
 //
 // How much it is, the maxima of the lanes' groups tell: of g groups, n entries in
 // random order leave a share of exp(-n / g) without one.  If they are not in random
-// order and the list is too short, the last block takes the steps of a short row.
+// order and the list is too short, the pieces whose entries it does not hold add
+// them to the bins, the last block those that it does, and the row goes on like
+// one without a list (64 x 151936, top-p 0.95 at T 0.7, 4000 candidates side by
+// side: 66 us; 183 with one block for such a row's passes, 69 without lists).
 template <typename T>
 __global__ __launch_bounds__(SNT) void sample_select_kernel(
     int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
@@ -797,6 +821,7 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
       with += __popcll(__ballot(i < g && tops[row * g + i] >= cut));
     listing = with <= g * (1.f - __expf(-0.7f * LISTED / g));
   }
+  bool to_bins = !listing;
   if (listing) {
     int* own_i = reinterpret_cast<int*>(cnt);
     float* own_v = mass;
@@ -821,40 +846,80 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     }
     __syncthreads();
     const int n = min(found, LISTED + 1);
-    if (threadIdx.x == 0) base = n ? atomicAdd(&state->listed, (uint32_t)n) : 0;
-    __syncthreads();
-    for (int t = threadIdx.x; t < n && base + t < LISTED; t += SNT) {
-      write_through(&list_v[base + t], own_v[t]);
-      write_through(&list_i[base + t], own_i[t]);
+    if (threadIdx.x == 0) {
+      base = n ? atomicAdd(&state->listed, (uint32_t)n) : 0;
+      // (only the first one past the end: what comes later starts behind it)
+      if (base <= LISTED && base + n > LISTED)
+        write_through(&state->overfull, base + 1);
     }
-  } else {
-    add_bins(r, piece, split, 0, plan, inv_temp, cnt, mass, h);
+    __syncthreads();
+    if (base + n <= LISTED) {
+      for (int t = threadIdx.x; t < n; t += SNT) {
+        write_through(&list_v[base + t], own_v[t]);
+        write_through(&list_i[base + t], own_i[t]);
+      }
+    } else if (n <= LISTED) {           // all that it has are in its own list
+      float v[LISTED / SNT];
+#pragma unroll
+      for (int i = 0; i < LISTED / SNT; ++i)
+        v[i] = own_v[i * SNT + threadIdx.x];
+      __syncthreads();                  // (the list is where the bins will be)
+      add_bins<T>(0, cnt, mass, h, [&] {
+#pragma unroll
+        for (int i = 0; i < LISTED / SNT; ++i)
+          if (i * SNT + (int)threadIdx.x < n)
+            add_entry<T>(v[i], 0, plan, inv_temp, cnt, mass);
+      });
+    } else {
+      to_bins = true;
+    }
   }
+  if (to_bins)
+    add_bins<T>(0, cnt, mass, h, [&] {
+      fill_bins(r, piece * SNT, split * SNT, 0, plan, inv_temp, cnt, mass);
+    });
   if (!last_of_row(&state->arrived[0], split)) return;
 
-  if (!listing) {
-    walk_bins<T>(plan, h, 0, k, lds);
+  // this thread's entries of the list, all on their way at once
+  float own[LISTED / SNT];
+#pragma unroll
+  for (int i = 0; i < LISTED / SNT; ++i)
+    own[i] = read_through(&list_v[i * SNT + threadIdx.x]);
+  auto each = [&](int n, auto take) {
+#pragma unroll
+    for (int i = 0; i < LISTED / SNT; ++i)
+      if (i * SNT + (int)threadIdx.x < n) take(i * SNT + threadIdx.x, own[i]);
+  };
+  const int overfull = listing ? read_through(&state->overfull) : 0;
+  if (!listing || overfull) {
+    read_bins<T>(0, h, cnt, mass);
+    if (overfull) {
+      each(overfull - 1, [&](int, float v) {
+        add_entry<T>(v, 0, plan, inv_temp, cnt, mass);
+      });
+      __syncthreads();
+    }
+    walk_bins<SNT, T>(plan, cnt, mass, 0, k, lds);
     if (threadIdx.x == 0) plans[row] = plan;
     return;
   }
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  const int listed = min(read_through(&state->listed), LISTED + 1u);
-  Draw d;
-  if (listed > LISTED) {
-    select_alone<SNT>(r, plan, k, inv_temp, cnt, mass, lds);
-    Sums<false> none;
-    walk<2, SNT>(r, 0, SNT, false, inv_temp, rowkey, plan.threshold(), none, d);
+  const int listed = read_through(&state->listed);
+  if (listed > COUNTED) {
+    select_alone<SNT, T>(plan, k, cnt, mass, lds, [&](int digit) {
+      each(listed, [&](int, float v) {
+        add_entry<T>(v, digit, plan, inv_temp, cnt, mass);
+      });
+    });
   } else {
     // (four at a time; what fills up is no larger than any and weighs nothing)
-    for (int t = threadIdx.x; t < (listed + 3) / 4 * 4; t += SNT) {
-      const float v = t < listed ? read_through(&list_v[t]) : 0.f;
-      cnt[t] = t < listed ? enc_f32(v) : 0u;
-      mass[t] = t < listed ? __expf((v - all.m) * inv_temp) : 0.f;
-    }
-    if (threadIdx.x == 0) thr[0] = thr[1] = 0;
+    const int t = threadIdx.x;
+    const uint32_t e = t < listed ? enc_f32(own[0]) : 0u;
+    cnt[t] = e;
+    mass[t] = t < listed ? __expf((own[0] - all.m) * inv_temp) : 0.f;
+    if (t == 0) thr[0] = thr[1] = 0;
     __syncthreads();
-    for (int t = threadIdx.x; t < listed; t += SNT) {
-      const uint32_t e = cnt[t];
+    if (t < listed) {
       int count = 0;
       float sum = 0.f;
       for (int j = 0; j < listed; j += 4) {
@@ -869,15 +934,15 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     }
     __syncthreads();
     plan.prefix_k = thr[0], plan.prefix_p = thr[1];
-    const uint32_t tau = plan.threshold();
-    for (int t = threadIdx.x; t < listed; t += SNT) {
-      if (cnt[t] < tau) continue;
-      const int i = read_through(&list_i[t]);
-      const float z = __fmaf_rn(read_through(&list_v[t]), inv_temp,
-                                gumbel(rng_bits(rowkey, rng_at(i))));
-      if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
-    }
   }
+  const uint32_t tau = plan.threshold();
+  Draw d;
+  each(listed, [&](int t, float v) {
+    if (enc_f32(v) < tau) return;
+    const int i = read_through(&list_i[t]);
+    const float z = __fmaf_rn(v, inv_temp, gumbel(rng_bits(rowkey, rng_at(i))));
+    if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
+  });
   block_best(d.best, d.best_i, part);
   if (threadIdx.x == 0) {
     out_tokens[row] = d.best_i;
@@ -901,10 +966,15 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
   Plan plan = plans[row];
   if (plan.by == 0) return;
   uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
-  add_bins(VocabRow<T>(logits + row * V, V), blockIdx.x % split, split, digit,
-           plan, 1.0f / temperature[row], cnt, mass, h);
+  const VocabRow<T> r(logits + row * V, V);
+  const int piece = blockIdx.x % split;
+  const float inv_temp = 1.0f / temperature[row];
+  add_bins<T>(digit, cnt, mass, h, [&] {
+    fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
+  });
   if (!last_of_row(&state->arrived[digit], split)) return;
-  walk_bins<T>(plan, h, digit, top_k[row], lds);
+  read_bins<T>(digit, h, cnt, mass);
+  walk_bins<SNT, T>(plan, cnt, mass, digit, top_k[row], lds);
   if (threadIdx.x == 0) plans[row] = plan;
 }
 
@@ -961,7 +1031,9 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
       if (by_k || by_p) {
         Plan plan(cut_of<NT>(tops, NTOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
                   sums, p, by_k, by_p);
-        select_alone<NT>(r, plan, k, inv_temp, cnt, mass, lds);
+        select_alone<NT, T>(plan, k, cnt, mass, lds, [&](int digit) {
+          fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
+        });
         tau = plan.threshold();
       }
       Draw pick;

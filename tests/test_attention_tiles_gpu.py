@@ -649,3 +649,29 @@ def test_tables_of_some_tiles(nseq, d, what):
     for a, b in list(zip(grads(some), grads((t_seq, t_r0))))[::2]:
         assert torch.equal(a[named], b[named])
         assert (a[~named] == -7).all()
+
+
+@pytest.mark.parametrize("scale", [0.125, 0.0, -0.125])
+@pytest.mark.parametrize("d", [64, 128])
+def test_values_of_keys_that_a_nan_row_does_not_see(d, scale):
+    """A row whose log-sum-exp is NaN: gradients of the values behind it are
+    what they are without it, those that it sees are NaN."""
+    torch.manual_seed(16)
+    n, bad, hq, hk = 70, 5, 4, 2
+    cu_cpu = cu_of([n])
+    cu, tiles = cu_cpu.to(DEV), ops.build_varlen_tiles(cu_cpu, DEV)[:2]
+    q, dout = (torch.randn(n, hq, d, device=DEV).bfloat16() for _ in range(2))
+    k, v = (torch.randn(n, hk, d, device=DEV).bfloat16() for _ in range(2))
+    out, lse = ops.varlen_prefill_attention(q, k, v, cu, cu, scale, True,
+                                            return_lse=True)
+
+    def grad_v(lse):
+        g = [torch.empty_like(t) for t in (q, k, v)]
+        ops._require_ext().varlen_attention_backward_v3(
+            *g, q, k, v, out, dout, lse, cu, cu, *tiles, scale, True)
+        return g[2]
+    want = grad_v(lse)
+    lse[bad] = float("nan")
+    got = grad_v(lse)
+    assert torch.equal(got[bad + 1:], want[bad + 1:])
+    assert torch.isnan(got[:bad + 1]).all()

@@ -375,3 +375,52 @@ def test_sample_candidate_lists(what, k, p, dtype):
         z = row / temp + noise(seed, r, v)
         # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
         assert z[t] >= z[sure].max() - 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [9, 40])
+def test_sample_rows_of_every_kind(n, dtype):
+    """One call whose rows go every way that a long row can: the largest logit,
+    no filter, few candidates, many, neighbours that a list does not hold
+    (from one piece, or from several), all alike, NaN; an odd row length."""
+    torch.manual_seed(15)
+    v, seed = 70001, 123
+    x = torch.randn(n, v, device=DEV) * 2
+    temp, k, p = [], [], []
+    kinds = [("greedy", 0.0, 40, 0.9), ("plain", 0.9, -1, 1.0),
+             ("few", 0.7, 50, 0.9), ("flat", 1.3, -1, 0.95),
+             ("next", 0.8, -1, 0.9), ("wide", 0.8, 90, 0.97),
+             ("alike", 1.0, 20, 1.0), ("greedy", 0.0, -1, 1.0),
+             ("nan", 0.8, 30, 0.9)]
+    what = [kinds[(r * 7) % len(kinds)] for r in range(n)]
+    for r, (kind, t, kk, pp) in enumerate(what):
+        temp.append(t), k.append(kk), p.append(pp)
+        if kind == "flat":
+            x[r] = torch.rand(v, device=DEV)
+        elif kind == "next":
+            x[r, 3000:4500] = 12 + torch.rand(1500, device=DEV)
+        elif kind == "wide":            # several pieces list, the last do not fit
+            x[r, 1000:20000:9] = 12 + torch.rand(2112, device=DEV)
+        elif kind == "alike":
+            x[r] = 1.0
+        elif kind == "nan":
+            x[r, 777] = float("nan")
+    x = x.to(dtype)
+    tok, lp = ops.sample(x, torch.tensor(temp, device=DEV),
+                         torch.tensor(k, dtype=torch.int32, device=DEV),
+                         torch.tensor(p, device=DEV), seed, no_filter=False)
+    for r, (kind, t, kk, pp) in enumerate(what):
+        row, got = x[r].double().cpu(), int(tok[r])
+        if kind == "nan":
+            assert 0 <= got < v and torch.isnan(lp[r])
+            continue
+        want = torch.log_softmax(row, -1)[got]
+        assert abs(float(lp[r]) - want) <= 1e-5 * (1 + abs(want)), r
+        if t == 0.0:
+            assert row[got] == row.max(), r
+            continue
+        sure, maybe = kept(row, t, kk, pp)
+        assert maybe[got], (r, kind)
+        z = row / t + noise(seed, r, v)
+        # (as above)
+        assert z[got] >= z[sure].max() - 1e-3, (r, kind)
