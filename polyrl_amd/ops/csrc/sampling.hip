@@ -463,16 +463,11 @@ DEV_INLINE float wave_cut(const float* tops, int n, bool by_k, bool by_p, int k,
 
 // What the passes over a filtered row tell each other, zeros at first: the
 // entries at or above the cut so far, the blocks that are through with each
-// pass, whether the row's token is written, and, if the list was too short, one
-// more than the entries in it.
+// pass, and whether the row's token is written.
 struct RowState {
-  uint32_t listed, arrived[4], done, overfull, pad;
+  uint32_t listed, arrived[4], done, pad[2];
 };
 constexpr int LISTED = 1024;          // entries that a row's list holds
-// Up to which they are counted, one a thread, and not binned: counting takes the
-// square of their number (64 x 151936, top-p 0.95 at T 0.7, 500 candidates: 65 us
-// counted, 38 binned; 58 without lists).
-constexpr int COUNTED = SNT;
 
 // Whether this block is the last of its row's to come here: what the others added
 // with atomics or wrote through can then be read through.  Nobody waits for
@@ -693,27 +688,17 @@ __global__ __launch_bounds__(64) void sample_merge_kernel(
             VocabRow<T>(logits + row * V, V), row, split);
 }
 
-// an entry into the bins of a digit, if it shares the digits before it with a
-// threshold
-template <typename T>
-DEV_INLINE void add_entry(float v, int digit, const Plan& plan, float inv_temp,
-                          uint32_t* cnt, float* mass) {
-  const uint32_t above = digit == 0 ? 0u
-      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
-  const uint32_t e = enc_f32(v);
-  const uint32_t bin = (e >> digit_low<T>(digit)) & (digit_bins<T>(digit) - 1);
-  if ((plan.by & 1) && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
-  if ((plan.by & 2) && (e & above) == plan.prefix_p && v != -INFINITY)
-    atomicAdd(&mass[bin], __expf((v - plan.m) * inv_temp));
-}
-
 // a thread's entries of the groups [first, ..) of every ``stride`` into the
-// bins of a digit
+// bins of a digit, if they share the digits before it with a threshold
 template <typename T>
 DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
                           int digit, const Plan& plan, float inv_temp,
                           uint32_t* cnt, float* mass) {
   constexpr int VEC = VocabRow<T>::VEC;
+  const int bins = digit_bins<T>(digit), low = digit_low<T>(digit);
+  const uint32_t above = digit == 0 ? 0u
+      : 0xFFFFFFFFu << digit_low<T>(digit - 1);
+  const bool by_k = plan.by & 1, by_p = plan.by & 2;
   const int groups = r.groups();
   for (int g = first + threadIdx.x; g < groups; g += stride) {
     float v[VEC];
@@ -722,34 +707,40 @@ DEV_INLINE void fill_bins(const VocabRow<T>& r, int first, int stride,
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       if (v[j] < plan.cut || (unsigned)(i0 + j) >= (unsigned)r.V) continue;
-      add_entry<T>(v[j], digit, plan, inv_temp, cnt, mass);
+      const uint32_t e = enc_f32(v[j]);
+      const uint32_t bin = (e >> low) & (bins - 1);
+      if (by_k && (e & above) == plan.prefix_k) atomicAdd(&cnt[bin], 1u);
+      if (by_p && (e & above) == plan.prefix_p && v[j] != -INFINITY)
+        atomicAdd(&mass[bin], __expf((v[j] - plan.m) * inv_temp));
     }
   }
 }
 
-// both selections by one block; ``fill(digit)`` adds the entries to its bins
-template <int NT, typename T, typename F>
-DEV_INLINE void select_alone(Plan& plan, int k, uint32_t* cnt, float* mass,
-                             float* lds, F fill) {
+// both selections of a row by one block
+template <int NT, typename T>
+DEV_INLINE void select_alone(const VocabRow<T>& r, Plan& plan, int k,
+                             float inv_temp, uint32_t* cnt, float* mass,
+                             float* lds) {
   for (int digit = 0; digit < (sizeof(T) == 2 ? 2 : 3); ++digit) {
     const int bins = digit_bins<T>(digit);
     for (int i = threadIdx.x; i < bins; i += NT) cnt[i] = 0, mass[i] = 0.f;
     __syncthreads();
-    fill(digit);
+    fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
     __syncthreads();
     walk_bins<NT, T>(plan, cnt, mass, digit, k, lds);
     __syncthreads();                    // the bins were read
   }
 }
 
-// entries into the row's bins of a digit: ``fill`` adds them to the block's own
-template <typename T, typename F>
-DEV_INLINE void add_bins(int digit, uint32_t* cnt, float* mass, uint32_t* h,
-                         F fill) {
+// a piece's entries into the row's bins of a digit
+template <typename T>
+DEV_INLINE void add_bins(const VocabRow<T>& r, int piece, int split, int digit,
+                         const Plan& plan, float inv_temp, uint32_t* cnt,
+                         float* mass, uint32_t* h) {
   const int bins = digit_bins<T>(digit);
   for (int i = threadIdx.x; i < bins; i += SNT) cnt[i] = 0, mass[i] = 0.f;
   __syncthreads();
-  fill();
+  fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
   __syncthreads();
   float* hm = reinterpret_cast<float*>(h + DIGIT);
   for (int i = threadIdx.x; i < bins; i += SNT) {
@@ -766,10 +757,7 @@ DEV_INLINE void add_bins(int digit, uint32_t* cnt, float* mass, uint32_t* h,
 //
 // How much it is, the maxima of the lanes' groups tell: of g groups, n entries in
 // random order leave a share of exp(-n / g) without one.  If they are not in random
-// order and the list is too short, the pieces whose entries it does not hold add
-// them to the bins, the last block those that it does, and the row goes on like
-// one without a list (64 x 151936, top-p 0.95 at T 0.7, 4000 candidates side by
-// side: 66 us; 183 with one block for such a row's passes, 69 without lists).
+// order and the list is too short, the last block takes the steps of a short row.
 template <typename T>
 __global__ __launch_bounds__(SNT) void sample_select_kernel(
     int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
@@ -821,7 +809,6 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
       with += __popcll(__ballot(i < g && tops[row * g + i] >= cut));
     listing = with <= g * (1.f - __expf(-0.7f * LISTED / g));
   }
-  bool to_bins = !listing;
   if (listing) {
     int* own_i = reinterpret_cast<int*>(cnt);
     float* own_v = mass;
@@ -846,80 +833,41 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     }
     __syncthreads();
     const int n = min(found, LISTED + 1);
-    if (threadIdx.x == 0) {
-      base = n ? atomicAdd(&state->listed, (uint32_t)n) : 0;
-      // (only the first one past the end: what comes later starts behind it)
-      if (base <= LISTED && base + n > LISTED)
-        write_through(&state->overfull, base + 1);
-    }
+    if (threadIdx.x == 0) base = n ? atomicAdd(&state->listed, (uint32_t)n) : 0;
     __syncthreads();
-    if (base + n <= LISTED) {
-      for (int t = threadIdx.x; t < n; t += SNT) {
-        write_through(&list_v[base + t], own_v[t]);
-        write_through(&list_i[base + t], own_i[t]);
-      }
-    } else if (n <= LISTED) {           // all that it has are in its own list
-      float v[LISTED / SNT];
-#pragma unroll
-      for (int i = 0; i < LISTED / SNT; ++i)
-        v[i] = own_v[i * SNT + threadIdx.x];
-      __syncthreads();                  // (the list is where the bins will be)
-      add_bins<T>(0, cnt, mass, h, [&] {
-#pragma unroll
-        for (int i = 0; i < LISTED / SNT; ++i)
-          if (i * SNT + (int)threadIdx.x < n)
-            add_entry<T>(v[i], 0, plan, inv_temp, cnt, mass);
-      });
-    } else {
-      to_bins = true;
+    for (int t = threadIdx.x; t < n && base + t < LISTED; t += SNT) {
+      write_through(&list_v[base + t], own_v[t]);
+      write_through(&list_i[base + t], own_i[t]);
     }
+  } else {
+    add_bins(r, piece, split, 0, plan, inv_temp, cnt, mass, h);
   }
-  if (to_bins)
-    add_bins<T>(0, cnt, mass, h, [&] {
-      fill_bins(r, piece * SNT, split * SNT, 0, plan, inv_temp, cnt, mass);
-    });
   if (!last_of_row(&state->arrived[0], split)) return;
 
-  // this thread's entries of the list, all on their way at once
-  float own[LISTED / SNT];
-#pragma unroll
-  for (int i = 0; i < LISTED / SNT; ++i)
-    own[i] = read_through(&list_v[i * SNT + threadIdx.x]);
-  auto each = [&](int n, auto take) {
-#pragma unroll
-    for (int i = 0; i < LISTED / SNT; ++i)
-      if (i * SNT + (int)threadIdx.x < n) take(i * SNT + threadIdx.x, own[i]);
-  };
-  const int overfull = listing ? read_through(&state->overfull) : 0;
-  if (!listing || overfull) {
+  if (!listing) {
     read_bins<T>(0, h, cnt, mass);
-    if (overfull) {
-      each(overfull - 1, [&](int, float v) {
-        add_entry<T>(v, 0, plan, inv_temp, cnt, mass);
-      });
-      __syncthreads();
-    }
     walk_bins<SNT, T>(plan, cnt, mass, 0, k, lds);
     if (threadIdx.x == 0) plans[row] = plan;
     return;
   }
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  const int listed = read_through(&state->listed);
-  if (listed > COUNTED) {
-    select_alone<SNT, T>(plan, k, cnt, mass, lds, [&](int digit) {
-      each(listed, [&](int, float v) {
-        add_entry<T>(v, digit, plan, inv_temp, cnt, mass);
-      });
-    });
+  const int listed = min(read_through(&state->listed), LISTED + 1u);
+  Draw d;
+  if (listed > LISTED) {
+    select_alone<SNT>(r, plan, k, inv_temp, cnt, mass, lds);
+    Sums<false> none;
+    walk<2, SNT>(r, 0, SNT, false, inv_temp, rowkey, plan.threshold(), none, d);
   } else {
     // (four at a time; what fills up is no larger than any and weighs nothing)
-    const int t = threadIdx.x;
-    const uint32_t e = t < listed ? enc_f32(own[0]) : 0u;
-    cnt[t] = e;
-    mass[t] = t < listed ? __expf((own[0] - all.m) * inv_temp) : 0.f;
-    if (t == 0) thr[0] = thr[1] = 0;
+    for (int t = threadIdx.x; t < (listed + 3) / 4 * 4; t += SNT) {
+      const float v = t < listed ? read_through(&list_v[t]) : 0.f;
+      cnt[t] = t < listed ? enc_f32(v) : 0u;
+      mass[t] = t < listed ? __expf((v - all.m) * inv_temp) : 0.f;
+    }
+    if (threadIdx.x == 0) thr[0] = thr[1] = 0;
     __syncthreads();
-    if (t < listed) {
+    for (int t = threadIdx.x; t < listed; t += SNT) {
+      const uint32_t e = cnt[t];
       int count = 0;
       float sum = 0.f;
       for (int j = 0; j < listed; j += 4) {
@@ -934,15 +882,15 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     }
     __syncthreads();
     plan.prefix_k = thr[0], plan.prefix_p = thr[1];
+    const uint32_t tau = plan.threshold();
+    for (int t = threadIdx.x; t < listed; t += SNT) {
+      if (cnt[t] < tau) continue;
+      const int i = read_through(&list_i[t]);
+      const float z = __fmaf_rn(read_through(&list_v[t]), inv_temp,
+                                gumbel(rng_bits(rowkey, rng_at(i))));
+      if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
+    }
   }
-  const uint32_t tau = plan.threshold();
-  Draw d;
-  each(listed, [&](int t, float v) {
-    if (enc_f32(v) < tau) return;
-    const int i = read_through(&list_i[t]);
-    const float z = __fmaf_rn(v, inv_temp, gumbel(rng_bits(rowkey, rng_at(i))));
-    if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
-  });
   block_best(d.best, d.best_i, part);
   if (threadIdx.x == 0) {
     out_tokens[row] = d.best_i;
@@ -966,12 +914,8 @@ __global__ __launch_bounds__(SNT) void sample_digit_kernel(
   Plan plan = plans[row];
   if (plan.by == 0) return;
   uint32_t* h = hist + row * hist_words + digit * 2 * DIGIT;
-  const VocabRow<T> r(logits + row * V, V);
-  const int piece = blockIdx.x % split;
-  const float inv_temp = 1.0f / temperature[row];
-  add_bins<T>(digit, cnt, mass, h, [&] {
-    fill_bins(r, piece * SNT, split * SNT, digit, plan, inv_temp, cnt, mass);
-  });
+  add_bins(VocabRow<T>(logits + row * V, V), blockIdx.x % split, split, digit,
+           plan, 1.0f / temperature[row], cnt, mass, h);
   if (!last_of_row(&state->arrived[digit], split)) return;
   read_bins<T>(digit, h, cnt, mass);
   walk_bins<SNT, T>(plan, cnt, mass, digit, top_k[row], lds);
@@ -1031,9 +975,7 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
       if (by_k || by_p) {
         Plan plan(cut_of<NT>(tops, NTOPS, by_k, by_p, k, p, inv_temp, sums, V, lds),
                   sums, p, by_k, by_p);
-        select_alone<NT, T>(plan, k, cnt, mass, lds, [&](int digit) {
-          fill_bins(r, 0, NT, digit, plan, inv_temp, cnt, mass);
-        });
+        select_alone<NT>(r, plan, k, inv_temp, cnt, mass, lds);
         tau = plan.threshold();
       }
       Draw pick;
