@@ -419,25 +419,34 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // so that a captured graph may replay it with longer contexts.  No stretch
   // under 128 keys (a round of the four waves) of the longest context that the
   // page table holds: there the merging launch costs more than the split gains
-  // (37 cached tokens: 16.8 us in 16 stretches, 6.8 in one).  Of contexts of up to
-  // 1024 it costs as much already from 512 blocks on (two per CU; before: 1024):
-  // 64 rows of 500 .. 1000, 32/8 heads of 64, 22.6 us in two, 19.8 in one; 64 of
-  // 12/2 heads of 128 19.0 in eight, 15.6 in four; 16 of 64/8 heads 20.3 in
-  // eight, 17.0 in four.  Longer and ragged ones end together with 1600 blocks
-  // (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 11 and 15: 82, 76, 76, 76,
-  // 78; 40 of 1100 .. 2048, 32/8, in 4 and 5: 50.2, 47.7), but more than ten
-  // stretches of a row only where that is needed for 1024 (20 rows of 3000 .. 8000,
-  // 28/4 heads, in 13 and 16: 43.6, 45.0), and from 512 rows and heads on with two
-  // (110 rows of 1000 .. 2000, 32/8 heads of 64, in one and two: 75.8, 74.6).
+  // (37 cached tokens: 16.8 us in 16 stretches, 6.8 in one).
+  //
+  // Contexts of up to 1024: up to 512 blocks (two per CU), more cost more in the
+  // merging launch than they give (64 of 12/2 heads of 128 19.0 us in eight, 15.6
+  // in four; 16 of 64/8 heads 20.3 in eight, 17.0 in four; 64 of 32/8 heads of 64,
+  // 500 .. 1000, 22.6 in two, 19.8 in one; 56 of 128 35.5, 36.5, 35.9, 38.0 in one to
+  // four).  Where less than half of the CUs have a second block the others wait for
+  // it: in three (33 rows of 500 .. 1000, 32/8 heads of 128, in one to four 30.4,
+  // 28.0, 26.7, 27.8; of 257 .. 1024 tokens and heads of 64 19.8, 19.5, 16.9, 17.8;
+  // of 300 .. 600 tokens 17.5, 18.9, 18.8, 19.6; 50 of 500 .. 1000 33.4, 34.8, 33.0,
+  // 35.7, of 450 .. 900 29.9, 32.2, 31.2, 33.4).
+  //
+  // Longer ones: 1024 blocks (25 rows of 1024 .. 2048, 32/8 heads of 128, in 5, 6,
+  // 8 and 10: 39.3, 41.4, 43.9, 44.3; 50 in 2, 3, 4 and 5: 67.9, 65.4, 69.1, 65.9;
+  // inputs of several layers in turn), but five stretches where four are 1024 to
+  // 1364 (33 rows of 2049 .. 8192 in 4, 5 and 6: 137, 130, 129; of 1024 .. 2048 53.1,
+  // 52.5, 53.1), and ten of the longest where seven or eight are 1024 to 1272
+  // (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 11 and 15: 82, 76, 76, 76, 78).
   const long base_blocks = B * Hk;
   const long most = (long)max_pages * page_size;
   int nsplit = 1;
   if (base_blocks < 1024) {
-    const long fill = (1024 + base_blocks - 1) / base_blocks;
     const long want =
-        most <= 1024 ? 512 / base_blocks
-        : base_blocks >= 512 ? fill
-                             : std::min(1600 / base_blocks, std::max(10L, fill));
+        most <= 1024 ? (most > 700 && base_blocks > 256 && base_blocks < 384
+                            ? 3 : 512 / base_blocks)
+        : base_blocks >= 256 && base_blocks <= 341 ? 5
+        : most > 4096 && base_blocks >= 128 && base_blocks < 160
+            ? 10 : (1024 + base_blocks - 1) / base_blocks;
     nsplit = (int)std::max<long>(
         1, std::min<long>({want, 16, (most + 127) / 128}));
   }
@@ -467,12 +476,14 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // of 64: 300 rows of 16, 40 keys 12.8 and 15.0, 300 keys 75.7 and 72.4, 128
   // rows 1000 keys 97.7 and 103), and where the page table holds short contexts
   // only (128 wide, 4 heads, 128 rows of 300 keys: 18.2 and 20.0).
-  // Values go past the caches where the rows may hold more than the 256 MB cache
-  // behind the L2s does, as the layers of a model do in turn: V, read once in whole
-  // rows, then leaves the cache's ways to K, whose lines two instructions read
-  // (128 rows of 257 .. 512, 32/8 heads of 128, 268 MB: 44.9 us and 37.6, K past
-  // the caches too 45.9; 256 rows of 700 .. 1000, 64/8 heads, 170 and 158; but two
-  // calls in turn on 64 rows of 500 .. 1000, 32/8 heads of 64, 132 MB: 22.5 and 24.5).
+  // Values go past the caches, read once in whole rows: that leaves the ways of the
+  // 256 MB cache behind the L2s to K, whose lines two instructions read (K past the
+  // caches too 45.9 us where V alone gave 37.6).  On inputs that no cache holds, as
+  // the layers of a model come in turn, it takes 3 to 8% less time at every size
+  // (128 rows of 257 .. 512, 32/8 heads of 128, 43.9 -> 41.2; 56 of 1024 .. 2048,
+  // 77.6 -> 72.3).  Small calls keep V in the caches for those who repeat them on
+  // the same tensors: up to 10% slower past them with two of up to 128 MiB in turn
+  // (128 to 192 MiB: 11% slower to 2% faster; 256 MiB: 10 to 17% faster).
   const bool once = B * most * Hk * D * 4 > (128L << 20);
   // Groups of two and three heads of 128 keep three blocks on a CU, which short
   // contexts need (300 rows of 16 groups of two, 5 keys: 28 us with two, 19.7

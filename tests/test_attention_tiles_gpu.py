@@ -675,3 +675,34 @@ def test_values_of_keys_that_a_nan_row_does_not_see(d, scale):
     got = grad_v(lse)
     assert torch.equal(got[bad + 1:], want[bad + 1:])
     assert torch.isnan(got[:bad + 1]).all()
+
+
+@pytest.mark.parametrize("rows,hk,most", [
+    (256, 1, 720), (257, 1, 704), (257, 1, 720), (383, 1, 1024), (384, 1, 1024),
+    (255, 1, 1040), (128, 2, 1040), (341, 1, 1040), (342, 1, 1040),
+    (64, 2, 4112), (53, 3, 4112), (160, 1, 4112)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_stretches(rows, hk, most, d):
+    """Both sides of the numbers of rows, and of tokens that the table holds,
+    at which a row is divided otherwise; contexts that end in each stretch."""
+    torch.manual_seed(17)
+    hq, page, scale = 4 * hk, 16, d ** -0.5
+    lens = [1 + (most - 1) * i // (rows - 1) for i in range(rows)]
+    pages = torch.randperm(40, device=DEV).int()      # shared by the rows
+    at = torch.randint(40, (rows, -(-most // page)), device=DEV)
+    table = pages[at]
+    k, v = (torch.randn(40, page, hk, d, device=DEV).bfloat16()
+            for _ in range(2))
+    q = torch.randn(rows, hq, d, device=DEV).bfloat16()
+    got = ops.paged_attention_decode(
+        q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+        scale)
+    for i in sorted({0, 1, rows // 3, rows // 2, rows - 2, rows - 1}):
+        n = lens[i]
+        kk = heads(k[table[i].long()].view(-1, hk, d)[:n].double(), hq)
+        vv = heads(v[table[i].long()].view(-1, hk, d)[:n].double(), hq)
+        want, _ = attend(q[i:i + 1].double(), kk, vv, n - 1, True, scale)
+        mass, _ = attend(q[i:i + 1].double(), kk, vv.abs(), n - 1, True, scale)
+        # weights have all their bits, the result is rounded once
+        bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
+        assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
