@@ -706,3 +706,99 @@ def test_decode_stretches(rows, hk, most, d):
         # weights have all their bits, the result is rounded once
         bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
         assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
+
+
+FORMS = ["plain", "extras", "negative", "zero", "large", "negative_large",
+         "infinite"]
+
+
+def form_of(what, d):
+    """Scale and, for the window kernel, further arguments of a form."""
+    scale = {"negative": -0.1, "zero": 0.0, "large": 2.0 ** 40,
+             "negative_large": -2.0 ** 40}.get(what, d ** -0.5)
+    return scale, dict(q_temp_coef=0.1, q_temp_every=16, chunk=96,
+                       out_scale=0.5) if what == "extras" else {}
+
+
+@pytest.mark.parametrize("what", FORMS)
+@pytest.mark.parametrize("hq,hk", [(8, 2), (4, 4), (7, 1)])
+def test_window_copies_of_a_batch(hq, hk, what):
+    """Heads of 128 with more blocks than run at a time have one buffer of
+    values: a batch many times over gives each copy the bits that it has alone,
+    with two, in every form that the tests above check there; and an infinite
+    entry of a sequence's last value row shows where that row is seen, beside
+    finite ones."""
+    torch.manual_seed(18)
+    d, page, window, keep, copies = 128, 16, 70, 3, 50
+    lens, hist = [1, 31, 33, 64, 65, 200, 7], [0, 5, 0, 300, 63, 0, 129]
+    need = [-(-(n + m) // page) for n, m in zip(lens, hist)]
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32, device=DEV)
+    pages = torch.randperm(sum(need), device=DEV).int()
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    rows = torch.randn(sum(need), page, 2 * hk * d, device=DEV).bfloat16()
+    n = sum(lens)
+    ends = torch.tensor(lens, device=DEV).cumsum(0) - 1
+    if what == "infinite":
+        for i, (x, m) in enumerate(zip(lens, hist)):
+            last = x + m - 1
+            rows[table[i, last // page].long(), last % page].view(2, hk, d)[
+                1, :, 5] = float("inf")
+    q = torch.randn(n, hq * d, device=DEV).bfloat16()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    pos = torch.cat([torch.arange(m, m + x, **i32)
+                     for x, m in zip(lens, hist)])
+    gate = torch.randn(n, hq, device=DEV).bfloat16()
+    sink = torch.randn(hq, device=DEV) * 3 if what == "extras" else None
+    scale, more = form_of(what, d)
+
+    def run(times):
+        many = lens * times
+        seq = torch.repeat_interleave(torch.arange(len(many), **i32),
+                                      torch.tensor(many, device=DEV))
+        return ops.seq.gqa_window_attention(
+            q.repeat(times, 1), rows, table.repeat(times, 1), seq,
+            pos.repeat(times), hq, hk, d, d, window, keep, None, None,
+            gate.repeat(times, 1) if what == "extras" else None, scale,
+            torch.bfloat16, tiles=ops.seq.attention_tiles(many, DEV),
+            sink=sink, **more).view(times, n, hq * d)
+    alone, got = run(1), run(copies)
+    # (bits: rows that do not see an infinite value weigh it with 0)
+    assert torch.equal(got.view(torch.int16),
+                       alone.view(torch.int16).expand(copies, -1, -1))
+    if what == "infinite":
+        seen = got[:, ends].view(copies, len(lens), hq, d)
+        assert (seen[..., 5] == float("inf")).all()
+        assert seen[..., [j for j in range(d) if j != 5]].isfinite().all()
+
+
+@pytest.mark.parametrize("what", [f for f in FORMS if f != "extras"])
+@pytest.mark.parametrize("hq,hk", [(8, 2), (4, 4), (7, 1)])
+def test_forward_copies_of_a_batch(hq, hk, what):
+    """The same for packed prompts, some of them behind cached keys."""
+    torch.manual_seed(19)
+    d, copies = 128, 60
+    lens, hist = [1, 31, 33, 64, 65, 200, 7], [0, 5, 0, 300, 63, 0, 129]
+    klens = [x + m for x, m in zip(lens, hist)]
+    n, nk = sum(lens), sum(klens)
+    q = torch.randn(n, hq, d, device=DEV).bfloat16()
+    k, v = (torch.randn(nk, hk, d, device=DEV).bfloat16() for _ in range(2))
+    if what == "infinite":
+        v[torch.tensor(klens, device=DEV).cumsum(0) - 1, :, 5] = float("inf")
+    ends = torch.tensor(lens, device=DEV).cumsum(0) - 1
+    scale, _ = form_of(what, d)
+
+    def run(times):
+        return ops.varlen_prefill_attention(
+            *(t.repeat(times, 1, 1) for t in (q, k, v)),
+            cu_of(lens * times).to(DEV), cu_of(klens * times).to(DEV), scale,
+            True).view(times, n, hq, d)
+    alone, got = run(1), run(copies)
+    assert torch.equal(got.view(torch.int16),
+                       alone.view(torch.int16).expand(copies, -1, -1, -1))
+    if what == "infinite":
+        seen = got[:, ends]
+        assert (seen[..., 5] == float("inf")).all()
+        assert seen[..., [j for j in range(d) if j != 5]].isfinite().all()
