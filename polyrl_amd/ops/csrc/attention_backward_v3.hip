@@ -60,11 +60,11 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
   const int G = Hq / Hk;
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
   const int t = item / nparts, part = (item + t) % nparts;
-  int seq, q0;
-  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, seq, q0))
+  RowTile tile;
+  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
     return;
-  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
-  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
+  const int q0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
+  const int kbeg = tile.kbeg, Lk = tile.Lk;
   const int qk_off = Lk - Lq;
 
   const int lane = threadIdx.x & 63;
@@ -240,11 +240,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
   const int t = item / nsplit, split = (item + t) % nsplit;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
-  int seq, t0;
-  if (!row_tile<true>(t, ntiles, tile_seq, tile_k0, cu_q, cu_k, nseq, seq, t0))
+  RowTile tile;
+  if (!row_tile<true>(t, ntiles, tile_seq, tile_k0, cu_q, cu_k, nseq, tile))
     return;
-  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
-  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
+  const int t0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
+  const int kbeg = tile.kbeg, Lk = tile.Lk;
   const int qk_off = Lk - Lq;
   if (t0 >= Lk) return;
 

@@ -72,11 +72,11 @@ void prefill_attn_kernel(
   // to tile, so that no die has only the short ones
   const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
   const int t = item / nparts, part = (item + t) % nparts;
-  int seq, q0;
-  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, seq, q0))
+  RowTile tile;
+  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
     return;
-  const int qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
-  const int kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
+  const int q0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
+  const int kbeg = tile.kbeg, Lk = tile.Lk;
   const int qk_off = Lk - Lq;                      // chunked-prefill alignment
 
   const int lane = threadIdx.x & 63;

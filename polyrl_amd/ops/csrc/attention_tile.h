@@ -240,7 +240,8 @@ DEV_INLINE int wave_total(int x) {
   return __builtin_amdgcn_readlane(x, 63);
 }
 
-// Row tile of block ``t`` of ``ntiles``; false past the last.
+// Row tile of block ``t`` of ``ntiles``, and its sequence's rows and keys; false
+// past the last.
 //
 // Of at most 64 sequences: in the order of their walks, longest first.  A causal
 // walk is as long as the row tile is late (EARLY: the walk over the query tiles
@@ -249,26 +250,50 @@ DEV_INLINE int wave_total(int x) {
 // 3500 .. 4096, 28/4 heads of 128, kept 1.3 of two waves a SIMD on average.
 // ``above(L)`` counts the tiles whose walk is longer than L tiles.  A table of as
 // many tiles as the sequences have is read at the place that this tile has in
-// the sequences' order, so that every entry is taken once, whatever it names.
+// the sequences' order, so that every entry is taken once, whatever it names (the
+// lengths are on their way meanwhile, in case it names this tile: one wait after
+// the other cost 64 sequences of 33 .. 128, 32/8 heads of 128, 95.8 -> 100.7 us).
 //
-// Tables of another length (of some of the tiles) and more sequences than lanes:
-// in the table's order, from the end where late tiles walk longest.
+// In the table's order, from the end where late tiles walk longest: tables of
+// another length (of some of the tiles), more sequences than lanes, and calls
+// whose blocks all start at once, no two on a CU, or whose walks are one tile
+// each, where order is worth less than the time to find it (backward of one
+// sequence of 300, 8/8 heads of 128: 25.8 us in the order of the walks, 25.1; 64
+// sequences of 17 .. 64, 16/4 heads of 64, 24.6 and 24.1; with the line at 512
+// blocks 8 of 63 .. 250, 32/8 heads of 128, would take 47.8 for 45.3).
+struct RowTile {
+  int seq, r0, qbeg, Lq, kbeg, Lk;
+
+  DEV_INLINE void lengths(const int* cu_q, const int* cu_k) {
+    qbeg = cu_q[seq], Lq = cu_q[seq + 1] - qbeg;
+    kbeg = cu_k[seq], Lk = cu_k[seq + 1] - kbeg;
+  }
+};
+
 template <bool EARLY>
 DEV_INLINE bool row_tile(int t, int ntiles, const int* tile_seq,
                          const int* tile_r0, const int* cu_q, const int* cu_k,
-                         int nseq, int& seq, int& r0) {
+                         int nseq, RowTile& at) {
+  auto in_order = [&] {
+    if (!find_tile(EARLY ? t : ntiles - 1 - t, tile_seq, tile_r0, cu_q, nseq,
+                   at.seq, at.r0))
+      return false;
+    at.lengths(cu_q, cu_k);
+    return true;
+  };
+  if (nseq > 64 ||
+      (tile_seq != nullptr && (gridDim.x <= 256 || ntiles <= nseq)))
+    return in_order();
   const int lane = threadIdx.x & 63;
   int n = 0, h = 0;                    // row tiles; key tiles before the first
-  if (nseq <= 64 && lane < nseq) {
+  if (lane < nseq) {
     const int lq = max(cu_q[lane + 1] - cu_q[lane], 0);
     n = (lq + ATILE - 1) / ATILE;
     if (!EARLY) h = max(cu_k[lane + 1] - cu_k[lane] - lq, 0) / ATILE;
   }
   auto above = [&](int L) { return wave_total(min(max(h + n - L, 0), n)); };
   const int total = above(0);
-  if (nseq > 64 || (tile_seq != nullptr && ntiles != total))
-    return find_tile(EARLY ? t : ntiles - 1 - t, tile_seq, tile_r0, cu_q, nseq,
-                     seq, r0);
+  if (tile_seq != nullptr && ntiles != total) return in_order();
   if (total <= t) return false;
   int lo = 0, hi = 1;
   while (above(hi) > t) lo = hi, hi *= 2;
@@ -278,20 +303,24 @@ DEV_INLINE bool row_tile(int t, int ntiles, const int* tile_seq,
     else hi = mid;
   }
   // of the sequences with a tile of this length, the one that t stands for
-  const int at = t - above(lo + 1);
+  const int which = t - above(lo + 1);
   const unsigned long long has = __ballot(h <= lo && lo < h + n);
   const int rank = __builtin_amdgcn_mbcnt_hi(
       (unsigned)(has >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has, 0));
   const unsigned long long me =
-      __ballot((has >> lane & 1) && rank == at);
-  seq = __ffsll((long long)me) - 1;
-  const int nth = EARLY ? __builtin_amdgcn_readlane(n, seq) - 1 - lo
-                        : lo - __builtin_amdgcn_readlane(h, seq);
-  r0 = nth * ATILE;
+      __ballot((has >> lane & 1) && rank == which);
+  at.seq = __ffsll((long long)me) - 1;
+  const int nth = EARLY ? __builtin_amdgcn_readlane(n, at.seq) - 1 - lo
+                        : lo - __builtin_amdgcn_readlane(h, at.seq);
+  at.r0 = nth * ATILE;
+  at.lengths(cu_q, cu_k);
   if (tile_seq != nullptr) {
-    const int i = wave_total(lane < seq ? n : 0) + nth;
-    seq = uniform(tile_seq[i]);
-    r0 = uniform(tile_r0[i]);
+    const int i = wave_total(lane < at.seq ? n : 0) + nth;
+    const int seq = uniform(tile_seq[i]), r0 = uniform(tile_r0[i]);
+    if (seq != at.seq || r0 != at.r0) {
+      at.seq = seq, at.r0 = r0;
+      at.lengths(cu_q, cu_k);
+    }
   }
   return true;
 }
