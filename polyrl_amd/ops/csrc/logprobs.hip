@@ -27,9 +27,8 @@ DEV_INLINE Word16 load16(const void* p) {
   return ONCE ? __builtin_nontemporal_load(w) : *w;
 }
 
-template <bool ONCE, typename T>
-DEV_INLINE void unpack16(const T* p, float (&v)[16 / sizeof(T)]) {
-  const Word16 w = load16<ONCE>(p);
+template <typename T>
+DEV_INLINE void unpack16(const Word16& w, float (&v)[16 / sizeof(T)]) {
 #pragma unroll
   for (int j = 0; j < (int)(16 / sizeof(T)); ++j)
     v[j] = __uint_as_float(sizeof(T) == 4 ? w[j % 4]
@@ -94,16 +93,23 @@ __global__ __launch_bounds__(NT) void gather_logprobs_kernel(
     constexpr bool ONCE = decltype(once)::value;
     int i = threadIdx.x;
     for (; i + (UN - 1) * NT < nvec; i += UN * NT) {
-      float v[UN][VEC];
+      Word16 w[UN];
 #pragma unroll
       for (int u = 0; u < UN; ++u)
-        unpack16<ONCE>(xv + (long)(i + u * NT) * VEC, v[u]);
+        w[u] = load16<ONCE>(xv + (long)(i + u * NT) * VEC);
+      // (else the first word is waited for before the others are on their way:
+      // 2000 x 32000 24.7 us for 23.5; past the caches it makes no difference)
+      if constexpr (!ONCE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < UN; ++u) a.add(v[u]);
+      for (int u = 0; u < UN; ++u) {
+        float v[VEC];
+        unpack16<T>(w[u], v);
+        a.add(v);
+      }
     }
     for (; i < nvec; i += NT) {
       float v[VEC];
-      unpack16<ONCE>(xv + (long)i * VEC, v);
+      unpack16<T>(load16<ONCE>(xv + (long)i * VEC), v);
       a.add(v);
     }
   };
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(1024) void gather_logprobs_bwd_kernel(
     const bf16_t* at = x + lead + (long)i * 8;
     float v[8];
     if (same) {
-      unpack16<ONCE>(at, v);
+      unpack16<bf16_t>(load16<ONCE>(at), v);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = bf2f(at[j]);
@@ -221,9 +227,13 @@ static void launch_gather(float* lp, float* lse, float* ent,
 }
 
 // Rows of logits that the 256 MB cache behind the L2s holds.  The rows that the
-// forward reads last stay there for the backward; the others, and where no
-// backward follows all, are read past the caches.  Measured, 4096 x 128256 forward
-// and backward: with 160 MB kept 542 us, 200 535, 240 534, 300 529, none 554.
+// forward reads last stay there for the backward; the others are read past the
+// caches.  Measured, 4096 x 128256 forward and backward: with 160 MB kept 542 us,
+// 200 535, 240 534, 300 529, none 554.  Where no backward follows, logits that fit
+// are read through the caches, which may hold them from the product that wrote
+// them (written and read, 1024 x 50257 bf16: 49 us, past the caches 58; 1 x 128256
+// fp32, read alone, 10.9 and 14.6), and larger ones past them (1023 x 151936, 310
+// MB: 142 us for 150; 4096 x 128256 504 for 562).
 static long cached_rows(const torch::Tensor& logits) {
   return (256L << 20) /
          std::max<long>(1, logits.size(1) * (long)logits.element_size());
@@ -270,12 +280,14 @@ void gather_logprobs(torch::Tensor out_lp, torch::Tensor out_ent,
   TORCH_CHECK(out_lp.dtype() == torch::kFloat32);
   float* lp = out_lp.data_ptr<float>();
   float* ent = want_entropy ? out_ent.data_ptr<float>() : nullptr;
+  const long kept =
+      logits.size(0) <= cached_rows(logits) ? logits.size(0) : 0;
   if (logits.dtype() == torch::kBFloat16) {
     (want_entropy ? launch_gather<bf16_t, true> : launch_gather<bf16_t, false>)(
-        lp, nullptr, ent, logits, labels, 0);
+        lp, nullptr, ent, logits, labels, kept);
   } else if (logits.dtype() == torch::kFloat32) {
     (want_entropy ? launch_gather<float, true> : launch_gather<float, false>)(
-        lp, nullptr, ent, logits, labels, 0);
+        lp, nullptr, ent, logits, labels, kept);
   } else {
     TORCH_CHECK(false, "gather_logprobs: dtype must be bf16 or fp32");
   }

@@ -611,7 +611,7 @@ def test_forward_many_tiles(hq, hk, d):
 
 
 @pytest.mark.parametrize("what", ["some", "turned", "one_of_them"])
-@pytest.mark.parametrize("nseq", [3, 66])
+@pytest.mark.parametrize("nseq", [3, 60, 66])
 @pytest.mark.parametrize("d", [64, 128])
 def test_tables_of_some_tiles(nseq, d, what):
     """A table names the tiles that are computed, in any order: rows of named
