@@ -154,10 +154,10 @@ __global__ __launch_bounds__(NT) void gather_logprobs_kernel(
 
 // ---------------------------------------------------- training backward
 // d lp / d logits = onehot(label) - softmax(logits); chain with dlp.
-// One streaming pass per row using the forward-saved logsumexp.  dx goes past the
-// caches, which keep the rows that the forward read last for as long as they are
-// needed; the logits too, where they are more than fits (ONCE).
-template <bool ONCE>
+// One streaming pass per row using the forward-saved logsumexp.  Large dx go past
+// the caches (DX_ONCE), which keep the rows that the forward read last for as long
+// as they are needed; the logits too, where they are more than fits (ONCE).
+template <bool ONCE, bool DX_ONCE>
 __global__ __launch_bounds__(1024) void gather_logprobs_bwd_kernel(
     bf16_t* __restrict__ dlogits,
     const bf16_t* __restrict__ logits,
@@ -188,9 +188,10 @@ __global__ __launch_bounds__(1024) void gather_logprobs_bwd_kernel(
     bf16x8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j) o.v[j] = f2bf(-g * __expf(v[j] - l));
-    __builtin_nontemporal_store(
-        __builtin_bit_cast(Word16, o),
-        reinterpret_cast<Word16*>(dx + lead + (long)i * 8));
+    const Word16 w = __builtin_bit_cast(Word16, o);
+    Word16* to = reinterpret_cast<Word16*>(dx + lead + (long)i * 8);
+    if (DX_ONCE) __builtin_nontemporal_store(w, to);
+    else *to = w;
   }
   // the numbers before the first and behind the last whole word
   const int rest = V - lead - n8 * 8;
@@ -262,9 +263,18 @@ torch::Tensor gather_logprobs_train_bwd(torch::Tensor logits,
   auto dlogits = torch::empty_like(logits);
   auto stream = at::hip::getCurrentHIPStream();
   if (N == 0) return dlogits;
-  auto kern = N > cached_rows(logits) ? gather_logprobs_bwd_kernel<true>
-                                      : gather_logprobs_bwd_kernel<false>;
-  kern<<<dim3(N), dim3(1024), 0, stream>>>(
+  // dx stays in the caches for its next reader where it fits there beside the
+  // logits (4096 x 5000, dx read again: 54 us, past the caches 60; 1000 x 50257 109
+  // and 120, but the call alone 54 and 51; 2000 x 32000, 128 MB, 134 and 146, alone
+  // 78 and 62; 1000 x 128256, 256 MB, 296 and 273, alone 153 and 126)
+  const long rows = cached_rows(logits);
+  auto kern = N > rows            ? gather_logprobs_bwd_kernel<true, true>
+              : N > rows * 7 / 16 ? gather_logprobs_bwd_kernel<false, true>
+                                  : gather_logprobs_bwd_kernel<false, false>;
+  // 1024 threads of rows that give each two words or more (of 16384 entries and
+  // more: 4096 x 20000 84 us with 1024, 88 with 256; 16000 x 10000 165 and 156,
+  // 4096 x 5000 28 and 26, 4096 x 500 16.4 and 11.4, forward and backward)
+  kern<<<dim3(N), dim3(V < 16384 ? 256 : 1024), 0, stream>>>(
       (bf16_t*)dlogits.data_ptr(), (const bf16_t*)logits.data_ptr(),
       labels.data_ptr<int64_t>(), lse.data_ptr<float>(),
       dlp.contiguous().data_ptr<float>(), V);

@@ -424,3 +424,31 @@ def test_sample_rows_of_every_kind(n, dtype):
         z = row / t + noise(seed, r, v)
         # (as above)
         assert z[got] >= z[sure].max() - 1e-3, (r, kind)
+
+
+@pytest.mark.parametrize("n,v", [(5, 16383), (3, 16384), (1100, 16385),
+                                 (896, 65536), (897, 65536), (2048, 65536),
+                                 (2049, 65536)])
+def test_logprobs_on_both_sides_of_the_caches(n, v):
+    """Rows that the gradient's blocks of 256 and of 1024 threads take, and
+    logits that the cache behind the L2s just holds, alone or with their
+    gradient, and just does not."""
+    x = torch.randn(n, v, generator=torch.Generator(DEV).manual_seed(7),
+                    device=DEV).bfloat16().requires_grad_()
+    lab = torch.arange(n, device=DEV) * 7 % v
+    dlp = torch.randn(n, device=DEV)
+    lp = ops.gather_logprobs_train(x, lab)
+    lp.backward(dlp)
+    assert torch.equal(ops.gather_logprobs(x.detach(), lab), lp)
+    for a in range(0, n, 256):
+        b = slice(a, min(a + 256, n))
+        want = torch.log_softmax(x.detach()[b].double(), -1)
+        at = want.gather(1, lab[b, None])
+        assert (lp[b].double() - at[:, 0]).abs().max() < 1e-5 * at.abs().max()
+        g = dlp[b, None].double()
+        dx = -g * want.exp()
+        dx.scatter_add_(1, lab[b, None], g)
+        # rounded once to bf16, the label's entry twice
+        tol = 2 ** -7 * dx.abs() + 1e-6
+        tol.scatter_add_(1, lab[b, None], 2 ** -8 * g.abs())
+        assert ((x.grad[b].double() - dx).abs() <= tol).all()
