@@ -274,7 +274,8 @@ torch::Tensor gather_logprobs_train_bwd(torch::Tensor logits,
   // 1024 threads of rows that give each two words or more (of 16384 entries and
   // more: 4096 x 20000 84 us with 1024, 88 with 256; 16000 x 10000 165 and 156,
   // 4096 x 5000 28 and 26, 4096 x 500 16.4 and 11.4, forward and backward)
-  kern<<<dim3(N), dim3(V < 16384 ? 256 : 1024), 0, stream>>>(
+  const int threads = V < 16384 ? 256 : 1024;
+  kern<<<dim3(N), dim3(threads), 0, stream>>>(
       (bf16_t*)dlogits.data_ptr(), (const bf16_t*)logits.data_ptr(),
       labels.data_ptr<int64_t>(), lse.data_ptr<float>(),
       dlp.contiguous().data_ptr<float>(), V);
