@@ -17,8 +17,9 @@
 // What bounds it: reading K and V once.  (With per-key dot products, shuffles
 // and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
 // at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
-// tokens, 32/8 heads of 128, 59.5 -> 45.2 us, 37.6 with V read past the caches
-// (5.6 TB/s); 33 rows of 1900 .. 8192, 28/4 heads, 264 -> 86.5 -> 82 us, 76 in ten stretches.
+// tokens, 32/8 heads of 128, 59.5 -> 45.2 us, with V read past the caches 41 (5.1
+// TB/s; on inputs that no cache holds 43.9 and 41.2); 33 rows of 1900 .. 8192, 28/4
+// heads, 264 -> 86.5 -> 82 us, 77 in ten stretches.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

@@ -11,7 +11,8 @@
 // 64: two buffers of both, 32 KiB, and no more than 128 registers, so that four
 // blocks run per CU.  Heads of 128: two of K and one of V, whose next tile is
 // on its way from the last value product to the next softmax (a second barrier
-// a tile), 48 KiB and 165 registers: three blocks.
+// a tile, where the next keys have to be there too), 48 KiB and 165 registers:
+// three blocks.
 //
 // Products.  Scores are computed as S^T = K Q^T with the queries held in
 // registers: a lane's accumulators are 16 keys of ONE row, so the softmax
@@ -30,9 +31,11 @@
 // holds no row still fetch the tiles (7% of the walks of 16 sequences of up to
 // 512 rows).  Measured, eight ragged prompts of 1200 .. 2048 tokens, 32/8 heads
 // of 64: 671 us a call with those and the tile table's trip through the host (50
-// us), 154 with tiles through registers and three blocks per CU, 138 now (780
-// TFLOP/s of live pairs); of 128: 283 in the sequences' order, 280, 243 now; two sequences of 3500 ..
-// 4096, 28/4 heads of 128, 323, 265, 222.  A maximum that may lag by 2^6 saves
+// us), 154 with tiles through registers and three blocks per CU, 141 now (757
+// TFLOP/s of live pairs); of 128: 283 in the sequences' order, 280, 243 now; two
+// sequences of 3500 .. 4096, 28/4 heads of 128, 323, 265, 222.  Up to 64 sequences
+// run in the order of their walks, more in the table's (as all did before: 100
+// prompts of 21 .. 80 take what they took).  A maximum that may lag by 2^6 saves
 // the rescaling in most tiles (5 to 7%), but then a row's largest weight is no
 // longer exactly 1 and takes part in the rounding to bf16: the error against 64
 // bits grows by 2 to 3% (2.03e-3 for 1.98e-3, rms, 1024 keys).
@@ -210,7 +213,8 @@ void prefill_attn_kernel(
       l_run += sum;
     }
     if (ONE_V) {
-      // this tile's values are there, the next keys may still be on their way
+      // this tile's values are there.  (The next keys need not be, but the barrier
+      // waits for them too: the compiler sees copies that write LDS.)
       if (more) wait_all_but<T::LOADS>();
       else wait_loads();
       __syncthreads();

@@ -24,7 +24,7 @@
 // walks the bins, and the draw over the kept set, whose last block merges.  Short
 // rows take the same steps in one launch, a block each.  (64 x 151936, T 0.7, k
 // 50, p 0.9: 52.8 us with plans and a merge in launches of their own, eight in all,
-// 28 now; top-p 0.95 alone 81 and 79; at a temperature of 0 33 and 17.)
+// 27 now; top-p 0.95 alone 70 and 64; at a temperature of 0 33 and 17.)
 //
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
@@ -33,8 +33,9 @@
 // nucleus ends above them.  (Total and bins add the same exp((x - m)/T), which
 // is exact near m however large m/T is; should rounding leave the bins short
 // of p all the same, the nucleus ends at the cut.)  All entries of 64 x 151936
-// (0.7, 50, 0.9) in LDS atomics took 73 us a digit; half of 1 - p in place of
-// 0.99 takes top-p 0.95 of 256 x 152064 from 229 to 254 us.
+// (0.7, 50, 0.9) in LDS atomics took 73 us a digit; half of 1 - p in place of 0.99
+// took 11% longer (top-p 0.95 of 256 x 152064, 229 and 254 us in the eight launches
+// of before, 157 now).
 //
 // What bounds it: integer multiplies of the generator (two 64-bit products a
 // number; a number's place in the sequence is the last one's plus a constant, kept
@@ -193,22 +194,6 @@ struct Sums {
       for (int j = 0; j < N; ++j)
         st += v[j] == -INFINITY ? 0.f : __expf((v[j] - m) * inv_temp);
     }
-  }
-  // relative to the larger maximum of the two
-  DEV_INLINE void merge(float om, float os, float ot, float inv_temp) {
-    const float c = fmaxf(m, om);
-    if (c == -INFINITY) {              // zeros, or NaN
-      s += os;
-      if (TEMP) st += ot;
-      return;
-    }
-    const float a = m == c ? 1.f : __expf(m - c);
-    const float b = om == c ? 1.f : __expf(om - c);
-    s = s * a + os * b;
-    if (TEMP) {
-      st = st * shift(m, c, inv_temp) + ot * shift(om, c, inv_temp);
-    }
-    m = c;
   }
   // the wave's, in every lane
   DEV_INLINE void wave(float inv_temp) {
@@ -1068,14 +1053,16 @@ static void launch_sample(torch::Tensor& out_tokens,
   // Rows in one launch, a block each, while that is no longer than the pieces and
   // their passes.  Without a filter: with few rows up to 16384 numbers (64 x 16000
   // bf16 12.1 us, in pieces 12.6; 64 x 32000 18.3 and 13.6), with a block for most
-  // CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768 (64 x 9000 31
-  // us, in pieces 70, 64 x 16000 33 and 53; 64 x 32000 37 and 26, but at a
-  // temperature of 0, where nothing is selected, 7.8 and 19).  What stays dearer
-  // than a block a row everywhere is the draw at a temperature of 0 without a
+  // CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768.  Pieces are
+  // quicker from there down to 24000 (fp32 9000) with both filters (64 x 24000 36.5
+  // us, in pieces 23, 64 x 16000 33 and 42; fp32 64 x 9000 39 and 25), but not with
+  // top-p 0.95 alone (64 x 24000 37 and 41, 256 x 32000 45 and 59, fp32 57 and 84)
+  // nor at a temperature of 0, where nothing is selected (9 and 20).  What stays
+  // dearer than a block a row everywhere is the draw at a temperature of 0 without a
   // filter from 16384 numbers on, 11.3 us for 8 to 10: the temperature is on the
   // device, and at 1 the pieces take 11.5 for 21.
   // A block of 1024 threads takes rows of more than one round of 256 words (64 x
-  // 9000 both filters 31 us, with 256 threads 37; 64 x 32000 37 and 72); where
+  // 9000 both filters 31 us, with 256 threads 37; 64 x 32000 38 and 72); where
   // there are more rows than CUs, 256 threads take them up to ten rounds (512 x
   // 9000 41 us, with 1024 threads 64).
   auto rows = [&](auto kern, int threads) {
@@ -1097,10 +1084,10 @@ static void launch_sample(torch::Tensor& out_tokens,
     }
     return;
   }
-  // pieces of a row: 1024 blocks in all (four per CU; 128 x 128256 without a
-  // filter takes 29.8 us with 768 blocks, 28.7 with 1024, 29.4 with 2048; 64 x
-  // 151936 with both filters 63, 55, 60, 62 with 512, 1024, 2048, 4096), none
-  // under two rounds of 256 words
+  // pieces of a row: 1024 blocks in all (four per CU; with 512, 768, 1024, 1536 and
+  // 2048 128 x 128256 without a filter takes 31.6, 30.5, 29.3, 29.5, 29.9 us, 64 x
+  // 151936 with both filters 29.3, 27.9, 27.6, 31.4, 36.9, with top-p 0.95 alone 69,
+  // 64, 64, 65, 77), none under two rounds of 256 words
   const int split = (int)std::max<long>(
       1, std::min<long>({64, (1024 + N - 1) / N,
                          words / (2 * SNT)}));

@@ -380,7 +380,7 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
 // into LDS (AttnTile::gather), buffers and blocks per CU as in
 // attention_prefill.hip.  Measured, eight prompts of 1200 .. 2048 tokens, window
 // 1024, 32/8 heads of 64: 547 us in the general kernel, 155 with tiles through
-// registers and three blocks per CU, 139 here (119 with no tile loaded after the
+// registers and three blocks per CU, 138 here (119 with no tile loaded after the
 // first); of 128: 270 and 243.  Row tiles run by their number: longest walk first
 // found from the tables, as attention_prefill.hip finds it from the lengths, took
 // 157 for 156 (windowed walks are alike).
@@ -580,7 +580,7 @@ void gqa_attn_tile_kernel(
       l_run += sum;
     }
     if (ONE_V) {
-      // this tile's values are there, the next keys may still be on their way
+      // this tile's values are there (and the next keys, see attention_prefill.hip)
       if (more) wait_all_but<T::LOADS>();
       else wait_loads();
       end_rows(vs_, ti);
@@ -770,7 +770,9 @@ void seq_gqa_window_attention_mfma(
     // One buffer of values costs a wait in the middle of a tile, which only a
     // third block per CU makes up for: two prompts of 200 .. 300, 32/8 heads of 128
     // (160 blocks), 15.1 us with one and 14.3 with two; six of 300 .. 500 (670) 29.9
-    // and 30.8; eight of 1200 .. 2048 (3400) 241 and 254.
+    // and 30.8; eight of 1200 .. 2048 (3400) 241 and 254.  Between 513 and 640 it
+    // depends on how unlike the walks are: 32 of 63 .. 250, 12/2 heads (534) 17.9
+    // and 19.9, eight of 251 .. 1000, 8/8 heads (616) 37 and 33.5.
     if (D == 64) launch(gqa_attn_tile_kernel<64, false>);
     else if (items <= 512) launch(gqa_attn_tile_kernel<128, false>);
     else launch(gqa_attn_tile_kernel<128, true>);
