@@ -6,20 +6,26 @@
 // A block serves one key/value head of one sequence (or a stretch of its
 // context) for all G query heads of the group; each of its four waves takes
 // 32 keys at a time, on its own: no barrier until the waves' results meet.
-//   * S^T = K Q^T on v_mfma_f32_16x16x32_bf16, 16 keys x 16 head columns (G of
-//     them in use): a lane's K fragment is 16 bytes of one cached row, loaded
-//     straight from the page, and its accumulators are keys of ONE head, so
-//     maximum and sum take two lane exchanges per 32 keys.
+//   * S^T = K Q^T on v_mfma_f32_16x16x32_bf16, 16 keys x 16 columns: a lane's
+//     accumulators are keys of ONE head, so maximum and sum take two lane
+//     exchanges per 32 keys.  Large calls read K in whole rows past the caches and
+//     take the fragments from LDS; small ones, which the caches may hold, load
+//     them straight from the page, 64 bytes of a row at a time.
 //   * O^T += V^T P^T: V rows go through 8 KiB of LDS of the wave's own and come
 //     back turned (ds_read_b64_tr_b16); the weights are the operand as they
 //     stand in the accumulators.  They stay the 32-bit numbers they are: each
-//     is the sum of three bf16 numbers, and all three are multiplied.
-// What bounds it: reading K and V once.  (With per-key dot products, shuffles
-// and exponentials on the vector units the kernel was bound by those: 1.4 TB/s
-// at seven heads a group, 4.1 at four.)  Measured: 128 rows of 257 .. 512
-// tokens, 32/8 heads of 128, 59.5 -> 45.2 us, with V read past the caches 41 (5.1
-// TB/s; on inputs that no cache holds 43.9 and 41.2); 33 rows of 1900 .. 8192, 28/4
-// heads, 264 -> 86.5 -> 82 us, 77 in ten stretches.
+//     is the sum of three bf16 numbers, and all three are multiplied, in columns
+//     that the heads leave free: one product for up to four heads, two for eight.
+// What bounds it: reading K and V once, at the rate that this order of pages and
+// heads reaches (the same loads alone, 128 rows of 257 .. 512 tokens, 32/8 heads of
+// 128: 35.7 us; 33 rows of 1900 .. 8192, 28/4: 59).  Loads of the next round ahead of
+// this one's products, and three blocks of large calls on a CU, change nothing
+// (38.2 and 68.0 us with, 38.6 and 68.4 without; both together 38.0 and 76).
+// Measured (inputs of three layers in turn): those 128 rows 41.2 us with K in 64-byte
+// pieces through the caches, 38.6 now (5.2 TB/s); those 33 rows 77.1, 68.5, of which
+// the merge's loads one after the other were 2.5.  (With per-key dot products,
+// shuffles and exponentials on the vector units it was bound by those: 1.4 TB/s at
+// seven heads a group, 4.1 at four.)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -42,9 +48,9 @@ DEV_INLINE float quad_sum(float x) {
   return half_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
 }
 
-// WAVES: of a SIMD, at least; ONCE: values are read past the caches
-template <int D, int WAVES, bool ONCE>
-__global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
+// FEW: four heads or less; ONCE: keys and values are read past the caches
+template <int D, bool FEW, bool ONCE>
+__global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
     bf16_t* __restrict__ out,              // (B, Hq, D)
     float* __restrict__ partial,           // (B, Hq, S, D+2) when nsplit>1
     const bf16_t* __restrict__ q,          // (B, Hq, D)
@@ -56,9 +62,12 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
     int nsplit) {
   typedef AttnTile<D> T;
   constexpr int KS = D / 32, DT = D / 16;
-  constexpr int RPI = 64 / T::GR;          // V rows of one load instruction
+  constexpr int RPI = 64 / T::GR;          // cache rows of one load instruction
   constexpr int NV = DEC_KEYS / RPI;
-  __shared__ __attribute__((aligned(16))) char lds[4][DEC_KEYS * D * 2];
+  constexpr int HC = FEW ? 4 : DEC_HEADS;  // columns of a part of the weights
+  // a wave's values, and at the end its sums; its keys
+  __shared__ __attribute__((aligned(16))) char lds[4][DEC_KEYS * D * 2],
+      keys[ONCE ? 4 : 1][ONCE ? DEC_KEYS * D * 2 : 16];
   __shared__ float ml[4][DEC_HEADS][2];
 
   const int b = blockIdx.x / (Hk * nsplit);
@@ -66,21 +75,43 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
   const int hk = rem / nsplit;
   const int sp = rem % nsplit;
   const int G = Hq / Hk;
-  const int L = context_lens[b];
+  const int L = max(context_lens[b], 0);
   // a stretch per block, in whole rounds of a wave
-  const int Lc = ((L + nsplit - 1) / nsplit + DEC_KEYS - 1) / DEC_KEYS *
-                 DEC_KEYS;
+  const int Lc = nsplit == 1 ? L : ((L + nsplit - 1) / nsplit + DEC_KEYS - 1) /
+                                       DEC_KEYS * DEC_KEYS;
   const int cbeg = sp * Lc;
   const int cend = min(cbeg + Lc, L);
   const int lane = threadIdx.x & 63;
   const int wid = wave_id();
   const int l15 = lane & 15, lhi = lane >> 4;
+  const int vrow = lane / T::GR, vcol = lane % T::GR;
 
-  // Q of head l15 (columns past the group repeat its last head)
+  // Cache rows of keys t0 + lane % 32.  The table is read before the row's length
+  // is known; an entry past the stretch may be anything, and the round's first key
+  // stands in for it.
+  const int* ptab = page_table + (long)b * max_pages;
+  const bool pow2 = (page_size & (page_size - 1)) == 0;
+  const int shift = 31 - __builtin_clz(page_size);
+  auto look_up = [&](int t0) {
+    const int t = t0 + (lane & 31);
+    return ptab[min(pow2 ? t >> shift : t / page_size, max_pages - 1)];
+  };
+  auto rows_of = [&](int page, int t0) {
+    const int t = t0 + (lane & 31);
+    const int slot =
+        page * page_size + (pow2 ? t & (page_size - 1) : t % page_size);
+    // (outside the choice: in it the first lane would be one past the stretch)
+    const int first = uniform(slot);
+    return t < cend ? slot : first;
+  };
+  int t0 = cbeg + wid * DEC_KEYS;
+  int page = max_pages > 0 ? look_up(t0) : 0;
+
+  // Q of this column's head (columns past the group repeat its last head)
   bf16x8_t qf[KS];
   {
     const bf16_t* qp = q + (long)b * ldq +
-                       (long)(hk * G + min(l15, G - 1)) * D + lhi * 8;
+                       (long)(hk * G + min(l15 % HC, G - 1)) * D + lhi * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
@@ -93,45 +124,73 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = {0.f, 0.f, 0.f, 0.f};
 
-  const long kv_stride = (long)Hk * D;
-  const int* ptab = page_table + (long)b * max_pages;
+  const unsigned row_bytes = (unsigned)(Hk * D) * 2;
   char* vs = lds[wid];
+  char* kt = keys[ONCE ? wid : 0];
   // turned reads of V: rows 4 * lhi + l15 / 4 (+16), columns 16 dt + ..
   const int ra = 4 * lhi + (l15 >> 2), rb = ra + 16;
   const int vg = (l15 & 3) >> 1;
-  const int va = ra * (2 * D) + ((vg ^ T::swz(ra)) << 4) + (l15 & 1) * 8;
-  const int vb = rb * (2 * D) + ((vg ^ T::swz(rb)) << 4) + (l15 & 1) * 8;
-  const int vrow = lane / T::GR, vcol = lane % T::GR;
+  int va = ra * (2 * D) + ((vg ^ T::swz(ra)) << 4) + (l15 & 1) * 8;
+  int vb = rb * (2 * D) + ((vg ^ T::swz(rb)) << 4) + (l15 & 1) * 8;
+  // rows of K: l15 (+16), numbers 32 ks + 8 lhi ..
+  int ka = l15 * (2 * D) + ((lhi ^ T::swz(l15)) << 4);
+  // whole rows to their places
+  int to = vrow * (2 * D) + ((vcol ^ T::swz(vrow)) << 4);
 
-  // cache row of key t0 + lane % 32 (keys past the stretch: its last)
-  auto slot_of = [&](int t0) {
-    const int t = min(t0 + (lane & 31), cend - 1);
-    const int pg = t / page_size;
-    return ptab[pg] * page_size + (t - pg * page_size);
-  };
-  int t0 = cbeg + wid * DEC_KEYS;
-  int slot = t0 < cend ? slot_of(t0) : 0;
-  for (; t0 < cend; t0 += 4 * DEC_KEYS) {
-    bf16x8_t kf[2][KS];
-    i32x4_t vv[NV];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const bf16_t* kp = k_cache + __shfl(slot, n * 16 + l15, 64) * kv_stride +
-                         hk * D + lhi * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        kf[n][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 32);
-    }
+  // the round's rows into registers, and from there to the wave's LDS
+  auto load_rows = [&](i32x4_t (&w)[NV], const bf16_t* cache, int slot) {
+    const char* base =
+        reinterpret_cast<const char*>(cache + hk * D + vcol * 8);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const i32x4_t* vp = reinterpret_cast<const i32x4_t*>(
-          v_cache + __shfl(slot, i * RPI + vrow, 64) * kv_stride + hk * D +
-          vcol * 8);
-      vv[i] = ONCE ? __builtin_nontemporal_load(vp) : *vp;
+      const i32x4_t* p = reinterpret_cast<const i32x4_t*>(
+          base + (uint64_t)(unsigned)__shfl(slot, i * RPI + vrow, 64) *
+                     row_bytes);
+      w[i] = ONCE ? __builtin_nontemporal_load(p) : *p;
     }
-    if (t0 + 4 * DEC_KEYS < cend) slot = slot_of(t0 + 4 * DEC_KEYS);
+  };
+  auto store_rows = [&](char* tile, const i32x4_t (&w)[NV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      *reinterpret_cast<i32x4_t*>(tile + i * RPI * (2 * D) +
+                                  (to ^ (T::swz(i * RPI) << 4))) = w[i];
+    __builtin_amdgcn_wave_barrier();
+  };
 
-    // ---- S^T: 32 keys x 16 heads; this lane: head l15, keys 4 lhi + r -------
+  for (; t0 < cend; t0 += 4 * DEC_KEYS) {
+    // (new to the compiler: else the addresses derived from them live in
+    // registers through the loop)
+    asm volatile("" : "+v"(to), "+v"(ka), "+v"(va), "+v"(vb));
+    const int slot = rows_of(page, t0);
+    bf16x8_t kf[2][KS];
+    i32x4_t kk[NV], vv[NV];
+    if constexpr (ONCE) {
+      load_rows(kk, k_cache, slot);
+    } else {
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const char* kp =
+            reinterpret_cast<const char*>(k_cache + hk * D + lhi * 8) +
+            (uint64_t)(unsigned)__shfl(slot, n * 16 + l15, 64) * row_bytes;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          kf[n][ks] = *reinterpret_cast<const bf16x8_t*>(kp + ks * 64);
+      }
+    }
+    load_rows(vv, v_cache, slot);
+    if (t0 + 4 * DEC_KEYS < cend) page = look_up(t0 + 4 * DEC_KEYS);
+    if constexpr (ONCE) {
+      __builtin_amdgcn_sched_barrier(0);
+      store_rows(kt, kk);
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          kf[n][ks] = *reinterpret_cast<const bf16x8_t*>(
+              kt + n * 16 * (2 * D) + (ka ^ (ks << 6)));
+    }
+
+    // ---- S^T: 32 keys x 16 columns; this lane: column l15, keys 4 lhi + r ----
     f32x4_t s[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
@@ -159,49 +218,53 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[n][r]);
     const float mn = fmaxf(m_run, quad_max(mx));
-    const float alpha = exp2_hw(m_run - mn);
-    m_run = mn;
-    l_run *= alpha;
-    // weights as the sum of three bf16 numbers, the 24 bits of a 32-bit one in
+    if (__any(mn > m_run)) {
+      const float alpha = exp2_hw(m_run - mn);
+      m_run = mn;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
+    }
+    // Weights as the sum of three bf16 numbers, the 24 bits of a 32-bit one in
     // groups of eight.  None is 0 unless the weight is (the smallest bf16
-    // number stands in), so that an infinite value stays infinite.
-    i16x8_t w3[3];
+    // number stands in), so that an infinite value stays infinite.  The columns
+    // past the heads take the second and third part of the same heads; of eight
+    // heads the third part and, beside it, that smallest number make a second
+    // product.
+    i16x8_t w3[FEW ? 1 : 2];
 #pragma unroll
     for (int n = 0; n < 2; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = exp2_hw(s[n][r] - mn);
+        const float p = exp2_hw(s[n][r] - m_run);
         l_run += p;
-        float rest = p;
-        unsigned least = 0;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const unsigned bits = __float_as_uint(rest);
-          w3[i][4 * n + r] = (short)max(bits >> 16, least);
-          if (i == 0) least = min(bits, 1u);
-          rest -= __uint_as_float(bits & 0xFFFF0000u);
+        const unsigned b0 = __float_as_uint(p);
+        const float r1 = p - __uint_as_float(b0 & 0xFFFF0000u);
+        const unsigned b1 = __float_as_uint(r1);
+        const float r2 = r1 - __uint_as_float(b1 & 0xFFFF0000u);
+        const unsigned b2 = __float_as_uint(r2);
+        const unsigned least = min(b0, 1u);
+        if constexpr (FEW) {
+          const unsigned w = l15 < 4 ? b0 : l15 < 8 ? b1 : b2;
+          w3[0][4 * n + r] = (short)max(w >> 16, least);
+        } else {
+          w3[0][4 * n + r] = (short)max((l15 < 8 ? b0 : b1) >> 16, least);
+          w3[1][4 * n + r] =
+              (short)(l15 < 8 ? max(b2 >> 16, least) : least);
         }
       }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
 
     // ---- V rows into the wave's LDS, turned fragments back --------------------
-    // (zeros past the stretch: its last row, which stands in, need not be
-    // finite, and 0 * inf is NaN)
+    // (zeros past the stretch: the row that stands in need not be finite, and
+    // 0 * inf is NaN)
     if (t0 + DEC_KEYS > cend) {
 #pragma unroll
       for (int i = 0; i < NV; ++i)
         if (t0 + i * RPI + vrow >= cend) vv[i] = {0, 0, 0, 0};
     }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int r = i * RPI + vrow;
-      *reinterpret_cast<i32x4_t*>(vs + r * (2 * D) +
-                                  ((vcol ^ T::swz(r)) << 4)) = vv[i];
-    }
-    __builtin_amdgcn_wave_barrier();
+    store_rows(vs, vv);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const i16x4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -211,7 +274,7 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
       const bf16x8_t vt = __builtin_bit_cast(
           bf16x8_t, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < (FEW ? 1 : 2); ++i)
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             vt, __builtin_bit_cast(bf16x8_t, w3[i]), o[dt], 0, 0, 0);
     }
@@ -220,12 +283,12 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
   l_run = quad_sum(l_run);
 
   // ---- the four waves' shares meet in LDS ------------------------------------
-  if (l15 < G) {
+  {
     float* mine = reinterpret_cast<float*>(vs) + l15 * D + lhi * 4;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
       *reinterpret_cast<f32x4_t*>(mine + dt * 16) = o[dt];
-    if (lhi == 0) {
+    if (lhi == 0 && l15 < G) {
       ml[wid][l15][0] = m_run;
       ml[wid][l15][1] = l_run;
     }
@@ -240,8 +303,11 @@ __global__ __launch_bounds__(256, WAVES) void paged_decode_attn_kernel(
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float a = exp2_hw(ml[w][h][0] - gm);
+      const float* part = reinterpret_cast<const float*>(lds[w]) + i;
       l += ml[w][h][1] * a;
-      acc += reinterpret_cast<const float*>(lds[w])[i] * a;
+      float sum = part[0] + part[HC * D];
+      if (FEW) sum += part[2 * HC * D];
+      acc += sum * a;
     }
     const long row = (long)b * Hq + hk * G + h;
     if (nsplit == 1) {
@@ -391,15 +457,21 @@ __global__ void paged_decode_merge_kernel(
   const float w = __expf(m - wave_reduce_max(m));
   const float gl_sum = wave_reduce_sum(
       lane < nsplit ? base[lane * (D + 2) + D + 1] * w : 0.f);
-  float acc[EPL];
+  // (all stretches, 16 at most, on their way at once: 5.5 us one after the other, 3)
+  float acc[EPL], part[16][EPL];
+#pragma unroll
+  for (int sp = 0; sp < 16; ++sp)
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      part[sp][j] = sp < nsplit ? base[sp * (D + 2) + lane + j * 64] : 0.f;
 #pragma unroll
   for (int j = 0; j < EPL; ++j) acc[j] = 0.f;
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const float* pp = base + sp * (D + 2);
+#pragma unroll
+  for (int sp = 0; sp < 16; ++sp) {
     const float a = __shfl(w, sp, 64);
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
-      acc[j] += pp[lane + j * 64] * a;
+      if (sp < nsplit) acc[j] += part[sp][j] * a;
   }
   const float inv = (gl_sum > 0.f) ? 1.0f / gl_sum : 0.f;
 #pragma unroll
@@ -419,33 +491,37 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // Context split: from the sizes alone, not from the lengths on the device,
   // so that a captured graph may replay it with longer contexts.  No stretch
   // under 128 keys (a round of the four waves) of the longest context that the
-  // page table holds: there the merging launch costs more than the split gains
-  // (37 cached tokens: 16.8 us in 16 stretches, 6.8 in one).
+  // page table holds.
   //
-  // Contexts of up to 1024: up to 512 blocks (two per CU), more cost more in the
-  // merging launch than they give (64 of 12/2 heads of 128 19.0 us in eight, 15.6
-  // in four; 16 of 64/8 heads 20.3 in eight, 17.0 in four; 64 of 32/8 heads of 64,
-  // 500 .. 1000, 22.6 in two, 19.8 in one; 56 of 128 35.5, 36.5, 35.9, 38.0 in one to
-  // four).  Where less than half of the CUs have a second block the others wait for
-  // it: in three (33 rows of 500 .. 1000, 32/8 heads of 128, in one to four 30.4,
-  // 28.0, 26.7, 27.8; of 257 .. 1024 tokens and heads of 64 19.8, 19.5, 16.9, 17.8;
-  // of 300 .. 600 tokens 17.5, 18.9, 18.8, 19.6; 50 of 500 .. 1000 33.4, 34.8, 33.0,
-  // 35.7, of 450 .. 900 29.9, 32.2, 31.2, 33.4).
+  // Contexts of up to 1024 are divided where the blocks leave half of the CUs
+  // idle, but not up to 384: a second launch costs as much (us in a graph, rows of
+  // 2/3 of the longest and more; 8 rows of 32/8 heads of 128, up to 256 in one and
+  // two stretches 7.0 and 8.5, 384 in one and three 9.0 and 8.9, 512 in one and four
+  // 10.7 and 9.3, 1024 in one, four and eight 16.3, 12.2, 12.4; 16 rows 7.9 and 9.7, 9.4
+  // and 11.3, 11.0 and 12.0, 16.7, 17.0, 16.9; 24 rows 1024 in one and two 19.8 and
+  // 22.9).  Where less than half of the CUs have a second block the others wait for
+  // it: heads of 128 in three (33 rows of 682 .. 1024, 32/8 heads, 31.9, 30.6, 29.2 in
+  // one to three; of 512 .. 768 24.1, 23.2, 21.9; heads of 64 13.7, 18.4, 17.4).
   //
   // Longer ones: 1024 blocks (25 rows of 1024 .. 2048, 32/8 heads of 128, in 5, 6,
-  // 8 and 10: 39.3, 41.4, 43.9, 44.3; 50 in 2, 3, 4 and 5: 67.9, 65.4, 69.1, 65.9;
-  // inputs of several layers in turn), but five stretches where four are 1024 to
-  // 1364 (33 rows of 2049 .. 8192 in 4, 5 and 6: 137, 130, 129; of 1024 .. 2048 53.1,
-  // 52.5, 53.1), and ten of the longest where seven or eight are 1024 to 1272
-  // (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 11 and 15: 82, 76, 76, 76, 78).
+  // 8 and 10: 34.8, 35.4, 37.4, 38.3), but ten of the longest where seven or eight
+  // are 1024 to 1272 (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 12: 72.6, 70.0,
+  // 68.5, 69.5).  From 256 rows and heads on an odd number, which turns the
+  // stretches of a row from die to die: five (33 rows of 2049 .. 8192, 32/8 heads of
+  // 128, in 4, 5, 6: 127, 121, 120; 64 of 2000 .. 4096, heads of 64, in 1 to 6: 85, 89,
+  // 77, 85, 75, 77; 100 of 1500 .. 3000 102, 96, 84, 94, 84, 87), of heads of 128 three
+  // where five are too many (56 of 1024 .. 2048 in 2 to 5: 68.0, 65.0, 67.2, 65.1; 90
+  // of 2000 .. 4096 194, 192, 196, 194).
   const long base_blocks = B * Hk;
   const long most = (long)max_pages * page_size;
   int nsplit = 1;
-  if (base_blocks < 1024) {
+  if (most > 384 && base_blocks < 1024) {
     const long want =
-        most <= 1024 ? (most > 700 && base_blocks > 256 && base_blocks < 384
-                            ? 3 : 512 / base_blocks)
-        : base_blocks >= 256 && base_blocks <= 341 ? 5
+        most <= 1024
+            ? (base_blocks < 128 ? 512 / base_blocks
+               : D == 128 && most > 700 && base_blocks > 256 &&
+                         base_blocks < 384 ? 3 : 1)
+        : base_blocks >= 256 ? (D == 64 || base_blocks <= 341 ? 5 : 3)
         : most > 4096 && base_blocks >= 128 && base_blocks < 160
             ? 10 : (1024 + base_blocks - 1) / base_blocks;
     nsplit = (int)std::max<long>(
@@ -477,27 +553,21 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // of 64: 300 rows of 16, 40 keys 12.8 and 15.0, 300 keys 75.7 and 72.4, 128
   // rows 1000 keys 97.7 and 103), and where the page table holds short contexts
   // only (128 wide, 4 heads, 128 rows of 300 keys: 18.2 and 20.0).
-  // Values go past the caches, read once in whole rows: that leaves the ways of the
-  // 256 MB cache behind the L2s to K, whose lines two instructions read (K past the
-  // caches too 45.9 us where V alone gave 37.6).  On inputs that no cache holds, as
-  // the layers of a model come in turn, it takes 3 to 8% less time at every size
-  // (128 rows of 257 .. 512, 32/8 heads of 128, 43.9 -> 41.2; 56 of 1024 .. 2048,
-  // 77.6 -> 72.3).  Small calls keep V in the caches for those who repeat them on
-  // the same tensors: up to 10% slower past them with two of up to 128 MiB in turn
-  // (128 to 192 MiB: 11% slower to 2% faster; 256 MiB: 10 to 17% faster).
+  // Keys and values go past the caches, read once in whole rows: on inputs that no
+  // cache holds, as the layers of a model come in turn, that is the faster the
+  // larger the call (128 rows of 257 .. 512, 32/8 heads of 128, 40.4 us with K
+  // through the caches in pieces of rows, 44.1 in whole rows, 38.6 past them; 56 of
+  // 1024 .. 2048 69.8, 74.6, 65.0; 64 of 257 .. 1024, 64/8 heads, 33.9 and 35.7).  Small
+  // calls keep both in the caches for those who repeat them on the same tensors.
   const bool once = B * most * Hk * D * 4 > (128L << 20);
-  // Groups of two and three heads of 128 keep three blocks on a CU, which short
-  // contexts need (300 rows of 16 groups of two, 5 keys: 28 us with two, 19.7
-  // with three); at larger groups the registers that this takes cost more (32
-  // rows of 8000 keys, 28/4 heads: 106 and 110 us).
   if (G == 1 && (base_blocks >= 2048 || most <= (D == 128 ? 512 : 64)))
     args(paged_decode_attn_one_kernel<D>);
-  else if (D == 128 && G <= 3)
-    once ? args(paged_decode_attn_kernel<D, 3, true>)
-         : args(paged_decode_attn_kernel<D, 3, false>);
+  else if (G <= 4)
+    once ? args(paged_decode_attn_kernel<D, true, true>)
+         : args(paged_decode_attn_kernel<D, true, false>);
   else
-    once ? args(paged_decode_attn_kernel<D, 1, true>)
-         : args(paged_decode_attn_kernel<D, 1, false>);
+    once ? args(paged_decode_attn_kernel<D, false, true>)
+         : args(paged_decode_attn_kernel<D, false, false>);
 }
 
 void paged_attention_decode(torch::Tensor out, torch::Tensor q,

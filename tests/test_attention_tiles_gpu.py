@@ -708,6 +708,52 @@ def test_decode_stretches(rows, hk, most, d):
         assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
 
 
+@pytest.mark.parametrize("rows,hk,most", [
+    (8, 1, 384), (8, 1, 400), (127, 1, 400), (128, 1, 1024), (255, 1, 2064),
+    (256, 1, 2064), (342, 1, 1040), (85, 12, 1040), (128, 8, 1040)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_divided_or_not(rows, hk, most, d):
+    """Both sides of the lines from which on rows are divided at all, and among
+    an odd number of blocks."""
+    test_decode_stretches(rows, hk, most, d)
+
+
+@pytest.mark.parametrize("page", [1, 12, 16])
+@pytest.mark.parametrize("group", [1, 4, 5, 8])
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_past_the_caches(d, group, page):
+    """Tables that could hold more than the caches do, whose entries past the
+    contexts name no page: keys go through LDS, and the weights' parts take the
+    columns that the heads leave free."""
+    torch.manual_seed(18)
+    lens, hk, scale = [1, 32, 33, 161, 640], 4, d ** -0.5
+    hq = group * hk
+    wide = (128 << 20) // (len(lens) * page * hk * d * 4) + 1
+    need = [-(-n // page) for n in lens]
+    table = torch.full((len(lens), wide), -(1 << 30), dtype=torch.int32,
+                       device=DEV)
+    pages = torch.randperm(sum(need), device=DEV).int()
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = pages[at:at + n]
+        at += n
+    k, v = (torch.randn(sum(need), page, hk, d, device=DEV).bfloat16()
+            for _ in range(2))
+    q = torch.randn(len(lens), hq, d, device=DEV).bfloat16()
+    got = ops.paged_attention_decode(
+        q, k, v, table, torch.tensor(lens, dtype=torch.int32, device=DEV),
+        scale)
+    for i, n in enumerate(lens):
+        rows = table[i, :need[i]].long()
+        kk = heads(k[rows].view(-1, hk, d)[:n].double(), hq)
+        vv = heads(v[rows].view(-1, hk, d)[:n].double(), hq)
+        want, _ = attend(q[i:i + 1].double(), kk, vv, n - 1, True, scale)
+        mass, _ = attend(q[i:i + 1].double(), kk, vv.abs(), n - 1, True, scale)
+        # weights have all their bits, the result is rounded once
+        bound = 2 ** -8 * want.abs() + 2 ** -14 * mass
+        assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
+
+
 FORMS = ["plain", "extras", "negative", "zero", "large", "negative_large",
          "infinite"]
 
