@@ -37,17 +37,20 @@
 // took 11% longer (top-p 0.95 of 256 x 152064, 229 and 254 us in the eight launches
 // of before, 157 now).
 //
-// What bounds it: integer multiplies of the generator (two 64-bit products a
-// number; a number's place in the sequence is the last one's plus a constant, kept
-// from the compiler, which would multiply).  Vector instructions are 88% of the
-// cycles, 250 a word of eight numbers and as many again a wave for the exchange
-// of its lanes, which goes by DPP (128 x 128256 at temperature 1: 33.1 us with a
-// product for the place and exchanges through LDS, 28.7 now; each lane's most
-// promising number of the first word first, as a bound, took 29.4).  The two
-// logarithms of a number's noise are only taken where its 24 random bits can beat
-// the wave's best so far: z > best means u > exp(-exp(x/T - best)), one threshold
-// per 16-byte word of logits from the word's largest, with a margin far above the
-// rounding of either side.
+// What bounds it: vector instructions, most of them the generator's integer
+// multiplies (two 64-bit products a number; a number's place in the sequence is
+// the last one's plus a constant, kept from the compiler, which would multiply; of
+// the second product the upper word alone).  The two logarithms of a number's noise
+// are only taken where its 24 random bits can beat the best so far: z > best means
+// u > exp(-exp(x/T - best)), one threshold per 16-byte word of logits from the
+// word's largest, with a margin far above the rounding of either side.  The best so
+// far is the block's: its waves raise a number in LDS, which only ever holds what
+// some entry has, so that whoever is late reads less and nobody waits; and the
+// first words, which know of none, take it from noise in seven instructions, less
+// its error.  (128 x 128256 at temperature 1: 33.1 us with a product for the place
+// and exchanges of a wave's lanes through LDS, 28.7 with each wave's own best, every
+// number of its first word by the full logarithms, 25.8 so in blocks of four waves,
+// 23.1 of sixteen; 256 x 32000, a block a row, 17.1 and 13.7.)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -58,21 +61,23 @@ DEV_INLINE uint32_t enc_f32(float x) {
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-DEV_INLINE uint64_t splitmix64(uint64_t z) {
+// The upper word of splitmix64(z) but for its lowest bit (the last step's z >> 31
+// reaches no other)
+DEV_INLINE uint32_t splitmix64_upper(uint64_t z) {
   z += 0x9e3779b97f4a7c15ull;
   z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
   z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-  return z ^ (z >> 31);
+  return (uint32_t)(z >> 32);
 }
 
-// 32 random bits of an entry, of which the upper 24 are used.  ``at``: the entry's
+// Random bits of an entry, of which the upper 24 are used.  ``at``: the entry's
 // place in the sequence, rng_at() of it or of another one plus the distance
 constexpr uint64_t RNG_STEP = 0xd1342543de82ef95ull;
 DEV_INLINE uint64_t rng_at(int i) {
   return (uint64_t)(int64_t)i * RNG_STEP + 0x2545f4914f6cdd1dull;
 }
 DEV_INLINE uint32_t rng_bits(uint64_t rowkey, uint64_t at) {
-  return (uint32_t)(splitmix64(rowkey ^ at) >> 32);
+  return splitmix64_upper(rowkey ^ at);
 }
 
 // Gumbel noise of 24 bits: u = (bits + 1) / 2^24.  The largest bits stand
@@ -82,6 +87,13 @@ DEV_INLINE uint32_t rng_bits(uint64_t rowkey, uint64_t at) {
 DEV_INLINE float gumbel(uint32_t bits) {
   const float u = ((float)(bits >> 8) + 1.0f) * (1.0f / 16777216.0f);
   return -__logf(fmaxf(-__logf(u), 0x1p-25f));
+}
+
+// The same noise within 1e-6 of itself and 1e-6, in seven instructions for thirty
+DEV_INLINE float gumbel_about(uint32_t bits) {
+  const float u = ((float)(bits >> 8) + 1.0f) * (1.0f / 16777216.0f);
+  const float l = -0.6931471805599453f * __builtin_amdgcn_logf(u);
+  return -0.6931471805599453f * __builtin_amdgcn_logf(fmaxf(l, 0x1p-25f));
 }
 
 constexpr int SNT = 256;              // threads of a block
@@ -206,10 +218,27 @@ struct Sums {
   }
 };
 
-// the draw of a thread, pruned by the wave's best
+DEV_INLINE float dec_f32(uint32_t e) {
+  return __uint_as_float(e & 0x80000000u ? e ^ 0x80000000u : ~e);
+}
+
+// The draw of a thread, pruned by the best that the block's waves know of: a number
+// in LDS that they raise and read in passing.
 struct Draw {
   float best = -INFINITY, wbest = -INFINITY;
   int best_i = 0;
+  uint32_t* known;                     // encoding of the block's best so far
+
+  DEV_INLINE explicit Draw(uint32_t* known_) : known(known_) {}
+  // before the block's waves start (a barrier is between)
+  DEV_INLINE static void start(uint32_t* known) {
+    if (threadIdx.x == 0) *known = enc_f32(-INFINITY);
+  }
+
+  DEV_INLINE void raise(float z) {
+    wbest = wave_largest(z);
+    if ((threadIdx.x & 63) == 0) atomicMax(known, enc_f32(wbest));
+  }
 
   // v: entries i0 .. of the row, c the largest; tau: encoding that an entry
   // must reach (0: all)
@@ -217,6 +246,7 @@ struct Draw {
   DEV_INLINE void add(const float (&v)[N], float c, int i0, int V,
                       uint64_t rowkey, float inv_temp, uint32_t tau) {
     if (tau != 0 && !__any(enc_f32(c) >= tau)) return;
+    wbest = fmaxf(wbest, dec_f32(*(volatile uint32_t*)known));
     uint32_t bits[N];
     {
       uint64_t at = rng_at(i0), step = RNG_STEP;
@@ -231,6 +261,14 @@ struct Draw {
     // is not positive, where c is no bound)
     uint32_t least = 0;
     if (inv_temp > 0.f) {
+      if (tau == 0 && __all(wbest == -INFINITY)) {
+        // the first words: what some entry certainly has
+        float z = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          z = fmaxf(z, __fmaf_rn(v[j], inv_temp, gumbel_about(bits[j])));
+        raise(z - (1e-4f + 1e-5f * fabsf(z)));
+      }
       const float u = __expf(-__expf(__fmaf_rn(c, inv_temp, -wbest)));
       least = (uint32_t)max((int)(u * (16777216.f * (1.f - 1e-5f))) - 2, 0) << 8;
     }
@@ -243,7 +281,7 @@ struct Draw {
       const float z = __fmaf_rn(v[j], inv_temp, gumbel(bits[j]));
       if (better(z, i0 + j, best, best_i)) best = z, best_i = i0 + j;
     }
-    wbest = wave_largest(best);
+    raise(fmaxf(best, wbest));
   }
 };
 
@@ -608,15 +646,15 @@ DEV_INLINE void write_row(int64_t* out_tokens, float* out_logprobs,
   }
 }
 
-template <typename T, int MODE>
-__global__ __launch_bounds__(SNT) void sample_pass_kernel(
+template <typename T, int MODE, int NT = SNT>
+__global__ __launch_bounds__(NT) void sample_pass_kernel(
     int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
     Share* __restrict__ share, float* __restrict__ tops,
     uint32_t* __restrict__ hist, int hist_words,
     const Plan* __restrict__ plans, const T* __restrict__ logits,
     const float* __restrict__ temperature, uint64_t seed,
     const long long* __restrict__ seed_ptr, int V, int split) {
-  __shared__ Share part[SNW];
+  __shared__ Share part[(NT / 64)];
   const long row = blockIdx.x / split;
   const int piece = blockIdx.x % split;
   if (seed_ptr != nullptr) seed = (uint64_t)*seed_ptr;
@@ -630,13 +668,16 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
   const uint32_t tau = MODE == 2 ? plans[row].threshold() : 0;
   if (MODE == 1) {                    // the bins and the state start at 0
     uint32_t* h = hist + row * hist_words;
-    for (int i = piece * SNT + threadIdx.x; i < hist_words; i += split * SNT)
+    for (int i = piece * NT + threadIdx.x; i < hist_words; i += split * NT)
       h[i] = 0;
   }
 
+  __shared__ uint32_t known;
+  Draw::start(&known);
+  __syncthreads();
   Sums<MODE == 1> sums;
-  Draw d;
-  walk<MODE, SNT>(r, piece * SNT, split * SNT, greedy, inv_temp, rowkey, tau, sums,
+  Draw d(&known);
+  walk<MODE, NT>(r, piece * NT, split * NT, greedy, inv_temp, rowkey, tau, sums,
              d);
   if (MODE == 1) {                    // largest of each 16 lanes
     float t = d.best;
@@ -651,8 +692,8 @@ __global__ __launch_bounds__(SNT) void sample_pass_kernel(
     part[threadIdx.x >> 6] = {sums.m, sums.s, sums.st, d.best, d.best_i, 0};
   __syncthreads();
   if (threadIdx.x < 64) {               // the waves' shares, each once
-    const Share o = part[threadIdx.x % SNW];
-    const bool one = threadIdx.x < SNW;
+    const Share o = part[threadIdx.x % (NT / 64)];
+    const bool one = threadIdx.x < (NT / 64);
     sums.m = o.m, sums.s = one ? o.s : 0.f, sums.st = one ? o.st : 0.f;
     if (MODE != 2) sums.wave(inv_temp);
     d.best = o.best, d.best_i = o.best_i;
@@ -921,17 +962,18 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     plan.prefix_k = thr[0], plan.prefix_p = thr[1];
   }
   const uint32_t tau = plan.threshold();
-  Draw d;
+  float best = -INFINITY;
+  int best_i = 0;
   each(listed, [&](int t, float v) {
     if (enc_f32(v) < tau) return;
     const int i = read_through(&list_i[t]);
     const float z = __fmaf_rn(v, inv_temp, gumbel(rng_bits(rowkey, rng_at(i))));
-    if (better(z, i, d.best, d.best_i)) d.best = z, d.best_i = i;
+    if (better(z, i, best, best_i)) best = z, best_i = i;
   });
-  block_best(d.best, d.best_i, part);
+  block_best(best, best_i, part);
   if (threadIdx.x == 0) {
-    out_tokens[row] = d.best_i;
-    out_logprobs[row] = (float)r.x[d.best_i] - (all.m + __logf(all.s));
+    out_tokens[row] = best_i;
+    out_logprobs[row] = (float)r.x[best_i] - (all.m + __logf(all.s));
     state->done = 1;
   }
 }
@@ -986,8 +1028,11 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 
+  __shared__ uint32_t known;
+  Draw::start(&known);
+  __syncthreads();
   Sums<FILTER> sums;
-  Draw d;
+  Draw d(&known);
   walk<FILTER ? 1 : 0, NT>(r, 0, NT, greedy, inv_temp, rowkey, 0u, sums, d);
   if (FILTER) {                       // largest of each 16 lanes
     float t = d.best;
@@ -1021,7 +1066,7 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
         });
         tau = plan.threshold();
       }
-      Draw pick;
+      Draw pick(&known);              // (the first walk did not raise it)
       Sums<false> none;
       walk<2, NT>(r, 0, NT, false, inv_temp, rowkey, tau, none, pick);
       wave_best(pick.best, pick.best_i);
@@ -1084,13 +1129,36 @@ static void launch_sample(torch::Tensor& out_tokens,
     }
     return;
   }
-  // pieces of a row: 1024 blocks in all (four per CU; with 512, 768, 1024, 1536 and
-  // 2048 128 x 128256 without a filter takes 31.6, 30.5, 29.3, 29.5, 29.9 us, 64 x
-  // 151936 with both filters 29.3, 27.9, 27.6, 31.4, 36.9, with top-p 0.95 alone 69,
-  // 64, 64, 65, 77), none under two rounds of 256 words
-  const int split = (int)std::max<long>(
-      1, std::min<long>({64, (1024 + N - 1) / N,
-                         words / (2 * SNT)}));
+  // Pieces of a row, 1024 threads a CU in all.  With a filter blocks of 256 (with 512,
+  // 768, 1024, 1536 and 2048 of them 64 x 151936 with both filters takes 29.3, 27.9,
+  // 27.6, 31.4, 36.9 us, with top-p 0.95 alone 69, 64, 64, 65, 77), none under two
+  // rounds of 256 words.  Without one the largest blocks, whose waves share what
+  // they know, that fill 7/8 of the chip or of the 2048 threads that a CU holds and
+  // have three rounds in two blocks (128 x 128256 in blocks of 256, 512 and 1024: 25.8,
+  // 24.5 and 23.1; 100 x 128256 in 1100, 500 and 500: 24.9, 22.3, 22.1, but in 300 of
+  // 1024 31.5; 200 x 128256 in 1200 of 256, 1000 of 512 and 200 of 1024 35.8, 33.3, 36.9; 100
+  // x 50257 in 1100 of 256, 500 of 512, 500 of 1024 16.0, 14.5, 16).
+  int nt = SNT, split = 0;
+  if (no_filter) {
+    const int most_blocks[][2] = {{1024, 256}, {1024, 512}, {512, 512},
+                                  {512, 1024}, {256, 1024}};
+    for (const auto& o : most_blocks) {
+      const long each = o[1] / N;
+      if (each < 1 || each > 64 || each * N * 8 < o[1] * 7L ||
+          words * 2 < each * o[0] * 3L)
+        continue;
+      nt = o[0], split = (int)each;
+      break;
+    }
+    if (split == 0 && N > 256) {
+      nt = 512;
+      split = (int)std::max<long>(
+          1, std::min<long>((1024 + N - 1) / N, words / 1024));
+    }
+  }
+  if (split == 0)
+    split = (int)std::max<long>(
+        1, std::min<long>({64, (1024 + N - 1) / N, words / (2 * SNT)}));
   const int digits = sizeof(T) == 2 ? 2 : 3;
   const int hist_words =
       no_filter ? 0 : digits * 2 * DIGIT + (int)sizeof(RowState) / 4;
@@ -1115,7 +1183,7 @@ static void launch_sample(torch::Tensor& out_tokens,
   const T* x = (const T*)logits.data_ptr();
   const float* temp = temperature.data_ptr<float>();
   TORCH_CHECK(N * split < (1L << 31), "too many rows");
-  const dim3 grid((unsigned)(N * split)), block(SNT);
+  const dim3 grid((unsigned)(N * split)), block(nt);
   const int* k = top_k.data_ptr<int>();
   auto pass = [&](auto kern) {
     kern<<<grid, block, 0, stream>>>(tokens, logprobs, share, tops, hist,
@@ -1123,7 +1191,9 @@ static void launch_sample(torch::Tensor& out_tokens,
                                      V, split);
   };
   if (no_filter) {
-    pass(sample_pass_kernel<T, 0>);
+    if (nt == 1024) pass(sample_pass_kernel<T, 0, 1024>);
+    else if (nt == 512) pass(sample_pass_kernel<T, 0, 512>);
+    else pass(sample_pass_kernel<T, 0>);
     sample_merge_kernel<T><<<dim3(N), dim3(64), 0, stream>>>(
         tokens, logprobs, share, x, V, split);
   } else {

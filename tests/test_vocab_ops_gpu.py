@@ -452,3 +452,35 @@ def test_logprobs_on_both_sides_of_the_caches(n, v):
         tol = 2 ** -7 * dx.abs() + 1e-6
         tol.scatter_add_(1, lab[b, None], 2 ** -8 * g.abs())
         assert ((x.grad[b].double() - dx).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v", [(64, 98305), (100, 33001), (128, 65537),
+                                 (180, 40003), (256, 65539), (257, 66001),
+                                 (700, 65540), (1030, 65537), (16, 128256)])
+def test_sample_block_sizes(n, v, dtype):
+    """Without a filter, over the numbers of rows at which blocks of 256, 512
+    and 1024 threads take the pieces: the draw is the filtered path's, which
+    has other pieces, entry by entry.  Rows of few possible entries, of one, of
+    large logits and of a temperature that is not positive among them."""
+    torch.manual_seed(21)
+    x = (torch.randn(n, v, device=DEV) * 3).to(dtype)
+    x[1, 100:] = -float("inf")
+    x[2, :] = -float("inf")
+    x[2, v - 1] = -5.0
+    x[3] *= 1000
+    x[4, 300:] -= 40
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    temp = full(0.9, torch.float32)
+    temp[5], temp[6], temp[7] = 0.0, -1.0, 1e-6
+    args = (x, temp, full(-1, torch.int32), full(1.0, torch.float32), 77)
+    tok, lp = ops.sample(*args, no_filter=True)
+    other, _ = ops.sample(*args, no_filter=False)
+    assert torch.equal(tok, other)
+    assert int(tok[2]) == v - 1 and int(tok[1]) < 100
+    want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+    assert ((lp.double() - want).abs() <= 1e-5 * (1 + want.abs())).all()
+    for r in (0, 1, 4, n - 1):
+        z = x[r].double().cpu() / float(temp[r]) + noise(77, r, v)
+        # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
+        assert z[int(tok[r])] >= z.max() - 1e-3
