@@ -51,17 +51,16 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
     const float* __restrict__ lse, const int* __restrict__ cu_q,
     const int* __restrict__ cu_k, const int* __restrict__ tile_seq,
     const int* __restrict__ tile_q0, int nseq, int ntiles, int nparts, int Hq,
-    int Hk, float scale, int causal, long ldq, long ldk, long ldv) {
+    int Hk, int G, float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   // two buffers of K and V each; at the end the waves' rows of the gradient
   __shared__ __attribute__((aligned(16))) char k0_s[T::BYTES], v0_s[T::BYTES],
       k1_s[T::BYTES], v1_s[T::BYTES];
 
-  const int G = Hq / Hk;
-  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
-  const int t = item / nparts, part = (item + t) % nparts;
+  const BlockItem item(Hk, nparts);
+  const int hk = item.head, part = item.part;
   RowTile tile;
-  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
+  if (!row_tile<false>(item.tile, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
     return;
   const int q0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
   const int kbeg = tile.kbeg, Lk = tile.Lk;
@@ -71,15 +70,16 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
   const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
   const int unit = part * 4 + wid;        // (row half, head)
-  const int wq0 = q0 + unit / G * 32;
+  const int half = (unit >= G) + (unit >= 2 * G);
+  const int wq0 = q0 + half * 32;
   const bool busy = unit < 2 * G && wq0 < Lq;
-  const int hq = busy ? hk * G + unit % G : hk * G;
+  const int hq = busy ? hk * G + unit - half * G : hk * G;
   const int row = wq0 + (lane & 31);
   const int qpos = causal ? qk_off + row : Lk;
 
   const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
   const int wend = busy ? seen : 0;
-  const int last_half = min(part * 4 + 3, 2 * G - 1) / G;
+  const int last_half = min(part * 4 + 3, 2 * G - 1) >= G;
   const int bend = causal
       ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
@@ -208,16 +208,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_bwd_dq_kernel(
     }
   __syncthreads();
   if (!busy) return;
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) {
-    const int at16 = lane + i * 64;
-    const int r = at16 / T::GR, g = at16 % T::GR;
-    if (wq0 + r < Lq)
-      *reinterpret_cast<bf16x8*>(
-          dq + (((long)qbeg + wq0 + r) * Hq + hq) * D + g * 8) =
-          *reinterpret_cast<const bf16x8*>(mine + r * (2 * D) +
-                                           ((g ^ T::swz(r)) << 4));
-  }
+  T::store32(mine, dq + (((long)qbeg + wq0) * Hq + hq) * D, (long)Hq * D,
+             Lq - wq0);
 }
 
 // ---------------------------------------------------------------- dK/dV
@@ -231,7 +223,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     const float* __restrict__ lse, const float* __restrict__ delta,
     const int* __restrict__ cu_q, const int* __restrict__ cu_k,
     const int* __restrict__ tile_seq, const int* __restrict__ tile_k0,
-    int nseq, int ntiles, int nsplit, long total_k, int Hq, int Hk,
+    int nseq, int ntiles, int nsplit, long total_k, int Hq, int Hk, int G,
     float scale, int causal, long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   constexpr bool V_LDS = D == 128;   // V does not fit beside the gradients
@@ -240,12 +232,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
   // log-sum-exp (in powers of two) and scale * delta of the rows
   __shared__ __attribute__((aligned(16))) float r0_s[2][ATILE], r1_s[2][ATILE];
 
-  const int G = Hq / Hk;
-  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
-  const int t = item / nsplit, split = (item + t) % nsplit;
+  const BlockItem item(Hk, nsplit);
+  const int hk = item.head, split = item.part;
   const int g0 = G * split / nsplit, g1 = G * (split + 1) / nsplit;
   RowTile tile;
-  if (!row_tile<true>(t, ntiles, tile_seq, tile_k0, cu_q, cu_k, nseq, tile))
+  if (!row_tile<true>(item.tile, ntiles, tile_seq, tile_k0, cu_q, cu_k, nseq, tile))
     return;
   const int t0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
   const int kbeg = tile.kbeg, Lk = tile.Lk;
@@ -525,7 +516,7 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
           (const bf16_t*)v.data_ptr(), (const bf16_t*)out.data_ptr(),
           (const bf16_t*)dout.data_ptr(), lse.data_ptr<float>(),
           cu_q.data_ptr<int>(), cu_k.data_ptr<int>(), t_seq.data_ptr<int>(),
-          t_q0.data_ptr<int>(), nseq, (int)ntiles, nparts, Hq, Hk, scale,
+          t_q0.data_ptr<int>(), nseq, (int)ntiles, nparts, Hq, Hk, G, scale,
           causal ? 1 : 0, q.stride(0), k.stride(0), v.stride(0));
   // Blocks of the dkv kernel are as long as their key is early and run longest
   // first, 512 at a time (two per CU).  For all to end together the longest may
@@ -560,7 +551,7 @@ static void launch_bwd(torch::Tensor& dq, torch::Tensor& dk,
       (const bf16_t*)v.data_ptr(), (const bf16_t*)dout.data_ptr(),
       lse.data_ptr<float>(), delta.data_ptr<float>(), cu_q.data_ptr<int>(),
       cu_k.data_ptr<int>(), t_seq.data_ptr<int>(), t_q0.data_ptr<int>(),
-      nseq, (int)ntiles, nsplit, total_k, Hq, Hk, scale, causal ? 1 : 0,
+      nseq, (int)ntiles, nsplit, total_k, Hq, Hk, G, scale, causal ? 1 : 0,
       q.stride(0), k.stride(0), v.stride(0));
   if (nsplit > 1) {
     const long n = total_k * Hk * D;

@@ -60,7 +60,8 @@ void prefill_attn_kernel(
     const int* __restrict__ cu_k,
     const int* __restrict__ tile_seq,  // (ntiles,) or null
     const int* __restrict__ tile_q0,   // (ntiles,) local first q row
-    int nseq, int ntiles, int nparts, int Hq, int Hk, float scale, int causal,
+    int nseq, int ntiles, int nparts, int Hq, int Hk, int G, float scale,
+    int causal,
     long ldq, long ldk, long ldv) {
   typedef AttnTile<D> T;
   // two buffers of K and V each; at the end the waves' rows of the output
@@ -68,15 +69,14 @@ void prefill_attn_kernel(
       k1_s[T::BYTES], vx_s[ONE_V ? 16 : T::BYTES];
   char* const v1_s = ONE_V ? v0_s : vx_s;
 
-  const int G = Hq / Hk;
   // Blocks go to the dies in turn (id % 8): with the key/value head innermost a
   // die has one head or few, and every die a share of every length.  The parts
   // of a tile are not equal (the last may have fewer heads): they turn from tile
   // to tile, so that no die has only the short ones
-  const int hk = blockIdx.x % Hk, item = blockIdx.x / Hk;
-  const int t = item / nparts, part = (item + t) % nparts;
+  const BlockItem item(Hk, nparts);
+  const int hk = item.head, part = item.part;
   RowTile tile;
-  if (!row_tile<false>(t, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
+  if (!row_tile<false>(item.tile, ntiles, tile_seq, tile_q0, cu_q, cu_k, nseq, tile))
     return;
   const int q0 = tile.r0, qbeg = tile.qbeg, Lq = tile.Lq;
   const int kbeg = tile.kbeg, Lk = tile.Lk;
@@ -86,8 +86,9 @@ void prefill_attn_kernel(
   const int wid = wave_id();
   constexpr int KS = D / 16, DT = D / 32;
   const int unit = part * 4 + wid;        // (row half, head)
-  const int hq = hk * G + unit % G;
-  const int wq0 = q0 + unit / G * 32;              // this wave's first row
+  const int half = (unit >= G) + (unit >= 2 * G);
+  const int hq = hk * G + unit - half * G;
+  const int wq0 = q0 + half * 32;                  // this wave's first row
   const bool busy = unit < 2 * G && wq0 < Lq;
   const int row = wq0 + (lane & 31);               // this lane's row
   const int qpos = causal ? qk_off + row : Lk;     // last key it sees
@@ -95,7 +96,7 @@ void prefill_attn_kernel(
   // keys that this wave and this block walk
   const int seen = causal ? min(Lk, qk_off + min(wq0 + 32, Lq)) : Lk;
   const int wend = busy ? seen : 0;
-  const int last_half = min(part * 4 + 3, 2 * G - 1) / G;
+  const int last_half = min(part * 4 + 3, 2 * G - 1) >= G;
   const int bend = causal
       ? min(Lk, qk_off + min(q0 + last_half * 32 + 32, Lq)) : Lk;
 
@@ -273,16 +274,8 @@ void prefill_attn_kernel(
   }
   __syncthreads();
   if (!busy) return;
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) {
-    const int at16 = lane + i * 64;
-    const int r = at16 / T::GR, g = at16 % T::GR;
-    if (wq0 + r < Lq)
-      *reinterpret_cast<bf16x8*>(
-          out + (((long)qbeg + wq0 + r) * Hq + hq) * D + g * 8) =
-          *reinterpret_cast<const bf16x8*>(mine + r * (2 * D) +
-                                           ((g ^ T::swz(r)) << 4));
-  }
+  T::store32(mine, out + (((long)qbeg + wq0) * Hq + hq) * D, (long)Hq * D,
+             Lq - wq0);
 }
 
 // tile_seq / tile_q0: the 64-row tiles of the packed rows to compute (all or some
@@ -339,7 +332,7 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
       cu_seqlens_q.data_ptr<int>(), cu_seqlens_k.data_ptr<int>(),
       table ? tile_seq.data_ptr<int>() : nullptr,
       table ? tile_q0.data_ptr<int>() : nullptr, nseq, (int)ntiles, nparts,
-      Hq, Hk, (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0),
+      Hq, Hk, Hq / Hk, (float)scale, causal ? 1 : 0, q.stride(0), k.stride(0),
       v.stride(0));
   HIP_CHECK_KERNEL();
 }

@@ -24,6 +24,7 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) int i32x4_t;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
 typedef __attribute__((ext_vector_type(4))) short i16x4_t;
 typedef __attribute__((ext_vector_type(8))) short i16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
@@ -86,6 +87,27 @@ struct AttnTile {
       __builtin_amdgcn_global_load_lds(
           (global_p)(from + start[r + i * (256 / GR)]), (lds_p)(to + i * 4096),
           16, 0, 0);
+  }
+
+  // 32 rows of a wave's own, laid out like a tile's, to rows [0, min(live, 32)) of
+  // memory: the buffer ends with the last one, and what is behind it is not written
+  DEV_INLINE static void store32(const char* rows, bf16_t* to, long ld,
+                                 int live) {
+    constexpr int RS = 64 / GR;         // rows of a step
+    const int ldb = (int)ld * 2;
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+        to, 0, live > 0 ? (min(live, 32) - 1) * ldb + 2 * D : 0, 0x00020000);
+    const int lane = threadIdx.x & 63, r = lane / GR, g = lane % GR;
+    const int from = r * (2 * D) + ((g ^ swz(r)) << 4);
+    int at = r * ldb + (g << 4);
+#pragma unroll
+    for (int i = 0; i < 32 / RS; ++i) {
+      __builtin_amdgcn_raw_buffer_store_b128(
+          *reinterpret_cast<const u32x4_t*>(rows + i * RS * (2 * D) +
+                                            (from ^ (swz(i * RS) << 4))),
+          out, at, 0, 0);
+      at += RS * ldb;
+    }
   }
 
   // zeros for this thread's granules of the rows from ``live`` on
@@ -253,6 +275,12 @@ DEV_INLINE int wave_total(int x) {
 // the sequences' order, so that every entry is taken once, whatever it names (the
 // lengths are on their way meanwhile, in case it names this tile: one wait after
 // the other cost 64 sequences of 33 .. 128, 32/8 heads of 128, 95.8 -> 100.7 us).
+// Up to 16 sequences the count is taken for 64 lengths at once, one a lane, five
+// instructions a sequence; of more a search by halves sums over the lanes ten times.
+// (With blocks that find their heads and parts without divisions, and rows written
+// by stores that end with the buffer, eight prompts of 1200 .. 2048, 32/8 heads of 64,
+// 143.8 -> 139.8 us; 16 sequences of 300 .. 512, 32/8 of 128, forward and backward 224.4
+// -> 221.1; one prompt of 512 14.9 -> 14.4.)
 //
 // In the table's order, from the end where late tiles walk longest: tables of
 // another length (of some of the tiles), more sequences than lanes, and calls
@@ -292,18 +320,47 @@ DEV_INLINE bool row_tile(int t, int ntiles, const int* tile_seq,
     if (!EARLY) h = max(cu_k[lane + 1] - cu_k[lane] - lq, 0) / ATILE;
   }
   auto above = [&](int L) { return wave_total(min(max(h + n - L, 0), n)); };
-  const int total = above(0);
-  if (tile_seq != nullptr && ntiles != total) return in_order();
-  if (total <= t) return false;
-  int lo = 0, hi = 1;
-  while (above(hi) > t) lo = hi, hi *= 2;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) / 2;
-    if (above(mid) > t) lo = mid;
-    else hi = mid;
+  int lo, longer, total;               // the walk's length less one; above(lo + 1)
+  if (nseq <= 16) {
+    // 64 lengths at a time, one a lane
+    for (int base = 0;; base += 64) {
+      int sum = 0;
+      for (int s = 0; s < nseq; s += 4)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int ns = __builtin_amdgcn_readlane(n, s + i);
+          const int end = __builtin_amdgcn_readlane(h, s + i) + ns;
+          sum += min(max(end - (base + lane), 0), ns);
+        }
+      if (base == 0) {
+        total = __builtin_amdgcn_readlane(sum, 0);
+        if (total <= t || (tile_seq != nullptr && ntiles != total)) break;
+      }
+      const unsigned long long more = __ballot(sum > t);
+      if (more == ~0ull) continue;
+      const int c = __popcll(more);
+      lo = base + c - 1;
+      longer = __builtin_amdgcn_readlane(sum, c);
+      break;
+    }
+    if (tile_seq != nullptr && ntiles != total) return in_order();
+    if (total <= t) return false;
+  } else {
+    total = above(0);
+    if (tile_seq != nullptr && ntiles != total) return in_order();
+    if (total <= t) return false;
+    lo = 0;
+    int hi = 1;
+    while (above(hi) > t) lo = hi, hi *= 2;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (above(mid) > t) lo = mid;
+      else hi = mid;
+    }
+    longer = above(lo + 1);
   }
   // of the sequences with a tile of this length, the one that t stands for
-  const int which = t - above(lo + 1);
+  const int which = t - longer;
   const unsigned long long has = __ballot(h <= lo && lo < h + n);
   const int rank = __builtin_amdgcn_mbcnt_hi(
       (unsigned)(has >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has, 0));
@@ -324,6 +381,27 @@ DEV_INLINE bool row_tile(int t, int ntiles, const int* tile_seq,
   }
   return true;
 }
+
+// id / n and id % n of uniform numbers (heads and parts are mostly powers of two)
+DEV_INLINE int split_id(int id, int n, int& rest) {
+  if ((n & (n - 1)) == 0) {
+    rest = id & (n - 1);
+    return id >> __builtin_ctz(n);
+  }
+  rest = (unsigned)id % (unsigned)n;
+  return (unsigned)id / (unsigned)n;
+}
+
+// Tile, part of it and key/value head of a block: the head innermost, and the
+// parts, which are not equal, turning from tile to tile
+struct BlockItem {
+  int tile, part, head;
+  DEV_INLINE BlockItem(int heads, int parts) {
+    int turn;
+    tile = split_id(split_id(blockIdx.x, heads, head), parts, turn);
+    split_id(turn + tile, parts, part);
+  }
+};
 
 // wave of the block, known to the compiler to be the same for all its lanes
 DEV_INLINE int wave_id() {

@@ -637,16 +637,7 @@ void gqa_attn_tile_kernel(
     }
   __syncthreads();
   if (!busy) return;
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) {
-    const int a = lane + i * 64;
-    const int r = a / T::GR, gr = a % T::GR;
-    if (w0 + r < cnt)
-      *reinterpret_cast<i32x4_t*>(out + (n0 + w0 + r) * ldo + (long)h * D +
-                                  gr * 8) =
-          *reinterpret_cast<const i32x4_t*>(mine + r * (2 * D) +
-                                            ((gr ^ T::swz(r)) << 4));
-  }
+  T::store32(mine, out + (n0 + w0) * ldo + (long)h * D, ldo, cnt - w0);
 }
 
 void gqa_attention_check(torch::Tensor out, torch::Tensor q,

@@ -754,6 +754,47 @@ def test_decode_past_the_caches(d, group, page):
         assert ((got[i:i + 1].double() - want).abs() <= bound).all(), n
 
 
+@pytest.mark.parametrize("count", [1, 15, 16, 17])
+@pytest.mark.parametrize("hist", [0, 130])
+def test_row_tiles_of_few_and_long_sequences(count, hist):
+    """Both sides of the number of sequences up to which a row tile is found 64
+    lengths at a time, walks on both sides of 64 and 128 tiles: every sequence's
+    rows and their gradients are those of a call of its own."""
+    torch.manual_seed(19)
+    hq, hk, d = 2, 1, 64
+    lens = ([4097, 1, 64, 65, 8200, 130, 4032, 4096, 63, 2, 200, 128, 129, 1000,
+             5, 77, 300])[:count]
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    cuk = torch.tensor([0] + [n + hist for n in lens]).cumsum(0).int()
+    q, do = (torch.randn(sum(lens), hq, d, device=DEV).bfloat16()
+             for _ in range(2))
+    k, v = (torch.randn(int(cuk[-1]), hk, d, device=DEV).bfloat16()
+            for _ in range(2))
+    out = ops.varlen_prefill_attention(q, k, v, cu.to(DEV), cuk.to(DEV),
+                                       d ** -0.5, causal=True)
+    grads = []
+    if hist == 0:
+        x = [t.clone().requires_grad_() for t in (q, k, v)]
+        y = ops.flash_attn_varlen(*x, cu.to(DEV), d ** -0.5, causal=True)
+        assert torch.equal(y, out)
+        grads = torch.autograd.grad(y, x, do)
+    for i, n in enumerate(lens):
+        a, b = slice(int(cu[i]), int(cu[i + 1])), slice(int(cuk[i]),
+                                                        int(cuk[i + 1]))
+        one = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+        onek = torch.tensor([0, n + hist], dtype=torch.int32, device=DEV)
+        assert torch.equal(out[a], ops.varlen_prefill_attention(
+            q[a], k[b], v[b], one, onek, d ** -0.5, causal=True)), i
+        if grads:
+            x = [t[a].clone().requires_grad_() for t in (q, k, v)]
+            y = ops.flash_attn_varlen(*x, one, d ** -0.5, causal=True)
+            own = torch.autograd.grad(y, x, do[a])
+            assert torch.equal(grads[0][a], own[0]), i
+            # (heads are divided otherwise: 32-bit sums in another order)
+            for g, w in zip(grads[1:], own[1:]):
+                assert (g[a] - w).abs().max() <= 2 ** -7 * w.abs().max(), i
+
+
 FORMS = ["plain", "extras", "negative", "zero", "large", "negative_large",
          "infinite"]
 
