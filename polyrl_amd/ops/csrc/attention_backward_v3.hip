@@ -320,6 +320,31 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
     at.renew();
     f32x16_t s, dp;
     bf16x8_t p[2], ds[2];
+    const int r0 = qh * 32 + 4 * (lane >> 5);
+    // The weights need no dO: at 64 they come before the barrier that waits for it
+    // (8 sequences of 300 .. 1024, 32/8 heads, forward and backward 163.4 us behind
+    // it, 160.3 before), at 128 their exponentials do better beside dP (2 of 3500 ..
+    // 4096, 28/4 heads, 986 and 996).
+    auto weights = [&] {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 le = *reinterpret_cast<const float4*>(&row_s[0][r0 + 8 * i]);
+        const float l4[4] = {le.x, le.y, le.z, le.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          s[4 * i + t] = __builtin_fmaf(s[4 * i + t], s2, -l4[t]);
+      }
+      // rows before this lane's key (compared with literals), whatever their
+      // log-sum-exp: it may be NaN
+      if (causal && qk_off + wq0 < wk0 + 31) {
+        const int border = key - (qk_off + wq0) - 4 * (lane >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) < border) s[r] = -INFINITY;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = exp2_hw(s[r]);
+    };
     if (work) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = 0.f;
@@ -334,6 +359,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         SCHED_LDS(1);
       }
       SCHED_MFMA(3);
+      if constexpr (D == 64) weights();
     }
     wait_loads();
     __syncthreads();
@@ -358,23 +384,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
         SCHED_LDS(PER);
       }
       SCHED_MFMA(3);
-      const int r0 = qh * 32 + 4 * (lane >> 5);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 le = *reinterpret_cast<const float4*>(&row_s[0][r0 + 8 * i]);
-        const float l4[4] = {le.x, le.y, le.z, le.w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          s[4 * i + t] = __builtin_fmaf(s[4 * i + t], s2, -l4[t]);
-      }
-      // rows before this lane's key (compared with literals), whatever their
-      // log-sum-exp: it may be NaN
-      if (causal && qk_off + wq0 < wk0 + 31) {
-        const int border = key - (qk_off + wq0) - 4 * (lane >> 5);
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (8 * (r >> 2) + (r & 3) < border) s[r] = -INFINITY;
-      }
+      if constexpr (D == 128) weights();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float4 de = *reinterpret_cast<const float4*>(&row_s[1][r0 + 8 * i]);
@@ -382,9 +392,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkv_kernel(
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int r = 4 * i + t;
-          const float w = exp2_hw(s[r]);
-          s[r] = w;
-          dp[r] = w * __builtin_fmaf(dp[r], scale, -d4[t]);
+          dp[r] = s[r] * __builtin_fmaf(dp[r], scale, -d4[t]);
         }
       }
 #pragma unroll
