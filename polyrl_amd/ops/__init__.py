@@ -71,6 +71,24 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return ref.silu_mul(gate, up)
 
 
+def linear_swiglu_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_swiglu`` has a kernel for these operands."""
+    return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and x.is_contiguous()
+            and w.is_contiguous() and w.shape[0] % 256 == 0
+            and 0 < w.shape[1] < 1 << 20 and w.shape[1] % 64 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ Wg.T) * (x @ Wu.T) with w = [Wg; Wu], (2 I, H): the gated MLP's
+    first half without its intermediate rows (no autograd)."""
+    if x.is_cuda:
+        return _require_ext().linear_swiglu(x, w)
+    gate, up = (x @ w.t()).chunk(2, dim=-1)
+    return ref.silu_mul(gate, up)
+
+
 # ---------------------------------------------------------------------- RoPE
 
 

@@ -39,6 +39,22 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return x @ w.t()
 
 
+def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x @ Wg.T) * (x @ Wu.T), w = [Wg; Wu].  Prompts (the rows that
+    ``_mm_nt`` leaves to torch) of widths up to 2048 take both products and the
+    activation in one kernel; at larger widths the library's product alone is
+    the faster by more than the activation takes (us, library and activation
+    against one kernel: 513 .. 16384 rows, 1024 -> 4096, 30.5 .. 293 and 13.8 ..
+    228; 2048 -> 8192 42.7 .. 909 and 38.5 .. 832; 3584 -> 18944 148 .. 3386 and
+    171 .. 3393; 4096 -> 14336 133 .. 2805 and 190 .. 3042)."""
+    if x.shape[0] > 512 and x.shape[1] <= 2048 \
+            and ops.linear_swiglu_takes(x, w):
+        return ops.linear_swiglu(x, w)
+    i = w.shape[0] // 2
+    gate_up = _mm_nt(x, w)
+    return ops.silu_mul(gate_up.narrow(1, 0, i), gate_up.narrow(1, i, i))
+
+
 # graphed-decode batch buckets (POLYRL_DECODE_BUCKETS=1): capture counts
 # chosen so padding waste stays <= 50% while EOS-staggered batches reuse
 # at most ~16 captures over the whole 1..256 running-batch range
@@ -315,11 +331,7 @@ class InferenceModel:
             self.tp.all_reduce_(hidden)               # col-parallel o_proj
             hidden, residual = ops.fused_add_rmsnorm(
                 hidden, residual, lw.post_ln, cfg.rms_norm_eps)
-            gate_up = _mm_nt(hidden, lw.w_gate_up)
-            i_sz = cfg.intermediate_size // tp
-            hidden = _mm_nt(ops.silu_mul(gate_up.narrow(1, 0, i_sz),
-                                         gate_up.narrow(1, i_sz, i_sz)),
-                            lw.w_down)
+            hidden = _mm_nt(_gate_up(hidden, lw.w_gate_up), lw.w_down)
             self.tp.all_reduce_(hidden)               # col-parallel down_proj
         # final residual add + norm (fused; residual buffer is dead after)
         normed, _ = ops.fused_add_rmsnorm(hidden, residual, self.final_norm,

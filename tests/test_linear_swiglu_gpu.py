@@ -1,0 +1,81 @@
+"""The gated MLP's products and activation in one kernel: every number of row
+tiles a block may have, the edges of its tiles, the engine's use of it."""
+import pytest
+import torch
+
+import polyrl_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def check(m, n, k, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(m * 31 + n * 7 + k)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(2 * n, k, generator=g, device=DEV) * scale
+         / k ** 0.5).bfloat16()
+    assert ops.linear_swiglu_takes(x, w)
+    got = ops.linear_swiglu(x, w)
+    assert got.shape == (m, n)
+    for at in range(0, m, 8192):
+        gate, up = (x[at:at + 8192].double() @ w.double().t()).chunk(2, -1)
+        want = gate * torch.sigmoid(gate) * up
+        # 32-bit sums of k products, each off by 2^-24 of the sum of magnitudes
+        # at most, and one rounding to bf16
+        mass = x[at:at + 8192].double().abs() @ w.double().abs().t()
+        mg, mu = mass.chunk(2, -1)
+        bound = 2 ** -8 * want.abs() + k * 2.0 ** -24 * (
+            1.1 * mg * up.abs() + gate.abs() * mu) + 2.0 ** -30
+        assert ((got[at:at + 8192].double() - want).abs() <= bound).all(), at
+    return x, w, got
+
+
+@pytest.mark.parametrize("tiles", [2, 3, 4, 5, 6, 7, 8, 9])
+def test_row_tiles(tiles):
+    """Rows that fill 256 blocks of ``tiles`` row tiles but for a remainder."""
+    check(8192 * tiles - 17, 128, 64)
+
+
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 64, 65, 127, 513, 700])
+@pytest.mark.parametrize("n,k", [(128, 64), (128, 192), (640, 128),
+                                 (1152, 320)])
+def test_edges(m, n, k):
+    """Single rows and remainders; one, an odd and an even number of inner
+    tiles; column tiles that do not fill a group or the dies."""
+    check(m, n, k)
+
+
+def test_large_gates():
+    """Gates far from 0: the sigmoid ends at 0 and 1."""
+    x, w, got = check(600, 256, 128, scale=60.0)
+    assert got.isfinite().all()
+
+
+def test_what_it_takes():
+    x = torch.randn(600, 128, device=DEV).bfloat16()
+    w = torch.randn(512, 128, device=DEV).bfloat16()
+    takes = ops.linear_swiglu_takes
+    assert takes(x, w)
+    assert not takes(x.float(), w) and not takes(x, w.float())
+    assert not takes(x[:, :96], w[:, :96])
+    assert not takes(x, w[:384]) and not takes(x.t(), w)
+    flat = torch.randn(600 * 128 + 1, device=DEV).bfloat16()
+    assert not takes(flat[1:].view(600, 128), w)
+    for a, b in ((x, w[:384]), (x[:, :96].contiguous(), w[:, :96].contiguous()),
+                 (x, torch.randn(512, 64, device=DEV).bfloat16())):
+        with pytest.raises(RuntimeError):
+            ops.linear_swiglu(a, b)
+    assert ops.linear_swiglu(x[:0], w).shape == (0, 256)
+
+
+@pytest.mark.parametrize("m", [512, 513])
+def test_engine_prompts(m):
+    """Both sides of the rows from which the engine takes it."""
+    from polyrl_amd.rollout.engine import _gate_up
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x = torch.randn(m, 256, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(1024, 256, generator=g, device=DEV) / 16).bfloat16()
+    gate, up = (x.double() @ w.double().t()).chunk(2, -1)
+    want = gate * torch.sigmoid(gate) * up
+    off = (_gate_up(x, w).double() - want).norm() / want.norm()
+    assert off <= 5e-3                 # three roundings to bf16 at most
