@@ -71,13 +71,19 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return ref.silu_mul(gate, up)
 
 
-def linear_swiglu_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``linear_swiglu`` has a kernel for these operands."""
+def linear_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_rows`` and ``linear_swiglu`` have a kernel for these
+    operands."""
     return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and x.is_contiguous()
             and w.is_contiguous() and w.shape[0] % 256 == 0
             and 0 < w.shape[1] < 1 << 20 and w.shape[1] % 64 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T of many rows (no autograd)."""
+    return _require_ext().linear_rows(x, w) if x.is_cuda else x @ w.t()
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

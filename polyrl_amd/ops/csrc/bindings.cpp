@@ -7,6 +7,7 @@ void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor weight,
 void fused_add_rmsnorm(torch::Tensor out, torch::Tensor residual,
                        torch::Tensor x, torch::Tensor weight, double eps);
 void silu_mul(torch::Tensor out, torch::Tensor gate, torch::Tensor up);
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor linear_swiglu(torch::Tensor x, torch::Tensor w);
 void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
                   torch::Tensor cos_tab, torch::Tensor sin_tab);
@@ -75,6 +76,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm,
         "residual-add + RMSNorm, residual updated in place");
   m.def("silu_mul", &silu_mul, "SiLU(gate) * up");
+  m.def("linear_rows", &linear_rows, "x W^T of prompts");
   m.def("linear_swiglu", &linear_swiglu, "SiLU(x Wg^T) * (x Wu^T)");
   m.def("rope_inplace", &rope_inplace, "NEOX RoPE in place (table-driven)");
   m.def("rope_kv_append", &rope_kv_append,

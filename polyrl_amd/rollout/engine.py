@@ -31,24 +31,32 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T; decode-sized GEMMs (M <= 512) go through the
     algo-pinned hipBLASLt path (ops.tuned_mm_nt) — the heuristic pick runs
     skinny decode projections far off the weight-read bound.  Prefill Ms
-    are ragged (chunk sums), so they keep the torch path to bound the
-    number of shape searches."""
+    are ragged (chunk sums), so they are not searched: widths up to 1024 take
+    the kernel of this repository, whose call costs the host 15 us less than
+    torch's (a step of 2, 4, 8 and 12 x 256 tokens, 12 layers of 1024, 1080, 1138,
+    1742 and 1884 us with it and 1459, 1496, 1792 and 1909 without; 8192 tokens
+    3845 and 3998); at larger widths and beyond 8192 rows the library's product
+    is the faster by more (2048 -> 3072 of 8192 rows 93 us and 105)."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 512 \
             and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
+    if 512 < x.shape[0] <= 8192 and x.shape[1] <= 1024 \
+            and ops.linear_takes(x, w):
+        return ops.linear_rows(x, w)
     return x @ w.t()
 
 
 def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ Wg.T) * (x @ Wu.T), w = [Wg; Wu].  Prompts (the rows that
-    ``_mm_nt`` leaves to torch) of widths up to 2048 take both products and the
-    activation in one kernel; at larger widths the library's product alone is
-    the faster by more than the activation takes (us, library and activation
-    against one kernel: 513 .. 16384 rows, 1024 -> 4096, 30.5 .. 293 and 13.8 ..
-    228; 2048 -> 8192 42.7 .. 909 and 38.5 .. 832; 3584 -> 18944 148 .. 3386 and
-    171 .. 3393; 4096 -> 14336 133 .. 2805 and 190 .. 3042)."""
+    ``_mm_nt`` does not search for) of widths up to 2048 take both products and
+    the activation in one kernel; at larger widths the library's product alone
+    is the faster by more than the activation takes (us, library and activation
+    against one kernel, 513 .. 16384 rows: 1024 -> 4096 21.2 .. 297 and 15.2 .. 259;
+    1536 -> 8960 42 .. 867 and 36 .. 788; 2048 -> 8192 47 .. 925 and 44 .. 930;
+    3584 -> 18944 148 .. 3386 and 171 .. 3393; 4096 -> 14336 133 .. 2805 and 190 ..
+    3042)."""
     if x.shape[0] > 512 and x.shape[1] <= 2048 \
-            and ops.linear_swiglu_takes(x, w):
+            and ops.linear_takes(x, w):
         return ops.linear_swiglu(x, w)
     i = w.shape[0] // 2
     gate_up = _mm_nt(x, w)

@@ -1,5 +1,5 @@
-"""The gated MLP's products and activation in one kernel: every number of row
-tiles a block may have, the edges of its tiles, the engine's use of it."""
+"""Products of prompts, and the gated MLP's two with its activation: every number
+of row tiles a block may have, the edges of its tiles, the engine's use of them."""
 import pytest
 import torch
 
@@ -14,7 +14,7 @@ def check(m, n, k, scale=1.0):
     x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
     w = (torch.randn(2 * n, k, generator=g, device=DEV) * scale
          / k ** 0.5).bfloat16()
-    assert ops.linear_swiglu_takes(x, w)
+    assert ops.linear_takes(x, w)
     got = ops.linear_swiglu(x, w)
     assert got.shape == (m, n)
     for at in range(0, m, 8192):
@@ -45,6 +45,24 @@ def test_edges(m, n, k):
     check(m, n, k)
 
 
+@pytest.mark.parametrize("m", [1, 33, 65, 513, 700] + [
+    8192 * t - 17 for t in range(2, 10)])
+@pytest.mark.parametrize("n,k", [(256, 64), (768, 192), (1280, 128)])
+def test_rows(m, n, k):
+    """The product alone at the same edges, column tiles in one group and two."""
+    if m > 1000 and n > 256:
+        return
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = torch.randn(n, k, generator=g, device=DEV).bfloat16()
+    got = ops.linear_rows(x, w)
+    for at in range(0, m, 8192):
+        a = x[at:at + 8192].double()
+        want, mass = a @ w.double().t(), a.abs() @ w.double().abs().t()
+        bound = 2 ** -8 * want.abs() + k * 2.0 ** -24 * mass
+        assert ((got[at:at + 8192].double() - want).abs() <= bound).all(), at
+
+
 def test_large_gates():
     """Gates far from 0: the sigmoid ends at 0 and 1."""
     x, w, got = check(600, 256, 128, scale=60.0)
@@ -54,7 +72,7 @@ def test_large_gates():
 def test_what_it_takes():
     x = torch.randn(600, 128, device=DEV).bfloat16()
     w = torch.randn(512, 128, device=DEV).bfloat16()
-    takes = ops.linear_swiglu_takes
+    takes = ops.linear_takes
     assert takes(x, w)
     assert not takes(x.float(), w) and not takes(x, w.float())
     assert not takes(x[:, :96], w[:, :96])
@@ -71,7 +89,7 @@ def test_what_it_takes():
 @pytest.mark.parametrize("m", [512, 513])
 def test_engine_prompts(m):
     """Both sides of the rows from which the engine takes it."""
-    from polyrl_amd.rollout.engine import _gate_up
+    from polyrl_amd.rollout.engine import _gate_up, _mm_nt
     g = torch.Generator(device=DEV).manual_seed(m)
     x = torch.randn(m, 256, generator=g, device=DEV).bfloat16()
     w = (torch.randn(1024, 256, generator=g, device=DEV) / 16).bfloat16()
@@ -79,3 +97,6 @@ def test_engine_prompts(m):
     want = gate * torch.sigmoid(gate) * up
     off = (_gate_up(x, w).double() - want).norm() / want.norm()
     assert off <= 5e-3                 # three roundings to bf16 at most
+    both = _mm_nt(x, w)
+    off = (both.double() - x.double() @ w.double().t()).norm() / both.norm()
+    assert off <= 5e-3
