@@ -24,7 +24,7 @@
 // walks the bins, and the draw over the kept set, whose last block merges.  Short
 // rows take the same steps in one launch, a block each.  (64 x 151936, T 0.7, k
 // 50, p 0.9: 52.8 us with plans and a merge in launches of their own, eight in all,
-// 27 now; top-p 0.95 alone 70 and 64; at a temperature of 0 33 and 17.)
+// 24 now; top-p 0.95 alone 70 and 61; at a temperature of 0 33 and 17.)
 //
 // Only entries that can stand at a threshold go into a digit's bins (cut_of):
 // with k at most the number of lane groups, the k-th largest of the groups'
@@ -443,44 +443,66 @@ DEV_INLINE float cut_of(const float* tops, int n, bool by_k, bool by_p, int k,
   return fmaxf(cut, kth);
 }
 
-// The same from a wave of a block of the passes: the k-th largest maximum is
-// found bit by bit, the lanes counting those that are no smaller.
-template <int J>
-DEV_INLINE uint32_t kth_largest(const float* tops, int m, int width, int k) {
-  const int lane = threadIdx.x & 63;
-  uint32_t e[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    e[j] = 0;
-    const int i = j * 64 + lane;
-    if (i < m) {
-      float t = tops[i * width];
-      for (int w = 1; w < width; ++w) t = fmaxf(t, tops[i * width + w]);
-      e[j] = enc_f32(t);
-    }
-  }
+// The same from a wave of a block of the passes, which has the maxima in registers
+// (lane l's are 4 l .. 4 l + 3 of each 256, a wave's in turn; -inf past the last):
+// the k-th largest is found bit by bit, the lanes counting those that are no smaller.
+// Of bf16 numbers' encodings the lower half is all sign.
+template <typename T, int J>
+DEV_INLINE uint32_t kth_largest(const uint32_t (&e)[J], int k) {
   uint32_t found = 0;
-  for (int bit = 31; bit >= 0; --bit) {
+  for (int bit = 31; bit >= (sizeof(T) == 2 ? 16 : 0); --bit) {
     const uint32_t at = found | 1u << bit;
     int n = 0;
 #pragma unroll
     for (int j = 0; j < J; ++j) n += __popcll(__ballot(e[j] >= at));
     if (n >= k) found = at;
   }
-  return found;
+  return sizeof(T) == 2 && !(found >> 31) ? found | 0xffff : found;
 }
-DEV_INLINE float wave_cut(const float* tops, int n, bool by_k, bool by_p, int k,
-                          float p, float inv_temp, const Sums<true>& all,
-                          int V) {
+constexpr int MOST_TOPS = 64 * TOPS / 256;     // of 256 maxima, in 64 pieces
+template <typename T, int C>
+DEV_INLINE uint32_t kth_of_tops(const float (&tops)[MOST_TOPS][4], int n, int k) {
+  const int lane = threadIdx.x & 63;
+  if (k <= n / 4) {                    // waves' maxima, as above
+    uint32_t e[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float t = tops[c][0];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) t = fmaxf(t, tops[c][w]);
+      e[c] = c * 256 + lane * 4 < n ? enc_f32(t) : 0u;
+    }
+    return kth_largest<T>(e, k);
+  }
+  if (C == 1 && n <= 64) {             // one a lane
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float o = __shfl(tops[0][w], lane / 4, 64);
+      if (lane % 4 == w) t = o;
+    }
+    const uint32_t e[1] = {lane < n ? enc_f32(t) : 0u};
+    return kth_largest<T>(e, k);
+  }
+  uint32_t e[4 * C];
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      e[c * 4 + w] = c * 256 + lane * 4 < n ? enc_f32(tops[c][w]) : 0u;
+  return kth_largest<T>(e, k);
+}
+template <typename T>
+DEV_INLINE float wave_cut(const float (&tops)[MOST_TOPS][4], int n, bool by_k,
+                          bool by_p, int k, float p, float inv_temp,
+                          const Sums<true>& all, int V) {
   float cut = -INFINITY;
   if (by_p && inv_temp > 0.f && p > 0.f)
     cut = all.m + __logf(0.99f * (1.f - p) * all.st / V) / inv_temp;
   if (!(cut > -INFINITY)) cut = -INFINITY;   // (NaN logits)
   if (!by_k || k > n) return cut;
-  const int width = k <= n / 4 ? 4 : 1, m = n / width;
-  const uint32_t e = m <= 64 ? kth_largest<1>(tops, m, width, k)
-                   : m <= 256 ? kth_largest<4>(tops, m, width, k)
-                              : kth_largest<16>(tops, m, width, k);
+  const uint32_t e = n <= 256 ? kth_of_tops<T, 1>(tops, n, k)
+                              : kth_of_tops<T, MOST_TOPS>(tops, n, k);
   return fmaxf(cut, __uint_as_float(e >> 31 ? e ^ 0x80000000u : ~e));
 }
 
@@ -796,6 +818,14 @@ DEV_INLINE void add_bins(int digit, uint32_t* cnt, float* mass, uint32_t* h,
 // them to the bins, the last block those that it does, and the row goes on like
 // one without a list (64 x 151936, top-p 0.95 at T 0.7, 4000 candidates side by
 // side: 66 us; 183 with one block for such a row's passes, 69 without lists).
+// What bounds it: a chain of short waits.  So what can be read early is read at once:
+// the maxima with the sums, the whole list with its length, the winner's logit with
+// the list; and one wave of a block searches the cut, whose counts are scalar work
+// that the sixteen waves of a CU would take turns at.  (64 x 151936, T 0.7, k 50, p
+// 0.9, all launches: 26.7 us as it was, 25.3 read early, 24.9 with half of the bits of
+// bf16 maxima, 24.1 with one wave; 128 rows 35.1 and 31.8, one of 128256 18.6 and
+// 16.4, 32 x 128256 fp32, k 200, 53.6 and 46.  The list's logits asked for before the
+// cut, or two bits of it a step: no gain, 25.5 for 24.9.)
 template <typename T>
 __global__ __launch_bounds__(SNT) void sample_select_kernel(
     int64_t* __restrict__ out_tokens, float* __restrict__ out_logprobs,
@@ -824,6 +854,27 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
   RowState* state = row_state(hist, hist_words, row);
   share += row * split;
   list_v += row * LISTED, list_i += row * LISTED;
+  // The maxima come with the pieces' sums, not once for the cut and once more for
+  // the list's length: the block is a chain of such waits.
+  const int most = split * TOPS;
+  float top[MOST_TOPS][4];
+  auto read_tops = [&](int c) {
+    const int at = c * 256 + (threadIdx.x & 63) * 4;    // (four lanes a piece)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float t = tops[row * most + (at < most ? at : 0) + w];
+      top[c][w] = at < most ? t : -INFINITY;
+    }
+  };
+  read_tops(0);
+  if (most > 256) {
+#pragma unroll
+    for (int c = 1; c < MOST_TOPS; ++c) read_tops(c);
+  } else {
+#pragma unroll
+    for (int c = 1; c < MOST_TOPS; ++c)
+      top[c][0] = top[c][1] = top[c][2] = top[c][3] = -INFINITY;
+  }
   const Sums<true> all = row_sums<true>(share, split, inv_temp);
   if (!by_k && !by_p) {
     if (piece != 0) return;
@@ -834,25 +885,33 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     }
     return;
   }
-  const float cut = wave_cut(tops + row * split * TOPS, split * TOPS, by_k,
-                             by_p, k, p, inv_temp, all, V);
-  Plan plan(cut, all, p, by_k, by_p);
-  // (a list needs numbers that add up)
-  bool listing = cut > -INFINITY && inv_temp > 0.f &&
-                 fabsf(all.m) < INFINITY && all.st < INFINITY;
-  if (listing) {
-    const int g = split * TOPS, lane = threadIdx.x & 63;
-    int with = 0;
-    for (int i = lane; i - lane < g; i += 64)
-      with += __popcll(__ballot(i < g && tops[row * g + i] >= cut));
-    listing = with <= g * (1.f - __expf(-0.7f * LISTED / g));
+  // (one wave looks: sixteen a CU would take turns at the same scalar counts)
+  if (threadIdx.x < 64) {
+    const float c = wave_cut<T>(top, most, by_k, by_p, k, p, inv_temp, all, V);
+    // (a list needs numbers that add up)
+    bool list = c > -INFINITY && inv_temp > 0.f && fabsf(all.m) < INFINITY &&
+                all.st < INFINITY;
+    if (list) {
+      int with = 0;
+#pragma unroll
+      for (int i = 0; i < MOST_TOPS; ++i) {
+        if (i * 256 >= most) break;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) with += __popcll(__ballot(top[i][w] >= c));
+      }
+      list = with <= most * (1.f - __expf(-0.7f * LISTED / most));
+    }
+    if (threadIdx.x == 0) lds[0] = c, found = list ? 0 : -1;
   }
+  __syncthreads();
+  const float cut = lds[0];
+  const bool listing = found == 0;
+  Plan plan(cut, all, p, by_k, by_p);
   bool to_bins = !listing;
   if (listing) {
     int* own_i = reinterpret_cast<int*>(cnt);
     float* own_v = mass;
-    if (threadIdx.x == 0) found = 0;
-    __syncthreads();
+    __syncthreads();                    // (found was read)
     const int groups = r.groups();
     for (int g = piece * SNT + threadIdx.x; g < groups; g += split * SNT) {
       if (*(volatile int*)&found > LISTED) break;
@@ -906,17 +965,22 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     });
   if (!last_of_row(&state->arrived[0], split)) return;
 
-  // this thread's entries of the list, all on their way at once
+  // this thread's entries of the list and how many there are, all on their way at
+  // once
   float own[LISTED / SNT];
+  int own_at[LISTED / SNT];
 #pragma unroll
-  for (int i = 0; i < LISTED / SNT; ++i)
+  for (int i = 0; i < LISTED / SNT; ++i) {
     own[i] = read_through(&list_v[i * SNT + threadIdx.x]);
+    own_at[i] = read_through(&list_i[i * SNT + threadIdx.x]);
+  }
+  const int overfull = read_through(&state->overfull);
+  const int listed = read_through(&state->listed);
   auto each = [&](int n, auto take) {
 #pragma unroll
     for (int i = 0; i < LISTED / SNT; ++i)
-      if (i * SNT + (int)threadIdx.x < n) take(i * SNT + threadIdx.x, own[i]);
+      if (i * SNT + (int)threadIdx.x < n) take(own_at[i], own[i]);
   };
-  const int overfull = listing ? read_through(&state->overfull) : 0;
   if (!listing || overfull) {
     read_bins<T>(0, h, cnt, mass);
     if (overfull) {
@@ -930,7 +994,6 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     return;
   }
   const uint64_t rowkey = seed + (uint64_t)row * 0x9e3779b97f4a7c15ull;
-  const int listed = read_through(&state->listed);
   if (listed > COUNTED) {
     select_alone<SNT, T>(plan, k, cnt, mass, lds, [&](int digit) {
       each(listed, [&](int, float v) {
@@ -962,18 +1025,22 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     plan.prefix_k = thr[0], plan.prefix_p = thr[1];
   }
   const uint32_t tau = plan.threshold();
-  float best = -INFINITY;
+  float best = -INFINITY, best_v = 0.f;
   int best_i = 0;
-  each(listed, [&](int t, float v) {
+  each(listed, [&](int i, float v) {
     if (enc_f32(v) < tau) return;
-    const int i = read_through(&list_i[t]);
     const float z = __fmaf_rn(v, inv_temp, gumbel(rng_bits(rowkey, rng_at(i))));
-    if (better(z, i, best, best_i)) best = z, best_i = i;
+    if (better(z, i, best, best_i)) best = z, best_i = i, best_v = v;
   });
+  const float own_best = best;
+  const int own_i = best_i;
   block_best(best, best_i, part);
-  if (threadIdx.x == 0) {
+  // the thread that has the entry has its logit too; without one the row is read
+  const bool none = !(best > -INFINITY);
+  if (none && threadIdx.x == 0) best_v = (float)r.x[best_i];
+  if (none ? threadIdx.x == 0 : own_best == best && own_i == best_i) {
     out_tokens[row] = best_i;
-    out_logprobs[row] = (float)r.x[best_i] - (all.m + __logf(all.s));
+    out_logprobs[row] = best_v - (all.m + __logf(all.s));
     state->done = 1;
   }
 }

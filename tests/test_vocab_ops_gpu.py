@@ -484,3 +484,39 @@ def test_sample_block_sizes(n, v, dtype):
         z = x[r].double().cpu() / float(temp[r]) + noise(77, r, v)
         # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
         assert z[int(tok[r])] >= z.max() - 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v,ks", [(300, 40001, (1, 16, 17, 64, 65)),
+                                    (64, 131073, (1, 64, 65, 256, 257)),
+                                    (52, 200003, (79, 80, 303, 320, 321)),
+                                    (16, 262147, (200, 256, 257, 1000, 1024))])
+def test_sample_cut_of_few_and_many_pieces(n, v, ks, dtype):
+    """The cut below the k-th largest of the pieces' maxima: 4, 16, 20 and 64
+    pieces, 16 maxima each, and a k on both sides of where waves' maxima, all of
+    them and no cut take turns.  Rows whose k-th largest is positive, negative,
+    tied, zero, infinite."""
+    torch.manual_seed(23)
+    x = torch.randn(n, v, device=DEV) * 2
+    x[1::5] -= 300
+    x[2::5] = x[2::5].round()
+    # (zeros of one sign: the kernels' order has -0 below +0, the oracle's does not,
+    # and a row of ties of both keeps the positive ones only)
+    x[3::5] = x[3::5].clamp(max=0.0)
+    x[4::5, 11:] = -float("inf")
+    x = x.to(dtype)
+    k = torch.tensor([ks[(r // 5) % len(ks)] for r in range(n)],
+                     dtype=torch.int32, device=DEV)
+    p = torch.tensor([1.0 if r % 2 else 0.95 for r in range(n)], device=DEV)
+    temp = torch.full((n,), 0.8, device=DEV)
+    tok, lp = ops.sample(x, temp, k, p, 31, no_filter=False)
+    want = torch.log_softmax(x.double(), -1).gather(1, tok[:, None])[:, 0]
+    assert ((lp.double() - want).abs() <= 1e-5 * (1 + want.abs())).all()
+    for r in range(min(n, 25)):
+        row, got = x[r].double().cpu(), int(tok[r])
+        sure, maybe = kept(row, float(temp[r]), int(k[r]), float(p[r]))
+        assert maybe[got], r
+        z = row / float(temp[r]) + noise(31, r, v)
+        # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large; at
+        # 300 / T a multiply-add of 32 bits is off by another 3e-5
+        assert z[got] >= z[sure].max() - 1e-3, r
