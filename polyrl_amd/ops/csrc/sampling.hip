@@ -556,7 +556,7 @@ DEV_INLINE void walk_bins(Plan& plan, const uint32_t* cnt, const float* mass,
 // The row's bins, to which the other blocks added, into LDS: whole lines, all on
 // their way at once.  No load stands under a condition: its wait would stand there
 // too, and with sixteen waits in turn for what comes past the L2 64 x 50257 fp32,
-// top-p 0.8 at T 0.7, took 62 us (the three plan launches before it 61), 58 now.
+// top-p 0.8 at T 0.7, took 62 us (the three plan launches before it 61), 56 now.
 template <typename T>
 DEV_INLINE void read_bins(int digit, const uint32_t* h, uint32_t* cnt,
                           float* mass) {
@@ -1164,19 +1164,19 @@ static void launch_sample(torch::Tensor& out_tokens,
   auto stream = at::hip::getCurrentHIPStream();
   // Rows in one launch, a block each, while that is no longer than the pieces and
   // their passes.  Without a filter: with few rows up to 16384 numbers (64 x 16000
-  // bf16 12.1 us, in pieces 12.6; 64 x 32000 18.3 and 13.6), with a block for most
-  // CUs up to 65536 (256 x 50257 26 and 32).  With one: up to 32768.  Pieces are
-  // quicker from there down to 24000 (fp32 9000) with both filters (64 x 24000 36.5
-  // us, in pieces 23, 64 x 16000 33 and 42; fp32 64 x 9000 39 and 25), but not with
-  // top-p 0.95 alone (64 x 24000 37 and 41, 256 x 32000 45 and 59, fp32 57 and 84)
-  // nor at a temperature of 0, where nothing is selected (9 and 20).  What stays
-  // dearer than a block a row everywhere is the draw at a temperature of 0 without a
-  // filter from 16384 numbers on, 11.3 us for 8 to 10: the temperature is on the
-  // device, and at 1 the pieces take 11.5 for 21.
+  // bf16 9.1 us, in pieces 10.0), with a block for most CUs up to 65536 (256 x 50257
+  // 18.4 and 20.7).  With one: up to 32768.  Pieces are quicker from there down to
+  // 24000 (fp32 9000) with both filters (64 x 24000 34.7 us, in pieces 20.1, 64 x
+  // 16000 32.2 and 41.1; fp32 64 x 9000 37.7 and 21.3), but not with top-p 0.95 alone
+  // (64 x 24000 35.3 and 39.3, 256 x 32000 41.8 and 56.8, fp32 54.4 and 81.9) nor at a
+  // temperature of 0, where nothing is selected (6.9 and 16.6).  What stays dearer
+  // than a block a row is the draw at a temperature of 0 without a filter from 16384
+  // numbers on, 10.3 us for 6.8: the temperature is on the device, and at 1 the pieces
+  // take no more.
   // A block of 1024 threads takes rows of more than one round of 256 words (64 x
-  // 9000 both filters 31 us, with 256 threads 37; 64 x 32000 38 and 72); where
+  // 9000 both filters 30.5 us, with 256 threads 35.1; 64 x 32000 36.4 and 65.5); where
   // there are more rows than CUs, 256 threads take them up to ten rounds (512 x
-  // 9000 41 us, with 1024 threads 64).
+  // 9000 39.7 us, with 1024 threads 59.9; 512 x 24000 65.7 and 65.4).
   auto rows = [&](auto kern, int threads) {
     kern<<<dim3((unsigned)N), dim3(threads), 0, stream>>>(
         out_tokens.data_ptr<int64_t>(), out_logprobs.data_ptr<float>(),
@@ -1198,13 +1198,14 @@ static void launch_sample(torch::Tensor& out_tokens,
   }
   // Pieces of a row, 1024 threads a CU in all.  With a filter blocks of 256 (with 512,
   // 768, 1024, 1536 and 2048 of them 64 x 151936 with both filters takes 29.3, 27.9,
-  // 27.6, 31.4, 36.9 us, with top-p 0.95 alone 69, 64, 64, 65, 77), none under two
-  // rounds of 256 words.  Without one the largest blocks, whose waves share what
-  // they know, that fill 7/8 of the chip or of the 2048 threads that a CU holds and
-  // have three rounds in two blocks (128 x 128256 in blocks of 256, 512 and 1024: 25.8,
-  // 24.5 and 23.1; 100 x 128256 in 1100, 500 and 500: 24.9, 22.3, 22.1, but in 300 of
-  // 1024 31.5; 200 x 128256 in 1200 of 256, 1000 of 512 and 200 of 1024 35.8, 33.3, 36.9; 100
-  // x 50257 in 1100 of 256, 500 of 512, 500 of 1024 16.0, 14.5, 16).
+  // 27.6, 31.4, 36.9 us, with top-p 0.95 alone 69, 64, 64, 65, 77; 24 and 61 with 1024
+  // since the candidates' kernel waits less), none under two rounds of 256 words.
+  // Without one the largest blocks, whose waves share what they know, that fill 7/8
+  // of the chip or of the 2048 threads that a CU holds and have three rounds in two
+  // blocks (128 x 128256 in blocks of 256, 512 and 1024: 25.8, 24.5 and 23.1; 100 x
+  // 128256 in 1100, 500 and 500: 24.9, 22.3, 22.1, but in 300 of 1024 31.5; 200 x
+  // 128256 in 1200 of 256, 1000 of 512 and 200 of 1024 35.8, 33.3, 36.9; 100 x 50257
+  // in 1100 of 256, 500 of 512, 500 of 1024 16.0, 14.5, 16).
   int nt = SNT, split = 0;
   if (no_filter) {
     const int most_blocks[][2] = {{1024, 256}, {1024, 512}, {512, 512},
