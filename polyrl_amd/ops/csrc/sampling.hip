@@ -269,7 +269,10 @@ struct Draw {
           z = fmaxf(z, __fmaf_rn(v[j], inv_temp, gumbel_about(bits[j])));
         raise(z - (1e-4f + 1e-5f * fabsf(z)));
       }
-      const float u = __expf(-__expf(__fmaf_rn(c, inv_temp, -wbest)));
+      // (an entry whose z rounds to the best one's wins by a lower index, whichever
+      // wave comes first: less twice the last place of the best)
+      const float bound = __fmaf_rn(fminf(fabsf(wbest), 3.4e38f), -0x1p-22f, wbest);
+      const float u = __expf(-__expf(__fmaf_rn(c, inv_temp, -bound)));
       least = (uint32_t)max((int)(u * (16777216.f * (1.f - 1e-5f))) - 2, 0) << 8;
     }
     if (!__any(most >= least)) return;

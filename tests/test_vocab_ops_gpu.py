@@ -520,3 +520,39 @@ def test_sample_cut_of_few_and_many_pieces(n, v, ks, dtype):
         # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large; at
         # 300 / T a multiply-add of 32 bits is off by another 3e-5
         assert z[got] >= z[sure].max() - 1e-3, r
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v", [(64, 9000), (128, 40001), (256, 65539),
+                                 (100, 98305)])
+def test_sample_ties_of_rounded_sums(n, v, dtype):
+    """At a temperature of 1e-6 logits of 11 are 1.1e7, where 32-bit numbers are
+    whole: of equal logits those whose noise rounds alike tie, and the first of them
+    wins, whichever wave is first.  Without a filter and with one that keeps all."""
+    m = 200
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, v, generator=g)
+    at = torch.stack([torch.randperm(v, generator=g)[:m].sort()[0]
+                      for _ in range(n)])
+    x.scatter_(1, at, 11.0)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    temp = full(1e-6, torch.float32)
+    by = torch.tensor(1.0) / torch.tensor(1e-6)
+    checked = 0
+    for seed in (5, 1 << 40):
+        args = (x.to(dtype).to(DEV), temp, full(-1, torch.int32),
+                full(1.0, torch.float32), seed)
+        got = [ops.sample(*args, no_filter=f)[0].cpu() for f in (True, False)]
+        for r in range(n):
+            # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large;
+            # rows that this could decide are passed over
+            z = 11.0 * by.double() + noise(seed, r, v)[at[r]]
+            lo, hi = ((z + d).float() for d in (-2e-4, 2e-4))
+            if not torch.equal(lo, hi):
+                sure = hi < lo.max()
+                if not torch.equal(lo[~sure], hi[~sure]):
+                    continue
+            checked += 1
+            first = int(at[r][(lo == lo.max()).nonzero()[0, 0]])
+            assert [int(t[r]) for t in got] == [first, first], (seed, r)
+    assert checked > n
