@@ -180,9 +180,11 @@ DEV_INLINE void linear_wave(char* lds, int row0, int tiles, FetchX fetch_x,
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const float g = acc[i][j][4 * q + t];
-          v.v[t] = f2bf(GLU ? g * acc[1][j][4 * q + t] *
-                                  __builtin_amdgcn_rcpf(
-                                      1.f + exp2_hw(g * -1.4426950408889634f))
+          // (the activation first: gate times up may be beyond 32 bits where the
+          // sigmoid is 0)
+          v.v[t] = f2bf(GLU ? g * __builtin_amdgcn_rcpf(
+                                      1.f + exp2_hw(g * -1.4426950408889634f)) *
+                                  acc[1][j][4 * q + t]
                             : g);
         }
         *reinterpret_cast<bf16x4*>(

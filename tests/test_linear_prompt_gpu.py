@@ -69,6 +69,17 @@ def test_large_gates():
     assert got.isfinite().all()
 
 
+def test_gate_times_up_beyond_32_bits():
+    """A closed gate gives 0 whatever the up projection, as silu(gate) * up."""
+    x = torch.randn(600, 128, device=DEV).abs().add_(1.0).bfloat16()
+    w = torch.zeros(512, 128, device=DEV).bfloat16()
+    w[:256, 0], w[256:, 0] = -1e25, 1e25
+    w[256::2, 0] = -1e25
+    got = ops.linear_swiglu(x, w)
+    gate, up = (x @ w.t()).chunk(2, -1)
+    assert torch.equal(got, ops.silu_mul(gate, up)) and not got.any()
+
+
 def test_what_it_takes():
     x = torch.randn(600, 128, device=DEV).bfloat16()
     w = torch.randn(512, 128, device=DEV).bfloat16()
