@@ -74,9 +74,10 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 def linear_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``linear_rows`` and ``linear_swiglu`` have a kernel for these
     operands."""
-    return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and x.is_contiguous()
-            and w.is_contiguous() and w.shape[0] % 256 == 0
+    return (x.is_cuda and x.device == w.device and x.dim() == 2
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.is_contiguous() and w.is_contiguous()
+            and w.shape[0] % 256 == 0 and w.shape[0] < 1 << 25
             and 0 < w.shape[1] < 1 << 20 and w.shape[1] % 64 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 

@@ -90,7 +90,9 @@ struct AttnTile {
   }
 
   // 32 rows of a wave's own, laid out like a tile's, to rows [0, min(live, 32)) of
-  // memory: the buffer ends with the last one, and what is behind it is not written
+  // memory: the buffer ends with the last one, and what is behind it is not written.
+  // Offsets have 32 bits: ld is below STORE_LD.
+  static constexpr long STORE_LD = 1L << 25;
   DEV_INLINE static void store32(const char* rows, bf16_t* to, long ld,
                                  int live) {
     constexpr int RS = 64 / GR;         // rows of a step

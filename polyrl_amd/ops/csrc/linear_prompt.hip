@@ -247,14 +247,15 @@ __global__ __launch_bounds__(512, 2) void linear_kernel(
 template <bool GLU>
 torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
   for (const auto* t : {&x, &w})
-    TORCH_CHECK(t->is_cuda() && t->dim() == 2 && t->is_contiguous() &&
-                    t->dtype() == torch::kBFloat16 &&
+    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&
+                    t->is_contiguous() && t->dtype() == torch::kBFloat16 &&
                     ((uintptr_t)t->data_ptr() & 15) == 0,
-                "linear: contiguous 2-D bf16 at a 16-byte address");
+                "linear: contiguous 2-D bf16 at 16-byte addresses of one device");
   const long M = x.size(0), K = x.size(1), N = w.size(0) / (GLU ? 2 : 1);
   TORCH_CHECK(w.size(1) == K && K % 64 == 0 && K > 0 && w.size(0) % 256 == 0 &&
-                  K < (1L << 20) && N < (1L << 30) && M < (1L << 30),
-              "linear: inner numbers in 64s, the weight's rows in 256s");
+                  K < (1L << 20) && N < OutTile::STORE_LD && M < (1L << 30),
+              "linear: inner numbers in 64s, the weight's rows in 256s, outputs "
+              "below 2^25");
   auto out = torch::empty({M, N}, x.options());
   if (M == 0 || N == 0) return out;
   // Rows of a block: as many as end the last round of 256 blocks, one per CU,

@@ -95,6 +95,13 @@ def test_what_it_takes():
         with pytest.raises(RuntimeError):
             ops.linear_swiglu(a, b)
     assert ops.linear_swiglu(x[:0], w).shape == (0, 256)
+    assert not takes(x, w.cpu())
+    # (rows of outputs end at 32-bit offsets)
+    far = torch.empty(1 << 26, 64, dtype=torch.bfloat16, device=DEV)
+    for op, n in ((ops.linear_rows, 1 << 25), (ops.linear_swiglu, 1 << 26)):
+        assert not takes(x[:, :64].contiguous(), far[:n])
+        with pytest.raises(RuntimeError):
+            op(x[:1, :64].contiguous(), far[:n])
 
 
 @pytest.mark.parametrize("m", [512, 513])
