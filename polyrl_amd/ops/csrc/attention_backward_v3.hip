@@ -593,7 +593,7 @@ void varlen_attention_backward_v3(
     TORCH_CHECK(g->dtype() == torch::kBFloat16 && g->is_contiguous());
   const int Hq = q.size(1), D = q.size(2), Hk = k.size(1);
   TORCH_CHECK(D == 128 || D == 64, "backward v3 supports head_dim 64/128");
-  TORCH_CHECK(Hq % Hk == 0);
+  TORCH_CHECK(Hq % Hk == 0 && (long)Hq * D < AttnTile<64>::STORE_LD);
   if (t64_seq.size(0) == 0) return;
   (D == 128 ? launch_bwd<128> : launch_bwd<64>)(
       dq, dk, dv, rows_by16(q), rows_by16(k), rows_by16(v), out,

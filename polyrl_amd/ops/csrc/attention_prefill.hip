@@ -308,7 +308,7 @@ void varlen_prefill_attention(torch::Tensor out, torch::Tensor q,
   v = rows_by16(v);
   const int Hq = q.size(1), D = q.size(2), Hk = k.size(1);
   TORCH_CHECK(D == 128 || D == 64, "prefill kernel supports head_dim 64/128");
-  TORCH_CHECK(Hq % Hk == 0);
+  TORCH_CHECK(Hq % Hk == 0 && (long)Hq * D < AttnTile<64>::STORE_LD);
   const int nseq = cu_seqlens_q.size(0) - 1;
   const long ntiles = table ? tile_seq.size(0)
                             : q.size(0) / ATILE + nseq;

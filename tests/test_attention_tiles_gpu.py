@@ -590,6 +590,26 @@ def test_window_many_tiles(hq, hk, d):
         a += x
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("stride", [1 << 24, 1 << 25, 1 << 27])
+def test_window_rows_far_apart(stride, d):
+    """Output rows whose distances 32-bit offsets hold, just do not, and do not."""
+    torch.manual_seed(22)
+    hq, hk, n, page = 8, 2, 70, 16
+    i32 = dict(dtype=torch.int32, device=DEV)
+    rows = torch.randn(5, page, 2 * hk * d, device=DEV).bfloat16()
+    q = torch.randn(n, hq * d, device=DEV).bfloat16()
+    far = torch.empty((n - 1) * stride + hq * d, dtype=torch.bfloat16,
+                      device=DEV).as_strided((n, hq * d), (stride, 1))
+    got, want = (ops.seq.gqa_window_attention(
+        q, rows, torch.randperm(5, generator=torch.Generator().manual_seed(1))
+        .int().to(DEV)[None], torch.zeros(n, **i32), torch.arange(n, **i32), hq,
+        hk, d, d, 40, 0, None, None, None, d ** -0.5, torch.bfloat16,
+        tiles=ops.seq.attention_tiles([n], DEV), out=out) for out in (far, None))
+    # two kernels, each within 2^-7 of the values' magnitude of the true result
+    assert (got - want).abs().max() <= 2 ** -6 * rows.abs().max()
+
+
 @pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (8, 2, 128)])
 def test_forward_many_tiles(hq, hk, d):
     """More row tiles than run at a time with two blocks per CU: heads of 128
