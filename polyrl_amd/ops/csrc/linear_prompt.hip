@@ -70,8 +70,8 @@ struct RowsFrom {
 #pragma unroll
     for (int i = 0; i < (ROWS + 63) / 64; ++i) {
       asm volatile(
-          "s_mov_b32 m0, %0\n\ts_nop 4\n\t"
-          "buffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(to + i * 8192),
+          "s_nop 4\n\t"
+          "buffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(to + i * 8192),
           "v"(a), "s"(from)
           : "memory");
       a += 64 * ldb;                   // (whole periods of the swizzle)
