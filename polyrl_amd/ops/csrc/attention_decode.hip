@@ -70,25 +70,18 @@ __global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
       keys[ONCE ? 4 : 1][ONCE ? DEC_KEYS * D * 2 : 16];
   __shared__ float ml[4][DEC_HEADS][2];
 
-  const int b = blockIdx.x / (Hk * nsplit);
-  const int rem = blockIdx.x % (Hk * nsplit);
-  const int hk = rem / nsplit;
-  const int sp = rem % nsplit;
-  const int G = Hq / Hk;
-  const int L = max(context_lens[b], 0);
-  // a stretch per block, in whole rounds of a wave
-  const int Lc = nsplit == 1 ? L : ((L + nsplit - 1) / nsplit + DEC_KEYS - 1) /
-                                       DEC_KEYS * DEC_KEYS;
-  const int cbeg = sp * Lc;
-  const int cend = min(cbeg + Lc, L);
+  int rem, sp, none;
+  const int b = split_id(blockIdx.x, Hk * nsplit, rem);
+  const int hk = split_id(rem, nsplit, sp);
+  const int G = split_id(Hq, Hk, none);
   const int lane = threadIdx.x & 63;
   const int wid = wave_id();
   const int l15 = lane & 15, lhi = lane >> 4;
   const int vrow = lane / T::GR, vcol = lane % T::GR;
 
-  // Cache rows of keys t0 + lane % 32.  The table is read before the row's length
-  // is known; an entry past the stretch may be anything, and the round's first key
-  // stands in for it.
+  // Cache rows of keys t0 + lane % 32.  The table of a row that is not divided is
+  // read before its length is known; an entry past the stretch may be anything, and
+  // the round's first key stands in for it.
   const int* ptab = page_table + (long)b * max_pages;
   const bool pow2 = (page_size & (page_size - 1)) == 0;
   const int shift = 31 - __builtin_clz(page_size);
@@ -96,6 +89,14 @@ __global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
     const int t = t0 + (lane & 31);
     return ptab[min(pow2 ? t >> shift : t / page_size, max_pages - 1)];
   };
+  int page = 0;
+  if (nsplit == 1 && max_pages > 0) page = look_up(wid * DEC_KEYS);
+  const int L = max(context_lens[b], 0);
+  // a stretch per block, in whole rounds of a wave
+  const int Lc = nsplit == 1 ? L : ((L + nsplit - 1) / nsplit + DEC_KEYS - 1) /
+                                       DEC_KEYS * DEC_KEYS;
+  const int cbeg = sp * Lc;
+  const int cend = min(cbeg + Lc, L);
   auto rows_of = [&](int page, int t0) {
     const int t = t0 + (lane & 31);
     const int slot =
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
     return t < cend ? slot : first;
   };
   int t0 = cbeg + wid * DEC_KEYS;
-  int page = max_pages > 0 ? look_up(t0) : 0;
+  if (nsplit > 1 && max_pages > 0) page = look_up(t0);
 
   // Q of this column's head (columns past the group repeat its last head)
   bf16x8_t qf[KS];
@@ -265,19 +266,25 @@ __global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
         if (t0 + i * RPI + vrow >= cend) vv[i] = {0, 0, 0, 0};
     }
     store_rows(vs, vv);
+    bf16x8_t vt[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const i16x4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (lds_i16x4_p)(vs + (va ^ (dt << 5))));
       const i16x4_t c = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (lds_i16x4_p)(vs + (vb ^ (dt << 5))));
-      const bf16x8_t vt = __builtin_bit_cast(
+      vt[dt] = __builtin_bit_cast(
           bf16x8_t, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-      for (int i = 0; i < (FEW ? 1 : 2); ++i)
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            vt, __builtin_bit_cast(bf16x8_t, w3[i]), o[dt], 0, 0, 0);
     }
+    // (small calls, whose rounds are a chain of waits: all reads on their way before
+    // the first product; 256 rows of 100 .. 300, 12/2 heads of 128, 14.1 -> 13.9 us)
+    if constexpr (!ONCE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < (FEW ? 1 : 2); ++i)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            vt[dt], __builtin_bit_cast(bf16x8_t, w3[i]), o[dt], 0, 0, 0);
     __builtin_amdgcn_wave_barrier();
   }
   l_run = quad_sum(l_run);
@@ -294,27 +301,44 @@ __global__ __launch_bounds__(256, ONCE ? 2 : 3) void paged_decode_attn_kernel(
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < G * D; i += 256) {
+  // Neighbouring sums of a thread, as many as take all threads once: in rounds of one
+  // sum a thread the reads were half a microsecond of the smallest calls (64 rows of
+  // 19 .. 31, 64/8 heads of 128, 5.9 -> 5.3 us; 58 of 14 .. 36, 12/2 heads, 4.7 -> 4.2).
+  constexpr int N = (FEW ? 4 : 8) * D / 256;
+  typedef __attribute__((ext_vector_type(N))) float part_t;
+  const int i = threadIdx.x * N;
+  if (i < G * D) {
     const int h = i / D, d = i % D;
     float gm = ml[0][h][0];
 #pragma unroll
     for (int w = 1; w < 4; ++w) gm = fmaxf(gm, ml[w][h][0]);
-    float l = 0.f, acc = 0.f;
+    float l = 0.f, acc[N];
+#pragma unroll
+    for (int t = 0; t < N; ++t) acc[t] = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float a = exp2_hw(ml[w][h][0] - gm);
-      const float* part = reinterpret_cast<const float*>(lds[w]) + i;
+      const part_t* part = reinterpret_cast<const part_t*>(lds[w]) + threadIdx.x;
+      const part_t p0 = part[0], p1 = part[HC * D / N],
+                   p2 = FEW ? part[2 * HC * D / N] : p1;
       l += ml[w][h][1] * a;
-      float sum = part[0] + part[HC * D];
-      if (FEW) sum += part[2 * HC * D];
-      acc += sum * a;
+#pragma unroll
+      for (int t = 0; t < N; ++t) {
+        float sum = p0[t] + p1[t];
+        if (FEW) sum += p2[t];
+        acc[t] += sum * a;
+      }
     }
     const long row = (long)b * Hq + hk * G + h;
     if (nsplit == 1) {
-      out[row * D + d] = f2bf(l > 0.f ? acc / l : 0.f);
+      struct alignas(2 * N) { bf16_t v[N]; } to;
+#pragma unroll
+      for (int t = 0; t < N; ++t) to.v[t] = f2bf(l > 0.f ? acc[t] / l : 0.f);
+      *reinterpret_cast<decltype(to)*>(out + row * D + d) = to;
     } else {
       float* pp = partial + (row * nsplit + sp) * (D + 2);
-      pp[d] = acc;
+#pragma unroll
+      for (int t = 0; t < N; ++t) pp[d + t] = acc[t];
       if (d == 0) {
         pp[D] = gm * 0.6931471805599453f;
         pp[D + 1] = l;
