@@ -35,6 +35,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 constexpr int DEC_KEYS = 32;          // keys of a wave's round
 constexpr int DEC_HEADS = 8;          // most query heads of a group
+constexpr int DEC_SPLITS = 16;        // most stretches of a row
 
 // the larger / the sum of the four lanes l, l+16, l+32, l+48
 DEV_INLINE float quad_max(float x) {
@@ -476,22 +477,23 @@ __global__ void paged_decode_merge_kernel(
   const long row = blockIdx.x;             // b*Hq + hq
   const int lane = threadIdx.x;
   const float* base = partial + row * (long)nsplit * (D + 2);
-  // stretch lane: its maximum and sum (nsplit <= 64)
+  static_assert(DEC_SPLITS <= 64, "a stretch a lane");
+  // stretch lane: its maximum and sum
   const float m = lane < nsplit ? base[lane * (D + 2) + D] : -1e30f;
   const float w = __expf(m - wave_reduce_max(m));
   const float gl_sum = wave_reduce_sum(
       lane < nsplit ? base[lane * (D + 2) + D + 1] * w : 0.f);
-  // (all stretches, 16 at most, on their way at once: 5.5 us one after the other, 3)
-  float acc[EPL], part[16][EPL];
+  // (all stretches on their way at once: 5.5 us one after the other, 3)
+  float acc[EPL], part[DEC_SPLITS][EPL];
 #pragma unroll
-  for (int sp = 0; sp < 16; ++sp)
+  for (int sp = 0; sp < DEC_SPLITS; ++sp)
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
       part[sp][j] = sp < nsplit ? base[sp * (D + 2) + lane + j * 64] : 0.f;
 #pragma unroll
   for (int j = 0; j < EPL; ++j) acc[j] = 0.f;
 #pragma unroll
-  for (int sp = 0; sp < 16; ++sp) {
+  for (int sp = 0; sp < DEC_SPLITS; ++sp) {
     const float a = __shfl(w, sp, 64);
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
@@ -549,7 +551,7 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
         : most > 4096 && base_blocks >= 128 && base_blocks < 160
             ? 10 : (1024 + base_blocks - 1) / base_blocks;
     nsplit = (int)std::max<long>(
-        1, std::min<long>({want, 16, (most + 127) / 128}));
+        1, std::min<long>({want, DEC_SPLITS, (most + 127) / 128}));
   }
   torch::Tensor ws;                     // per call: any stream, any capture
   float* ppart = nullptr;
