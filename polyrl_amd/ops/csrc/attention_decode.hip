@@ -530,26 +530,32 @@ static void dispatch_g(torch::Tensor& out, const torch::Tensor& q,
   // one to three; of 512 .. 768 24.1, 23.2, 21.9; heads of 64 13.7, 18.4, 17.4).
   //
   // Longer ones: 1024 blocks (25 rows of 1024 .. 2048, 32/8 heads of 128, in 5, 6,
-  // 8 and 10: 34.8, 35.4, 37.4, 38.3), but ten of the longest where seven or eight
-  // are 1024 to 1272 (33 rows of 1900 .. 8192, 28/4 heads, in 8, 9, 10, 12: 72.6, 70.0,
-  // 68.5, 69.5).  From 256 rows and heads on an odd number, which turns the
-  // stretches of a row from die to die: five (33 rows of 2049 .. 8192, 32/8 heads of
-  // 128, in 4, 5, 6: 127, 121, 120; 64 of 2000 .. 4096, heads of 64, in 1 to 6: 85, 89,
-  // 77, 85, 75, 77; 100 of 1500 .. 3000 102, 96, 84, 94, 84, 87), of heads of 128 three
-  // where five are too many (56 of 1024 .. 2048 in 2 to 5: 68.0, 65.0, 67.2, 65.1; 90
-  // of 2000 .. 4096 194, 192, 196, 194).
+  // 8 and 10: 34.8, 35.4, 37.4, 38.3), but never in eight: blocks go to the eight dies
+  // in turn, so that a stretch of every row would go to one die, and the last ones
+  // are the shorter (128, 132, 136, 140 and 144 rows and heads of 28/4, 1900 .. 8192, in
+  // 7, 8, 9 and 10: 65.2, 66.9, 63.1, 63.3; 69.2, 72.3, 68.2, 69.0; 72.9, 74.5, 73.3, 74.3;
+  // 67.4, 68.8, 66.8, 66.7; 72.4, 73.9, 72.2, 72.1; of 1025 .. 5000 45.8, 47.0, 44.4, 45.4
+  // at 132; of heads of 64, 32/8, 1900 .. 8192, 38.3, 39.3, 37.6, 37.6 at 136).  From 256
+  // rows and heads on an odd number for the same reason: five (33 rows of 2049 ..
+  // 8192, 32/8 heads of 128, in 4, 5, 6: 127, 121, 120; 64 of 2000 .. 4096, heads of 64, in
+  // 1 to 6: 85, 89, 77, 85, 75, 77; 100 of 1500 .. 3000 102, 96, 84, 94, 84, 87), of heads
+  // of 128 three where five are too many (56 of 1024 .. 2048 in 2 to 5: 68.0, 65.0, 67.2,
+  // 65.1; 90 of 2000 .. 4096 194, 192, 196, 194).  Of 320 to 960 rows and heads of 1280
+  // to 4096 keys that is 2% from the best of one to seven on average; most of it is
+  // lost up to 2048 keys, where one is up to 15% quicker (heads of 128 from 512 rows
+  // and heads on, of 64 up to 383).
   const long base_blocks = B * Hk;
   const long most = (long)max_pages * page_size;
   int nsplit = 1;
   if (most > 384 && base_blocks < 1024) {
+    const long fill = (1024 + base_blocks - 1) / base_blocks;
     const long want =
         most <= 1024
             ? (base_blocks < 128 ? 512 / base_blocks
                : D == 128 && most > 700 && base_blocks > 256 &&
                          base_blocks < 384 ? 3 : 1)
         : base_blocks >= 256 ? (D == 64 || base_blocks <= 341 ? 5 : 3)
-        : most > 4096 && base_blocks >= 128 && base_blocks < 160
-            ? 10 : (1024 + base_blocks - 1) / base_blocks;
+        : fill == 8 ? 9 : fill;
     nsplit = (int)std::max<long>(
         1, std::min<long>({want, DEC_SPLITS, (most + 127) / 128}));
   }

@@ -730,7 +730,8 @@ def test_decode_stretches(rows, hk, most, d):
 
 @pytest.mark.parametrize("rows,hk,most", [
     (8, 1, 384), (8, 1, 400), (127, 1, 400), (128, 1, 1024), (255, 1, 2064),
-    (256, 1, 2064), (342, 1, 1040), (85, 12, 1040), (128, 8, 1040)])
+    (256, 1, 2064), (342, 1, 1040), (85, 12, 1040), (128, 8, 1040),
+    (127, 1, 2064), (128, 1, 2064), (146, 1, 2064), (147, 1, 2064)])
 @pytest.mark.parametrize("d", [64, 128])
 def test_decode_divided_or_not(rows, hk, most, d):
     """Both sides of the lines from which on rows are divided at all, and among
