@@ -4,8 +4,9 @@ Replaces the reference's external inference engine (SGLang
 behind HTTP).  Token-in / token-out.  The model forward here is a separate
 no-autograd path over the hand-written HIP kernels (ops/): fused-add-RMSNorm,
 table-RoPE, paged decode attention, MFMA varlen prefill attention, SiLU-mul,
-fused sampling with logprob capture; projections on hipBLASLt via torch.matmul
-against fused QKV / gate-up weight buffers.
+fused sampling with logprob capture.  Projections against fused QKV / gate-up
+weight buffers: hipBLASLt, with algorithms chosen per shape for decode steps, and
+for prompts of small models a kernel of this repository (_mm_nt, _gate_up).
 
 Engine weights live in their own contiguous per-layer buffers, decoupled from
 the trainer's FSDP parameters, so weight-version updates are plain copies
@@ -31,17 +32,26 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T; decode-sized GEMMs (M <= 512) go through the
     algo-pinned hipBLASLt path (ops.tuned_mm_nt) — the heuristic pick runs
     skinny decode projections far off the weight-read bound.  Prefill Ms
-    are ragged (chunk sums), so they are not searched: widths up to 1024 take
-    the kernel of this repository, whose call costs the host 15 us less than
-    torch's (a step of 2, 4, 8 and 12 x 256 tokens, 12 layers of 1024, 1080, 1138,
-    1742 and 1884 us with it and 1459, 1496, 1792 and 1909 without; 8192 tokens
-    3845 and 3998); at larger widths and beyond 8192 rows the library's product
-    is the faster by more (2048 -> 3072 of 8192 rows 93 us and 105)."""
+    are ragged (chunk sums), so they are not searched: inner widths up to
+    1024 and up to 3 x 2^22 outputs take the kernel of this repository, whose
+    call costs the host 5 us for the 20 of torch's (a step of 3, 4, 6 and 8 x 256
+    tokens, 12 layers of 1024, 1109, 1124, 1286 and 1447 us with it and 1471, 1491,
+    1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the
+    device it is up to 3.5 us slower within these lines (us, kernel and library,
+    of 513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 7.8, 8.0, 8.5, 10.2, 15.0
+    and 7.2, 7.6, 9.1, 11.6, 16.6; 1024 -> 1024 12.3, 12.3, 13.1, 16.6, 23.9 and
+    8.9, 9.1, 10.9, 14.7, 22.6; 1024 -> 1536 12.4, 12.9, 14.2, 20.4, 32.3 and 9.0,
+    10.5, 13.8, 19.0, 30.2; 1024 -> 4096 of 513 .. 3072 13.5 .. 30.8 and 13.4 ..
+    28.7), beyond them by more than the host gains (1024 -> 4096 of 8192 rows 71.5
+    and 58.2, 1024 -> 32000 of 2048 131 and 116, 2048 -> 3072 of 8192 105 and 93);
+    a captured graph, where the host's time does not count, takes the library's."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 512 \
             and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
     if 512 < x.shape[0] <= 8192 and x.shape[1] <= 1024 \
-            and ops.linear_takes(x, w):
+            and x.shape[0] * w.shape[0] <= 3 << 22 \
+            and ops.linear_takes(x, w) \
+            and not torch.cuda.is_current_stream_capturing():
         return ops.linear_rows(x, w)
     return x @ w.t()
 

@@ -104,17 +104,43 @@ def test_what_it_takes():
             op(x[:1, :64].contiguous(), far[:n])
 
 
-@pytest.mark.parametrize("m", [512, 513])
-def test_engine_prompts(m):
-    """Both sides of the rows from which the engine takes it."""
+@pytest.mark.parametrize("m,n,k,rows,glu", [
+    (512, 1024, 256, False, False), (513, 1024, 256, True, True),
+    (8192, 1536, 128, True, True), (8193, 1280, 128, False, True),
+    (700, 1024, 1024, True, True), (700, 1024, 1088, False, True),
+    (513, 24320, 64, True, True), (513, 24576, 64, False, True),
+    (600, 512, 2048, False, True), (600, 512, 2112, False, False)])
+def test_engine_prompts(m, n, k, rows, glu, monkeypatch):
+    """Both sides of the rows and widths from which the engine takes it, which
+    of the two ran, and that a captured step has the library's product."""
     from polyrl_amd.rollout.engine import _gate_up, _mm_nt
+    ran = []
+    for name in ("linear_rows", "linear_swiglu"):
+        def spy(x, w, name=name, op=getattr(ops, name)):
+            ran.append(name)
+            return op(x, w)
+        monkeypatch.setattr(ops, name, spy)
     g = torch.Generator(device=DEV).manual_seed(m)
-    x = torch.randn(m, 256, generator=g, device=DEV).bfloat16()
-    w = (torch.randn(1024, 256, generator=g, device=DEV) / 16).bfloat16()
-    gate, up = (x.double() @ w.double().t()).chunk(2, -1)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) / k ** 0.5).bfloat16()
+    exact = x.double() @ w.double().t()
+    gate, up = exact.chunk(2, -1)
     want = gate * torch.sigmoid(gate) * up
     off = (_gate_up(x, w).double() - want).norm() / want.norm()
     assert off <= 5e-3                 # three roundings to bf16 at most
+    # (not taken, _gate_up's product goes through _mm_nt)
+    assert ran == ["linear_swiglu"] * glu + ["linear_rows"] * (rows and not glu)
+    del ran[:]
     both = _mm_nt(x, w)
-    off = (both.double() - x.double() @ w.double().t()).norm() / both.norm()
-    assert off <= 5e-3
+    assert (both.double() - exact).norm() / exact.norm() <= 5e-3
+    assert ran == ["linear_rows"] * rows
+    if rows:
+        x @ w.t()                      # (the library's handle and workspace)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            both = _mm_nt(x, w)
+        for _ in range(3):
+            both.zero_()
+            graph.replay()
+            assert (both.double() - exact).norm() / exact.norm() <= 5e-3
+        assert ran == ["linear_rows"]
