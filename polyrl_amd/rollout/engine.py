@@ -58,14 +58,16 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ Wg.T) * (x @ Wu.T), w = [Wg; Wu].  Prompts (the rows that
-    ``_mm_nt`` does not search for) of widths up to 2048 take both products and
-    the activation in one kernel; at larger widths the library's product alone
-    is the faster by more than the activation takes (us, library and activation
-    against one kernel, 513 .. 16384 rows: 1024 -> 4096 21.2 .. 297 and 15.2 .. 259;
-    1536 -> 8960 42 .. 867 and 36 .. 788; 2048 -> 8192 47 .. 925 and 44 .. 930;
-    3584 -> 18944 148 .. 3386 and 171 .. 3393; 4096 -> 14336 133 .. 2805 and 190 ..
-    3042)."""
+    ``_mm_nt`` does not search for) of widths up to 1536, and of up to 8191 rows
+    of widths up to 2048, take both products and the activation in one kernel;
+    elsewhere the library's product alone is the faster by more than the
+    activation takes (us, one kernel against library and activation, of 513,
+    4096, 8192 and 16384 rows: 1024 -> 4096 15.9, 65.5, 121, 247 and 20.8, 76.5,
+    146, 287; 1536 -> 8960 35.4, 202, 382, 756 and 41.5, 228, 443, 839; 2048 ->
+    8192 44.5, 227, 448, 889 and 47.8, 228, 446, 883; of 513 and 16384 3584 -> 18944
+    171, 3393 and 148, 3386; 4096 -> 14336 190, 3042 and 133, 2805)."""
     if x.shape[0] > 512 and x.shape[1] <= 2048 \
+            and (x.shape[1] <= 1536 or x.shape[0] < 8192) \
             and ops.linear_takes(x, w):
         return ops.linear_swiglu(x, w)
     i = w.shape[0] // 2

@@ -109,7 +109,9 @@ def test_what_it_takes():
     (8192, 1536, 128, True, True), (8193, 1280, 128, False, True),
     (700, 1024, 1024, True, True), (700, 1024, 1088, False, True),
     (513, 24320, 64, True, True), (513, 24576, 64, False, True),
-    (600, 512, 2048, False, True), (600, 512, 2112, False, False)])
+    (600, 512, 2048, False, True), (600, 512, 2112, False, False),
+    (8192, 512, 1536, False, True), (8191, 512, 1600, False, True),
+    (8192, 512, 1600, False, False)])
 def test_engine_prompts(m, n, k, rows, glu, monkeypatch):
     """Both sides of the rows and widths from which the engine takes it, which
     of the two ran, and that a captured step has the library's product."""
