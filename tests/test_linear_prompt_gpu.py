@@ -30,10 +30,40 @@ def check(m, n, k, scale=1.0):
     return x, w, got
 
 
+def check_rows(x, w, got):
+    k = x.shape[1]
+    assert got.shape == (x.shape[0], w.shape[0])
+    for at in range(0, x.shape[0], 8192):
+        a = x[at:at + 8192].double()
+        want, mass = a @ w.double().t(), a.abs() @ w.double().abs().t()
+        bound = 2 ** -8 * want.abs() + k * 2.0 ** -24 * mass
+        assert ((got[at:at + 8192].double() - want).abs() <= bound).all(), at
+
+
+def row_tiles(m, cols, k):
+    """The row tiles of a block: the fewest that end the last round of 256 blocks
+    earliest."""
+    def cost(jt):
+        blocks = -(-m // (32 * jt)) * cols
+        return -(-blocks // 256) * ((jt + 1) * (k // 64) + 20)
+    return min(range(2, 9), key=cost)
+
+
 @pytest.mark.parametrize("tiles", [2, 3, 4, 5, 6, 7, 8, 9])
 def test_row_tiles(tiles):
     """Rows that fill 256 blocks of ``tiles`` row tiles but for a remainder."""
     check(8192 * tiles - 17, 128, 64)
+
+
+@pytest.mark.parametrize("tiles", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("inner", [2, 3, 4, 5, 16])
+def test_inner_tiles(tiles, inner):
+    """Every number of row tiles with inner tiles that fill the buffers just, take
+    their places in turn and go round; an incomplete last row tile."""
+    m, k = 8192 * tiles - 17, 64 * inner
+    assert row_tiles(m, 1, k) == tiles
+    x, w, _ = check(m, 128, k)
+    check_rows(x, w, ops.linear_rows(x, w))
 
 
 @pytest.mark.parametrize("m", [1, 31, 32, 33, 64, 65, 127, 513, 700])
@@ -50,17 +80,10 @@ def test_edges(m, n, k):
 @pytest.mark.parametrize("n,k", [(256, 64), (768, 192), (1280, 128)])
 def test_rows(m, n, k):
     """The product alone at the same edges, column tiles in one group and two."""
-    if m > 1000 and n > 256:
-        return
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
     w = torch.randn(n, k, generator=g, device=DEV).bfloat16()
-    got = ops.linear_rows(x, w)
-    for at in range(0, m, 8192):
-        a = x[at:at + 8192].double()
-        want, mass = a @ w.double().t(), a.abs() @ w.double().abs().t()
-        bound = 2 ** -8 * want.abs() + k * 2.0 ** -24 * mass
-        assert ((got[at:at + 8192].double() - want).abs() <= bound).all(), at
+    check_rows(x, w, ops.linear_rows(x, w))
 
 
 def test_large_gates():
