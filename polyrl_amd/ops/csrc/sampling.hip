@@ -89,7 +89,8 @@ DEV_INLINE float gumbel(uint32_t bits) {
   return -__logf(fmaxf(-__logf(u), 0x1p-25f));
 }
 
-// The same noise within 1e-6 of itself and 1e-6, in seven instructions for thirty
+// The same noise in seven instructions for thirty.  Over all 2^24 inputs the two
+// are at most 1.91e-6 apart, and at most 2.2e-7 of 1 + the noise.
 DEV_INLINE float gumbel_about(uint32_t bits) {
   const float u = ((float)(bits >> 8) + 1.0f) * (1.0f / 16777216.0f);
   const float l = -0.6931471805599453f * __builtin_amdgcn_logf(u);
@@ -580,7 +581,7 @@ DEV_INLINE void read_bins(int digit, const uint32_t* h, uint32_t* cnt,
   __syncthreads();
 }
 
-// the block's best entry, in the first wave
+// the block's best entry, in every wave
 DEV_INLINE void block_best(float& best, int& best_i, Share* part) {
   wave_best(best, best_i);
   if ((threadIdx.x & 63) == 0)

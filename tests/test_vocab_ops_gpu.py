@@ -461,8 +461,9 @@ def test_logprobs_on_both_sides_of_the_caches(n, v):
 def test_sample_block_sizes(n, v, dtype):
     """Without a filter, over the numbers of rows at which blocks of 256, 512
     and 1024 threads take the pieces: the draw is the filtered path's, which
-    has other pieces, entry by entry.  Rows of few possible entries, of one, of
-    large logits and of a temperature that is not positive among them."""
+    has other pieces, entry by entry (both judge first words by approximate
+    noise; the next test's other side does not).  Rows of few possible entries,
+    of one, of large logits and of a temperature that is not positive among them."""
     torch.manual_seed(21)
     x = (torch.randn(n, v, device=DEV) * 3).to(dtype)
     x[1, 100:] = -float("inf")
@@ -484,6 +485,34 @@ def test_sample_block_sizes(n, v, dtype):
         z = x[r].double().cpu() / float(temp[r]) + noise(77, r, v)
         # 32-bit logarithms of 24-bit numbers: 1e-4 where the noise is large
         assert z[int(tok[r])] >= z.max() - 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,v", [(64, 98305), (128, 65537), (180, 40003),
+                                 (256, 65539), (1030, 65537), (16, 128256),
+                                 (300, 9000)])
+def test_sample_draw_without_approximate_noise(n, v, dtype):
+    """Without a filter the draw is that of a filter which keeps the entries that
+    can win: that one has a threshold, and takes the exact noise of all of them.
+    Half of the entries stand in the words that the blocks' waves read first."""
+    m = 12
+    g = torch.Generator().manual_seed(n)
+    x = torch.full((n, v), -200.0)
+    at = torch.stack([torch.cat([
+        torch.randperm(4096, generator=g)[:m // 2],
+        4096 + torch.randperm(v - 4096, generator=g)[:m // 2]])
+        for _ in range(n)])
+    x = x.scatter_(1, at, torch.randn(n, m, generator=g)).to(dtype).to(DEV)
+    full = lambda t, ty: torch.full((n,), t, dtype=ty, device=DEV)
+    for seed in range(8):
+        temp, p = full(0.9, torch.float32), full(1.0, torch.float32)
+        tok, lp = ops.sample(x, temp, full(-1, torch.int32), p, seed,
+                             no_filter=True)
+        other, olp = ops.sample(x, temp, full(m, torch.int32), p, seed,
+                                no_filter=False)
+        assert torch.equal(tok, other), seed
+        assert (x.gather(1, tok[:, None]) > -100).all()
+        assert (lp - olp).abs().max() <= 1e-5
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
