@@ -570,3 +570,21 @@ def test_prompts_on_any_name_of_the_cpu(device):
                  dtype=torch.float32, page_size=4, kv_token_capacity=64,
                  max_running_requests=2)
     assert eng.step_forced([("r", [1, 2, 3], [2])]).shape[0] == 1
+
+
+def test_prompt_products_on_the_cpu():
+    """The products of prompts without a GPU: what the layers compute there."""
+    import polyrl_amd.ops as ops
+    from polyrl_amd.rollout.engine import _gate_up, _mm_nt
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(600, 64, generator=g)
+    w = torch.randn(256, 64, generator=g) / 8
+    assert not ops.linear_takes(x.bfloat16(), w.bfloat16())
+    gate, up = (x.double() @ w.double().t()).chunk(2, -1)
+    want = gate * torch.sigmoid(gate) * up
+    # 32-bit sums of 64 products
+    for got in (ops.linear_swiglu(x, w), _gate_up(x, w)):
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()
+    for got in (ops.linear_rows(x, w), _mm_nt(x, w)):
+        want = x.double() @ w.double().t()
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()
