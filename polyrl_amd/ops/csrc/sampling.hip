@@ -289,13 +289,18 @@ struct Draw {
   }
 };
 
-// sums of a whole row (every lane of the wave gets them); split <= 64
+// sums of a whole row (every lane of the wave gets them, after wave()); split <= 64
 template <bool TEMP>
-DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
+DEV_INLINE Sums<TEMP> piece_sums(const Share* share, int split) {
   const int lane = threadIdx.x & 63;
   Sums<TEMP> a;
   if (lane < split)
     a.m = share[lane].m, a.s = share[lane].s, a.st = share[lane].st;
+  return a;
+}
+template <bool TEMP>
+DEV_INLINE Sums<TEMP> row_sums(const Share* share, int split, float inv_temp) {
+  Sums<TEMP> a = piece_sums<TEMP>(share, split);
   a.wave(inv_temp);
   return a;
 }
@@ -699,8 +704,10 @@ __global__ __launch_bounds__(NT) void sample_pass_kernel(
   }
 
   __shared__ uint32_t known;
-  Draw::start(&known);
-  __syncthreads();
+  if (MODE != 1 && !greedy) {         // (who draws)
+    Draw::start(&known);
+    __syncthreads();
+  }
   Sums<MODE == 1> sums;
   Draw d(&known);
   walk<MODE, NT>(r, piece * NT, split * NT, greedy, inv_temp, rowkey, tau, sums,
@@ -860,15 +867,16 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
   list_v += row * LISTED, list_i += row * LISTED;
   // The maxima come with the pieces' sums, not once for the cut and once more for
   // the list's length: the block is a chain of such waits.
+  // (behind them: a row at a temperature of 0 waits for the sums alone)
+  Sums<true> all = piece_sums<true>(share, split);
   const int most = split * TOPS;
   float top[MOST_TOPS][4];
+  const int top_at = (threadIdx.x & 63) * 4;            // (four lanes a piece)
   auto read_tops = [&](int c) {
-    const int at = c * 256 + (threadIdx.x & 63) * 4;    // (four lanes a piece)
+    const int at = c * 256 + top_at;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float t = tops[row * most + (at < most ? at : 0) + w];
-      top[c][w] = at < most ? t : -INFINITY;
-    }
+    for (int w = 0; w < 4; ++w)
+      top[c][w] = tops[row * most + (at < most ? at : 0) + w];
   };
   read_tops(0);
   if (most > 256) {
@@ -879,7 +887,7 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
     for (int c = 1; c < MOST_TOPS; ++c)
       top[c][0] = top[c][1] = top[c][2] = top[c][3] = -INFINITY;
   }
-  const Sums<true> all = row_sums<true>(share, split, inv_temp);
+  all.wave(inv_temp);
   if (!by_k && !by_p) {
     if (piece != 0) return;
     if (threadIdx.x == 0) plans[row] = Plan(-INFINITY, all, p, false, false);
@@ -891,6 +899,11 @@ __global__ __launch_bounds__(SNT) void sample_select_kernel(
   }
   // (one wave looks: sixteen a CU would take turns at the same scalar counts)
   if (threadIdx.x < 64) {
+#pragma unroll
+    for (int i = 0; i < MOST_TOPS; ++i)
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (i * 256 + top_at >= most) top[i][w] = -INFINITY;
     const float c = wave_cut<T>(top, most, by_k, by_p, k, p, inv_temp, all, V);
     // (a list needs numbers that add up)
     bool list = c > -INFINITY && inv_temp > 0.f && fabsf(all.m) < INFINITY &&
@@ -1101,7 +1114,7 @@ __global__ __launch_bounds__(NT) void sample_row_kernel(
 
   __shared__ uint32_t known;
   Draw::start(&known);
-  __syncthreads();
+  if (!FILTER && !greedy) __syncthreads();   // (with a filter others are between)
   Sums<FILTER> sums;
   Draw d(&known);
   walk<FILTER ? 1 : 0, NT>(r, 0, NT, greedy, inv_temp, rowkey, 0u, sums, d);
