@@ -22,7 +22,7 @@
 // this one's products, and three blocks of large calls on a CU, change nothing
 // (38.2 and 68.0 us with, 38.6 and 68.4 without; both together 38.0 and 76).
 // Measured (inputs of three layers in turn): those 128 rows 41.2 us with K in 64-byte
-// pieces through the caches, 38.6 now (5.2 TB/s); those 33 rows 77.1, 68.5, of which
+// pieces through the caches, 38.0 now (5.3 TB/s); those 33 rows 77.1, 68.0, of which
 // the merge's loads one after the other were 2.5.  (With per-key dot products,
 // shuffles and exponentials on the vector units it was bound by those: 1.4 TB/s at
 // seven heads a group, 4.1 at four.)

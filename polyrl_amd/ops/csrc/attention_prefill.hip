@@ -33,7 +33,9 @@
 // of 64: 671 us a call with those and the tile table's trip through the host (50
 // us), 154 with tiles through registers and three blocks per CU, 141 now (757
 // TFLOP/s of live pairs); of 128: 283 in the sequences' order, 280, 243 now; two
-// sequences of 3500 .. 4096, 28/4 heads of 128, 323, 265, 222.  Up to 64 sequences
+// sequences of 3500 .. 4096, 28/4 heads of 128, 323, 265, 222.  Where the prompts took
+// 147.5 (another card) they took 128 with no tile loaded after the first and 128
+// without exponentials, of 128 248, 205 and 231.  Up to 64 sequences
 // run in the order of their walks, more in the table's (as all did before: 100
 // prompts of 21 .. 80 take what they took).  A maximum that may lag by 2^6 saves
 // the rescaling in most tiles (5 to 7%), but then a row's largest weight is no

@@ -280,9 +280,9 @@ DEV_INLINE int wave_total(int x) {
 // Up to 16 sequences the count is taken for 64 lengths at once, one a lane, five
 // instructions a sequence; of more a search by halves sums over the lanes ten times.
 // (With blocks that find their heads and parts without divisions, and rows written
-// by stores that end with the buffer, eight prompts of 1200 .. 2048, 32/8 heads of 64,
-// 143.8 -> 139.8 us; 16 sequences of 300 .. 512, 32/8 of 128, forward and backward 224.4
-// -> 221.1; one prompt of 512 14.9 -> 14.4.)
+// by stores that end with the buffer, timed in turn on one card: eight prompts of 1200
+// .. 2048, 32/8 heads of 64, 149.7 -> 147.5 us; 16 sequences of 300 .. 512, 32/8 of 128,
+// forward and backward 225 -> 221; one prompt of 512 15.4 -> 14.7.)
 //
 // In the table's order, from the end where late tiles walk longest: tables of
 // another length (of some of the tiles), more sequences than lanes, and calls

@@ -27,8 +27,10 @@
 // one tile ahead 5135 rows, 1024 -> 4096, 88.9, 513 rows 16.3, 1024 rows, 1536 -> 8960,
 // 71.6.  Reading the fragments of the next 16 inner numbers ahead of the barrier
 // takes 5% more, rows in groups of 64 (four row groups, two column groups) the
-// same.  x W^T alone: 1024 -> 1024 of 1024, 4096, 5135 and 16384 rows 12.4, 14.6, 17.6, 36
-// for 9.1, 13.7, 20.4, 33; 2048 -> 3072 22, 54, 62, 183 for 20, 47, 53, 152.
+// same.  x W^T alone, for the library: 1024 -> 1024 of 1024, 4096, 5135 and 8192 rows
+// 12.3, 16.6, 19.1, 23.9 for 9.1, 14.7, 21.3, 22.6; 512 -> 1536 8.3, 13.2, 14.8, 21.2 for 9.3,
+// 15.0, 16.8, 28.7; 1024 -> 4096 16.3, 37.1, 53.4, 71.5 for 14.4, 31.8, 49.4, 58.2; 2048 -> 3072
+// of 1024 and 4096 22, 54 for 20, 47.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

@@ -380,10 +380,11 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(
 // into LDS (AttnTile::gather), buffers and blocks per CU as in
 // attention_prefill.hip.  Measured, eight prompts of 1200 .. 2048 tokens, window
 // 1024, 32/8 heads of 64: 547 us in the general kernel, 155 with tiles through
-// registers and three blocks per CU, 138 here (119 with no tile loaded after the
-// first); of 128: 270 and 243.  Row tiles run by their number: longest walk first
-// found from the tables, as attention_prefill.hip finds it from the lengths, took
-// 157 for 156 (windowed walks are alike).
+// registers and three blocks per CU, 138 here; of 128: 270 and 243.  Where that took
+// 149 (another card) it took 126 with no tile loaded after the first and 131 without
+// exponentials.  Row tiles run by their number: longest walk first found from the
+// tables, as attention_prefill.hip finds it from the lengths, took 157 for 156 when
+// tiles went through registers (windowed walks are alike).
 // ONE_V: one buffer of values, heads of 128 then run three blocks per CU, not two
 template <int D, bool ONE_V>
 __global__ __launch_bounds__(256, D == 64 ? 4 : ONE_V ? 3 : 2)
