@@ -17,6 +17,7 @@
 //   fwd  (nt): Y[M,N] = X[M,K] @ W[N,K]^T  ->  C(N,M) = op_T(W) op_N(X)
 //   dgrad(nn): dX[M,K] = dY[M,N] @ W[N,K]  ->  C(K,M) = op_N(W) op_N(dY)
 //   wgrad(tn): dW[N,K] = dY[M,N]^T @ X[M,K]->  C(K,N) = op_N(X) op_T(dY)
+// Weight gradients of many rows are the kernel's in linear_wgrad.hip.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hipblaslt/hipblaslt.h>
@@ -32,6 +33,10 @@
     TORCH_CHECK(s_ == HIPBLAS_STATUS_SUCCESS, "hipblaslt error ", (int)s_, \
                 " at " #expr);                                            \
   } while (0)
+
+// linear_wgrad.hip
+bool linear_wgrad_takes(const torch::Tensor& dy, const torch::Tensor& x);
+torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x);
 
 namespace {
 
@@ -230,6 +235,7 @@ torch::Tensor tuned_linear_wgrad(torch::Tensor dy, torch::Tensor x) {
   check2d(x, "x");
   const int64_t M = dy.size(0), N = dy.size(1), K = x.size(1);
   TORCH_CHECK(x.size(0) == M, "shape mismatch");
+  if (linear_wgrad_takes(dy, x)) return linear_wgrad(dy, x);
   auto dw = torch::empty({N, K}, dy.options());
   tuned_mm(2, dy, x, dw, M, N, K);
   return dw;
