@@ -95,8 +95,12 @@ class RotaryCache(nn.Module):
         self.register_buffer("cos_cached", torch.empty(0), persistent=False)
         self.register_buffer("sin_cached", torch.empty(0), persistent=False)
 
-    def get(self, positions: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-        need = int(positions.max().item()) + 1 if positions.numel() else 1
+    def get(self, positions: torch.Tensor, need: Optional[int] = None
+            ) -> Tuple[torch.Tensor, torch.Tensor]:
+        """``need``: one more than the largest position, where the host has it
+        (else it waits for the device)."""
+        if need is None:
+            need = int(positions.max().item()) + 1 if positions.numel() else 1
         if self.cos_cached.numel() == 0 or self.cos_cached.shape[0] < need or \
                 self.cos_cached.device != positions.device:
             n = max(need, 512)
@@ -339,36 +343,110 @@ class DecoderModel(nn.Module):
                              "shard": shard}
         return x                                    # (Tp/sp, H)
 
-    def _forward_packed(self, input_ids, attention_mask, position_ids):
+    def _embed(self, ids):
+        """Embedding rows of packed tokens, by ops.embed_train where the module
+        does nothing else."""
+        m = self.embed_tokens
+        w = m.weight
+        if (type(m) is nn.Embedding and w.is_cuda
+                and w.dtype == torch.bfloat16 and not hasattr(w, "placements")
+                and w.shape[1] % 8 == 0 and ids.shape[0] <= 32768
+                and m.padding_idx is None and m.max_norm is None
+                and not m.scale_grad_by_freq and not m.sparse
+                and not (m._forward_hooks or m._forward_pre_hooks
+                         or m._backward_hooks or m._backward_pre_hooks)):
+            import polyrl_amd.ops as pops
+            return pops.embed_train(ids, w)
+        return m(ids)
+
+    def _padded_tokens(self, T: int) -> int:
+        """Rows of a packed batch of T tokens.
+
+        Dynamic token-budget micros produce arbitrary totals (6472, 7216, ...)
+        and hipBLASLt loses ~35-45% on the [M,14336]x[14336,4096] trunk
+        GEMMs at unaligned M (profiles/PROFILES.md).  Fixed-M padding only pays off when the micro is nearly full
+        (dense packing leaves one small tail micro — padding THAT to the
+        whole budget would waste more GEMM work than the shape buys)."""
+        align = _pack_align()
+        pad_to = _pack_pad_to(self)
+        if pad_to and 0.75 * pad_to <= T <= pad_to:
+            return pad_to
+        return -(-T // align) * align if align > 1 else T
+
+    def _pack_gpu(self, valid, input_ids, position_ids, lo, hi):
+        """The packed batch by the kernels of pack_train.hip, one wait of the
+        host: (tokens, positions, one more than the largest position,
+        (cu, tiles), packed rows of places [lo, hi), place of every packed row)
+        or None where there is no token."""
+        import polyrl_amd.ops as pops
+        ext = pops._require_ext()
+        lens, most = ext.pack_lengths(valid, position_ids).tolist()
+        T = sum(lens)
+        if T == 0:
+            return None
+        Tp = self._padded_tokens(T)
+        if Tp != T:
+            lens.append(Tp - T)
+        cu, tiles = pops.packed_tables(lens, input_ids.device)
+        ids_p, pos_p, packed, place = ext.pack_rows(
+            valid, input_ids, position_ids, cu, T, Tp, lo, hi)
+        return (ids_p, pos_p, max(max(most), Tp - T - 1) + 1, (cu, tiles),
+                packed, place)
+
+    def _packed_layers(self, x, cos, sin, cu_pack):
+        for layer in self.layers:
+            if self.gradient_checkpointing and self.training:
+                x = torch.utils.checkpoint.checkpoint(
+                    layer, x, cos, sin, None, None, cu_pack,
+                    use_reentrant=False)
+            else:
+                x = layer(x, cos, sin, None, None, cu_pack)
+        return _norm(self.norm, x)
+
+    def _forward_packed(self, input_ids, attention_mask, position_ids,
+                        rows: Optional[slice] = None):
         """Remove-padding path (reference: use_remove_padding + flash varlen,
         SURVEY.md §5.7): pack the valid tokens of all rows, run every layer
         on (total, H) with block-diagonal causal flash attention, scatter
         back to (B, L, H).  12-25%% fewer tokens through every GEMM on
-        typical left-padded prompt batches, and no SDPA mask fallback."""
+        typical left-padded prompt batches, and no SDPA mask fallback.
+        ``rows``: the places along L whose hidden rows are wanted."""
         B, L = input_ids.shape
         valid = attention_mask.bool()
+        rows = slice(None) if rows is None else rows
+        w = self.embed_tokens.weight
+        if input_ids.is_cuda and w.dtype == torch.bfloat16 \
+                and w.shape[1] % 8 == 0 and valid.dim() == 2 \
+                and valid.shape == position_ids.shape == (B, L) \
+                and B > 0 and B * L < 2 ** 31:
+            lo, hi, step = rows.indices(L)
+            if step != 1:
+                lo, hi = 0, L
+            pack = self._pack_gpu(
+                valid.contiguous(), input_ids.long().contiguous(),
+                position_ids.long().contiguous(), lo, max(lo, hi))
+            if pack is not None:
+                import polyrl_amd.ops as pops
+                ids_p, pos_p, need, cu_pack, packed, place = pack
+                cos, sin = self.rotary.get(pos_p, need)
+                x = self._packed_layers(self._embed(ids_p), cos, sin, cu_pack)
+                if x.dtype == torch.bfloat16:
+                    out = pops.rows_from_packed(x, packed, place)
+                else:
+                    out = x.new_zeros(*packed.shape, x.shape[-1])
+                    out[packed >= 0] = x[place >= 0]
+                return out if step == 1 else out[:, rows]
         seqlens = valid.sum(-1).int()
         cu = torch.zeros(B + 1, dtype=torch.int32, device=input_ids.device)
         torch.cumsum(seqlens, 0, out=cu[1:])
         ids_p = input_ids[valid]                     # (total,)
         pos_p = position_ids[valid]
-        # Pad the packed token count to a multiple of PACK_ALIGN: dynamic
-        # token-budget micros produce arbitrary totals (6472, 7216, ...)
-        # and hipBLASLt loses ~35-45% on the [M,14336]x[14336,4096] trunk
-        # GEMMs at unaligned M (measured: profiles/PROFILES.md round 2).
+        # Pad the packed token count to a multiple of PACK_ALIGN.
         # The pad rows form one trailing fake sequence so attention output
         # stays finite (their grads are exactly zero — the scatter below
         # never reads them).
         T = int(ids_p.shape[0])
-        align = _pack_align()
-        pad_to = _pack_pad_to(self)
-        # fixed-M padding only pays off when the micro is nearly full
-        # (dense packing leaves one small tail micro — padding THAT to the
-        # whole budget would waste more GEMM work than the shape buys)
-        if pad_to and 0.75 * pad_to <= T <= pad_to:
-            Tp = pad_to
-        else:
-            Tp = -(-T // align) * align if align > 1 else T
+        Tp = self._padded_tokens(T)
         if Tp != T:
             padn = Tp - T
             ids_p = torch.cat([ids_p, ids_p.new_zeros(padn)])
@@ -383,21 +461,17 @@ class DecoderModel(nn.Module):
             tiles = pops.build_varlen_tiles(cu.cpu(), input_ids.device)
         else:
             tiles = None
-        cu_pack = (cu, tiles)
-        for layer in self.layers:
-            if self.gradient_checkpointing and self.training:
-                x = torch.utils.checkpoint.checkpoint(
-                    layer, x, cos, sin, None, None, cu_pack,
-                    use_reentrant=False)
-            else:
-                x = layer(x, cos, sin, None, None, cu_pack)
-        x = _norm(self.norm, x)
+        x = self._packed_layers(x, cos, sin, (cu, tiles))
         out = torch.zeros(B, L, x.shape[-1], dtype=x.dtype, device=x.device)
         out[valid] = x[:T]
-        return out
+        return out[:, rows]
 
-    def forward(self, input_ids, attention_mask=None, position_ids=None):
-        """With Ulysses SP enabled, every SP rank passes the SAME full
+    def forward(self, input_ids, attention_mask=None, position_ids=None,
+                rows: Optional[slice] = None):
+        """``rows``: a slice along L, the places whose hidden rows are returned
+        (not under Ulysses SP, whose ranks hold shards).
+
+        With Ulysses SP enabled, every SP rank passes the SAME full
         (B, L) inputs (L divisible by sp); the returned hidden states are
         this rank's (B, L/sp, H) sequence shard."""
         B, L = input_ids.shape
@@ -416,7 +490,7 @@ class DecoderModel(nn.Module):
                 # head count not divisible: padded SDPA fallback below
             else:
                 return self._forward_packed(input_ids, attention_mask,
-                                            position_ids)
+                                            position_ids, rows)
         if position_ids is None:
             position_ids = torch.arange(L, device=input_ids.device).expand(B, L)
         # per-row rope tables shaped for broadcast: (B, 1, L, D/2)
@@ -450,7 +524,8 @@ class DecoderModel(nn.Module):
                     use_reentrant=False)
             else:
                 x = layer(x, cos, sin, attn_bias_mask, sp_group)
-        return self.norm(x)
+        x = self.norm(x)
+        return x if rows is None or sp_on else x[:, rows]
 
 
 class CausalLM(nn.Module):
@@ -482,10 +557,9 @@ class CausalLM(nn.Module):
         BEFORE lm_head — avoids materializing vocab logits over prompt
         positions when only response logprobs are needed.  Ignored under
         Ulysses SP (hidden is a sequence shard; the worker gathers)."""
-        hidden = self.model(input_ids, attention_mask, position_ids)
         sp_on = self.model.ulysses is not None and self.model.ulysses.enabled
-        if logits_slice is not None and not sp_on:
-            hidden = hidden[:, logits_slice]
+        rows = {} if logits_slice is None or sp_on else {"rows": logits_slice}
+        hidden = self.model(input_ids, attention_mask, position_ids, **rows)
         return _lin(self.lm_head, hidden.contiguous())
 
     @torch.no_grad()

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import ref
@@ -522,6 +523,70 @@ def build_varlen_tiles(cu_seqlens_cpu: torch.Tensor, device):
     t32 = _build_prefill_tiles(cu_seqlens_cpu, qtile=32)
     return (t64[0].to(device), t64[1].to(device),
             t32[0].to(device), t32[1].to(device))
+
+
+def packed_tables(lens, device):
+    """(cu_seqlens, tiles of :func:`build_varlen_tiles`) of packed sequences
+    whose lengths the host has: one upload that nothing waits for."""
+    n = np.asarray(lens, np.int64)
+
+    def tiles(rows):
+        per = -(-n // rows)
+        first = np.repeat(np.cumsum(per) - per, per)
+        return (np.repeat(np.arange(len(n)), per),
+                (np.arange(len(first)) - first) * rows)
+
+    parts = [np.concatenate([[0], np.cumsum(n)]), *tiles(64), *tiles(32)]
+    host = torch.empty(sum(map(len, parts)), dtype=torch.int32,
+                       pin_memory=True)
+    np.concatenate(parts, out=host.numpy(), casting="unsafe")
+    cu, *rest = host.to(device, non_blocking=True).split(
+        [len(p) for p in parts])
+    return cu, tuple(rest)
+
+
+class _RowsFromPacked(torch.autograd.Function):
+    """Rows of packed hidden states at the places of a padded batch (zeros
+    where a place has no token), and the gradient back by the same gather the
+    other way (pack_train.hip)."""
+
+    @staticmethod
+    def forward(ctx, x, packed, place):
+        ctx.save_for_backward(place)
+        return _require_ext().gather_rows(x.contiguous(), packed)
+
+    @staticmethod
+    def backward(ctx, dout):
+        place, = ctx.saved_tensors
+        dout = dout.reshape(-1, dout.shape[-1]).contiguous()
+        return _require_ext().gather_rows(dout, place), None, None
+
+
+def rows_from_packed(x: torch.Tensor, packed: torch.Tensor,
+                     place: torch.Tensor) -> torch.Tensor:
+    """x (T, H), packed (B, L') row of x of every place or -1, place (T) the
+    place of every row or -1 -> (B, L', H), differentiable."""
+    return _RowsFromPacked.apply(x, packed, place)
+
+
+class _EmbedTrain(torch.autograd.Function):
+    """Embedding rows; the weight's gradient in four launches and a fill."""
+
+    @staticmethod
+    def forward(ctx, weight, ids):
+        ctx.save_for_backward(ids)
+        ctx.vocab = weight.shape[0]
+        return torch.nn.functional.embedding(ids, weight)
+
+    @staticmethod
+    def backward(ctx, dy):
+        ids, = ctx.saved_tensors
+        return _require_ext().embed_grad(dy.contiguous(), ids, ctx.vocab), None
+
+
+def embed_train(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """weight[ids] of ids (T) int64, T <= 32768, bf16 on the GPU."""
+    return _EmbedTrain.apply(weight, ids)
 
 
 def flash_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

@@ -60,6 +60,13 @@ torch::Tensor gather_logprobs_train_bwd(torch::Tensor logits,
                                         torch::Tensor dlp);
 torch::Tensor rope_train_apply(torch::Tensor x, torch::Tensor cos_t,
                                torch::Tensor sin_t, bool backward);
+torch::Tensor pack_lengths(torch::Tensor mask, torch::Tensor pos);
+std::vector<torch::Tensor> pack_rows(torch::Tensor mask, torch::Tensor ids,
+                                     torch::Tensor pos, torch::Tensor cu,
+                                     int64_t total, int64_t padded, int64_t lo,
+                                     int64_t hi);
+torch::Tensor gather_rows(torch::Tensor x, torch::Tensor map);
+torch::Tensor embed_grad(torch::Tensor dy, torch::Tensor ids, int64_t V);
 torch::Tensor tuned_linear_fwd(torch::Tensor x, torch::Tensor w);
 torch::Tensor tuned_linear_dgrad(torch::Tensor dy, torch::Tensor w);
 torch::Tensor tuned_linear_wgrad(torch::Tensor dy, torch::Tensor x);
@@ -104,6 +111,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "dlogits = dlp * (onehot - softmax), one pass");
   m.def("rope_train_apply", &rope_train_apply,
         "trainer NEOX RoPE (one pass; backward = rotate by -theta)");
+  m.def("pack_lengths", &pack_lengths,
+        "real tokens of a padded batch's rows, their largest positions");
+  m.def("pack_rows", &pack_rows,
+        "packed tokens and positions, packed rows of places and back");
+  m.def("gather_rows", &gather_rows, "rows that a map names, zeros where none");
+  m.def("embed_grad", &embed_grad, "embedding gradient, fp32 sums in row order");
   m.def("tuned_linear_fwd", &tuned_linear_fwd,
         "Y = X W^T via hipBLASLt with per-shape in-process algo search");
   m.def("tuned_linear_dgrad", &tuned_linear_dgrad, "dX = dY W (algo-pinned)");
