@@ -102,9 +102,11 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
 // -------------------------------------------------------- embedding gradient
 // Tokens in the order (id, row): a token's place is the number of tokens before it
 // in that order, counted by comparing it with all, 256 of them and a stretch of the
-// others a block (16384 tokens, 2.7e8 comparisons, take what a radix sort's ten
-// launches do; the counts add up the same in any order).
-constexpr int STRETCH = 1024;
+// others a block; the counts add up the same in any order.  (7168 tokens, rows of 4096
+// numbers, 128256 ids: ranks 11 us, order 5, sums 39, shares 5, the fill 139; a sort's
+// scans and merges, sums and their scatter took 300 beside the fill.  Comparisons grow
+// with the square of the tokens: beyond 32768 the library's backward.)
+constexpr int STRETCH = 256;
 
 __global__ __launch_bounds__(256) void embed_rank_kernel(
     int* __restrict__ rank, const int64_t* __restrict__ ids, int T) {
@@ -117,6 +119,7 @@ __global__ __launch_bounds__(256) void embed_rank_kernel(
   int n = 0;
   // an earlier row of the same id counts, a later one does not
   const int same = min(max(t - o0, 0), STRETCH);
+#pragma unroll 8
   for (int i = 0; i < STRETCH; i += 4) {
     const i32x4_t o = *reinterpret_cast<const i32x4_t*>(other + i);
 #pragma unroll
@@ -145,21 +148,39 @@ __global__ __launch_bounds__(256) void embed_sum_kernel(
     bf16_t* __restrict__ dw, float* __restrict__ shares,
     const bf16_t* __restrict__ dy, const int* __restrict__ order,
     const int* __restrict__ sorted, int T, int H, int V) {
-  const int p = blockIdx.x, id = sorted[p];
-  const bool starts = p == 0 || sorted[p - 1] != id;
-  if ((!starts && p % WINDOW != 0) || (unsigned)id >= (unsigned)V) return;
+  const int p = blockIdx.x, lane = threadIdx.x & 63;
   const int border = min((p / WINDOW + 1) * WINDOW, T);
-  int end = p + 1;
-  while (end < border && sorted[end] == id) ++end;
-  const bool goes_on = end == border && end < T && sorted[end] == id;
+  // lane l < 32: place p + l and its row; lane 63: the place before
+  const int at = lane == 63 ? p - 1 : p + lane;
+  int own = -1, row = 0;
+  if (at >= 0 && at <= border && at < T) own = sorted[at], row = order[at];
+  const int id = uniform(own);
+  const bool starts = p == 0 || __builtin_amdgcn_readlane(own, 63) != id;
+  if ((!starts && p % WINDOW != 0) || (unsigned)id >= (unsigned)V) return;
+  const unsigned long long same = __ballot(own == id && lane <= WINDOW);
+  const int n = min(__ffsll((long long)~same) - 1, border - p);
+  const bool goes_on = border < T && (same >> (border - p) & 1) &&
+                       n == border - p;
   const int windows = (T + WINDOW - 1) / WINDOW;
   for (int h = threadIdx.x * 8; h < H; h += 256 * 8) {
     float sum[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) sum[e] = 0.f;
-    for (int r = p; r < end; ++r) {
-      const bf16x8_t v =
-          *reinterpret_cast<const bf16x8_t*>(dy + (long)order[r] * H + h);
+    int r = 0;
+    for (; r + 4 <= n; r += 4) {       // (four rows on their way at once)
+      bf16x8_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = *reinterpret_cast<const bf16x8_t*>(
+            dy + (long)__builtin_amdgcn_readlane(row, r + i) * H + h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] += (float)v[i][e];
+    }
+    for (; r < n; ++r) {
+      const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(
+          dy + (long)__builtin_amdgcn_readlane(row, r) * H + h);
 #pragma unroll
       for (int e = 0; e < 8; ++e) sum[e] += (float)v[e];
     }
