@@ -71,6 +71,7 @@ torch::Tensor tuned_linear_fwd(torch::Tensor x, torch::Tensor w);
 torch::Tensor tuned_linear_dgrad(torch::Tensor dy, torch::Tensor w);
 torch::Tensor tuned_linear_wgrad(torch::Tensor dy, torch::Tensor x);
 torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x);
+torch::Tensor linear_dgrad(torch::Tensor dy, torch::Tensor w);
 void varlen_attention_backward_v3(
     torch::Tensor dq, torch::Tensor dk, torch::Tensor dv,
     torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -119,10 +120,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_grad", &embed_grad, "embedding gradient, fp32 sums in row order");
   m.def("tuned_linear_fwd", &tuned_linear_fwd,
         "Y = X W^T via hipBLASLt with per-shape in-process algo search");
-  m.def("tuned_linear_dgrad", &tuned_linear_dgrad, "dX = dY W (algo-pinned)");
+  m.def("tuned_linear_dgrad", &tuned_linear_dgrad, "dX = dY W: the kernel where it is the faster, else algo-pinned");
   m.def("tuned_linear_wgrad", &tuned_linear_wgrad,
         "dW = dY^T X: the kernel for many rows, else algo-pinned");
   m.def("linear_wgrad", &linear_wgrad, "dW = dY^T X, the kernel");
+  m.def("linear_dgrad", &linear_dgrad, "dX = dY W, the kernel");
   m.def("varlen_attention_backward_v3", &varlen_attention_backward_v3,
         "varlen flash-attention backward v3 (atomic-free dkv+dq split, "
         "head_dim 64/128)");

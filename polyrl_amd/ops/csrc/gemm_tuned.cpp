@@ -17,7 +17,7 @@
 //   fwd  (nt): Y[M,N] = X[M,K] @ W[N,K]^T  ->  C(N,M) = op_T(W) op_N(X)
 //   dgrad(nn): dX[M,K] = dY[M,N] @ W[N,K]  ->  C(K,M) = op_N(W) op_N(dY)
 //   wgrad(tn): dW[N,K] = dY[M,N]^T @ X[M,K]->  C(K,N) = op_N(X) op_T(dY)
-// Weight gradients of many rows are the kernel's in linear_wgrad.hip.
+// Most gradients of many rows are the kernels' in linear_backward.hip.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hipblaslt/hipblaslt.h>
@@ -34,9 +34,11 @@
                 " at " #expr);                                            \
   } while (0)
 
-// linear_wgrad.hip
+// linear_backward.hip
 bool linear_wgrad_takes(const torch::Tensor& dy, const torch::Tensor& x);
+bool linear_dgrad_takes(const torch::Tensor& dy, const torch::Tensor& w);
 torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x);
+torch::Tensor linear_dgrad(torch::Tensor dy, torch::Tensor w);
 
 namespace {
 
@@ -224,6 +226,7 @@ torch::Tensor tuned_linear_dgrad(torch::Tensor dy, torch::Tensor w) {
   check2d(w, "w");
   const int64_t M = dy.size(0), N = dy.size(1), K = w.size(1);
   TORCH_CHECK(w.size(0) == N, "shape mismatch");
+  if (linear_dgrad_takes(dy, w)) return linear_dgrad(dy, w);
   auto dx = torch::empty({M, K}, dy.options());
   tuned_mm(1, dy, w, dx, M, N, K);
   return dx;

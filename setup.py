@@ -25,7 +25,7 @@ CSRC = os.path.join("polyrl_amd", "ops", "csrc")
 
 CORE = ("bindings.cpp", "gemm_tuned.cpp", "elementwise.hip",
         "rmsnorm_train.hip", "rope_train.hip", "pack_train.hip", "logprobs.hip",
-        "sampling.hip", "kv_cache.hip", "linear_prompt.hip", "linear_wgrad.hip",
+        "sampling.hip", "kv_cache.hip", "linear_prompt.hip", "linear_backward.hip",
         "attention_decode.hip", "attention_prefill.hip", "attention_backward.hip",
         "attention_backward_v3.hip")
 SEQ = ("seq_bindings.cpp", "seq_ops.hip", "seq_scan.hip", "seq_attn.hip",

@@ -1,5 +1,5 @@
-"""Weight gradients dY^T X: the edges of stages and tiles, tiles whose rows are
-shared among blocks, the trainer's use of them."""
+"""Gradients of linear layers, dY^T X and dY W: the edges of steps and tiles, tiles
+whose inner numbers are shared among blocks, the trainer's use of them."""
 import pytest
 import torch
 
@@ -14,70 +14,99 @@ def rand(m, n, seed):
     return torch.randn(m, n, generator=g, device=DEV).bfloat16()
 
 
-def check(dy, x, got):
-    a, b = dy.double(), x.double()
-    want, mass = a.t() @ b, a.abs().t() @ b.abs()
-    # 32-bit sums of M products, each off by 2^-24 of the sum of magnitudes at
-    # most, and one rounding to bf16
-    bound = 2 ** -8 * want.abs() + len(dy) * 2.0 ** -24 * mass
+def check(a, b, got):
+    """got = a b"""
+    a, b = a.double(), b.double()
+    want, mass = a @ b, a.abs() @ b.abs()
+    # 32-bit sums of the inner products, each off by 2^-24 of the sum of
+    # magnitudes at most, and one rounding to bf16
+    bound = 2 ** -8 * want.abs() + a.shape[1] * 2.0 ** -24 * mass
     assert got.shape == want.shape
     assert ((got.double() - want).abs() <= bound).all()
 
 
-def direct(m, n, k):
+def wgrad(m, n, k):
     dy, x = rand(m, n, m + n), rand(m, k, m + k + 1)
-    check(dy, x, ops._require_ext().linear_wgrad(dy, x))
+    check(dy.t(), x, ops._require_ext().linear_wgrad(dy, x))
+
+
+def dgrad(m, n, k):
+    dy, w = rand(m, n, m + n), rand(n, k, n + k + 1)
+    check(dy, w, ops._require_ext().linear_dgrad(dy, w))
 
 
 @pytest.mark.parametrize("m", [1, 31, 32, 33, 64, 65, 127, 128, 129, 160, 200,
                                257, 450])
-def test_rows(m):
-    """Fewer stages than are on their way at once, odd ones, a last one of some
+def test_wgrad_inner(m):
+    """Fewer steps than are on their way at once, odd ones, a last one of some
     rows."""
-    direct(m, 256, 264)
+    wgrad(m, 256, 264)
 
 
 @pytest.mark.parametrize("n,k", [(8, 8), (8, 520), (248, 256), (264, 1000),
                                  (2048, 256), (2312, 512), (4360, 264)])
-def test_columns(n, k):
+def test_wgrad_outer(n, k):
     """Columns short of a tile, one tile more than a group of rows of tiles."""
-    direct(96, n, k)
+    wgrad(96, n, k)
 
 
-@pytest.mark.parametrize("m", [1280, 1283, 1950, 5121, 8191])
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 320, 384, 448, 576])
+@pytest.mark.parametrize("m,k", [(256, 264), (3, 256)])
+def test_dgrad_inner(m, n, k):
+    """One pair of steps to more than two rounds of the three that LDS holds."""
+    dgrad(m, n, k)
+
+
+@pytest.mark.parametrize("m,k", [(1, 8), (8, 520), (255, 256), (257, 1000),
+                                 (2049, 256), (2311, 512), (4353, 264)])
+def test_dgrad_outer(m, k):
+    """Rows and columns short of a tile, one tile more than a group of rows of
+    tiles."""
+    dgrad(m, 192, k)
+
+
+@pytest.mark.parametrize("inner", [1280, 1344, 1984, 5120, 8192])
 @pytest.mark.parametrize("n,k", [(256, 256), (264, 520), (1024, 1304)])
-def test_shared_rows(m, n, k):
+def test_shared(inner, n, k):
     """Two blocks and more for a tile, unequal parts, edges in the sums."""
-    direct(m, n, k)
+    wgrad(inner - 1, n, k)
+    dgrad(n, inner, k)
 
 
-def test_rows_behind_the_last_are_zero():
+def test_behind_the_last():
     """What stands in memory behind an operand has no part in its product."""
-    m, n, k = 70, 136, 72
+    m, n, k = 70, 192, 72
     dy = torch.full((m + 64, n), float("nan"), device=DEV).bfloat16()
     x = torch.full((m + 64, k), float("inf"), device=DEV).bfloat16()
-    dy[:m], x[:m] = rand(m, n, 3), rand(m, k, 4)
-    check(dy[:m], x[:m], ops._require_ext().linear_wgrad(dy[:m], x[:m]))
+    w = torch.full((n + 64, k), float("inf"), device=DEV).bfloat16()
+    dy[:m], x[:m], w[:n] = rand(m, n, 3), rand(m, k, 4), rand(n, k, 5)
+    ext = ops._require_ext()
+    check(dy[:m].t(), x[:m], ext.linear_wgrad(dy[:m], x[:m]))
+    check(dy[:m], w[:n], ext.linear_dgrad(dy[:m], w[:n]))
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (511, 5120, 2048), (512, 5120, 2048), (600, 5112, 2040),  # 160 tiles
-    (5119, 512, 256), (5120, 512, 256), (600, 5116, 2048)])
+    (511, 5120, 2048), (512, 5120, 2048), (600, 5112, 2040),  # 160 tiles of dW
+    (5119, 512, 256), (5120, 512, 256), (600, 5116, 2048),
+    (2600, 256, 4096), (2700, 256, 4096), (5200, 320, 4096),  # 176, 336 of dX
+    (64, 8128, 264), (63, 8192, 264), (64, 8192, 264), (130, 8224, 520)])
 def test_linear_backward(m, n, k):
-    """Both sides of the lines where the trainer's linears take the kernel, and
-    columns that it does not take."""
+    """Both sides of the lines where the trainer's linears take the kernels, and
+    columns that they do not take."""
     x = rand(m, k, 5).requires_grad_()
     w = (rand(n, k, 6) / 8).requires_grad_()
     dy = rand(m, n, 7)
     ops.tuned_linear(x, w).backward(dy)
-    check(dy, x.detach(), w.grad)
+    check(dy.t(), x.detach(), w.grad)
+    check(dy, w.detach(), x.grad)
 
 
 def test_refused():
     ext = ops._require_ext()
-    with pytest.raises(RuntimeError):
-        ext.linear_wgrad(rand(64, 12, 0), rand(64, 16, 0))
-    with pytest.raises(RuntimeError):
-        ext.linear_wgrad(rand(0, 16, 0), rand(0, 16, 0))
-    with pytest.raises(RuntimeError):
-        ext.linear_wgrad(rand(64, 16, 0), rand(65, 16, 0))
+    for dy, x in (((64, 12), (64, 16)), ((0, 16), (0, 16)), ((64, 16), (65, 16))):
+        with pytest.raises(RuntimeError):
+            ext.linear_wgrad(rand(*dy, 0), rand(*x, 0))
+    for dy, w in (((64, 96), (96, 16)), ((64, 64), (64, 12)), ((0, 64), (64, 8)),
+                  ((64, 64), (128, 16))):
+        with pytest.raises(RuntimeError):
+            ext.linear_dgrad(rand(*dy, 0), rand(*w, 0))
