@@ -1,0 +1,361 @@
+// Products of bf16 matrices by tiles of 256 x 256 outputs (linear_backward.hip,
+// linear_prompt.hip).
+//
+// Split.  A block has four waves, 128 x 128 outputs each: 256 accumulator registers a
+// lane, 128 more for the fragments of two steps, one wave a SIMD, one block a CU.  A
+// step is 32 inner numbers.  Two steps of an operand, 32 KiB, are loaded as one unit
+// straight into LDS, five units' room; a barrier every two steps.  Where an operand's
+// inner dimension is its memory's rows' own (LINES: x and W in x W^T, dY in dY W) a unit
+// is 256 rows of 128 bytes, whole lines, and fragments are read as they are; where it
+// runs over the memory's rows (COLUMNS: W in dY W, both in dY^T X) a unit is 64 rows of 512
+// bytes and fragments come by transposed reads (ds_read_b64_tr_b16).  Both leave a
+// lane eight inner numbers from 8 * (lane / 16) of 32.
+//
+// Schedule.  One wave a SIMD has nobody to take its turn: the order is fixed instruction
+// by instruction (order()).  Behind each of a step's 64 v_mfma_f32_16x16x32_bf16, 16
+// cycles each, stands at most one of the next step's fragment reads, of the unit's
+// loads, of the words that say where a load goes, or of the next addresses.  A block's
+// tiles are one stream of units: at a tile's end the next one's first are there.
+#pragma once
+
+#include "attention_tile.h"
+
+namespace product {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef f32x4_t Acc[8][8];             // columns, rows: 16 x 16 outputs each
+
+constexpr int SIDE = 256;              // outputs of a tile, each way
+constexpr int PAIR = 64;               // inner numbers of a unit
+constexpr int UNIT = SIDE * PAIR * 2;  // bytes
+constexpr int LDS_BYTES = 5 * UNIT;
+constexpr int CUS = 256;
+constexpr int GROUP = 8;               // rows of tiles that a die walks together
+
+DEV_INLINE void order() { __builtin_amdgcn_sched_barrier(0); }
+
+DEV_INLINE void aim(unsigned to) {
+  asm volatile("s_mov_b32 m0, %0" ::"s"(to) : "m0");
+}
+
+// Sums of an accumulator, read where they are asked for: left to the compiler all are
+// read at once, into registers that the next tile's fragments hold
+DEV_INLINE f32x4_t sums_of(const f32x4_t& c) {
+  f32x4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(c[e]));
+    v[e] = x;
+  }
+  return v;
+}
+
+// all but N loads of this wave are there, and all waves are here
+template <int N>
+DEV_INLINE void arrived() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// An operand of one tile: its first unit's address, the bytes from there to the
+// operand's end, the units
+struct Units {
+  const void* at;
+  long bytes;
+  int n;
+};
+
+template <bool LINES>
+struct Operand {
+  static constexpr int FRAGS = LINES ? 2 : 8;
+  u32x4_t from;                        // descriptor of the unit to load
+  unsigned step, left;                 // bytes to the next one; units to the tile's end
+  unsigned after_lo, after_hi, after_bytes, after_n;   // the next tile
+  unsigned load_at[8];                 // of this lane's loads
+  int frag_at[FRAGS];  // this lane's place, slot 0, of 16 columns (LINES: of a step)
+
+  // COLUMNS: a row's 512 bytes stand in windows of 32, turned by the row, so that
+  // eight rows of a window meet no bank twice
+  DEV_INLINE static int turn(int r) { return (r & 3) | ((r >> 3) & 1) << 2; }
+  // LINES: a row's granules are turned by the row, so that 16 rows of a granule meet
+  // no bank twice
+  DEV_INLINE static int place(int g, int r) { return g ^ (r >> 1 & 7); }
+
+  // ld: numbers of a memory row; half: which 128 of the outer numbers are the wave's
+  DEV_INLINE Operand(const char* lds, long ld, int half) {
+    const unsigned ldb = (unsigned)ld * 2;
+    step = LINES ? 2 * PAIR : PAIR * ldb;
+    const int lane = threadIdx.x & 63, wid = wave_id();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (LINES) {
+        const int r = wid * 64 + i * 8 + (lane >> 3);
+        load_at[i] = r * ldb + (place(lane & 7, r) << 4);
+      } else {
+        const int r = wid * 16 + i * 2 + (lane >> 5);
+        load_at[i] = r * ldb + (((lane & 31) ^ (turn(r) << 1)) << 4);
+      }
+    }
+    const int lds0 = (int)(uintptr_t)(lds_p)lds, c = lane & 15, h = lane >> 4;
+#pragma unroll
+    for (int d = 0; d < FRAGS; ++d) {
+      if (LINES) {
+        frag_at[d] = lds0 + half * 16384 + c * 128 + (place(4 * d + h, c) << 4);
+      } else {
+        const int r = 8 * h + (c >> 2);
+        frag_at[d] = lds0 + half * 256 + r * 512 + ((d ^ turn(r)) << 5) +
+                     (c & 3) * 8;
+      }
+    }
+  }
+  // The tile that follows; what is behind ``bytes`` reads as 0
+  DEV_INLINE void follow(const Units& u) {
+    const uint64_t b = (uint64_t)u.at;
+    after_lo = (unsigned)uniform((int)b);
+    after_hi = (unsigned)uniform((int)(b >> 32)) & 0xffffu;
+    after_bytes = (unsigned)uniform((int)u.bytes), after_n = uniform(u.n);
+    // (a scalar that a vector instruction wrote is not to be used at once)
+    asm volatile("s_nop 4"
+                 : "+s"(after_lo), "+s"(after_hi), "+s"(after_bytes),
+                   "+s"(after_n));
+  }
+  DEV_INLINE void start() {
+    from = {after_lo, after_hi, after_bytes, 0x00020000u};
+    left = after_n;
+    asm volatile("s_nop 4" : "+s"(from), "+s"(left), "+s"(step));
+  }
+  // In assembly, so that the compiler does not wait for it on its own account; no
+  // register is written.
+  DEV_INLINE void go(int i) const {
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(load_at[i]),
+                 "s"(from)
+                 : "memory");
+  }
+  // on to the next unit, in three parts
+  template <int PART>
+  DEV_INLINE void next() {
+    unsigned lo = from[0], hi = from[1], bytes = from[2];
+    if (PART == 0)
+      asm volatile("s_add_u32 %0, %0, %2\n\ts_addc_u32 %1, %1, 0"
+                   : "+s"(lo), "+s"(hi)
+                   : "s"(step)
+                   : "scc");
+    if (PART == 1)
+      asm volatile(
+          "s_sub_u32 %0, %0, %2\n\ts_cselect_b32 %0, 0, %0\n\ts_sub_u32 %1, %1, 1"
+          : "+s"(bytes), "+s"(left)
+          : "s"(step)
+          : "scc");
+    if (PART == 2)
+      asm volatile(
+          "s_cmp_eq_u32 %3, 0\n\ts_cselect_b32 %0, %4, %0\n\t"
+          "s_cselect_b32 %1, %5, %1\n\ts_cselect_b32 %2, %6, %2\n\t"
+          "s_cselect_b32 %3, %7, %3"
+          : "+s"(lo), "+s"(hi), "+s"(bytes), "+s"(left)
+          : "s"(after_lo), "s"(after_hi), "s"(after_bytes), "s"(after_n)
+          : "scc");
+    from[0] = lo, from[1] = hi, from[2] = bytes;
+  }
+  DEV_INLINE void load(unsigned to) {  // a unit, at once
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      aim(to + i * 1024);
+      asm volatile("s_nop 0");
+      go(i);
+    }
+    next<0>(), next<1>(), next<2>();
+  }
+};
+
+// 16 outer numbers, a step's 32 inner ones: of lane l number l % 16, inner ones from
+// 8 * (l / 16)
+template <bool LINES>
+struct Frag {
+  i16x8_t all;
+  i16x4_t half[2];
+  // frag_at[] of the unit; d: which 16 of the wave's 128
+  template <int STEP, int H>
+  DEV_INLINE void read(const int* at, int d) {
+    typedef __attribute__((address_space(3))) const i16x8_t* lds_i16x8_p;
+    if constexpr (!LINES)
+      half[H] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_i16x4_p)(uintptr_t)(at[d] + STEP * 16384 + H * 2048));
+    else if constexpr (H == 0)
+      all = *(lds_i16x8_p)(uintptr_t)(at[STEP] + d * 2048);
+  }
+  DEV_INLINE i16x8_t whole() const {
+    return LINES ? all
+                 : __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+// Tiles r = 0, 1, ..: units(r, left, right) says where tile r's operands are, false
+// behind the last one; finish(r, acc) takes its sums: accumulator e of column part i, row
+// part j is column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 128 x
+// 128 (row half wave % 2, column half wave / 2).  A tile that another one follows has
+// four units and more.
+template <bool LL, bool RL, typename UnitsOf, typename Finish>
+DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
+                    Finish finish) {
+  const int wid = wave_id();
+  Operand<LL> a(lds, left_ld, wid & 1);
+  Operand<RL> b(lds, right_ld, wid >> 1);
+  const unsigned to = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
+  Units ua, ub;
+  int now = 0;
+  bool more = units(0, ua, ub);
+  if (!more) return;
+  a.follow(ua), b.follow(ub);
+  a.start(), b.start();
+  int pairs = ua.n;
+  auto look_ahead = [&] {              // (behind the last tile nothing is read)
+    more = units(now + 1, ua, ub);
+    if (!more) ua.bytes = ub.bytes = 0, ua.n = ub.n = 1 << 30;
+    a.follow(ua), b.follow(ub);
+  };
+  look_ahead();
+  a.load(to), b.load(to + UNIT), a.load(to + 2 * UNIT), b.load(to + 3 * UNIT);
+
+  Acc acc;
+  Frag<LL> fa[2][8];
+  Frag<RL> fb[2][8];
+  int na[a.FRAGS], nb[b.FRAGS];        // where the next fragments are
+  arrived<16>();
+#pragma unroll
+  for (int d = 0; d < a.FRAGS; ++d) na[d] = a.frag_at[d];
+#pragma unroll
+  for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + UNIT;
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    fa[0][d].template read<0, 0>(na, d), fa[0][d].template read<0, 1>(na, d);
+    fb[0][d].template read<0, 0>(nb, d), fb[0][d].template read<0, 1>(nb, d);
+  }
+
+  // The products of a step, whose fragments are registers N, the reads of the next one's,
+  // and the loads of a unit to ``slot``.  (Loads behind the end read nothing: the
+  // count of them is the same in every step.)
+  auto step = [&](auto n_, auto& load, unsigned slot, int a_next, int b_next) {
+    constexpr int N = decltype(n_)::value, O = 1 - N;
+    __builtin_amdgcn_s_waitcnt(0xc07f);            // fragments: lgkmcnt(0)
+    // The next unit of both is there, and this one's, read to the end, make room
+    if (N == 1) arrived<8>();
+#pragma unroll
+    for (int k = 0; k < 64; ++k) {
+      const int i = k >> 3, j = i & 1 ? 7 - (k & 7) : k & 7;
+      order();
+      // (in assembly, else the compiler moves accumulators about)
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                   : "+a"(acc[i][j])
+                   : "v"(fb[N][i].whole()), "v"(fa[N][j].whole()));
+      order();
+      const int f = k / 3;             // fragment: one column's, all rows', the rest
+      if (k < 48 && k % 3 < 2) {
+        if (f >= 1 && f <= 8) {
+          if (k % 3 == 0) fa[O][f - 1].template read<O, 0>(na, f - 1);
+          else fa[O][f - 1].template read<O, 1>(na, f - 1);
+        } else {
+          const int d = f == 0 ? 0 : f - 8;
+          if (k % 3 == 0) fb[O][d].template read<O, 0>(nb, d);
+          else fb[O][d].template read<O, 1>(nb, d);
+        }
+      } else if (k < 48) {
+        if (f % 2 == 0) aim(slot + f / 2 * 1024);
+        else load.go(f / 2);
+      } else {
+        const int d = k - 48;
+        if (N == 0 && d < 8 && d < a.FRAGS) {
+          na[d < a.FRAGS ? d : 0] = a.frag_at[d < a.FRAGS ? d : 0] + a_next;
+          asm volatile("" : "+v"(na[d < a.FRAGS ? d : 0]));
+        }
+        if (N == 0 && d >= 8 && d - 8 < b.FRAGS) {
+          const int e = d - 8 < b.FRAGS ? d - 8 : 0;
+          nb[e] = b.frag_at[e] + b_next;
+          asm volatile("" : "+v"(nb[e]));
+        }
+        if (d == 3) load.template next<0>();
+        if (d == 8) load.template next<1>();
+        if (d == 13) load.template next<2>();
+      }
+    }
+  };
+
+  // slots: this pair's units, the next pair's, the left one behind that
+  int s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < pairs; ++p) {
+      step(std::integral_constant<int, 0>(), a, to + s4, s2, s3);
+      step(std::integral_constant<int, 1>(), b, to + s0, s2, s3);
+      const int t0 = s0, t1 = s1;
+      s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
+    }
+    // (the compiler does not know that these are products, whose results take a while;
+    // they are read by sums_of())
+    asm volatile("s_nop 15\n\ts_nop 15");
+    finish(now, acc);
+    if (!more) break;
+    ++now;
+    pairs = ua.n;
+    look_ahead();
+  }
+  // (no load is on its way to LDS when the block ends)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Row and column of a tile: GROUP rows of tiles, one column after the other, so that
+// the blocks that run on a die at once share 8 x 4 tiles' operands
+struct Place {
+  int row, col;
+  DEV_INLINE Place(int tile, int row_tiles, int col_tiles) {
+    const int group = tile / (GROUP * col_tiles);
+    const int rest = tile - group * GROUP * col_tiles;
+    const int high = min(GROUP, row_tiles - group * GROUP);
+    row = uniform(group * GROUP + rest % high), col = uniform(rest / high);
+  }
+};
+
+// Item r of this block: blocks go to the dies in turn, each die takes one stretch of
+// the items, its blocks every ``blocks / dies``-th of it; -1 behind the last
+DEV_INLINE int item_of(int r, int items, int blocks) {
+  const int per = (items + ATTN_XCDS - 1) / ATTN_XCDS;
+  const int in = (int)blockIdx.x / ATTN_XCDS + r * (blocks / ATTN_XCDS);
+  const int item = (int)(blockIdx.x % ATTN_XCDS) * per + in;
+  return in < per && item < items ? item : -1;
+}
+
+// Units of 256 rows from ``first`` of an operand in LINES: inner numbers from inner0 on
+DEV_INLINE Units lines(const bf16_t* p, long outer, long inner, long first,
+                       long inner0, int n) {
+  const long skip = first * inner + inner0;
+  return {p + skip, min(2 * (outer * inner - skip), 2 * SIDE * inner), n};
+}
+// of 256 columns of one in COLUMNS.  (Columns behind the last one are the next row's,
+// and whoever reads them stores nothing.)
+DEV_INLINE Units columns(const bf16_t* p, long outer, long inner, long first,
+                         long inner0, int n) {
+  const long skip = inner0 * outer + first;
+  return {p + skip, 2 * (inner * outer - skip), n};
+}
+
+// Two column parts of a row part as rows of bf16 numbers: this lane's 8 columns are 16 i +
+// 8 (lane / 16) of the wave's, of row 16 j + lane % 16
+DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
+  u32x4_t out;
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    union { bf16_t h[2]; unsigned u; } x, y;
+    x.h[0] = f2bf(c0[2 * w]), x.h[1] = f2bf(c0[2 * w + 1]);
+    y.h[0] = f2bf(c1[2 * w]), y.h[1] = f2bf(c1[2 * w + 1]);
+    const auto p = __builtin_amdgcn_permlane32_swap(x.u, y.u, false, false);
+    const auto q = __builtin_amdgcn_permlane16_swap(p[0], p[1], false, false);
+    out[w] = q[0], out[2 + w] = q[1];
+  }
+  return out;
+}
+
+}  // namespace product

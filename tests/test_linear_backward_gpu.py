@@ -65,6 +65,15 @@ def test_dgrad_outer(m, k):
     dgrad(m, 192, k)
 
 
+@pytest.mark.parametrize("inner", [193, 256, 320, 384, 448])
+def test_tiles_in_turn(inner):
+    """More tiles than blocks that run at once: a block's second tile and third,
+    whose first units are loaded during the one before; fewer units than that
+    takes."""
+    wgrad(inner, 4360, 4104)
+    dgrad(4353, (inner + 63) // 64 * 64, 8200)
+
+
 @pytest.mark.parametrize("inner", [1280, 1344, 1984, 5120, 8192])
 @pytest.mark.parametrize("n,k", [(256, 256), (264, 520), (1024, 1304)])
 def test_shared(inner, n, k):
