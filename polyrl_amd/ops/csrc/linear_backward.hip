@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
     b = columns(right, C, inner, c0, i0, n);
     return true;
   };
-  auto finish = [&](int r, Acc& acc) {
+  auto finish = [&](int r, Acc<>& acc) {
     const int lane = threadIdx.x & 63, wid = wave_id();
     const int item = item_of(r, items, gridDim.x), part = item / tiles;
     const int tile = item - part * tiles;
@@ -146,13 +146,6 @@ long tiles_of(long R, long C) {
 // 69, 68 us with 1 to 4 blocks a tile; 16 tiles 74, 45, 34, 34, 39 with 2, 4, 8, 12, 16)
 long ways_of(long tiles, long inner) {
   return std::max(1L, std::min(CUS / tiles, inner / 640));
-}
-
-// Blocks: as many as run at once, each with its tiles one after the other, but of few
-// units a tile a block each
-long blocks_of(long items, long inner) {
-  const long most = inner >= 4 * PAIR ? CUS : items;
-  return (std::min(items, most) + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
 }
 
 template <bool LINES>

@@ -2,7 +2,8 @@
 // linear_prompt.hip).
 //
 // Split.  A block has four waves, 128 x 128 outputs each: 256 accumulator registers a
-// lane, 128 more for the fragments of two steps, one wave a SIMD, one block a CU.  A
+// lane, 128 more for the fragments of two steps, one wave a SIMD, one block a CU.  (Tiles
+// of fewer rows, 32 J, where both operands are LINES: a wave has J row parts for eight.)  A
 // step is 32 inner numbers.  Two steps of an operand, 32 KiB, are loaded as one unit
 // straight into LDS, five units' room; a barrier every two steps.  Where an operand's
 // inner dimension is its memory's rows' own (LINES: x and W in x W^T, dY in dY W) a unit
@@ -18,12 +19,15 @@
 // tiles are one stream of units: at a tile's end the next one's first are there.
 #pragma once
 
+#include <utility>
+
 #include "attention_tile.h"
 
 namespace product {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef f32x4_t Acc[8][8];             // columns, rows: 16 x 16 outputs each
+template <int J = 8>
+using Acc = f32x4_t[8][J];             // columns, rows: 16 x 16 outputs each
 
 constexpr int SIDE = 256;              // outputs of a tile, each way
 constexpr int PAIR = 64;               // inner numbers of a unit
@@ -31,6 +35,12 @@ constexpr int UNIT = SIDE * PAIR * 2;  // bytes
 constexpr int LDS_BYTES = 5 * UNIT;
 constexpr int CUS = 256;
 constexpr int GROUP = 8;               // rows of tiles that a die walks together
+
+// f(0), f(1), .., as constants
+template <typename F, int... K>
+DEV_INLINE void each(std::integer_sequence<int, K...>, F f) {
+  (f(std::integral_constant<int, K>()), ...);
+}
 
 DEV_INLINE void order() { __builtin_amdgcn_sched_barrier(0); }
 
@@ -67,13 +77,15 @@ struct Units {
   int n;
 };
 
-template <bool LINES>
+// P: 16-row parts of a wave's half
+template <bool LINES, int P = 8>
 struct Operand {
+  static_assert(LINES || P == 8, "COLUMNS are 256");
   static constexpr int FRAGS = LINES ? 2 : 8;
   u32x4_t from;                        // descriptor of the unit to load
   unsigned step, left;                 // bytes to the next one; units to the tile's end
   unsigned after_lo, after_hi, after_bytes, after_n;   // the next tile
-  unsigned load_at[8];                 // of this lane's loads
+  unsigned load_at[P];                 // of this lane's loads
   int frag_at[FRAGS];  // this lane's place, slot 0, of 16 columns (LINES: of a step)
 
   // COLUMNS: a row's 512 bytes stand in windows of 32, turned by the row, so that
@@ -89,9 +101,9 @@ struct Operand {
     step = LINES ? 2 * PAIR : PAIR * ldb;
     const int lane = threadIdx.x & 63, wid = wave_id();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < P; ++i) {
       if (LINES) {
-        const int r = wid * 64 + i * 8 + (lane >> 3);
+        const int r = wid * (8 * P) + i * 8 + (lane >> 3);
         load_at[i] = r * ldb + (place(lane & 7, r) << 4);
       } else {
         const int r = wid * 16 + i * 2 + (lane >> 5);
@@ -102,7 +114,7 @@ struct Operand {
 #pragma unroll
     for (int d = 0; d < FRAGS; ++d) {
       if (LINES) {
-        frag_at[d] = lds0 + half * 16384 + c * 128 + (place(4 * d + h, c) << 4);
+        frag_at[d] = lds0 + half * (P * 2048) + c * 128 + (place(4 * d + h, c) << 4);
       } else {
         const int r = 8 * h + (c >> 2);
         frag_at[d] = lds0 + half * 256 + r * 512 + ((d ^ turn(r)) << 5) +
@@ -160,7 +172,7 @@ struct Operand {
   }
   DEV_INLINE void load(unsigned to) {  // a unit, at once
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < P; ++i) {
       aim(to + i * 1024);
       asm volatile("s_nop 0");
       go(i);
@@ -193,16 +205,18 @@ struct Frag {
 
 // Tiles r = 0, 1, ..: units(r, left, right) says where tile r's operands are, false
 // behind the last one; finish(r, acc) takes its sums: accumulator e of column part i, row
-// part j is column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 128 x
+// part j is column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 16 J x
 // 128 (row half wave % 2, column half wave / 2).  A tile that another one follows has
 // four units and more.
-template <bool LL, bool RL, typename UnitsOf, typename Finish>
+template <bool LL, bool RL, int J = 8, typename UnitsOf, typename Finish>
 DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
                     Finish finish) {
   const int wid = wave_id();
-  Operand<LL> a(lds, left_ld, wid & 1);
+  Operand<LL, J> a(lds, left_ld, wid & 1);
   Operand<RL> b(lds, right_ld, wid >> 1);
-  const unsigned to = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
+  // (of a unit a wave loads 1 KiB for each of its row parts)
+  const unsigned to_a = (unsigned)(uintptr_t)(lds_p)lds + wid * (J * 1024);
+  const unsigned to_b = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
   Units ua, ub;
   int now = 0;
   bool more = units(0, ua, ub);
@@ -216,20 +230,24 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
     a.follow(ua), b.follow(ub);
   };
   look_ahead();
-  a.load(to), b.load(to + UNIT), a.load(to + 2 * UNIT), b.load(to + 3 * UNIT);
+  a.load(to_a), b.load(to_b + UNIT);
+  a.load(to_a + 2 * UNIT), b.load(to_b + 3 * UNIT);
 
-  Acc acc;
-  Frag<LL> fa[2][8];
+  Acc<J> acc;
+  Frag<LL> fa[2][J];
   Frag<RL> fb[2][8];
   int na[a.FRAGS], nb[b.FRAGS];        // where the next fragments are
-  arrived<16>();
+  arrived<J + 8>();
 #pragma unroll
   for (int d = 0; d < a.FRAGS; ++d) na[d] = a.frag_at[d];
 #pragma unroll
   for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + UNIT;
 #pragma unroll
   for (int d = 0; d < 8; ++d) {
-    fa[0][d].template read<0, 0>(na, d), fa[0][d].template read<0, 1>(na, d);
+    if (d < J) {
+      fa[0][d < J ? d : 0].template read<0, 0>(na, d);
+      fa[0][d < J ? d : 0].template read<0, 1>(na, d);
+    }
     fb[0][d].template read<0, 0>(nb, d), fb[0][d].template read<0, 1>(nb, d);
   }
 
@@ -238,47 +256,56 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
   // count of them is the same in every step.)
   auto step = [&](auto n_, auto& load, unsigned slot, int a_next, int b_next) {
     constexpr int N = decltype(n_)::value, O = 1 - N;
+    constexpr int FRAGS = 8 + J, LOADS = N == 0 ? J : 8, ALL = 8 * J;
+    // instructions of a fragment (and a load's two, or with the load's first)
+    constexpr int PER = LL && RL ? 2 : 3;
+    static_assert(PER * FRAGS <= ALL && 2 * LOADS <= PER * FRAGS, "the order");
     __builtin_amdgcn_s_waitcnt(0xc07f);            // fragments: lgkmcnt(0)
     // The next unit of both is there, and this one's, read to the end, make room
-    if (N == 1) arrived<8>();
-#pragma unroll
-    for (int k = 0; k < 64; ++k) {
-      const int i = k >> 3, j = i & 1 ? 7 - (k & 7) : k & 7;
+    if constexpr (N == 1) arrived<J>();
+    each(std::make_integer_sequence<int, ALL>(), [&](auto k_) {
+      constexpr int k = decltype(k_)::value;
+      constexpr int i = k / J, j = i & 1 ? J - 1 - k % J : k % J;
       order();
       // (in assembly, else the compiler moves accumulators about)
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
                    : "+a"(acc[i][j])
                    : "v"(fb[N][i].whole()), "v"(fa[N][j].whole()));
       order();
-      const int f = k / 3;             // fragment: one column's, all rows', the rest
-      if (k < 48 && k % 3 < 2) {
-        if (f >= 1 && f <= 8) {
-          if (k % 3 == 0) fa[O][f - 1].template read<O, 0>(na, f - 1);
-          else fa[O][f - 1].template read<O, 1>(na, f - 1);
-        } else {
-          const int d = f == 0 ? 0 : f - 8;
-          if (k % 3 == 0) fb[O][d].template read<O, 0>(nb, d);
-          else fb[O][d].template read<O, 1>(nb, d);
+      constexpr int f = k / PER;       // fragment: one column's, all rows', the rest
+      if constexpr (f < FRAGS) {
+        constexpr int H = k % PER;
+        if constexpr (H < 2 && f >= 1 && f <= J)
+          fa[O][f - 1].template read<O, H>(na, f - 1);
+        else if constexpr (H < 2)
+          fb[O][f == 0 ? 0 : f - J].template read<O, H>(nb, f == 0 ? 0 : f - J);
+        if constexpr (PER == 2 && f < LOADS) {
+          if constexpr (H == 0) aim(slot + f * 1024);
+          else load.go(f);
+        } else if constexpr (PER == 3 && H == 2 && f / 2 < LOADS) {
+          if constexpr (f % 2 == 0) aim(slot + f / 2 * 1024);
+          else load.go(f / 2);
         }
-      } else if (k < 48) {
-        if (f % 2 == 0) aim(slot + f / 2 * 1024);
-        else load.go(f / 2);
       } else {
-        const int d = k - 48;
-        if (N == 0 && d < 8 && d < a.FRAGS) {
-          na[d < a.FRAGS ? d : 0] = a.frag_at[d < a.FRAGS ? d : 0] + a_next;
-          asm volatile("" : "+v"(na[d < a.FRAGS ? d : 0]));
-        }
-        if (N == 0 && d >= 8 && d - 8 < b.FRAGS) {
-          const int e = d - 8 < b.FRAGS ? d - 8 : 0;
-          nb[e] = b.frag_at[e] + b_next;
-          asm volatile("" : "+v"(nb[e]));
-        }
-        if (d == 3) load.template next<0>();
-        if (d == 8) load.template next<1>();
-        if (d == 13) load.template next<2>();
+        // the addresses of the pair that comes next, and the next unit to load
+        constexpr int d = k - PER * FRAGS, REST = ALL - PER * FRAGS;
+        constexpr int FA = Operand<LL, J>::FRAGS, FB = Operand<RL>::FRAGS;
+        if constexpr (N == 0)
+          each(std::make_integer_sequence<int, FA + FB>(), [&](auto e_) {
+            constexpr int e = decltype(e_)::value;
+            if constexpr (e * REST / (FA + FB) == d && e < FA) {
+              na[e] = a.frag_at[e] + a_next;
+              asm volatile("" : "+v"(na[e]));
+            } else if constexpr (e * REST / (FA + FB) == d) {
+              nb[e - FA] = b.frag_at[e - FA] + b_next;
+              asm volatile("" : "+v"(nb[e - FA]));
+            }
+          });
+        if constexpr (d == REST / 5) load.template next<0>();
+        if constexpr (d == REST / 2) load.template next<1>();
+        if constexpr (d == REST * 4 / 5) load.template next<2>();
       }
-    }
+    });
   };
 
   // slots: this pair's units, the next pair's, the left one behind that
@@ -287,10 +314,10 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int p = 0; p < pairs; ++p) {
-      step(std::integral_constant<int, 0>(), a, to + s4, s2, s3);
-      step(std::integral_constant<int, 1>(), b, to + s0, s2, s3);
+      step(std::integral_constant<int, 0>(), a, to_a + s4, s2, s3);
+      step(std::integral_constant<int, 1>(), b, to_b + s0, s2, s3);
       const int t0 = s0, t1 = s1;
       s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
     }
@@ -328,7 +355,7 @@ DEV_INLINE int item_of(int r, int items, int blocks) {
   return in < per && item < items ? item : -1;
 }
 
-// Units of 256 rows from ``first`` of an operand in LINES: inner numbers from inner0 on
+// Units of rows from ``first`` of an operand in LINES: inner numbers from inner0 on
 DEV_INLINE Units lines(const bf16_t* p, long outer, long inner, long first,
                        long inner0, int n) {
   const long skip = first * inner + inner0;
@@ -356,6 +383,13 @@ DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
     out[w] = q[0], out[2 + w] = q[1];
   }
   return out;
+}
+
+// Blocks: as many as run at once, each with its tiles one after the other, but of few
+// units a tile a block each
+inline long blocks_of(long items, long inner) {
+  const long most = inner >= 4 * PAIR ? CUS : items;
+  return (std::min(items, most) + ATTN_XCDS - 1) / ATTN_XCDS * ATTN_XCDS;
 }
 
 }  // namespace product

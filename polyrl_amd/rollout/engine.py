@@ -37,14 +37,14 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     call costs the host 5 us for the 20 of torch's (a step of 3, 4, 6 and 8 x 256
     tokens, 12 layers of 1024, 1109, 1124, 1286 and 1447 us with it and 1471, 1491,
     1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the
-    device it is up to 3.5 us slower within these lines (us, kernel and library,
-    of 513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 7.8, 8.0, 8.5, 10.2, 15.0
-    and 7.2, 7.6, 9.1, 11.6, 16.6; 1024 -> 1024 12.3, 12.3, 13.1, 16.6, 23.9 and
-    8.9, 9.1, 10.9, 14.7, 22.6; 1024 -> 1536 12.4, 12.9, 14.2, 20.4, 32.3 and 9.0,
-    10.5, 13.8, 19.0, 30.2; 1024 -> 4096 of 513 .. 3072 13.5 .. 30.8 and 13.4 ..
-    28.7), beyond them by more than the host gains (1024 -> 4096 of 8192 rows 71.5
-    and 58.2, 1024 -> 32000 of 2048 131 and 116, 2048 -> 3072 of 8192 105 and 93);
-    a captured graph, where the host's time does not count, takes the library's."""
+    device it is up to 4 us slower within these lines (us, kernel and library, of
+    513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 8.3, 8.5, 8.8, 9.4, 13.0 and 6.3,
+    6.6, 7.7, 9.7, 14.9; 1024 -> 1024 11.7, 12.0, 12.7, 14.9, 19.4 and 7.7, 8.0, 10.4,
+    13.3, 21.5; 1024 -> 1536 11.8, 12.2, 13.8, 17.1, 28.4 and 7.8, 9.8, 13.1, 18.5,
+    29.3), beyond them by more than the host gains where outputs are few (1024 of
+    600 .. 4700 rows 0.55 to 0.91 of the library's speed at an inner width of 4096)
+    and about as fast elsewhere; a captured graph, where the host's time does not
+    count, takes the library's."""
     if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 512 \
             and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
@@ -58,17 +58,17 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x @ Wg.T) * (x @ Wu.T), w = [Wg; Wu].  Prompts (the rows that
-    ``_mm_nt`` does not search for) of widths up to 1536, and of up to 8191 rows
-    of widths up to 2048, take both products and the activation in one kernel;
-    elsewhere the library's product alone is the faster by more than the
-    activation takes (us, one kernel against library and activation, of 513,
-    4096, 8192 and 16384 rows: 1024 -> 4096 15.9, 65.5, 121, 247 and 20.8, 76.5,
-    146, 287; 1536 -> 8960 35.4, 202, 382, 756 and 41.5, 228, 443, 839; 2048 ->
-    8192 44.5, 227, 448, 889 and 47.8, 228, 446, 883; of 513 and 16384 3584 -> 18944
-    171, 3393 and 148, 3386; 4096 -> 14336 190, 3042 and 133, 2805)."""
-    if x.shape[0] > 512 and x.shape[1] <= 2048 \
-            and (x.shape[1] <= 1536 or x.shape[0] < 8192) \
-            and ops.linear_takes(x, w):
+    ``_mm_nt`` does not search for) of widths up to 1536, of up to 8191 rows of
+    widths up to 2048, and of 2^22 outputs and more whatever the width take both
+    products and the activation in one kernel (us, beside the library's product
+    and the activation, of 513, 1024, 5135 and 8192 rows: 1024 -> 4096 15.0, 18.5,
+    74.0, 113 and 23.8, 28.2, 103, 149; 1536 -> 8960 29.7, 52.8, 226, 337 and 39.2,
+    70.9, 276, 452; 2048 -> 8192 34.1, 51.8, 256, 391 and 44.7, 69.0, 316, 472; 4096
+    -> 14336 117, 183, 868, 1301 and 131, 207, 996, 1408).  Few outputs of wide
+    models leave most of the chip idle."""
+    if x.shape[0] > 512 and (
+            x.shape[1] <= 1536 or x.shape[1] <= 2048 and x.shape[0] < 8192
+            or x.shape[0] * w.shape[0] >= 1 << 23) and ops.linear_takes(x, w):
         return ops.linear_swiglu(x, w)
     i = w.shape[0] // 2
     gate_up = _mm_nt(x, w)
