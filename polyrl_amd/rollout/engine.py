@@ -28,7 +28,8 @@ from .kv_cache import (PagedKVCache, PagedLatentCache, RadixCache,
                        StateSlots)
 
 
-def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def _mm_nt(x: torch.Tensor, w: torch.Tensor, search: bool = True
+           ) -> torch.Tensor:
     """y = x @ w.T; decode-sized GEMMs (M <= 512) go through the
     algo-pinned hipBLASLt path (ops.tuned_mm_nt) — the heuristic pick runs
     skinny decode projections far off the weight-read bound.  Prefill Ms
@@ -44,9 +45,10 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     29.3), beyond them by more than the host gains where outputs are few (1024 of
     600 .. 4700 rows 0.55 to 0.91 of the library's speed at an inner width of 4096)
     and about as fast elsewhere; a captured graph, where the host's time does not
-    count, takes the library's."""
-    if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 512 \
-            and _tuned_decode_enabled():
+    count, takes the library's.  ``search``: False for few rows whose number is not
+    a decode batch's."""
+    if search and x.is_cuda and x.dtype == torch.bfloat16 \
+            and x.shape[0] <= 512 and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
     if 512 < x.shape[0] <= 8192 and x.shape[1] <= 1024 \
             and x.shape[0] * w.shape[0] <= 3 << 22 \
@@ -56,7 +58,8 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return x @ w.t()
 
 
-def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def _gate_up(x: torch.Tensor, w: torch.Tensor, search: bool = True
+             ) -> torch.Tensor:
     """silu(x @ Wg.T) * (x @ Wu.T), w = [Wg; Wu].  Prompts (the rows that
     ``_mm_nt`` does not search for) of widths up to 1536, of up to 8191 rows of
     widths up to 2048, and of 2^22 outputs and more whatever the width take both
@@ -71,7 +74,7 @@ def _gate_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             or x.shape[0] * w.shape[0] >= 1 << 23) and ops.linear_takes(x, w):
         return ops.linear_swiglu(x, w)
     i = w.shape[0] // 2
-    gate_up = _mm_nt(x, w)
+    gate_up = _mm_nt(x, w, search)
     return ops.silu_mul(gate_up.narrow(1, 0, i), gate_up.narrow(1, i, i))
 
 
@@ -316,12 +319,15 @@ class InferenceModel:
     @torch.no_grad()
     def forward_tokens(self, token_ids: torch.Tensor, positions: torch.Tensor,
                        kv: PagedKVCache, slot_mapping: torch.Tensor,
-                       attn_fn) -> torch.Tensor:
+                       attn_fn, rows: Optional[torch.Tensor] = None
+                       ) -> torch.Tensor:
         """Shared trunk: embed -> L x (norm, qkv, rope, kv-append, attn(fn),
-        o-proj, norm, mlp) -> final norm.  Returns hidden (N, H)."""
+        o-proj, norm, mlp) -> final norm.  Returns hidden (N, H), or of the
+        tokens that ``rows`` names."""
         if self.cfg.arch == "gpt2":
-            return self._forward_tokens_gpt2(token_ids, positions, kv,
-                                             slot_mapping, attn_fn)
+            hidden = self._forward_tokens_gpt2(token_ids, positions, kv,
+                                               slot_mapping, attn_fn)
+            return hidden if rows is None else hidden.index_select(0, rows)
         cfg = self.cfg
         tp = self.tp.size
         Hq = cfg.num_attention_heads // tp
@@ -330,6 +336,11 @@ class InferenceModel:
         x = self.embed[token_ids]                     # (N, H) gather
         residual = x.clone()
         hidden = None
+        # behind the last layer's attention nothing depends on the other tokens
+        # (16 prompts, 5135 tokens, 12 layers of 1024: 150 of 2500 us).  Of up to
+        # 512 tokens the products' algorithms were searched for as many rows as
+        # there are, in the layers before: all of them go on.
+        early = rows is not None and x.shape[0] > 512
         for li, lw in enumerate(self.layers):
             if li == 0:
                 hidden = ops.rmsnorm(residual, lw.input_ln, cfg.rms_norm_eps)
@@ -346,17 +357,25 @@ class InferenceModel:
             v = qkv.narrow(1, (Hq + Hk) * D, Hk * D).unflatten(1, (Hk, D))
             ops.rope_kv_append(q, k, v, positions, self.rope,
                                kv.k_cache[li], kv.v_cache[li], slot_mapping)
-            attn_out = attn_fn(li, q, k, v)           # (N, Hq, D)
-            hidden = _mm_nt(attn_out.reshape(-1, Hq * D), lw.wo)
+            attn_out = attn_fn(li, q, k, v).reshape(-1, Hq * D)
+            few = early and li == len(self.layers) - 1
+            if few:
+                if not rows.numel():
+                    return x.new_empty(0, x.shape[1])
+                attn_out = attn_out.index_select(0, rows)
+                residual = residual.index_select(0, rows)
+            hidden = _mm_nt(attn_out, lw.wo, not few)
             self.tp.all_reduce_(hidden)               # col-parallel o_proj
             hidden, residual = ops.fused_add_rmsnorm(
                 hidden, residual, lw.post_ln, cfg.rms_norm_eps)
-            hidden = _mm_nt(_gate_up(hidden, lw.w_gate_up), lw.w_down)
+            hidden = _mm_nt(_gate_up(hidden, lw.w_gate_up, not few),
+                            lw.w_down, not few)
             self.tp.all_reduce_(hidden)               # col-parallel down_proj
         # final residual add + norm (fused; residual buffer is dead after)
         normed, _ = ops.fused_add_rmsnorm(hidden, residual, self.final_norm,
                                           cfg.rms_norm_eps)
-        return normed
+        return normed if rows is None or early \
+            else normed.index_select(0, rows)
 
     @torch.no_grad()
     def _forward_tokens_gpt2(self, token_ids, positions, kv, slot_mapping,
@@ -1026,13 +1045,15 @@ class Engine:
             if self.hybrid:
                 bt, _ = self._hybrid_batch(items)
                 hidden = self.model.forward_batch(bt, self.kv, self.states)
+                if rows:
+                    idx, = self._upload([np.asarray(rows, np.int32)])
+                    hidden = hidden.index_select(0, idx)
             else:
                 hidden = self._forward_portions(
                     [it[0] for it in items], [it[1] for it in items],
-                    [len(it[2]) for it in items])[0]
+                    [len(it[2]) for it in items], rows)
             if rows:
-                idx, = self._upload([np.asarray(rows, np.int32)])
-                logits = self.model.logits(hidden.index_select(0, idx)).float()
+                logits = self.model.logits(hidden).float()
         for rid in end:
             r = self._forced.pop(rid, None)
             if r is not None:
@@ -1041,9 +1062,10 @@ class Engine:
         return logits
 
     def _forward_portions(self, reqs: List[Request], starts: List[int],
-                          lens: List[int]):
-        """Hidden rows of each request's tokens [start, start+len) against
-        its cached history (dense decoders); returns (hidden, cu_q)."""
+                          lens: List[int], rows: List[int]) -> torch.Tensor:
+        """Each request's tokens [start, start+len) against its cached history
+        (dense decoders); hidden rows of those of them, counted through the
+        requests, that ``rows`` names."""
         cu_q, cu_k = [0], [0]
         for start, take in zip(starts, lens):
             cu_q.append(cu_q[-1] + take)
@@ -1062,14 +1084,16 @@ class Engine:
         slots = [self.kv.slots_for_host(sid, s, m)
                  for sid, s, m in zip(sids, starts, lens)]
         parts = [tok, pos, np.concatenate(slots),
-                 np.asarray(cu_q, np.int32), np.asarray(cu_k, np.int32)]
+                 np.asarray(cu_q, np.int32), np.asarray(cu_k, np.int32),
+                 np.asarray(rows, np.int32)]
         if not fresh:
             # portions behind cached tokens attend to the FULL history: the
             # cache rows of every key, gathered once per layer
             parts.append(np.concatenate(
                 [self.kv.slots_for_host(sid, 0, s + m)
                  for sid, s, m in zip(sids, starts, lens)]))
-        tokens, positions, slots, cu_q_t, cu_k_t, *hist = self._upload(parts)
+        tokens, positions, slots, cu_q_t, cu_k_t, rows_t, *hist = \
+            self._upload(parts)
 
         def attn_fn(li, q, k, v):
             if not fresh:
@@ -1079,9 +1103,8 @@ class Engine:
             return ops.varlen_prefill_attention(q, k, v, cu_q_t, cu_k_t,
                                                 self._scale, causal=True)
 
-        hidden = self.model.forward_tokens(tokens.long(), positions, self.kv,
-                                           slots, attn_fn)
-        return hidden, cu_q
+        return self.model.forward_tokens(tokens.long(), positions, self.kv,
+                                         slots, attn_fn, rows_t)
 
     def _upload(self, parts) -> List[torch.Tensor]:
         """int32 arrays as device tensors, through one pinned buffer and one
@@ -1093,26 +1116,27 @@ class Engine:
         return list(flat.split([len(p) for p in parts]))
 
     def _run_prefill(self, reqs: List[Request], lens: List[int]):
-        dev = self.device
-        hidden, cu_q = self._forward_portions(
-            reqs, [r.prefill_pos for r in reqs], lens)
         # requests whose prefill completes sample their first token;
         # group parents fork their children first (shared prompt pages)
-        done_rows, done_reqs = [], []
-        fork_list = []
-        for i, (r, take) in enumerate(zip(reqs, lens)):
+        rows, done, at = [], [], 0
+        for r, take in zip(reqs, lens):
+            at += take
+            if r.prefill_pos + take >= len(r.input_ids):
+                rows.append(at - 1)
+                done.append(r)
+        hidden = self._forward_portions(
+            reqs, [r.prefill_pos for r in reqs], lens, rows)
+        for r, take in zip(reqs, lens):
             r.prefill_pos += take
-            if r.prefill_pos >= len(r.input_ids):
-                if r.group_children:
-                    fork_list.append((r, cu_q[i + 1] - 1))
-                else:
-                    done_rows.append(cu_q[i + 1] - 1)
-                    done_reqs.append(r)
-        if done_reqs:
-            rows = hidden[torch.tensor(done_rows, dtype=torch.long, device=dev)]
-            self._sample_last(done_reqs, rows)
-        for r, row in fork_list:
-            self._fork_group(r, hidden[row])
+        alone = [i for i, r in enumerate(done) if not r.group_children]
+        if alone:
+            self._sample_last([done[i] for i in alone],
+                              hidden if len(alone) == len(done)
+                              else hidden[torch.tensor(alone, dtype=torch.long,
+                                                       device=self.device)])
+        for i, r in enumerate(done):
+            if r.group_children:
+                self._fork_group(r, hidden[i])
 
     def _fork_group(self, parent: Request, last_hidden: torch.Tensor):
         """Fork n-1 children off a freshly prefilled group parent: shared
