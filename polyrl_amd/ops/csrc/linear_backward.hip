@@ -27,13 +27,14 @@ using namespace product;
 
 // out (R, C): sums over inner of left(row, inner) right(inner, column), right in
 // COLUMNS.  ``ways`` blocks share a tile's inner numbers, whose fp32 sums (tiles, ways,
-// SIDE * SIDE) are added up afterwards.
-template <bool LINES>
+// SIDE * SIDE) are added up afterwards.  LINES: tiles of 32 J rows.
+template <bool LINES, int J>
 __global__ __launch_bounds__(256, 1) void product_kernel(
     bf16_t* __restrict__ out, float* __restrict__ shares,
     const bf16_t* __restrict__ left, const bf16_t* __restrict__ right, long R,
     long C, long inner, int row_tiles, int col_tiles, int ways) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  constexpr int ROWS = 32 * J;
   const int tiles = row_tiles * col_tiles, items = tiles * ways;
   const int all = (int)((inner + PAIR - 1) / PAIR);
   auto units = [&](int r, Units& a, Units& b) {
@@ -43,31 +44,31 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
     const Place at(item - part * tiles, row_tiles, col_tiles);
     const int p0 = (int)((long)all * part / ways);
     const int n = (int)((long)all * (part + 1) / ways) - p0;
-    const long r0 = (long)at.row * SIDE, c0 = (long)at.col * SIDE;
+    const long r0 = (long)at.row * ROWS, c0 = (long)at.col * SIDE;
     const long i0 = (long)p0 * PAIR;
     a = LINES ? lines(left, R, inner, r0, i0, n) : columns(left, R, inner, r0, i0, n);
     b = columns(right, C, inner, c0, i0, n);
     return true;
   };
-  auto finish = [&](int r, Acc<>& acc) {
+  auto finish = [&](int r, Acc<J>& acc) {
     const int lane = threadIdx.x & 63, wid = wave_id();
     const int item = item_of(r, items, gridDim.x), part = item / tiles;
     const int tile = item - part * tiles;
-    if (ways > 1) {
+    if (J == 8 && ways > 1) {
       f32x4_t* p = reinterpret_cast<f32x4_t*>(
                        shares + ((long)tile * ways + part) * SIDE * SIDE) +
                    wid * 4096 + lane;
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p[(i * 8 + j) * 64] = sums_of(acc[i][j]);
+        for (int j = 0; j < J; ++j) p[(i * 8 + j) * 64] = sums_of(acc[i][j]);
       return;
     }
     const Place at(tile, row_tiles, col_tiles);
-    const long r0 = (long)at.row * SIDE + (wid & 1) * 128 + (lane & 15);
+    const long r0 = (long)at.row * ROWS + (wid & 1) * (ROWS / 2) + (lane & 15);
     const long c0 = (long)at.col * SIDE + (wid >> 1) * 128 + 8 * (lane >> 4);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < J; ++j) {
       const long row = r0 + 16 * j;
       order();
 #pragma unroll
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
       }
     }
   };
-  run<LINES, false>(lds, LINES ? inner : R, C, units, finish);
+  run<LINES, false, J>(lds, LINES ? inner : R, C, units, finish);
 }
 
 // Sums of the shares: a wave takes 16 rows of 32 outputs
@@ -152,9 +153,11 @@ template <bool LINES>
 torch::Tensor product_of(const torch::Tensor& left, const torch::Tensor& right, long R,
                       long C, long inner) {
   auto out = torch::empty({R, C}, left.options());
-  const long row_tiles = (R + SIDE - 1) / SIDE, col_tiles = (C + SIDE - 1) / SIDE;
-  const long tiles = row_tiles * col_tiles, ways = ways_of(tiles, inner);
-  const long items = tiles * ways;
+  const long col_tiles = (C + SIDE - 1) / SIDE;
+  const long ways = ways_of(tiles_of(R, C), inner);
+  const int parts = LINES && ways == 1 ? rows_of(R, col_tiles, inner, 6).parts : 8;
+  const long row_tiles = (R + 32 * parts - 1) / (32 * parts);
+  const long tiles = row_tiles * col_tiles, items = tiles * ways;
   TORCH_CHECK(items < (1L << 31) - ATTN_XCDS, "grid too large");
   const long grid = blocks_of(items, inner / ways);
   torch::Tensor shares;
@@ -163,10 +166,15 @@ torch::Tensor product_of(const torch::Tensor& left, const torch::Tensor& right, 
                           out.options().dtype(torch::kFloat32));
   float* sums = ways > 1 ? shares.data_ptr<float>() : nullptr;
   auto stream = at::hip::getCurrentHIPStream();
-  product_kernel<LINES><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(
-      (bf16_t*)out.data_ptr(), sums, (const bf16_t*)left.data_ptr(),
-      (const bf16_t*)right.data_ptr(), R, C, inner, (int)row_tiles,
-      (int)col_tiles, (int)ways);
+  auto launch = [&](auto kern) {
+    kern<<<dim3((unsigned)grid), dim3(256), 0, stream>>>(
+        (bf16_t*)out.data_ptr(), sums, (const bf16_t*)left.data_ptr(),
+        (const bf16_t*)right.data_ptr(), R, C, inner, (int)row_tiles,
+        (int)col_tiles, (int)ways);
+  };
+  if (LINES && parts == 6) launch(product_kernel<LINES, LINES ? 6 : 8>);
+  else if (LINES && parts == 7) launch(product_kernel<LINES, LINES ? 7 : 8>);
+  else launch(product_kernel<LINES, 8>);
   if (ways > 1)
     product_sum_kernel<<<dim3((unsigned)tiles * 32), dim3(256), 0, stream>>>(
         (bf16_t*)out.data_ptr(), sums, R, C, (int)row_tiles, (int)col_tiles,
@@ -190,19 +198,19 @@ bool linear_wgrad_takes(const torch::Tensor& dy, const torch::Tensor& x) {
          (tiles_of(dy.size(1), x.size(1)) >= 160 ? M >= 512 : M >= 5120);
 }
 
-// The same for linear_dgrad, where the library does better.  Tiles that fill two thirds
-// of each round of 256 take 0.78 to 1.02 of its time, less full ones up to 1.19 (of 2816,
-// 3072, 4096, 4608, 5376 rows through 4096 x 4096, 176 to 336 tiles: 78, 80, 95, 157, 159 us
-// for 80, 85, 103, 135, 159); fewer tiles pay where the inner dimension is long enough
-// to be shared (256, 1024, 2048 rows through 14336 x 4096 46, 98, 176 for 69, 134, 209;
-// through 8192 x 2048 26, 46, 70 for 37, 60, 75; through 4096 x 4096 26, 47, 70 for 25,
-// 42, 63).
+// The same for linear_dgrad, where the library does better.  Where tiles fill rounds of
+// 256 to two thirds of what whole ones would cost it takes 0.70 to 0.93 of the library's
+// time, less full ones up to 1.09 (through 4096 x 4096 of 2048, 2600, 4600, 5135, 7168 rows,
+// 1.64, 1.29, 1.46, 1.31, 1.04 of that cost: 71, 68, 130, 133, 164 us for 65, 79, 144, 178,
+// 204); half a chip's tiles and less pay where the inner dimension is long enough to be
+// shared (256, 1024, 2048 rows through 14336 x 4096 46, 98, 176 for 69, 134, 209; through
+// 8192 x 2048 26, 46, 70 for 37, 60, 75; through 4096 x 4096 26, 47, 70 for 25, 42, 63).
 bool linear_dgrad_takes(const torch::Tensor& dy, const torch::Tensor& w) {
   if (!dgrad_fits(dy, w)) return false;
-  const long M = dy.size(0), N = dy.size(1), tiles = tiles_of(M, w.size(1));
-  if (tiles <= CUS / 2) return N >= 8192 && M >= 64;
-  const long rounds = (tiles + CUS - 1) / CUS;
-  return 3 * tiles >= 2 * rounds * CUS - 16;
+  const long M = dy.size(0), N = dy.size(1), K = w.size(1);
+  if (tiles_of(M, K) <= CUS / 2) return N >= 8192 && M >= 64;
+  const double whole = (double)M * K / (CUS * SIDE * SIDE) * cost_of(8, N);
+  return rows_of(M, (K + SIDE - 1) / SIDE, N, 6).cost <= 1.5 * whole;
 }
 
 // dW (N, K) = dY^T X of dY (M, N), X (M, K)

@@ -11,7 +11,7 @@
 // of an output meet in one lane.  Nothing is rounded but the result.
 //
 // What bounds it: the matrix cores and, in few rounds of tiles, how full the last one
-// is (linear_rows_of).  Measured (us, beside the kernel that this replaces, eight waves of
+// is (rows_of).  Measured (us, beside the kernel that this replaces, eight waves of
 // 128 x 64 and a block a tile, and the library's product with the activation's pass):
 // 1024 -> 4096 of 513, 1024, 5135 and 8192 rows 15.0, 18.5, 74.0, 113 for 15.8, 20.1, 86.9,
 // 128 and 23.8, 28.2, 103, 149; 2048 -> 8192 34.1, 51.8, 256, 391 for 39.0, 60.8, 310, 461
@@ -85,22 +85,6 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
   run<true, true, J>(lds, K, K, units, finish);
 }
 
-// Rows of a tile, in 32s: as many as end the last round of 256 tiles earliest.  A unit of
-// 64 inner numbers costs 0.105 us a row part and 0.25 for the columns' fragments and loads,
-// a tile 5 us more.  (1024 -> 4096, tiles of 128, 192, 224 and 256 rows: 5135 rows 89.2, 81.4,
-// 74.0, 81.0 us; 1500 rows 30.0, 24.7, 26.8, 28.8; 1024 rows 18.5, 22.8, 24.0, 25.8; 3072
-// rows, 1536 -> 8960, 145, 142, 136, 147; 5135 rows, 4096 -> 14336, 1068, 875, 868, 888.)
-int linear_rows_of(long M, long cols, long K) {
-  int best = 8;
-  long least = -1;
-  for (int j = 3; j <= 8; ++j) {
-    const long items = (M + 32 * j - 1) / (32 * j) * cols;
-    const long cost = (items + CUS - 1) / CUS * (K / PAIR * (10 * j + 24) + 480);
-    if (least < 0 || cost <= least) least = cost, best = j;
-  }
-  return best;
-}
-
 template <bool GLU>
 torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
   for (const auto* t : {&x, &w})
@@ -116,7 +100,7 @@ torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
   auto out = torch::empty({M, N}, x.options());
   if (M == 0 || N == 0) return out;
   const long cols = w.size(0) / 256;
-  const int best = linear_rows_of(M, cols, K);
+  const int best = rows_of(M, cols, K, 3).parts;
   const long rows = (M + 32 * best - 1) / (32 * best), items = rows * cols;
   TORCH_CHECK(items < (1L << 31) - ATTN_XCDS, "grid too large");
   const dim3 grid((unsigned)blocks_of(items, K));

@@ -3,8 +3,8 @@
 //
 // Split.  A block has four waves, 128 x 128 outputs each: 256 accumulator registers a
 // lane, 128 more for the fragments of two steps, one wave a SIMD, one block a CU.  (Tiles
-// of fewer rows, 32 J, where both operands are LINES: a wave has J row parts for eight.)  A
-// step is 32 inner numbers.  Two steps of an operand, 32 KiB, are loaded as one unit
+// of fewer rows, 32 J, where the left operand is LINES: a wave has J row parts for eight.)
+// A step is 32 inner numbers.  Two steps of an operand, 32 KiB, are loaded as one unit
 // straight into LDS, five units' room; a barrier every two steps.  Where an operand's
 // inner dimension is its memory's rows' own (LINES: x and W in x W^T, dY in dY W) a unit
 // is 256 rows of 128 bytes, whole lines, and fragments are read as they are; where it
@@ -15,7 +15,8 @@
 // Schedule.  One wave a SIMD has nobody to take its turn: the order is fixed instruction
 // by instruction (order()).  Behind each of a step's 64 v_mfma_f32_16x16x32_bf16, 16
 // cycles each, stands at most one of the next step's fragment reads, of the unit's
-// loads, of the words that say where a load goes, or of the next addresses.  A block's
+// loads, of the words that say where a load goes, or of the next addresses, a fragment
+// to three products (two: 3% slower, 582 for 566 us at 7168 x 14336 x 4096).  A block's
 // tiles are one stream of units: at a tile's end the next one's first are there.
 #pragma once
 
@@ -257,9 +258,11 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
   auto step = [&](auto n_, auto& load, unsigned slot, int a_next, int b_next) {
     constexpr int N = decltype(n_)::value, O = 1 - N;
     constexpr int FRAGS = 8 + J, LOADS = N == 0 ? J : 8, ALL = 8 * J;
-    // instructions of a fragment (and a load's two, or with the load's first)
-    constexpr int PER = LL && RL ? 2 : 3;
-    static_assert(PER * FRAGS <= ALL && 2 * LOADS <= PER * FRAGS, "the order");
+    // instructions of a fragment (and a load's two, or with the load's first; few row
+    // parts leave room for two)
+    constexpr int PER = LL && RL && J < 6 ? 2 : 3;
+    static_assert(PER == 2 ? LOADS <= FRAGS : 2 * LOADS <= FRAGS + 2, "the order");
+    static_assert(PER * FRAGS + 2 <= ALL, "the order");
     __builtin_amdgcn_s_waitcnt(0xc07f);            // fragments: lgkmcnt(0)
     // The next unit of both is there, and this one's, read to the end, make room
     if constexpr (N == 1) arrived<J>();
@@ -290,6 +293,11 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
         // the addresses of the pair that comes next, and the next unit to load
         constexpr int d = k - PER * FRAGS, REST = ALL - PER * FRAGS;
         constexpr int FA = Operand<LL, J>::FRAGS, FB = Operand<RL>::FRAGS;
+        // (what of the loads had no place beside a fragment)
+        if constexpr (PER == 3 && (FRAGS + d) / 2 < LOADS) {
+          if constexpr ((FRAGS + d) % 2 == 0) aim(slot + (FRAGS + d) / 2 * 1024);
+          else load.go((FRAGS + d) / 2);
+        }
         if constexpr (N == 0)
           each(std::make_integer_sequence<int, FA + FB>(), [&](auto e_) {
             constexpr int e = decltype(e_)::value;
@@ -383,6 +391,31 @@ DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
     out[w] = q[0], out[2 + w] = q[1];
   }
   return out;
+}
+
+// Rows of a tile whose left operand is LINES, in 32s from LEAST on (6 where the right one
+// is COLUMNS): as many as end the last round of 256 tiles earliest.  A unit of 64 inner
+// numbers costs 0.105 us a row part and 0.25 for the columns' fragments and loads, a tile
+// 5 us more.  (1024 -> 4096, tiles of 128, 192, 224 and 256 rows: 5135 rows 89.2, 81.4,
+// 74.0, 81.0 us; 1500 rows 30.0, 24.7, 26.8, 28.8; 1024 rows 18.5, 22.8, 24.0, 25.8; 3072
+// rows, 1536 -> 8960, 145, 142, 136, 147; 5135 rows, 4096 -> 14336, 1068, 875, 868, 888; the
+// gradient of 7168 rows through 14336 x 4096, 192 to 256 rows a tile, 703, 539, 573, of 8192
+// 767, 748, 615.)
+struct Rows {
+  int parts;
+  long cost;
+};
+inline long cost_of(int parts, long inner) {
+  return inner / PAIR * (10 * parts + 24) + 480;
+}
+inline Rows rows_of(long rows, long cols, long inner, int least) {
+  Rows best{8, -1};
+  for (int j = least; j <= 8; ++j) {
+    const long items = (rows + 32 * j - 1) / (32 * j) * cols;
+    const long cost = (items + CUS - 1) / CUS * cost_of(j, inner);
+    if (best.cost < 0 || cost <= best.cost) best = {j, cost};
+  }
+  return best;
 }
 
 // Blocks: as many as run at once, each with its tiles one after the other, but of few

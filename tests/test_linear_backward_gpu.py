@@ -65,6 +65,13 @@ def test_dgrad_outer(m, k):
     dgrad(m, 192, k)
 
 
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("m", [1500, 1791, 1799, 2041])
+def test_dgrad_rows(m, n):
+    """Tiles of 192 rows, 224 and 256: one round of them each."""
+    dgrad(m, n, 8184)
+
+
 @pytest.mark.parametrize("inner", [193, 256, 320, 384, 448])
 def test_tiles_in_turn(inner):
     """More tiles than blocks that run at once: a block's second tile and third,
