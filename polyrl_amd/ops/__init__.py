@@ -83,6 +83,12 @@ def linear_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def linear_rows_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_rows``, which takes these operands, is the faster one on
+    the device."""
+    return _require_ext().linear_rows_pays(x.shape[0], w.shape[0], x.shape[1])
+
+
 def linear_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w.T of many rows (no autograd)."""
     return _require_ext().linear_rows(x, w) if x.is_cuda else x @ w.t()

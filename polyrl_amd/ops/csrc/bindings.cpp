@@ -9,6 +9,9 @@ void fused_add_rmsnorm(torch::Tensor out, torch::Tensor residual,
 void silu_mul(torch::Tensor out, torch::Tensor gate, torch::Tensor up);
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor linear_swiglu(torch::Tensor x, torch::Tensor w);
+bool linear_rows_pays(long M, long N, long K);
+void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
+                      const torch::Tensor& w);
 void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
                   torch::Tensor cos_tab, torch::Tensor sin_tab);
 void rope_kv_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -86,6 +89,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual-add + RMSNorm, residual updated in place");
   m.def("silu_mul", &silu_mul, "SiLU(gate) * up");
   m.def("linear_rows", &linear_rows, "x W^T of prompts");
+  m.def("linear_rows_into", &linear_rows_into, "x W^T, W's rows in 8s");
+  m.def("linear_rows_pays", &linear_rows_pays, "linear_rows for the library's product");
   m.def("linear_swiglu", &linear_swiglu, "SiLU(x Wg^T) * (x Wu^T)");
   m.def("rope_inplace", &rope_inplace, "NEOX RoPE in place (table-driven)");
   m.def("rope_kv_append", &rope_kv_append,

@@ -17,7 +17,12 @@
 //   fwd  (nt): Y[M,N] = X[M,K] @ W[N,K]^T  ->  C(N,M) = op_T(W) op_N(X)
 //   dgrad(nn): dX[M,K] = dY[M,N] @ W[N,K]  ->  C(K,M) = op_N(W) op_N(dY)
 //   wgrad(tn): dW[N,K] = dY[M,N]^T @ X[M,K]->  C(K,N) = op_N(X) op_T(dY)
-// Most gradients of many rows are the kernels' in linear_backward.hip.
+// Most gradients of many rows are the kernels' in linear_backward.hip, and the forward
+// product of linear_prompt.hip is one more candidate of the search: of 1000 to 8192 rows
+// it takes 0.86 to 0.98 of the best algorithm's time where tiles of 256 rows are not
+// whole (7168 rows, 4096 -> 14336, 14336 -> 4096, 4096 -> 4096 559, 542, 158 us for 575, 576,
+// 164; 1000, 4096 and 8192 rows to 128256 744, 2867, 5623 for 864, 2935, 5890), 1.02 to 1.04
+// where they are.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hipblaslt/hipblaslt.h>
@@ -39,19 +44,28 @@ bool linear_wgrad_takes(const torch::Tensor& dy, const torch::Tensor& x);
 bool linear_dgrad_takes(const torch::Tensor& dy, const torch::Tensor& w);
 torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x);
 torch::Tensor linear_dgrad(torch::Tensor dy, torch::Tensor w);
+// linear_prompt.hip
+bool linear_rows_fits(const torch::Tensor& x, const torch::Tensor& w);
+void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
+                      const torch::Tensor& w);
 
 namespace {
 
 constexpr size_t kWorkspaceBytes = 128ull << 20;
 constexpr int kMaxAlgos = 48;
 constexpr int kTimedIters = 3;
+constexpr int64_t kKernelRows = 513;   // fewer leave the kernel's tiles empty
+
+struct Pick {
+  hipblasLtMatmulAlgo_t algo;
+  bool kernel;                         // linear_prompt.hip's is the faster one
+};
 
 struct LtState {
   hipblasLtHandle_t handle = nullptr;
   std::mutex mu;
   // key: (mode, M, N, K) -> winning algo
-  std::map<std::tuple<int, int64_t, int64_t, int64_t>, hipblasLtMatmulAlgo_t>
-      cache;
+  std::map<std::tuple<int, int64_t, int64_t, int64_t>, Pick> cache;
 };
 
 LtState& lt() {
@@ -130,20 +144,27 @@ void tuned_mm(int mode, const torch::Tensor& A_row, const torch::Tensor& B_row,
     Bptr = A_row.data_ptr();  // dY
   }
 
-  Plan p;
-  build_plan(p, opA, opB, m, n, k, lda, ldb, ldc);
-  const float alpha = 1.f, beta = 0.f;
-
-  hipblasLtMatmulAlgo_t algo;
+  // (an address of another alignment than the searched one's has the algorithm)
+  const bool kernel_fits =
+      mode == 0 && M >= kKernelRows && linear_rows_fits(A_row, B_row);
+  Pick pick;
   bool have_algo = false;
   {
     std::lock_guard<std::mutex> g(s.mu);
     auto it = s.cache.find({mode, M, N, K});
     if (it != s.cache.end()) {
-      algo = it->second;
+      pick = it->second;
       have_algo = true;
     }
   }
+  if (have_algo && pick.kernel && kernel_fits) {
+    linear_rows_into(C_row, A_row, B_row);
+    return;
+  }
+
+  Plan p;
+  build_plan(p, opA, opB, m, n, k, lda, ldb, ldc);
+  const float alpha = 1.f, beta = 0.f;
 
   if (!have_algo) {
     hipblasLtMatmulPreference_t pref;
@@ -185,20 +206,33 @@ void tuned_mm(int mode, const torch::Tensor& A_row, const torch::Tensor& B_row,
         best = i;
       }
     }
+    pick.kernel = false;
+    if (kernel_fits) {
+      linear_rows_into(C_row, A_row, B_row);
+      hipEventRecord(ev0, stream);
+      for (int it2 = 0; it2 < kTimedIters; ++it2)
+        linear_rows_into(C_row, A_row, B_row);
+      hipEventRecord(ev1, stream);
+      hipEventSynchronize(ev1);
+      float ms = 1e30f;
+      hipEventElapsedTime(&ms, ev0, ev1);
+      pick.kernel = ms < best_ms;
+    }
     hipEventDestroy(ev0);
     hipEventDestroy(ev1);
     TORCH_CHECK(best_ms < 1e29f, "hipblaslt: every candidate failed, mode=",
                 mode, " M=", M, " N=", N, " K=", K);
-    algo = results[best].algo;
+    pick.algo = results[best].algo;
     {
       std::lock_guard<std::mutex> g(s.mu);
-      s.cache[{mode, M, N, K}] = algo;
+      s.cache[{mode, M, N, K}] = pick;
     }
+    if (pick.kernel) return;           // (its product is the one there)
   }
 
   HIPBLASLT_CHECK(hipblasLtMatmul(
       s.handle, p.op, &alpha, Aptr, p.la, Bptr, p.lb, &beta, Cptr, p.lc,
-      Cptr, p.lc, &algo, workspace, kWorkspaceBytes, stream));
+      Cptr, p.lc, &pick.algo, workspace, kWorkspaceBytes, stream));
 }
 
 void check2d(const torch::Tensor& t, const char* name) {

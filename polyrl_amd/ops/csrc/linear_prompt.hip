@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
                       u[e];
         }
         const u32x4_t v = eight_columns(y[0], y[1]);
-        if (row < M)
+        if (row < M && (GLU || c0 + 16 * i < N))
           *reinterpret_cast<u32x4_t*>(out + row * N + c0 + 16 * i) = v;
       }
     }
@@ -86,20 +86,10 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
 }
 
 template <bool GLU>
-torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
-  for (const auto* t : {&x, &w})
-    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&
-                    t->is_contiguous() && t->dtype() == torch::kBFloat16 &&
-                    ((uintptr_t)t->data_ptr() & 15) == 0,
-                "linear: contiguous 2-D bf16 at 16-byte addresses of one device");
-  const long M = x.size(0), K = x.size(1), N = w.size(0) / (GLU ? 2 : 1);
-  TORCH_CHECK(w.size(1) == K && K % PAIR == 0 && K > 0 && w.size(0) % 256 == 0 &&
-                  K < (1L << 20) && N < (1L << 25) && M < (1L << 30),
-              "linear: inner numbers in 64s, the weight's rows in 256s, outputs "
-              "below 2^25");
-  auto out = torch::empty({M, N}, x.options());
-  if (M == 0 || N == 0) return out;
-  const long cols = w.size(0) / 256;
+void launch_linear(torch::Tensor& out, const torch::Tensor& x, const torch::Tensor& w) {
+  const long M = x.size(0), K = x.size(1), N = out.size(1);
+  if (M == 0 || N == 0) return;
+  const long cols = (w.size(0) + SIDE - 1) / SIDE;
   const int best = rows_of(M, cols, K, 3).parts;
   const long rows = (M + 32 * best - 1) / (32 * best), items = rows * cols;
   TORCH_CHECK(items < (1L << 31) - ATTN_XCDS, "grid too large");
@@ -119,10 +109,62 @@ torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
     default: launch(linear_kernel<8, GLU>);
   }
   HIP_CHECK_KERNEL();
+}
+
+template <bool GLU>
+torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
+  for (const auto* t : {&x, &w})
+    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&
+                    t->is_contiguous() && t->dtype() == torch::kBFloat16 &&
+                    ((uintptr_t)t->data_ptr() & 15) == 0,
+                "linear: contiguous 2-D bf16 at 16-byte addresses of one device");
+  const long M = x.size(0), K = x.size(1), N = w.size(0) / (GLU ? 2 : 1);
+  TORCH_CHECK(w.size(1) == K && K % PAIR == 0 && K > 0 && w.size(0) % 256 == 0 &&
+                  K < (1L << 20) && N < (1L << 25) && M < (1L << 30),
+              "linear: inner numbers in 64s, the weight's rows in 256s, outputs "
+              "below 2^25");
+  auto out = torch::empty({M, N}, x.options());
+  launch_linear<GLU>(out, x, w);
   return out;
 }
 
 }  // namespace
+
+// Whether linear_rows_into has these contiguous bf16 matrices: as linear_rows, but the
+// weight's rows, which are whole 16-byte granules of the output, in 8s
+bool linear_rows_fits(const torch::Tensor& x, const torch::Tensor& w) {
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  return M > 0 && M < (1L << 30) && K > 0 && K % PAIR == 0 && K < (1L << 20) && N > 0 &&
+         N % 8 == 0 && N < (1L << 25) &&
+         (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
+}
+
+void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
+                      const torch::Tensor& w) {
+  for (const auto* t : {(const torch::Tensor*)&out, &x, &w})
+    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&
+                    t->is_contiguous() && t->dtype() == torch::kBFloat16,
+                "linear: contiguous 2-D bf16 of one device");
+  TORCH_CHECK(w.size(1) == x.size(1) && out.size(0) == x.size(0) &&
+                  out.size(1) == w.size(0) && linear_rows_fits(x, w) &&
+                  ((uintptr_t)out.data_ptr() & 15) == 0,
+              "linear: inner numbers in 64s, outputs in 8s, 16-byte addresses");
+  launch_linear<false>(out, x, w);
+}
+
+// Whether linear_rows is the better choice than the library's own: tiles that fill
+// rounds of 256 to 0.74 of what whole ones would cost, but not whole tiles of 256 rows,
+// which the library multiplies 1 to 4% faster.  (us, beside the library's, of 2600, 4096,
+// 5135 and 7168 rows: 2048 -> 2048 25.0, 29.8, 36.0, 44.0 and 29.1, 32.8, 48.6, 45.1;
+// 8192 -> 2048 81.5, 99.6, 123, 151 and 82.0, 107, 146, 156; 8960 -> 1536 94.7, 98.3,
+// 108, 138 and 72.5, 96.7, 117, 151, whose first two fill 0.44 and 0.6; 4096 of 14336 ->
+// 4096 296 and 289.)
+bool linear_rows_pays(long M, long N, long K) {
+  if (M <= 0 || N <= 0 || K < PAIR) return false;
+  const Rows best = rows_of(M, (N + SIDE - 1) / SIDE, K, 3);
+  const double whole = (double)M * N / (CUS * SIDE * SIDE) * cost_of(8, K);
+  return best.cost <= 1.35 * whole && (best.parts < 8 || M % SIDE != 0);
+}
 
 // x (M, K), w (N, K)
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w) {

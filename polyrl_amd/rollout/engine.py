@@ -34,25 +34,25 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor, search: bool = True
     algo-pinned hipBLASLt path (ops.tuned_mm_nt) — the heuristic pick runs
     skinny decode projections far off the weight-read bound.  Prefill Ms
     are ragged (chunk sums), so they are not searched: inner widths up to
-    1024 and up to 3 x 2^22 outputs take the kernel of this repository, whose
-    call costs the host 5 us for the 20 of torch's (a step of 3, 4, 6 and 8 x 256
+    1024 and up to 3 x 2^22 outputs, and wider ones whose tiles fill the chip
+    (``ops.linear_rows_pays``), take the kernel of this repository, whose call
+    costs the host 5 us for the 20 of torch's (a step of 3, 4, 6 and 8 x 256
     tokens, 12 layers of 1024, 1109, 1124, 1286 and 1447 us with it and 1471, 1491,
-    1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the
-    device it is up to 4 us slower within these lines (us, kernel and library, of
+    1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the device it is up to 4 us slower within these lines (us, kernel and library, of
     513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 8.3, 8.5, 8.8, 9.4, 13.0 and 6.3,
     6.6, 7.7, 9.7, 14.9; 1024 -> 1024 11.7, 12.0, 12.7, 14.9, 19.4 and 7.7, 8.0, 10.4,
     13.3, 21.5; 1024 -> 1536 11.8, 12.2, 13.8, 17.1, 28.4 and 7.8, 9.8, 13.1, 18.5,
-    29.3), beyond them by more than the host gains where outputs are few (1024 of
-    600 .. 4700 rows 0.55 to 0.91 of the library's speed at an inner width of 4096)
-    and about as fast elsewhere; a captured graph, where the host's time does not
+    29.3); of wider ones it would be by more than the host gains where outputs are few
+    (1024 of 600 .. 4096 rows 0.5 to 0.83 of the library's speed at an inner width of
+    4096); a captured graph, where the host's time does not
     count, takes the library's.  ``search``: False for few rows whose number is not
     a decode batch's."""
     if search and x.is_cuda and x.dtype == torch.bfloat16 \
             and x.shape[0] <= 512 and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
-    if 512 < x.shape[0] <= 8192 and x.shape[1] <= 1024 \
-            and x.shape[0] * w.shape[0] <= 3 << 22 \
-            and ops.linear_takes(x, w) \
+    if 512 < x.shape[0] and ops.linear_takes(x, w) and (
+            ops.linear_rows_pays(x, w) if x.shape[1] > 1024 else
+            x.shape[0] <= 8192 and x.shape[0] * w.shape[0] <= 3 << 22) \
             and not torch.cuda.is_current_stream_capturing():
         return ops.linear_rows(x, w)
     return x @ w.t()

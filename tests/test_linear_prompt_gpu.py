@@ -169,3 +169,49 @@ def test_engine_prompts(m, n, k, rows, glu, monkeypatch):
             graph.replay()
             assert (both.double() - exact).norm() / exact.norm() <= 5e-3
         assert ran == ["linear_rows"]
+
+
+@pytest.mark.parametrize("n", [8, 248, 264, 504, 1016])
+@pytest.mark.parametrize("m", [1, 97, 600])
+def test_columns_short_of_a_tile(m, n):
+    """Outputs in 8s, what stands behind them is not touched."""
+    x = torch.randn(m, 320, device=DEV).bfloat16()
+    w = torch.randn(n, 320, device=DEV).bfloat16()
+    flat = torch.full((m * n + 4096,), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = flat[:m * n].view(m, n)
+    ops._require_ext().linear_rows_into(out, x, w)
+    want, mass = x.double() @ w.double().t(), x.abs().double() @ w.abs().double().t()
+    assert ((out.double() - want).abs()
+            <= 2 ** -8 * want.abs() + 320 * 2.0 ** -24 * mass).all()
+    assert (flat[m * n:] == 7).all()
+
+
+def test_linears_search():
+    """A linear layer of many rows: whichever product the search finds, again and
+    at an address that the kernel does not take."""
+    m, n, k = 1400, 1096, 1088
+    flat = torch.randn(m * k + 1, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16() / k ** 0.5
+    for x in (flat[:-1].view(m, k), flat[1:].view(m, k)):
+        want = x.double() @ w.double().t()
+        for _ in range(2):
+            y = ops.tuned_linear(x, w)
+            assert (y.double() - want).norm() / want.norm() <= 5e-3
+
+
+@pytest.mark.parametrize("m,n,k,rows", [
+    (2600, 2048, 2048, False), (4096, 2048, 2048, True), (4100, 2048, 2048, False),
+    (2048, 4096, 2048, True),
+    (4096, 4096, 2048, False), (4095, 4096, 2048, True), (5000, 512, 4096, False)])
+def test_engine_wide_prompts(m, n, k, rows, monkeypatch):
+    """Both sides of the line for widths beyond 1024."""
+    from polyrl_amd.rollout.engine import _mm_nt
+    ran = []
+    real = ops.linear_rows
+    monkeypatch.setattr(ops, "linear_rows",
+                        lambda x, w: ran.append(1) or real(x, w))
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16() / k ** 0.5
+    want = x.float() @ w.float().t()
+    assert (_mm_nt(x, w).float() - want).norm() / want.norm() <= 5e-3
+    assert bool(ran) == rows
