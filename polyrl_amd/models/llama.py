@@ -115,6 +115,13 @@ class RotaryCache(nn.Module):
         return self.cos_cached[idx], self.sin_cached[idx]
 
 
+def _lins(mods, x: torch.Tensor):
+    """``_lin`` of several layers of one input."""
+    import polyrl_amd.ops as pops
+    ys = pops.joint_linear(x, mods)
+    return [_lin(m, x) for m in mods] if ys is None else ys
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: DecoderConfig):
         super().__init__()
@@ -141,9 +148,10 @@ class Attention(nn.Module):
         the reverse all-to-all restores the token shard."""
         import polyrl_amd.ops as pops
         T = x.shape[0]
-        q = _lin(self.q_proj, x).view(T, self.num_heads, self.head_dim)
-        k = _lin(self.k_proj, x).view(T, self.num_kv_heads, self.head_dim)
-        v = _lin(self.v_proj, x).view(T, self.num_kv_heads, self.head_dim)
+        q, k, v = _lins((self.q_proj, self.k_proj, self.v_proj), x)
+        q = q.view(T, self.num_heads, self.head_dim)
+        k = k.view(T, self.num_kv_heads, self.head_dim)
+        v = v.view(T, self.num_kv_heads, self.head_dim)
         if q.is_cuda and q.dtype == torch.bfloat16 \
                 and self.head_dim in (64, 128):
             # single-pass fused rotation fwd/bwd (ops/csrc/rope_train.hip)
@@ -186,9 +194,10 @@ class Attention(nn.Module):
         all-to-all trades it for a head shard over the full sequence
         (parallel/ulysses.py)."""
         B, Ls, _ = x.shape
-        q = _lin(self.q_proj, x).view(B, Ls, self.num_heads, self.head_dim)
-        k = _lin(self.k_proj, x).view(B, Ls, self.num_kv_heads, self.head_dim)
-        v = _lin(self.v_proj, x).view(B, Ls, self.num_kv_heads, self.head_dim)
+        q, k, v = _lins((self.q_proj, self.k_proj, self.v_proj), x)
+        q = q.view(B, Ls, self.num_heads, self.head_dim)
+        k = k.view(B, Ls, self.num_kv_heads, self.head_dim)
+        v = v.view(B, Ls, self.num_kv_heads, self.head_dim)
         if sp_group is not None:
             from ..parallel.ulysses import all_to_all_4d
             import torch.distributed as _dist
@@ -232,11 +241,14 @@ class MLP(nn.Module):
         self.down_proj = nn.Linear(i, h, bias=cfg.mlp_bias)
 
     def forward(self, x):
+        import polyrl_amd.ops as pops
+        act = pops.gated_linear(x, self.gate_proj, self.up_proj)
+        if act is not None:
+            return _lin(self.down_proj, act)
         g = _lin(self.gate_proj, x)
         u = _lin(self.up_proj, x)
         if g.is_cuda and g.dtype == torch.bfloat16 \
                 and g.shape[-1] % 8 == 0:
-            import polyrl_amd.ops as pops
             return _lin(self.down_proj, pops.silu_mul_train(g, u))
         return _lin(self.down_proj, F.silu(g) * u)
 

@@ -522,6 +522,99 @@ def tuned_linear(x: torch.Tensor, w: torch.Tensor,
     return torch.nn.functional.linear(x, w, b)
 
 
+class _JointLinear(torch.autograd.Function):
+    """Linear layers of one input: their products in one launch, the input's
+    gradient as one sum of products (linear_prompt.hip, linear_backward.hip)."""
+
+    @staticmethod
+    def forward(ctx, x, *ws):
+        ctx.save_for_backward(x, *ws)
+        return tuple(_require_ext().linear_joint(x, list(ws)))
+
+    @staticmethod
+    def backward(ctx, *dys):
+        x, *ws = ctx.saved_tensors
+        return _joint_backward(ctx.needs_input_grad, x, ws,
+                               [dy.contiguous() for dy in dys])
+
+
+def _joint_backward(needs, x, ws, dys):
+    ext = _require_ext()
+    dx = None
+    if needs[0]:
+        if ext.linear_dgrad_sum_takes(dys, ws):
+            dx = ext.linear_dgrad_sum(dys, ws)
+        else:
+            for dy, w in zip(dys, ws):
+                d = ext.tuned_linear_dgrad(dy, w)
+                dx = d if dx is None else dx.add_(d)
+    return dx, *(ext.tuned_linear_wgrad(dy, x) if need else None
+                 for dy, need in zip(dys, needs[1:]))
+
+
+class _GatedLinear(torch.autograd.Function):
+    """silu(x Wg^T) * (x Wu^T): both products and the activation in one kernel,
+    which keeps the products for the way back."""
+
+    @staticmethod
+    def forward(ctx, x, wg, wu):
+        keep = any(ctx.needs_input_grad)
+        out, *kept = _require_ext().linear_gated(x, wg, wu, keep)
+        if keep:
+            ctx.save_for_backward(x, wg, wu, *kept)
+        return out
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, wg, wu, gate, up = ctx.saved_tensors
+        dgate, dup = torch.empty_like(gate), torch.empty_like(up)
+        _require_ext().silu_mul_bwd(dgate, dup, dy.contiguous(), gate, up)
+        return _joint_backward(ctx.needs_input_grad, x, [wg, wu], [dgate, dup])
+
+
+def _plain_weights(x: torch.Tensor, mods):
+    """Weights of linear layers of one input where the trainer's products may take
+    them (as :func:`tuned_linear`), else None."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and _tuned_gemm_enabled()
+            and not hasattr(x, "placements")):
+        return None
+    ws = []
+    for m in mods:
+        if type(m) is not torch.nn.Linear:
+            return None
+        w = m.weight
+        if w.dtype != torch.bfloat16 or hasattr(w, "placements"):
+            return None
+        ws.append(w)
+    return ws
+
+
+def joint_linear(x: torch.Tensor, mods):
+    """Outputs of two or three ``nn.Linear`` of one input in one product, or None
+    where a product each is the better choice or the only one."""
+    ws = _plain_weights(x, mods)
+    if ws is None:
+        return None
+    rows = x.reshape(-1, x.shape[-1]).contiguous()
+    if not _require_ext().linear_joint_takes(rows, ws):
+        return None
+    return [y.view(*x.shape[:-1], y.shape[-1]) if m.bias is None
+            else y.view(*x.shape[:-1], y.shape[-1]) + m.bias
+            for y, m in zip(_JointLinear.apply(rows, *ws), mods)]
+
+
+def gated_linear(x: torch.Tensor, gate, up) -> Optional[torch.Tensor]:
+    """silu(gate(x)) * up(x) of two ``nn.Linear`` in one kernel, or None as
+    :func:`joint_linear`."""
+    ws = _plain_weights(x, (gate, up))
+    if ws is None or gate.bias is not None or up.bias is not None:
+        return None
+    rows = x.reshape(-1, x.shape[-1]).contiguous()
+    if not _require_ext().linear_gated_takes(rows, *ws):
+        return None
+    return _GatedLinear.apply(rows, *ws).view(*x.shape[:-1], ws[0].shape[0])
+
+
 def build_varlen_tiles(cu_seqlens_cpu: torch.Tensor, device):
     """Precompute the (64-row forward, 32-key backward) tile tables once per
     packed batch; reused by every layer's flash_attn_varlen call."""

@@ -10,6 +10,16 @@ void silu_mul(torch::Tensor out, torch::Tensor gate, torch::Tensor up);
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor linear_swiglu(torch::Tensor x, torch::Tensor w);
 bool linear_rows_pays(long M, long N, long K);
+bool linear_joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws);
+std::vector<torch::Tensor> linear_joint(torch::Tensor x, std::vector<torch::Tensor> ws);
+bool linear_gated_takes(const torch::Tensor& x, const torch::Tensor& wg,
+                        const torch::Tensor& wu);
+std::vector<torch::Tensor> linear_gated(torch::Tensor x, torch::Tensor wg,
+                                        torch::Tensor wu, bool keep);
+bool linear_dgrad_sum_takes(const std::vector<torch::Tensor>& dys,
+                            const std::vector<torch::Tensor>& ws);
+torch::Tensor linear_dgrad_sum(std::vector<torch::Tensor> dys,
+                               std::vector<torch::Tensor> ws);
 void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
                       const torch::Tensor& w);
 void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
@@ -89,6 +99,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual-add + RMSNorm, residual updated in place");
   m.def("silu_mul", &silu_mul, "SiLU(gate) * up");
   m.def("linear_rows", &linear_rows, "x W^T of prompts");
+  m.def("linear_joint_takes", &linear_joint_takes, "linear_joint for a product each");
+  m.def("linear_joint", &linear_joint, "x W^T of several weights");
+  m.def("linear_gated_takes", &linear_gated_takes, "linear_gated for a product each");
+  m.def("linear_gated", &linear_gated, "silu(x Wg^T) * (x Wu^T), and both products");
+  m.def("linear_dgrad_sum_takes", &linear_dgrad_sum_takes,
+        "linear_dgrad_sum for a product each");
+  m.def("linear_dgrad_sum", &linear_dgrad_sum, "the sum of dY_p W_p");
   m.def("linear_rows_into", &linear_rows_into, "x W^T, W's rows in 8s");
   m.def("linear_rows_pays", &linear_rows_pays, "linear_rows for the library's product");
   m.def("linear_swiglu", &linear_swiglu, "SiLU(x Wg^T) * (x Wu^T)");

@@ -1,6 +1,6 @@
 // Products of prompts (hundreds of rows and more) with a weight's rows, bf16:
-// x W^T, and silu(x Wg^T) * (x Wu^T), the gated MLP's two products and its
-// activation, in one kernel.
+// x W^T of one weight or several, and silu(x Wg^T) * (x Wu^T), the gated MLP's two
+// products and its activation, in one kernel.
 //
 // Reference capability: the engine-side projections and the fused gate/up
 // projection with its activation.
@@ -8,7 +8,12 @@
 // Tiles, schedule and layouts: product_tile.h, both operands in LINES.  A tile is 32 J
 // rows by 256 columns of the product, or (GLU) 128 of the gate's and 128 of the up
 // projection's, of which it makes 128 outputs: each wave has 64 of both, so gate and up
-// of an output meet in one lane.  Nothing is rounded but the result.
+// of an output meet in one lane.  Nothing is rounded but what is stored: the result, and
+// for the trainer the two products (KEPT).
+//
+// In a layer of the trainer of 7168 rows (its kernels one after the other): gate, up and
+// activation of 4096 -> 14336 1200 us for 585 + 585 + 112 of two products and a pass, q, k
+// and v of 4096 -> 4096, 1024, 1024 244 for 175 + 59 + 58.
 //
 // What bounds it: the matrix cores and, in few rounds of tiles, how full the last one
 // is (rows_of).  Measured (us, beside the kernel that this replaces, eight waves of
@@ -26,33 +31,66 @@ namespace {
 
 using namespace product;
 
-template <int J, bool GLU>
+// Outputs of one matrix of weights; of several products of the same rows each but the
+// last has whole tiles of columns
+struct Part {
+  bf16_t* out;                         // (M, n)
+  const bf16_t* w;                     // (n, K)
+  long n;
+};
+constexpr int MOST = 3;
+struct Parts {
+  Part p[MOST];
+};
+
+// PLAIN: the products.  GATED: out = silu(gate) * up of the products with p[0], gate, and
+// p[1], up.  KEPT: the products too.
+enum Kind { PLAIN, GATED, KEPT };
+
+template <int J, Kind KIND>
 __global__ __launch_bounds__(256, 1) void linear_kernel(
-    bf16_t* __restrict__ out,          // (M, N)
+    bf16_t* __restrict__ out,          // (M, n), but PLAIN
     const bf16_t* __restrict__ x,      // (M, K)
-    const bf16_t* __restrict__ w,      // (N, K), or (2 N, K): gate, up
-    long M, long N, long K, int row_tiles, int col_tiles) {
+    const Parts parts, long M, long K, int row_tiles, int col_tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  constexpr int ROWS = 32 * J, COLS = GLU ? 128 : 256;
+  constexpr int ROWS = 32 * J, COLS = KIND == PLAIN ? 256 : 128;
   const int items = row_tiles * col_tiles, n = (int)(K / PAIR);
+  const long N = parts.p[0].n;
+  // part of a tile of columns, and which column of it
+  auto part_of = [&](long& col) {
+    Part p = parts.p[0];
+    if (col >= p.n) {
+      col -= p.n, p = parts.p[1];
+      if (col >= p.n) col -= p.n, p = parts.p[2];
+    }
+    return p;
+  };
   auto units = [&](int r, Units& a, Units& b) {
     const int item = item_of(r, items, gridDim.x);
     if (item < 0) return false;
     const Place at(item, row_tiles, col_tiles);
     a = lines(x, M, K, (long)at.row * ROWS, 0, n);
-    if (GLU) {
+    long col = (long)at.col * COLS;
+    if (KIND != PLAIN) {
       // a wave loads the 64 rows of its number: gate, up, gate, up
       const int wid = wave_id();
-      const long row = (long)at.col * COLS + (wid >> 1) * 64 + (wid & 1) * N;
-      b = lines(w, 2 * N, K, row - wid * 64, 0, n);
+      b = lines(wid & 1 ? parts.p[1].w : parts.p[0].w, N, K,
+                col + (wid >> 1) * 64 - wid * 64, 0, n);
     } else {
-      b = lines(w, N, K, (long)at.col * COLS, 0, n);
+      const Part p = part_of(col);
+      b = lines(p.w, p.n, K, col, 0, n);
     }
     return true;
   };
   auto finish = [&](int r, Acc<J>& acc) {
     const int lane = threadIdx.x & 63, wid = wave_id();
     const Place at(item_of(r, items, gridDim.x), row_tiles, col_tiles);
+    if (KIND == PLAIN) {
+      long col = (long)at.col * COLS;
+      const Part p = part_of(col);
+      store_tile<J>(p.out, M, p.n, (long)at.row * ROWS, col, acc);
+      return;
+    }
     const long r0 = (long)at.row * ROWS + (wid & 1) * (16 * J) + (lane & 15);
     const long c0 = (long)at.col * COLS + (wid >> 1) * (COLS / 2) + 8 * (lane >> 4);
 #pragma unroll
@@ -60,55 +98,66 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
       const long row = r0 + 16 * j;
       order();
 #pragma unroll
-      for (int i = 0; i < (GLU ? 4 : 8); i += 2) {
-        f32x4_t y[2];
+      for (int i = 0; i < 4; i += 2) {
+        f32x4_t g[2], u[2], y[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          y[h] = sums_of(acc[i + h][j]);
-          if (!GLU) continue;
-          const f32x4_t u = sums_of(acc[(i + h + 4) % 8][j]);
+          g[h] = sums_of(acc[i + h][j]);
+          u[h] = sums_of(acc[i + h + 4][j]);
           // (the activation first: gate times up may be beyond 32 bits where the
           // sigmoid is 0)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            y[h][e] = y[h][e] *
+            y[h][e] = g[h][e] *
                       __builtin_amdgcn_rcpf(
-                          1.f + exp2_hw(y[h][e] * -1.4426950408889634f)) *
-                      u[e];
+                          1.f + exp2_hw(g[h][e] * -1.4426950408889634f)) *
+                      u[h][e];
         }
         const u32x4_t v = eight_columns(y[0], y[1]);
-        if (row < M && (GLU || c0 + 16 * i < N))
-          *reinterpret_cast<u32x4_t*>(out + row * N + c0 + 16 * i) = v;
+        const long at_out = row * N + c0 + 16 * i;
+        if (row < M) *reinterpret_cast<u32x4_t*>(out + at_out) = v;
+        if (KIND == KEPT) {
+          const u32x4_t gv = eight_columns(g[0], g[1]), uv = eight_columns(u[0], u[1]);
+          if (row < M) {
+            *reinterpret_cast<u32x4_t*>(parts.p[0].out + at_out) = gv;
+            *reinterpret_cast<u32x4_t*>(parts.p[1].out + at_out) = uv;
+          }
+        }
       }
     }
   };
-  run<true, true, J>(lds, K, K, units, finish);
+  run<true, true, J>(lds, [&](int) { return K; }, K, units, finish);
 }
 
-template <bool GLU>
-void launch_linear(torch::Tensor& out, const torch::Tensor& x, const torch::Tensor& w) {
-  const long M = x.size(0), K = x.size(1), N = out.size(1);
-  if (M == 0 || N == 0) return;
-  const long cols = (w.size(0) + SIDE - 1) / SIDE;
-  const int best = rows_of(M, cols, K, 3).parts;
+// cols: tiles of columns of the weights together
+template <Kind KIND>
+void launch_linear(bf16_t* out, const torch::Tensor& x, const Parts& parts, long cols) {
+  const long M = x.size(0), K = x.size(1);
+  if (M == 0 || cols == 0) return;
+  // (what is kept of the trainer's few rows is no path of its own)
+  const int best = rows_of(M, cols, K, KIND == KEPT ? 6 : 3).parts;
   const long rows = (M + 32 * best - 1) / (32 * best), items = rows * cols;
   TORCH_CHECK(items < (1L << 31) - ATTN_XCDS, "grid too large");
   const dim3 grid((unsigned)blocks_of(items, K));
   auto stream = at::hip::getCurrentHIPStream();
   auto launch = [&](auto kern) {
-    kern<<<grid, dim3(256), 0, stream>>>(
-        (bf16_t*)out.data_ptr(), (const bf16_t*)x.data_ptr(),
-        (const bf16_t*)w.data_ptr(), M, N, K, (int)rows, (int)cols);
+    kern<<<grid, dim3(256), 0, stream>>>(out, (const bf16_t*)x.data_ptr(), parts, M, K,
+                                         (int)rows, (int)cols);
   };
-  switch (best) {
-    case 3: launch(linear_kernel<3, GLU>); break;
-    case 4: launch(linear_kernel<4, GLU>); break;
-    case 5: launch(linear_kernel<5, GLU>); break;
-    case 6: launch(linear_kernel<6, GLU>); break;
-    case 7: launch(linear_kernel<7, GLU>); break;
-    default: launch(linear_kernel<8, GLU>);
+  if constexpr (KIND != KEPT) {
+    if (best == 3) launch(linear_kernel<3, KIND>);
+    if (best == 4) launch(linear_kernel<4, KIND>);
+    if (best == 5) launch(linear_kernel<5, KIND>);
   }
+  if (best == 6) launch(linear_kernel<6, KIND>);
+  if (best == 7) launch(linear_kernel<7, KIND>);
+  if (best == 8) launch(linear_kernel<8, KIND>);
   HIP_CHECK_KERNEL();
+}
+
+Part part(const torch::Tensor* out, const torch::Tensor& w, long first, long n) {
+  return {out ? (bf16_t*)out->data_ptr() : nullptr,
+          (const bf16_t*)w.data_ptr() + first * w.size(1), n};
 }
 
 template <bool GLU>
@@ -124,7 +173,11 @@ torch::Tensor linear_prompt(const torch::Tensor& x, const torch::Tensor& w) {
               "linear: inner numbers in 64s, the weight's rows in 256s, outputs "
               "below 2^25");
   auto out = torch::empty({M, N}, x.options());
-  launch_linear<GLU>(out, x, w);
+  if (GLU)
+    launch_linear<GATED>((bf16_t*)out.data_ptr(), x,
+                         {{part(nullptr, w, 0, N), part(nullptr, w, N, N)}}, N / 128);
+  else
+    launch_linear<PLAIN>(nullptr, x, {{part(&out, w, 0, N)}}, N / SIDE);
   return out;
 }
 
@@ -149,7 +202,8 @@ void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
                   out.size(1) == w.size(0) && linear_rows_fits(x, w) &&
                   ((uintptr_t)out.data_ptr() & 15) == 0,
               "linear: inner numbers in 64s, outputs in 8s, 16-byte addresses");
-  launch_linear<false>(out, x, w);
+  const long N = w.size(0);
+  launch_linear<PLAIN>(nullptr, x, {{part(&out, w, 0, N)}}, (N + SIDE - 1) / SIDE);
 }
 
 // Whether linear_rows is the better choice than the library's own: tiles that fill
@@ -174,4 +228,72 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w) {
 // x (M, K), w (2 N, K): rows of the gate, then of the up projection
 torch::Tensor linear_swiglu(torch::Tensor x, torch::Tensor w) {
   return linear_prompt<true>(x, w);
+}
+
+namespace {
+
+// of weights of one input: the operands' form, and whether the tiles fill their rounds
+bool joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws, long each) {
+  if (ws.size() < 2 || ws.size() > MOST || x.dim() != 2 || !x.is_cuda() ||
+      !x.is_contiguous() || x.dtype() != torch::kBFloat16)
+    return false;
+  long N = 0;
+  for (const auto& w : ws) {
+    if (!w.is_cuda() || w.device() != x.device() || w.dim() != 2 || !w.is_contiguous() ||
+        w.dtype() != torch::kBFloat16 || w.size(1) != x.size(1) ||
+        w.size(0) % each != 0 || !linear_rows_fits(x, w))
+      return false;
+    N += w.size(0);
+  }
+  const long M = x.size(0), K = x.size(1);
+  const double whole = (double)M * N / (CUS * SIDE * SIDE) * cost_of(8, K);
+  return M > 512 && N < (1L << 25) &&
+         rows_of(M, (N + SIDE - 1) / SIDE, K, 6).cost <= 1.35 * whole;
+}
+
+}  // namespace
+
+// Whether linear_joint has these operands (contiguous bf16 matrices, the weights' rows in
+// 256s) and is the better choice than a product each.  4096 -> 4096, 1024, 1024 of 7168
+// rows: 229 us for 158, 52 and 52.
+bool linear_joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws) {
+  return joint_takes(x, ws, SIDE);
+}
+
+// x W_p^T of two or three weights (N_p, K)
+std::vector<torch::Tensor> linear_joint(torch::Tensor x, std::vector<torch::Tensor> ws) {
+  TORCH_CHECK(joint_takes(x, ws, SIDE), "linear_joint: operands that it does not take");
+  std::vector<torch::Tensor> outs;
+  Parts parts = {};
+  long cols = 0;
+  for (size_t i = 0; i < ws.size(); ++i) {
+    outs.push_back(torch::empty({x.size(0), ws[i].size(0)}, x.options()));
+    parts.p[i] = part(&outs[i], ws[i], 0, ws[i].size(0));
+    cols += ws[i].size(0) / SIDE;
+  }
+  launch_linear<PLAIN>(nullptr, x, parts, cols);
+  return outs;
+}
+
+// The same for linear_gated: rows of weights in 128s, as many of both
+bool linear_gated_takes(const torch::Tensor& x, const torch::Tensor& wg,
+                        const torch::Tensor& wu) {
+  return wg.dim() == 2 && wu.dim() == 2 && wg.size(0) == wu.size(0) &&
+         joint_takes(x, {wg, wu}, 128);
+}
+
+// silu(gate) * up, and with keep gate = x Wg^T and up = x Wu^T behind it
+std::vector<torch::Tensor> linear_gated(torch::Tensor x, torch::Tensor wg,
+                                        torch::Tensor wu, bool keep) {
+  TORCH_CHECK(linear_gated_takes(x, wg, wu),
+              "linear_gated: operands that it does not take");
+  const long N = wg.size(0);
+  std::vector<torch::Tensor> outs;
+  for (int i = 0; i < (keep ? 3 : 1); ++i)
+    outs.push_back(torch::empty({x.size(0), N}, x.options()));
+  const Parts parts = {{part(keep ? &outs[1] : nullptr, wg, 0, N),
+                        part(keep ? &outs[2] : nullptr, wu, 0, N)}};
+  (keep ? launch_linear<KEPT> : launch_linear<GATED>)((bf16_t*)outs[0].data_ptr(), x,
+                                                      parts, N / 128);
+  return outs;
 }

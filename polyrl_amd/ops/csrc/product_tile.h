@@ -98,6 +98,21 @@ struct Operand {
 
   // ld: numbers of a memory row; half: which 128 of the outer numbers are the wave's
   DEV_INLINE Operand(const char* lds, long ld, int half) {
+    pitch(ld);
+    const int lane = threadIdx.x & 63;
+    const int lds0 = (int)(uintptr_t)(lds_p)lds, c = lane & 15, h = lane >> 4;
+#pragma unroll
+    for (int d = 0; d < FRAGS; ++d) {
+      if (LINES) {
+        frag_at[d] = lds0 + half * (P * 2048) + c * 128 + (place(4 * d + h, c) << 4);
+      } else {
+        const int r = 8 * h + (c >> 2);
+        frag_at[d] = lds0 + half * 256 + r * 512 + ((d ^ turn(r)) << 5) +
+                     (c & 3) * 8;
+      }
+    }
+  }
+  DEV_INLINE void pitch(long ld) {
     const unsigned ldb = (unsigned)ld * 2;
     step = LINES ? 2 * PAIR : PAIR * ldb;
     const int lane = threadIdx.x & 63, wid = wave_id();
@@ -109,17 +124,6 @@ struct Operand {
       } else {
         const int r = wid * 16 + i * 2 + (lane >> 5);
         load_at[i] = r * ldb + (((lane & 31) ^ (turn(r) << 1)) << 4);
-      }
-    }
-    const int lds0 = (int)(uintptr_t)(lds_p)lds, c = lane & 15, h = lane >> 4;
-#pragma unroll
-    for (int d = 0; d < FRAGS; ++d) {
-      if (LINES) {
-        frag_at[d] = lds0 + half * (P * 2048) + c * 128 + (place(4 * d + h, c) << 4);
-      } else {
-        const int r = 8 * h + (c >> 2);
-        frag_at[d] = lds0 + half * 256 + r * 512 + ((d ^ turn(r)) << 5) +
-                     (c & 3) * 8;
       }
     }
   }
@@ -209,48 +213,59 @@ struct Frag {
 // part j is column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 16 J x
 // 128 (row half wave % 2, column half wave / 2).  A tile that another one follows has
 // four units and more.
-template <bool LL, bool RL, int J = 8, typename UnitsOf, typename Finish>
-DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
+//
+// PARTS > 1: the sum of that many products, part p of tile t as number PARTS t + p, whose
+// left operand's rows may be of another length each (left_ld(part)).  Each starts anew,
+// which costs some 2 us.
+template <bool LL, bool RL, int J = 8, int PARTS = 1, typename LeftLd,
+          typename UnitsOf, typename Finish>
+DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
                     Finish finish) {
   const int wid = wave_id();
-  Operand<LL, J> a(lds, left_ld, wid & 1);
+  Operand<LL, J> a(lds, left_ld(0), wid & 1);
   Operand<RL> b(lds, right_ld, wid >> 1);
   // (of a unit a wave loads 1 KiB for each of its row parts)
   const unsigned to_a = (unsigned)(uintptr_t)(lds_p)lds + wid * (J * 1024);
   const unsigned to_b = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
   Units ua, ub;
-  int now = 0;
+  int now = 0, pairs = 0;
   bool more = units(0, ua, ub);
   if (!more) return;
-  a.follow(ua), b.follow(ub);
-  a.start(), b.start();
-  int pairs = ua.n;
   auto look_ahead = [&] {              // (behind the last tile nothing is read)
     more = units(now + 1, ua, ub);
-    if (!more) ua.bytes = ub.bytes = 0, ua.n = ub.n = 1 << 30;
+    if (!more || PARTS > 1) {
+      ua.bytes = ub.bytes = 0;
+      if (PARTS == 1) ua.n = ub.n = 1 << 30;
+    }
     a.follow(ua), b.follow(ub);
   };
-  look_ahead();
-  a.load(to_a), b.load(to_b + UNIT);
-  a.load(to_a + 2 * UNIT), b.load(to_b + 3 * UNIT);
-
   Acc<J> acc;
   Frag<LL> fa[2][J];
   Frag<RL> fb[2][8];
   int na[a.FRAGS], nb[b.FRAGS];        // where the next fragments are
-  arrived<J + 8>();
+  // the first units and fragments
+  auto begin = [&] {
+    a.follow(ua), b.follow(ub);
+    a.start(), b.start();
+    pairs = ua.n;
+    look_ahead();
+    a.load(to_a), b.load(to_b + UNIT);
+    a.load(to_a + 2 * UNIT), b.load(to_b + 3 * UNIT);
+    arrived<J + 8>();
 #pragma unroll
-  for (int d = 0; d < a.FRAGS; ++d) na[d] = a.frag_at[d];
+    for (int d = 0; d < a.FRAGS; ++d) na[d] = a.frag_at[d];
 #pragma unroll
-  for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + UNIT;
+    for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + UNIT;
 #pragma unroll
-  for (int d = 0; d < 8; ++d) {
-    if (d < J) {
-      fa[0][d < J ? d : 0].template read<0, 0>(na, d);
-      fa[0][d < J ? d : 0].template read<0, 1>(na, d);
+    for (int d = 0; d < 8; ++d) {
+      if (d < J) {
+        fa[0][d < J ? d : 0].template read<0, 0>(na, d);
+        fa[0][d < J ? d : 0].template read<0, 1>(na, d);
+      }
+      fb[0][d].template read<0, 0>(nb, d), fb[0][d].template read<0, 1>(nb, d);
     }
-    fb[0][d].template read<0, 0>(nb, d), fb[0][d].template read<0, 1>(nb, d);
-  }
+  };
+  begin();
 
   // The products of a step, whose fragments are registers N, the reads of the next one's,
   // and the loads of a unit to ``slot``.  (Loads behind the end read nothing: the
@@ -319,24 +334,37 @@ DEV_INLINE void run(char* lds, long left_ld, long right_ld, UnitsOf units,
   // slots: this pair's units, the next pair's, the left one behind that
   int s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
   for (;;) {
+    if (PARTS == 1 || now % PARTS == 0)
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int p = 0; p < pairs; ++p) {
       step(std::integral_constant<int, 0>(), a, to_a + s4, s2, s3);
       step(std::integral_constant<int, 1>(), b, to_b + s0, s2, s3);
       const int t0 = s0, t1 = s1;
       s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
     }
-    // (the compiler does not know that these are products, whose results take a while;
-    // they are read by sums_of())
-    asm volatile("s_nop 15\n\ts_nop 15");
-    finish(now, acc);
+    if (PARTS == 1 || now % PARTS == PARTS - 1) {
+      // (the compiler does not know that these are products, whose results take a
+      // while; they are read by sums_of())
+      asm volatile("s_nop 15\n\ts_nop 15");
+      finish(now / PARTS, acc);
+    }
     if (!more) break;
     ++now;
-    pairs = ua.n;
-    look_ahead();
+    if constexpr (PARTS == 1) {
+      pairs = ua.n;
+      look_ahead();
+    } else {
+      // (no load on its way, no wave at the last fragments)
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      arrived<0>();
+      a.pitch(left_ld(now % PARTS));
+      units(now, ua, ub);
+      s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
+      begin();
+    }
   }
   // (no load is on its way to LDS when the block ends)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -391,6 +419,26 @@ DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
     out[w] = q[0], out[2 + w] = q[1];
   }
   return out;
+}
+
+// A tile's sums from (row0, col0) on as rows of bf16 numbers; cols is in 8s
+template <int J>
+DEV_INLINE void store_tile(bf16_t* out, long rows, long cols, long row0, long col0,
+                           const Acc<J>& acc) {
+  const int lane = threadIdx.x & 63, wid = wave_id();
+  const long r0 = row0 + (wid & 1) * (16 * J) + (lane & 15);
+  const long c0 = col0 + (wid >> 1) * 128 + 8 * (lane >> 4);
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const long row = r0 + 16 * j;
+    order();
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const u32x4_t w = eight_columns(sums_of(acc[i][j]), sums_of(acc[i + 1][j]));
+      if (row < rows && c0 + 16 * i < cols)
+        *reinterpret_cast<u32x4_t*>(out + row * cols + c0 + 16 * i) = w;
+    }
+  }
 }
 
 // Rows of a tile whose left operand is LINES, in 32s from LEAST on (6 where the right one

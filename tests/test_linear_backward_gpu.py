@@ -126,3 +126,99 @@ def test_refused():
                   ((64, 64), (128, 16))):
         with pytest.raises(RuntimeError):
             ext.linear_dgrad(rand(*dy, 0), rand(*w, 0))
+
+
+@pytest.mark.parametrize("m", [1, 190, 449])
+@pytest.mark.parametrize("ns", [(64, 128), (256, 64, 320), (448, 64, 64),
+                                (512, 512)])
+def test_dgrad_sum(m, ns):
+    """Products of unequal inner dimensions, from one unit on, edges of tiles."""
+    dys = [rand(m, n, 3 + i) for i, n in enumerate(ns)]
+    ws = [rand(n, 520, 13 + i) for i, n in enumerate(ns)]
+    got = ops._require_ext().linear_dgrad_sum(dys, ws)
+    check(torch.cat(dys, 1), torch.cat(ws), got)
+
+
+@pytest.mark.parametrize("m", [1500, 1791, 1799, 2041, 4700])
+def test_dgrad_sum_rows(m):
+    """Tiles of 192, 224 and 256 rows; blocks with a second tile and third."""
+    dys, ws = [rand(m, 192, 3), rand(m, 64, 4)], [rand(192, 8184, 5), rand(64, 8184, 6)]
+    got = ops._require_ext().linear_dgrad_sum(dys, ws)
+    check(torch.cat(dys, 1), torch.cat(ws), got)
+
+
+def test_dgrad_sum_refused():
+    ext = ops._require_ext()
+    dy, w = rand(64, 64, 1), rand(64, 128, 2)
+    for dys, ws in (([dy], [w]), ([dy, dy], [w]), ([dy] * 4, [w] * 4),
+                    ([dy, dy[:32]], [w, w]), ([dy, dy], [w, rand(64, 136, 3)]),
+                    ([dy, rand(64, 72, 1)], [w, rand(72, 128, 2)])):
+        with pytest.raises(RuntimeError):
+            ext.linear_dgrad_sum(dys, ws)
+        assert len(dys) == len(ws) == 2 or not ext.linear_dgrad_sum_takes(dys, ws)
+
+
+@pytest.mark.parametrize("m,ns,k", [(760, (8192, 7936, 256), 128),
+                                    (1700, (6144, 2048), 192),
+                                    (4400, (2048, 512, 512), 256)])
+def test_joint_linear(m, ns, k):
+    """Forward and gradients of layers of one input, against each layer's own."""
+    mods = [torch.nn.Linear(k, n, bias=i == 1, device=DEV, dtype=torch.bfloat16)
+            for i, n in enumerate(ns)]
+    x = rand(m, k, 5).requires_grad_()
+    ys = ops.joint_linear(x, mods)
+    assert ys is not None
+    dys = [rand(m, n, 7 + i) for i, n in enumerate(ns)]
+    torch.autograd.backward(ys, dys)
+    for y, dy, mod in zip(ys, dys, mods):
+        want = x.detach().double() @ mod.weight.detach().double().t()
+        if mod.bias is None:
+            check(x.detach(), mod.weight.detach().t(), y.detach())
+        else:
+            want += mod.bias.detach().double()
+            assert (y - want).norm() <= 5e-3 * want.norm()
+            assert (mod.bias.grad - dy.sum(0)).norm() <= 1e-2 * dy.sum(0).norm()
+        check(dy.t(), x.detach(), mod.weight.grad)
+    want = sum(dy.double() @ m.weight.detach().double() for dy, m in zip(dys, mods))
+    assert (x.grad - want).norm() <= 5e-3 * want.norm()
+
+
+@pytest.mark.parametrize("m,n,k", [(760, 8192, 128), (1700, 4096, 192),
+                                   (2041, 4096, 320), (4400, 1664, 256)])
+def test_gated_linear(m, n, k):
+    """Gate, up and activation of one kernel with their gradients, and without
+    what is kept for them."""
+    gate, up = (torch.nn.Linear(k, n, bias=False, device=DEV, dtype=torch.bfloat16)
+                for _ in range(2))
+    x = rand(m, k, 5).requires_grad_()
+    y = ops.gated_linear(x, gate, up)
+    with torch.no_grad():
+        assert torch.equal(ops.gated_linear(x, gate, up), y)
+    dy = rand(m, n, 7)
+    y.backward(dy)
+    xd = x.detach().double().requires_grad_()
+    wd = [l.weight.detach().double().requires_grad_() for l in (gate, up)]
+    want = torch.nn.functional.silu(xd @ wd[0].t()) * (xd @ wd[1].t())
+    want.backward(dy.double())
+    for got, exact in ((y, want), (x.grad, xd.grad), (gate.weight.grad, wd[0].grad),
+                       (up.weight.grad, wd[1].grad)):
+        # (roundings to bf16 of the products, their gradients and the result)
+        assert (got - exact).norm() <= 1e-2 * exact.norm()
+
+
+def test_joint_other_layers():
+    """Who is not a plain layer of bf16 weights has its own forward."""
+    class Other(torch.nn.Linear):
+        pass
+
+    def lin(cls=torch.nn.Linear, k=128, bias=False, **kw):
+        return cls(k, 8192, bias=bias, device=DEV, **{"dtype": torch.bfloat16, **kw})
+
+    x = rand(760, 128, 1)
+    assert ops.joint_linear(x, (lin(), lin())) is not None
+    for bad in (lin(Other), lin(dtype=torch.float32)):
+        assert ops.joint_linear(x, (lin(), bad)) is None
+        assert ops.gated_linear(x, lin(), bad) is None
+    assert ops.gated_linear(x, lin(), lin(bias=True)) is None
+    assert ops.joint_linear(x[:500], (lin(), lin())) is None
+    assert ops.joint_linear(x.cpu(), (lin(), lin())) is None
