@@ -25,9 +25,39 @@ namespace {
 
 using namespace product;
 
+// A tile's outputs, or where blocks share its inner numbers its fp32 sums, which are added
+// up afterwards: (tiles, ways, SIDE * SIDE)
+template <int J>
+struct Outputs : TileRows<J> {
+  bf16_t* const out;
+  float* const shares;
+  const long R, C;
+  f32x4_t* to_share;
+  DEV_INLINE Outputs(bf16_t* out_, float* shares_, long R_, long C_)
+      : out(out_), shares(shares_), R(R_), C(C_) {}
+  DEV_INLINE void tile(const Place& at) {
+    if (J == 8 && shares != nullptr)
+      to_share = reinterpret_cast<f32x4_t*>(shares + (long)at.share * SIDE * SIDE) +
+                 wave_id() * 4096 + (threadIdx.x & 63);
+    else
+      this->start(out, R, C, at, (long)at.col * SIDE);
+  }
+  DEV_INLINE void rows(int) {
+    if (J < 8 || shares == nullptr) this->to.next();
+  }
+  // (a share's block has no other tile: nothing counts these stores)
+  DEV_INLINE void put(int j, int q, const f32x4_t (&sums)[2]) const {
+    if (J == 8 && shares != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) to_share[((2 * q + e) * 8 + j) * 64] = sums[e];
+    } else {
+      TileRows<J>::put(j, q, sums);
+    }
+  }
+};
+
 // out (R, C): sums over inner of left(row, inner) right(inner, column), right in
-// COLUMNS.  ``ways`` blocks share a tile's inner numbers, whose fp32 sums (tiles, ways,
-// SIDE * SIDE) are added up afterwards.  LINES: tiles of 32 J rows.
+// COLUMNS.  ``ways`` blocks share a tile's inner numbers.  LINES: tiles of 32 J rows.
 template <bool LINES, int J>
 __global__ __launch_bounds__(256, 1) void product_kernel(
     bf16_t* __restrict__ out, float* __restrict__ shares,
@@ -37,11 +67,11 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
   constexpr int ROWS = 32 * J;
   const int tiles = row_tiles * col_tiles, items = tiles * ways;
   const int all = (int)((inner + PAIR - 1) / PAIR);
-  auto units = [&](int r, Units& a, Units& b) {
+  auto units = [&](int r, Units& a, Units& b, Place& at) {
     const int item = item_of(r, items, gridDim.x);
     if (item < 0) return false;
-    const int part = item / tiles;
-    const Place at(item - part * tiles, row_tiles, col_tiles);
+    const int part = item / tiles, tile = item - part * tiles;
+    at = Place(tile, row_tiles, col_tiles, tile * ways + part);
     const int p0 = (int)((long)all * part / ways);
     const int n = (int)((long)all * (part + 1) / ways) - p0;
     const long r0 = (long)at.row * ROWS, c0 = (long)at.col * SIDE;
@@ -50,25 +80,9 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
     b = columns(right, C, inner, c0, i0, n);
     return true;
   };
-  auto finish = [&](int r, Acc<J>& acc) {
-    const int lane = threadIdx.x & 63, wid = wave_id();
-    const int item = item_of(r, items, gridDim.x), part = item / tiles;
-    const int tile = item - part * tiles;
-    if (J == 8 && ways > 1) {
-      f32x4_t* p = reinterpret_cast<f32x4_t*>(
-                       shares + ((long)tile * ways + part) * SIDE * SIDE) +
-                   wid * 4096 + lane;
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < J; ++j) p[(i * 8 + j) * 64] = sums_of(acc[i][j]);
-      return;
-    }
-    const Place at(tile, row_tiles, col_tiles);
-    store_tile<J>(out, R, C, (long)at.row * ROWS, (long)at.col * SIDE, acc);
-  };
+  Outputs<J> outputs(out, shares, R, C);
   run<LINES, false, J>(
-      lds, [&](int) { return LINES ? inner : R; }, C, units, finish);
+      lds, [&](int) { return LINES ? inner : R; }, C, units, outputs);
 }
 
 // out (R, C): the sum of left_p(row, inner) right_p(inner, column) over the parts, the
@@ -90,10 +104,10 @@ __global__ __launch_bounds__(256, 1) void parts_kernel(
   auto inner_of = [&](int p) {
     return p == 0 ? parts.inner[0] : p == 1 ? parts.inner[1] : parts.inner[2];
   };
-  auto units = [&](int r, Units& a, Units& b) {
+  auto units = [&](int r, Units& a, Units& b, Place& at) {
     const int item = item_of(r / PARTS, items, gridDim.x), p = r % PARTS;
     if (item < 0) return false;
-    const Place at(item, row_tiles, col_tiles);
+    at = Place(item, row_tiles, col_tiles);
     const bf16_t* left = p == 0 ? parts.left[0] : p == 1 ? parts.left[1] : parts.left[2];
     const bf16_t* right =
         p == 0 ? parts.right[0] : p == 1 ? parts.right[1] : parts.right[2];
@@ -102,11 +116,8 @@ __global__ __launch_bounds__(256, 1) void parts_kernel(
     b = columns(right, C, inner, (long)at.col * SIDE, 0, (int)(inner / PAIR));
     return true;
   };
-  auto finish = [&](int t, Acc<J>& acc) {
-    const Place at(item_of(t, items, gridDim.x), row_tiles, col_tiles);
-    store_tile<J>(out, R, C, (long)at.row * (32 * J), (long)at.col * SIDE, acc);
-  };
-  run<true, false, J, PARTS>(lds, inner_of, C, units, finish);
+  Outputs<J> outputs(out, nullptr, R, C);
+  run<true, false, J, PARTS>(lds, inner_of, C, units, outputs);
 }
 
 // Sums of the shares: a wave takes 16 rows of 32 outputs

@@ -21,7 +21,11 @@
 // 1024 -> 4096 of 513, 1024, 5135 and 8192 rows 15.0, 18.5, 74.0, 113 for 15.8, 20.1, 86.9,
 // 128 and 23.8, 28.2, 103, 149; 2048 -> 8192 34.1, 51.8, 256, 391 for 39.0, 60.8, 310, 461
 // and 44.7, 69.0, 316, 472; 4096 -> 14336 117, 183, 868, 1301 for 136, 210, 1035, 1544 and
-// 131, 207, 996, 1408.
+// 131, 207, 996, 1408.  Since then a tile's sums are taken out beside the next one's
+// products and outputs go past the L2s: 1024 -> 4096 of 5135 and 8192 rows 70.3, 105 ->
+// 66.7, 101 (on another card), 1024 -> 1536 and 1024 of 5135 19.0, 15.2 -> 17.0, 14.0.  What
+// is left above the products' own time in 1024 -> 4096 of 7168 rows, one tile a block: the
+// stores 2 us and the activation 1 of 26.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -43,9 +47,84 @@ struct Parts {
   Part p[MOST];
 };
 
+// part of a column of the products together, and which of its columns
+DEV_INLINE Part part_of(const Parts& parts, long& col) {
+  Part p = parts.p[0];
+  if (col >= p.n) {
+    col -= p.n, p = parts.p[1];
+    if (col >= p.n) col -= p.n, p = parts.p[2];
+  }
+  return p;
+}
+
 // PLAIN: the products.  GATED: out = silu(gate) * up of the products with p[0], gate, and
 // p[1], up.  KEPT: the products too.
 enum Kind { PLAIN, GATED, KEPT };
+
+// Where a tile's outputs go
+template <int J, Kind KIND>
+struct Outputs;
+
+template <int J>
+struct Outputs<J, PLAIN> : TileRows<J> {
+  const Parts& parts;
+  const long M;
+  DEV_INLINE Outputs(bf16_t*, const Parts& parts_, long M_) : parts(parts_), M(M_) {}
+  DEV_INLINE void tile(const Place& at) {
+    long col = (long)at.col * SIDE;
+    const Part p = part_of(parts, col);
+    this->start(p.out, M, p.n, at, col);
+  }
+};
+
+// Gate's and up projection's column parts are four apart
+template <int J, Kind KIND>
+struct Outputs {
+  static constexpr int COLS = 4, STORES = KIND == KEPT ? 6 : 2;
+  static constexpr int column_of(int q, int e) { return 2 * q + (e & 1) + 4 * (e >> 1); }
+  bf16_t* const out;
+  const Parts& parts;
+  const long M;
+  OutRows to, gate, up;
+  unsigned offset[2];
+  DEV_INLINE Outputs(bf16_t* out_, const Parts& parts_, long M_)
+      : out(out_), parts(parts_), M(M_) {}
+  DEV_INLINE void tile(const Place& at) {
+    const int lane = threadIdx.x & 63, wid = wave_id();
+    const long N = parts.p[0].n;
+    const long row0 = (long)at.row * (32 * J) + (wid & 1) * (16 * J);
+    to.start(out, M, N, row0);
+    if (KIND == KEPT)
+      gate.start(parts.p[0].out, M, N, row0), up.start(parts.p[1].out, M, N, row0);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      offset[q] = OutRows::offset(
+          N, (long)at.col * 128 + (wid >> 1) * 64 + 32 * q + 8 * (lane >> 4));
+  }
+  DEV_INLINE void rows(int) {
+    to.next();
+    if (KIND == KEPT) gate.next(), up.next();
+  }
+  DEV_INLINE void put(int, int q, const f32x4_t (&sums)[4]) const {
+    f32x4_t y[2];
+    // (the activation first: gate times up may be beyond 32 bits where the sigmoid is 0)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[h][e] = sums[h][e] *
+                  __builtin_amdgcn_rcpf(1.f +
+                                        exp2_hw(sums[h][e] * -1.4426950408889634f)) *
+                  sums[2 + h][e];
+    // (a choice at each store costs the prompts' tiles 1.2 us of 67 together; 16384 rows,
+    // 2048 -> 8192, 268 MB, 754 us through the L2s and 726 past them)
+    to.put(offset[q], eight_columns(y[0], y[1]), KIND == GATED);
+    if (KIND == KEPT) {
+      gate.put(offset[q], eight_columns(sums[0], sums[1]), false);
+      up.put(offset[q], eight_columns(sums[2], sums[3]), false);
+    }
+  }
+};
 
 template <int J, Kind KIND>
 __global__ __launch_bounds__(256, 1) void linear_kernel(
@@ -56,19 +135,10 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
   constexpr int ROWS = 32 * J, COLS = KIND == PLAIN ? 256 : 128;
   const int items = row_tiles * col_tiles, n = (int)(K / PAIR);
   const long N = parts.p[0].n;
-  // part of a tile of columns, and which column of it
-  auto part_of = [&](long& col) {
-    Part p = parts.p[0];
-    if (col >= p.n) {
-      col -= p.n, p = parts.p[1];
-      if (col >= p.n) col -= p.n, p = parts.p[2];
-    }
-    return p;
-  };
-  auto units = [&](int r, Units& a, Units& b) {
+  auto units = [&](int r, Units& a, Units& b, Place& at) {
     const int item = item_of(r, items, gridDim.x);
     if (item < 0) return false;
-    const Place at(item, row_tiles, col_tiles);
+    at = Place(item, row_tiles, col_tiles);
     a = lines(x, M, K, (long)at.row * ROWS, 0, n);
     long col = (long)at.col * COLS;
     if (KIND != PLAIN) {
@@ -77,56 +147,13 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
       b = lines(wid & 1 ? parts.p[1].w : parts.p[0].w, N, K,
                 col + (wid >> 1) * 64 - wid * 64, 0, n);
     } else {
-      const Part p = part_of(col);
+      const Part p = part_of(parts, col);
       b = lines(p.w, p.n, K, col, 0, n);
     }
     return true;
   };
-  auto finish = [&](int r, Acc<J>& acc) {
-    const int lane = threadIdx.x & 63, wid = wave_id();
-    const Place at(item_of(r, items, gridDim.x), row_tiles, col_tiles);
-    if (KIND == PLAIN) {
-      long col = (long)at.col * COLS;
-      const Part p = part_of(col);
-      store_tile<J>(p.out, M, p.n, (long)at.row * ROWS, col, acc);
-      return;
-    }
-    const long r0 = (long)at.row * ROWS + (wid & 1) * (16 * J) + (lane & 15);
-    const long c0 = (long)at.col * COLS + (wid >> 1) * (COLS / 2) + 8 * (lane >> 4);
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const long row = r0 + 16 * j;
-      order();
-#pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        f32x4_t g[2], u[2], y[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          g[h] = sums_of(acc[i + h][j]);
-          u[h] = sums_of(acc[i + h + 4][j]);
-          // (the activation first: gate times up may be beyond 32 bits where the
-          // sigmoid is 0)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            y[h][e] = g[h][e] *
-                      __builtin_amdgcn_rcpf(
-                          1.f + exp2_hw(g[h][e] * -1.4426950408889634f)) *
-                      u[h][e];
-        }
-        const u32x4_t v = eight_columns(y[0], y[1]);
-        const long at_out = row * N + c0 + 16 * i;
-        if (row < M) *reinterpret_cast<u32x4_t*>(out + at_out) = v;
-        if (KIND == KEPT) {
-          const u32x4_t gv = eight_columns(g[0], g[1]), uv = eight_columns(u[0], u[1]);
-          if (row < M) {
-            *reinterpret_cast<u32x4_t*>(parts.p[0].out + at_out) = gv;
-            *reinterpret_cast<u32x4_t*>(parts.p[1].out + at_out) = uv;
-          }
-        }
-      }
-    }
-  };
-  run<true, true, J>(lds, [&](int) { return K; }, K, units, finish);
+  Outputs<J, KIND> outputs(out, parts, M);
+  run<true, true, J>(lds, [&](int) { return K; }, K, units, outputs);
 }
 
 // cols: tiles of columns of the weights together

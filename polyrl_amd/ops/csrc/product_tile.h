@@ -17,7 +17,9 @@
 // cycles each, stands at most one of the next step's fragment reads, of the unit's
 // loads, of the words that say where a load goes, or of the next addresses, a fragment
 // to three products (two: 3% slower, 582 for 566 us at 7168 x 14336 x 4096).  A block's
-// tiles are one stream of units: at a tile's end the next one's first are there.
+// tiles are one stream of units: at a tile's end the next one's first are there, and its
+// sums are read, rounded and stored between the products of the next one's first step,
+// which start from 0 instead of from a cleared accumulator.
 #pragma once
 
 #include <utility>
@@ -208,19 +210,36 @@ struct Frag {
   }
 };
 
-// Tiles r = 0, 1, ..: units(r, left, right) says where tile r's operands are, false
-// behind the last one; finish(r, acc) takes its sums: accumulator e of column part i, row
-// part j is column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 16 J x
-// 128 (row half wave % 2, column half wave / 2).  A tile that another one follows has
-// four units and more.
+// Row and column of a tile: GROUP rows of tiles, one column after the other, so that
+// the blocks that run on a die at once share 8 x 4 tiles' operands
+struct Place {
+  int row, col, share;                 // (share: of the tile's inner numbers)
+  DEV_INLINE Place() {}
+  DEV_INLINE Place(int tile, int row_tiles, int col_tiles, int share_ = 0)
+      : share(share_) {
+    const int group = tile / (GROUP * col_tiles);
+    const int rest = tile - group * GROUP * col_tiles;
+    const int high = min(GROUP, row_tiles - group * GROUP);
+    row = uniform(group * GROUP + rest % high), col = uniform(rest / high);
+  }
+};
+
+// Tiles r = 0, 1, ..: units(r, left, right, place) says where tile r and its operands
+// are, false behind the last one.  Its sums go to ``sink``: sink.tile(place), then for each
+// row part j sink.rows(j), and sink.put(j, q, sums) of each of its groups of COLS column
+// parts, columns_of(q, e) for e = 0, 1, ..  Accumulator e of column part i, row part j is
+// column 16 i + 4 (lane / 16) + e of row 16 j + lane % 16 of the wave's 16 J x 128 (row half
+// wave % 2, column half wave / 2).  A row part is STORES stores in every wave, whatever of
+// it is within the matrix: the waits count them.  A tile that another one follows has four
+// units and more.
 //
 // PARTS > 1: the sum of that many products, part p of tile t as number PARTS t + p, whose
 // left operand's rows may be of another length each (left_ld(part)).  Each starts anew,
 // which costs some 2 us.
 template <bool LL, bool RL, int J = 8, int PARTS = 1, typename LeftLd,
-          typename UnitsOf, typename Finish>
+          typename UnitsOf, typename Sink>
 DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
-                    Finish finish) {
+                    Sink& sink) {
   const int wid = wave_id();
   Operand<LL, J> a(lds, left_ld(0), wid & 1);
   Operand<RL> b(lds, right_ld, wid >> 1);
@@ -228,11 +247,12 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
   const unsigned to_a = (unsigned)(uintptr_t)(lds_p)lds + wid * (J * 1024);
   const unsigned to_b = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
   Units ua, ub;
+  Place last, here, next;              // the tiles behind, at and ahead of this step
   int now = 0, pairs = 0;
-  bool more = units(0, ua, ub);
+  bool more = units(0, ua, ub, here);
   if (!more) return;
   auto look_ahead = [&] {              // (behind the last tile nothing is read)
-    more = units(now + 1, ua, ub);
+    more = units(now + 1, ua, ub, next);
     if (!more || PARTS > 1) {
       ua.bytes = ub.bytes = 0;
       if (PARTS == 1) ua.n = ub.n = 1 << 30;
@@ -267,11 +287,16 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
   };
   begin();
 
+  constexpr int COLS = Sink::COLS, GROUPS = 8 / COLS;
   // The products of a step, whose fragments are registers N, the reads of the next one's,
   // and the loads of a unit to ``slot``.  (Loads behind the end read nothing: the
-  // count of them is the same in every step.)
-  auto step = [&](auto n_, auto& load, unsigned slot, int a_next, int b_next) {
+  // count of them is the same in every step.)  ENDS: the first pair of steps of a tile,
+  // which take the last one's sums out of the accumulators and start them anew; columns
+  // go fastest there, as the sink has them.
+  auto step = [&](auto n_, auto ends_, auto& load, unsigned slot, int a_next,
+                  int b_next) {
     constexpr int N = decltype(n_)::value, O = 1 - N;
+    constexpr bool ENDS = decltype(ends_)::value;
     constexpr int FRAGS = 8 + J, LOADS = N == 0 ? J : 8, ALL = 8 * J;
     // instructions of a fragment (and a load's two, or with the load's first; few row
     // parts leave room for two)
@@ -279,16 +304,33 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
     static_assert(PER == 2 ? LOADS <= FRAGS : 2 * LOADS <= FRAGS + 2, "the order");
     static_assert(PER * FRAGS + 2 <= ALL, "the order");
     __builtin_amdgcn_s_waitcnt(0xc07f);            // fragments: lgkmcnt(0)
-    // The next unit of both is there, and this one's, read to the end, make room
-    if constexpr (N == 1) arrived<J>();
+    // The next unit of both is there, and this one's, read to the end, make room.  (The
+    // last tile's stores are as young as this step's loads, and still on their way.)
+    if constexpr (N == 1)
+      arrived<ENDS ? std::min(63, J + J * Sink::STORES) : J>();
+    constexpr bool FIRST = ENDS && N == 0;
+    f32x4_t sums[COLS];
     each(std::make_integer_sequence<int, ALL>(), [&](auto k_) {
       constexpr int k = decltype(k_)::value;
-      constexpr int i = k / J, j = i & 1 ? J - 1 - k % J : k % J;
+      constexpr int q = k / COLS % GROUPS, e = k % COLS;
+      constexpr int i = FIRST ? Sink::column_of(q, e) : k / J;
+      constexpr int j = FIRST ? k / 8 : i & 1 ? J - 1 - k % J : k % J;
       order();
       // (in assembly, else the compiler moves accumulators about)
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[i][j])
-                   : "v"(fb[N][i].whole()), "v"(fa[N][j].whole()));
+      if constexpr (FIRST) {
+        if constexpr (k % 8 == 0) sink.rows(j);
+        sums[e] = sums_of(acc[i][j]);
+        order();
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
+                     : "+a"(acc[i][j])
+                     : "v"(fb[N][i].whole()), "v"(fa[N][j].whole()));
+        order();
+        if constexpr (e == COLS - 1) sink.put(j, q, sums);
+      } else {
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                     : "+a"(acc[i][j])
+                     : "v"(fb[N][i].whole()), "v"(fa[N][j].whole()));
+      }
       order();
       constexpr int f = k / PER;       // fragment: one column's, all rows', the rest
       if constexpr (f < FRAGS) {
@@ -333,26 +375,43 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
 
   // slots: this pair's units, the next pair's, the left one behind that
   int s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
+  auto pair = [&](auto ends) {
+    step(std::integral_constant<int, 0>(), ends, a, to_a + s4, s2, s3);
+    step(std::integral_constant<int, 1>(), ends, b, to_b + s0, s2, s3);
+    const int t0 = s0, t1 = s1;
+    s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
+  };
   for (;;) {
-    if (PARTS == 1 || now % PARTS == 0)
+    int p = 0;
+    if (PARTS == 1 && now > 0) {
+      sink.tile(last);
+      pair(std::true_type());
+      p = 1;
+    } else if (PARTS == 1 || now % PARTS == 0) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int p = 0; p < pairs; ++p) {
-      step(std::integral_constant<int, 0>(), a, to_a + s4, s2, s3);
-      step(std::integral_constant<int, 1>(), b, to_b + s0, s2, s3);
-      const int t0 = s0, t1 = s1;
-      s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
     }
-    if (PARTS == 1 || now % PARTS == PARTS - 1) {
+    for (; p < pairs; ++p) pair(std::false_type());
+    if (!more || (PARTS > 1 && now % PARTS == PARTS - 1)) {
       // (the compiler does not know that these are products, whose results take a
       // while; they are read by sums_of())
       asm volatile("s_nop 15\n\ts_nop 15");
-      finish(now / PARTS, acc);
+      sink.tile(here);
+      each(std::make_integer_sequence<int, J * GROUPS>(), [&](auto g_) {
+        constexpr int j = decltype(g_)::value / GROUPS, q = decltype(g_)::value % GROUPS;
+        order();
+        if constexpr (q == 0) sink.rows(j);
+        f32x4_t sums[COLS];
+#pragma unroll
+        for (int e = 0; e < COLS; ++e) sums[e] = sums_of(acc[Sink::column_of(q, e)][j]);
+        sink.put(j, q, sums);
+      });
     }
     if (!more) break;
     ++now;
+    last = here, here = next;
     if constexpr (PARTS == 1) {
       pairs = ua.n;
       look_ahead();
@@ -361,7 +420,7 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
       __builtin_amdgcn_s_waitcnt(0xc07f);
       arrived<0>();
       a.pitch(left_ld(now % PARTS));
-      units(now, ua, ub);
+      units(now, ua, ub, here);
       s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
       begin();
     }
@@ -369,18 +428,6 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
   // (no load is on its way to LDS when the block ends)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
-
-// Row and column of a tile: GROUP rows of tiles, one column after the other, so that
-// the blocks that run on a die at once share 8 x 4 tiles' operands
-struct Place {
-  int row, col;
-  DEV_INLINE Place(int tile, int row_tiles, int col_tiles) {
-    const int group = tile / (GROUP * col_tiles);
-    const int rest = tile - group * GROUP * col_tiles;
-    const int high = min(GROUP, row_tiles - group * GROUP);
-    row = uniform(group * GROUP + rest % high), col = uniform(rest / high);
-  }
-};
 
 // Item r of this block: blocks go to the dies in turn, each die takes one stretch of
 // the items, its blocks every ``blocks / dies``-th of it; -1 behind the last
@@ -421,25 +468,65 @@ DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
   return out;
 }
 
-// A tile's sums from (row0, col0) on as rows of bf16 numbers; cols is in 8s
-template <int J>
-DEV_INLINE void store_tile(bf16_t* out, long rows, long cols, long row0, long col0,
-                           const Acc<J>& acc) {
-  const int lane = threadIdx.x & 63, wid = wave_id();
-  const long r0 = row0 + (wid & 1) * (16 * J) + (lane & 15);
-  const long c0 = col0 + (wid >> 1) * 128 + 8 * (lane >> 4);
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const long row = r0 + 16 * j;
-    order();
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const u32x4_t w = eight_columns(sums_of(acc[i][j]), sums_of(acc[i + 1][j]));
-      if (row < rows && c0 + 16 * i < cols)
-        *reinterpret_cast<u32x4_t*>(out + row * cols + c0 + 16 * i) = w;
-    }
+// Rows of a matrix (rows, cols), cols in 8s, from a wave's first one on, 16 at a time, as a
+// buffer: what would be behind the last row is not written, nor are columns behind the last
+// one, whose offsets are behind every buffer's end.  In every wave each store is an
+// instruction that is counted.
+//
+// Outputs that the 256 MB cache behind the L2s holds go straight there (``past``), so that
+// nothing is left in the L2s when the kernel ends, or drives operands out of them (us,
+// through the L2s and past them: 5135 rows, 1024 -> 1536 18.2 and 16.3, 1024 -> 1024 15.0
+// and 13.8; gate, up and activation of 1024 -> 4096 68.6 and 66.9, of 8192 rows 103.5 and
+// 101.0; 8192 rows, 4096 -> 16384 736 and 696; input gradients of 7168 x 14336 571 and 537);
+// more than that passes through them (4096 rows, 4096 -> 128256 2816 and 2992; the trainer's
+// gate, up and activation of 7168 x 14336 each 1166 and 1288).
+constexpr long CACHED_OUT = 256L << 20;
+struct OutRows {
+  char* at;
+  long left, pitch;                    // bytes: to the matrix's end, of 16 rows
+  __amdgpu_buffer_rsrc_t buffer;
+  DEV_INLINE void start(bf16_t* out, long rows, long cols, long row0) {
+    pitch = 32 * cols, at = (char*)(out + row0 * cols) - pitch;
+    left = 2 * cols * (rows - row0) + pitch;
   }
-}
+  DEV_INLINE void next() {
+    at += pitch, left -= pitch;
+    buffer = __builtin_amdgcn_make_buffer_rsrc(
+        at, 0, (int)max(0L, min(left, 0x7fffffffL)), 0x00020000);
+  }
+  // this lane's 8 columns from col on of row lane % 16
+  DEV_INLINE static unsigned offset(long cols, long col) {
+    return col < cols ? (unsigned)((threadIdx.x & 15) * cols + col) * 2 : 0x80000000u;
+  }
+  DEV_INLINE void put(unsigned offset, const u32x4_t& w, bool past) const {
+    constexpr int PAST = 18;           // (sc1 and nt)
+    if (past) __builtin_amdgcn_raw_buffer_store_b128(w, buffer, offset, 0, PAST);
+    else __builtin_amdgcn_raw_buffer_store_b128(w, buffer, offset, 0, 0);
+  }
+};
+
+// A tile's sums as rows of bf16 numbers
+template <int J>
+struct TileRows {
+  static constexpr int COLS = 2, STORES = 4;
+  static constexpr int column_of(int q, int e) { return 2 * q + e; }
+  OutRows to;
+  unsigned offset[4];
+  bool past;
+  DEV_INLINE void start(bf16_t* out, long rows, long cols, const Place& at, long col0) {
+    const int lane = threadIdx.x & 63, wid = wave_id();
+    to.start(out, rows, cols, (long)at.row * (32 * J) + (wid & 1) * (16 * J));
+    past = 2 * rows * cols <= CACHED_OUT;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      offset[q] = OutRows::offset(
+          cols, col0 + (wid >> 1) * 128 + 32 * q + 8 * (lane >> 4));
+  }
+  DEV_INLINE void rows(int) { to.next(); }
+  DEV_INLINE void put(int, int q, const f32x4_t (&sums)[2]) const {
+    to.put(offset[q], eight_columns(sums[0], sums[1]), past);
+  }
+};
 
 // Rows of a tile whose left operand is LINES, in 32s from LEAST on (6 where the right one
 // is COLUMNS): as many as end the last round of 256 tiles earliest.  A unit of 64 inner

@@ -215,3 +215,51 @@ def test_engine_wide_prompts(m, n, k, rows, monkeypatch):
     want = x.float() @ w.float().t()
     assert (_mm_nt(x, w).float() - want).norm() / want.norm() <= 5e-3
     assert bool(ran) == rows
+
+
+@pytest.mark.parametrize("parts,m", [(3, 93), (4, 125), (5, 157), (6, 189),
+                                     (7, 445), (8, 253)])
+@pytest.mark.parametrize("k", [256, 320, 384])
+def test_sums_beside_the_next_tile(parts, m, k):
+    """Two tiles and three a block, of every number of row parts: a tile's sums
+    leave the accumulators while the next one's first step fills them.  Rows and
+    columns short of a tile; what stands behind the outputs is not touched."""
+    cols = 300
+    n = 256 * cols - 8
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    w = torch.randn(n, k, device=DEV).bfloat16()
+    flat = torch.full((m * n + 65536,), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops._require_ext().linear_rows_into(flat[:m * n].view(m, n), x, w)
+    check_rows(x, w, flat[:m * n].view(m, n))
+    assert (flat[m * n:] == 7).all()
+    half = 128 * cols
+    wg, wu = w[:half] / k ** 0.5, torch.randn(half, k, device=DEV).bfloat16()
+    got = ops.linear_swiglu(x, torch.cat([wg, wu]))
+    for at in range(0, half, 128 * 64):
+        a = slice(at, min(half, at + 128 * 64))
+        assert torch.equal(got[:, a], ops.linear_swiglu(
+            x, torch.cat([wg[a], wu[a]])))
+
+
+@pytest.mark.parametrize("m", [1149, 1300, 1530, 1785])
+def test_kept_beside_the_next_tile(m):
+    """The same where gate and up projection are kept."""
+    x = torch.randn(m, 320, device=DEV).bfloat16()
+    wg, wu = (torch.randn(10240, 320, device=DEV).bfloat16() for _ in range(2))
+    y, gate, up = ops._require_ext().linear_gated(x, wg, wu, True)
+    check_rows(x, wg, gate)
+    check_rows(x, wu, up)
+    assert torch.equal(y, ops.linear_swiglu(x, torch.cat([wg, wu])))
+
+
+def test_outputs_beyond_the_cache():
+    """More outputs than go past the L2s: the same as in pieces that do."""
+    x = torch.randn(1100, 256, device=DEV).bfloat16()
+    w = torch.randn(128264, 256, device=DEV).bfloat16()
+    op = ops._require_ext().linear_rows_into
+
+    def rows(w):
+        out = x.new_empty(x.shape[0], w.shape[0])
+        op(out, x, w)
+        return out
+    assert torch.equal(rows(w), torch.cat([rows(w[:64136]), rows(w[64136:])], 1))
