@@ -473,14 +473,17 @@ DEV_INLINE u32x4_t eight_columns(const f32x4_t& c0, const f32x4_t& c1) {
 // one, whose offsets are behind every buffer's end.  In every wave each store is an
 // instruction that is counted.
 //
-// Outputs that the 256 MB cache behind the L2s holds go straight there (``past``), so that
-// nothing is left in the L2s when the kernel ends, or drives operands out of them (us,
-// through the L2s and past them: 5135 rows, 1024 -> 1536 18.2 and 16.3, 1024 -> 1024 15.0
-// and 13.8; gate, up and activation of 1024 -> 4096 68.6 and 66.9, of 8192 rows 103.5 and
-// 101.0; 8192 rows, 4096 -> 16384 736 and 696; input gradients of 7168 x 14336 571 and 537);
-// more than that passes through them (4096 rows, 4096 -> 128256 2816 and 2992; the trainer's
-// gate, up and activation of 7168 x 14336 each 1166 and 1288).
-constexpr long CACHED_OUT = 256L << 20;
+// Outputs that the L2s hold, 4 MiB each, go past them (``past``), so that the kernel's end
+// has nothing to write back (us, through and past them: 5135 rows, 1024 -> 1536 18.2 and
+// 16.3, 1024 -> 1024 15.0 and 13.8; gate, up and activation of 1024 -> 4096 68.6 and 66.9, of
+// 8192 rows 103.5 and 101.0).  Not as nontemporal ones, which the next kernel would have to
+// read from memory (the rotation behind 1024 -> 1536 10.1 us for 8.1).  Larger ones pass
+// through them: repeated alone they gain too where the 256 MB behind hold them (8192 rows,
+// 4096 -> 16384 736 and 696), but not in a trainer's step (input gradients of 7168 rows
+// through 4096 x 4096 and 4096 x 14336 together 747 and 790), nor where nothing does (4096
+// rows, 4096 -> 128256 2816 and 2992; the trainer's gate, up and activation of 7168 x 14336
+// each 1166 and 1288).
+constexpr long L2_OUT = ATTN_XCDS * (4L << 20);
 struct OutRows {
   char* at;
   long left, pitch;                    // bytes: to the matrix's end, of 16 rows
@@ -499,7 +502,7 @@ struct OutRows {
     return col < cols ? (unsigned)((threadIdx.x & 15) * cols + col) * 2 : 0x80000000u;
   }
   DEV_INLINE void put(unsigned offset, const u32x4_t& w, bool past) const {
-    constexpr int PAST = 18;           // (sc1 and nt)
+    constexpr int PAST = 17;           // (sc0 and sc1)
     if (past) __builtin_amdgcn_raw_buffer_store_b128(w, buffer, offset, 0, PAST);
     else __builtin_amdgcn_raw_buffer_store_b128(w, buffer, offset, 0, 0);
   }
@@ -516,7 +519,7 @@ struct TileRows {
   DEV_INLINE void start(bf16_t* out, long rows, long cols, const Place& at, long col0) {
     const int lane = threadIdx.x & 63, wid = wave_id();
     to.start(out, rows, cols, (long)at.row * (32 * J) + (wid & 1) * (16 * J));
-    past = 2 * rows * cols <= CACHED_OUT;
+    past = 2 * rows * cols < L2_OUT;
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       offset[q] = OutRows::offset(
