@@ -234,17 +234,18 @@ void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
 }
 
 // Whether linear_rows is the better choice than the library's own: tiles that fill
-// rounds of 256 to 0.74 of what whole ones would cost, but not whole tiles of 256 rows,
-// which the library multiplies 1 to 4% faster.  (us, beside the library's, of 2600, 4096,
-// 5135 and 7168 rows: 2048 -> 2048 25.0, 29.8, 36.0, 44.0 and 29.1, 32.8, 48.6, 45.1;
-// 8192 -> 2048 81.5, 99.6, 123, 151 and 82.0, 107, 146, 156; 8960 -> 1536 94.7, 98.3,
-// 108, 138 and 72.5, 96.7, 117, 151, whose first two fill 0.44 and 0.6; 4096 of 14336 ->
-// 4096 296 and 289.)
+// rounds of 256 to 0.53 of what whole ones would cost, but not whole tiles of 256 rows,
+// which the library multiplies 1 to 6% faster.  (us, beside the library's: 4096 -> 1024 of
+// 3500, 4090, 4600, 5135, 8000 rows, 0.43, 0.50, 0.56, 0.63, 0.83 of that cost, 38.3, 38.6,
+// 40.0, 41.1, 51.3 and 35.0, 36.9, 44.6, 45.6, 57.5; 2048 -> 2048 of 2600, 4090, 5135 rows
+// 22.9, 29.1, 35.3 and 31.1, 34.2, 50.7, of 8000, whole tiles, 52.6 and 49.4; 8960 -> 1536 of
+// 2600, 3072, 3500 rows, 0.50, 0.59, 0.67, 77.9, 81.6, 83.0 and 70.9, 82.4, 92.3; of 120
+// shapes the 89 within the line take 0.51 to 1.00 of the library's time.)
 bool linear_rows_pays(long M, long N, long K) {
   if (M <= 0 || N <= 0 || K < PAIR) return false;
   const Rows best = rows_of(M, (N + SIDE - 1) / SIDE, K, 3);
   const double whole = (double)M * N / (CUS * SIDE * SIDE) * cost_of(8, K);
-  return best.cost <= 1.35 * whole && (best.parts < 8 || M % SIDE != 0);
+  return best.cost <= 1.9 * whole && (best.parts < 8 || best.cost >= 1.05 * whole);
 }
 
 // x (M, K), w (N, K)

@@ -5,7 +5,8 @@
 // lane, 128 more for the fragments of two steps, one wave a SIMD, one block a CU.  (Tiles
 // of fewer rows, 32 J, where the left operand is LINES: a wave has J row parts for eight.)
 // A step is 32 inner numbers.  Two steps of an operand, 32 KiB, are loaded as one unit
-// straight into LDS, five units' room; a barrier every two steps.  Where an operand's
+// straight into LDS, five units' room, three of both operands for tiles of up to 160 rows,
+// whose short steps would wait for their loads; a barrier every two steps.  Where an operand's
 // inner dimension is its memory's rows' own (LINES: x and W in x W^T, dY in dY W) a unit
 // is 256 rows of 128 bytes, whole lines, and fragments are read as they are; where it
 // runs over the memory's rows (COLUMNS: W in dY W, both in dY^T X) a unit is 64 rows of 512
@@ -244,6 +245,13 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
   Operand<LL, J> a(lds, left_ld(0), wid & 1);
   Operand<RL> b(lds, right_ld, wid >> 1);
   // (of a unit a wave loads 1 KiB for each of its row parts)
+  // DEEP: three pairs' units fit
+  constexpr int LEFT = J * 4096, THIRD = LEFT + UNIT;
+  constexpr bool DEEP = LL && RL && 3 * THIRD <= LDS_BYTES;
+  constexpr int B0 = DEEP ? LEFT : UNIT;
+  // Loads that may be on their way when the next pair's units have to be there: of the pair
+  // after that the left operand's, and (DEEP) the right one's
+  constexpr int YOUNG = DEEP ? J + 8 : J;
   const unsigned to_a = (unsigned)(uintptr_t)(lds_p)lds + wid * (J * 1024);
   const unsigned to_b = (unsigned)(uintptr_t)(lds_p)lds + wid * 8192;
   Units ua, ub;
@@ -269,13 +277,18 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
     a.start(), b.start();
     pairs = ua.n;
     look_ahead();
-    a.load(to_a), b.load(to_b + UNIT);
-    a.load(to_a + 2 * UNIT), b.load(to_b + 3 * UNIT);
-    arrived<J + 8>();
+    a.load(to_a), b.load(to_b + B0);
+    if constexpr (DEEP) {
+      a.load(to_a + THIRD), b.load(to_b + THIRD + B0), a.load(to_a + 2 * THIRD);
+      arrived<J + YOUNG>();
+    } else {
+      a.load(to_a + 2 * UNIT), b.load(to_b + 3 * UNIT);
+      arrived<J + 8>();
+    }
 #pragma unroll
     for (int d = 0; d < a.FRAGS; ++d) na[d] = a.frag_at[d];
 #pragma unroll
-    for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + UNIT;
+    for (int d = 0; d < b.FRAGS; ++d) nb[d] = b.frag_at[d] + B0;
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
       if (d < J) {
@@ -297,7 +310,7 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
                   int b_next) {
     constexpr int N = decltype(n_)::value, O = 1 - N;
     constexpr bool ENDS = decltype(ends_)::value;
-    constexpr int FRAGS = 8 + J, LOADS = N == 0 ? J : 8, ALL = 8 * J;
+    constexpr int FRAGS = 8 + J, LOADS = (N == 0) == DEEP ? 8 : J, ALL = 8 * J;
     // instructions of a fragment (and a load's two, or with the load's first; few row
     // parts leave room for two)
     constexpr int PER = LL && RL && J < 6 ? 2 : 3;
@@ -307,7 +320,7 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
     // The next unit of both is there, and this one's, read to the end, make room.  (The
     // last tile's stores are as young as this step's loads, and still on their way.)
     if constexpr (N == 1)
-      arrived<ENDS ? std::min(63, J + J * Sink::STORES) : J>();
+      arrived<ENDS ? std::min(63, YOUNG + J * Sink::STORES) : YOUNG>();
     constexpr bool FIRST = ENDS && N == 0;
     f32x4_t sums[COLS];
     each(std::make_integer_sequence<int, ALL>(), [&](auto k_) {
@@ -375,11 +388,20 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
 
   // slots: this pair's units, the next pair's, the left one behind that
   int s0 = 0, s1 = UNIT, s2 = 2 * UNIT, s3 = 3 * UNIT, s4 = 4 * UNIT;
+  // (DEEP: where they, the next pair and the one behind that are)
+  int d0 = 0, d1 = THIRD, d2 = 2 * THIRD;
   auto pair = [&](auto ends) {
-    step(std::integral_constant<int, 0>(), ends, a, to_a + s4, s2, s3);
-    step(std::integral_constant<int, 1>(), ends, b, to_b + s0, s2, s3);
-    const int t0 = s0, t1 = s1;
-    s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
+    if constexpr (DEEP) {
+      step(std::integral_constant<int, 0>(), ends, b, to_b + d2 + B0, d1, d1 + B0);
+      step(std::integral_constant<int, 1>(), ends, a, to_a + d0, d1, d1 + B0);
+      const int t = d0;
+      d0 = d1, d1 = d2, d2 = t;
+    } else {
+      step(std::integral_constant<int, 0>(), ends, a, to_a + s4, s2, s3);
+      step(std::integral_constant<int, 1>(), ends, b, to_b + s0, s2, s3);
+      const int t0 = s0, t1 = s1;
+      s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
+    }
   };
   for (;;) {
     int p = 0;
@@ -533,8 +555,8 @@ struct TileRows {
 
 // Rows of a tile whose left operand is LINES, in 32s from LEAST on (6 where the right one
 // is COLUMNS): as many as end the last round of 256 tiles earliest.  A unit of 64 inner
-// numbers costs 0.105 us a row part and 0.25 for the columns' fragments and loads, a tile
-// 5 us more.  (1024 -> 4096, tiles of 128, 192, 224 and 256 rows: 5135 rows 89.2, 81.4,
+// numbers costs 0.105 us a row part and 0.25 for the columns' fragments and loads (0.19 of
+// the tiles with three pairs of units in LDS), a tile 5 us more.  (1024 -> 4096, tiles of 128, 192, 224 and 256 rows: 5135 rows 89.2, 81.4,
 // 74.0, 81.0 us; 1500 rows 30.0, 24.7, 26.8, 28.8; 1024 rows 18.5, 22.8, 24.0, 25.8; 3072
 // rows, 1536 -> 8960, 145, 142, 136, 147; 5135 rows, 4096 -> 14336, 1068, 875, 868, 888; the
 // gradient of 7168 rows through 14336 x 4096, 192 to 256 rows a tile, 703, 539, 573, of 8192
@@ -544,7 +566,7 @@ struct Rows {
   long cost;
 };
 inline long cost_of(int parts, long inner) {
-  return inner / PAIR * (10 * parts + 24) + 480;
+  return inner / PAIR * (10 * parts + (parts <= 5 ? 18 : 24)) + 480;
 }
 inline Rows rows_of(long rows, long cols, long inner, int least) {
   Rows best{8, -1};

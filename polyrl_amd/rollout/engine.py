@@ -38,12 +38,13 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor, search: bool = True
     (``ops.linear_rows_pays``), take the kernel of this repository, whose call
     costs the host 5 us for the 20 of torch's (a step of 3, 4, 6 and 8 x 256
     tokens, 12 layers of 1024, 1109, 1124, 1286 and 1447 us with it and 1471, 1491,
-    1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the device it is up to 4 us slower within these lines (us, kernel and library, of
-    513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 8.3, 8.5, 8.8, 9.4, 13.0 and 6.3,
-    6.6, 7.7, 9.7, 14.9; 1024 -> 1024 11.7, 12.0, 12.7, 14.9, 19.4 and 7.7, 8.0, 10.4,
-    13.3, 21.5; 1024 -> 1536 11.8, 12.2, 13.8, 17.1, 28.4 and 7.8, 9.8, 13.1, 18.5,
+    1544 and 1560 without; 12 x 256 the same, 16 x 330 2591 and 2647).  On the
+    device it is up to 4 us slower within these lines (us, kernel and library, of
+    513, 1024, 2048, 4096 and 8192 rows: 512 -> 1024 8.0, 8.0, 8.2, 8.4, 10.7 and 6.3,
+    6.6, 7.7, 9.7, 14.9; 1024 -> 1024 11.7, 11.8, 11.8, 12.3, 16.2 and 7.7, 8.0, 10.4,
+    13.3, 21.5; 1024 -> 1536 11.6, 11.8, 12.2, 14.5, 22.8 and 7.8, 9.8, 13.1, 18.5,
     29.3); of wider ones it would be by more than the host gains where outputs are few
-    (1024 of 600 .. 4096 rows 0.5 to 0.83 of the library's speed at an inner width of
+    (1024 of 700 .. 3500 rows 0.54 to 0.91 of the library's speed at an inner width of
     4096); a captured graph, where the host's time does not
     count, takes the library's.  ``search``: False for few rows whose number is not
     a decode batch's."""

@@ -200,9 +200,9 @@ def test_linears_search():
 
 
 @pytest.mark.parametrize("m,n,k,rows", [
-    (2600, 2048, 2048, False), (4096, 2048, 2048, True), (4100, 2048, 2048, False),
-    (2048, 4096, 2048, True),
-    (4096, 4096, 2048, False), (4095, 4096, 2048, True), (5000, 512, 4096, False)])
+    (2300, 2048, 2048, True), (2200, 2048, 2048, False), (4096, 2048, 2048, True),
+    (2048, 4096, 2048, True), (4096, 4096, 2048, False), (4095, 4096, 2048, False),
+    (4300, 1024, 4096, True), (4200, 1024, 4096, False), (5000, 512, 4096, False)])
 def test_engine_wide_prompts(m, n, k, rows, monkeypatch):
     """Both sides of the line for widths beyond 1024."""
     from polyrl_amd.rollout.engine import _mm_nt
