@@ -49,6 +49,30 @@ def test_fused_add_rmsnorm():
     assert rel_err(out.cpu(), expect_norm) < 2e-2
 
 
+@pytest.mark.parametrize("d", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 4096,
+                               4104, 8192, 8200, 12288])
+@pytest.mark.parametrize("rows", [1, 130, 1024])
+def test_rmsnorm_widths(rows, d):
+    """Both sides of the widths from which a row takes more waves and more words
+    a thread."""
+    g = torch.Generator(device=DEV).manual_seed(d + rows)
+    x, res = (torch.randn(rows, d, generator=g, device=DEV).bfloat16()
+              for _ in range(2))
+    w = torch.randn(d, generator=g, device=DEV).bfloat16()
+
+    def close(got, y):
+        want = y.double() * (y.double().square().mean(-1, keepdim=True)
+                             + 1e-6).rsqrt() * w.double()
+        # one rounding to bf16, 32-bit sums of squares
+        assert ((got.double() - want).abs() <= (2 ** -8 + 1e-5)
+                * want.abs()).all()
+    close(ops.rmsnorm(x, w), x)
+    total = (x.float() + res.float()).bfloat16()
+    out, new = ops.fused_add_rmsnorm(x, res, w)
+    assert torch.equal(new, total)
+    close(out, total)
+
+
 def test_silu_mul():
     torch.manual_seed(2)
     g = torch.randn(64, 5632, dtype=torch.bfloat16, device=DEV)
