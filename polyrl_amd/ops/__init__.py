@@ -548,6 +548,9 @@ def _joint_backward(needs, x, ws, dys):
             for dy, w in zip(dys, ws):
                 d = ext.tuned_linear_dgrad(dy, w)
                 dx = d if dx is None else dx.add_(d)
+    if len(dys) == 2 and all(needs[1:]) \
+            and ext.linear_wgrad_pair_takes(*dys, x):
+        return dx, *ext.linear_wgrad_pair(*dys, x)
     return dx, *(ext.tuned_linear_wgrad(dy, x) if need else None
                  for dy, need in zip(dys, needs[1:]))
 

@@ -14,6 +14,10 @@ bool linear_joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>
 std::vector<torch::Tensor> linear_joint(torch::Tensor x, std::vector<torch::Tensor> ws);
 bool linear_gated_takes(const torch::Tensor& x, const torch::Tensor& wg,
                         const torch::Tensor& wu);
+bool linear_wgrad_pair_takes(const torch::Tensor& dy0, const torch::Tensor& dy1,
+                             const torch::Tensor& x);
+std::vector<torch::Tensor> linear_wgrad_pair(torch::Tensor dy0, torch::Tensor dy1,
+                                             torch::Tensor x);
 std::vector<torch::Tensor> linear_gated(torch::Tensor x, torch::Tensor wg,
                                         torch::Tensor wu, bool keep);
 bool linear_dgrad_sum_takes(const std::vector<torch::Tensor>& dys,
@@ -101,6 +105,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows", &linear_rows, "x W^T of prompts");
   m.def("linear_joint_takes", &linear_joint_takes, "linear_joint for a product each");
   m.def("linear_joint", &linear_joint, "x W^T of several weights");
+  m.def("linear_wgrad_pair_takes", &linear_wgrad_pair_takes,
+        "linear_wgrad_pair for a product each");
+  m.def("linear_wgrad_pair", &linear_wgrad_pair, "dY0^T X and dY1^T X");
   m.def("linear_gated_takes", &linear_gated_takes, "linear_gated for a product each");
   m.def("linear_gated", &linear_gated, "silu(x Wg^T) * (x Wu^T), and both products");
   m.def("linear_dgrad_sum_takes", &linear_dgrad_sum_takes,

@@ -18,12 +18,21 @@
 // rows through the latter 137 for 343.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+#include <climits>
 
 #include "product_tile.h"
 
 namespace {
 
 using namespace product;
+
+// A second product of the same size and right operand: its row tiles are those from
+// ``first`` on
+struct Twin {
+  bf16_t* out;
+  const bf16_t* left;
+  int first;
+};
 
 // A tile's outputs, or where blocks share its inner numbers its fp32 sums, which are added
 // up afterwards: (tiles, ways, SIDE * SIDE)
@@ -32,15 +41,19 @@ struct Outputs : TileRows<J> {
   bf16_t* const out;
   float* const shares;
   const long R, C;
+  const Twin twin;
   f32x4_t* to_share;
-  DEV_INLINE Outputs(bf16_t* out_, float* shares_, long R_, long C_)
-      : out(out_), shares(shares_), R(R_), C(C_) {}
+  DEV_INLINE Outputs(bf16_t* out_, float* shares_, long R_, long C_, const Twin& twin_)
+      : out(out_), shares(shares_), R(R_), C(C_), twin(twin_) {}
   DEV_INLINE void tile(const Place& at) {
-    if (J == 8 && shares != nullptr)
+    if (J == 8 && shares != nullptr) {
       to_share = reinterpret_cast<f32x4_t*>(shares + (long)at.share * SIDE * SIDE) +
                  wave_id() * 4096 + (threadIdx.x & 63);
-    else
-      this->start(out, R, C, at, (long)at.col * SIDE);
+    } else {
+      Place in = at;
+      if (at.row >= twin.first) in.row -= twin.first;
+      this->start(at.row >= twin.first ? twin.out : out, R, C, in, (long)at.col * SIDE);
+    }
   }
   DEV_INLINE void rows(int) {
     if (J < 8 || shares == nullptr) this->to.next();
@@ -61,8 +74,9 @@ struct Outputs : TileRows<J> {
 template <bool LINES, int J>
 __global__ __launch_bounds__(256, 1) void product_kernel(
     bf16_t* __restrict__ out, float* __restrict__ shares,
-    const bf16_t* __restrict__ left, const bf16_t* __restrict__ right, long R,
-    long C, long inner, int row_tiles, int col_tiles, int ways) {
+    const bf16_t* __restrict__ left, const bf16_t* __restrict__ right,
+    const Twin twin, long R, long C, long inner, int row_tiles, int col_tiles,
+    int ways) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   constexpr int ROWS = 32 * J;
   const int tiles = row_tiles * col_tiles, items = tiles * ways;
@@ -74,13 +88,15 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
     at = Place(tile, row_tiles, col_tiles, tile * ways + part);
     const int p0 = (int)((long)all * part / ways);
     const int n = (int)((long)all * (part + 1) / ways) - p0;
-    const long r0 = (long)at.row * ROWS, c0 = (long)at.col * SIDE;
-    const long i0 = (long)p0 * PAIR;
-    a = LINES ? lines(left, R, inner, r0, i0, n) : columns(left, R, inner, r0, i0, n);
+    const bool second = !LINES && at.row >= twin.first;
+    const bf16_t* l = second ? twin.left : left;
+    const long r0 = (long)(at.row - (second ? twin.first : 0)) * ROWS;
+    const long c0 = (long)at.col * SIDE, i0 = (long)p0 * PAIR;
+    a = LINES ? lines(l, R, inner, r0, i0, n) : columns(l, R, inner, r0, i0, n);
     b = columns(right, C, inner, c0, i0, n);
     return true;
   };
-  Outputs<J> outputs(out, shares, R, C);
+  Outputs<J> outputs(out, shares, R, C, twin);
   run<LINES, false, J>(
       lds, [&](int) { return LINES ? inner : R; }, C, units, outputs);
 }
@@ -116,7 +132,7 @@ __global__ __launch_bounds__(256, 1) void parts_kernel(
     b = columns(right, C, inner, (long)at.col * SIDE, 0, (int)(inner / PAIR));
     return true;
   };
-  Outputs<J> outputs(out, nullptr, R, C);
+  Outputs<J> outputs(out, nullptr, R, C, {nullptr, nullptr, INT_MAX});
   run<true, false, J, PARTS>(lds, inner_of, C, units, outputs);
 }
 
@@ -207,8 +223,8 @@ torch::Tensor product_of(const torch::Tensor& left, const torch::Tensor& right, 
   auto launch = [&](auto kern) {
     kern<<<dim3((unsigned)grid), dim3(256), 0, stream>>>(
         (bf16_t*)out.data_ptr(), sums, (const bf16_t*)left.data_ptr(),
-        (const bf16_t*)right.data_ptr(), R, C, inner, (int)row_tiles,
-        (int)col_tiles, (int)ways);
+        (const bf16_t*)right.data_ptr(), Twin{nullptr, nullptr, INT_MAX}, R, C, inner,
+        (int)row_tiles, (int)col_tiles, (int)ways);
   };
   if (LINES && parts == 6) launch(product_kernel<LINES, LINES ? 6 : 8>);
   else if (LINES && parts == 7) launch(product_kernel<LINES, LINES ? 7 : 8>);
@@ -257,6 +273,40 @@ torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x) {
   TORCH_CHECK(x.size(0) == dy.size(0) && wgrad_fits(dy, x),
               "linear_wgrad: rows in 16-byte granules, at most 4 GiB");
   return product_of<false>(dy, x, dy.size(1), x.size(1), dy.size(0));
+}
+
+// Whether linear_wgrad_pair has these operands and is the better choice than a product
+// each: two of one size whose tiles are not shared.  Their tiles fill rounds of 256
+// together (7168 rows, 14336 x 4096 each: 7 rounds for 4 and 4, 1120 us for 1224; 7168
+// rows, 11008 x 2048 458 for 542; 512 rows, 14336 x 4096 119 for 136; 3000 rows, 8960 x 1536
+// 126 for 131; 5135 rows, 5120 x 2048, whose rounds are as many, 191 both).
+bool linear_wgrad_pair_takes(const torch::Tensor& dy0, const torch::Tensor& dy1,
+                             const torch::Tensor& x) {
+  return dy0.sizes() == dy1.sizes() && wgrad_fits(dy1, x) && linear_wgrad_takes(dy0, x) &&
+         tiles_of(dy0.size(1), x.size(1)) >= 160;
+}
+
+// dW_p (N, K) = dY_p^T X of dY_p (M, N), X (M, K)
+std::vector<torch::Tensor> linear_wgrad_pair(torch::Tensor dy0, torch::Tensor dy1,
+                                             torch::Tensor x) {
+  check_operands(dy0, x);
+  check_operands(dy1, x);
+  TORCH_CHECK(x.size(0) == dy0.size(0) && linear_wgrad_pair_takes(dy0, dy1, x),
+              "linear_wgrad_pair: operands that it does not take");
+  const long R = dy0.size(1), C = x.size(1), inner = dy0.size(0);
+  std::vector<torch::Tensor> outs;
+  for (int i = 0; i < 2; ++i) outs.push_back(torch::empty({R, C}, x.options()));
+  const long rows = (R + SIDE - 1) / SIDE, cols = (C + SIDE - 1) / SIDE;
+  const long items = 2 * rows * cols;
+  TORCH_CHECK(items < (1L << 31) - ATTN_XCDS, "grid too large");
+  product_kernel<false, 8><<<dim3((unsigned)blocks_of(items, inner)), dim3(256), 0,
+                             at::hip::getCurrentHIPStream()>>>(
+      (bf16_t*)outs[0].data_ptr(), nullptr, (const bf16_t*)dy0.data_ptr(),
+      (const bf16_t*)x.data_ptr(),
+      Twin{(bf16_t*)outs[1].data_ptr(), (const bf16_t*)dy1.data_ptr(), (int)rows}, R, C,
+      inner, (int)(2 * rows), (int)cols, 1);
+  HIP_CHECK_KERNEL();
+  return outs;
 }
 
 // dX (M, K) = dY W of dY (M, N), W (N, K)

@@ -222,3 +222,18 @@ def test_joint_other_layers():
     assert ops.gated_linear(x, lin(), lin(bias=True)) is None
     assert ops.joint_linear(x[:500], (lin(), lin())) is None
     assert ops.joint_linear(x.cpu(), (lin(), lin())) is None
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 5120, 2048), (520, 4104, 2568),
+                                   (700, 14336, 1000)])
+def test_wgrad_pair(m, n, k):
+    """Two layers of one input: as a product each, edges of tiles at both ends."""
+    ext = ops._require_ext()
+    x, dys = rand(m, k, 1), [rand(m, n, 2), rand(m, n, 3)]
+    assert ext.linear_wgrad_pair_takes(*dys, x)
+    for dy, got in zip(dys, ext.linear_wgrad_pair(*dys, x)):
+        assert torch.equal(got, ext.linear_wgrad(dy, x))
+    for other in (rand(m, n + 8, 4), rand(m + 1, n, 4)):
+        assert not ext.linear_wgrad_pair_takes(dys[0], other, x)
+        with pytest.raises(RuntimeError):
+            ext.linear_wgrad_pair(dys[0], other, x)
