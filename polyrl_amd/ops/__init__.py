@@ -83,6 +83,13 @@ def linear_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def linear_rows_add(out: torch.Tensor, x: torch.Tensor,
+                    w: torch.Tensor) -> torch.Tensor:
+    """out += x @ w.T in place, rounded once (what ``linear_takes``)."""
+    _require_ext().linear_rows_add(out, x, w)
+    return out
+
+
 def linear_rows_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``linear_rows``, which takes these operands, is the faster one on
     the device."""

@@ -58,8 +58,9 @@ DEV_INLINE Part part_of(const Parts& parts, long& col) {
 }
 
 // PLAIN: the products.  GATED: out = silu(gate) * up of the products with p[0], gate, and
-// p[1], up.  KEPT: the products too.
-enum Kind { PLAIN, GATED, KEPT };
+// p[1], up.  KEPT: the products too.  ADDED: the product added to what its output holds.
+enum Kind { PLAIN, GATED, KEPT, ADDED };
+constexpr bool halves(Kind kind) { return kind == GATED || kind == KEPT; }
 
 // Where a tile's outputs go
 template <int J, Kind KIND>
@@ -74,6 +75,50 @@ struct Outputs<J, PLAIN> : TileRows<J> {
     long col = (long)at.col * SIDE;
     const Part p = part_of(parts, col);
     this->start(p.out, M, p.n, at, col);
+  }
+};
+
+// Two row parts' old numbers are on their way at once (all of a tile's: no gain)
+template <int J>
+struct Outputs<J, ADDED> : TileRows<J> {
+  const Part part;
+  const long M;
+  OutRows old;
+  static constexpr int AHEAD = 2;
+  u32x4_t held[AHEAD][4];
+  DEV_INLINE Outputs(bf16_t*, const Parts& parts, long M_) : part(parts.p[0]), M(M_) {}
+  DEV_INLINE void load(int j) {
+    old.next();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) held[j % AHEAD][q] = old.get(this->offset[q]);
+  }
+  DEV_INLINE void tile(const Place& at) {
+    this->start(part.out, M, part.n, at, (long)at.col * SIDE);
+    old = this->to;
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) load(j);
+  }
+  // (the part before is stored)
+  DEV_INLINE void rows(int j) {
+    this->to.next();
+    if (j > 0 && j - 1 + AHEAD < J) load(j - 1 + AHEAD);
+  }
+  DEV_INLINE void put(int j, int q, const f32x4_t (&sums)[2]) const {
+    // the old numbers where the sums' lanes have theirs: lanes exchanged as in
+    // eight_columns, the other way
+    f32x4_t c[2] = {sums[0], sums[1]};
+    const u32x4_t& now = held[j % AHEAD][q];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const auto p = __builtin_amdgcn_permlane16_swap(now[w], now[2 + w], false, false);
+      const auto x = __builtin_amdgcn_permlane32_swap(p[0], p[1], false, false);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        c[h][2 * w] += __uint_as_float(x[h] << 16);
+        c[h][2 * w + 1] += __uint_as_float(x[h] & 0xffff0000u);
+      }
+    }
+    this->to.put(this->offset[q], eight_columns(c[0], c[1]), this->past);
   }
 };
 
@@ -128,11 +173,11 @@ struct Outputs {
 
 template <int J, Kind KIND>
 __global__ __launch_bounds__(256, 1) void linear_kernel(
-    bf16_t* __restrict__ out,          // (M, n), but PLAIN
+    bf16_t* __restrict__ out,          // (M, n), GATED and KEPT
     const bf16_t* __restrict__ x,      // (M, K)
     const Parts parts, long M, long K, int row_tiles, int col_tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  constexpr int ROWS = 32 * J, COLS = KIND == PLAIN ? 256 : 128;
+  constexpr int ROWS = 32 * J, COLS = halves(KIND) ? 128 : 256;
   const int items = row_tiles * col_tiles, n = (int)(K / PAIR);
   const long N = parts.p[0].n;
   auto units = [&](int r, Units& a, Units& b, Place& at) {
@@ -141,7 +186,7 @@ __global__ __launch_bounds__(256, 1) void linear_kernel(
     at = Place(item, row_tiles, col_tiles);
     a = lines(x, M, K, (long)at.row * ROWS, 0, n);
     long col = (long)at.col * COLS;
-    if (KIND != PLAIN) {
+    if (halves(KIND)) {
       // a wave loads the 64 rows of its number: gate, up, gate, up
       const int wid = wave_id();
       b = lines(wid & 1 ? parts.p[1].w : parts.p[0].w, N, K,
@@ -251,6 +296,23 @@ bool linear_rows_pays(long M, long N, long K) {
 // x (M, K), w (N, K)
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w) {
   return linear_prompt<false>(x, w);
+}
+
+// out += x W^T, rounded once: what follows need not add it.  (us, the product and a norm
+// that adds, and this and a norm: 4096 -> 1024 of 1024, 2600, 5135, 8192 rows 38.3, 40.9,
+// 46.6, 61.7 and 39.4, 40.6, 45.2, 59.6; 2048 -> 2048 24.3, 29.9, 46.7, 70.0 and 24.8, 29.2,
+// 45.1, 66.7; 1024 -> 1024 15.7, 18.1, 21.0, 27.9 and 17.1, 18.8, 20.9, 25.7)
+void linear_rows_add(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
+  for (const auto* t : {&out, &x, &w})
+    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&
+                    t->is_contiguous() && t->dtype() == torch::kBFloat16,
+                "linear: contiguous 2-D bf16 of one device");
+  TORCH_CHECK(w.size(1) == x.size(1) && out.size(0) == x.size(0) &&
+                  out.size(1) == w.size(0) && linear_rows_fits(x, w) &&
+                  ((uintptr_t)out.data_ptr() & 15) == 0,
+              "linear: inner numbers in 64s, outputs in 8s, 16-byte addresses");
+  const long N = w.size(0);
+  launch_linear<ADDED>(nullptr, x, {{part(&out, w, 0, N)}}, (N + SIDE - 1) / SIDE);
 }
 
 // x (M, K), w (2 N, K): rows of the gate, then of the up projection

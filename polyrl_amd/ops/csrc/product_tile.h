@@ -523,6 +523,9 @@ struct OutRows {
   DEV_INLINE static unsigned offset(long cols, long col) {
     return col < cols ? (unsigned)((threadIdx.x & 15) * cols + col) * 2 : 0x80000000u;
   }
+  DEV_INLINE u32x4_t get(unsigned offset) const {
+    return __builtin_amdgcn_raw_buffer_load_b128(buffer, offset, 0, 0);
+  }
   DEV_INLINE void put(unsigned offset, const u32x4_t& w, bool past) const {
     constexpr int PAST = 17;           // (sc0 and sc1)
     if (past) __builtin_amdgcn_raw_buffer_store_b128(w, buffer, offset, 0, PAST);

@@ -51,12 +51,15 @@ def _mm_nt(x: torch.Tensor, w: torch.Tensor, search: bool = True
     if search and x.is_cuda and x.dtype == torch.bfloat16 \
             and x.shape[0] <= 512 and _tuned_decode_enabled():
         return ops.tuned_mm_nt(x, w)
-    if 512 < x.shape[0] and ops.linear_takes(x, w) and (
-            ops.linear_rows_pays(x, w) if x.shape[1] > 1024 else
-            x.shape[0] <= 8192 and x.shape[0] * w.shape[0] <= 3 << 22) \
-            and not torch.cuda.is_current_stream_capturing():
-        return ops.linear_rows(x, w)
-    return x @ w.t()
+    return ops.linear_rows(x, w) if _takes_rows(x, w) else x @ w.t()
+
+
+def _takes_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``_mm_nt`` has this repository's kernel for a prompt's x @ w.T."""
+    return 512 < x.shape[0] and ops.linear_takes(x, w) and (
+        ops.linear_rows_pays(x, w) if x.shape[1] > 1024 else
+        x.shape[0] <= 8192 and x.shape[0] * w.shape[0] <= 3 << 22) \
+        and not torch.cuda.is_current_stream_capturing()
 
 
 def _gate_up(x: torch.Tensor, w: torch.Tensor, search: bool = True
@@ -342,8 +345,11 @@ class InferenceModel:
         # 512 tokens the products' algorithms were searched for as many rows as
         # there are, in the layers before: all of them go on.
         early = rows is not None and x.shape[0] > 512
+        # prompts' projections add to the residual themselves, from 2^22 outputs on:
+        # fewer wait for the old numbers longer than the norm behind them gains
+        adds = tp == 1 and residual.numel() >= 1 << 22
         for li, lw in enumerate(self.layers):
-            if li == 0:
+            if hidden is None:                        # (the residual has it)
                 hidden = ops.rmsnorm(residual, lw.input_ln, cfg.rms_norm_eps)
             else:
                 hidden, residual = ops.fused_add_rmsnorm(
@@ -365,18 +371,29 @@ class InferenceModel:
                     return x.new_empty(0, x.shape[1])
                 attn_out = attn_out.index_select(0, rows)
                 residual = residual.index_select(0, rows)
-            hidden = _mm_nt(attn_out, lw.wo, not few)
-            self.tp.all_reduce_(hidden)               # col-parallel o_proj
-            hidden, residual = ops.fused_add_rmsnorm(
-                hidden, residual, lw.post_ln, cfg.rms_norm_eps)
-            hidden = _mm_nt(_gate_up(hidden, lw.w_gate_up, not few),
-                            lw.w_down, not few)
-            self.tp.all_reduce_(hidden)               # col-parallel down_proj
+            if adds and not few and _takes_rows(attn_out, lw.wo):
+                ops.linear_rows_add(residual, attn_out, lw.wo)
+                hidden = ops.rmsnorm(residual, lw.post_ln, cfg.rms_norm_eps)
+            else:
+                hidden = _mm_nt(attn_out, lw.wo, not few)
+                self.tp.all_reduce_(hidden)           # col-parallel o_proj
+                hidden, residual = ops.fused_add_rmsnorm(
+                    hidden, residual, lw.post_ln, cfg.rms_norm_eps)
+            act = _gate_up(hidden, lw.w_gate_up, not few)
+            if adds and not few and _takes_rows(act, lw.w_down):
+                ops.linear_rows_add(residual, act, lw.w_down)
+                hidden = None
+            else:
+                hidden = _mm_nt(act, lw.w_down, not few)
+                self.tp.all_reduce_(hidden)           # col-parallel down_proj
         # final residual add + norm (fused; residual buffer is dead after)
-        normed, _ = ops.fused_add_rmsnorm(hidden, residual, self.final_norm,
-                                          cfg.rms_norm_eps)
-        return normed if rows is None or early \
-            else normed.index_select(0, rows)
+        if hidden is None:
+            hidden = ops.rmsnorm(residual, self.final_norm, cfg.rms_norm_eps)
+        else:
+            hidden, _ = ops.fused_add_rmsnorm(hidden, residual, self.final_norm,
+                                              cfg.rms_norm_eps)
+        return hidden if rows is None or early \
+            else hidden.index_select(0, rows)
 
     @torch.no_grad()
     def _forward_tokens_gpt2(self, token_ids, positions, kv, slot_mapping,

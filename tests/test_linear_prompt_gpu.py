@@ -263,3 +263,70 @@ def test_outputs_beyond_the_cache():
         op(out, x, w)
         return out
     assert torch.equal(rows(w), torch.cat([rows(w[:64136]), rows(w[64136:])], 1))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 64), (97, 512, 128), (700, 1024, 320),
+                                   (513, 256, 1024), (93, 76800, 256),
+                                   (445, 76800, 320), (253, 76800, 384)])
+def test_added(m, n, k):
+    """Outputs that hold numbers already: one rounding of the whole sum, edges of
+    tiles, a block's tiles one after the other; what stands behind is not touched."""
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = torch.randn(n, k, generator=g, device=DEV).bfloat16()
+    flat = torch.randn(m * n + 65536, generator=g, device=DEV).bfloat16()
+    out, behind, old = flat[:m * n].view(m, n), flat[m * n:].clone(), \
+        flat[:m * n].view(m, n).double()
+    ops.linear_rows_add(out, x, w)
+    a, b = x.double(), w.double().t()
+    want = a @ b + old
+    bound = 2 ** -8 * want.abs() + (k + 1) * 2.0 ** -24 * (
+        a.abs() @ b.abs() + old.abs())
+    assert ((out.double() - want).abs() <= bound).all()
+    assert torch.equal(flat[m * n:], behind)
+
+
+@pytest.mark.parametrize("tokens,calls", [(4095, 0), (4096, 2)])
+def test_engine_adds(tokens, calls, monkeypatch):
+    """From 2^22 outputs on the projections add to the residual: both sides of the
+    line, the same logits as by a product and a norm that adds but for roundings."""
+    from polyrl_amd.models import get_model_config
+    from polyrl_amd.rollout import engine
+    cfg = get_model_config("llama-400m", {"num_hidden_layers": 2})
+    eng = engine.Engine(cfg, device=DEV, dtype=torch.bfloat16, page_size=16,
+                        kv_token_capacity=tokens + 64, max_running_requests=4)
+    h, i, d = cfg.hidden_size, cfg.intermediate_size, cfg.head_dim
+    assert h == 1024
+    g = torch.Generator(device=DEV).manual_seed(5)
+    nq, nk = cfg.num_attention_heads * d, cfg.num_key_value_heads * d
+    shapes = {"model.embed_tokens": (cfg.vocab_size, h), "model.norm": (h,),
+              "lm_head": (cfg.vocab_size, h)}
+    for li in range(2):
+        at = "model.layers.%d." % li
+        for name, shape in (
+                ("self_attn.q_proj", (nq, h)), ("self_attn.k_proj", (nk, h)),
+                ("self_attn.v_proj", (nk, h)), ("self_attn.o_proj", (h, nq)),
+                ("mlp.gate_proj", (i, h)), ("mlp.up_proj", (i, h)),
+                ("mlp.down_proj", (h, i)), ("input_layernorm", (h,)),
+                ("post_attention_layernorm", (h,))):
+            shapes[at + name] = shape
+    eng.model.load_state_dict({
+        n + ".weight": (torch.ones(s, device=DEV) if len(s) == 1 else 0.03
+                        * torch.randn(s, generator=g, device=DEV)).bfloat16()
+        for n, s in shapes.items()})
+    ids = torch.randint(cfg.vocab_size, (tokens,), generator=g, device=DEV).tolist()
+    cuts = [0, 900, 1901, 2600, tokens]
+    ran, real = [], ops.linear_rows_add
+
+    def step():
+        prompts = [("r%d" % k, ids[a:b], [b - a - 1])
+                   for k, (a, b) in enumerate(zip(cuts, cuts[1:]))]
+        return eng.step_forced(prompts, end=[p[0] for p in prompts])
+    monkeypatch.setattr(ops, "linear_rows_add",
+                        lambda *a: ran.append(1) or real(*a))
+    got = step()
+    # (the first layer's two at most: the last one goes on with few rows)
+    assert bool(ran) == bool(calls) and len(ran) <= calls
+    monkeypatch.setattr(engine, "_takes_rows", lambda x, w: False)
+    want = step()
+    assert (got - want).norm() / want.norm() <= 2e-2
