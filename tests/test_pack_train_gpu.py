@@ -1,5 +1,6 @@
 """The trainer's packed rows: maps of padded batches, hidden rows at the places
 asked for, the embedding's gradient."""
+import numpy as np
 import pytest
 import torch
 
@@ -95,9 +96,11 @@ def test_embed_grad(t, v, h):
 
 
 @pytest.mark.parametrize("rows", [slice(-41, -1), slice(None), slice(3, 50, 2), slice(60, 61),
-                                  None])
+                                  None, -1, [7, 3, 80], np.array([5, 5]),
+                                  torch.arange(90) % 3 == 0])
 def test_model(rows):
-    """A model's logits and gradients against the same with boolean indices."""
+    """A model's logits and gradients against the same with boolean indices: of the
+    places of a slice, or of whatever else indexes a dimension."""
     torch.manual_seed(0)
     cfg = get_model_config("llama-tiny")
     m = CausalLM(cfg).to(DEV, torch.bfloat16).train()
