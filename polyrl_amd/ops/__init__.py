@@ -654,6 +654,12 @@ def packed_tables(lens, device):
     return cu, tuple(rest)
 
 
+def _in_words(t: torch.Tensor) -> torch.Tensor:
+    """t contiguous at a 16-byte address (a gradient may be a part of any buffer)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _RowsFromPacked(torch.autograd.Function):
     """Rows of packed hidden states at the places of a padded batch (zeros
     where a place has no token), and the gradient back by the same gather the
@@ -662,12 +668,12 @@ class _RowsFromPacked(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, packed, place):
         ctx.save_for_backward(place)
-        return _require_ext().gather_rows(x.contiguous(), packed)
+        return _require_ext().gather_rows(_in_words(x), packed)
 
     @staticmethod
     def backward(ctx, dout):
         place, = ctx.saved_tensors
-        dout = dout.reshape(-1, dout.shape[-1]).contiguous()
+        dout = _in_words(dout.reshape(-1, dout.shape[-1]))
         return _require_ext().gather_rows(dout, place), None, None
 
 
@@ -690,7 +696,7 @@ class _EmbedTrain(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         ids, = ctx.saved_tensors
-        return _require_ext().embed_grad(dy.contiguous(), ids, ctx.vocab), None
+        return _require_ext().embed_grad(_in_words(dy), ids, ctx.vocab), None
 
 
 def embed_train(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

@@ -95,6 +95,27 @@ def test_embed_grad(t, v, h):
     assert ((w.grad.double() - want).abs() <= bound).all()
 
 
+def test_gradients_anywhere():
+    """Gradients that are a part of a buffer, at an address of no whole word, and
+    strided ones."""
+    ids = torch.tensor([3, 0, 3, 2], device=DEV)
+    place = torch.tensor([2, 0, -1, 3], dtype=torch.int32, device=DEV)
+    packed = torch.tensor([[1, -1], [0, 3]], dtype=torch.int32, device=DEV)
+    flat = torch.randn(4 * 24 + 1, generator=gen(1), device=DEV).bfloat16()
+    for g in (flat[1:].view(4, 24), flat[:-1].view(24, 4).t()):
+        w = torch.randn(5, 24, device=DEV).bfloat16().requires_grad_()
+        ops.embed_train(ids, w).backward(g)
+        want = torch.zeros(5, 24, device=DEV).index_add(0, ids, g.float())
+        assert torch.equal(w.grad, want.bfloat16())
+        x = g.detach().requires_grad_()
+        out = ops.rows_from_packed(x, packed, place)
+        assert torch.equal(out.view(4, 24)[[2, 0, 3]], g[[0, 1, 3]])
+        out.backward(g.view(2, 2, 24) if g.is_contiguous() else
+                     g.reshape(2, 2, 24))
+        assert torch.equal(x.grad[[0, 1, 3]], g[[2, 0, 3]])
+        assert not x.grad[2].any() and not out[0, 1].any()
+
+
 @pytest.mark.parametrize("rows", [slice(-41, -1), slice(None), slice(3, 50, 2), slice(60, 61),
                                   None, -1, [7, 3, 80], np.array([5, 5]),
                                   torch.arange(90) % 3 == 0])
