@@ -17,6 +17,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from .registry import DecoderConfig
 
@@ -360,7 +361,8 @@ class DecoderModel(nn.Module):
         does nothing else."""
         m = self.embed_tokens
         w = m.weight
-        if (type(m) is nn.Embedding and w.is_cuda
+        if (type(m) is nn.Embedding and "forward" not in vars(m)
+                and not _has_any_global_hook() and w.is_cuda
                 and w.dtype == torch.bfloat16 and not hasattr(w, "placements")
                 and w.shape[1] % 8 == 0 and ids.shape[0] <= 32768
                 and m.padding_idx is None and m.max_norm is None

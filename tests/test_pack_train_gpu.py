@@ -153,3 +153,42 @@ def test_model(rows):
         # 32-bit sums in another order, rounded to bf16
         a, b_ = a.double(), b_.double()
         assert (a - b_).norm() <= 2 ** -8 * b_.norm() + 1e-30
+
+
+@pytest.mark.parametrize("how", ["forward", "hook", "global"])
+def test_embedding_with_more(how, monkeypatch):
+    """An embedding whose forward was replaced, or that hooks watch, is called."""
+    cfg = get_model_config("llama-tiny")
+    m = CausalLM(cfg).to(DEV, torch.bfloat16)
+    m.model.use_remove_padding = True
+    emb, ran = m.model.embed_tokens, []
+    fused = []
+    monkeypatch.setattr(ops, "embed_train",
+                        lambda ids, w: fused.append(1) or w[ids])
+    ids = torch.arange(12, device=DEV).view(2, 6)
+
+    def step():
+        m(ids, attention_mask=torch.ones_like(ids),
+          position_ids=ids % 6)
+
+    def hook(mod, *_):
+        if mod is emb:
+            ran.append(1)
+    step()
+    assert fused == [1] and not ran
+    if how == "forward":
+        plain = emb.forward
+        emb.forward = lambda x: ran.append(1) or plain(x)
+    elif how == "hook":
+        emb.register_forward_hook(hook)
+    else:
+        handle = torch.nn.modules.module.register_module_forward_hook(hook)
+    try:
+        step()
+    finally:
+        if how == "global":
+            handle.remove()
+    assert fused == ran == [1]
+    if how == "global":
+        step()
+        assert fused == [1, 1] and ran == [1]
