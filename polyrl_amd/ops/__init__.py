@@ -564,11 +564,10 @@ def _joint_backward(needs, x, ws, dys):
 
 class _GatedLinear(torch.autograd.Function):
     """silu(x Wg^T) * (x Wu^T): both products and the activation in one kernel,
-    which keeps the products for the way back."""
+    which with ``keep`` stores the products for the way back."""
 
     @staticmethod
-    def forward(ctx, x, wg, wu):
-        keep = any(ctx.needs_input_grad)
+    def forward(ctx, x, wg, wu, keep):
         out, *kept = _require_ext().linear_gated(x, wg, wu, keep)
         if keep:
             ctx.save_for_backward(x, wg, wu, *kept)
@@ -579,7 +578,8 @@ class _GatedLinear(torch.autograd.Function):
         x, wg, wu, gate, up = ctx.saved_tensors
         dgate, dup = torch.empty_like(gate), torch.empty_like(up)
         _require_ext().silu_mul_bwd(dgate, dup, dy.contiguous(), gate, up)
-        return _joint_backward(ctx.needs_input_grad, x, [wg, wu], [dgate, dup])
+        return *_joint_backward(ctx.needs_input_grad[:3], x, [wg, wu],
+                                [dgate, dup]), None
 
 
 def _plain_weights(x: torch.Tensor, mods):
@@ -622,7 +622,10 @@ def gated_linear(x: torch.Tensor, gate, up) -> Optional[torch.Tensor]:
     rows = x.reshape(-1, x.shape[-1]).contiguous()
     if not _require_ext().linear_gated_takes(rows, *ws):
         return None
-    return _GatedLinear.apply(rows, *ws).view(*x.shape[:-1], ws[0].shape[0])
+    # (inside the function weights need gradients under no_grad too: 7168 rows, 4096 ->
+    # 14336, 1174 us with the products stored and 1127 without)
+    keep = torch.is_grad_enabled() and any(t.requires_grad for t in (rows, *ws))
+    return _GatedLinear.apply(rows, *ws, keep).view(*x.shape[:-1], ws[0].shape[0])
 
 
 def build_varlen_tiles(cu_seqlens_cpu: torch.Tensor, device):

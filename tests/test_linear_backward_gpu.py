@@ -185,15 +185,27 @@ def test_joint_linear(m, ns, k):
 
 @pytest.mark.parametrize("m,n,k", [(760, 8192, 128), (1700, 4096, 192),
                                    (2041, 4096, 320), (4400, 1664, 256)])
-def test_gated_linear(m, n, k):
-    """Gate, up and activation of one kernel with their gradients, and without
-    what is kept for them."""
+def test_gated_linear(m, n, k, monkeypatch):
+    """Gate, up and activation of one kernel with their gradients; the products are
+    stored for a way back alone, and the result is the same without."""
     gate, up = (torch.nn.Linear(k, n, bias=False, device=DEV, dtype=torch.bfloat16)
                 for _ in range(2))
     x = rand(m, k, 5).requires_grad_()
+    ext, kept = ops._require_ext(), []
+    real = ext.linear_gated
+    monkeypatch.setattr(ext, "linear_gated",
+                        lambda *a: kept.append(a[-1]) or real(*a))
     y = ops.gated_linear(x, gate, up)
-    with torch.no_grad():
+    with torch.no_grad():              # (a log-probability pass)
         assert torch.equal(ops.gated_linear(x, gate, up), y)
+    for l in (gate, up):
+        l.requires_grad_(False)
+    assert torch.equal(ops.gated_linear(x.detach(), gate, up), y)
+    for l in (gate, up):
+        l.requires_grad_(True)
+    assert kept == [True, False, False]
+    alone, = real(x.detach(), gate.weight, up.weight, False)
+    assert torch.equal(alone, y)
     dy = rand(m, n, 7)
     y.backward(dy)
     xd = x.detach().double().requires_grad_()
