@@ -102,9 +102,9 @@ __global__ __launch_bounds__(256, 1) void product_kernel(
 }
 
 // out (R, C): the sum of left_p(row, inner) right_p(inner, column) over the parts, the
-// input's gradient of layers that share it.  In a layer of 7168 rows: through gate and up,
-// 14336 x 4096 each, 1019 us for 555 + 555 + 28 of two products and an addition, through
-// q, k and v 245 for 165 + 57 + 56 + 2 x 28.
+// input's gradient of layers that share it.  In a layer of 7168 and of 8192 rows: through
+// gate and up, 14336 x 4096 each, 1101 and 1245 us for 1132 and 1283 of two products and an
+// addition, through q, k and v 238 and 275 for 321 and 363 of three.
 constexpr int MOST = 3;
 struct Parts {
   const bf16_t *left[MOST], *right[MOST];

@@ -403,17 +403,21 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
       s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
     }
   };
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  if (PARTS > 1) clear();
   for (;;) {
     int p = 0;
     if (PARTS == 1 && now > 0) {
       sink.tile(last);
       pair(std::true_type());
       p = 1;
-    } else if (PARTS == 1 || now % PARTS == 0) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    } else if (PARTS == 1) {
+      clear();
     }
     for (; p < pairs; ++p) pair(std::false_type());
     if (!more || (PARTS > 1 && now % PARTS == PARTS - 1)) {
@@ -430,6 +434,9 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
         for (int e = 0; e < COLS; ++e) sums[e] = sums_of(acc[Sink::column_of(q, e)][j]);
         sink.put(j, q, sums);
       });
+      // (here and not where the next one begins: the compiler keeps numbers that nobody
+      // reads and spills others)
+      if (PARTS > 1) clear();
     }
     if (!more) break;
     ++now;
