@@ -253,18 +253,26 @@ bool linear_wgrad_takes(const torch::Tensor& dy, const torch::Tensor& x) {
 }
 
 // The same for linear_dgrad, where the library does better.  Where tiles fill rounds of
-// 256 to two thirds of what whole ones would cost it takes 0.70 to 0.93 of the library's
-// time, less full ones up to 1.09 (through 4096 x 4096 of 2048, 2600, 4600, 5135, 7168 rows,
-// 1.64, 1.29, 1.46, 1.31, 1.04 of that cost: 71, 68, 130, 133, 164 us for 65, 79, 144, 178,
-// 204); half a chip's tiles and less pay where the inner dimension is long enough to be
-// shared (256, 1024, 2048 rows through 14336 x 4096 46, 98, 176 for 69, 134, 209; through
-// 8192 x 2048 26, 46, 70 for 37, 60, 75; through 4096 x 4096 26, 47, 70 for 25, 42, 63).
+// 256 to 0.69 of what whole ones would cost it takes 0.61 to 1.02 of the library's time (at
+// 0.67 to 0.69 of it, through 18944 x 3584 of 2600 and 5120 rows 327 and 688 us for 320 and
+// 640, through 1536 x 1536 of 6144 34.6 for 34.1; through 4096 x 4096 of 2600, 5120, 7168 rows,
+// 0.77, 0.76, 0.96 of it, 79, 140, 164 for 89, 164, 204); half a chip's tiles and less pay
+// where the inner dimension is long enough to be shared (256, 1024, 2048 rows through 14336 x
+// 4096 61, 110, 190 for 77, 150, 241; through 4096 x 4096 26, 47, 70 for 25, 42, 63), unless
+// two blocks a tile at most leave much of the chip idle (through 8192 x 28672 of 64 and 130
+// rows 121 and 124 for 93 and 107, through 28672 x 8192 of 513, 700, 768 290, 310, 317 for 266,
+// 331, 336: 0.22, 0.44, 0.50, 0.68, 0.75 of it), and but for the fewest rows (64 and 130
+// through 8192 x 8192 49, 51 for 46, 65; 64 through 14336 x 4096 47 for 70).  Weights in turn
+// from memory.
 bool linear_dgrad_takes(const torch::Tensor& dy, const torch::Tensor& w) {
   if (!dgrad_fits(dy, w)) return false;
-  const long M = dy.size(0), N = dy.size(1), K = w.size(1);
-  if (tiles_of(M, K) <= CUS / 2) return N >= 8192 && M >= 64;
-  const double whole = (double)M * K / (CUS * SIDE * SIDE) * cost_of(8, N);
-  return rows_of(M, (K + SIDE - 1) / SIDE, N, 6).cost <= 1.5 * whole;
+  const long M = dy.size(0), N = dy.size(1), K = w.size(1), tiles = tiles_of(M, K);
+  const double rounds = (double)M * K / (CUS * SIDE * SIDE);
+  if (tiles <= CUS / 2) {
+    const long ways = ways_of(tiles, N);
+    return N >= 8192 && M >= (N > K ? 64 : 128) && (ways > 2 || rounds * ways >= 0.6);
+  }
+  return rows_of(M, (K + SIDE - 1) / SIDE, N, 6).cost <= 1.45 * rounds * cost_of(8, N);
 }
 
 // dW (N, K) = dY^T X of dY (M, N), X (M, K)
@@ -328,7 +336,12 @@ long inner_of(const std::vector<torch::Tensor>& dys) {
 }  // namespace
 
 // Whether linear_dgrad_sum has these operands and is the better choice than a product
-// each and additions: by the line of linear_dgrad's tiles that are not shared
+// each and additions: not where tiles leave rounds emptier than linear_dgrad's may, which
+// shares them.  (Rounds' cost by whole ones', us for a product each, weights in turn from
+// memory: gate and up 1.46, 1.48 635, 1333 for 642, 1326 of 2600 and 5120 rows of 3584; 1.62,
+// 1.62, 1.73, 1.85 266, 928, 300, 630 for 269, 795, 297, 585; 2.16 471 for 355.  q, k and v,
+// whose products alone are small, would gain beyond the line too: 1.63, 1.65, 1.78 112, 59,
+// 44 for 137, 91, 75, from 2.2 on as much.)
 bool linear_dgrad_sum_takes(const std::vector<torch::Tensor>& dys,
                             const std::vector<torch::Tensor>& ws) {
   if (dys.size() < 2 || dys.size() > MOST || dys.size() != ws.size()) return false;

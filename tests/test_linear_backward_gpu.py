@@ -105,7 +105,8 @@ def test_behind_the_last():
     (511, 5120, 2048), (512, 5120, 2048), (600, 5112, 2040),  # 160 tiles of dW
     (5119, 512, 256), (5120, 512, 256), (600, 5116, 2048),
     (2600, 256, 4096), (2700, 256, 4096), (5200, 320, 4096),  # 176, 336 of dX
-    (64, 8128, 264), (63, 8192, 264), (64, 8192, 264), (130, 8224, 520)])
+    (64, 8128, 264), (63, 8192, 264), (64, 8192, 264), (130, 8224, 520),
+    (270, 8192, 11264), (460, 8192, 11264)])          # two blocks a tile of dX
 def test_linear_backward(m, n, k):
     """Both sides of the lines where the trainer's linears take the kernels, and
     columns that they do not take."""
