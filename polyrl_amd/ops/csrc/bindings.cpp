@@ -10,6 +10,7 @@ void silu_mul(torch::Tensor out, torch::Tensor gate, torch::Tensor up);
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor linear_swiglu(torch::Tensor x, torch::Tensor w);
 bool linear_rows_pays(long M, long N, long K);
+std::vector<long> product_rows(long M, long cols, long K, long least);
 void linear_rows_add(torch::Tensor out, torch::Tensor x, torch::Tensor w);
 bool linear_joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws);
 std::vector<torch::Tensor> linear_joint(torch::Tensor x, std::vector<torch::Tensor> ws);
@@ -117,6 +118,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_rows_into", &linear_rows_into, "x W^T, W's rows in 8s");
   m.def("linear_rows_add", &linear_rows_add, "out += x W^T, rounded once");
   m.def("linear_rows_pays", &linear_rows_pays, "linear_rows for the library's product");
+  m.def("product_rows", &product_rows, "row parts of a product's tiles, their cost");
   m.def("linear_swiglu", &linear_swiglu, "SiLU(x Wg^T) * (x Wu^T)");
   m.def("rope_inplace", &rope_inplace, "NEOX RoPE in place (table-driven)");
   m.def("rope_kv_append", &rope_kv_append,

@@ -280,17 +280,36 @@ void linear_rows_into(torch::Tensor& out, const torch::Tensor& x,
 
 // Whether linear_rows is the better choice than the library's own: tiles that fill
 // rounds of 256 to 0.53 of what whole ones would cost, but not whole tiles of 256 rows,
-// which the library multiplies 1 to 6% faster.  (us, beside the library's: 4096 -> 1024 of
-// 3500, 4090, 4600, 5135, 8000 rows, 0.43, 0.50, 0.56, 0.63, 0.83 of that cost, 38.3, 38.6,
-// 40.0, 41.1, 51.3 and 35.0, 36.9, 44.6, 45.6, 57.5; 2048 -> 2048 of 2600, 4090, 5135 rows
-// 22.9, 29.1, 35.3 and 31.1, 34.2, 50.7, of 8000, whole tiles, 52.6 and 49.4; 8960 -> 1536 of
-// 2600, 3072, 3500 rows, 0.50, 0.59, 0.67, 77.9, 81.6, 83.0 and 70.9, 82.4, 92.3; of 120
-// shapes the 89 within the line take 0.51 to 1.00 of the library's time.)
+// which the library multiplies 1 to 6% faster where it has no long inner dimension to
+// choose for.  Weights beyond 16 MB come from memory: tiles of 96 rows, whose steps are
+// shorter than that takes, are left to the library, ones of 128 where there are few of them.
+// (us, beside the library's, weights in turn from memory: 4096 -> 1024 of 5135, 6145, 8192
+// rows 46, 46, 54 and 46, 51, 58; 2048 -> 2048 of 2300, 3072, 5135 26, 27, 38 and 30, 28, 49;
+// 96 rows a tile, 14336 -> 4096 of 1024, 28672 -> 8192 of 600, 8192 -> 8192 of 560, 8960 ->
+// 1536 of 3072 169, 324, 107, 105 and 132, 259, 87, 93; 128, 4096 -> 6144 of 1024 and 4096, 8960
+// -> 1536 of 4096, 4096 -> 4096 of 2048 56, 169, 114, 58 and 53, 156, 107, 63; 3584 -> 3584 of
+// 8192 152 and 146, 18944 -> 3584 of 4096 363 and 539.  Of 399 shapes the 149 within the line
+// take 0.52 to 1.06 of the library's time, 0.89 on average, six of them more than 1.02.)
 bool linear_rows_pays(long M, long N, long K) {
   if (M <= 0 || N <= 0 || K < PAIR) return false;
-  const Rows best = rows_of(M, (N + SIDE - 1) / SIDE, K, 3);
+  const long cols = (N + SIDE - 1) / SIDE;
+  const Rows best = rows_of(M, cols, K, 3);
   const double whole = (double)M * N / (CUS * SIDE * SIDE) * cost_of(8, K);
-  return best.cost <= 1.9 * whole && (best.parts < 8 || best.cost >= 1.05 * whole);
+  if (best.cost > 1.9 * whole) return false;
+  if (best.parts == 8)
+    return best.cost >= 1.05 * whole && (M % SIDE != 0 || K > 2 * N);
+  if (best.parts > 4 || N * K <= 1L << 23) return true;
+  const long tiles = (M + 32 * best.parts - 1) / (32 * best.parts) * cols;
+  return best.parts == 4 && M > 1024 && best.cost <= 1.5 * whole && tiles <= 2 * CUS;
+}
+
+// Row parts of a tile, 32 rows each, of M rows by ``cols`` tiles of columns with K inner
+// numbers, at least ``least`` (6 where products are kept or an operand is in COLUMNS, else
+// 3), and what the rounds cost
+std::vector<long> product_rows(long M, long cols, long K, long least) {
+  TORCH_CHECK(M > 0 && cols > 0 && K > 0 && least > 0 && least <= 8, "product_rows");
+  const Rows r = rows_of(M, cols, K, (int)least);
+  return {r.parts, r.cost};
 }
 
 // x (M, K), w (N, K)
