@@ -87,6 +87,7 @@ std::vector<torch::Tensor> pack_rows(torch::Tensor mask, torch::Tensor ids,
 torch::Tensor gather_rows(torch::Tensor x, torch::Tensor map);
 torch::Tensor embed_grad(torch::Tensor dy, torch::Tensor ids, int64_t V);
 torch::Tensor tuned_linear_fwd(torch::Tensor x, torch::Tensor w);
+long tuned_linear_pick(long M, long N, long K);
 torch::Tensor tuned_linear_dgrad(torch::Tensor dy, torch::Tensor w);
 torch::Tensor tuned_linear_wgrad(torch::Tensor dy, torch::Tensor x);
 torch::Tensor linear_wgrad(torch::Tensor dy, torch::Tensor x);
@@ -153,6 +154,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_grad", &embed_grad, "embedding gradient, fp32 sums in row order");
   m.def("tuned_linear_fwd", &tuned_linear_fwd,
         "Y = X W^T via hipBLASLt with per-shape in-process algo search");
+  m.def("tuned_linear_pick", &tuned_linear_pick,
+        "what tuned_linear_fwd found: 1 the kernel, 0 an algorithm, -1 nothing yet");
   m.def("tuned_linear_dgrad", &tuned_linear_dgrad, "dX = dY W: the kernel where it is the faster, else algo-pinned");
   m.def("tuned_linear_wgrad", &tuned_linear_wgrad,
         "dW = dY^T X: the kernel for many rows, else algo-pinned");
