@@ -49,12 +49,12 @@ def test_fused_add_rmsnorm():
     assert rel_err(out.cpu(), expect_norm) < 2e-2
 
 
-@pytest.mark.parametrize("d", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 4096,
-                               4104, 8192, 8200, 12288])
-@pytest.mark.parametrize("rows", [1, 130, 1024])
+@pytest.mark.parametrize("d", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 3064,
+                               3072, 4096, 4104, 8192, 8200, 12288])
+@pytest.mark.parametrize("rows", [1, 130, 1024, 1792])
 def test_rmsnorm_widths(rows, d):
     """Both sides of the widths from which a row takes more waves and more words
-    a thread."""
+    a thread, and rows that are read again."""
     g = torch.Generator(device=DEV).manual_seed(d + rows)
     x, res = (torch.randn(rows, d, generator=g, device=DEV).bfloat16()
               for _ in range(2))
