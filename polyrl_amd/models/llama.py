@@ -46,7 +46,12 @@ def _lin(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
 
 
 def _pack_align() -> int:
-    """GEMM M-alignment for the packed varlen path (0/1 disables)."""
+    """Packed rows come in multiples of this many (0/1: as they are).  The products'
+    time does not ask for it: steps of 897, 2204, 4412 and 7014 tokens of four models
+    take the same time in multiples of 1, 64, 128 and 256 rows but for 3% (two layers of
+    the 8B stack 5.0, 9.0, 16.4, 23.7 and 5.1, 8.9, 16.5, 23.8 ms in 1s and 256s).  But
+    each new number of rows has its algorithms searched for, a search for each of a
+    model's products, and micro-batches of whatever lengths have few numbers in 256s."""
     import os
     try:
         return max(int(os.environ.get("POLYRL_PACK_ALIGN", "256")), 1)
@@ -55,12 +60,8 @@ def _pack_align() -> int:
 
 
 def _pack_pad_to(model) -> int:
-    """Fixed-M padding target for the packed path (0 disables).  Measured
-    (profiles/PROFILES.md round 2): hipBLASLt loses 20-45% at mid-size M
-    from CU-grid tail quantization — M=8192 fills 256 CUs in exactly 2
-    waves (1.6 PF nt) while M~7000 strands a partial wave (0.88-1.27 PF),
-    and 256-alignment alone does NOT recover it.  Padding every micro to
-    the token budget makes all trunk GEMM shapes fixed AND optimal."""
+    """Packed rows of every micro-batch that nearly fills them (0: none), where a
+    trainer wants one number of rows, searched for once."""
     import os
     env = os.environ.get("POLYRL_PACK_PAD_TO")
     if env is not None:
@@ -374,13 +375,8 @@ class DecoderModel(nn.Module):
         return m(ids)
 
     def _padded_tokens(self, T: int) -> int:
-        """Rows of a packed batch of T tokens.
-
-        Dynamic token-budget micros produce arbitrary totals (6472, 7216, ...)
-        and hipBLASLt loses ~35-45% on the [M,14336]x[14336,4096] trunk
-        GEMMs at unaligned M (profiles/PROFILES.md).  Fixed-M padding only pays off when the micro is nearly full
-        (dense packing leaves one small tail micro — padding THAT to the
-        whole budget would waste more GEMM work than the shape buys)."""
+        """Rows of a packed batch of T tokens: a multiple, and the fixed number where
+        the batch nearly fills it (one small last micro-batch would cost more)."""
         align = _pack_align()
         pad_to = _pack_pad_to(self)
         if pad_to and 0.75 * pad_to <= T <= pad_to:

@@ -1,14 +1,11 @@
 // Per-shape hipBLASLt algo search for the trainer's hot GEMMs (host code).
 //
-// Why: hipBLASLt's default heuristic picks 20-45%-off algorithms for the
-// trainer's in-situ shapes (measured, profiles/PROFILES.md round 2: nt at
-// M~7000 runs 0.88-1.27 PF vs 1.6 PF for the best shape; committed
-// TunableOp tables proved NON-transferable across boxes in round 1).  This
-// is the robust in-process alternative: on the first call for a (layout,
-// M, N, K) key, request a heuristic candidate list, time each candidate on
-// the live stream, and cache the winner for the process lifetime.  No
-// files, no cross-box reuse, bounded cost (~32 algos x 4 runs per shape,
-// once).
+// Why: hipBLASLt's default heuristic picks algorithms that are 20 to 45% off for the
+// trainer's shapes (nt of some 7000 rows 0.88 to 1.27 PFLOP/s where the best runs at 1.6),
+// and tables of algorithms from one machine do not hold on another.  On the first call
+// for a (layout, M, N, K) key a list of candidates is asked for, each is timed on the
+// live stream, and the winner is kept for the process's life.  No files, bounded cost
+// (at most 48 algorithms, 4 runs each, once a shape).
 //
 // Reference capability: the update-loop GEMM throughput the reference gets
 // from cuBLAS/flash-attn inside torch (stream_dp_actor.py:153-224).

@@ -318,9 +318,10 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w) {
 }
 
 // out += x W^T, rounded once: what follows need not add it.  (us, the product and a norm
-// that adds, and this and a norm: 4096 -> 1024 of 1024, 2600, 5135, 8192 rows 38.3, 40.9,
-// 46.6, 61.7 and 39.4, 40.6, 45.2, 59.6; 2048 -> 2048 24.3, 29.9, 46.7, 70.0 and 24.8, 29.2,
-// 45.1, 66.7; 1024 -> 1024 15.7, 18.1, 21.0, 27.9 and 17.1, 18.8, 20.9, 25.7)
+// that adds, and this and a norm: 1024 -> 1024 of 1024, 3072, 4096, 8192 rows 14.7, 17.2, 19.0,
+// 26.6 and 16.2, 18.0, 19.2, 25.3; 4096 -> 1024 of 5135, 8192 45.5, 62.4 and 45.7, 60.0; 2048 ->
+// 2048 of 2600, 4096 28.7, 38.0 and 28.3, 36.4; 4096 -> 4096 of 1300, 2048, 6145 45.1, 62.0, 174
+// and 45.9, 60.7, 166; 14336 -> 4096 of 1300, 2600 135, 242 and 135, 224)
 void linear_rows_add(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   for (const auto* t : {&out, &x, &w})
     TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->dim() == 2 &&

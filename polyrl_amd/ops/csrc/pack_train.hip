@@ -104,8 +104,12 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
 // in that order, counted by comparing it with all, 256 of them and a stretch of the
 // others a block; the counts add up the same in any order.  (7168 tokens, rows of 4096
 // numbers, 128256 ids: ranks 11 us, order 5, sums 39, shares 5, the fill 139; a sort's
-// scans and merges, sums and their scatter took 300 beside the fill.  Comparisons grow
-// with the square of the tokens: beyond 32768 the library's backward.)
+// scans and merges, sums and their scatter took 300 beside the fill.  The whole, beside
+// the library's backward, which sorts, of 512, 2048, 7168 and 32768 tokens 172, 180, 208, 403
+// and 202, 336, 429, 1276; an id that a fourth, half and all of 32768 tokens have 692, 969,
+// 1538 and 1188, 1424, 1529, of 7168 all 450 and 487: its shares are added up one after the
+// other.  32768 tokens of 32000 ids, 1024 numbers, 157 and 248, ids by Zipf's law 211 and 222:
+// comparisons grow with the square of the tokens, and beyond that it is the library's.)
 constexpr int STRETCH = 256;
 
 __global__ __launch_bounds__(256) void embed_rank_kernel(

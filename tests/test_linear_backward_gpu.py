@@ -81,6 +81,16 @@ def test_tiles_in_turn(inner):
     dgrad(4353, (inner + 63) // 64 * 64, 8200)
 
 
+@pytest.mark.parametrize("n", [256, 320, 384])
+@pytest.mark.parametrize("m,parts", [(189, 6), (221, 7), (445, 7), (253, 8), (509, 8)])
+def test_dgrad_rows_in_turn(m, parts, n):
+    """A block's second tile and third of every number of row parts: a tile's sums
+    leave beside the next one's first step."""
+    cols = 290                         # (more tiles than blocks that run at once)
+    assert ops._require_ext().product_rows(m, cols, n, 6)[0] == parts
+    dgrad(m, n, 256 * cols - 8)
+
+
 @pytest.mark.parametrize("inner", [1280, 1344, 1984, 5120, 8192])
 @pytest.mark.parametrize("n,k", [(256, 256), (264, 520), (1024, 1304)])
 def test_shared(inner, n, k):
@@ -99,6 +109,44 @@ def test_behind_the_last():
     ext = ops._require_ext()
     check(dy[:m].t(), x[:m], ext.linear_wgrad(dy[:m], x[:m]))
     check(dy[:m], w[:n], ext.linear_dgrad(dy[:m], w[:n]))
+
+
+def same_kinds(got, want):
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(got), kind(want))
+    live = want.isfinite()
+    assert live.any() and not live.all()
+    assert (got.double() - want)[live].norm() <= 5e-3 * want[live].norm()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_not_finite(bad):
+    """Numbers that are not finite reach the sums that they are a part of, and no
+    other ones."""
+    ext = ops._require_ext()
+    m, n, k = 600, 320, 264
+    dy, x, w = rand(m, n, 3), rand(m, k, 4), rand(n, k, 5)
+    dy[17, 3] = dy[m - 1, n - 1] = x[40, 9] = w[250, 100] = bad
+    x[17, 5] = w[3, 7] = 0             # (times infinity)
+    d, f, v = dy.double(), x.double(), w.double()
+    same_kinds(ext.linear_wgrad(dy, x), d.t() @ f)
+    same_kinds(ext.linear_dgrad(dy, w), d @ v)
+    same_kinds(ext.linear_dgrad_sum([dy, dy[:, :64].contiguous()],
+                                    [w, w[:64].contiguous()]),
+               d @ v + d[:, :64] @ v[:64])
+    m, k = 1700, 192
+    x, wg, wu = rand(m, k, 6), rand(4096, k, 7), rand(4096, k, 8)
+    x[m - 1, 0] = wg[2000, k - 1] = wu[4095, 5] = bad
+    y, gate, up = ext.linear_gated(x, wg, wu, True)
+    g, u = x.double() @ wg.double().t(), x.double() @ wu.double().t()
+    same_kinds(gate, g)
+    same_kinds(up, u)
+    same_kinds(y, g * torch.sigmoid(g) * u)
+    out = rand(m, 4096, 9)
+    out[5, 6] = out[m - 1, 2000] = -bad
+    old = out.double()
+    ops.linear_rows_add(out, x, wg)
+    same_kinds(out, old + g)
 
 
 @pytest.mark.parametrize("m,n,k", [

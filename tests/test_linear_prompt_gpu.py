@@ -40,13 +40,10 @@ def check_rows(x, w, got):
         assert ((got[at:at + 8192].double() - want).abs() <= bound).all(), at
 
 
-def row_tiles(m, cols, k):
-    """The row tiles of a block: the fewest that end the last round of 256 blocks
-    earliest."""
-    def cost(jt):
-        blocks = -(-m // (32 * jt)) * cols
-        return -(-blocks // 256) * ((jt + 1) * (k // 64) + 20)
-    return min(range(2, 9), key=cost)
+def row_parts(m, cols, k):
+    """Row parts, 32 rows each, of the tiles that the library takes for ``cols`` tiles
+    of columns."""
+    return ops._require_ext().product_rows(m, cols, k, 3)[0]
 
 
 @pytest.mark.parametrize("tiles", [2, 3, 4, 5, 6, 7, 8, 9])
@@ -55,13 +52,13 @@ def test_row_tiles(tiles):
     check(8192 * tiles - 17, 128, 64)
 
 
-@pytest.mark.parametrize("tiles", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("parts", [3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("inner", [2, 3, 4, 5, 16])
-def test_inner_tiles(tiles, inner):
-    """Every number of row tiles with inner tiles that fill the buffers just, take
+def test_inner_tiles(parts, inner):
+    """Every number of row parts with inner tiles that fill the buffers just, take
     their places in turn and go round; an incomplete last row tile."""
-    m, k = 8192 * tiles - 17, 64 * inner
-    assert row_tiles(m, 1, k) == tiles
+    m, k = 8192 * parts - 17, 64 * inner
+    assert row_parts(m, 1, k) == parts
     x, w, _ = check(m, 128, k)
     check_rows(x, w, ops.linear_rows(x, w))
 
@@ -236,6 +233,7 @@ def test_sums_beside_the_next_tile(parts, m, k):
     leave the accumulators while the next one's first step fills them.  Rows and
     columns short of a tile; what stands behind the outputs is not touched."""
     cols = 300
+    assert row_parts(m, cols, k) == parts
     n = 256 * cols - 8
     x = torch.randn(m, k, device=DEV).bfloat16()
     w = torch.randn(n, k, device=DEV).bfloat16()
@@ -276,12 +274,14 @@ def test_outputs_beyond_the_cache():
     assert torch.equal(rows(w), torch.cat([rows(w[:64136]), rows(w[64136:])], 1))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 256, 64), (97, 512, 128), (700, 1024, 320),
-                                   (513, 256, 1024), (93, 76800, 256),
-                                   (445, 76800, 320), (253, 76800, 384)])
-def test_added(m, n, k):
+@pytest.mark.parametrize("m,n,k,parts", [
+    (1, 256, 64, 3), (97, 512, 128, 3), (700, 1024, 320, 3), (513, 256, 1024, 3),
+    (93, 76800, 256, 3), (125, 76800, 256, 4), (157, 76800, 320, 5),
+    (189, 76800, 384, 6), (445, 76800, 320, 7), (253, 76800, 384, 8)])
+def test_added(m, n, k, parts):
     """Outputs that hold numbers already: one rounding of the whole sum, edges of
     tiles, a block's tiles one after the other; what stands behind is not touched."""
+    assert row_parts(m, n // 256, k) == parts
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
     w = torch.randn(n, k, generator=g, device=DEV).bfloat16()

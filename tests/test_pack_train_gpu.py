@@ -155,6 +155,28 @@ def test_model(rows):
         assert (a - b_).norm() <= 2 ** -8 * b_.norm() + 1e-30
 
 
+def test_checkpointing():
+    """A packed step whose layers are computed again on the way back."""
+    torch.manual_seed(0)
+    cfg = get_model_config("llama-tiny")
+    m = CausalLM(cfg).to(DEV, torch.bfloat16).train()
+    m.model.use_remove_padding = True
+    mask = masks("left", 5, 90)
+    ids = torch.randint(cfg.vocab_size, (5, 90), generator=gen(6), device=DEV)
+    pos = (mask.long().cumsum(-1) - 1).clamp_(min=0)
+
+    def run():
+        out = m(ids, attention_mask=mask, position_ids=pos,
+                logits_slice=slice(-41, -1))
+        return [out.detach()] + list(torch.autograd.grad(
+            out.float().square().sum(), list(m.parameters())))
+    want = run()
+    m.gradient_checkpointing_enable()
+    assert m.model.gradient_checkpointing
+    for a, b in zip(run(), want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("how", ["forward", "hook", "global"])
 def test_embedding_with_more(how, monkeypatch):
     """An embedding whose forward was replaced, or that hooks watch, is called."""
