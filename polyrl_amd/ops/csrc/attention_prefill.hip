@@ -23,7 +23,8 @@
 // lift some row's maximum; only tiles that touch the causal border or the
 // sequence's end are masked.
 //
-// What bounds it: at 64 the vector instructions, 76% of the cycles (185 a tile of
+// What bounds it: at 64 the vector instructions, 76% of the cycles, 87% of those in which
+// a CU has a wave, beside matrix instructions at 38 and 44 (185 vector instructions a tile of
 // a wave: exponential, scale, sum, maximum, rounding, and the rescaling of the
 // output); at 128 those and the matrix instructions, 58% and 44%, and what is
 // left of their taking turns (the 16-row score tiles with scalar LDS gathers for

@@ -403,13 +403,12 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
       s0 = s2, s1 = s3, s2 = s4, s3 = t0, s4 = t1;
     }
   };
-  auto clear = [&] {
+  if constexpr (PARTS > 1) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  };
-  if (PARTS > 1) clear();
+  }
   for (;;) {
     int p = 0;
     if (PARTS == 1 && now > 0) {
@@ -417,7 +416,10 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
       pair(std::true_type());
       p = 1;
     } else if (PARTS == 1) {
-      clear();
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     for (; p < pairs; ++p) pair(std::false_type());
     if (!more || (PARTS > 1 && now % PARTS == PARTS - 1)) {
@@ -436,7 +438,12 @@ DEV_INLINE void run(char* lds, LeftLd left_ld, long right_ld, UnitsOf units,
       });
       // (here and not where the next one begins: the compiler keeps numbers that nobody
       // reads and spills others)
-      if (PARTS > 1) clear();
+      if constexpr (PARTS > 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < J; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
     }
     if (!more) break;
     ++now;
