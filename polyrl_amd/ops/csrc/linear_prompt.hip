@@ -364,8 +364,11 @@ bool joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws, l
 }  // namespace
 
 // Whether linear_joint has these operands (contiguous bf16 matrices, the weights' rows in
-// 256s) and is the better choice than a product each.  4096 -> 4096, 1024, 1024 of 7168
-// rows: 229 us for 158, 52 and 52.
+// 256s) and is the better choice than a product each: rounds that cost up to 1.35 of whole
+// ones.  (That, us and a product each, weights in turn from memory: 4096 -> 4096, 1024, 1024
+// of 7168, 4096, 2048 rows, 1.04, 1.21, 1.21, 249, 169, 80 and 291, 181, 125; 8192 -> 8192, 1024,
+// 1024 of 2048, 1.30, 288 and 280.  Beyond the line it would gain as well: 4096 of 3072 and
+// 1536 rows, both 1.46, 131, 65 and 150, 107, 1536 -> 1536, 256, 256 of 4096, 1.68, 25 and 57.)
 bool linear_joint_takes(const torch::Tensor& x, const std::vector<torch::Tensor>& ws) {
   return joint_takes(x, ws, SIDE);
 }
@@ -385,7 +388,11 @@ std::vector<torch::Tensor> linear_joint(torch::Tensor x, std::vector<torch::Tens
   return outs;
 }
 
-// The same for linear_gated: rows of weights in 128s, as many of both
+// The same for linear_gated: rows of weights in 128s, as many of both.  (With the products
+// stored, us and two products with the activation's pass: 2048 -> 8192 of 8192 rows, 1.00, 462
+// and 468, 4096 -> 14336 of 2048, 7168, 1.14, 1.04, 382, 1186 and 384, 1323; beyond the line
+// 4096 -> 14336 of 700 and 520, 1.37, 1.85, 157, 151 and 181, 145, 1024 -> 4096 of 1024, 1.70, 26
+// and 43.)
 bool linear_gated_takes(const torch::Tensor& x, const torch::Tensor& wg,
                         const torch::Tensor& wu) {
   return wg.dim() == 2 && wu.dim() == 2 && wg.size(0) == wu.size(0) &&
