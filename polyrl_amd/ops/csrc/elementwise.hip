@@ -92,12 +92,13 @@ static void launch_rmsnorm(torch::Tensor& out, bf16_t* residual,
   if (D <= 512) launch(rmsnorm_kernel<FUSED_ADD, 64, 1>, 64);
   else if (D <= 1024) launch(rmsnorm_kernel<FUSED_ADD, 128, 1>, 128);
   else if (D <= 2048) launch(rmsnorm_kernel<FUSED_ADD, 256, 1>, 256);
-  // (rows of 3072 to 4096 numbers, 11 to 18 MiB of them, are read again the faster: 2048 of
-  // 3072 and 4096 6.4 and 9.0 us, from registers 7.5 and 10.7, 3072 of 3072 11.7 and 12.6; of
-  // 1536 x 3328 and 1280 x 4096 6.2, 6.0 and 6.1, 5.9, 3072 x 4096 15.8 and 15.3, and of 2048 to
+  // (rows of 3072 to 8192 numbers, 10 to 20 MiB of them, are read again the faster: 2048 of
+  // 3072 and 4096, 1792 of 4608, 1536 of 5120, 1024 of 8192 6.4, 9.0, 8.7, 8.4, 8.9 us, from
+  // registers 7.5, 10.7, 10.4, 9.5, 9.5; 1792 of 5632 12.0 and 12.5; not of 1280 x 4096, 1024 x
+  // 5120 6.0, 6.3 and 5.9, 5.8, 3072 x 4096, 2304 x 5120 15.8, 15.7 and 15.3, 14.6, nor 2048 to
   // 4096 rows of 2560 6.1, 14.0 and 6.1, 13.3)
-  else if (FUSED_ADD && D >= 3072 && D <= 4096 && rows * D >= 21 << 18 &&
-           rows * D <= 9 << 20)
+  else if (FUSED_ADD && D >= 3072 && D <= 8192 && rows * D >= 21 << 18 &&
+           rows * D <= 10 << 20)
     launch(rmsnorm_kernel<FUSED_ADD, 256, 0>, 256);
   else if (D <= 4096) launch(rmsnorm_kernel<FUSED_ADD, 512, 1>, 512);
   else if (D <= 8192) launch(rmsnorm_kernel<FUSED_ADD, 512, 2>, 512);
